@@ -50,7 +50,7 @@ class WinoConvFunction(torch.autograd.Function):
     def forward(ctx, x, w, bias, stride, padding, m, U):
         ctx.save_for_backward(x, w)
         ctx.conf = (stride, padding, m, bias is not None)
-        return engine.conv_forward(x, w, bias, stride, padding, m, U=U)
+        return engine.conv_forward(x, w, bias, stride, padding, m, U=U, row=True)
 
     @staticmethod
     def backward(ctx, dy):
@@ -142,15 +142,15 @@ class _WinoConvNd(nn.Module):
         m = self._tile_for(x.dtype)
         # the form of the plan (Winograd pieces, or the direct form the library takes for large strided problems)
         # depends on the batch size too, and the transformed filter of one form does not fit the other
-        form = engine.plan_form(x.shape, w.shape, x.dtype, self.stride[0], self.padding, m)
+        form = engine.plan_form(x.shape, w.shape, x.dtype, self.stride[0], self.padding, m, row=True)
         key = (self.weight._version, self.weight.data_ptr(), tuple(x.shape[2:]), x.dtype, m, form)
         if self._cache is None or self._cache[0] != key:
-            U = engine.transform_filter(w.detach(), x.shape, self.stride[0], self.padding, m)
+            U = engine.transform_filter(w.detach(), x.shape, self.stride[0], self.padding, m, row=True)
             self._cache = (key, U)
         b = None if self.bias is None else self.bias.to(x.dtype)
         if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (b is not None and b.requires_grad)):
             return WinoConvFunction.apply(x, w, b, self.stride[0], self.padding, m, self._cache[1])
-        return engine.conv_forward(x, w.detach(), b, self.stride[0], self.padding, m, U=self._cache[1])
+        return engine.conv_forward(x, w.detach(), b, self.stride[0], self.padding, m, U=self._cache[1], row=True)
 
 
 class WinoConv2d(_WinoConvNd):

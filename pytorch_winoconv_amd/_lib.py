@@ -35,7 +35,7 @@ class ConvDesc(ctypes.Structure):
                 ("stride", ctypes.c_int), ("m", ctypes.c_int), ("dtype", ctypes.c_int),
                 ("chunk_images", ctypes.c_int), ("whole_kernel", ctypes.c_int), ("stacked", ctypes.c_int),
                 ("unfused", ctypes.c_int), ("x_layout", ctypes.c_int), ("y_layout", ctypes.c_int),
-                ("direct", ctypes.c_int)]
+                ("direct", ctypes.c_int), ("row", ctypes.c_int)]
 
 
 # name -> (restype, argtypes); every symbol include/winoconv.h declares

@@ -56,6 +56,8 @@ struct Layout {
   size_t u_bytes, v_bytes, m_bytes;   // each rounded up to 256
   bool thin;                          // the one-kernel path runs: V and M are not needed
   bool direct;                        // the direct form: the product reads x itself, V and M are not needed
+  bool row;                           // the row form: one kernel as well
+  bool whole() const { return thin || direct || row; }      // one pass over the whole batch, only U in the workspace
   bool x_direct;                      // channel-first x is read by the input transform itself
   size_t xcl_bytes, ycl_bytes;        // channel-last scratch copies of a chunk of x / of y (0 if not needed)
   // 3-D F(2,3)^3 plans in 16-bit types: the width axis is taken inside the product (fold_filter_w, gemm.hip).  V and M
@@ -65,7 +67,7 @@ struct Layout {
   size_t fold_bytes;
   SharedShift fold_shift;             // one run of three pieces, each one row of V further
   long long fold_rows_per_image;      // rows of V and M: the pixel columns of all tile rows (tiles_per_image where the plan is not folded)
-  size_t need() const { return (thin || direct ? u_bytes : u_bytes + fold_bytes + v_bytes + m_bytes) + xcl_bytes + ycl_bytes; }
+  size_t need() const { return (whole() ? u_bytes : u_bytes + fold_bytes + v_bytes + m_bytes) + xcl_bytes + ycl_bytes; }
 };
 
 size_t round256(size_t v) { return (v + 255) / 256 * 256; }
@@ -83,6 +85,12 @@ int make_layout(const wc_conv_desc* d_in, Layout* L) {
   // the direct form has no tiles: its shapes are those of the plain plan with the same kernel, stride and padding
   wc_conv_desc plain = *d_in;
   L->direct = d_in->direct == 1;
+  L->row = d_in->row == 1;
+  if (L->row) {
+    if (!row_conv_fits(d_in)) return fail(WC_ERR_UNSUPPORTED, "row form: 16-bit types, stride 1, 3x3 or 3x3x3 kernels, x below 1 GiB");
+    plain.direct = 0; plain.stacked = 0; plain.m = 2; plain.whole_kernel = 0; plain.unfused = 1; plain.row = 0;
+    L->direct = false;
+  }
   if (L->direct) {
     if (!direct_conv_fits(d_in))
       return fail(WC_ERR_UNSUPPORTED, "direct form: 2-D, input channels a multiple of 32 (fp32: 16; or at most 4 at stride 2 in a 16-bit type), "
@@ -118,16 +126,16 @@ int make_layout(const wc_conv_desc* d_in, Layout* L) {
   const long long Pc = L->tiles_per_image * chunk;
   if (T * Pc * (long long)(L->Cp > L->ldm ? L->Cp : L->ldm) >= (1ll << 40))
     return fail(WC_ERR_UNSUPPORTED, "chunk of %d images is too large", chunk);
-  L->u_bytes = L->direct ? round256(direct_u_elems(d) * L->es)
+  L->u_bytes = L->row ? round256(row_u_elems(d) * L->es) : L->direct ? round256(direct_u_elems(d) * L->es)
                          : round256((size_t)T * d->K * L->Cp * L->es);
   L->v_bytes = round256((size_t)T * (Pc + (L->shared ? L->shift.tail : 0)) * L->vrow * L->es);
   L->m_bytes = round256((size_t)T * Pc * L->ldm * L->es);
-  L->thin = !L->direct && !d->unfused && thin_conv_fits(d, &L->plan);
+  L->thin = !L->direct && !L->row && !d->unfused && thin_conv_fits(d, &L->plan);
   L->fold = false; L->fold_bytes = 0;
   L->fold_rows_per_image = L->tiles_per_image;
   {
     const wc_plan& pl = L->plan;
-    const bool cube = !L->direct && !L->shared && !d->whole_kernel && d->ndim == 3 && pl.n_pieces == 1 &&
+    const bool cube = !L->direct && !L->row && !L->shared && !d->whole_kernel && d->ndim == 3 && pl.n_pieces == 1 &&
                       pl.tap_step == 1 && pl.m[0] == 2 && pl.m[1] == 2 && pl.m[2] == 2 && pl.piece[0].r[0] == 3 &&
                       pl.piece[0].r[1] == 3 && pl.piece[0].r[2] == 3 && (d->dtype == WC_F16 || d->dtype == WC_BF16);
     // Half the V and M traffic for half more multiplications and one more launch: it pays where the pipeline waits
@@ -154,12 +162,13 @@ int make_layout(const wc_conv_desc* d_in, Layout* L) {
   }
   // channel-first tensors: the input transform of small single-piece plans reads x as it is; everything else goes
   // through a channel-last copy of one chunk (the one-kernel path: of the whole batch)
-  L->x_direct = d->x_layout == 1 && ((!L->thin && !L->direct && input_transform_nchw_fits(d, &L->plan)) ||
+  L->x_direct = d->x_layout == 1 && ((!L->whole() && input_transform_nchw_fits(d, &L->plan)) ||
                                      (L->direct && (direct_first_fits(d_in) || direct_first3d_fits(d_in))));      // ... and so do the first-layer kernels
-  const size_t images = L->thin || L->direct ? d->N : chunk;
-  const size_t x_image = (size_t)d->in[0] * d->in[1] * d->in[2] * d->C * L->es;
+  const size_t images = L->whole() ? d->N : chunk;
+  // the row form reads channel-last x with its channels padded to a multiple of 8
+  const size_t x_image = (size_t)d->in[0] * d->in[1] * d->in[2] * (L->row ? wc_padded_channels8(d->C) : d->C) * L->es;
   const size_t y_image = (size_t)L->out[0] * L->out[1] * L->out[2] * d->K * L->es;
-  L->xcl_bytes = d->x_layout == 1 && !L->x_direct ? round256(images * x_image) : 0;
+  L->xcl_bytes = (d->x_layout == 1 && !L->x_direct) || (L->row && d->C % 8 != 0) ? round256(images * x_image) : 0;
   L->ycl_bytes = d->y_layout == 1 ? round256(images * y_image) : 0;
   return WC_OK;
 }
@@ -222,7 +231,7 @@ int wc_conv_u_elems(const wc_conv_desc* d, size_t* elems) {
   Layout L;
   int rc = make_layout(d, &L);
   if (rc) return rc;
-  *elems = L.direct ? direct_u_elems(d) : (size_t)L.plan.t_total * d->K * L.Cp;
+  *elems = L.row ? row_u_elems(d) : L.direct ? direct_u_elems(d) : (size_t)L.plan.t_total * d->K * L.Cp;
   return WC_OK;
 }
 
@@ -266,10 +275,10 @@ int forward_impl(const wc_conv_desc* d, const void* x, const void* w, const int6
                  d->ndim, dt[d->dtype], d->N, d->C, d->K, d->in[0], d->in[1], d->in[2], d->kernel[0], d->kernel[1], d->kernel[2],
                  d->stride, d->pad[0], d->pad[1], d->pad[2], L.plan.m[0], L.plan.m[1], L.plan.m[2], L.plan.n_pieces, L.plan.t_total,
                  d->stacked, d->whole_kernel ? " whole-kernel tile" : "",
-                 L.direct ? "direct form: the product reads x" : L.thin ? "one fused kernel" : L.fold ? "input transform (depth, height), shifted batched GEMM with the width taps along its reduction, output transform" : (L.shared ? "input transform, shifted batched GEMM, output transform"
+                 L.row ? "row form: one fused kernel, F(4,3) along the width" : L.direct ? "direct form: the product reads x" : L.thin ? "one fused kernel" : L.fold ? "input transform (depth, height), shifted batched GEMM with the width taps along its reduction, output transform" : (L.shared ? "input transform, shifted batched GEMM, output transform"
                                                          : "input transform, batched GEMM, output transform"),
-                 L.thin || L.direct ? d->N : L.chunk, L.tiles_per_image, need, L.u_bytes, L.thin || L.direct ? (size_t)0 : L.v_bytes,
-                 L.thin || L.direct ? (size_t)0 : L.m_bytes, L.xcl_bytes, L.ycl_bytes,
+                 L.whole() ? d->N : L.chunk, L.tiles_per_image, need, L.u_bytes, L.whole() ? (size_t)0 : L.v_bytes,
+                 L.whole() ? (size_t)0 : L.m_bytes, L.xcl_bytes, L.ycl_bytes,
                  d->x_layout ? (L.x_direct ? "channel-first, read by the input transform" : "channel-first, copied") : "channel-last",
                  d->y_layout ? "channel-first, copied" : "channel-last", U_cached ? "transformed by the caller" : "transformed here");
   }
@@ -278,7 +287,7 @@ int forward_impl(const wc_conv_desc* d, const void* x, const void* w, const int6
   void* Ufold = ws + L.u_bytes;
   void* V = ws + L.u_bytes + L.fold_bytes;
   void* M = ws + L.u_bytes + L.fold_bytes + L.v_bytes;
-  unsigned char* tail = ws + (L.thin || L.direct ? L.u_bytes : L.u_bytes + L.fold_bytes + L.v_bytes + L.m_bytes);
+  unsigned char* tail = ws + (L.whole() ? L.u_bytes : L.u_bytes + L.fold_bytes + L.v_bytes + L.m_bytes);
   bool folded = false;
   void* Xcl = tail;                       // channel-last copies of channel-first tensors, one chunk each
   void* Ycl = tail + L.xcl_bytes;
@@ -286,7 +295,7 @@ int forward_impl(const wc_conv_desc* d, const void* x, const void* w, const int6
   const void* U = U_cached;
   // the three-kernel path transforms the filter in the launch of the first chunk's input transform (unless the
   // stages are being timed one by one)
-  bool filter_with_input = !U && !stage_ms && !L.thin && !L.direct;
+  bool filter_with_input = !U && !stage_ms && !L.whole();
   if (!U && !filter_with_input) {
     rc = timer.run(WC_STAGE_FILTER, [&] { return wc_filter_transform(d, &L.plan, w, w_strides, Uws, stream); });
     if (rc) return rc;
@@ -299,18 +308,24 @@ int forward_impl(const wc_conv_desc* d, const void* x, const void* w, const int6
   const long long out_pos = (long long)L.out[0] * L.out[1] * L.out[2];
   const size_t x_image = (size_t)in_pos * d->C * L.es;
   const size_t y_image = (size_t)out_pos * d->K * L.es;
-  const int step = L.thin || L.direct ? d->N : L.chunk;
+  const int step = L.whole() ? d->N : L.chunk;
   for (int b0 = 0; b0 < d->N; b0 += step) {
     const int n = (d->N - b0 < step) ? d->N - b0 : step;
     const void* xin = static_cast<const unsigned char*>(x) + b0 * x_image;
     void* yout = static_cast<unsigned char*>(y) + b0 * y_image;
     if (L.xcl_bytes) {
-      rc = timer.run(WC_STAGE_LAYOUT_IN, [&] { return transpose_images(xin, Xcl, n, d->C, in_pos, (int)L.es, stream); });
+      rc = timer.run(WC_STAGE_LAYOUT_IN, [&] {
+        if (L.row) return pad_channels(xin, Xcl, n, d->C, wc_padded_channels8(d->C), in_pos, d->x_layout == 1, stream);
+        return transpose_images(xin, Xcl, n, d->C, in_pos, (int)L.es, stream);
+      });
       if (rc) return rc;
       xin = Xcl;
     }
     void* ydst = L.ycl_bytes ? Ycl : yout;
-    if (L.direct) {
+    if (L.row) {
+      rc = timer.run(WC_STAGE_PRODUCT, [&] { return row_conv(&dcl, xin, n, U, bias, ydst, stream); });
+      if (rc) return rc;
+    } else if (L.direct) {
       rc = timer.run(WC_STAGE_PRODUCT, [&] { return direct_conv(&dcl, xin, n, U, bias, ydst, stream); });
       if (rc) return rc;
     } else if (L.thin) {

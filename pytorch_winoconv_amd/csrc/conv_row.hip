@@ -1,0 +1,675 @@
+// One-kernel convolution on the tile F(4, 3) along the width axis only ("row form"): 16-bit types, stride 1, kernels
+// whose rows have three taps.
+//
+//   y[o_d, o_h, 4 w + i] = sum_t A^T[i][t]  sum_(r_d, r_h) sum_c  U[r][t][k][c]  V[o_d + r_d, o_h + r_h, w][t][c]
+//   V[., w][t] = sum_j B^T[t][j] x[., 4 w + j],      U[r][t] = sum_j G[t][j] w[r, j]
+//
+// The three-kernel path writes V and M to memory and reads them back (2.25 times the input and the output each way for
+// F(4x4, 3x3), 4 times for F(2x2, 3x3)), which is what bounds it: at N=64, 256 -> 256 channels, 56x56 its three kernels
+// move 1.13 GB at 5 TB/s.  Here one axis is transformed and the other axes' taps stay in the reduction: half the
+// multiplications of the plain sum (the 2-D tile saves three quarters of them), but V lives in LDS, the products in
+// accumulators, and x, U and y are all the memory traffic there is.  The sum over taps and channels is taken in fp32
+// before the output transform, so only V and U are rounded to the storage type.
+//
+// Points of the tile: 0, +-a, +-1/a, infinity with a^2 = 0.425 instead of the customary 0, +-1, +-2.  They spread the
+// rounding of U and V evenly: with independent roundings of relative size e in both, the output's is 3.1 e in the root
+// mean square against 4.6 e with integer points, and against 2.4 e (products rounded to the storage type on top) for
+// F(2x2, 3x3).  Measured over 64 channels, fp16: 6e-4 of the output in the 2-norm, as F(2x2, 3x3), and a sixth of
+// F(4x4, 3x3)'s 3.7e-3.
+#include "wc_transform.h"
+
+#include <algorithm>
+
+namespace wc {
+
+namespace {
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr float kA2 = 0.425f, kB2 = 1.0f / 0.425f;             // a^2 and 1 / a^2
+constexpr float kA = 0.65192024f, kB = 1.0f / 0.65192024f;      // a (its square differs from kA2 by 5e-9)
+constexpr float kS = kA2 + kB2;
+
+template <typename T> struct MfmaRow;
+template <> struct MfmaRow<half_t> {
+  using Frag = f16x8;
+  static __device__ __forceinline__ f32x16 run(Frag a, Frag b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
+};
+template <> struct MfmaRow<bf16_t> {
+  using Frag = bf16x8;
+  static __device__ __forceinline__ f32x16 run(Frag a, Frag b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+};
+
+// d + f in fp32, rounded to T
+__device__ __forceinline__ bf16_t plus(bf16_t d, float f) { return static_cast<bf16_t>(static_cast<float>(d) + f); }
+__device__ __forceinline__ half_t plus(half_t d, float f) {
+  float one = 1.0f;
+  asm("" : "+s"(one));                  // d * 1 + f stays one v_fma_mix instead of a conversion, an addition and a conversion
+  return static_cast<half_t>(__builtin_fmaf(static_cast<float>(d), one, f));
+}
+
+struct RowArgs {
+  const void* x; const void* U; const void* bias; void* y;
+  int N, D, H, W, C, K;           // x (N, D, H, W, C), y (N, oD, oH, oW, K)
+  int oD, oH, oW, nW;             // nW tiles of 4 outputs per row
+  int pd, ph, pw;
+  int bn, bd, bh, bw;             // output box of a workgroup: images, planes, rows, tiles of a row
+  FastDiv f_bw, f_bh, f_bd, f_prow, f_irow;
+  int prow, irow;                 // LDS rows of a plane and of an image of the box's input (tile rows, with the halo and padding)
+  int n_d, n_h, n_w;              // boxes per axis
+  int n_kb, n_box, per_xcd;       // channel blocks, boxes
+  int box_fast;                   // 1: neighbouring workgroups share a channel block, 0: a box
+  int steps, local_steps;         // ceil(C / 32), and the share of one of the CS groups of wavefronts that split the channels
+  int x_bytes, u_bytes;
+};
+
+constexpr int kRowPitch = 64;     // LDS bytes per (element, row of a tile): 32 channels in four chunks of 16 bytes
+// Chunk g of row s lies at position g ^ (s / 4 % 4).  A 16-byte read is served in four phases of sixteen lanes over 64
+// banks, lanes 0-3, 12-15, 20-27 in the first, 4-11, 16-19, 28-31 in the second and the same 32 further up: of the lanes of
+// a phase with the same row modulo 4 each has another row / 4 modulo 4, so one chunk of 32 consecutive rows, from any
+// row on, is read without conflicts, and so is what a store writes, all chunks of 16 rows.
+__device__ __forceinline__ int v_offset(int s, int g) { return s * kRowPitch + ((g ^ (s >> 2)) & 3) * 16; }
+
+// What the NI items of a step carry beside their products: the transform of 8 UN channels, over the first two thirds of the
+// items, and for each unit six moves (an element to LDS, the next load of its register) behind its last channel
+template <int UN, int NI>
+struct RowItems {
+  // one unit: the middle of the step, so that its loads, issued in the last quarter, have the first one to arrive
+  static constexpr int from = UN == 1 ? NI / 4 : 0, to = UN == 1 ? 3 * NI / 4 : 2 * NI / 3;
+  static constexpr int first_channel(int item) {
+    const int n = item < from ? 0 : ((item - from) * 8 * UN + to - from - 1) / (to - from);
+    return n < 8 * UN ? n : 8 * UN;
+  }
+  static constexpr int channels(int item) { return first_channel(item + 1) - first_channel(item); }
+  static constexpr int window = UN == 1 ? NI - to : UN > 2 ? NI / 6 : NI / 3;
+  static constexpr int at(int v) { return from + (v / 6 + 1) * (to - from) / UN + v % 6 * window / 6; }
+  static constexpr int first_move(int item) { int n = 0; while (n < 6 * UN && at(n) < item) ++n; return n; }
+  static constexpr int moves(int item) { return first_move(item + 1) - first_move(item); }
+  static constexpr bool ok() {
+    if (at(6 * UN - 1) >= NI) return false;
+    for (int v = 0; v < 6 * UN; ++v)
+      if (first_channel(at(v)) < (v / 6 + 1) * 8) return false;       // moved before its unit is transformed
+    return true;
+  }
+};
+
+template <int KG, int TB, int S, int CS>
+constexpr int row_lds_bytes() {
+  const int v = CS * 2 * 6 * S * kRowPitch, ex = 2 * KG * 3 * TB * 8 * 256, part = (CS - 1) * 2 * KG * 3 * TB * 16 * 256;
+  return v > ex ? (v > part ? v : part) : (ex > part ? ex : part);
+}
+
+// KT: rows of y that are no multiple of 16 bytes
+template <typename T, int KD, int KH, int KG, int TB, int S, int CS, bool KT>
+__global__ __launch_bounds__(128 * KG * CS) __attribute__((amdgpu_waves_per_eu(2, TB == 2 ? 2 : 3)))
+void row_conv_kernel(RowArgs a) {
+  using Frag = typename MfmaRow<T>::Frag;
+  constexpr int R = KD * KH, Q = 2 * R, NI = 3 * Q, THREADS = 128 * KG, UN = S * 4 / THREADS;
+  constexpr int TS = S * kRowPitch, BUF = 6 * TS;
+  constexpr int UD = 3, VD = 3;      // depth of the rings of filter and input fragments
+  static_assert(RowItems<UN, NI>::ok(), "items of a step");
+  static_assert(S * 4 % THREADS == 0 && Q % UD == 0, "whole units per thread, ring of three");
+  extern __shared__ unsigned char lds_all[];
+  const int wg = xcd_remap(blockIdx.x, a.per_xcd);
+  if (wg >= a.n_kb * a.n_box) return;
+  int kb, box;
+  if (a.box_fast) { kb = wg / a.n_box; box = wg - kb * a.n_box; }
+  else { box = wg / a.n_kb; kb = wg - box * a.n_kb; }
+  const int b_w = box % a.n_w;
+  int q_ = box / a.n_w;
+  const int b_h = q_ % a.n_h; q_ /= a.n_h;
+  const int b_d = q_ % a.n_d;
+  const int n0 = q_ / a.n_d * a.bn, d0 = b_d * a.bd, h0 = b_h * a.bh, w0 = b_w * a.bw;
+  const int sd = a.bd + KD - 1, sh = a.bh + KH - 1;
+
+  const int lane = threadIdx.x & 63, wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int cs = wave_all / (2 * KG), wave = wave_all - cs * 2 * KG, tid = wave * 64 + lane;
+  const int tg = wave / KG, kg = wave % KG;
+  unsigned char* const lds = lds_all + cs * 2 * BUF;
+  const int step0 = cs * a.local_steps;                 // the channel blocks of this share: step0 .. + local_steps, as far as they exist
+  const __amdgpu_buffer_rsrc_t xdesc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.x), 0, a.x_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t udesc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.U), 0, a.u_bytes, 0x00020000);
+
+  // ---- filter fragments: a ring of three groups (row tap, half of a channel block) of three elements
+  const int n_groups = a.steps * Q, k_blocks = (a.K + 31) / 32;
+  const int u_lane = lane * 16 + tg * 3072;
+  const int u_base = min(kb * KG + kg, k_blocks - 1) * n_groups * 6144;
+  u32x4 uf[UD][3];
+  auto load_u = [&](int slot, int group, int t) {
+    uf[slot][t] = __builtin_amdgcn_raw_buffer_load_b128(udesc, u_lane + t * 1024, u_base + min(step0 * Q + group, n_groups - 1) * 6144, 0);
+  };
+
+  // ---- input: units of (row of a tile, 8 channels)
+  int xo[UN][6];
+  u32x4 xr[UN][6];
+#pragma unroll
+  for (int i = 0; i < UN; ++i) {
+    const int u = tid + i * THREADS, g = u & 3;
+    int s = u >> 2;
+    const int in = fast_div(s, a.f_irow); s -= in * a.irow;
+    const int zd = fast_div(s, a.f_prow); s -= zd * a.prow;
+    const int zh = fast_div(s, a.f_bw), iw = s - zh * a.bw;
+    const int n = n0 + in, d = d0 + zd - a.pd, h = h0 + zh - a.ph, w = (w0 + iw) * 4 - a.pw;
+    const bool ok = in < a.bn && zd < sd && zh < sh && n < a.N && (unsigned)d < (unsigned)a.D && (unsigned)h < (unsigned)a.H;
+    const int base = (((n * a.D + d) * a.H + h) * a.W + w) * a.C * 2 + g * 16;
+#pragma unroll
+    for (int j = 0; j < 6; ++j) xo[i][j] = ok && (unsigned)(w + j) < (unsigned)a.W ? base + j * a.C * 2 : (int)kOutside;
+  }
+  // the channel block is in the scalar offset; beyond the last channel of the last block lanes load zeros (cut_x)
+  auto load_x = [&](int i, int j, int step) {
+    xr[i][j] = __builtin_amdgcn_raw_buffer_load_b128(xdesc, xo[i][j], min(step0 + step, a.steps - 1) * 64, 0);
+  };
+  auto cut_x = [&](int step) {
+    if (step0 + step >= a.steps - 1 && (tid & 3) * 8 + (step0 + step) * 32 >= a.C) {
+#pragma unroll
+      for (int i = 0; i < UN; ++i)
+#pragma unroll
+        for (int j = 0; j < 6; ++j) xo[i][j] = (int)kOutside;
+    }
+  };
+  // one of a unit's eight channels at a time, in place: the six inputs of xr become the six elements of the tile
+  auto transform_channel = [&](auto i_c, auto e_c) {
+    constexpr int i = decltype(i_c)::value, word = decltype(e_c)::value / 2, e = decltype(e_c)::value % 2;
+    Pack<T, 2> x[6];
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+      const unsigned two = xr[i][j][word];
+      x[j] = __builtin_bit_cast(Pack<T, 2>, two);
+    }
+    float d[6];
+#pragma unroll
+    for (int j = 0; j < 6; ++j) d[j] = static_cast<float>(x[j].v[e]);
+    const float ea = __builtin_fmaf(-kB2, d[2], d[4]), oa = __builtin_fmaf(-kB2, d[1], d[3]);
+    const float eb = __builtin_fmaf(-kA2, d[2], d[4]), ob = __builtin_fmaf(-kA2, d[1], d[3]);
+    const float e0 = __builtin_fmaf(-kS, d[2], d[4]), o0 = __builtin_fmaf(-kS, d[3], d[5]);
+    x[0].v[e] = plus(x[0].v[e], e0);
+    x[5].v[e] = plus(x[1].v[e], o0);
+    x[1].v[e] = static_cast<T>(__builtin_fmaf(kA, oa, ea));
+    x[2].v[e] = static_cast<T>(__builtin_fmaf(-kA, oa, ea));
+    x[3].v[e] = static_cast<T>(__builtin_fmaf(kB, ob, eb));
+    x[4].v[e] = static_cast<T>(__builtin_fmaf(-kB, ob, eb));
+#pragma unroll
+    for (int t = 0; t < 6; ++t) xr[i][t][word] = __builtin_bit_cast(unsigned, x[t]);
+  };
+  const int vst = v_offset(tid >> 2, tid & 3);       // THREADS / 4 rows further on, the chunk has the same position
+  auto store_v = [&](int i, int t, int buf) {
+    *reinterpret_cast<u32x4*>(lds + buf * BUF + vst + i * (THREADS / 4) * kRowPitch + t * TS) = xr[i][t];
+  };
+
+  auto tile_of = [&](int i, int& iw, int& ih, int& id, int& in) {
+    const int q1 = fast_div(i, a.f_bw), q2 = fast_div(q1, a.f_bh);
+    iw = i - q1 * a.bw; ih = q1 - q2 * a.bh;
+    in = fast_div(q2, a.f_bd); id = q2 - in * a.bd;
+  };
+
+  // ---- LDS address of this lane's tile in each 32-tile block
+  int vo[TB];            // in rows
+#pragma unroll
+  for (int b = 0; b < TB; ++b) {
+    int i = b * 32 + (lane & 31);
+    if (i >= a.bn * a.bd * a.bh * a.bw) i = 0;
+    int iw, ih, id, in;
+    tile_of(i, iw, ih, id, in);
+    vo[b] = in * a.irow + id * a.prow + ih * a.bw + iw;
+  }
+
+  f32x16 acc[3][TB];
+#pragma unroll
+  for (int t = 0; t < 3; ++t)
+#pragma unroll
+    for (int b = 0; b < TB; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[t][b][e] = 0.f;
+
+  cut_x(0);
+#pragma unroll
+  for (int i = 0; i < UN; ++i)
+#pragma unroll
+    for (int j = 0; j < 6; ++j) load_x(i, j, 0);
+  cut_x(1);
+  // Loads return in order and the compiler counts them over both ways into the loop: the order of the loads here is that of
+  // a step, the input of step 1 ahead of the filter's later groups, or every step would wait for its last loads.
+  auto load_u_groups = [&](int from, int to) {
+#pragma unroll
+    for (int i = from; i < to; ++i) load_u(i / 3, i / 3, i % 3);
+  };
+  load_u_groups(0, UD * 3 / 2);
+  static_for<0, 8 * UN>([&](auto h_c) { transform_channel(ic<decltype(h_c)::value / 8>{}, ic<decltype(h_c)::value % 8>{}); });
+#pragma unroll
+  for (int i = 0; i < UN; ++i) {
+#pragma unroll
+    for (int t = 0; t < 6; ++t) store_v(i, t, 0);
+#pragma unroll
+    for (int j = 0; j < 6; ++j) load_x(i, j, 1);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  load_u_groups(UD * 3 / 2, UD * 3 - 1);           // the last one: in item 0
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+
+  for (int step = 0; step < a.local_steps; ++step) {
+    const int cur = (step & 1) * BUF + tg * 3 * TS;
+    if constexpr (R > 3) {               // keeps the compiler from holding the addresses of all taps in registers
+#pragma unroll
+      for (int b = 0; b < TB; ++b) asm volatile("" : "+v"(vo[b]));
+    }
+    cut_x(step + 2);
+    u32x4 vf[VD][TB];
+    auto load_v = [&](int item) {                  // element item % 3 of group item / 3
+      const int q = item / 3, r = q >> 1, off = (r / KH) * a.prow + r % KH * a.bw;
+#pragma unroll
+      for (int b = 0; b < TB; ++b)
+        vf[item % VD][b] = *reinterpret_cast<const u32x4*>(lds + cur + v_offset(vo[b] + off, (lane >> 5) + (q & 1) * 2) + item % 3 * TS);
+    };
+    // A step is a stream of items, one element of one group each.  The loads that refill the rings, the transform of the
+    // next step's input, its stores to LDS and the loads of the step after are dealt out over the items and, in an item,
+    // over its MFMAs: a wavefront issues in order, and what stands between two MFMAs beyond the 32 cycles of the first
+    // leaves the matrix core idle.
+#pragma unroll
+    for (int i = 0; i < VD - 1; ++i) load_v(i);
+    static_for<0, NI>([&](auto item_c) {
+      constexpr int item = decltype(item_c)::value, q = item / 3, t = item % 3, last = (item + NI - 1) % NI;
+      constexpr int channels = RowItems<UN, NI>::channels(item), moves = RowItems<UN, NI>::moves(item);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (item + VD - 1 < NI) load_v(item + VD - 1);
+#pragma unroll
+      for (int b = 0; b < TB; ++b)
+        acc[t][b] = MfmaRow<T>::run(__builtin_bit_cast(Frag, uf[q % UD][t]), __builtin_bit_cast(Frag, vf[item % VD][b]), acc[t][b]);
+      // the ring slot of the item before: its fragment of UD groups later
+      load_u(last / 3 % UD, step * Q + last / 3 + UD - (item == 0 ? Q : 0), last % 3);
+      static_for<0, channels>([&](auto n_c) {
+        constexpr int h = RowItems<UN, NI>::first_channel(item) + decltype(n_c)::value;
+        transform_channel(ic<h / 8>{}, ic<h % 8>{});
+      });
+      static_for<0, moves>([&](auto n_c) {
+        constexpr int v = RowItems<UN, NI>::first_move(item) + decltype(n_c)::value;
+        store_v(v / 6, v % 6, (step + 1) & 1);
+        load_x(v / 6, v % 6, step + 2);
+      });
+      __builtin_amdgcn_sched_group_barrier(0x100, TB, 0);
+#pragma unroll
+      for (int g = 0; g < TB; ++g) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, (14 * channels + 3 + TB - 1) / TB, 0);
+        __builtin_amdgcn_sched_group_barrier(0x200, (moves + TB - 1) / TB, 0);
+        __builtin_amdgcn_sched_group_barrier(0x20, (moves + TB) / TB, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+  }
+
+  if constexpr (CS > 1) {                // the shares' sums come together in the first share's registers
+    f32x4* part = reinterpret_cast<f32x4*>(lds_all) + lane;
+    constexpr int NV = 3 * TB * 4;
+    if (cs > 0) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        const f32x16& c = acc[v / 4 % 3][v / 12];
+        f32x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = c[v % 4 * 4 + e];
+        part[(((cs - 1) * 2 * KG + wave) * NV + v) * 64] = o;
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    if (cs == 0) {
+#pragma unroll
+      for (int o = 0; o < CS - 1; ++o)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+          const f32x4 p = part[((o * 2 * KG + wave) * NV + v) * 64];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[v / 4 % 3][v / 12][v % 4 * 4 + e] += p[e];
+        }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    if (cs > 0) {                        // the barrier of the output transform below
+      __builtin_amdgcn_s_barrier();
+      return;
+    }
+  }
+
+  // ---- output transform.  Elements 0 to 2 (points 0, a, -a) are with the first half of the wavefronts, 3 to 5 (1/a,
+  // -1/a, infinity) with the second; each half finishes one half of the outputs (two blocks: a block each; one block: half
+  // of its channels each) and hands three sums of the other half over through LDS.
+  // Each wavefront reduces its three elements to (x, s, d): the element at 0 or infinity, and sum and difference of the pair.
+  constexpr int NC = TB;              // chunks of 8 accumulator registers a wavefront finishes
+  auto finish = [&](auto tg_c) {
+    constexpr int TG = decltype(tg_c)::value, X = TG == 0 ? 0 : 2, P0 = TG == 0 ? 1 : 0;
+    // chunk c of a half: tile block, first register
+    auto tile_block = [](int half, int c) { return (half * TB + c) / 2; };
+    auto first = [](int half, int c) { return (half * TB + c) % 2 * 8; };
+    auto reg = [&](int t, int half, int c, int e) -> float { return acc[t][tile_block(half, c)][first(half, c) + e]; };
+    f32x4* ex = reinterpret_cast<f32x4*>(lds) + (size_t)(TG * KG + kg) * 6 * NC * 64 + lane;
+    const f32x4* other = reinterpret_cast<const f32x4*>(lds) + (size_t)((1 - TG) * KG + kg) * 6 * NC * 64 + lane;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int i4 = 0; i4 < 2; ++i4) {
+        f32x4 x, s, d;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float p = reg(P0, 1 - TG, c, i4 * 4 + e), m = reg(P0 + 1, 1 - TG, c, i4 * 4 + e);
+          x[e] = reg(X, 1 - TG, c, i4 * 4 + e); s[e] = p + m; d[e] = p - m;
+        }
+        ex[((c * 2 + i4) * 3 + 0) * 64] = x; ex[((c * 2 + i4) * 3 + 1) * 64] = s; ex[((c * 2 + i4) * 3 + 2) * 64] = d;
+      }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int k0 = (kb * KG + kg) * 32 + (lane >> 5) * 16 + first(TG, c);
+      const int ti = tile_block(TG, c) * 32 + (lane & 31);
+      int iw, ih, id, in;
+      tile_of(ti, iw, ih, id, in);
+      const int n = n0 + in, od = d0 + id, oh = h0 + ih, ow = (w0 + iw) * 4;
+      const bool ok = ti < a.bn * a.bd * a.bh * a.bw && n < a.N && od < a.oD && oh < a.oH && k0 < a.K;
+      T* const yp = static_cast<T*>(a.y) + ((((size_t)n * a.oD + od) * a.oH + oh) * a.oW + ow) * a.K + k0;
+      const T* const bp = static_cast<const T*>(a.bias);
+      Pack<T, 8> bv, o[4];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) bv.v[e] = T(0);
+      if (bp) {
+        if constexpr (!KT) {
+          __builtin_memcpy(&bv, bp + min(k0, a.K - 8), 16);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) bv.v[e] = bp[min(k0 + e, a.K - 1)];
+        }
+      }
+#pragma unroll
+      for (int i4 = 0; i4 < 2; ++i4) {
+        f32x4 g[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) g[j] = other[((c * 2 + i4) * 3 + j) * 64];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int i = i4 * 4 + e;
+          const float p = reg(P0, TG, c, i), m = reg(P0 + 1, TG, c, i), x = reg(X, TG, c, i), b = static_cast<float>(bv.v[i]);
+          const float m0 = TG == 0 ? x : g[0][e], mi = TG == 0 ? g[0][e] : x;
+          const float sa = TG == 0 ? p + m : g[1][e], sb = TG == 0 ? g[1][e] : p + m;
+          const float da = TG == 0 ? p - m : g[2][e], db = TG == 0 ? g[2][e] : p - m;
+          o[0].v[i] = static_cast<T>(m0 + sa + sb + b);
+          o[1].v[i] = static_cast<T>(__builtin_fmaf(kA, da, __builtin_fmaf(kB, db, b)));
+          o[2].v[i] = static_cast<T>(__builtin_fmaf(kA2, sa, __builtin_fmaf(kB2, sb, b)));
+          o[3].v[i] = static_cast<T>(__builtin_fmaf(kA * kA2, da, __builtin_fmaf(kB * kB2, db, mi + b)));
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        T* const dst = yp + (size_t)i * a.K;
+        const bool in_row = ok && ow + i < a.oW;
+        if constexpr (!KT) {
+          if (in_row) *reinterpret_cast<u32x4*>(dst) = __builtin_bit_cast(u32x4, o[i]);
+        } else {
+          if (in_row && k0 + 8 <= a.K) {
+            __builtin_memcpy(dst, &o[i], 16);          // rows of y start at any multiple of the element size
+          } else if (in_row) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              if (k0 + e < a.K) dst[e] = o[i].v[e];
+          }
+        }
+      }
+    }
+  };
+  if (tg == 0) finish(ic<0>{});
+  else finish(ic<1>{});
+}
+
+// ---- U[k / 32][channel block][row tap][half][element][lane][8]: the order in which the wavefronts read it.  Lane l holds
+// row l % 32 of a 32 x 16 fragment, channels 8 (l / 32) .. + 8 of the half; row 8 i + 4 h + j of a block is output channel
+// 16 h + 4 i + j, which puts 16 consecutive channels of a tile into the accumulators of a lane.
+struct RowFilterArgs {
+  const void* w; void* U;
+  long long s[5];
+  int K, C, kd, kh, steps;
+  long long total;
+};
+
+template <typename T>
+__global__ __launch_bounds__(256) void row_filter_kernel(RowFilterArgs a) {
+  const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (idx >= a.total) return;
+  const int R = a.kd * a.kh;
+  const int e2 = (int)(idx & 3) * 2;
+  const int lane = (int)(idx >> 2) & 63;
+  long long q = idx >> 8;
+  const int half = (int)(q & 1); q >>= 1;
+  const int r = (int)(q % R); q /= R;
+  const int step = (int)(q % a.steps);
+  const int kb = (int)(q / a.steps);
+  const int m = lane & 31;
+  const int k = kb * 32 + ((m >> 2) & 1) * 16 + (m >> 3) * 4 + (m & 3);
+  const int c = step * 32 + half * 16 + (lane >> 5) * 8 + e2;
+  const int rd = r / a.kh, rh = r - rd * a.kh;
+  Pack<T, 2> out[6];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    float g[3] = {0.f, 0.f, 0.f};
+    if (k < a.K && c + e < a.C) {
+      const T* p = static_cast<const T*>(a.w) + k * a.s[0] + (c + e) * a.s[1] + rd * a.s[2] + rh * a.s[3];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) g[j] = static_cast<float>(p[j * a.s[4]]);
+    }
+    // denominators: prod over the other points; 1 for 0 (a^2 b^2), 2 a^2 (a^2 - b^2) for +-a, 2 b^2 (b^2 - a^2) for +-b
+    const float fa = 1.f / (2.f * kA2 * (kA2 - kB2)), fb = 1.f / (2.f * kB2 * (kB2 - kA2));
+    const float ea = __builtin_fmaf(kA2, g[2], g[0]), oa = kA * g[1];
+    const float eb = __builtin_fmaf(kB2, g[2], g[0]), ob = kB * g[1];
+    out[0].v[e] = static_cast<T>(g[0]);
+    out[1].v[e] = static_cast<T>((ea + oa) * fa);
+    out[2].v[e] = static_cast<T>((ea - oa) * fa);
+    out[3].v[e] = static_cast<T>((eb + ob) * fb);
+    out[4].v[e] = static_cast<T>((eb - ob) * fb);
+    out[5].v[e] = static_cast<T>(g[2]);
+  }
+  T* dst = static_cast<T*>(a.U) + ((idx >> 8) * 6) * 512 + lane * 8 + e2;
+#pragma unroll
+  for (int t = 0; t < 6; ++t) *reinterpret_cast<Pack<T, 2>*>(dst + t * 512) = out[t];
+}
+
+// Box of a workgroup: at most `tiles` tiles whose input rows, with the halo of the taps, fill at most `slots` rows of LDS;
+// the fewest boxes over the output, and among those the fewest rows.  Fragment reads take the tiles of a box in order, which
+// is free of bank conflicts where their rows are consecutive: planes and images are padded to row counts that continue the
+// count of their tiles modulo 16 (the period of v_offset) across the halo.
+struct RowBox { int bn, bd, bh, bw, n_n, n_d, n_h, n_w, prow, irow; long long boxes; };
+RowBox choose_box(int N, int oD, int oH, int nW, int kd, int kh, int tiles, int slots) {
+  RowBox best{};
+  long long best_rows = 0;
+  auto padded = [](int rows, int like) { return rows + ((like - rows) & 7); };
+  for (int bw = 1; bw <= tiles && bw <= nW; ++bw)
+    for (int bd = 1; bd * bw <= tiles && bd <= oD; ++bd)
+      for (int bh = 1; bh * bd * bw <= tiles && bh <= oH; ++bh) {
+        RowBox b;
+        const int plane = bw * (bh + kh - 1);
+        b.prow = bd > 1 ? padded(plane, bw * bh) : plane;
+        const int image = (bd + kd - 2) * b.prow + plane, image_p = padded(image, bd * bh * bw);
+        if (image > slots) break;
+        const int bn = std::min(std::min(tiles / (bw * bd * bh), (slots - image) / image_p + 1), N);
+        b.irow = image_p;
+        b.bn = bn; b.bd = bd; b.bh = bh; b.bw = bw;
+        b.n_n = ceil_div(N, bn); b.n_d = ceil_div(oD, bd); b.n_h = ceil_div(oH, bh); b.n_w = ceil_div(nW, bw);
+        b.boxes = (long long)b.n_n * b.n_d * b.n_h * b.n_w;
+        const long long rows = b.boxes * (image * bn * 16 - bw);      // wide boxes: neighbouring tiles share two of their six pixels
+        if (!best.boxes || b.boxes < best.boxes || (b.boxes == best.boxes && rows < best_rows)) { best = b; best_rows = rows; }
+      }
+  return best;
+}
+
+// The shapes of workgroup, by what fills the chip.  Measured, fp16, us (wide | half | small | split):
+//   wide   eight wavefronts, 64 tiles x 128 channels, one workgroup per CU: every byte of V is used for 128 channels
+//   half   four, 64 tiles x 64 channels, two per CU: the transform of one runs beside the products of the other, finer rounds
+//   small  four, 32 tiles x 64 channels: more workgroups, shorter steps
+//   split  eight, 32 tiles x 32 channels, the channel blocks shared out over four pairs of wavefronts
+// N=64: 256 -> 256 channels, 56x56 188 | 190 | 231, 14x14 22 | 17 | 20; 128 -> 128, 28x28 17.2 | 18.0 | 22.5, 56x56
+// 68 | 60 | 74; N=16, 256 -> 256, 14x14 21 | 15 | 12.4 | 10.6; N=1, 512 -> 512, 7x7 33 | 22 | 19 | 12.
+enum RowShape { kRowWide, kRowHalf, kRowSmall, kRowSplit };
+struct RowPlan { RowShape shape; RowBox box; long long wide_groups; };
+
+RowPlan make_row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int steps) {
+  RowPlan p;
+  const RowBox wide = choose_box(N, oD, oH, nW, kd, kh, 64, 128), half = kd == 1 ? choose_box(N, oD, oH, nW, kd, kh, 64, 64) : wide;
+  const long long n_wide = wide.boxes * ceil_div(K, 128), n_half = half.boxes * ceil_div(K, 64);
+  p.wide_groups = n_wide;
+  const RowBox small = choose_box(N, oD, oH, nW, kd, kh, 32, 64);
+  if (steps >= 4) {
+    const RowBox split = choose_box(N, oD, oH, nW, kd, kh, 32, 32);
+    if (split.boxes * ceil_div(K, 32) <= kCus) { p.shape = kRowSplit; p.box = split; return p; }
+  }
+  if (small.boxes * ceil_div(K, 64) <= kCus) { p.shape = kRowSmall; p.box = small; return p; }
+  // rounds of the chip; of two workgroups per CU one starts as soon as another ends, so their last round is not a whole one.
+  // 3-D boxes of the half shape take two units of input per thread
+  const double t_wide = n_wide <= kCus ? 0.86 : 0.92 * (double)((n_wide + kCus - 1) / kCus), t_half = (kd == 1 ? 1.0 : 1.2) * (n_half / (2.0 * kCus) + 0.12);
+  p.shape = t_wide <= t_half ? kRowWide : kRowHalf;
+  p.box = p.shape == kRowWide ? wide : half;
+  return p;
+}
+
+// The search over boxes takes some microseconds: the last plans of a host thread are kept.
+RowPlan row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int steps) {
+  struct Entry { int key[8]; RowPlan plan; };
+  thread_local Entry cache[64] = {};
+  const int key[8] = {N, oD, oH, nW, kd, kh, K, steps};
+  unsigned h = 2166136261u;
+  for (int v : key) h = (h ^ (unsigned)v) * 16777619u;
+  Entry& e = cache[(h ^ (h >> 15)) % 64];
+  if (!std::equal(key, key + 8, e.key)) {
+    e.plan = make_row_plan(N, oD, oH, nW, kd, kh, K, steps);
+    std::copy(key, key + 8, e.key);
+  }
+  return e.plan;
+}
+
+template <typename T, int KD, int KH, int KG, int TB, int S, int CS = 1>
+int launch_row(const RowArgs& args, const RowBox& b, void* stream) {
+  RowArgs a = args;
+  a.bn = b.bn; a.bd = b.bd; a.bh = b.bh; a.bw = b.bw; a.prow = b.prow; a.irow = b.irow;
+  a.f_bw = make_fast_div(b.bw); a.f_bh = make_fast_div(b.bh); a.f_bd = make_fast_div(b.bd);
+  a.f_prow = make_fast_div(b.prow); a.f_irow = make_fast_div(b.irow);
+  a.n_d = b.n_d; a.n_h = b.n_h; a.n_w = b.n_w;
+  a.n_box = (int)b.boxes;
+  a.local_steps = ceil_div(a.steps, CS);
+  a.n_kb = ceil_div(a.K, 32 * KG);
+  // filters that overflow an XCD's 4 MB of L2: its workgroups work on one channel block at a time
+  a.box_fast = a.u_bytes > (3 << 20);
+  a.per_xcd = ceil_div(a.n_kb * a.n_box, kXcds);
+  constexpr int bytes = row_lds_bytes<KG, TB, S, CS>();
+  const bool whole = a.K % 8 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
+  auto fn = whole ? row_conv_kernel<T, KD, KH, KG, TB, S, CS, false> : row_conv_kernel<T, KD, KH, KG, TB, S, CS, true>;
+  int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), bytes);
+  if (rc) return rc;
+  hipLaunchKernelGGL(fn, dim3(a.per_xcd * kXcds), dim3(128 * KG * CS), bytes, as_stream(stream), a);
+  WC_CHECK_LAUNCH("row_conv_kernel");
+  return WC_OK;
+}
+
+}  // namespace
+
+bool row_conv_fits(const wc_conv_desc* d) {
+  if (d->dtype == WC_F32 || d->stride != 1 || d->whole_kernel || d->kernel[2] != 3) return false;
+  const int kd = d->kernel[0], kh = d->kernel[1];
+  if (!((kd == 1 && kh == 3) || (kd == 3 && kh == 3))) return false;
+  const int cp = wc_padded_channels8(d->C);
+  for (int q = 0; q < 3; ++q)
+    if (d->in[q] + 2 * d->pad[q] < d->kernel[q]) return false;
+  const long long out = (long long)d->N * (d->in[0] + 2 * d->pad[0] - kd + 1) * (d->in[1] + 2 * d->pad[1] - kh + 1) *
+                        (d->in[2] + 2 * d->pad[2] - 2);
+  return (long long)d->N * d->in[0] * d->in[1] * d->in[2] * cp * 2 < (1ll << 30) && out < (1ll << 31) &&
+         row_u_elems(d) * 2 < (1ull << 30);
+}
+
+size_t row_u_elems(const wc_conv_desc* d) {
+  return (size_t)ceil_div(d->K, 32) * ceil_div(d->C, 32) * d->kernel[0] * d->kernel[1] * 2 * 6 * 512;
+}
+
+int row_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5], void* U, void* stream) {
+  WC_CHECK_ARG(w && w_strides && U, "row form filter: null pointer");
+  RowFilterArgs a;
+  a.w = w; a.U = U;
+  for (int i = 0; i < 5; ++i) a.s[i] = w_strides[i];
+  a.K = d->K; a.C = d->C; a.kd = d->kernel[0]; a.kh = d->kernel[1]; a.steps = ceil_div(d->C, 32);
+  a.total = (long long)ceil_div(d->K, 32) * a.steps * a.kd * a.kh * 2 * 256;
+  const unsigned blocks = (unsigned)ceil_div_ll(a.total, 256);
+  if (d->dtype == WC_F16) hipLaunchKernelGGL(row_filter_kernel<half_t>, dim3(blocks), dim3(256), 0, as_stream(stream), a);
+  else hipLaunchKernelGGL(row_filter_kernel<bf16_t>, dim3(blocks), dim3(256), 0, as_stream(stream), a);
+  WC_CHECK_LAUNCH("row_filter_kernel");
+  return WC_OK;
+}
+
+// Against the other forms, fp16, us (row | other), channels -> channels on P output pixels:
+//  * 3-D: always (8x28x28 to 16x56x56, 32 to 128 channels: 1.3 to 3 times faster).
+//  * 2-D with V and M in memory: F(4x4, 3x3) needs half the products, so it overtakes on large problems with many
+//    channels.  Per pixel it takes about 1500 (C + K) + C K units, the row form 10.5 of them per product of padded channels:
+//    256 -> 256 on 200704 pixels 188 | 219, 384 on 50176 108 | 111, 512 on 50176 178 | 140, 300 -> 200 76 | 67.  Up to one and a
+//    half rounds of the chip the row form's single launch decides (512 on 12544: 47 | 54; 256 on 12544: 17 | 30; 512 on 49: 12 | 17).
+//    Tile 2 (bfloat16) needs 4/9 more products than F(4x4, 3x3) saves: never ahead.
+//  * Layers with the one-kernel F(2x2, 3x3) form (conv_thin.hip), tile 2: that form up to 32 channels; up to 64 outside 2.4
+//    to 8 million output values (64 -> 64 on 50176 pixels 9.1 | 11.6, on 200704 25 | 23, on 12544 6.8 | 6.3); up to 128 below
+//    1.2 million (128 -> 128 on 3136 pixels 8.1 | 6.7, on 12544 8.8 | 11.3, on 50176 17 | 25).
+bool row_preferred(const wc_conv_desc* d) {
+  if (d->kernel[0] > 1) return true;
+  const int oD = 1, oH = d->in[1] + 2 * d->pad[1] - 2, oW = d->in[2] + 2 * d->pad[2] - 2;
+  const long long P = (long long)d->N * oH * oW, outputs = P * d->K;
+  wc_plan plan;
+  wc_conv_desc e = *d;
+  e.stacked = 0; e.direct = 0; e.row = 0;
+  if (wc_plan_conv(&e, &plan) == WC_OK && thin_conv_fits(&e, &plan)) {
+    const int cp = wc_padded_channels(d->C);
+    if (cp <= 32) return false;
+    return cp <= 64 ? outputs >= 2400000 && outputs <= 8000000 : outputs >= 1200000;
+  }
+  if (d->m != 4 || d->dtype != WC_F16) return true;
+  if (row_plan(d->N, oD, oH, ceil_div(oW, 4), 1, 3, d->K, ceil_div(d->C, 32)).wide_groups <= 3 * kCus / 2) return true;
+  const double C = d->C, K = d->K, Cp = wc_padded_channels(d->C), Kp = ceil_div(d->K, 64) * 64.0;
+  return 10.5 * Cp * Kp < 1500.0 * (C + K) + C * K;
+}
+
+// x (N, D, H, W, Cx) channel-last with Cx = C rounded up to 8 (zeros beyond C), 16-byte aligned
+int row_conv(const wc_conv_desc* d, const void* x, int n_images, const void* U, const void* bias, void* y, void* stream) {
+  WC_CHECK_ARG(row_conv_fits(d), "row form: 16-bit, stride 1, kernel rows of three taps");
+  WC_CHECK_ARG(((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(U)) & 15) == 0, "row form: x and U must be 16-byte aligned");
+  RowArgs a{};
+  a.x = x; a.U = U; a.bias = bias; a.y = y;
+  a.N = n_images; a.D = d->in[0]; a.H = d->in[1]; a.W = d->in[2]; a.C = wc_padded_channels8(d->C); a.K = d->K;
+  a.pd = d->pad[0]; a.ph = d->pad[1]; a.pw = d->pad[2];
+  a.oD = a.D + 2 * a.pd - d->kernel[0] + 1; a.oH = a.H + 2 * a.ph - d->kernel[1] + 1; a.oW = a.W + 2 * a.pw - 2;
+  a.nW = ceil_div(a.oW, 4);
+  a.steps = ceil_div(a.C, 32);
+  a.x_bytes = (int)((long long)a.N * a.D * a.H * a.W * a.C * 2);
+  a.u_bytes = (int)(row_u_elems(d) * 2);
+  const int force = test_gemm_config();
+  return dispatch_dtype(d->dtype, [&](auto t) -> int {
+    using T = decltype(t);
+    if constexpr (sizeof(T) == 2) {
+      auto go = [&](auto kd, auto kh) -> int {
+        constexpr int KD = decltype(kd)::value, KH = decltype(kh)::value;
+        RowPlan p = row_plan(a.N, a.oD, a.oH, a.nW, KD, KH, a.K, a.steps);
+        if (force >= 16 && force <= 19) {
+          p.shape = (RowShape)(force - 16);
+          const int tiles = p.shape <= kRowHalf ? 64 : 32, slots = p.shape == kRowWide ? 128 : p.shape == kRowSplit ? 32 : p.shape == kRowHalf && KD > 1 ? 128 : 64;
+          p.box = choose_box(a.N, a.oD, a.oH, a.nW, KD, KH, tiles, slots);
+        }
+        switch (p.shape) {
+          case kRowWide: return launch_row<T, KD, KH, 4, 2, 128>(a, p.box, stream);
+          case kRowHalf: return launch_row<T, KD, KH, 2, 2, KD == 1 ? 64 : 128>(a, p.box, stream);
+          case kRowSmall: return launch_row<T, KD, KH, 2, 1, 64>(a, p.box, stream);
+          default: return launch_row<T, KD, KH, 1, 1, 32, 4>(a, p.box, stream);
+        }
+      };
+      if (d->kernel[0] == 1) return go(ic<1>{}, ic<3>{});
+      return go(ic<3>{}, ic<3>{});
+    }
+    return fail(WC_ERR_UNSUPPORTED, "row form: 16-bit types");
+  });
+}
+
+}  // namespace wc

@@ -160,6 +160,10 @@ extern "C" int wc_filter_transform(const wc_conv_desc* d, const wc_plan* plan, c
     if (!direct_conv_fits(d)) return fail(WC_ERR_UNSUPPORTED, "wc_filter_transform: problem outside the direct form's range");
     return direct_filter(d, w, w_strides, U, stream);
   }
+  if (d->row == 1) {
+    if (!row_conv_fits(d)) return fail(WC_ERR_UNSUPPORTED, "wc_filter_transform: problem outside the row form's range");
+    return row_filter(d, w, w_strides, U, stream);
+  }
   int out[3], grid[3];
   int rc = wc_conv_out_dims(d, out, grid);   // validates the descriptor
   if (rc) return rc;

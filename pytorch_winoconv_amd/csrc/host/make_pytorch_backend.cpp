@@ -315,7 +315,7 @@ std::vector<int> ints_of(py::object v, int nd, const char* what) {
 // of the reference end in the same call).
 at::Tensor conv_forward(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bias, py::object stride, py::object padding,
                         int m, std::optional<at::Tensor> U, int chunk_images, bool whole_kernel, py::object stacked,
-                        bool unfused, bool channels_first_out, py::object direct) {
+                        bool unfused, bool channels_first_out, py::object direct, bool row) {
   const int nd = (int)x.dim() - 2;
   if ((nd != 2 && nd != 3) || w.dim() != nd + 2)
     throw std::invalid_argument("expected 4-D or 5-D input and matching filter, got " + shape_str(x.sizes()) + " and " + shape_str(w.sizes()));
@@ -366,6 +366,8 @@ at::Tensor conv_forward(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bi
   d.whole_kernel = whole_kernel;
   d.stacked = stacked.is_none() ? -1 : (py::isinstance<py::bool_>(stacked) ? (int)stacked.cast<bool>() : stacked.cast<int>());
   d.direct = direct.is_none() ? 0 : (direct.cast<bool>() ? 1 : -1);      // None: the library may choose it
+  d.unfused = unfused;
+  d.row = row && !unfused ? -1 : 0;                                       // -1: the library may choose it
   check(wc_conv_auto(&d));
   int out[3], grid[3];
   check(wc_conv_out_dims(&d, out, grid));
@@ -386,6 +388,10 @@ at::Tensor conv_forward(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bi
   }
   d.y_layout = channels_first_out;
   auto misaligned = [](const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) != 0; };
+  if (d.row) {                                             // the row form reads aligned operands: copies of those that are not
+    if (misaligned(x_mem)) x_mem = x_mem.clone();
+    if (U && U->defined() && misaligned(*U)) U = U->clone();
+  }
   d.unfused = unfused || misaligned(x_mem) || (U && U->defined() && misaligned(*U));
   if (U && U->defined()) {
     size_t ue = 0;
@@ -445,6 +451,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("conv_forward", &conv_forward, py::arg("x"), py::arg("w"), py::arg("bias") = py::none(), py::arg("stride") = 1,
         py::arg("padding") = 0, py::arg("m") = 2, py::arg("U") = py::none(), py::arg("chunk_images") = 0,
         py::arg("whole_kernel") = false, py::arg("stacked") = py::none(), py::arg("unfused") = false,
-        py::arg("channels_first_out") = false, py::arg("direct") = py::none());
+        py::arg("channels_first_out") = false, py::arg("direct") = py::none(), py::arg("row") = false);
   m.def("version", []() { return std::string(wc_version()); });
 }

@@ -108,7 +108,7 @@ using namespace wc;
 extern "C" {
 
 int wc_test_gemm_override(int config, int rows_mode) {
-  WC_CHECK_ARG(config >= -1 && config < 16 && rows_mode >= 0 && rows_mode <= 4,
+  WC_CHECK_ARG(config >= -1 && config < 20 && rows_mode >= 0 && rows_mode <= 4,
                "wc_test_gemm_override: config %d, rows_mode %d", config, rows_mode);
   if (!test_hooks_enabled())
     return fail(WC_ERR_UNSUPPORTED, "wc_test_gemm_override: test hooks are off (set WINOCONV_TEST_HOOKS=1 before the first call)");
@@ -177,6 +177,7 @@ static int check_desc(const wc_conv_desc* d) {
   WC_CHECK_ARG(d->whole_kernel == 0 || d->whole_kernel == 1, "whole_kernel must be 0 or 1");
   WC_CHECK_ARG(d->stacked >= 0 && d->stacked <= 2, "stacked must be 0, 1 or 2");
   WC_CHECK_ARG(d->direct == 0 || d->direct == 1, "direct must be 0 or 1");
+  WC_CHECK_ARG(d->row == 0 || d->row == 1, "row must be 0 or 1");
   WC_CHECK_ARG((d->x_layout == 0 || d->x_layout == 1) && (d->y_layout == 0 || d->y_layout == 1),
                "x_layout and y_layout must be 0 (channel-last) or 1 (channel-first)");
   if (d->stacked && (d->whole_kernel || (d->ndim == 3 && d->m != 2)))
@@ -401,11 +402,15 @@ int wc_conv_auto(wc_conv_desc* d) {
   WC_CHECK_ARG(d->ndim == 2 || d->ndim == 3, "ndim must be 2 or 3, got %d", d->ndim);
   WC_CHECK_ARG(d->stacked >= -1 && d->stacked <= 2, "stacked must be -1 (choose), 0, 1 or 2");
   WC_CHECK_ARG(d->direct >= -1 && d->direct <= 1, "direct must be -1 (never), 0 (may be chosen) or 1");
+  WC_CHECK_ARG(d->row >= -1 && d->row <= 1, "row must be -1 (may be chosen), 0 or 1");
+  const bool may_row = d->row == -1;
+  if (may_row) d->row = 0;
   const bool never_direct = d->direct == -1;
   if (never_direct) d->direct = 0;
   if (d->stacked == -1) {
     if (!d->direct && !never_direct && direct_conv_fits(d) && direct_preferred(d)) d->direct = 1;
-    d->stacked = d->direct ? 0 : auto_stacked(d);
+    if (may_row && !d->direct && !d->unfused && row_conv_fits(d) && row_preferred(d)) d->row = 1;
+    d->stacked = d->direct || d->row ? 0 : auto_stacked(d);
   }
   if (d->stacked == 2 && d->m == 4) {
     // the shared-input plan exists for output tiles 2 and 3: tile 3 (F(3,3): fp16 error 3e-3 of the output

@@ -143,6 +143,8 @@ bool input_transform_nchw_fits(const wc_conv_desc* d, const wc_plan* plan);
 int input_transform_nchw(const wc_conv_desc* d, const wc_plan* plan, const void* x, int n_images, void* V, void* stream);
 // src (n, R, Q) -> dst (n, Q, R), elements of 2 or 4 bytes (layout_copy.hip)
 int transpose_images(const void* src, void* dst, long long n, long long R, long long Q, int elem_size, void* stream);
+// 16-bit x of n images, channel-first (n, C, S) or channel-last (n, S, C), to channel-last (n, S, Cx), zeros beyond C
+int pad_channels(const void* src, void* dst, long long n, int C, int Cx, long long S, bool channel_first, void* stream);
 
 // Direct form (wc_conv_desc.direct; direct_conv.hip, gemm.hip): whether a problem is in its range, the copy of the
 // filter to U (K, kh, kw, C), and the product that reads x itself.
@@ -150,6 +152,13 @@ bool direct_conv_fits(const wc_conv_desc* d);
 int direct_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5], void* U, void* stream);
 int direct_conv(const wc_conv_desc* d, const void* x, int n_images, const void* U, const void* bias, void* y, void* stream);
 size_t direct_u_elems(const wc_conv_desc* d);     // elements of the direct form's U
+// Row form (wc_conv_desc.row; conv_row.hip): F(4,3) along the width axis, the other axes' taps in the reduction, one kernel.
+// Its U is row_u_elems(d) elements in the kernel's own order; x has its channels padded with zeros to a multiple of 8.
+bool row_conv_fits(const wc_conv_desc* d);
+bool row_preferred(const wc_conv_desc* d);        // where it measured faster than the other forms
+size_t row_u_elems(const wc_conv_desc* d);
+int row_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5], void* U, void* stream);
+int row_conv(const wc_conv_desc* d, const void* x, int n_images, const void* U, const void* bias, void* y, void* stream);
 // Strided first layers (direct_first.hip): at most 4 input channels, stride 2, kernels of 3, 5 or 7 rows and at most 8
 // columns, 16-bit types.  U is (K, kh, 8 taps, 4 channels), zero where the filter has no tap or channel.
 bool direct_first_fits(const wc_conv_desc* d);

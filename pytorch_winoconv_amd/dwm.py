@@ -28,7 +28,7 @@ def _dwm(input, kernel, bias, stride, padding, groups, nd, output_block=2):
     if bias is not None:
         bias = bias.type_as(input)                                   # dwm.py:18,36
     return engine.conv_forward(input, kernel.type_as(input), bias, _norm_stride(stride, nd), padding,
-                               int(output_block))
+                               int(output_block), row=True)
 
 
 def dwm3d(input, kernel, bias=None, stride=(1, 1, 1), padding=0, groups=1, output_block=2):

@@ -76,11 +76,12 @@ def _triple(v, nd, fill):
 
 
 def make_desc(x_shape, w_shape, dtype, stride=1, padding=0, m=2, chunk_images=0, whole_kernel=False, stacked=False,
-              unfused=False, x_layout=0, y_layout=0, direct=None):
+              unfused=False, x_layout=0, y_layout=0, direct=None, row=False):
     """Descriptor for an NC[D]HW input and a (K, C, [kD,] kH, kW) filter.  `whole_kernel`: one
     F(2,k) tile per axis for a k x k kernel, k = 4..7, instead of the DWM pieces.  `stacked`: the
     DWM pieces share one tile and are added by the batched GEMM instead of by the output transform
-    (2-D; same sum, fewer bytes moved for kernels above 3 x 3)."""
+    (2-D; same sum, fewer bytes moved for kernels above 3 x 3).  `row`: the library may choose the row form
+    (wc_conv_desc.row; only where `stacked` is None)."""
     nd = len(x_shape) - 2
     if nd not in (2, 3) or len(w_shape) != nd + 2:
         raise ValueError("expected 4-D or 5-D input and matching filter, got %r and %r"
@@ -107,6 +108,7 @@ def make_desc(x_shape, w_shape, dtype, stride=1, padding=0, m=2, chunk_images=0,
     # the direct form (wc_conv_desc.direct): True asks for it, False rules it out, None leaves it to the library,
     # which takes it for 16-bit stride-2 layers when `stacked` is left open too
     d.direct = 1 if direct else (-1 if direct is False else 0)
+    d.row = -1 if row and not unfused else 0
     # what is left open is filled in by the library: the form of the plan if `stacked` is None, and the tile
     # 3 or 2 where a caller asked for tile 4 and gets the shared-input plan, which has no such tile (d.m then
     # tells the tile really used)
@@ -124,13 +126,13 @@ def effective_tile(x_shape, w_shape, dtype, stride=1, padding=0, m=2, whole_kern
     return d.m, d.stacked
 
 
-def plan_form(x_shape, w_shape, dtype, stride=1, padding=0, m=2):
-    """(direct, stacked, tile) of the plan conv_forward runs for this problem with everything left to the library:
+def plan_form(x_shape, w_shape, dtype, stride=1, padding=0, m=2, row=False):
+    """(direct, stacked, tile) - with `row` (direct, stacked, tile, row) - of the plan conv_forward runs for this problem with everything left to the library:
     what a cached transformed filter depends on beside the filter itself (the library's choice between the
     Winograd pieces and the direct form looks at the batch size)."""
     pad = padding if isinstance(padding, int) else tuple(padding)
-    d = _forward_setup(tuple(x_shape), tuple(w_shape), dtype, stride, pad, m, 0, False, None)[0]
-    return int(d.direct), int(d.stacked), int(d.m)
+    d = _forward_setup(tuple(x_shape), tuple(w_shape), dtype, stride, pad, m, 0, False, None, row=row)[0]
+    return (int(d.direct), int(d.stacked), int(d.m)) + ((int(d.row),) if row else ())
 
 
 def plan_conv(desc):
@@ -324,10 +326,16 @@ def check_u(desc, U):
                          "(transform_filter must be called with the same options)" % (U.numel(), n.value))
 
 
-def transform_filter(w, x_shape, stride=1, padding=0, m=2, whole_kernel=False, stacked=None, direct=None):
+def transform_filter(w, x_shape, stride=1, padding=0, m=2, whole_kernel=False, stacked=None, direct=None, row=False):
     """Transformed filter U for later calls of conv_forward(..., U=U) with the same options."""
     _require_gpu(w)
-    desc = make_desc(x_shape, w.shape, w.dtype, stride, padding, m, 0, whole_kernel, stacked, direct=direct)
+    desc = make_desc(x_shape, w.shape, w.dtype, stride, padding, m, 0, whole_kernel, stacked, direct=direct, row=row)
+    if desc.row:
+        n = ctypes.c_size_t()
+        check(_lib.load().wc_conv_u_elems(ctypes.byref(desc), ctypes.byref(n)))
+        U = torch.empty(n.value, dtype=w.dtype, device=w.device)          # in the kernel's own order
+        check(_lib.load().wc_filter_transform(ctypes.byref(desc), ctypes.byref(Plan()), _ptr(w), _w_strides(w), _ptr(U), _stream(w)))
+        return U
     if desc.direct:
         # the filter with its taps outermost and channels innermost, (K, kH, kW, C); strided first layers (at most 4
         # channels) pad every kernel row to 8 taps of 4 channels, (K, kH, 8, 4)
@@ -346,36 +354,37 @@ def transform_filter(w, x_shape, stride=1, padding=0, m=2, whole_kernel=False, s
 
 
 def conv_forward(x, w, bias=None, stride=1, padding=0, m=2, U=None, chunk_images=0, whole_kernel=False,
-                 stacked=None, unfused=False, channels_first_out=False, direct=None):
+                 stacked=None, unfused=False, channels_first_out=False, direct=None, row=False):
     """Winograd / DWM convolution of an NC[D]HW tensor.  Returns an NC[D]HW tensor whose memory
     is channel-last (torch.channels_last / channels_last_3d), or, with `channels_first_out`, plain
     contiguous.  A channel-last input is used without a copy; a contiguous (channel-first) one is
     handed to the library as it is (wc_conv_desc.x_layout: small single-piece plans read it inside the
     input transform, the others copy it to channel-last scratch with the library's own kernel); any
     other layout is made contiguous first.  `stacked`: see make_desc; None chooses.
-    `unfused=True` keeps thin 16-bit 3x3 layers on the three-kernel path (wc_conv_desc.unfused)."""
+    `unfused=True` keeps thin 16-bit 3x3 layers on the three-kernel path (wc_conv_desc.unfused).
+    `row=True` lets the library take the row form (wc_conv_desc.row), whatever tile is asked for."""
     if USE_EXT:
         return _ext.conv_forward(x, w, bias, stride, padding, m, U, chunk_images, bool(whole_kernel), stacked,
-                                 bool(unfused), bool(channels_first_out), direct)
+                                 bool(unfused), bool(channels_first_out), direct, bool(row))
     return _conv_forward(x, w, bias, stride, padding, m, U, chunk_images, whole_kernel, stacked, unfused,
-                         channels_first_out, direct, None)
+                         channels_first_out, direct, None, row)
 
 
 STAGES = ("filter_transform", "layout_in", "input_transform", "product", "output_transform", "layout_out")
 
 
 def conv_forward_timed(x, w, bias=None, stride=1, padding=0, m=2, U=None, chunk_images=0, whole_kernel=False,
-                       stacked=None, unfused=False, channels_first_out=False, direct=None):
+                       stacked=None, unfused=False, channels_first_out=False, direct=None, row=False):
     """conv_forward through wc_conv_forward_timed: returns (y, {stage: milliseconds on the device}) with the
     stages of STAGES; waits for the device (the reference's timing prints: dwm.py:44-106)."""
     times = (ctypes.c_float * len(STAGES))()
     y = _conv_forward(x, w, bias, stride, padding, m, U, chunk_images, whole_kernel, stacked, unfused,
-                      channels_first_out, direct, times)
+                      channels_first_out, direct, times, row)
     return y, dict(zip(STAGES, (float(t) for t in times)))
 
 
 def _conv_forward(x, w, bias, stride, padding, m, U, chunk_images, whole_kernel, stacked, unfused,
-                  channels_first_out, direct, times):
+                  channels_first_out, direct, times, row=False):
     check_operands(x, int(w.shape[0]), bias, U)
     _require_gpu(x, w, bias, U)
     if w.dtype != x.dtype or (bias is not None and bias.dtype != x.dtype):
@@ -399,9 +408,12 @@ def _conv_forward(x, w, bias, stride, padding, m, U, chunk_images, whole_kernel,
     y_layout = int(bool(channels_first_out))
     # the one-kernel path of thin layers needs 16-byte aligned operands; a legal view can start anywhere
     # (x[1:] of a channel-last tensor with 6 channels and 7 x 7 images is 4-byte aligned): three kernels then
+    row = bool(row) and not unfused
+    if row and misaligned(x_mem, U):                       # ... and so does the row form: aligned copies of them
+        x_mem, U = x_mem.clone(), U.clone() if U is not None else None
     unfused = bool(unfused) or misaligned(x_mem, U)
     desc, y_shape, nbytes, u_elems = _forward_setup(tuple(x.shape), tuple(w.shape), x.dtype, stride, padding, m,
-                                                    chunk_images, whole_kernel, stacked, unfused, x_layout, y_layout, direct)
+                                                    chunk_images, whole_kernel, stacked, unfused, x_layout, y_layout, direct, row)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
     if y_layout:
         y = torch.empty([y_shape[0], y_shape[-1]] + y_shape[1:-1], dtype=x.dtype, device=x.device)
@@ -424,18 +436,18 @@ _SETUPS = {}
 
 
 def _forward_setup(x_shape, w_shape, dtype, stride, padding, m, chunk_images, whole_kernel, stacked, unfused=False,
-                   x_layout=0, y_layout=0, direct=None):
+                   x_layout=0, y_layout=0, direct=None, row=False):
     """Descriptor, output shape (channel-last), workspace bytes and size of U for one problem.  Kept
     per problem: for small layers (a few tens of microseconds on the GPU) rebuilding them on every
     call costs as much host time as the launches themselves."""
     key = (x_shape, w_shape, dtype, stride if isinstance(stride, int) else tuple(stride),
            padding if isinstance(padding, int) else tuple(padding), m, chunk_images, whole_kernel, stacked, unfused,
-           x_layout, y_layout, direct)
+           x_layout, y_layout, direct, row)
     hit = _SETUPS.get(key)
     if hit is None:
         lib = _lib.load()
         desc = make_desc(x_shape, w_shape, dtype, stride, padding, m, chunk_images, whole_kernel, stacked, unfused,
-                         x_layout, y_layout, direct)
+                         x_layout, y_layout, direct, row)
         out, _ = out_dims(desc)
         nbytes, ue = ctypes.c_size_t(), ctypes.c_size_t()
         check(lib.wc_conv_workspace_bytes(ctypes.byref(desc), ctypes.byref(nbytes)))
@@ -527,7 +539,7 @@ def conv_backward_input(dy, w, x_spatial, stride=1, padding=0, m=2):
     # output channels, where the sum is too short to average it down either (fp16, K = 1: up to
     # 3e-2 with tile 4, 1e-3 with tile 2)
     mm = m if (stride == 1 and w.shape[0] >= 8 and (m == 2 or nd == 2 or ks == (3, 3, 3))) else 2
-    dx = conv_forward(dy, w_rot, None, 1, tuple(k - 1 - p for k, p in zip(ks, pads)), mm)
+    dx = conv_forward(dy, w_rot, None, 1, tuple(k - 1 - p for k, p in zip(ks, pads)), mm, row=True)
     if tuple(dx.shape[2:]) != want:
         raise ValueError("dy of shape %r does not belong to an input of extent %r" % (tuple(dy.shape), want))
     return dx
