@@ -157,6 +157,7 @@ const char* wc_last_error(void);
  * (transforms along depth and height only, the three width taps along the reduction; by size otherwise).
  * config 8 / 9: the one-kernel F(2x2,3x3) path with workgroups of 64 / 32 output channels whatever
  * the number of tiles (9 only where the channel count allows it).
+ * config 20: the weight gradient never takes the tap form (backward_taps.hip).
  * config 16 to 19: the row form with the wide, half, small or split workgroups whatever the problem (conv_row.hip).
  * Works only in a process started with WINOCONV_TEST_HOOKS=1 in its environment (WC_ERR_UNSUPPORTED
  * otherwise, and nothing changes); what it sets holds for the calling host thread only, so a caller

@@ -266,6 +266,7 @@ struct BwdLayout {
   size_t v_bytes, dm_bytes, du_bytes, acc_bytes;
   bool one_tap;                     // 1x1 kernel, stride 1, no padding: dw = dy^T x, no transforms
   bool gathered;                    // 2-D stride 2: dw[tap] = dy^T (the pixels of x that tap reads), no transforms
+  bool taps;                        // 16-bit 3x3 and 3x3x3 at stride 1: the tap form (backward_taps.hip), du_bytes of partial sums
 };
 
 // A 2-D layer at stride 2: the transform-domain gradient runs Winograd tiles on the parity phases of x (V and dM
@@ -324,7 +325,7 @@ int make_bwd_layout(const wc_conv_desc* d, BwdLayout* L) {
   WC_CHECK_ARG(d != nullptr, "null descriptor");
   WC_CHECK_ARG(d->dtype == WC_F32 || d->dtype == WC_F16 || d->dtype == WC_BF16, "dtype %d", d->dtype);
   WC_CHECK_ARG((d->ndim == 2 || d->ndim == 3) && d->N > 0 && d->C > 0 && d->K > 0, "ndim %d, N %d, C %d, K %d", d->ndim, d->N, d->C, d->K);
-  L->one_tap = L->gathered = false;
+  L->one_tap = L->gathered = L->taps = false;
   if (one_tap_layout(d, L)) return WC_OK;
   if (gathered_layout(d, L)) return WC_OK;
   if (d && d->stacked == 2)
@@ -334,6 +335,11 @@ int make_bwd_layout(const wc_conv_desc* d, BwdLayout* L) {
   rc = wc_conv_out_dims(d, L->out, L->grid);
   if (rc) return rc;
   if (L->plan.t_total > 0xffff) return fail(WC_ERR_UNSUPPORTED, "plan with %d transform elements is too large", L->plan.t_total);
+  if (taps_gradient_fits(d, L->out, &L->du_bytes)) {
+    L->taps = true;
+    L->v_bytes = L->dm_bytes = L->acc_bytes = 0;
+    return WC_OK;
+  }
   const bool stacked = d->stacked && L->plan.n_pieces > 1;
   L->Cp = stacked_row(d, &L->plan);
   L->ldm = wc_padded_channels8(d->K);
@@ -409,6 +415,7 @@ int wc_conv_backward_weight(const wc_conv_desc* d, const void* x, const void* dy
   const size_t y_image = (size_t)L.out[0] * L.out[1] * L.out[2] * d->K * L.es;
   const int taps = d->kernel[0] * d->kernel[1] * d->kernel[2];
 
+  if (L.taps) return taps_gradient(d, L.out, x, dy, dw, dw_strides, dU, stream);
   if (L.one_tap) {
     const long long P = L.tiles_per_image * d->N;
     rc = batched_gemm_tn(dy, x, dU, 1, P, d->K, d->C, d->K, d->C, d->C, L.S, L.Pq, d->dtype, stream);

@@ -217,6 +217,12 @@ int batched_gemm_tn(const void* A, const void* B, float* D, int T, long long P, 
 int gemm_tn_conv(const void* dy, const void* x, float* D, int N, int H, int W, int C, int K, int kh, int kw, int stride,
                  int pad_h, int pad_w, int oH, int oW, int S, int Pq, int dtype, void* stream);
 
+// The tap form of the weight gradient (backward_taps.hip; 16-bit 3x3 and 3x3x3 layers at stride 1 with output extents `out`):
+// whether it is taken and the bytes of its partial sums, and the launch
+bool taps_gradient_fits(const wc_conv_desc* d, const int out[3], size_t* workspace_bytes);
+int taps_gradient(const wc_conv_desc* d, const int out[3], const void* x, const void* dy, void* dw,
+                  const int64_t dw_strides[5], float* part, void* stream);
+
 // One-kernel F(2x2, 3x3) forward pass for thin 16-bit layers (conv_thin.hip): whether the problem
 // with this single-piece plan is in its range, and the launch.  U (16, K, Cp) from wc_filter_transform.
 bool thin_conv_fits(const wc_conv_desc* d, const wc_plan* plan);

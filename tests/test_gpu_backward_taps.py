@@ -1,0 +1,88 @@
+"""The tap form of the weight gradient (backward_taps.hip; 16-bit 3x3 and 3x3x3 layers at stride 1).  The reference has no
+backward pass (src/back/utils.cu:15-24); the gradient of a convolution in fp64 pins it.
+
+Bound: the operands are exact and the sums fp32, so the result carries its own rounding, at most 2^-(p+1) of each value
+relative for p + 1 bits of significand (11 in fp16, 8 in bf16), and the fp32 sum's: n 2^-24 of the sum of magnitudes for n
+products, below 1e-5 of the 2-norm at these sizes."""
+import pytest
+import torch
+
+from pytorch_winoconv_amd import _lib, engine
+
+pytestmark = pytest.mark.gpu
+BOUND = {torch.float16: 2.0 ** -11 + 1e-5, torch.bfloat16: 2.0 ** -8 + 1e-5}
+
+CASES = [
+    # x shape, K, pad
+    ((1, 8, 3, 3), 8, 0),                                    # one output pixel
+    ((1, 8, 1, 1), 8, 1),
+    ((2, 8, 5, 6), 16, 1),
+    ((3, 72, 9, 17), 136, 1),                                # remainders of channels on both sides, three blocks of 64
+    ((2, 40, 7, 7), 72, 0), ((2, 64, 30, 50), 64, (2, 0)),   # other paddings
+    ((1, 16, 4, 253), 24, 1), ((1, 16, 3, 254), 24, 1),      # the widest rows of the ring, and rows it does not hold
+    ((5, 128, 31, 31), 256, 1),                              # several parts, the last one short
+    ((1, 16, 4, 3, 9), 8, 1), ((2, 24, 3, 6, 5), 72, (0, 1, 2)), ((3, 64, 5, 12, 11), 128, 1),
+]
+
+
+def _last(t):
+    return t.contiguous(memory_format=torch.channels_last if t.dim() == 4 else torch.channels_last_3d)
+
+
+def _operands(xs, K, pad, dtype, seed=3):
+    g = torch.Generator().manual_seed(seed)
+    nd = len(xs) - 2
+    pads = (pad,) * nd if isinstance(pad, int) else pad
+    x = torch.randn(xs, generator=g).to(dtype)
+    dy = torch.randn([xs[0], K] + [xs[2 + i] + 2 * pads[i] - 2 for i in range(nd)], generator=g).to(dtype)
+    shape = (K, xs[1]) + (3,) * nd
+    grad = torch.nn.grad.conv2d_weight if nd == 2 else torch.nn.grad.conv3d_weight
+    return x, dy, pads, shape, grad(x.double(), shape, dy.double(), padding=pads)
+
+
+def _err(dw, ref):
+    return float((dw.double().cpu() - ref).norm() / ref.norm())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", CASES)
+def test_against_fp64(dev, dtype, case):
+    x, dy, pads, shape, ref = _operands(*case, dtype)
+    dw = engine.conv_backward_weight(_last(x.to(dev)), _last(dy.to(dev)), shape, 1, pads, 2)
+    wide = case[0][-1] == 254                                # the transform domain: test_gpu_backward.py's bound
+    assert _err(dw, ref) <= (2e-2 if wide else BOUND[dtype])
+
+
+@pytest.mark.parametrize("shift", [1, 4])
+def test_tensors_that_start_anywhere(dev, shift):
+    x, dy, pads, shape, ref = _operands((2, 24, 6, 7), 40, 1, torch.float16)
+
+    def view(t):
+        t = t.to(dev).permute(0, 2, 3, 1)
+        flat = torch.empty(t.numel() + 8, dtype=t.dtype, device=dev)[shift:shift + t.numel()]
+        return flat.view(t.shape).copy_(t).permute(0, 3, 1, 2)
+
+    dw = engine.conv_backward_weight(view(x), view(dy), shape, 1, pads, 2)
+    assert _err(dw, ref) <= BOUND[torch.float16]
+
+
+def test_parts_are_added_in_a_fixed_order(dev):
+    x, dy, pads, shape, _ = _operands((5, 128, 31, 31), 256, 1, torch.float16)
+    x, dy = _last(x.to(dev)), _last(dy.to(dev))
+    first = engine.conv_backward_weight(x, dy, shape, 1, pads, 2)
+    assert all(torch.equal(first, engine.conv_backward_weight(x, dy, shape, 1, pads, 2)) for _ in range(3))
+
+
+def test_same_as_the_transform_domain(dev):
+    """The tap form and the form it replaces agree within the second one's error."""
+    x, dy, pads, shape, ref = _operands((3, 64, 5, 12, 11), 128, 1, torch.float16)
+    x, dy = _last(x.to(dev)), _last(dy.to(dev))
+    taps = engine.conv_backward_weight(x, dy, shape, 1, pads, 2)
+    lib = _lib.load()
+    _lib.check(lib.wc_test_gemm_override(20, 1))
+    try:
+        other = engine.conv_backward_weight(x, dy, shape, 1, pads, 2)
+    finally:
+        _lib.check(lib.wc_test_gemm_override(-1, 1))
+    assert _err(taps, ref) < _err(other, ref)
+    assert float((taps.float() - other.float()).norm() / taps.float().norm()) <= 5e-3
