@@ -94,28 +94,38 @@ int direct_conv(const wc_conv_desc* d, const void* x, int n_images, const void* 
 // parity (py, px) of (iy + ph, ix + pw); a class only meets the taps of its own parity, ky = py + 2a, and with
 // iy + ph = 2 qy + py it is a stride-1 direct convolution of dy with that sub-kernel, flipped, its channel axes
 // exchanged: dx_class[qy, qx] = sum_a' sum_b' dy[qy - (A - 1) + a', qx - (B - 1) + b'] g[a', b'],
-// g[a', b'] = w[., ., py + 2 (A - 1 - a'), px + 2 (B - 1 - b')].  One launch of the direct form per class, each writing
-// every second pixel of dx: the multiplications of the forward pass and one pass over dy per class, where convolving a
-// zero-filled dy at stride 1 multiplies four times as much.
+// g[a', b'] = w[., ., py + 2 (A - 1 - a'), px + 2 (B - 1 - b')].  The classes are direct products that each write every
+// second pixel of dx, in one launch: the multiplications of the forward pass and one pass over dy per class, where convolving
+// a zero-filled dy at stride 1 multiplies four times as much.
 struct SubFilterArgs {
   const void* w;
-  void* U;            // (C, A, B, K): rows = input channels of the layer, reduction = its output channels
+  struct Class {
+    void* U;          // (C, A, B, K): rows = input channels of the layer, reduction = its output channels
+    int A, B, py, px;
+    long long end;    // elements of this class and those before it
+  } cls[4];
+  int n;
   long long s[5];
-  int K, C, A, B, py, px;
-  long long total;
+  int K, C;
 };
 
 template <typename T>
 __global__ __launch_bounds__(256) void sub_filter_kernel(SubFilterArgs a) {
-  const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= a.total) return;
+  long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
+  typename SubFilterArgs::Class g = a.cls[0];
+  long long begin = 0;
+#pragma unroll
+  for (int i = 1; i < 4; ++i)
+    if (i < a.n && idx >= a.cls[i - 1].end) { g = a.cls[i]; begin = a.cls[i - 1].end; }
+  if (idx >= g.end) return;
+  idx -= begin;
   const int k = (int)(idx % a.K);
   long long q = idx / a.K;
-  const int b = (int)(q % a.B); q /= a.B;
-  const int aa = (int)(q % a.A);
-  const long long c = q / a.A;
-  const int ky = a.py + 2 * (a.A - 1 - aa), kx = a.px + 2 * (a.B - 1 - b);
-  static_cast<T*>(a.U)[idx] = static_cast<const T*>(a.w)[k * a.s[0] + c * a.s[1] + ky * a.s[3] + kx * a.s[4]];
+  const int b = (int)(q % g.B); q /= g.B;
+  const int aa = (int)(q % g.A);
+  const long long c = q / g.A;
+  const int ky = g.py + 2 * (g.A - 1 - aa), kx = g.px + 2 * (g.B - 1 - b);
+  static_cast<T*>(g.U)[idx] = static_cast<const T*>(a.w)[k * a.s[0] + c * a.s[1] + ky * a.s[3] + kx * a.s[4]];
 }
 
 template <typename T>
@@ -177,6 +187,11 @@ extern "C" int wc_conv_backward_input(const wc_conv_desc* d, const void* dy, con
   const size_t es = d->dtype == WC_F32 ? 4 : 2;
   unsigned char* ws = static_cast<unsigned char*>(workspace);
   hipStream_t s = as_stream(stream);
+  SubFilterArgs a;
+  a.w = w; a.n = 0;
+  for (int i = 0; i < 5; ++i) a.s[i] = w_strides[i];
+  a.K = d->K; a.C = d->C;
+  DirectClass cls[4];
   for (int py = 0; py < 2; ++py) {
     for (int px = 0; px < 2; ++px) {
       const int A = (kh - py + 1) / 2, B = (kw - px + 1) / 2;                 // taps of this parity (may be none)
@@ -196,22 +211,29 @@ extern "C" int wc_conv_backward_input(const wc_conv_desc* d, const void* dy, con
         WC_CHECK_LAUNCH("zero_class_kernel");
         continue;
       }
-      SubFilterArgs a;
-      a.w = w; a.U = ws;
-      for (int i = 0; i < 5; ++i) a.s[i] = w_strides[i];
-      a.K = d->K; a.C = d->C; a.A = A; a.B = B; a.py = py; a.px = px;
-      a.total = (long long)d->C * A * B * d->K;
-      dispatch_dtype(d->dtype, [&](auto t) {
-        using T = decltype(t);
-        hipLaunchKernelGGL(sub_filter_kernel<T>, dim3((unsigned)ceil_div_ll(a.total, 256)), dim3(256), 0, s, a);
-        return 0;
-      });
-      WC_CHECK_LAUNCH("sub_filter_kernel");
-      rc = gemm_direct_conv(dy, ws, nullptr, dx, d->N, out[1], out[2], d->K, d->C, A, B, 1, A - 1 - qy0, B - 1 - qx0, Qh, Qw,
-                            d->dtype, stream, 2, y0, x0, H, W);
-      if (rc) return rc;
-      ws += (a.total * es + 255) / 256 * 256;
+      const long long elems = (long long)d->C * A * B * d->K;
+      a.cls[a.n] = {ws, A, B, py, px, (a.n ? a.cls[a.n - 1].end : 0) + elems};
+      cls[a.n] = {ws, A, B, A - 1 - qy0, B - 1 - qx0, Qh, Qw, y0, x0};
+      ++a.n;
+      ws += (elems * es + 255) / 256 * 256;
     }
+  }
+  if (a.n == 0) return WC_OK;
+  for (int i = a.n; i < 4; ++i) a.cls[i] = a.cls[a.n - 1];
+  dispatch_dtype(d->dtype, [&](auto t) {
+    using T = decltype(t);
+    hipLaunchKernelGGL(sub_filter_kernel<T>, dim3((unsigned)ceil_div_ll(a.cls[a.n - 1].end, 256)), dim3(256), 0, s, a);
+    return 0;
+  });
+  WC_CHECK_LAUNCH("sub_filter_kernel");
+  // kernel rows of four taps and more have a kernel of their own (direct_rows.hip), one launch per class
+  if ((kw + 1) / 2 <= 3)
+    return gemm_direct_classes(dy, cls, a.n, dx, d->N, out[1], out[2], d->K, d->C, d->dtype, stream, H, W);
+  for (int i = 0; i < a.n; ++i) {
+    const DirectClass& c = cls[i];
+    rc = gemm_direct_conv(dy, c.U, nullptr, dx, d->N, out[1], out[2], d->K, d->C, c.kh, c.kw, 1, c.pad_h, c.pad_w, c.oH, c.oW,
+                          d->dtype, stream, 2, c.o_y0, c.o_x0, H, W);
+    if (rc) return rc;
   }
   return WC_OK;
 }

@@ -21,6 +21,8 @@
 // run (neighbours along the width) from a single operand tile that is n_run - 1 rows taller.
 #include "wc_common.h"
 
+#include <algorithm>
+
 namespace wc {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -88,6 +90,18 @@ struct GemmArgs {
   int o_step, o_y0, o_x0, o_H, o_W;
 };
 
+// Up to four products of the direct form in one launch (the parity classes of a strided layer's input gradient): what each
+// replaces in the arguments.  Workgroup b works on class b % n, tile b / n, so that the classes, whose reductions
+// differ, share out every XCD and neighbours read the same pixels.
+struct GemmClassArgs : GemmArgs {
+  struct Class {
+    const void* U;
+    long long jump;
+    int P, Cp, tiles_p, run_blocks, plane_runs, oH, oW, pad_h, pad_w, kw, o_y0, o_x0;
+  } cls[4];
+  int n_classes;
+};
+
 typedef uint32_t Chunk16 __attribute__((ext_vector_type(4)));   // one 16-byte global/LDS access
 
 // Operand rows in LDS are 64 bytes (four 16-byte chunks) with no padding; chunk c of row r sits
@@ -97,9 +111,11 @@ typedef uint32_t Chunk16 __attribute__((ext_vector_type(4)));   // one 16-byte g
 // is conflict-free for 128-byte and for 256-byte wide bank sets alike.
 __device__ __forceinline__ int swizzle(int r) { return (((r >> 1) ^ (r >> 3)) & 1) | (((r >> 2) & 1) << 1); }
 
-template <typename T, int WM, int WN, int BK, int NWP = 2, int NWK = 2, bool SHIFT = false, bool DIRECT = false>
-__global__ __launch_bounds__(64 * NWP * NWK, (WM * WN <= 8 && NWP * NWK == 4 ? 2 : 1)) void gemm_kernel(GemmArgs g) {
-  static_assert(!DIRECT || SHIFT, "the direct form walks the taps like the shifted operand");
+template <typename T, int WM, int WN, int BK, int NWP = 2, int NWK = 2, bool SHIFT = false, bool DIRECT = false, bool CLASSES = false>
+__global__ __launch_bounds__(64 * NWP * NWK, (WM * WN <= 8 && NWP * NWK == 4 ? 2 : 1))
+void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
+  static_assert((!DIRECT || SHIFT) && (!CLASSES || DIRECT), "the direct form walks the taps like the shifted operand");
+  GemmArgs g = args;
   using MF = Mfma<T>;
   constexpr int NT = 64 * NWP * NWK;               // threads: NWP x NWK wavefronts
   constexpr int BM = 32 * NWP * WM, BN = 32 * NWK * WN;
@@ -116,8 +132,15 @@ __global__ __launch_bounds__(64 * NWP * NWK, (WM * WN <= 8 && NWP * NWK == 4 ? 2
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   T* lds = reinterpret_cast<T*>(lds_raw);
 
-  const int blk = xcd_remap(blockIdx.x, g.per_xcd);
+  int blk = xcd_remap(blockIdx.x, g.per_xcd);
   if (blk >= g.n_blocks) return;
+  if constexpr (CLASSES) {
+    const typename GemmClassArgs::Class& c = args.cls[blk % args.n_classes];
+    blk /= args.n_classes;
+    if (blk >= c.tiles_p * g.tiles_k) return;
+    g.U = c.U; g.jump = c.jump; g.P = c.P; g.Cp = c.Cp; g.tiles_p = c.tiles_p; g.run_blocks = c.run_blocks; g.plane_runs = c.plane_runs;
+    g.oH = c.oH; g.oW = c.oW; g.pad_h = c.pad_h; g.pad_w = c.pad_w; g.kw = c.kw; g.o_y0 = c.o_y0; g.o_x0 = c.o_x0;
+  }
   const int kt_ = blk % g.tiles_k;
   const int pt = (blk / g.tiles_k) % g.tiles_p;
   const int t = blk / (g.tiles_k * g.tiles_p);
@@ -884,6 +907,64 @@ int gemm_direct_conv(const void* x, const void* U, const void* bias, void* y, in
   hipLaunchKernelGGL(c.fn, dim3((unsigned)(g.per_xcd * kXcds)), dim3(c.threads), c.lds, as_stream(stream), g);
   WC_CHECK_LAUNCH("gemm_kernel (direct form)");
   return WC_OK;
+}
+
+// The direct products of `n` parity classes in one launch, classes as in gemm_direct_conv's arguments (kernel rows of at
+// most 3 taps).  A class has a quarter of the pixels and at most four of nine taps, so one by one they leave most of the
+// chip idle.  Whole input gradient with its filter copy (also one launch now), us, before | now: bf16 N=32, 256 -> 128
+// channels, 28x28 -> 56x56 72 | 52; fp16 N=8 128 -> 64, 56x56 36 | 14; N=2 512 -> 256, 15x17 89 | 40; N=64 512 -> 256, 28x28
+// 120 | 95; N=64 128 -> 64, 112x112 119 | 116; fp32 N=8 128 -> 64, 56x56 64 | 33.  Tiles (256x128 | 128x128 | 64x64): the
+// first 52 | 57 | 59, the second 24 | 17 | 14, N=64 28x28 93 | 103 | 116.
+int gemm_direct_classes(const void* x, const DirectClass* classes, int n, void* y, int N, int H, int W, int C, int K,
+                        int dtype, void* stream, int o_H, int o_W) {
+  WC_CHECK_ARG(x && y && n > 0 && n <= 4, "gemm_direct_classes: %d classes", n);
+  const int cq = dtype == WC_F32 ? 16 : 32;
+  WC_CHECK_ARG(C > 0 && C % cq == 0 && K > 0 && K % 8 == 0, "gemm_direct_classes: C %d (multiple of %d), K %d (multiple of 8)", C, cq, K);
+  return dispatch_dtype(dtype, [&](auto t) -> int {
+    using T = decltype(t);
+    constexpr int BK = sizeof(T) == 4 ? 16 : 32;
+    auto launch = [&](auto wm, auto wn) -> int {
+      constexpr int WM = decltype(wm)::value, WN = decltype(wn)::value;
+      const GemmConfig c = make_config<T, WM, WN, BK, 2, 2, true, true>();        // the sizes of the tile
+      auto fn = &gemm_kernel<T, WM, WN, BK, 2, 2, true, true, true>;
+      GemmClassArgs g;
+      g.V = x; g.U = nullptr; g.M = y; g.bias = nullptr;
+      g.P = 0; g.K = K; g.ldm = K; g.Cp = 0; g.ldv = C; g.run_blocks = 0; g.jump = g.jump2 = 0; g.plane_runs = 0;
+      g.n_run = g.total_runs = g.run_rows = g.plane_extra = 0;
+      g.H = H; g.W = W; g.oH = g.oW = 1; g.conv_stride = 1; g.pad_h = g.pad_w = 0; g.kw = 1; g.cblocks = C / BK;
+      g.o_step = 2; g.o_y0 = g.o_x0 = 0; g.o_H = o_H; g.o_W = o_W;
+      g.sV = g.sU = g.sM = 0; g.tiles_p = 0; g.tiles_k = ceil_div(K, c.bn); g.T = 1;
+      g.n_classes = n;
+      int most = 0;
+      for (int i = 0; i < n; ++i) {
+        const DirectClass& d = classes[i];
+        const long long P = (long long)N * d.oH * d.oW;
+        WC_CHECK_ARG(d.U && P > 0 && P < (1ll << 31) && (long long)d.kh * d.kw * C < (1ll << 24), "gemm_direct_classes: problem too large");
+        g.cls[i] = {d.U, (long long)(W - d.kw) * C, (int)P, d.kh * d.kw * C, ceil_div((int)P, c.bm), d.kw * C / BK, d.kh + 1,
+                    d.oH, d.oW, d.pad_h, d.pad_w, d.kw, d.o_y0, d.o_x0};
+        most = std::max(most, g.cls[i].tiles_p);
+      }
+      const long long blocks = (long long)most * g.tiles_k * n;
+      WC_CHECK_ARG(blocks < (1ll << 30), "gemm_direct_classes: problem too large");
+      g.n_blocks = (int)blocks;
+      g.per_xcd = ceil_div((int)blocks, kXcds);
+      if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), c.lds)) return rc;
+      hipLaunchKernelGGL(fn, dim3((unsigned)(g.per_xcd * kXcds)), dim3(c.threads), c.lds, as_stream(stream), g);
+      WC_CHECK_LAUNCH("gemm_kernel (direct form, classes)");
+      return WC_OK;
+    };
+    // the rule of choose_direct over the tiles of all classes
+    long long P = 0;
+    for (int i = 0; i < n; ++i) P += (long long)N * classes[i].oH * classes[i].oW;
+    const long long mid = ceil_div_ll(P, 128) * ceil_div(K, 128);
+    if constexpr (sizeof(T) == 4) {
+      if (K > 64 && mid >= 2048) return launch(ic<2>{}, ic<2>{});
+    } else if (K > 64) {
+      if (ceil_div_ll(P, 256) * ceil_div(K, 128) >= kCus) return launch(ic<4>{}, ic<2>{});
+      if (mid >= kCus) return launch(ic<2>{}, ic<2>{});
+    }
+    return launch(ic<1>{}, ic<1>{});
+  });
 }
 
 }  // namespace wc

@@ -179,6 +179,11 @@ int gemm_direct_conv(const void* x, const void* U, const void* bias, void* y, in
                      int kh, int kw, int stride, int pad_h, int pad_w, int oH, int oW, int dtype, void* stream,
                      int o_step = 0, int o_y0 = 0, int o_x0 = 0, int o_H = 0, int o_W = 0);
 
+// The same for up to four parity classes of the pixels of an (o_H, o_W) image, with a filter each, in one launch
+struct DirectClass { const void* U; int kh, kw, pad_h, pad_w, oH, oW, o_y0, o_x0; };
+int gemm_direct_classes(const void* x, const DirectClass* classes, int n, void* y, int N, int H, int W, int C, int K,
+                        int dtype, void* stream, int o_H, int o_W);
+
 // The direct form with one operand tile per kernel row (direct_rows.hip; 16-bit types, kernel rows of 4 to 8 taps, stride
 // 1 or 2): whether a problem is in its range (the input rows that 256 consecutive output pixels read, with their
 // padding, must fit a stage of kDirectRowsPixels pixels), and the launch, with the arguments of gemm_direct_conv.
