@@ -313,6 +313,11 @@ int wc_conv_backward_input(const wc_conv_desc* desc, const void* dy, const void*
 int wc_conv_backward_weight(const wc_conv_desc* desc, const void* x, const void* dy, void* dw,
                             const int64_t dw_strides[5], void* workspace, size_t workspace_bytes,
                             void* stream);
+/* Bias gradient (no counterpart in the reference): db[k] = sum over the rows of dy (rows, K), contiguous - the pixels of a
+ * channel-last tensor of K channels -, in fp32, rounded once.  Workspace 16-byte aligned. */
+int wc_bias_gradient_workspace_bytes(long long rows, int K, int dtype, size_t* bytes);
+int wc_bias_gradient(const void* dy, void* db, long long rows, int K, int dtype, void* workspace, size_t workspace_bytes,
+                     void* stream);
 #ifdef __cplusplus
 }
 #endif

@@ -62,7 +62,12 @@ class WinoConvFunction(torch.autograd.Function):
         if ctx.needs_input_grad[1]:
             dw = engine.conv_backward_weight(x, dy, w.shape, stride, padding, m)
         if has_bias and ctx.needs_input_grad[2]:
-            db = dy.sum(dim=[0] + list(range(2, dy.dim())))
+            # the engine's kernel where this pass runs on it anyway; a gradient that is itself differentiated, or a dy
+            # that the kernel would have to copy first, stays with torch
+            if ctx.needs_input_grad[1] and not torch.is_grad_enabled() and engine.channel_last_memory(dy):
+                db = engine.bias_gradient(dy)
+            else:
+                db = dy.sum(dim=[0] + list(range(2, dy.dim())))
         return dx, dw, db, None, None, None, None
 
 

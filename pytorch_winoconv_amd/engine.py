@@ -167,6 +167,11 @@ def channel_last(x):
     return v if v.is_contiguous() else v.contiguous()
 
 
+def channel_last_memory(x):
+    """True where channel_last(x) is a view."""
+    return x.permute((0,) + tuple(range(2, x.dim())) + (1,)).is_contiguous()
+
+
 def channel_first_view(y_cl):
     """(N, *sp, K) contiguous tensor -> (N, K, *sp) view (channels_last memory format)."""
     nd = y_cl.dim() - 2
@@ -487,6 +492,24 @@ def conv_backward_weight(x, dy, w_shape, stride=1, padding=0, m=2, whole_kernel=
     check(lib.wc_conv_backward_weight(ctypes.byref(desc), _ptr(x_cl), _ptr(dy_cl), _ptr(dw), _w_strides(dw),
                                       _ptr(ws), nbytes.value, _stream(x)))
     return dw
+
+
+def bias_gradient(dy):
+    """Sum of an NC[D]HW tensor over everything but its channels, in dy's dtype (fp32 sums, rounded once).  Channel-last
+    memory is read as it is."""
+    _require_gpu(dy)
+    lib = _lib.load()
+    K = dy.shape[1]
+    db = torch.empty(K, dtype=dy.dtype, device=dy.device)
+    rows = dy.numel() // max(K, 1)
+    if rows == 0:
+        return db.zero_()
+    dy_cl = channel_last(dy)
+    nbytes = ctypes.c_size_t()
+    check(lib.wc_bias_gradient_workspace_bytes(rows, K, _DTYPES[dy.dtype], ctypes.byref(nbytes)))
+    ws = torch.empty(nbytes.value, dtype=torch.uint8, device=dy.device)
+    check(lib.wc_bias_gradient(_ptr(dy_cl), _ptr(db), rows, K, _DTYPES[dy.dtype], _ptr(ws), nbytes.value, _stream(dy)))
+    return db
 
 
 def conv_backward_input(dy, w, x_spatial, stride=1, padding=0, m=2):
