@@ -296,7 +296,8 @@ int wc_conv_forward_static(const wc_conv_desc* desc, const void* x,
  * helper exists for one, src/back/utils.cu:15-24; include/split_functions_grad.h:3-6 is empty).
  * dw[k][c][taps] = gradient of sum(y * dy) with respect to the filter, for the same descriptor as
  * the forward call: x (N, D, H, W, C) and dy (N, oD, oH, oW, K) channel-last contiguous, dw written
- * through element strides for the axes (K, C, kD, kH, kW).  Computed in the transform domain
+ * through element strides for the axes (K, C, kD, kH, kW).  Computed directly for 1x1, strided 2-D and most 16-bit 3x3 and
+ * 3x3x3 layers, else in the transform domain
  * (dU = sum over tiles of dM x V, dw = G^T dU G) with every sum in fp32.  The input gradient needs
  * no entry point of its own: it is wc_conv_forward of dy with the flipped, transposed filter. */
 int wc_conv_backward_weight_workspace_bytes(const wc_conv_desc* desc, size_t* bytes);

@@ -313,9 +313,11 @@ std::vector<int> ints_of(py::object v, int nd, const char* what) {
 // used without a copy and a contiguous channel-first one is handed to the library as it is
 // (wc_conv_desc.x_layout); any other layout is made contiguous first.  The compiled form of the Python callers' common path (dwm.py:5-40, matrix_conv.py:70-135
 // of the reference end in the same call).
-at::Tensor conv_forward(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bias, py::object stride, py::object padding,
-                        int m, std::optional<at::Tensor> U, int chunk_images, bool whole_kernel, py::object stacked,
-                        bool unfused, bool channels_first_out, py::object direct, bool row) {
+// `flipped`: the filter is w reversed along every spatial axis, read through negative strides.  Only the row form's filter
+// kernel takes those: an undefined tensor, and nothing launched, where the library chooses another form.
+at::Tensor conv_impl(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bias, py::object stride, py::object padding,
+                     int m, std::optional<at::Tensor> U, int chunk_images, bool whole_kernel, py::object stacked,
+                     bool unfused, bool channels_first_out, py::object direct, bool row, bool flipped) {
   const int nd = (int)x.dim() - 2;
   if ((nd != 2 && nd != 3) || w.dim() != nd + 2)
     throw std::invalid_argument("expected 4-D or 5-D input and matching filter, got " + shape_str(x.sizes()) + " and " + shape_str(w.sizes()));
@@ -369,6 +371,7 @@ at::Tensor conv_forward(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bi
   d.unfused = unfused;
   d.row = row && !unfused ? -1 : 0;                                       // -1: the library may choose it
   check(wc_conv_auto(&d));
+  if (flipped && d.row != 1) return at::Tensor();
   int out[3], grid[3];
   check(wc_conv_out_dims(&d, out, grid));
   std::vector<int64_t> ys{x.size(0)};                      // channel-last shape of y
@@ -407,12 +410,102 @@ at::Tensor conv_forward(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bi
   at::Tensor bc = bias && bias->defined() ? bias->contiguous() : at::Tensor();
   int64_t s[5] = {w.stride(0), w.stride(1), 0, 0, 0};
   for (int a = 0; a < nd; ++a) s[5 - nd + a] = w.stride(2 + a);
+  const unsigned char* wp = static_cast<const unsigned char*>(w.data_ptr());
+  if (flipped)
+    for (int a = 0; a < nd; ++a) {
+      wp += (w.size(2 + a) - 1) * w.stride(2 + a) * w.element_size();
+      s[5 - nd + a] = -w.stride(2 + a);
+    }
   {
     py::gil_scoped_release nogil;
-    check(wc_conv_forward(&d, x_mem.data_ptr(), w.data_ptr(), s, U && U->defined() ? U->data_ptr() : nullptr,
+    check(wc_conv_forward(&d, x_mem.data_ptr(), wp, s, U && U->defined() ? U->data_ptr() : nullptr,
                           bc.defined() ? bc.data_ptr() : nullptr, y.data_ptr(), ws.data_ptr(), bytes, stream));
   }
   return channels_first_out ? y : y.permute(to_cf);
+}
+
+at::Tensor conv_forward(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bias, py::object stride, py::object padding,
+                        int m, std::optional<at::Tensor> U, int chunk_images, bool whole_kernel, py::object stacked,
+                        bool unfused, bool channels_first_out, py::object direct, bool row) {
+  return conv_impl(x, w, bias, stride, padding, m, U, chunk_images, whole_kernel, stacked, unfused, channels_first_out, direct,
+                   row, false);
+}
+
+// Input gradient of a stride-1 layer where the row form takes it (an undefined tensor elsewhere): dy convolved with w
+// flipped and its channel axes exchanged; `padding` is that convolution's.
+at::Tensor conv_backward_input_row(at::Tensor dy, at::Tensor w, py::object padding, int m) {
+  return conv_impl(dy, w.transpose(0, 1), std::nullopt, py::int_(1), padding, m, std::nullopt, 0, false, py::none(), false, false,
+                   py::none(), true, true);
+}
+
+// ---- gradients (the reference has no backward pass: src/back/utils.cu:15-24): engine.py's conv_backward_weight with the
+// form of the plan left to the library, and bias_gradient
+at::Tensor last_view(const at::Tensor& t) {       // (N, C, *) -> (N, *, C), contiguous
+  std::vector<int64_t> order{0};
+  for (int64_t a = 2; a < t.dim(); ++a) order.push_back(a);
+  order.push_back(1);
+  return t.permute(order).contiguous();
+}
+
+at::Tensor conv_backward_weight(at::Tensor x, at::Tensor dy, std::vector<int64_t> w_shape, py::object stride, py::object padding, int m) {
+  const int nd = (int)x.dim() - 2;
+  require_gpu(x, "conv_backward_weight");
+  require_gpu(dy, "conv_backward_weight");
+  if (dy.scalar_type() != x.scalar_type()) throw py::type_error("x and dy must share one dtype");
+  if ((nd != 2 && nd != 3) || (int)w_shape.size() != nd + 2)
+    throw std::invalid_argument("expected 4-D or 5-D input and matching filter, got " + shape_str(x.sizes()) + " and " + shape_str(w_shape));
+  if (x.size(1) != w_shape[1])
+    throw std::invalid_argument("input has " + std::to_string(x.size(1)) + " channels, filter expects " + std::to_string(w_shape[1]) +
+                                " (groups are not supported)");
+  const auto st = ints_of(stride, nd, "stride");
+  for (int a = 1; a < nd; ++a)
+    if (st[a] != st[0]) { PyErr_SetString(PyExc_NotImplementedError, "stride must be the same on every axis"); throw py::error_already_set(); }
+  const auto pd = ints_of(padding, nd, "padding");
+  wc_conv_desc d{};
+  d.ndim = nd;
+  d.C = (int)x.size(1); d.K = (int)w_shape[0];
+  d.kernel[0] = d.in[0] = 1;
+  for (int a = 0; a < nd; ++a) d.kernel[3 - nd + a] = (int)w_shape[2 + a];
+  d.stride = st[0]; d.m = m; d.dtype = dtype_of(x);
+  // the Winograd / DWM form of the forward plan, the direct one aside, whatever the batch; the gradient has no form whose
+  // pieces share one transformed input: pieces stacked with their own V
+  wc_conv_desc form = d;
+  form.N = 1; form.in[0] = 0; form.stacked = -1; form.direct = -1;
+  check(wc_conv_auto(&form));
+  d.N = (int)x.size(0);
+  for (int a = 0; a < nd; ++a) { d.in[3 - nd + a] = (int)x.size(2 + a); d.pad[3 - nd + a] = pd[a]; }
+  d.stacked = form.stacked != 0;
+  check(wc_conv_auto(&d));
+  int out[3], grid[3];
+  check(wc_conv_out_dims(&d, out, grid));
+  std::vector<int64_t> ys{x.size(0), w_shape[0]};
+  for (int a = 3 - nd; a < 3; ++a) ys.push_back(out[a]);
+  if (dy.sizes().vec() != ys) throw std::invalid_argument("dy has shape " + shape_str(dy.sizes()) + ", the convolution gives " + shape_str(ys));
+  at::Tensor dw = at::empty(w_shape, x.options());
+  const at::Tensor xl = last_view(x), dyl = last_view(dy);
+  size_t bytes = 0;
+  check(wc_conv_backward_weight_workspace_bytes(&d, &bytes));
+  void* stream = stream_of(x);
+  at::Tensor ws = workspace_for(x, bytes, stream);
+  int64_t s[5] = {dw.stride(0), dw.stride(1), 0, 0, 0};
+  for (int a = 0; a < nd; ++a) s[5 - nd + a] = dw.stride(2 + a);
+  py::gil_scoped_release nogil;
+  check(wc_conv_backward_weight(&d, xl.data_ptr(), dyl.data_ptr(), dw.data_ptr(), s, ws.data_ptr(), bytes, stream));
+  return dw;
+}
+
+at::Tensor bias_gradient(at::Tensor dy) {
+  require_gpu(dy, "bias_gradient");
+  at::Tensor db = at::empty({dy.size(1)}, dy.options());
+  const int64_t rows = dy.numel() / dy.size(1);
+  const at::Tensor dyl = last_view(dy);
+  size_t bytes = 0;
+  check(wc_bias_gradient_workspace_bytes(rows, (int)dy.size(1), dtype_of(dy), &bytes));
+  void* stream = stream_of(dy);
+  at::Tensor ws = workspace_for(dy, bytes, stream);
+  py::gil_scoped_release nogil;
+  check(wc_bias_gradient(dyl.data_ptr(), db.data_ptr(), rows, (int)dy.size(1), dtype_of(dy), ws.data_ptr(), bytes, stream));
+  return db;
 }
 
 // The reference's native entry point (pybind/extern.hpp:7-9): VALID convolution.  The four scratch tensors
@@ -452,5 +545,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("padding") = 0, py::arg("m") = 2, py::arg("U") = py::none(), py::arg("chunk_images") = 0,
         py::arg("whole_kernel") = false, py::arg("stacked") = py::none(), py::arg("unfused") = false,
         py::arg("channels_first_out") = false, py::arg("direct") = py::none(), py::arg("row") = false);
+  m.def("conv_backward_weight", &conv_backward_weight, py::arg("x"), py::arg("dy"), py::arg("w_shape"), py::arg("stride") = 1,
+        py::arg("padding") = 0, py::arg("m") = 2);
+  m.def("conv_backward_input_row", &conv_backward_input_row, py::arg("dy"), py::arg("w"), py::arg("padding"), py::arg("m"));
+  m.def("bias_gradient", &bias_gradient, py::arg("dy"));
   m.def("version", []() { return std::string(wc_version()); });
 }

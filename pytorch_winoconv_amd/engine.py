@@ -334,7 +334,10 @@ def check_u(desc, U):
 def transform_filter(w, x_shape, stride=1, padding=0, m=2, whole_kernel=False, stacked=None, direct=None, row=False):
     """Transformed filter U for later calls of conv_forward(..., U=U) with the same options."""
     _require_gpu(w)
-    desc = make_desc(x_shape, w.shape, w.dtype, stride, padding, m, 0, whole_kernel, stacked, direct=direct, row=row)
+    if row and x_shape[0] > 0:                  # the module's call, once in a training step: its descriptor is kept
+        desc = _forward_setup(tuple(x_shape), tuple(w.shape), w.dtype, stride, padding, m, 0, whole_kernel, stacked, direct=direct, row=row)[0]
+    else:
+        desc = make_desc(x_shape, w.shape, w.dtype, stride, padding, m, 0, whole_kernel, stacked, direct=direct, row=row)
     if desc.row:
         n = ctypes.c_size_t()
         check(_lib.load().wc_conv_u_elems(ctypes.byref(desc), ctypes.byref(n)))
@@ -468,8 +471,10 @@ def _forward_setup(x_shape, w_shape, dtype, stride, padding, m, chunk_images, wh
 def conv_backward_weight(x, dy, w_shape, stride=1, padding=0, m=2, whole_kernel=False, stacked=None):
     """Gradient of sum(y * dy) with respect to the filter of conv_forward(x, w, ...): a tensor of
     shape `w_shape` (K, C, [kD,] kH, kW) in x's dtype.  The reference has no backward pass; this one
-    works in the transform domain (see include/winoconv.h).  `stacked` as in conv_forward."""
+    works in the transform domain, or directly where that is faster (see include/winoconv.h).  `stacked` as in conv_forward."""
     _require_gpu(x, dy)
+    if USE_EXT and stacked is None and not whole_kernel and x.shape[0] > 0:
+        return _ext.conv_backward_weight(x, dy, tuple(w_shape), stride, padding, m)
     stacked = _stack(stacked, x.dtype, x.dim() - 2, whole_kernel, w_shape, stride, m)
     if stacked == 2:
         stacked = True               # the weight gradient has no shared-input form: pieces stacked with their own V
@@ -500,10 +505,12 @@ def bias_gradient(dy):
     _require_gpu(dy)
     lib = _lib.load()
     K = dy.shape[1]
-    db = torch.empty(K, dtype=dy.dtype, device=dy.device)
     rows = dy.numel() // max(K, 1)
     if rows == 0:
-        return db.zero_()
+        return torch.zeros(K, dtype=dy.dtype, device=dy.device)
+    if USE_EXT:
+        return _ext.bias_gradient(dy)
+    db = torch.empty(K, dtype=dy.dtype, device=dy.device)
     dy_cl = channel_last(dy)
     nbytes = ctypes.c_size_t()
     check(lib.wc_bias_gradient_workspace_bytes(rows, K, _DTYPES[dy.dtype], ctypes.byref(nbytes)))
@@ -555,14 +562,16 @@ def conv_backward_input(dy, w, x_spatial, stride=1, padding=0, m=2):
         dy = dyu
     elif stride != 1:
         raise NotImplementedError("stride must be 1 or 2")
-    w_rot = w.flip(tuple(range(2, 2 + nd))).transpose(0, 1)
     # output tile: the caller's, except where the 3-D tile 4 does not exist, for stride 2, where
     # three quarters of the zero-filled dy are zeros and the F(4,r) rounding error is not averaged
     # down (fp16: 2.6e-2 of the gradient's range against 2e-3 with tile 2), and for fewer than 8
     # output channels, where the sum is too short to average it down either (fp16, K = 1: up to
     # 3e-2 with tile 4, 1e-3 with tile 2)
     mm = m if (stride == 1 and w.shape[0] >= 8 and (m == 2 or nd == 2 or ks == (3, 3, 3))) else 2
-    dx = conv_forward(dy, w_rot, None, 1, tuple(k - 1 - p for k, p in zip(ks, pads)), mm, row=True)
+    pads = tuple(k - 1 - p for k, p in zip(ks, pads))
+    dx = _ext.conv_backward_input_row(dy, w, pads, mm) if USE_EXT and dy.shape[0] > 0 else None
+    if dx is None:
+        dx = conv_forward(dy, w.flip(tuple(range(2, 2 + nd))).transpose(0, 1), None, 1, pads, mm, row=True)
     if tuple(dx.shape[2:]) != want:
         raise ValueError("dy of shape %r does not belong to an input of extent %r" % (tuple(dy.shape), want))
     return dx
