@@ -176,22 +176,28 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
     loff[i] = row * LDS_STRIDE + (lpart ^ swizzle(row)) * EPC;
   }
 
-  Chunk16 regs[NLOAD];
+  // The direct form requests a reduction block two stages before it is multiplied where the registers allow it: a stage of
+  // the smaller tiles is over before its pixels, behind their bounds checks, are there (fp16 stride 2, us, one stage | two:
+  // N=1 128 -> 128, 56x56 16.5 | 12.7; N=2 256 -> 512, 15x17 30 | 22; N=64 256 -> 512, 28x28 55 | 51; the 256 x 128 tile
+  // spills that way, N=32 128 -> 128, 112x112 63 | 77).
+  constexpr int AHEAD = DIRECT && sizeof(T) == 2 && WM * WN <= 4 ? 2 : 1;
+  Chunk16 regs[AHEAD][NLOAD];
   // `vshift`: what the V operand has jumped by at reduction block kt (rows i < BM / RPP are V's)
   int tap_y = 0, tap_x = 0, tap_cb = 0;             // direct form: the tap and channel block of the next load
-  auto gload = [&](int kt, long long vshift) {
+  auto gload = [&](auto set_c, int kt, long long vshift) {
+    constexpr int set = decltype(set_c)::value;
 #pragma unroll
     for (int i = 0; i < NLOAD; ++i) {
       if constexpr (DIRECT) {
         if (i < BM / RPP) {
           const int j = i < BM / RPP ? i : 0;
           const bool inside = (unsigned)(iy0[j] + tap_y) < (unsigned)g.H && (unsigned)(ix0[j] + tap_x) < (unsigned)g.W;
-          regs[i] = Chunk16{0u, 0u, 0u, 0u};
-          if (inside) regs[i] = *reinterpret_cast<const Chunk16*>(gptr[i] + kt * BK + vshift);
+          regs[set][i] = Chunk16{0u, 0u, 0u, 0u};
+          if (inside) regs[set][i] = *reinterpret_cast<const Chunk16*>(gptr[i] + kt * BK + vshift);
           continue;
         }
       }
-      regs[i] = *reinterpret_cast<const Chunk16*>(gptr[i] + kt * BK + (SHIFT && i < BM / RPP ? vshift : 0));
+      regs[set][i] = *reinterpret_cast<const Chunk16*>(gptr[i] + kt * BK + (SHIFT && i < BM / RPP ? vshift : 0));
     }
     if constexpr (DIRECT) {
       if (++tap_cb == g.cblocks) {
@@ -200,9 +206,9 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
       }
     }
   };
-  auto lstore = [&](int buf) {
+  auto lstore = [&](auto set_c, int buf) {
 #pragma unroll
-    for (int i = 0; i < NLOAD; ++i) *reinterpret_cast<Chunk16*>(lds + buf * STAGE + loff[i]) = regs[i];
+    for (int i = 0; i < NLOAD; ++i) *reinterpret_cast<Chunk16*>(lds + buf * STAGE + loff[i]) = regs[decltype(set_c)::value][i];
   };
 
   const int lane = tid & 63, wave = tid >> 6;
@@ -228,11 +234,7 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
   const int nk = g.Cp / BK;
   long long vshift = 0;
   int run_left = SHIFT ? g.run_blocks : 0, plane_left = SHIFT ? g.plane_runs : 0;
-  gload(0, 0);
-  lstore(0);
-  __syncthreads();
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
+  auto next_block = [&]() {                        // on to the V operand's place for the next reduction block
     if constexpr (SHIFT) {
       if (--run_left == 0) {
         vshift += g.jump;
@@ -240,7 +242,17 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
         if (--plane_left == 0) { vshift += g.jump2; plane_left = g.plane_runs; }
       }
     }
-    if (kt + 1 < nk) gload(kt + 1, vshift);
+  };
+  gload(ic<0>{}, 0, 0);
+  lstore(ic<0>{}, 0);
+  if constexpr (AHEAD == 2) {
+    if (nk > 1) { next_block(); gload(ic<1>{}, 1, vshift); }
+  }
+  __syncthreads();
+  auto stage = [&](int kt, auto set_c) {           // set_c: kt % AHEAD
+    constexpr int set = decltype(set_c)::value;
+    const int cur = kt & 1;
+    if (kt + AHEAD < nk) { next_block(); gload(set_c, kt + AHEAD, vshift); }
     const T* st = lds + cur * STAGE;
     // fragments of step kk+1 are read from LDS while the MFMAs of step kk run
     constexpr int KK = BK / MF::kstep;
@@ -265,8 +277,14 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
         for (int j = 0; j < WN; ++j) acc[i][j] = MF::run(wf[kk & 1][j], xf[kk & 1][i], acc[i][j]);
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (kt + 1 < nk) lstore(cur ^ 1);
+    if (kt + 1 < nk) lstore(ic<AHEAD == 2 ? 1 - set : 0>{}, cur ^ 1);
     __syncthreads();
+  };
+  for (int kt = 0; kt < nk; kt += AHEAD) {
+    stage(kt, ic<0>{});
+    if constexpr (AHEAD == 2) {
+      if (kt + 1 < nk) stage(kt + 1, ic<1>{});
+    }
   }
 
   // Epilogue through LDS so that global stores are whole rows.  Accumulator (i, j), register
@@ -830,7 +848,7 @@ int fold_filter_w(const void* U, void* Uw, int K, int Cp, int dtype, void* strea
 
 // Tiles of the direct form, chosen like those of the shifted operand.
 template <typename T>
-static GemmConfig choose_direct(int P, int K) {
+static GemmConfig choose_direct(int P, int K, int reduction) {
   constexpr int BK = sizeof(T) == 4 ? 16 : 32;
   auto blocks = [&](const GemmConfig& c) { return (long long)ceil_div(P, c.bm) * ceil_div(K, c.bn); };
   switch (test_gemm_config()) {                       // wc_test_gemm_override: a tile shape forced by a test
@@ -853,7 +871,10 @@ static GemmConfig choose_direct(int P, int K) {
   }
   if (K > 64) {
     GemmConfig big = make_config<T, 4, 2, BK, 2, 2, true, true>();   // 256 x 128, four wavefronts
-    if (blocks(big) >= kCus) return big;
+    // a reduction of up to 24 blocks is mostly start and write-out, which 128 x 128 tiles, four to a CU and their loads two
+    // stages ahead, overlap better: 128 x 128 | 256 x 128, 64 -> 256 channels 1x1, N=64 56x56 28 | 34; 64 -> 128 3x3 at
+    // stride 2, N=64 112x112 60 | 62; 128 -> 128, N=32 64 | 58
+    if (reduction > 768 && blocks(big) >= kCus) return big;
     GemmConfig mid = make_config<T, 2, 2, BK, 2, 2, true, true>();   // 128 x 128
     if (blocks(mid) >= kCus) return mid;
   }
@@ -885,7 +906,7 @@ int gemm_direct_conv(const void* x, const void* U, const void* bias, void* y, in
       return direct_rows_conv(x, U, bias, y, N, H, W, C, K, kh, kw, stride, pad_h, pad_w, oH, oW, dtype, stream, o_step, o_y0,
                               o_x0, o_H, o_W);
   }
-  GemmConfig c = dispatch_dtype(dtype, [&](auto t) { return choose_direct<decltype(t)>((int)P, K); });
+  GemmConfig c = dispatch_dtype(dtype, [&](auto t) { return choose_direct<decltype(t)>((int)P, K, kh * kw * C); });
   GemmArgs g;
   g.V = x; g.U = U; g.M = y; g.bias = bias;
   g.P = (int)P; g.K = K; g.ldm = K;
