@@ -49,6 +49,7 @@ struct TapsArgs {
   const void* x; const void* dy; float* part;
   int D, H, W, C, K;               // x (N, D, H, W, C), dy (N, oD, oH, oW, K)
   int oD, oH, oW, pd, ph, pw;
+  long long x_elems, dy_elems;
   int Hp, Wp;                      // oH + 2, oW + 2
   FastDiv f_wp, f_hp, f_od;
   int total;                       // positions
@@ -89,9 +90,20 @@ void taps_kernel(TapsArgs a) {
     plane = fast_div(row, a.f_hp);
     h = row - plane * a.Hp;
   };
-  auto load16 = [&](const T* p, bool ok) {          // rows of a view start at any multiple of the element size
+  // rows start at any multiple of the element size; beyond the last channel of a position come the next one's, in columns
+  // that nobody writes out, and beyond the last position the tensor ends
+  auto load16 = [&](const T* p, const T* end, bool ok) {
     u32x4 v = zero;
-    if (ok) __builtin_memcpy(&v, p, 16);
+    if (ok) {
+      if (p + 8 <= end) {
+        __builtin_memcpy(&v, p, 16);
+      } else {
+        Pack<T, 8> o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o.v[e] = p + e < end ? p[e] : T(0);
+        v = __builtin_bit_cast(u32x4, o);
+      }
+    }
     return v;
   };
   auto load_x = [&](int pos, int c) {
@@ -100,13 +112,13 @@ void taps_kernel(TapsArgs a) {
     const int n = fast_div(plane, a.f_od), d = plane - n * a.oD + kd - a.pd;
     h -= a.ph; w -= a.pw;
     const bool ok = pos < a.total && c0 + c < a.C && (unsigned)d < (unsigned)a.D && (unsigned)h < (unsigned)a.H && (unsigned)w < (unsigned)a.W;
-    return load16(xp + ((((long long)n * a.D + d) * a.H + h) * a.W + w) * a.C + c, ok);
+    return load16(xp + ((((long long)n * a.D + d) * a.H + h) * a.W + w) * a.C + c, static_cast<const T*>(a.x) + a.x_elems, ok);
   };
   auto load_dy = [&](int pos, int k) {
     int plane, h, w;
     place(pos, plane, h, w);
     const bool ok = pos < q_end && k0 + k < a.K && h < a.oH && w < a.oW;
-    return load16(dp + (((long long)plane * a.oH + h) * a.oW + w) * a.K + k, ok);
+    return load16(dp + (((long long)plane * a.oH + h) * a.oW + w) * a.K + k, static_cast<const T*>(a.dy) + a.dy_elems, ok);
   };
 
   u32x4 reg[NU];
@@ -263,7 +275,7 @@ int taps_parts(int steps, int tiles, int kg) {
 }
 
 bool taps_plan(const wc_conv_desc* d, const int out[3], TapsPlan* p) {
-  if (d->dtype == WC_F32 || d->stride != 1 || d->whole_kernel || d->C % 8 != 0 || d->K % 8 != 0) return false;
+  if (d->dtype == WC_F32 || d->stride != 1 || d->whole_kernel) return false;
   if (d->kernel[1] != 3 || d->kernel[2] != 3 || (d->kernel[0] != 3 && d->kernel[0] != 1)) return false;
   const long long Wp = out[2] + 2, total = (long long)d->N * out[0] * (out[1] + 2) * Wp;
   if (Wp > 1024 || total >= (1ll << 31) - 4096) return false;       // positions stay ints, with a run's halo beyond the end
@@ -287,6 +299,7 @@ int launch_taps(const wc_conv_desc* d, const int out[3], const TapsPlan& p, cons
   a.x = x; a.dy = dy; a.part = part;
   a.D = d->in[0]; a.H = d->in[1]; a.W = d->in[2]; a.C = d->C; a.K = d->K;
   a.oD = out[0]; a.oH = out[1]; a.oW = out[2]; a.pd = d->pad[0]; a.ph = d->pad[1]; a.pw = d->pad[2];
+  a.x_elems = (long long)d->N * a.D * a.H * a.W * a.C; a.dy_elems = (long long)d->N * a.oD * a.oH * a.oW * a.K;
   a.Hp = a.oH + 2; a.Wp = a.oW + 2;
   a.f_wp = make_fast_div(a.Wp); a.f_hp = make_fast_div(a.Hp); a.f_od = make_fast_div(a.oD);
   a.total = p.total; a.part_steps = p.part_steps; a.halo = p.halo; a.ring = p.ring;
@@ -312,13 +325,14 @@ int launch_taps(const wc_conv_desc* d, const int out[3], const TapsPlan& p, cons
 // 119 | 72; N=64 256 -> 256, 14x14 45 | 50 | 49; N=1 128 -> 128, 28x28 15 | 20 | 21.  F(4,3) multiplies a quarter as much
 // and its traffic grows with C + K, the products here with C K (padded to tiles), so it is ahead on wide layers: 256 -> 256,
 // 56x56 257 | 420 | 275; 512 -> 512, 28x28 266 | 307 | 240, 14x14 52 | 60 | 54, N=64 7x7 55 | 62 | 53; 72 -> 136, N=30
-// 20x20 36 | 40 | 32.  Small problems are launches and latency: two of them here, six there (512 -> 512, N=1 7x7 28 | 39 | 48).
+// 20x20 33 | 39 | 32; 100 -> 150, N=64 28x28 56 | 65 | 53, against F(2,3) alone still ahead: 50 -> 64, N=32 56x56 32 | 71; 3 -> 64,
+// N=64 112x112 106 | 334; 45 -> 77, N=2 8x28x28 33 | 61.  Small problems are launches and latency: two of them here, six there (512 -> 512, N=1 7x7 28 | 39 | 48).
 bool taps_gradient_fits(const wc_conv_desc* d, const int out[3], size_t* workspace_bytes) {
   TapsPlan p;
   if (test_gemm_config() == 20 || !taps_plan(d, out, &p)) return false;
   if (d->ndim == 2 && d->m == 4 && (long long)p.steps * p.tiles > 2560) {
     const long long padded = (long long)ceil_div(d->K, 64 * p.kg) * 64 * p.kg * ceil_div(d->C, 64) * 64;
-    if (padded > 256 * 256 || padded * 5 > 12ll * d->C * d->K) return false;
+    if (padded > 256 * 256 || padded * 5 > 8ll * d->C * d->K) return false;
   }
   *workspace_bytes = (size_t)p.parts * p.tiles * (p.kg == 2 ? taps_tile_floats<2>() : taps_tile_floats<1>()) * 4;
   return true;
@@ -327,7 +341,7 @@ bool taps_gradient_fits(const wc_conv_desc* d, const int out[3], size_t* workspa
 int taps_gradient(const wc_conv_desc* d, const int out[3], const void* x, const void* dy, void* dw,
                   const int64_t dw_strides[5], float* part, void* stream) {
   TapsPlan p;
-  WC_CHECK_ARG(taps_plan(d, out, &p), "tap form of the weight gradient: 16-bit, 3x3 or 3x3x3, stride 1, channels multiples of 8");
+  WC_CHECK_ARG(taps_plan(d, out, &p), "tap form of the weight gradient: 16-bit, 3x3 or 3x3x3, stride 1");
   return dispatch_dtype(d->dtype, [&](auto t) -> int {
     using T = decltype(t);
     if constexpr (sizeof(T) == 2) {

@@ -18,6 +18,7 @@ CASES = [
     ((1, 8, 1, 1), 8, 1),
     ((2, 8, 5, 6), 16, 1),
     ((3, 72, 9, 17), 136, 1),                                # remainders of channels on both sides, three blocks of 64
+    ((1, 1, 1, 1), 1, 1), ((2, 7, 5, 6), 13, 1), ((3, 75, 9, 17), 133, 1), ((1, 3, 4, 3, 9), 5, 1),   # loads that cross the last channel
     ((2, 40, 7, 7), 72, 0), ((2, 64, 30, 50), 64, (2, 0)),   # other paddings
     ((1, 16, 4, 253), 24, 1), ((1, 16, 3, 254), 24, 1),      # the widest rows of the ring, and rows it does not hold
     ((5, 128, 31, 31), 256, 1),                              # several parts, the last one short
