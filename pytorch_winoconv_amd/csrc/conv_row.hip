@@ -103,8 +103,8 @@ constexpr int row_lds_bytes() {
   return v > ex ? (v > part ? v : part) : (ex > part ? ex : part);
 }
 
-// KT: rows of y that are no multiple of 16 bytes
-template <typename T, int KD, int KH, int KG, int TB, int S, int CS, bool KT>
+// KT: rows of y that are no multiple of 16 bytes.  STAY: a workgroup per CU that goes from box to box
+template <typename T, int KD, int KH, int KG, int TB, int S, int CS, bool STAY, bool KT>
 __global__ __launch_bounds__(128 * KG * CS) __attribute__((amdgpu_waves_per_eu(2, TB == 2 ? 2 : 3)))
 void row_conv_kernel(RowArgs a) {
   using Frag = typename MfmaRow<T>::Frag;
@@ -114,16 +114,24 @@ void row_conv_kernel(RowArgs a) {
   static_assert(RowItems<UN, NI>::ok(), "items of a step");
   static_assert(S * 4 % THREADS == 0 && Q % UD == 0, "whole units per thread, ring of three");
   extern __shared__ unsigned char lds_all[];
-  const int wg = xcd_remap(blockIdx.x, a.per_xcd);
-  if (wg >= a.n_kb * a.n_box) return;
-  int kb, box;
-  if (a.box_fast) { kb = wg / a.n_box; box = wg - kb * a.n_box; }
-  else { box = wg / a.n_kb; kb = wg - box * a.n_kb; }
-  const int b_w = box % a.n_w;
-  int q_ = box / a.n_w;
-  const int b_h = q_ % a.n_h; q_ /= a.n_h;
-  const int b_d = q_ % a.n_d;
-  const int n0 = q_ / a.n_d * a.bn, d0 = b_d * a.bd, h0 = b_h * a.bh, w0 = b_w * a.bw;
+  static_assert(!STAY || CS == 1, "shares end after their box");
+  // this XCD's boxes from the workgroup's own on; STAY: every (workgroups of the XCD)-th
+  int place = blockIdx.x / kXcds;
+  const int place0 = blockIdx.x % kXcds * a.per_xcd, places = min(a.per_xcd, a.n_kb * a.n_box - place0);
+  if (place >= places) return;
+  int kb, n0, d0, h0, w0;
+  auto go_to_box = [&]() {
+    const int wg = place0 + place;
+    int box;
+    if (a.box_fast) { kb = wg / a.n_box; box = wg - kb * a.n_box; }
+    else { box = wg / a.n_kb; kb = wg - box * a.n_kb; }
+    const int b_w = box % a.n_w;
+    int q_ = box / a.n_w;
+    const int b_h = q_ % a.n_h; q_ /= a.n_h;
+    const int b_d = q_ % a.n_d;
+    n0 = q_ / a.n_d * a.bn; d0 = b_d * a.bd; h0 = b_h * a.bh; w0 = b_w * a.bw;
+  };
+  go_to_box();
   const int sd = a.bd + KD - 1, sh = a.bh + KH - 1;
 
   const int lane = threadIdx.x & 63, wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -137,7 +145,7 @@ void row_conv_kernel(RowArgs a) {
   // ---- filter fragments: a ring of three groups (row tap, half of a channel block) of three elements
   const int n_groups = a.steps * Q, k_blocks = (a.K + 31) / 32;
   const int u_lane = lane * 16 + tg * 3072;
-  const int u_base = min(kb * KG + kg, k_blocks - 1) * n_groups * 6144;
+  int u_base = 0;
   u32x4 uf[UD][3];
   auto load_u = [&](int slot, int group, int t) {
     uf[slot][t] = __builtin_amdgcn_raw_buffer_load_b128(udesc, u_lane + t * 1024, u_base + min(step0 * Q + group, n_groups - 1) * 6144, 0);
@@ -146,19 +154,22 @@ void row_conv_kernel(RowArgs a) {
   // ---- input: units of (row of a tile, 8 channels)
   int xo[UN][6];
   u32x4 xr[UN][6];
+  auto find_x = [&]() {
 #pragma unroll
-  for (int i = 0; i < UN; ++i) {
-    const int u = tid + i * THREADS, g = u & 3;
-    int s = u >> 2;
-    const int in = fast_div(s, a.f_irow); s -= in * a.irow;
-    const int zd = fast_div(s, a.f_prow); s -= zd * a.prow;
-    const int zh = fast_div(s, a.f_bw), iw = s - zh * a.bw;
-    const int n = n0 + in, d = d0 + zd - a.pd, h = h0 + zh - a.ph, w = (w0 + iw) * 4 - a.pw;
-    const bool ok = in < a.bn && zd < sd && zh < sh && n < a.N && (unsigned)d < (unsigned)a.D && (unsigned)h < (unsigned)a.H;
-    const int base = (((n * a.D + d) * a.H + h) * a.W + w) * a.C * 2 + g * 16;
+    for (int i = 0; i < UN; ++i) {
+      const int u = tid + i * THREADS, g = u & 3;
+      int s = u >> 2;
+      const int in = fast_div(s, a.f_irow); s -= in * a.irow;
+      const int zd = fast_div(s, a.f_prow); s -= zd * a.prow;
+      const int zh = fast_div(s, a.f_bw), iw = s - zh * a.bw;
+      const int n = n0 + in, d = d0 + zd - a.pd, h = h0 + zh - a.ph, w = (w0 + iw) * 4 - a.pw;
+      const bool ok = in < a.bn && zd < sd && zh < sh && n < a.N && (unsigned)d < (unsigned)a.D && (unsigned)h < (unsigned)a.H;
+      const int base = (((n * a.D + d) * a.H + h) * a.W + w) * a.C * 2 + g * 16;
 #pragma unroll
-    for (int j = 0; j < 6; ++j) xo[i][j] = ok && (unsigned)(w + j) < (unsigned)a.W ? base + j * a.C * 2 : (int)kOutside;
-  }
+      for (int j = 0; j < 6; ++j) xo[i][j] = ok && (unsigned)(w + j) < (unsigned)a.W ? base + j * a.C * 2 : (int)kOutside;
+    }
+  };
+  find_x();
   // the channel block is in the scalar offset; beyond the last channel of the last block lanes load zeros (cut_x)
   auto load_x = [&](int i, int j, int step) {
     xr[i][j] = __builtin_amdgcn_raw_buffer_load_b128(xdesc, xo[i][j], min(step0 + step, a.steps - 1) * 64, 0);
@@ -218,212 +229,232 @@ void row_conv_kernel(RowArgs a) {
   }
 
   f32x16 acc[3][TB];
-#pragma unroll
-  for (int t = 0; t < 3; ++t)
-#pragma unroll
-    for (int b = 0; b < TB; ++b)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[t][b][e] = 0.f;
-
   cut_x(0);
 #pragma unroll
   for (int i = 0; i < UN; ++i)
 #pragma unroll
     for (int j = 0; j < 6; ++j) load_x(i, j, 0);
-  cut_x(1);
-  // Loads return in order and the compiler counts them over both ways into the loop: the order of the loads here is that of
-  // a step, the input of step 1 ahead of the filter's later groups, or every step would wait for its last loads.
-  auto load_u_groups = [&](int from, int to) {
+  for (;;) {                             // a box (not STAY: the only one); its first input is under way
 #pragma unroll
-    for (int i = from; i < to; ++i) load_u(i / 3, i / 3, i % 3);
-  };
-  load_u_groups(0, UD * 3 / 2);
-  static_for<0, 8 * UN>([&](auto h_c) { transform_channel(ic<decltype(h_c)::value / 8>{}, ic<decltype(h_c)::value % 8>{}); });
-#pragma unroll
-  for (int i = 0; i < UN; ++i) {
-#pragma unroll
-    for (int t = 0; t < 6; ++t) store_v(i, t, 0);
-#pragma unroll
-    for (int j = 0; j < 6; ++j) load_x(i, j, 1);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  load_u_groups(UD * 3 / 2, UD * 3 - 1);           // the last one: in item 0
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-
-  for (int step = 0; step < a.local_steps; ++step) {
-    const int cur = (step & 1) * BUF + tg * 3 * TS;
-    if constexpr (R > 3) {               // keeps the compiler from holding the addresses of all taps in registers
-#pragma unroll
-      for (int b = 0; b < TB; ++b) asm volatile("" : "+v"(vo[b]));
-    }
-    cut_x(step + 2);
-    u32x4 vf[VD][TB];
-    auto load_v = [&](int item) {                  // element item % 3 of group item / 3
-      const int q = item / 3, r = q >> 1, off = (r / KH) * a.prow + r % KH * a.bw;
+    for (int t = 0; t < 3; ++t)
 #pragma unroll
       for (int b = 0; b < TB; ++b)
-        vf[item % VD][b] = *reinterpret_cast<const u32x4*>(lds + cur + v_offset(vo[b] + off, (lane >> 5) + (q & 1) * 2) + item % 3 * TS);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[t][b][e] = 0.f;
+    u_base = min(kb * KG + kg, k_blocks - 1) * n_groups * 6144;
+    cut_x(1);
+    // Loads return in order and the compiler counts them over both ways into the loop: the order of the loads here is that of
+    // a step, the input of step 1 ahead of the filter's later groups, or every step would wait for its last loads.
+    auto load_u_groups = [&](int from, int to) {
+#pragma unroll
+      for (int i = from; i < to; ++i) load_u(i / 3, i / 3, i % 3);
     };
-    // A step is a stream of items, one element of one group each.  The loads that refill the rings, the transform of the
-    // next step's input, its stores to LDS and the loads of the step after are dealt out over the items and, in an item,
-    // over its MFMAs: a wavefront issues in order, and what stands between two MFMAs beyond the 32 cycles of the first
-    // leaves the matrix core idle.
+    load_u_groups(0, UD * 3 / 2);
+    static_for<0, 8 * UN>([&](auto h_c) { transform_channel(ic<decltype(h_c)::value / 8>{}, ic<decltype(h_c)::value % 8>{}); });
 #pragma unroll
-    for (int i = 0; i < VD - 1; ++i) load_v(i);
-    static_for<0, NI>([&](auto item_c) {
-      constexpr int item = decltype(item_c)::value, q = item / 3, t = item % 3, last = (item + NI - 1) % NI;
-      constexpr int channels = RowItems<UN, NI>::channels(item), moves = RowItems<UN, NI>::moves(item);
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (item + VD - 1 < NI) load_v(item + VD - 1);
+    for (int i = 0; i < UN; ++i) {
 #pragma unroll
-      for (int b = 0; b < TB; ++b)
-        acc[t][b] = MfmaRow<T>::run(__builtin_bit_cast(Frag, uf[q % UD][t]), __builtin_bit_cast(Frag, vf[item % VD][b]), acc[t][b]);
-      // the ring slot of the item before: its fragment of UD groups later
-      load_u(last / 3 % UD, step * Q + last / 3 + UD - (item == 0 ? Q : 0), last % 3);
-      static_for<0, channels>([&](auto n_c) {
-        constexpr int h = RowItems<UN, NI>::first_channel(item) + decltype(n_c)::value;
-        transform_channel(ic<h / 8>{}, ic<h % 8>{});
-      });
-      static_for<0, moves>([&](auto n_c) {
-        constexpr int v = RowItems<UN, NI>::first_move(item) + decltype(n_c)::value;
-        store_v(v / 6, v % 6, (step + 1) & 1);
-        load_x(v / 6, v % 6, step + 2);
-      });
-      __builtin_amdgcn_sched_group_barrier(0x100, TB, 0);
+      for (int t = 0; t < 6; ++t) store_v(i, t, 0);
 #pragma unroll
-      for (int g = 0; g < TB; ++g) {
-        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x2, (14 * channels + 3 + TB - 1) / TB, 0);
-        __builtin_amdgcn_sched_group_barrier(0x200, (moves + TB - 1) / TB, 0);
-        __builtin_amdgcn_sched_group_barrier(0x20, (moves + TB) / TB, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    });
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-  }
-
-  if constexpr (CS > 1) {                // the shares' sums come together in the first share's registers
-    f32x4* part = reinterpret_cast<f32x4*>(lds_all) + lane;
-    constexpr int NV = 3 * TB * 4;
-    if (cs > 0) {
-#pragma unroll
-      for (int v = 0; v < NV; ++v) {
-        const f32x16& c = acc[v / 4 % 3][v / 12];
-        f32x4 o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = c[v % 4 * 4 + e];
-        part[(((cs - 1) * 2 * KG + wave) * NV + v) * 64] = o;
-      }
+      for (int j = 0; j < 6; ++j) load_x(i, j, 1);
     }
+    __builtin_amdgcn_sched_barrier(0);
+    load_u_groups(UD * 3 / 2, UD * 3 - 1);           // the last one: in item 0
+    __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
-    if (cs == 0) {
+
+    for (int step = 0; step < a.local_steps; ++step) {
+      const int cur = (step & 1) * BUF + tg * 3 * TS;
+      if constexpr (R > 3) {               // keeps the compiler from holding the addresses of all taps in registers
 #pragma unroll
-      for (int o = 0; o < CS - 1; ++o)
+        for (int b = 0; b < TB; ++b) asm volatile("" : "+v"(vo[b]));
+      }
+      cut_x(step + 2);
+      u32x4 vf[VD][TB];
+      auto load_v = [&](int item) {                  // element item % 3 of group item / 3
+        const int q = item / 3, r = q >> 1, off = (r / KH) * a.prow + r % KH * a.bw;
+#pragma unroll
+        for (int b = 0; b < TB; ++b)
+          vf[item % VD][b] = *reinterpret_cast<const u32x4*>(lds + cur + v_offset(vo[b] + off, (lane >> 5) + (q & 1) * 2) + item % 3 * TS);
+      };
+      // A step is a stream of items, one element of one group each.  The loads that refill the rings, the transform of the
+      // next step's input, its stores to LDS and the loads of the step after are dealt out over the items and, in an item,
+      // over its MFMAs: a wavefront issues in order, and what stands between two MFMAs beyond the 32 cycles of the first
+      // leaves the matrix core idle.
+#pragma unroll
+      for (int i = 0; i < VD - 1; ++i) load_v(i);
+      static_for<0, NI>([&](auto item_c) {
+        constexpr int item = decltype(item_c)::value, q = item / 3, t = item % 3, last = (item + NI - 1) % NI;
+        constexpr int channels = RowItems<UN, NI>::channels(item), moves = RowItems<UN, NI>::moves(item);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (item + VD - 1 < NI) load_v(item + VD - 1);
+#pragma unroll
+        for (int b = 0; b < TB; ++b)
+          acc[t][b] = MfmaRow<T>::run(__builtin_bit_cast(Frag, uf[q % UD][t]), __builtin_bit_cast(Frag, vf[item % VD][b]), acc[t][b]);
+        // the ring slot of the item before: its fragment of UD groups later
+        load_u(last / 3 % UD, step * Q + last / 3 + UD - (item == 0 ? Q : 0), last % 3);
+        static_for<0, channels>([&](auto n_c) {
+          constexpr int h = RowItems<UN, NI>::first_channel(item) + decltype(n_c)::value;
+          transform_channel(ic<h / 8>{}, ic<h % 8>{});
+        });
+        static_for<0, moves>([&](auto n_c) {
+          constexpr int v = RowItems<UN, NI>::first_move(item) + decltype(n_c)::value;
+          store_v(v / 6, v % 6, (step + 1) & 1);
+          load_x(v / 6, v % 6, step + 2);
+        });
+        __builtin_amdgcn_sched_group_barrier(0x100, TB, 0);
+#pragma unroll
+        for (int g = 0; g < TB; ++g) {
+          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x2, (14 * channels + 3 + TB - 1) / TB, 0);
+          __builtin_amdgcn_sched_group_barrier(0x200, (moves + TB - 1) / TB, 0);
+          __builtin_amdgcn_sched_group_barrier(0x20, (moves + TB) / TB, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+    }
+
+    if constexpr (CS > 1) {                // the shares' sums come together in the first share's registers
+      f32x4* part = reinterpret_cast<f32x4*>(lds_all) + lane;
+      constexpr int NV = 3 * TB * 4;
+      if (cs > 0) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-          const f32x4 p = part[((o * 2 * KG + wave) * NV + v) * 64];
+          const f32x16& c = acc[v / 4 % 3][v / 12];
+          f32x4 o;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[v / 4 % 3][v / 12][v % 4 * 4 + e] += p[e];
+          for (int e = 0; e < 4; ++e) o[e] = c[v % 4 * 4 + e];
+          part[(((cs - 1) * 2 * KG + wave) * NV + v) * 64] = o;
         }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    if (cs > 0) {                        // the barrier of the output transform below
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
-      return;
+      if (cs == 0) {
+#pragma unroll
+        for (int o = 0; o < CS - 1; ++o)
+#pragma unroll
+          for (int v = 0; v < NV; ++v) {
+            const f32x4 p = part[((o * 2 * KG + wave) * NV + v) * 64];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[v / 4 % 3][v / 12][v % 4 * 4 + e] += p[e];
+          }
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      if (cs > 0) {                        // the barrier of the output transform below
+        __builtin_amdgcn_s_barrier();
+        return;
+      }
     }
-  }
 
-  // ---- output transform.  Elements 0 to 2 (points 0, a, -a) are with the first half of the wavefronts, 3 to 5 (1/a,
-  // -1/a, infinity) with the second; each half finishes one half of the outputs (two blocks: a block each; one block: half
-  // of its channels each) and hands three sums of the other half over through LDS.
-  // Each wavefront reduces its three elements to (x, s, d): the element at 0 or infinity, and sum and difference of the pair.
-  constexpr int NC = TB;              // chunks of 8 accumulator registers a wavefront finishes
-  auto finish = [&](auto tg_c) {
-    constexpr int TG = decltype(tg_c)::value, X = TG == 0 ? 0 : 2, P0 = TG == 0 ? 1 : 0;
-    // chunk c of a half: tile block, first register
-    auto tile_block = [](int half, int c) { return (half * TB + c) / 2; };
-    auto first = [](int half, int c) { return (half * TB + c) % 2 * 8; };
-    auto reg = [&](int t, int half, int c, int e) -> float { return acc[t][tile_block(half, c)][first(half, c) + e]; };
-    f32x4* ex = reinterpret_cast<f32x4*>(lds) + (size_t)(TG * KG + kg) * 6 * NC * 64 + lane;
-    const f32x4* other = reinterpret_cast<const f32x4*>(lds) + (size_t)((1 - TG) * KG + kg) * 6 * NC * 64 + lane;
+    // ---- output transform.  Elements 0 to 2 (points 0, a, -a) are with the first half of the wavefronts, 3 to 5 (1/a,
+    // -1/a, infinity) with the second; each half finishes one half of the outputs (two blocks: a block each; one block: half
+    // of its channels each) and hands three sums of the other half over through LDS.
+    // Each wavefront reduces its three elements to (x, s, d): the element at 0 or infinity, and sum and difference of the pair.
+    const int at_kb = kb, at_n = n0, at_d = d0, at_h = h0, at_w = w0;
+    bool more = false;
+    if constexpr (STAY) {                  // the next box's input comes while this one is written out
+      place += gridDim.x / kXcds;
+      more = place < places;
+      if (more) {
+        go_to_box();
+        find_x();
+        cut_x(0);
 #pragma unroll
-    for (int c = 0; c < NC; ++c)
+        for (int i = 0; i < UN; ++i)
 #pragma unroll
-      for (int i4 = 0; i4 < 2; ++i4) {
-        f32x4 x, s, d;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float p = reg(P0, 1 - TG, c, i4 * 4 + e), m = reg(P0 + 1, 1 - TG, c, i4 * 4 + e);
-          x[e] = reg(X, 1 - TG, c, i4 * 4 + e); s[e] = p + m; d[e] = p - m;
-        }
-        ex[((c * 2 + i4) * 3 + 0) * 64] = x; ex[((c * 2 + i4) * 3 + 1) * 64] = s; ex[((c * 2 + i4) * 3 + 2) * 64] = d;
+          for (int j = 0; j < 6; ++j) load_x(i, j, 0);
       }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
+    }
+    constexpr int NC = TB;              // chunks of 8 accumulator registers a wavefront finishes
+    auto finish = [&](auto tg_c) {
+      constexpr int TG = decltype(tg_c)::value, X = TG == 0 ? 0 : 2, P0 = TG == 0 ? 1 : 0;
+      // chunk c of a half: tile block, first register
+      auto tile_block = [](int half, int c) { return (half * TB + c) / 2; };
+      auto first = [](int half, int c) { return (half * TB + c) % 2 * 8; };
+      auto reg = [&](int t, int half, int c, int e) -> float { return acc[t][tile_block(half, c)][first(half, c) + e]; };
+      f32x4* ex = reinterpret_cast<f32x4*>(lds) + (size_t)(TG * KG + kg) * 6 * NC * 64 + lane;
+      const f32x4* other = reinterpret_cast<const f32x4*>(lds) + (size_t)((1 - TG) * KG + kg) * 6 * NC * 64 + lane;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const int k0 = (kb * KG + kg) * 32 + (lane >> 5) * 16 + first(TG, c);
-      const int ti = tile_block(TG, c) * 32 + (lane & 31);
-      int iw, ih, id, in;
-      tile_of(ti, iw, ih, id, in);
-      const int n = n0 + in, od = d0 + id, oh = h0 + ih, ow = (w0 + iw) * 4;
-      const bool ok = ti < a.bn * a.bd * a.bh * a.bw && n < a.N && od < a.oD && oh < a.oH && k0 < a.K;
-      T* const yp = static_cast<T*>(a.y) + ((((size_t)n * a.oD + od) * a.oH + oh) * a.oW + ow) * a.K + k0;
-      const T* const bp = static_cast<const T*>(a.bias);
-      Pack<T, 8> bv, o[4];
+      for (int c = 0; c < NC; ++c)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) bv.v[e] = T(0);
-      if (bp) {
-        if constexpr (!KT) {
-          __builtin_memcpy(&bv, bp + min(k0, a.K - 8), 16);
-        } else {
+        for (int i4 = 0; i4 < 2; ++i4) {
+          f32x4 x, s, d;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) bv.v[e] = bp[min(k0 + e, a.K - 1)];
+          for (int e = 0; e < 4; ++e) {
+            const float p = reg(P0, 1 - TG, c, i4 * 4 + e), m = reg(P0 + 1, 1 - TG, c, i4 * 4 + e);
+            x[e] = reg(X, 1 - TG, c, i4 * 4 + e); s[e] = p + m; d[e] = p - m;
+          }
+          ex[((c * 2 + i4) * 3 + 0) * 64] = x; ex[((c * 2 + i4) * 3 + 1) * 64] = s; ex[((c * 2 + i4) * 3 + 2) * 64] = d;
         }
-      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
 #pragma unroll
-      for (int i4 = 0; i4 < 2; ++i4) {
-        f32x4 g[3];
+      for (int c = 0; c < NC; ++c) {
+        const int k0 = (at_kb * KG + kg) * 32 + (lane >> 5) * 16 + first(TG, c);
+        const int ti = tile_block(TG, c) * 32 + (lane & 31);
+        int iw, ih, id, in;
+        tile_of(ti, iw, ih, id, in);
+        const int n = at_n + in, od = at_d + id, oh = at_h + ih, ow = (at_w + iw) * 4;
+        const bool ok = ti < a.bn * a.bd * a.bh * a.bw && n < a.N && od < a.oD && oh < a.oH && k0 < a.K;
+        T* const yp = static_cast<T*>(a.y) + ((((size_t)n * a.oD + od) * a.oH + oh) * a.oW + ow) * a.K + k0;
+        const T* const bp = static_cast<const T*>(a.bias);
+        Pack<T, 8> bv, o[4];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) g[j] = other[((c * 2 + i4) * 3 + j) * 64];
+        for (int e = 0; e < 8; ++e) bv.v[e] = T(0);
+        if (bp) {
+          if constexpr (!KT) {
+            __builtin_memcpy(&bv, bp + min(k0, a.K - 8), 16);
+          } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int i = i4 * 4 + e;
-          const float p = reg(P0, TG, c, i), m = reg(P0 + 1, TG, c, i), x = reg(X, TG, c, i), b = static_cast<float>(bv.v[i]);
-          const float m0 = TG == 0 ? x : g[0][e], mi = TG == 0 ? g[0][e] : x;
-          const float sa = TG == 0 ? p + m : g[1][e], sb = TG == 0 ? g[1][e] : p + m;
-          const float da = TG == 0 ? p - m : g[2][e], db = TG == 0 ? g[2][e] : p - m;
-          o[0].v[i] = static_cast<T>(m0 + sa + sb + b);
-          o[1].v[i] = static_cast<T>(__builtin_fmaf(kA, da, __builtin_fmaf(kB, db, b)));
-          o[2].v[i] = static_cast<T>(__builtin_fmaf(kA2, sa, __builtin_fmaf(kB2, sb, b)));
-          o[3].v[i] = static_cast<T>(__builtin_fmaf(kA * kA2, da, __builtin_fmaf(kB * kB2, db, mi + b)));
+            for (int e = 0; e < 8; ++e) bv.v[e] = bp[min(k0 + e, a.K - 1)];
+          }
         }
-      }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        T* const dst = yp + (size_t)i * a.K;
-        const bool in_row = ok && ow + i < a.oW;
-        if constexpr (!KT) {
-          if (in_row) *reinterpret_cast<u32x4*>(dst) = __builtin_bit_cast(u32x4, o[i]);
-        } else {
-          if (in_row && k0 + 8 <= a.K) {
-            __builtin_memcpy(dst, &o[i], 16);          // rows of y start at any multiple of the element size
-          } else if (in_row) {
+        for (int i4 = 0; i4 < 2; ++i4) {
+          f32x4 g[3];
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-              if (k0 + e < a.K) dst[e] = o[i].v[e];
+          for (int j = 0; j < 3; ++j) g[j] = other[((c * 2 + i4) * 3 + j) * 64];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int i = i4 * 4 + e;
+            const float p = reg(P0, TG, c, i), m = reg(P0 + 1, TG, c, i), x = reg(X, TG, c, i), b = static_cast<float>(bv.v[i]);
+            const float m0 = TG == 0 ? x : g[0][e], mi = TG == 0 ? g[0][e] : x;
+            const float sa = TG == 0 ? p + m : g[1][e], sb = TG == 0 ? g[1][e] : p + m;
+            const float da = TG == 0 ? p - m : g[2][e], db = TG == 0 ? g[2][e] : p - m;
+            o[0].v[i] = static_cast<T>(m0 + sa + sb + b);
+            o[1].v[i] = static_cast<T>(__builtin_fmaf(kA, da, __builtin_fmaf(kB, db, b)));
+            o[2].v[i] = static_cast<T>(__builtin_fmaf(kA2, sa, __builtin_fmaf(kB2, sb, b)));
+            o[3].v[i] = static_cast<T>(__builtin_fmaf(kA * kA2, da, __builtin_fmaf(kB * kB2, db, mi + b)));
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          T* const dst = yp + (size_t)i * a.K;
+          const bool in_row = ok && ow + i < a.oW;
+          if constexpr (!KT) {
+            if (in_row) *reinterpret_cast<u32x4*>(dst) = __builtin_bit_cast(u32x4, o[i]);
+          } else {
+            if (in_row && k0 + 8 <= a.K) {
+              __builtin_memcpy(dst, &o[i], 16);          // rows of y start at any multiple of the element size
+            } else if (in_row) {
+#pragma unroll
+              for (int e = 0; e < 8; ++e)
+                if (k0 + e < a.K) dst[e] = o[i].v[e];
+            }
           }
         }
       }
-    }
-  };
-  if (tg == 0) finish(ic<0>{});
-  else finish(ic<1>{});
+    };
+    if (tg == 0) finish(ic<0>{});
+    else finish(ic<1>{});
+    if (!more) return;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();          // the sums handed over have been read: LDS is free for the next box
+  }
 }
 
 // ---- U[k / 32][channel block][row tap][half][element][lane][8]: the order in which the wavefronts read it.  Lane l holds
@@ -505,7 +536,7 @@ RowBox choose_box(int N, int oD, int oH, int nW, int kd, int kh, int tiles, int 
   return best;
 }
 
-// The shapes of workgroup, by what fills the chip.  Measured, fp16, us (wide | half | small | split):
+// The shapes of workgroup, by what fills the chip.  Measured, fp16, us (wide, a workgroup per box | half | small | split):
 //   wide   eight wavefronts, 64 tiles x 128 channels, one workgroup per CU: every byte of V is used for 128 channels
 //   half   four, 64 tiles x 64 channels, two per CU: the transform of one runs beside the products of the other, finer rounds
 //   small  four, 32 tiles x 64 channels: more workgroups, shorter steps
@@ -549,7 +580,10 @@ RowPlan row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int steps
   return e.plan;
 }
 
-template <typename T, int KD, int KH, int KG, int TB, int S, int CS = 1>
+// Filters that overflow an XCD's 4 MB of L2: its workgroups work on one channel block at a time
+bool filter_fits_l2(const RowArgs& a) { return a.u_bytes <= (3 << 20); }
+
+template <typename T, int KD, int KH, int KG, int TB, int S, int CS = 1, bool STAY = false>
 int launch_row(const RowArgs& args, const RowBox& b, void* stream) {
   RowArgs a = args;
   a.bn = b.bn; a.bd = b.bd; a.bh = b.bh; a.bw = b.bw; a.prow = b.prow; a.irow = b.irow;
@@ -559,15 +593,14 @@ int launch_row(const RowArgs& args, const RowBox& b, void* stream) {
   a.n_box = (int)b.boxes;
   a.local_steps = ceil_div(a.steps, CS);
   a.n_kb = ceil_div(a.K, 32 * KG);
-  // filters that overflow an XCD's 4 MB of L2: its workgroups work on one channel block at a time
-  a.box_fast = a.u_bytes > (3 << 20);
+  a.box_fast = !filter_fits_l2(a);
   a.per_xcd = ceil_div(a.n_kb * a.n_box, kXcds);
   constexpr int bytes = row_lds_bytes<KG, TB, S, CS>();
   const bool whole = a.K % 8 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
-  auto fn = whole ? row_conv_kernel<T, KD, KH, KG, TB, S, CS, false> : row_conv_kernel<T, KD, KH, KG, TB, S, CS, true>;
+  auto fn = whole ? row_conv_kernel<T, KD, KH, KG, TB, S, CS, STAY, false> : row_conv_kernel<T, KD, KH, KG, TB, S, CS, STAY, true>;
   int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), bytes);
   if (rc) return rc;
-  hipLaunchKernelGGL(fn, dim3(a.per_xcd * kXcds), dim3(128 * KG * CS), bytes, as_stream(stream), a);
+  hipLaunchKernelGGL(fn, dim3(STAY ? std::min(a.per_xcd * kXcds, kCus) : a.per_xcd * kXcds), dim3(128 * KG * CS), bytes, as_stream(stream), a);
   WC_CHECK_LAUNCH("row_conv_kernel");
   return WC_OK;
 }
@@ -659,7 +692,13 @@ int row_conv(const wc_conv_desc* d, const void* x, int n_images, const void* U, 
           p.box = choose_box(a.N, a.oD, a.oH, a.nW, KD, KH, tiles, slots);
         }
         switch (p.shape) {
-          case kRowWide: return launch_row<T, KD, KH, 4, 2, 128>(a, p.box, stream);
+          case kRowWide:
+            // More boxes than CUs: a workgroup per CU that asks for its next box's input before it writes a box out, which
+            // hides that input's way from memory behind the write-out and saves the start of a workgroup.  Measured, fp16, us,
+            // a workgroup per box | this: N=64 256 -> 256, 56x56 196 | 185, 128 -> 128, 56x56 71 | 66, 256 -> 256, 28x28 53.3 | 52.0,
+            // N=8 128 -> 128, 16x56x56 242 | 239.  Filters beyond an XCD's L2 (box_fast): 512 -> 512, N=16 28x28 48.1 | 49.3.
+            if (!filter_fits_l2(a) || ceil_div(a.K, 128) * p.box.boxes <= kCus) return launch_row<T, KD, KH, 4, 2, 128>(a, p.box, stream);
+            return launch_row<T, KD, KH, 4, 2, 128, 1, true>(a, p.box, stream);
           case kRowHalf: return launch_row<T, KD, KH, 2, 2, KD == 1 ? 64 : 128>(a, p.box, stream);
           case kRowSmall: return launch_row<T, KD, KH, 2, 1, 64>(a, p.box, stream);
           default: return launch_row<T, KD, KH, 1, 1, 32, 4>(a, p.box, stream);

@@ -105,3 +105,12 @@ def test_special_values_stay_in_their_windows(dev):
     touched = torch.zeros(9, 24, dtype=torch.bool)
     touched[3:6, 4:12] = True                       # the tiles of four outputs whose six inputs hold column 9
     assert bool(torch.isfinite(y[1][:, ~touched]).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("xs,K,pad", [((70, 64, 30, 31), 136, 1), ((12, 40, 9, 30, 33), 40, 1), ((40, 72, 41, 29), 129, 0)])
+def test_more_boxes_than_workgroups(dev, dtype, xs, K, pad, gemm_override):
+    """Wide workgroups that go from box to box: boxes that do not share out evenly, the last of them partial."""
+    x, w, b = _operands(xs, K, dtype)
+    gemm_override(config=16)
+    assert _err(_row(x.to(dev), w.to(dev), b.to(dev), pad), _conv64(x, w, b, pad)) <= BOUND[dtype]
