@@ -143,7 +143,8 @@ class _WinoConvNd(nn.Module):
             raise NotImplementedError(f"WinoConv: dtype {x.dtype} (float32, float16 and bfloat16 only)")
         if not self._winograd_ok(x):
             return conv(x, self.weight, self.bias, self.stride, self.padding, self.dilation, self.groups)
-        w = self.weight.to(x.dtype)
+        # (to() and detach() that change nothing still cost a microsecond each of a 12 us call)
+        w = self.weight if self.weight.dtype == x.dtype else self.weight.to(x.dtype)
         m = self._tile_for(x.dtype)
         # the form of the plan (Winograd pieces, or the direct form the library takes for large strided problems)
         # depends on the batch size too, and the transformed filter of one form does not fit the other
@@ -152,10 +153,10 @@ class _WinoConvNd(nn.Module):
         if self._cache is None or self._cache[0] != key:
             U = engine.transform_filter(w.detach(), x.shape, self.stride[0], self.padding, m, row=True)
             self._cache = (key, U)
-        b = None if self.bias is None else self.bias.to(x.dtype)
+        b = self.bias if self.bias is None or self.bias.dtype == x.dtype else self.bias.to(x.dtype)
         if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (b is not None and b.requires_grad)):
             return WinoConvFunction.apply(x, w, b, self.stride[0], self.padding, m, self._cache[1])
-        return engine.conv_forward(x, w.detach(), b, self.stride[0], self.padding, m, U=self._cache[1], row=True)
+        return engine.conv_forward(x, w, b, self.stride[0], self.padding, m, U=self._cache[1], row=True)
 
 
 class WinoConv2d(_WinoConvNd):

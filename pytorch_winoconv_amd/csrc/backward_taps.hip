@@ -11,10 +11,11 @@
 // 1 and 2 out of them in registers, five LDS reads of 8 bytes for six products instead of ten.
 //
 // The transform domain multiplies less (8 products per pixel of a 3x3x3 filter against 27) but moves V and dM through
-// memory: N=8 128 -> 128, 16x56x56, fp16, 797 us of which 760 are that traffic; here 368 us, 0.95 PFLOP/s.  What bounds
-// this form is LDS: its counters show it busy 86 % of the time and the matrix unit 52 %.  A copy with dy turned channel by
-// channel in LDS, read in 16-byte pieces, measured 424 us (a wide read delivers no more bytes per cycle, and the turning
-// costs), one with the operands of a group read during the group before it 377.  Operands are exact, sums fp32.
+// memory: N=8 128 -> 128, 16x56x56, fp16, 797 us of which 760 are that traffic; here 368 us, 0.95 PFLOP/s (a library
+// matrix product reaches 1.1 on this card).  The matrix unit is busy 52 % of the time at 1.95 GHz, the rest goes to feeding it:
+// 114 vector instructions beside the 24 products of a wavefront's step, and the LDS reads.  Variants that took more of either
+// were slower: dy turned channel by channel in LDS and read 16 bytes at a time 424 us, four wavefronts of all nine taps 439; operands
+// read a group ahead changed nothing (377).  Operands are exact, sums fp32.
 #include "wc_transform.h"
 
 #include <algorithm>
