@@ -645,23 +645,19 @@ int row_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5],
 //    256 -> 256 on 200704 pixels 188 | 219, 384 on 50176 108 | 111, 512 on 50176 178 | 140, 300 -> 200 76 | 67.  Up to one and a
 //    half rounds of the chip the row form's single launch decides (512 on 12544: 47 | 54; 256 on 12544: 17 | 30; 512 on 49: 12 | 17).
 //    Tile 2 (bfloat16) needs 4/9 more products than F(4x4, 3x3) saves: never ahead.
-//  * Layers with the one-kernel F(2x2, 3x3) form (conv_thin.hip), tile 2: that form up to 32 channels; up to 64 outside 2.4
-//    to 8 million output values (64 -> 64 on 50176 pixels 9.1 | 11.6, on 200704 25 | 23, on 12544 6.8 | 6.3); up to 128 below
-//    1.2 million (128 -> 128 on 3136 pixels 8.1 | 6.7, on 12544 8.8 | 11.3, on 50176 17 | 25).
+//  * Never where the one-kernel F(2x2, 3x3) form (conv_thin.hip) runs, though it is up to a third slower on its larger layers
+//    (128 -> 128 on 50176 pixels 17 | 25): that form rounds no products either, and its error is the smaller one (against fp64
+//    in the 2-norm, fp16 6.2e-4 | 6.1e-4, bf16 5.0e-3 | 4.2e-3).
 bool row_preferred(const wc_conv_desc* d) {
   if (d->kernel[0] > 1) return true;
-  const int oD = 1, oH = d->in[1] + 2 * d->pad[1] - 2, oW = d->in[2] + 2 * d->pad[2] - 2;
-  const long long P = (long long)d->N * oH * oW, outputs = P * d->K;
+  const int oW = d->in[2] + 2 * d->pad[2] - 2;
   wc_plan plan;
   wc_conv_desc e = *d;
   e.stacked = 0; e.direct = 0; e.row = 0;
-  if (wc_plan_conv(&e, &plan) == WC_OK && thin_conv_fits(&e, &plan)) {
-    const int cp = wc_padded_channels(d->C);
-    if (cp <= 32) return false;
-    return cp <= 64 ? outputs >= 2400000 && outputs <= 8000000 : outputs >= 1200000;
-  }
+  if (wc_plan_conv(&e, &plan) == WC_OK && thin_conv_fits(&e, &plan)) return false;
   if (d->m != 4 || d->dtype != WC_F16) return true;
-  if (row_plan(d->N, oD, oH, ceil_div(oW, 4), 1, 3, d->K, ceil_div(d->C, 32)).wide_groups <= 3 * kCus / 2) return true;
+  const int oH = d->in[1] + 2 * d->pad[1] - 2;
+  if (row_plan(d->N, 1, oH, ceil_div(oW, 4), 1, 3, d->K, ceil_div(d->C, 32)).wide_groups <= 3 * kCus / 2) return true;
   const double C = d->C, K = d->K, Cp = wc_padded_channels(d->C), Kp = ceil_div(d->K, 64) * 64.0;
   return 10.5 * Cp * Kp < 1500.0 * (C + K) + C * K;
 }
