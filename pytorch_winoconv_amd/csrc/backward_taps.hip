@@ -290,7 +290,8 @@ bool taps_plan(const wc_conv_desc* d, const int out[3], TapsPlan* p) {
   const int S = taps_parts(p->steps, p->tiles, p->kg);
   p->part_steps = ceil_div(p->steps, std::min(S, p->steps));
   p->parts = ceil_div(p->steps, p->part_steps);
-  return true;
+  // the last part is cut off at `total`, but the kernel takes its full length first: up to 64 * parts positions more
+  return (long long)p->parts * p->part_steps * kStep < (1ll << 31);
 }
 
 template <typename T, int KG>

@@ -124,6 +124,20 @@ def test_workspace_size_is_u_plus_v_plus_m():
     assert nbytes.value == 2 * (16 * 64 * 64 + 2 * 16 * 64 * 28 * 28 * 64)
 
 
+@pytest.mark.parametrize("n,tap_form", [(57343, True), (57344, False)])
+def test_tap_form_of_the_weight_gradient_keeps_its_positions_in_ints(n, tap_form):
+    """One 169 x 217 channel, padding 1: n (169 + 2) (217 + 2) positions in 256 parts of whole steps of 64.  At 57344 images
+    they stay below 2^31 (2147475456), the end of the last part as the kernel first takes it does not (256 * 131072 * 64 is
+    2^31): the transform domain then.  Told apart by the workspace, which for the tap form is its partial sums."""
+    lib = _lib.load()
+    desc = engine.make_desc((n, 1, 169, 217), (1, 1, 3, 3), torch.bfloat16, 1, 1, 2)
+    nbytes = ctypes.c_size_t()
+    assert lib.wc_conv_backward_weight_workspace_bytes(ctypes.byref(desc), ctypes.byref(nbytes)) == 0
+    assert (nbytes.value == 256 * 6 * 24 * 64 * 4 * 4) == tap_form
+    steps = -(-n * 171 * 219 // 64)
+    assert (256 * -(-steps // 256) * 64 < 2 ** 31) == tap_form
+
+
 def test_python_layer_refuses_cpu_tensors_and_bad_shapes(host_layer):
     x = torch.randn(1, 4, 8, 8)
     w = torch.randn(4, 4, 3, 3)

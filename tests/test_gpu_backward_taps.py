@@ -87,3 +87,15 @@ def test_same_as_the_transform_domain(dev):
         _lib.check(lib.wc_test_gemm_override(-1, 1))
     assert _err(taps, ref) < _err(other, ref)
     assert float((taps.float() - other.float()).norm() / taps.float().norm()) <= 5e-3
+
+
+@pytest.mark.parametrize("n", [57343, 57344])
+def test_positions_close_to_2g(dev, n):
+    """The last images of a line of almost 2^31 positions: the largest that the tap form takes, and one that it leaves to the
+    transform domain because the end of its last part would be 2^31.  Everything before the last two images is zero."""
+    x = torch.zeros(n, 1, 169, 217, dtype=torch.bfloat16, device=dev)
+    dy = torch.zeros_like(x)
+    xl, dyl, pads, shape, ref = _operands((2, 1, 169, 217), 1, 1, torch.bfloat16)
+    x[-2:], dy[-2:] = xl.to(dev), dyl.to(dev)
+    # nine values of a sum over 73000 products: the transform domain as in test_gpu_backward.py
+    assert _err(engine.conv_backward_weight(x, dy, shape, 1, pads, 2), ref) <= (BOUND[x.dtype] if n == 57343 else 2e-2)
