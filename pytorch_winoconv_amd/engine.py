@@ -414,14 +414,17 @@ def _conv_forward(x, w, bias, stride, padding, m, U, chunk_images, whole_kernel,
         x_mem = x if x.is_contiguous() else x.contiguous()
         x_layout = 1
     y_layout = int(bool(channels_first_out))
-    # the one-kernel path of thin layers needs 16-byte aligned operands; a legal view can start anywhere
+    unfused = bool(unfused)
+    setup = lambda unfused, row: _forward_setup(tuple(x.shape), tuple(w.shape), x.dtype, stride, padding, m, chunk_images,
+                                                whole_kernel, stacked, unfused, x_layout, y_layout, direct, row)
+    desc, y_shape, nbytes, u_elems = setup(unfused, bool(row) and not unfused)
+    if desc.row:                                           # the row form reads aligned operands: copies of those that are not
+        x_mem = x_mem.clone() if misaligned(x_mem) else x_mem
+        U = U.clone() if misaligned(U) else U
+    # the one-kernel path of thin layers needs 16-byte aligned operands too; a legal view can start anywhere
     # (x[1:] of a channel-last tensor with 6 channels and 7 x 7 images is 4-byte aligned): three kernels then
-    row = bool(row) and not unfused
-    if row and misaligned(x_mem, U):                       # ... and so does the row form: aligned copies of them
-        x_mem, U = x_mem.clone(), U.clone() if U is not None else None
-    unfused = bool(unfused) or misaligned(x_mem, U)
-    desc, y_shape, nbytes, u_elems = _forward_setup(tuple(x.shape), tuple(w.shape), x.dtype, stride, padding, m,
-                                                    chunk_images, whole_kernel, stacked, unfused, x_layout, y_layout, direct, row)
+    if not unfused and misaligned(x_mem, U):
+        desc, y_shape, nbytes, u_elems = setup(True, False)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
     if y_layout:
         y = torch.empty([y_shape[0], y_shape[-1]] + y_shape[1:-1], dtype=x.dtype, device=x.device)

@@ -96,6 +96,27 @@ def test_modules_and_layouts(dev, host_layer):
         assert _err(mod(xcl), _conv64(x, 2 * w, b, 1)) <= BOUND[x.dtype]
 
 
+@pytest.mark.parametrize("dtype,ws,stride,m", [
+    (torch.float32, (64, 64, 3, 3), 1, 2), (torch.bfloat16, (64, 64, 3, 3), 1, 2),       # one kernel where x is aligned
+    (torch.float32, (40, 64, 3, 3), 1, 4), (torch.float16, (40, 64, 3, 3), 2, 2), (torch.float16, (40, 64, 5, 5), 1, 2),
+])
+def test_misaligned_operands_where_the_row_form_does_not_follow(dev, monkeypatch, dtype, ws, stride, m):
+    """Permission for the row form copies nothing where the library takes another form, and both host layers run the same
+    kernels: the same bits as without the permission."""
+    g = torch.Generator().manual_seed(4)
+    w = (torch.randn(ws, generator=g) * (2.0 / (ws[1] * ws[2] * ws[3])) ** 0.5).to(dtype).to(dev)
+    x = torch.empty(2 * 64 * 15 * 14 + 1, dtype=dtype, device=dev)[1:].view(2, 15, 14, 64).permute(0, 3, 1, 2)
+    x.copy_(torch.randn(x.shape, generator=g))
+    assert engine.misaligned(x) and engine.make_desc(x.shape, ws, dtype, stride, ws[2] // 2, m, stacked=None, row=True).row == 0
+    y = {}
+    for compiled in (True, False):
+        monkeypatch.setattr(engine, "USE_EXT", compiled)
+        monkeypatch.setattr(torch.Tensor, "clone", lambda *_: pytest.fail("a copy"))
+        y[compiled] = [engine.conv_forward(x, w, None, stride, ws[2] // 2, m, row=row) for row in (False, True)]
+        monkeypatch.undo()
+    assert all(torch.equal(v, y[True][0]) for v in y[True] + y[False])
+
+
 def test_special_values_stay_in_their_windows(dev):
     """An infinity in x reaches the outputs whose tiles contain it and no others; padding channels never do."""
     x, w, _ = _operands((2, 36, 9, 24), 40, torch.float16)
