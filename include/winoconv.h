@@ -75,7 +75,9 @@ typedef struct {
   int stride;      /* 1 or 2, same on every axis                                */
   int m;           /* Winograd output tile: 2, or 4 (2-D: 4 x 4; 3-D: 2 x 4 x 4, 3x3x3 stride 1 only), or 3 (with stacked = 2) */
   int dtype;       /* wc_dtype                                                  */
-  int chunk_images;/* images per pass of wc_conv_forward; 0 = choose automatically */
+  int chunk_images;/* images per pass of wc_conv_forward, which bounds its scratch; 0 = choose automatically.  The one-kernel
+                    * forms (unfused = 0, direct, row) have no V and M and take the batch in one pass, with scratch copies of
+                    * all of x and y where a layout needs them; the row form honours it where it copies x or y */
   int whole_kernel;/* 0: kernels > 3 are decomposed into pieces of <= 3 taps (DWM, dwm.py:107-146);
                     * 1: one F(2,k) x F(2,k) tile for the whole k x k kernel, k = 4..7, the arithmetic
                     *    of the reference's PyTorch path (matrix_conv.py:112-135, tables :31-35):

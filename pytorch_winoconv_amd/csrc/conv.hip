@@ -57,7 +57,8 @@ struct Layout {
   bool thin;                          // the one-kernel path runs: V and M are not needed
   bool direct;                        // the direct form: the product reads x itself, V and M are not needed
   bool row;                           // the row form: one kernel as well
-  bool whole() const { return thin || direct || row; }      // one pass over the whole batch, only U in the workspace
+  bool whole() const { return thin || direct || row; }      // one kernel: no V and M in the workspace
+  int images;                         // images per pass: the whole batch for the one-kernel forms, `chunk` for the others
   bool x_direct;                      // channel-first x is read by the input transform itself
   size_t xcl_bytes, ycl_bytes;        // channel-last scratch copies of a chunk of x / of y (0 if not needed)
   // 3-D F(2,3)^3 plans in 16-bit types: the width axis is taken inside the product (fold_filter_w, gemm.hip).  V and M
@@ -161,15 +162,17 @@ int make_layout(const wc_conv_desc* d_in, Layout* L) {
     }
   }
   // channel-first tensors: the input transform of small single-piece plans reads x as it is; everything else goes
-  // through a channel-last copy of one chunk (the one-kernel path: of the whole batch)
+  // through a channel-last copy of the images of a pass
   L->x_direct = d->x_layout == 1 && ((!L->whole() && input_transform_nchw_fits(d, &L->plan)) ||
                                      (L->direct && (direct_first_fits(d_in) || direct_first3d_fits(d_in))));      // ... and so do the first-layer kernels
-  const size_t images = L->whole() ? d->N : chunk;
   // the row form reads channel-last x with its channels padded to a multiple of 8
   const size_t x_image = (size_t)d->in[0] * d->in[1] * d->in[2] * (L->row ? wc_padded_channels8(d->C) : d->C) * L->es;
   const size_t y_image = (size_t)L->out[0] * L->out[1] * L->out[2] * d->K * L->es;
-  L->xcl_bytes = (d->x_layout == 1 && !L->x_direct) || (L->row && d->C % 8 != 0) ? round256(images * x_image) : 0;
-  L->ycl_bytes = d->y_layout == 1 ? round256(images * y_image) : 0;
+  const bool copy_x = (d->x_layout == 1 && !L->x_direct) || (L->row && d->C % 8 != 0), copy_y = d->y_layout == 1;
+  // the row form's copies are the scratch that chunk_images bounds; without copies there is nothing to bound
+  L->images = !L->whole() || (L->row && d->chunk_images > 0 && (copy_x || copy_y)) ? chunk : d->N;
+  L->xcl_bytes = copy_x ? round256(L->images * x_image) : 0;
+  L->ycl_bytes = copy_y ? round256(L->images * y_image) : 0;
   return WC_OK;
 }
 
@@ -277,7 +280,7 @@ int forward_impl(const wc_conv_desc* d, const void* x, const void* w, const int6
                  d->stacked, d->whole_kernel ? " whole-kernel tile" : "",
                  L.row ? "row form: one fused kernel, F(4,3) along the width" : L.direct ? "direct form: the product reads x" : L.thin ? "one fused kernel" : L.fold ? "input transform (depth, height), shifted batched GEMM with the width taps along its reduction, output transform" : (L.shared ? "input transform, shifted batched GEMM, output transform"
                                                          : "input transform, batched GEMM, output transform"),
-                 L.whole() ? d->N : L.chunk, L.tiles_per_image, need, L.u_bytes, L.whole() ? (size_t)0 : L.v_bytes,
+                 L.images, L.tiles_per_image, need, L.u_bytes, L.whole() ? (size_t)0 : L.v_bytes,
                  L.whole() ? (size_t)0 : L.m_bytes, L.xcl_bytes, L.ycl_bytes,
                  d->x_layout ? (L.x_direct ? "channel-first, read by the input transform" : "channel-first, copied") : "channel-last",
                  d->y_layout ? "channel-first, copied" : "channel-last", U_cached ? "transformed by the caller" : "transformed here");
@@ -308,7 +311,7 @@ int forward_impl(const wc_conv_desc* d, const void* x, const void* w, const int6
   const long long out_pos = (long long)L.out[0] * L.out[1] * L.out[2];
   const size_t x_image = (size_t)in_pos * d->C * L.es;
   const size_t y_image = (size_t)out_pos * d->K * L.es;
-  const int step = L.whole() ? d->N : L.chunk;
+  const int step = L.images;
   for (int b0 = 0; b0 < d->N; b0 += step) {
     const int n = (d->N - b0 < step) ? d->N - b0 : step;
     const void* xin = static_cast<const unsigned char*>(x) + b0 * x_image;

@@ -681,9 +681,10 @@ int row_conv(const wc_conv_desc* d, const void* x, int n_images, const void* U, 
     if constexpr (sizeof(T) == 2) {
       auto go = [&](auto kd, auto kh) -> int {
         constexpr int KD = decltype(kd)::value, KH = decltype(kh)::value;
-        RowPlan p = row_plan(a.N, a.oD, a.oH, a.nW, KD, KH, a.K, a.steps);
-        if (force >= 16 && force <= 19) {
-          p.shape = (RowShape)(force - 16);
+        // the shape is the whole batch's, so that the passes of a batch add in the order of the batch in one pass
+        RowPlan p = row_plan(d->N, a.oD, a.oH, a.nW, KD, KH, a.K, a.steps);
+        if (force >= 16 && force <= 19) p.shape = (RowShape)(force - 16);
+        if (a.N != d->N || (force >= 16 && force <= 19)) {
           const int tiles = p.shape <= kRowHalf ? 64 : 32, slots = p.shape == kRowWide ? 128 : p.shape == kRowSplit ? 32 : p.shape == kRowHalf && KD > 1 ? 128 : 64;
           p.box = choose_box(a.N, a.oD, a.oH, a.nW, KD, KH, tiles, slots);
         }

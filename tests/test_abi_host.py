@@ -124,6 +124,25 @@ def test_workspace_size_is_u_plus_v_plus_m():
     assert nbytes.value == 2 * (16 * 64 * 64 + 2 * 16 * 64 * 28 * 28 * 64)
 
 
+def test_row_form_copies_the_images_of_a_pass():
+    """chunk_images bounds the scratch copies of x (channels padded to 8) and y; without copies there is only U."""
+    lib = _lib.load()
+
+    def scratch(c, x_layout, y_layout, chunk):
+        desc = engine.make_desc((64, c, 56, 56), (256, c, 3, 3), torch.float16, 1, 1, 4, x_layout=x_layout, y_layout=y_layout)
+        desc.row, desc.chunk_images = 1, chunk
+        nbytes, ue = ctypes.c_size_t(), ctypes.c_size_t()
+        assert lib.wc_conv_workspace_bytes(ctypes.byref(desc), ctypes.byref(nbytes)) == 0
+        assert lib.wc_conv_u_elems(ctypes.byref(desc), ctypes.byref(ue)) == 0
+        return nbytes.value - 2 * ue.value
+
+    for chunk, n in ((0, 64), (8, 8), (64, 64), (100, 64)):
+        assert scratch(256, 0, 0, chunk) == 0
+        assert scratch(256, 1, 0, chunk) == scratch(256, 0, 1, chunk) == n * 56 * 56 * 256 * 2
+        assert scratch(250, 0, 0, chunk) == n * 56 * 56 * 256 * 2
+        assert scratch(250, 1, 1, chunk) == 2 * n * 56 * 56 * 256 * 2
+
+
 @pytest.mark.parametrize("n,tap_form", [(57343, True), (57344, False)])
 def test_tap_form_of_the_weight_gradient_keeps_its_positions_in_ints(n, tap_form):
     """One 169 x 217 channel, padding 1: n (169 + 2) (217 + 2) positions in 256 parts of whole steps of 64.  At 57344 images

@@ -117,6 +117,42 @@ def test_misaligned_operands_where_the_row_form_does_not_follow(dev, monkeypatch
     assert all(torch.equal(v, y[True][0]) for v in y[True] + y[False])
 
 
+@pytest.mark.parametrize("xs,K,chunk", [((5, 256, 7, 7), 64, 2), ((41, 156, 15, 14), 72, 7), ((3, 36, 4, 9, 10), 40, 1), ((70, 64, 30, 31), 130, 32)])
+def test_passes_over_a_batch_give_the_bits_of_one_pass(dev, xs, K, chunk, host_layer):
+    """Also where the whole batch and a pass would choose another shape of workgroup (shares of the channels or none)."""
+    x, w, b = _operands(xs, K, torch.float16)
+    xd, wd, bd = x.to(dev), w.to(dev), b.to(dev)
+    d = engine.make_desc(xs, w.shape, x.dtype, 1, 1, 2, stacked=None, row=True)
+    d.row = 1
+    lib, fmt = _lib.load(), torch.channels_last if x.dim() == 4 else torch.channels_last_3d
+    want = _row(xd, wd, bd, 1)
+    assert _err(want, _conv64(x, w, b, 1)) <= BOUND[x.dtype]
+    if engine.make_desc(xs, w.shape, x.dtype, 1, 1, 4, stacked=None, row=True).row:
+        for x_in in (xd, xd.contiguous(memory_format=fmt)):
+            for first in (False, True):
+                y = engine.conv_forward(x_in, wd, bd, 1, 1, 4, chunk_images=chunk, row=True, channels_first_out=first)
+                assert torch.equal(y, want)
+    # the library's own scratch, in as many passes as fit
+    for x_layout, x_in in ((1, xd), (0, engine.channel_last(xd))):
+        d.x_layout, d.y_layout, d.chunk_images = x_layout, 1, chunk
+        y = torch.full_like(want, float("nan")).contiguous()
+        _lib.check(lib.wc_conv_forward_static(ctypes.byref(d), x_in.data_ptr(), wd.data_ptr(), engine._w_strides(wd), None, bd.data_ptr(),
+                                              y.data_ptr(), torch.cuda.current_stream().cuda_stream))
+        assert torch.equal(y, want)
+
+
+def test_static_scratch_takes_a_batch_whose_copies_it_cannot_hold(dev):
+    """132 MB of channel-first x in 64 MB of scratch."""
+    x, w, b = _operands((41, 256, 80, 79), 32, torch.float16)
+    xd, wd, bd = x.to(dev), w.to(dev), b.to(dev)
+    d = engine.make_desc(x.shape, w.shape, x.dtype, 1, 1, 2, x_layout=1)
+    d.row = 1
+    y = torch.full((41, 80, 79, 32), float("nan"), dtype=x.dtype, device=dev)
+    _lib.check(_lib.load().wc_conv_forward_static(ctypes.byref(d), xd.data_ptr(), wd.data_ptr(), engine._w_strides(wd), None,
+                                                  bd.data_ptr(), y.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(engine.channel_first_view(y), _row(xd, wd, bd, 1))
+
+
 def test_special_values_stay_in_their_windows(dev):
     """An infinity in x reaches the outputs whose tiles contain it and no others; padding channels never do."""
     x, w, _ = _operands((2, 36, 9, 24), 40, torch.float16)
