@@ -638,28 +638,34 @@ int row_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5],
   return WC_OK;
 }
 
-// Against the other forms, fp16, us (row | other), channels -> channels on P output pixels:
-//  * 3-D: always (8x28x28 to 16x56x56, 32 to 128 channels: 1.3 to 3 times faster).
-//  * 2-D with V and M in memory: F(4x4, 3x3) needs half the products, so it overtakes on large problems with many
-//    channels.  Per pixel it takes about 1500 (C + K) + C K units, the row form 10.5 of them per product of padded channels:
-//    256 -> 256 on 200704 pixels 188 | 219, 384 on 50176 108 | 111, 512 on 50176 178 | 140, 300 -> 200 76 | 67.  Up to one and a
-//    half rounds of the chip the row form's single launch decides (512 on 12544: 47 | 54; 256 on 12544: 17 | 30; 512 on 49: 12 | 17).
-//    Tile 2 (bfloat16) needs 4/9 more products than F(4x4, 3x3) saves: never ahead.
-//  * Never where the one-kernel F(2x2, 3x3) form (conv_thin.hip) runs, though it is up to a third slower on its larger layers
-//    (128 -> 128 on 50176 pixels 17 | 25): that form rounds no products either, and its error is the smaller one (against fp64
-//    in the 2-norm, fp16 6.2e-4 | 6.1e-4, bf16 5.0e-3 | 4.2e-3).
+// Against the other forms, us (row | other), channels -> channels on P output pixels:
+//  * Where tile 2 is asked for (the modules in 3-D and in bfloat16): always.  The row form takes 9/8 (3-D: 27/16) times the products of
+//    the F(2, 3) tiles and none of their traffic.  fp16, 3-D: 32 -> 32 on 401408 60 | 107, 64 -> 64 on 50176 14 | 36, 128 -> 128 on 401408
+//    229 | 426, 192 -> 192 on 50176 85 | 121, 256 -> 256 on 200704 421 | 555, on 6272 30 | 35, on 3136 22 | 31, 384 -> 384 on
+//    50176 237 | 281, 512 -> 512 on 50176 425 | 476, on 12544 114 | 128, on 196 19 | 24; bf16 as fp16.  The exception, 512 -> 512
+//    on 16 clips of 2x7x7 (a row of 7 outputs fills two tiles of 4) 44 | 35, stays here for its error: against fp64 in the 2-norm
+//    fp16 6.3e-4 | 8.5e-4, bf16 5.1e-3 | 6.8e-3.  bf16, 2-D: 256 -> 256 on 200704 182 | 374, 512 -> 512 on 50176 187 | 225.
+//  * Where tile 4 is asked for, whose larger error the caller accepts (fp16 4e-3, bf16 3e-2; 3-D 2x4x4 5e-3, 4e-2), the faster
+//    one.  Up to one and a half rounds of the chip the row form's single launch decides (2-D: 512 on 12544 47 | 54, bf16 48 | 53;
+//    256 on 12544 17 | 30; 512 on 49 12 | 17; 3-D: 512 on 196 19 | 41, on 6272 70 | 69).  Beyond, F(4x4, 3x3) needs half the products
+//    and F(2x4x4, 3x3x3) a third, and they overtake with the channels.  Per pixel they take about 1500 (C + K) + C K units in 2-D,
+//    512 (C + K) + C K in 3-D, and the row form 10.5 and 3.6 of them per product of padded channels.  2-D, fp16 (bf16): 256 -> 256
+//    on 200704 188 | 219 (182 | 217), 384 on 50176 108 | 111 (112 | 107), 512 on 50176 178 | 140 (187 | 141), 300 -> 200 76 | 67
+//    (78 | 64).  3-D, fp16: 128 on 401408 229 | 539, 256 on 200704 421 | 580, 384 on 50176 237 | 260, 512 on 50176 425 | 349,
+//    on 25088 212 | 204, on 12544 114 | 114.
+//  * Never where the one-kernel F(2x2, 3x3) form runs (conv_thin.hip), though it is up to a third slower on its larger layers
+//    (128 -> 128 on 50176 pixels 17 | 25): that form rounds no products either, and its error is the smaller one (fp16 6.2e-4 |
+//    6.1e-4, bf16 5.0e-3 | 4.2e-3).
 bool row_preferred(const wc_conv_desc* d) {
-  if (d->kernel[0] > 1) return true;
-  const int oW = d->in[2] + 2 * d->pad[2] - 2;
   wc_plan plan;
   wc_conv_desc e = *d;
   e.stacked = 0; e.direct = 0; e.row = 0;
   if (wc_plan_conv(&e, &plan) == WC_OK && thin_conv_fits(&e, &plan)) return false;
-  if (d->m != 4 || d->dtype != WC_F16) return true;
-  const int oH = d->in[1] + 2 * d->pad[1] - 2;
-  if (row_plan(d->N, 1, oH, ceil_div(oW, 4), 1, 3, d->K, ceil_div(d->C, 32)).wide_groups <= 3 * kCus / 2) return true;
-  const double C = d->C, K = d->K, Cp = wc_padded_channels(d->C), Kp = ceil_div(d->K, 64) * 64.0;
-  return 10.5 * Cp * Kp < 1500.0 * (C + K) + C * K;
+  if (d->m != 4) return true;
+  const int kd = d->kernel[0], oD = d->in[0] + 2 * d->pad[0] - kd + 1, oH = d->in[1] + 2 * d->pad[1] - 2, oW = d->in[2] + 2 * d->pad[2] - 2;
+  if (row_plan(d->N, oD, oH, ceil_div(oW, 4), kd, 3, d->K, ceil_div(d->C, 32)).wide_groups <= 3 * kCus / 2) return true;
+  const double C = d->C, K = d->K, products = (double)wc_padded_channels(d->C) * (ceil_div(d->K, 64) * 64.0);
+  return kd == 1 ? 10.5 * products < 1500.0 * (C + K) + C * K : 3.6 * products < 512.0 * (C + K) + C * K;
 }
 
 // x (N, D, H, W, Cx) channel-last with Cx = C rounded up to 8 (zeros beyond C), 16-byte aligned

@@ -143,6 +143,18 @@ def test_row_form_copies_the_images_of_a_pass():
         assert scratch(250, 1, 1, chunk) == 2 * n * 56 * 56 * 256 * 2
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("x,k,m,row", [
+    ((64, 512, 28, 28), 512, 2, 1), ((64, 512, 28, 28), 512, 4, 0), ((16, 300, 56, 56), 200, 4, 0),       # wide layers, many pixels
+    ((64, 256, 56, 56), 256, 4, 1), ((64, 512, 14, 14), 512, 4, 1), ((1, 512, 7, 7), 512, 4, 1),          # fewer of either
+    ((8, 512, 8, 28, 28), 512, 2, 1), ((8, 512, 8, 28, 28), 512, 4, 0), ((8, 384, 8, 28, 28), 384, 4, 1), ((2, 512, 2, 7, 7), 512, 4, 1),
+    ((64, 128, 28, 28), 128, 2, 0),                                                                       # one kernel on F(2x2, 3x3)
+])
+def test_where_the_row_form_is_chosen(dtype, x, k, m, row):
+    """Both 16-bit types alike; a caller who asks for tile 4 gets it where it is faster."""
+    assert engine.make_desc(x, (k, x[1]) + (3,) * (len(x) - 2), dtype, 1, 1, m, stacked=None, row=True).row == row
+
+
 @pytest.mark.parametrize("n,tap_form", [(57343, True), (57344, False)])
 def test_tap_form_of_the_weight_gradient_keeps_its_positions_in_ints(n, tap_form):
     """One 169 x 217 channel, padding 1: n (169 + 2) (217 + 2) positions in 256 parts of whole steps of 64.  At 57344 images
