@@ -71,7 +71,8 @@ constexpr int kRowPitch = 64;     // LDS bytes per (element, row of a tile): 32 
 // Chunk g of row s lies at position g ^ (s / 4 % 4).  A 16-byte read is served in four phases of sixteen lanes over 64
 // banks, lanes 0-3, 12-15, 20-27 in the first, 4-11, 16-19, 28-31 in the second and the same 32 further up: of the lanes of
 // a phase with the same row modulo 4 each has another row / 4 modulo 4, so one chunk of 32 consecutive rows, from any
-// row on, is read without conflicts, and so is what a store writes, all chunks of 16 rows.
+// row on, is read without conflicts, and so is what a store writes, all chunks of 16 rows.  Two lanes of a phase whose
+// different rows agree modulo 16 take a cycle each: what the boxes make of that, see choose_box.
 __device__ __forceinline__ int v_offset(int s, int g) { return s * kRowPitch + ((g ^ (s >> 2)) & 3) * 16; }
 
 // What the NI items of a step carry beside their products: the transform of 8 UN channels, over the first two thirds of the
@@ -510,8 +511,12 @@ __global__ __launch_bounds__(256) void row_filter_kernel(RowFilterArgs a) {
 
 // Box of a workgroup: at most `tiles` tiles whose input rows, with the halo of the taps, fill at most `slots` rows of LDS;
 // the fewest boxes over the output, and among those the fewest rows.  Fragment reads take the tiles of a box in order, which
-// is free of bank conflicts where their rows are consecutive: planes and images are padded to row counts that continue the
-// count of their tiles modulo 16 (the period of v_offset) across the halo.
+// is free of bank conflicts where their rows are consecutive modulo 16 (the period of v_offset).  Planes and images are padded
+// to row counts that continue the count of their tiles across the halo modulo 8, which leaves reads whose sixteen lanes
+// cross an image or a plane 8 rows off: two cycles.  So do the lanes of a block that has fewer than 32 tiles, which all read
+// tile 0.  Cycles for the conflict-free number of them, per pass over the taps: N=64, 56x56 (4 images of 8 rows x 2 tiles) 24
+// for 12, 14x14 (14 rows x 4 tiles) 18 for 12, 28x28 15 for 12, 16x56x56 (4 planes of 14 rows x 1 tile) 72 for 36, N=1 7x7 6 for
+// 6; counted by SQ_LDS_BANK_CONFLICT at N=64 256 -> 256, 56x56: 14.45 M of 36.1 M cycles of the LDS.
 struct RowBox { int bn, bd, bh, bw, n_n, n_d, n_h, n_w, prow, irow; long long boxes; };
 RowBox choose_box(int N, int oD, int oH, int nW, int kd, int kh, int tiles, int slots) {
   RowBox best{};
@@ -542,7 +547,8 @@ RowBox choose_box(int N, int oD, int oH, int nW, int kd, int kh, int tiles, int 
 //   small  four, 32 tiles x 64 channels: more workgroups, shorter steps
 //   split  eight, 32 tiles x 32 channels, the channel blocks shared out over four pairs of wavefronts
 // N=64: 256 -> 256 channels, 56x56 188 | 190 | 231, 14x14 22 | 17 | 20; 128 -> 128, 28x28 17.2 | 18.0 | 22.5, 56x56
-// 68 | 60 | 74; N=16, 256 -> 256, 14x14 21 | 15 | 12.4 | 10.6; N=1, 512 -> 512, 7x7 33 | 22 | 19 | 12.
+// 68 | 60 | 74; N=16, 256 -> 256, 14x14 21 | 15 | 12.4 | 10.6; N=1, 512 -> 512, 7x7 33 | 22 | 19 | 12.  (Layers of up to 128 input
+// channels come here in 3-D or with tile 4; with tile 2 the one-kernel F(2x2, 3x3) form takes most of them, see row_preferred.)
 enum RowShape { kRowWide, kRowHalf, kRowSmall, kRowSplit };
 struct RowPlan { RowShape shape; RowBox box; long long wide_groups; };
 

@@ -536,8 +536,8 @@ def conv_backward_input(dy, w, x_spatial, stride=1, padding=0, m=2):
         raise NotImplementedError("input gradient needs padding <= kernel - 1 on every axis")
     want = tuple(int(v) for v in x_spatial)
     if stride == 2 and nd == 2 and dy.shape[0] > 0:
-        # the library's own input gradient of strided layers: one direct-form launch per parity class of the pixels of
-        # dx (wc_conv_backward_input); where it does not apply, the zero-filled dy below
+        # the library's own input gradient of strided layers: the direct form over the parity classes of the pixels of dx
+        # (wc_conv_backward_input); where it does not apply, the zero-filled dy below
         lib = _lib.load()
         x_shape = (dy.shape[0], w.shape[1]) + want
         desc = make_desc(x_shape, w.shape, dy.dtype, 2, padding, 2, 0, False, False, direct=False)
