@@ -161,6 +161,7 @@ const char* wc_last_error(void);
  * the number of tiles (9 only where the channel count allows it).
  * config 20: the weight gradient never takes the tap form (backward_taps.hip).
  * config 16 to 19: the row form with the wide, half, small or split workgroups whatever the problem (conv_row.hip).
+ * config 21: the row form on tall boxes whatever the problem (conv_row_tall.hip).
  * Works only in a process started with WINOCONV_TEST_HOOKS=1 in its environment (WC_ERR_UNSUPPORTED
  * otherwise, and nothing changes); what it sets holds for the calling host thread only, so a caller
  * cannot change what the launches of another thread do.  Production code never calls it. */

@@ -326,7 +326,7 @@ int forward_impl(const wc_conv_desc* d, const void* x, const void* w, const int6
     }
     void* ydst = L.ycl_bytes ? Ycl : yout;
     if (L.row) {
-      rc = timer.run(WC_STAGE_PRODUCT, [&] { return row_conv(&dcl, xin, n, U, bias, ydst, stream); });
+      rc = timer.run(WC_STAGE_PRODUCT, [&] { return row_conv(&dcl, xin, b0, n, U, bias, ydst, stream); });
       if (rc) return rc;
     } else if (L.direct) {
       rc = timer.run(WC_STAGE_PRODUCT, [&] { return direct_conv(&dcl, xin, n, U, bias, ydst, stream); });

@@ -10,47 +10,13 @@
 // multiplications of the plain sum (the 2-D tile saves three quarters of them), but V lives in LDS, the products in
 // accumulators, and x, U and y are all the memory traffic there is.  The sum over taps and channels is taken in fp32
 // before the output transform, so only V and U are rounded to the storage type.
-//
-// Points of the tile: 0, +-a, +-1/a, infinity with a^2 = 0.425 instead of the customary 0, +-1, +-2.  They spread the
-// rounding of U and V evenly: with independent roundings of relative size e in both, the output's is 3.1 e in the root
-// mean square against 4.6 e with integer points, and against 2.4 e (products rounded to the storage type on top) for
-// F(2x2, 3x3).  Measured over 64 channels, fp16: 6e-4 of the output in the 2-norm, as F(2x2, 3x3), and a sixth of
-// F(4x4, 3x3)'s 3.7e-3.
-#include "wc_transform.h"
+#include "row_form.h"
 
 #include <algorithm>
 
 namespace wc {
 
 namespace {
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-constexpr float kA2 = 0.425f, kB2 = 1.0f / 0.425f;             // a^2 and 1 / a^2
-constexpr float kA = 0.65192024f, kB = 1.0f / 0.65192024f;      // a (its square differs from kA2 by 5e-9)
-constexpr float kS = kA2 + kB2;
-
-template <typename T> struct MfmaRow;
-template <> struct MfmaRow<half_t> {
-  using Frag = f16x8;
-  static __device__ __forceinline__ f32x16 run(Frag a, Frag b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
-};
-template <> struct MfmaRow<bf16_t> {
-  using Frag = bf16x8;
-  static __device__ __forceinline__ f32x16 run(Frag a, Frag b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
-};
-
-// d + f in fp32, rounded to T
-__device__ __forceinline__ bf16_t plus(bf16_t d, float f) { return static_cast<bf16_t>(static_cast<float>(d) + f); }
-__device__ __forceinline__ half_t plus(half_t d, float f) {
-  float one = 1.0f;
-  asm("" : "+s"(one));                  // d * 1 + f stays one v_fma_mix instead of a conversion, an addition and a conversion
-  return static_cast<half_t>(__builtin_fmaf(static_cast<float>(d), one, f));
-}
 
 struct RowArgs {
   const void* x; const void* U; const void* bias; void* y;
@@ -192,18 +158,7 @@ void row_conv_kernel(RowArgs a) {
       const unsigned two = xr[i][j][word];
       x[j] = __builtin_bit_cast(Pack<T, 2>, two);
     }
-    float d[6];
-#pragma unroll
-    for (int j = 0; j < 6; ++j) d[j] = static_cast<float>(x[j].v[e]);
-    const float ea = __builtin_fmaf(-kB2, d[2], d[4]), oa = __builtin_fmaf(-kB2, d[1], d[3]);
-    const float eb = __builtin_fmaf(-kA2, d[2], d[4]), ob = __builtin_fmaf(-kA2, d[1], d[3]);
-    const float e0 = __builtin_fmaf(-kS, d[2], d[4]), o0 = __builtin_fmaf(-kS, d[3], d[5]);
-    x[0].v[e] = plus(x[0].v[e], e0);
-    x[5].v[e] = plus(x[1].v[e], o0);
-    x[1].v[e] = static_cast<T>(__builtin_fmaf(kA, oa, ea));
-    x[2].v[e] = static_cast<T>(__builtin_fmaf(-kA, oa, ea));
-    x[3].v[e] = static_cast<T>(__builtin_fmaf(kB, ob, eb));
-    x[4].v[e] = static_cast<T>(__builtin_fmaf(-kB, ob, eb));
+    row_input_channel(x, e);
 #pragma unroll
     for (int t = 0; t < 6; ++t) xr[i][t][word] = __builtin_bit_cast(unsigned, x[t]);
   };
@@ -426,10 +381,9 @@ void row_conv_kernel(RowArgs a) {
             const float m0 = TG == 0 ? x : g[0][e], mi = TG == 0 ? g[0][e] : x;
             const float sa = TG == 0 ? p + m : g[1][e], sb = TG == 0 ? g[1][e] : p + m;
             const float da = TG == 0 ? p - m : g[2][e], db = TG == 0 ? g[2][e] : p - m;
-            o[0].v[i] = static_cast<T>(m0 + sa + sb + b);
-            o[1].v[i] = static_cast<T>(__builtin_fmaf(kA, da, __builtin_fmaf(kB, db, b)));
-            o[2].v[i] = static_cast<T>(__builtin_fmaf(kA2, sa, __builtin_fmaf(kB2, sb, b)));
-            o[3].v[i] = static_cast<T>(__builtin_fmaf(kA * kA2, da, __builtin_fmaf(kB * kB2, db, mi + b)));
+            const RowOutputs out = row_outputs(m0, sa, da, mi, sb, db, b);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j].v[i] = static_cast<T>(out.o[j]);
           }
         }
 #pragma unroll
@@ -550,25 +504,53 @@ RowBox choose_box(int N, int oD, int oH, int nW, int kd, int kh, int tiles, int 
 // 68 | 60 | 74; N=16, 256 -> 256, 14x14 21 | 15 | 12.4 | 10.6; N=1, 512 -> 512, 7x7 33 | 22 | 19 | 12.  (Layers of up to 128 input
 // channels come here in 3-D or with tile 4; with tile 2 the one-kernel F(2x2, 3x3) form takes most of them, see row_preferred.)
 enum RowShape { kRowWide, kRowHalf, kRowSmall, kRowSplit };
-struct RowPlan { RowShape shape; RowBox box; long long wide_groups; };
+struct RowPlan { RowShape shape; RowBox box; long long wide_groups; int tall_images; double us; };
 
-RowPlan make_row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int steps) {
-  RowPlan p;
+RowPlan make_row_shape(int N, int oD, int oH, int nW, int kd, int kh, int K, int steps) {
+  RowPlan p{};
   const RowBox wide = choose_box(N, oD, oH, nW, kd, kh, 64, 128), half = kd == 1 ? choose_box(N, oD, oH, nW, kd, kh, 64, 64) : wide;
   const long long n_wide = wide.boxes * ceil_div(K, 128), n_half = half.boxes * ceil_div(K, 64);
   p.wide_groups = n_wide;
   const RowBox small = choose_box(N, oD, oH, nW, kd, kh, 32, 64);
+  const double us_small = 1.2 * steps * kd + 4;
   if (steps >= 4) {
     const RowBox split = choose_box(N, oD, oH, nW, kd, kh, 32, 32);
-    if (split.boxes * ceil_div(K, 32) <= kCus) { p.shape = kRowSplit; p.box = split; return p; }
+    if (split.boxes * ceil_div(K, 32) <= kCus) { p.shape = kRowSplit; p.box = split; p.us = us_small; return p; }
   }
-  if (small.boxes * ceil_div(K, 64) <= kCus) { p.shape = kRowSmall; p.box = small; return p; }
+  if (small.boxes * ceil_div(K, 64) <= kCus) { p.shape = kRowSmall; p.box = small; p.us = us_small; return p; }
   // rounds of the chip; of two workgroups per CU one starts as soon as another ends, so their last round is not a whole one.
   // 3-D boxes of the half shape take two units of input per thread
   const double t_wide = n_wide <= kCus ? 0.86 : 0.92 * (double)((n_wide + kCus - 1) / kCus), t_half = (kd == 1 ? 1.0 : 1.2) * (n_half / (2.0 * kCus) + 0.12);
   p.shape = t_wide <= t_half ? kRowWide : kRowHalf;
   p.box = p.shape == kRowWide ? wide : half;
+  p.us = std::min(t_wide, t_half) * ((kd == 1 ? 2.45 : 6.9) * steps + 7) / 0.92;
   return p;
+}
+
+// The first `tall_images` of a batch in tall boxes (conv_row_tall.hip), the rest in the shape above.  A tall box takes the CU
+// that has it 2.1 us per 16 channels and plane of taps and 10.5 beside them, so a batch is worth cutting where its last round
+// would be nearly empty: N=64 256 -> 256 channels, 56x56 has 784 boxes, three rounds and sixteen boxes; 61 images fill the
+// three and the other three images take 12 us.  The model's constants are measured ones (fp16, us, this shape alone in whole
+// rounds | a box: 512 -> 512, 28x28 157 | 78 for 32 half blocks, 256 -> 256, 56x56 175 | 44 for 16).
+RowPlan make_row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int steps) {
+  RowPlan best = make_row_shape(N, oD, oH, nW, kd, kh, K, steps);
+  const double box_us = 2.1 * 2 * steps * kd + 10.5;
+  const long long per_group = (long long)ceil_div(oH, 4) * ceil_div(K, 128), columns = (long long)oD * nW;
+  const long long boxes = ceil_div_ll(N * columns, 32) * per_group;
+  const long long groups = boxes / kCus * kCus / per_group;       // groups of 32 columns in whole rounds
+  const long long cut = groups * 32 / columns;
+  const double wide_groups = best.wide_groups;
+  for (const long long n : {(long long)N, std::min<long long>(cut, N - 1)}) {
+    if (n < 1) continue;
+    RowPlan p{};
+    if (n < N) p = make_row_shape((int)(N - n), oD, oH, nW, kd, kh, K, steps);
+    const long long rounds = ceil_div_ll(ceil_div_ll(n * columns, 32) * per_group, kCus);
+    p.us += rounds * box_us + (n < N ? 2 : 0);
+    p.tall_images = (int)n;
+    if (p.us < best.us) best = p;
+  }
+  best.wide_groups = (long long)wide_groups;
+  return best;
 }
 
 // The search over boxes takes some microseconds: the last plans of a host thread are kept.
@@ -674,8 +656,9 @@ bool row_preferred(const wc_conv_desc* d) {
   return kd == 1 ? 10.5 * products < 1500.0 * (C + K) + C * K : 3.6 * products < 512.0 * (C + K) + C * K;
 }
 
-// x (N, D, H, W, Cx) channel-last with Cx = C rounded up to 8 (zeros beyond C), 16-byte aligned
-int row_conv(const wc_conv_desc* d, const void* x, int n_images, const void* U, const void* bias, void* y, void* stream) {
+// x (N, D, H, W, Cx) channel-last with Cx = C rounded up to 8 (zeros beyond C), 16-byte aligned; images first_image ..
+// + n_images of the batch
+int row_conv(const wc_conv_desc* d, const void* x, int first_image, int n_images, const void* U, const void* bias, void* y, void* stream) {
   WC_CHECK_ARG(row_conv_fits(d), "row form: 16-bit, stride 1, kernel rows of three taps");
   WC_CHECK_ARG(((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(U)) & 15) == 0, "row form: x and U must be 16-byte aligned");
   RowArgs a{};
@@ -688,15 +671,26 @@ int row_conv(const wc_conv_desc* d, const void* x, int n_images, const void* U, 
   a.x_bytes = (int)((long long)a.N * a.D * a.H * a.W * a.C * 2);
   a.u_bytes = (int)(row_u_elems(d) * 2);
   const int force = test_gemm_config();
+  // the shapes are the whole batch's, so that the passes of a batch add in the order of the batch in one pass
+  RowPlan plan = row_plan(d->N, a.oD, a.oH, a.nW, d->kernel[0], d->kernel[1], a.K, a.steps);
+  if (force >= 16 && force <= 19) { plan.shape = (RowShape)(force - 16); plan.tall_images = 0; }
+  if (force == 21) plan.tall_images = d->N;
+  const int tall = std::min(std::max(plan.tall_images - first_image, 0), n_images);
+  if (tall > 0) {
+    const int rc = tall_row_conv(d, x, tall, U, bias, y, stream);
+    if (rc || tall == n_images) return rc;
+    a.x = static_cast<const unsigned char*>(x) + (long long)tall * a.D * a.H * a.W * a.C * 2;
+    a.y = static_cast<unsigned char*>(y) + (long long)tall * a.oD * a.oH * a.oW * a.K * 2;
+    a.N -= tall;
+    a.x_bytes = (int)((long long)a.N * a.D * a.H * a.W * a.C * 2);
+  }
   return dispatch_dtype(d->dtype, [&](auto t) -> int {
     using T = decltype(t);
     if constexpr (sizeof(T) == 2) {
       auto go = [&](auto kd, auto kh) -> int {
         constexpr int KD = decltype(kd)::value, KH = decltype(kh)::value;
-        // the shape is the whole batch's, so that the passes of a batch add in the order of the batch in one pass
-        RowPlan p = row_plan(d->N, a.oD, a.oH, a.nW, KD, KH, a.K, a.steps);
-        if (force >= 16 && force <= 19) p.shape = (RowShape)(force - 16);
-        if (a.N != d->N || (force >= 16 && force <= 19)) {
+        RowPlan p = plan;
+        if (a.N != d->N - p.tall_images || (force >= 16 && force <= 19)) {
           const int tiles = p.shape <= kRowHalf ? 64 : 32, slots = p.shape == kRowWide ? 128 : p.shape == kRowSplit ? 32 : p.shape == kRowHalf && KD > 1 ? 128 : 64;
           p.box = choose_box(a.N, a.oD, a.oH, a.nW, KD, KH, tiles, slots);
         }

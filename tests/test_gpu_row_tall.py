@@ -1,0 +1,49 @@
+"""The row form's tall boxes (conv_row_tall.hip): the bound and the operands of test_gpu_row.py, which pins the tile itself."""
+import pytest
+import torch
+
+from pytorch_winoconv_amd import engine
+from test_gpu_row import BOUND, CASES, _conv64, _err, _operands, _row
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [
+    ((1, 32, 4, 128), 128, 1), ((33, 40, 5, 4), 128, 1),              # 32 columns in one row; one column more, one row more
+    ((2, 8, 1, 260), 136, (1, 1)), ((31, 72, 9, 6), 8, 0),            # columns across images; one block of channels and 8 more
+    ((2, 64, 2, 3, 130), 129, 1), ((7, 96, 4, 6, 9), 40, (0, 1, 1)),  # tap planes beyond either end
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", CASES[2:] + EDGES)
+def test_against_fp64(dev, dtype, case, gemm_override):
+    xs, K, pad = case
+    x, w, b = _operands(xs, K, dtype)
+    gemm_override(config=21)
+    assert _err(_row(x.to(dev), w.to(dev), b.to(dev), pad), _conv64(x, w, b, pad)) <= BOUND[dtype]
+    assert _err(_row(x.to(dev), w.to(dev), None, pad), _conv64(x, w, None, pad)) <= BOUND[dtype]
+
+
+@pytest.mark.parametrize("xs,K", [((67, 64, 54, 60), 136), ((9, 40, 14, 50, 52), 129)])
+def test_several_boxes_a_workgroup(dev, xs, K, gemm_override):
+    """More boxes than CUs, the last of them partial; workgroups with one box more than others."""
+    x, w, b = _operands(xs, K, torch.float16)
+    gemm_override(config=21)
+    y = _row(x.to(dev), w.to(dev), b.to(dev), 1)
+    assert _err(y, _conv64(x, w, b, 1)) <= BOUND[torch.float16]
+    assert torch.equal(_row(x.to(dev), w.to(dev), b.to(dev), 1), y)
+
+
+def test_batch_cut_in_tall_boxes_and_others(dev, gemm_override):
+    """61 of 64 images fill three rounds of tall boxes, the rest takes another shape: each image has the bits of its shape, also
+    where the batch comes in passes that do not end at the cut."""
+    x, w, b = _operands((64, 160, 56, 56), 256, torch.float16)
+    xd, wd, bd = x.to(dev), w.to(dev), b.to(dev)
+    y = _row(xd, wd, bd, 1)
+    ref = torch.nn.functional.conv2d(x[58:].double(), w.double(), b.double(), padding=1)
+    assert _err(y[58:], ref) <= BOUND[x.dtype]
+    passes = engine.conv_forward(xd, wd, bd, 1, 1, 2, chunk_images=27, row=True)
+    gemm_override(config=21)
+    tall = _row(xd, wd, bd, 1)
+    assert torch.equal(y[:61], tall[:61]) and not torch.equal(y[61:], tall[61:])
+    assert torch.equal(passes, y)
