@@ -14,7 +14,8 @@
 // conflicts.  The MFMA "A" operand is the
 // filter block and "B" the input block: a lane then holds 4 consecutive output channels of
 // one tile row per accumulator group and stores them as one 8-byte (fp16) / 16-byte (fp32)
-// write.  fp16 and bf16 accumulate in fp32; fp32 uses v_mfma_f32_32x32x2_f32.
+// write.  fp16 and bf16 accumulate in fp32; fp32 uses three bf16 parts per operand (Split), its direct form
+// v_mfma_f32_32x32x2_f32.
 //
 // Plans whose pieces share one transformed input read V at a row offset per piece: gemm_kernel
 // with SHIFT walks the operand pointer piece by piece; gemm_rows_kernel serves the pieces of one
@@ -111,6 +112,27 @@ typedef uint32_t Chunk16 __attribute__((ext_vector_type(4)));   // one 16-byte g
 // is conflict-free for 128-byte and for 256-byte wide bank sets alike.
 __device__ __forceinline__ int swizzle(int r) { return (((r >> 1) ^ (r >> 3)) & 1) | (((r >> 2) & 1) << 1); }
 
+// fp32 products of the Winograd domain on the bf16 matrix cores: x = h + m + l with three bf16 numbers of 8 bits each, h the
+// upper half of x, m and l rounded to nearest, which together are x exactly, and x y = hh + hm + mh + mm + hl + lh, six of
+// the nine products.  What is left out, ml + lm + ll, is at most 2^-22 and in the root mean square 2^-26 of the product, less
+// than a rounding of fp32, and a sum of 16 products is rounded six times where eight v_mfma_f32_32x32x2_f32 round it eight.
+// 16-bit products have 16 times the rate of fp32 ones.
+struct Split { uint32_t h[2], m[2], l[2]; };
+__device__ __forceinline__ Split split_bf16(Chunk16 c) {
+  Split s;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const uint32_t a = c[2 * i], b = c[2 * i + 1];
+    s.h[i] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+    const float ra = __uint_as_float(a) - __uint_as_float(a & 0xffff0000u), rb = __uint_as_float(b) - __uint_as_float(b & 0xffff0000u);
+    const Pack<bf16_t, 2> m = {{static_cast<bf16_t>(ra), static_cast<bf16_t>(rb)}};
+    s.m[i] = __builtin_bit_cast(uint32_t, m);
+    const Pack<bf16_t, 2> l = {{static_cast<bf16_t>(ra - __uint_as_float(s.m[i] << 16)), static_cast<bf16_t>(rb - __uint_as_float(s.m[i] & 0xffff0000u))}};
+    s.l[i] = __builtin_bit_cast(uint32_t, l);
+  }
+  return s;
+}
+
 template <typename T, int WM, int WN, int BK, int NWP = 2, int NWK = 2, bool SHIFT = false, bool DIRECT = false, bool CLASSES = false>
 __global__ __launch_bounds__(64 * NWP * NWK, (WM * WN <= 8 && NWP * NWK == 4 ? 2 : 1))
 void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
@@ -125,7 +147,9 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
   constexpr int ROWS = BM + BN;
   constexpr int RPP = NT / CPR;                    // rows covered by one pass of the workgroup
   constexpr int NLOAD = ROWS / RPP;
-  constexpr int STAGE = ROWS * LDS_STRIDE;         // elements per LDS stage
+  constexpr bool SPLIT = sizeof(T) == 4 && !DIRECT;
+  constexpr int PLANE = ROWS * 32;                 // SPLIT: bytes of one of the three parts of a stage, rows of 16 bf16
+  constexpr int STAGE = SPLIT ? 3 * PLANE / 4 : ROWS * LDS_STRIDE;         // elements per LDS stage
   static_assert(ROWS % RPP == 0 && BM % RPP == 0, "tile rows must be a multiple of the load pass");
   static_assert(CPR == 4 && RPP % 16 == 0, "the swizzle assumes 64-byte rows and passes of whole 16-row groups");
 
@@ -173,14 +197,15 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
       const int k = min(k0 + row - BM, g.K - 1);
       gptr[i] = Ut + (long long)k * g.Cp + lpart * EPC;
     }
-    loff[i] = row * LDS_STRIDE + (lpart ^ swizzle(row)) * EPC;
+    // SPLIT (bytes): rows of two 16-byte chunks, exchanged in every other eight rows: fragment reads meet every bank once
+    loff[i] = SPLIT ? row * 32 + ((lpart >> 1) ^ ((row >> 3) & 1)) * 16 + (lpart & 1) * 8 : row * LDS_STRIDE + (lpart ^ swizzle(row)) * EPC;
   }
 
   // The direct form requests a reduction block two stages before it is multiplied where the registers allow it: a stage of
   // the smaller tiles is over before its pixels, behind their bounds checks, are there (fp16 stride 2, us, one stage | two:
   // N=1 128 -> 128, 56x56 16.5 | 12.7; N=2 256 -> 512, 15x17 30 | 22; N=64 256 -> 512, 28x28 55 | 51; the 256 x 128 tile
   // spills that way, N=32 128 -> 128, 112x112 63 | 77).
-  constexpr int AHEAD = DIRECT && sizeof(T) == 2 && WM * WN <= 4 ? 2 : 1;
+  constexpr int AHEAD = ((DIRECT && sizeof(T) == 2) || SPLIT) && WM * WN <= 4 ? 2 : 1;
   Chunk16 regs[AHEAD][NLOAD];
   // `vshift`: what the V operand has jumped by at reduction block kt (rows i < BM / RPP are V's)
   int tap_y = 0, tap_x = 0, tap_cb = 0;             // direct form: the tap and channel block of the next load
@@ -207,6 +232,18 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
     }
   };
   auto lstore = [&](auto set_c, int buf) {
+    if constexpr (SPLIT) {
+      typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+      unsigned char* const to = lds_raw + buf * 3 * PLANE;
+#pragma unroll
+      for (int i = 0; i < NLOAD; ++i) {
+        const Split p = split_bf16(regs[decltype(set_c)::value][i]);
+        *reinterpret_cast<u2*>(to + loff[i]) = u2{p.h[0], p.h[1]};
+        *reinterpret_cast<u2*>(to + PLANE + loff[i]) = u2{p.m[0], p.m[1]};
+        *reinterpret_cast<u2*>(to + 2 * PLANE + loff[i]) = u2{p.l[0], p.l[1]};
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < NLOAD; ++i) *reinterpret_cast<Chunk16*>(lds + buf * STAGE + loff[i]) = regs[decltype(set_c)::value][i];
   };
@@ -254,6 +291,27 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
     const int cur = kt & 1;
     if (kt + AHEAD < nk) { next_block(); gload(set_c, kt + AHEAD, vshift); }
     const T* st = lds + cur * STAGE;
+    if constexpr (SPLIT) {
+      const unsigned char* const sb = lds_raw + cur * 3 * PLANE + (lhi ^ ((l32 >> 3) & 1)) * 16;
+      bf16x8 xf[3][WM], wf[3][WN];
+#pragma unroll
+      for (int q : {2, 0, 1}) {
+#pragma unroll
+        for (int i = 0; i < WM; ++i) xf[q][i] = *reinterpret_cast<const bf16x8*>(sb + q * PLANE + (wp * WM * 32 + i * 32 + l32) * 32);
+#pragma unroll
+        for (int j = 0; j < WN; ++j) wf[q][j] = *reinterpret_cast<const bf16x8*>(sb + q * PLANE + (BM + wk * WN * 32 + j * 32 + l32) * 32);
+      }
+      static_for<0, 6>([&](auto q_c) {             // the small products first: they are rounded to less while the sum is still small
+        constexpr int q = decltype(q_c)::value, qx = q == 1 ? 2 : q == 2 || q == 4 ? 1 : 0, qw = q == 0 ? 2 : q == 2 || q == 3 ? 1 : 0;
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+          for (int j = 0; j < WN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[qw][j], xf[qx][i], acc[i][j], 0, 0, 0);
+      });
+      if (kt + 1 < nk) lstore(ic<AHEAD == 2 ? 1 - set : 0>{}, cur ^ 1);
+      __syncthreads();
+      return;
+    }
     // fragments of step kk+1 are read from LDS while the MFMAs of step kk run
     constexpr int KK = BK / MF::kstep;
     typename MF::Frag xf[2][WM], wf[2][WN];
@@ -361,7 +419,7 @@ static GemmConfig make_config() {
   constexpr int EPC = 16 / sizeof(T);
   constexpr int BM = 32 * NWP * WM, BN = 32 * NWK * WN;
   constexpr int EI = sizeof(T) == 4 ? 1 : (NWP * NWK == 4 ? WM : WM / 2);
-  constexpr size_t stages = (size_t)2 * (BM + BN) * BK * sizeof(T);
+  constexpr size_t stages = (size_t)2 * (BM + BN) * (sizeof(T) == 4 && !DIRECT ? 96 : BK * sizeof(T));
   constexpr size_t out_tile = (size_t)32 * NWP * EI * (BN + EPC) * sizeof(T);
   return GemmConfig{&gemm_kernel<T, WM, WN, BK, NWP, NWK, SHIFT, DIRECT>, BM, BN, BK,
                     stages > out_tile ? stages : out_tile, 64 * NWP * NWK};
@@ -657,21 +715,27 @@ template <> struct Configs<float> {
 
 // fp16: the largest tile that still gives the 256 CUs about two workgroups each and does not
 // waste more than half a tile on the channel axis (the big tile moves the fewest bytes, and the
-// fp16 product is bound by memory).  fp32: always the 64 x 64 tile.  One reduction step of an
-// fp32 stage is only 16 deep, so a big tile has too little work per stage to cover the load
-// latency with one or two workgroups per CU; the small tile runs 4+ workgroups per CU and
-// measured 1.0-1.3x faster than every larger tile on all VGG-16 layer shapes (N = 8), within 4 %
-// of the best tile on each.
+// fp16 product is bound by memory).
 template <typename T>
 static GemmConfig choose(int T_, int P, int K, int Cp) {
   const int force = test_gemm_config();
   if (force >= 0 && force < Configs<T>::n) return Configs<T>::get(force);
   constexpr int n_auto = 5;
-  // fp32 is bound by the MFMA rate: the 64 x 64 tile fills the chip best, except for long
-  // reductions with thousands of tiles, where 128 x 128 halves the LDS traffic (measured 5-9 %
-  // faster at Cp >= 256).  A reduction of <= 64 channels is one or two stages: small tiles again.
+  // fp32 (three bf16 parts, see Split).  us, 256x128 | 128x128 | 128x64 | 64x64 tile, T=36 (the fp32 instructions took):
+  //   P 1568, 256 -> 256: 50 | 58 | 64 | 66 (87)       1568, 512 -> 512: 173 | 180 | 202 | 224 (280)
+  //   6272, 128 -> 256: 113 | 107 | 123 | 140 (152)    6272, 128 -> 128: 66 | 61 | 65 | 72 (84)
+  //   25088, 64 -> 128: 153 | 141 | 164 | 178 (199)    25088, 64 -> 64: 165 | 134 | 100 | 102 (109)
+  //   392, 512 -> 512: 72 | 67 | 68 | 64 (81)          T=64, 3136, 64 -> 64: 36 | 31 | 25 | 22 (23)
+  //   T=16, 6272, 256 -> 256: 109 | 95 | 102 | 112 (145)   T=16, 12544, 96 -> 160: 81 | 74 | 69 | 76 (82)
+  // The larger the tile, the less its operands are split and loaded over again; it takes whole rounds of the chip (two
+  // workgroups of 256x128 to a CU, three of 128x128) and channels that fill it.
   if constexpr (sizeof(T) == 4) {
-    if (Cp >= 256 && K >= 128 && (long long)ceil_div(P, 128) * ceil_div(K, 128) * T_ >= 2048) return Configs<T>::get(1);
+    auto blocks = [&](int bm, int bn) { return (long long)ceil_div(P, bm) * ceil_div(K, bn) * T_; };
+    const bool wide = K > 64 && (K % 128 == 0 || K % 128 > 64);
+    const long long b0 = blocks(256, 128);
+    if (wide && Cp >= 256 && ((b0 >= 400 && b0 <= 512) || b0 >= 960)) return Configs<T>::get(0);
+    if (wide && blocks(128, 128) >= 768) return Configs<T>::get(1);
+    if (blocks(128, 64) >= 4096) return Configs<T>::get(3);
   }
   if (sizeof(T) == 4 || Cp <= 64) return Configs<T>::get(n_auto - 1);
   // Long reductions over many output channels: the 128 x 256 tile of eight wavefronts reads V
