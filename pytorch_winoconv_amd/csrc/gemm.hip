@@ -201,12 +201,15 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
     loff[i] = SPLIT ? row * 32 + ((lpart >> 1) ^ ((row >> 3) & 1)) * 16 + (lpart & 1) * 8 : row * LDS_STRIDE + (lpart ^ swizzle(row)) * EPC;
   }
 
-  // The direct form requests a reduction block two stages before it is multiplied where the registers allow it: a stage of
+  // A reduction block is requested two stages before it is multiplied where the registers allow it, in the direct form, of
+  // fp32 in three parts and on the smallest tile of all (T=36, 64x64, fp16, us, one stage | two: P 98, 512 -> 512 9.0 | 8.5;
+  // P 784, T=16, 64 -> 64 3.9 | 3.5; fp32 stride 2, N=1 128 -> 128, 56x56 42 | 35): a stage of
   // the smaller tiles is over before its pixels, behind their bounds checks, are there (fp16 stride 2, us, one stage | two:
   // N=1 128 -> 128, 56x56 16.5 | 12.7; N=2 256 -> 512, 15x17 30 | 22; N=64 256 -> 512, 28x28 55 | 51; the 256 x 128 tile
   // spills that way, N=32 128 -> 128, 112x112 63 | 77).
-  constexpr int AHEAD = ((DIRECT && sizeof(T) == 2) || SPLIT) && WM * WN <= 4 ? 2 : 1;
+  constexpr int AHEAD = (((DIRECT && sizeof(T) == 2) || SPLIT) && WM * WN <= 4) || WM * WN == 1 ? 2 : 1;
   Chunk16 regs[AHEAD][NLOAD];
+  bool in_image[AHEAD][DIRECT ? BM / RPP : 1];
   // `vshift`: what the V operand has jumped by at reduction block kt (rows i < BM / RPP are V's)
   int tap_y = 0, tap_x = 0, tap_cb = 0;             // direct form: the tap and channel block of the next load
   auto gload = [&](auto set_c, int kt, long long vshift) {
@@ -217,8 +220,11 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
         if (i < BM / RPP) {
           const int j = i < BM / RPP ? i : 0;
           const bool inside = (unsigned)(iy0[j] + tap_y) < (unsigned)g.H && (unsigned)(ix0[j] + tap_x) < (unsigned)g.W;
-          regs[set][i] = Chunk16{0u, 0u, 0u, 0u};
-          if (inside) regs[set][i] = *reinterpret_cast<const Chunk16*>(gptr[i] + kt * BK + vshift);
+          // always a load, of the first pixel where the tap is outside: behind a branch the compiler does not know how many
+          // loads are in flight and waits for all of them (N=32 128 -> 128, 112x112, fp16 at stride 2 69 us, now 63.5)
+          const T* const from = inside ? gptr[i] + kt * BK + vshift : Vt;
+          regs[set][i] = *reinterpret_cast<const Chunk16*>(from);
+          in_image[set][j] = inside;
           continue;
         }
       }
@@ -245,7 +251,13 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
       return;
     }
 #pragma unroll
-    for (int i = 0; i < NLOAD; ++i) *reinterpret_cast<Chunk16*>(lds + buf * STAGE + loff[i]) = regs[decltype(set_c)::value][i];
+    for (int i = 0; i < NLOAD; ++i) {
+      Chunk16 c = regs[decltype(set_c)::value][i];
+      if constexpr (DIRECT) {
+        if (i < BM / RPP && !in_image[decltype(set_c)::value][i < BM / RPP ? i : 0]) c = Chunk16{0u, 0u, 0u, 0u};
+      }
+      *reinterpret_cast<Chunk16*>(lds + buf * STAGE + loff[i]) = c;
+    }
   };
 
   const int lane = tid & 63, wave = tid >> 6;
