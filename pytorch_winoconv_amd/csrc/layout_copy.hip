@@ -3,10 +3,16 @@
 // (dwm.py:129-133,143-144; Split_and_Concat.py:25,47,64,81) for the plans whose transform kernels cannot read or
 // write channel-first memory themselves.
 //
-// Per image this is the transpose of an R x Q matrix into a Q x R one.  A workgroup moves a 64 x 64 tile
-// through LDS (pitch 65 elements: the row-wise writes and the column-wise reads both touch every bank once);
-// lanes run along the contiguous axis on both sides.
+// Per image this is the transpose of an R x Q matrix into a Q x R one.  A thread turns a square block of 16 bytes a side
+// in registers (8 x 8 elements of two bytes, 4 x 4 of four); the 64 blocks of a wavefront form a square, so that every access
+// of a wavefront is eight runs of 128 contiguous bytes.  Rows start at any multiple of the element size: accesses of 16 bytes
+// need no alignment here.  No LDS and no barrier: a small copy is a few loads in flight per wavefront and its stores.  us,
+// tiles of 64 x 64 through LDS in accesses of 2 or 4 bytes | this, 16 bit: 6 x 100 x 2745 7.8 | 3.9, 64 x 256 x 3136 51 | 35 (5.8 TB/s),
+// back 50 | 35, 64 x 128 x 3136 20.4 | 18.2; 32 bit, 64 x 256 x 3136 102 | 74, 8 x 256 x 3136 12.0 | 9.9; 32 x 3 x 50176 (a thread to a
+// column) 42 | 9.
 #include "wc_common.h"
+
+#include <algorithm>
 
 namespace wc {
 
@@ -18,61 +24,56 @@ struct TransposeArgs {
   long long n_blocks;
 };
 
+typedef uint32_t Words __attribute__((ext_vector_type(4)));
+
 template <typename U>
 __global__ __launch_bounds__(256) void transpose_kernel(TransposeArgs a) {
-  __shared__ U tile[64][65];
-  const long long blk = blockIdx.x;
+  constexpr int E = 16 / sizeof(U);
+  const long long blk = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (blk >= a.n_blocks) return;
   const int tq = (int)(blk % a.tiles_q);
   const long long rest = blk / a.tiles_q;
   const int tr = (int)(rest % a.tiles_r);
   const long long n = rest / a.tiles_r;
-  const long long r0 = (long long)tr * 64, q0 = (long long)tq * 64;
-  const U* src = static_cast<const U*>(a.src) + n * a.R * a.Q;
-  U* dst = static_cast<U*>(a.dst) + n * a.Rd * a.Q;
-  const int lx = threadIdx.x & 63, ly = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  // loads: the lanes of a row of blocks run along Q; stores: along R
+  long long q0 = (long long)tq * 8 * E + (lane & 7) * E, r0 = (long long)tr * 8 * E + (lane >> 3) * E;
+  if (q0 >= a.Q || r0 >= a.Rd) return;
+  // a block that would reach beyond the end overlaps its neighbour instead, and both write the same values there
+  if (q0 + E > a.Q) q0 = a.Q - E;
+  if (r0 + E > a.Rd) r0 = a.Rd - E;
+  const U* const src = static_cast<const U*>(a.src) + (n * a.R + r0) * a.Q + q0;
+  U* const dst = static_cast<U*>(a.dst) + (n * a.Q + q0) * a.Rd + r0;
+  Words in[E];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int r = ly + 4 * i;
-    if (r0 + r < a.Rd && q0 + lx < a.Q) tile[r][lx] = r0 + r < a.R ? src[(r0 + r) * a.Q + q0 + lx] : U(0);
+  for (int r = 0; r < E; ++r) {
+    in[r] = Words{0u, 0u, 0u, 0u};
+    if (r0 + r < a.R) __builtin_memcpy(&in[r], src + r * a.Q, 16);
   }
-  __syncthreads();
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int qq = ly + 4 * i;
-    if (q0 + qq < a.Q && r0 + lx < a.Rd) dst[(q0 + qq) * a.Rd + r0 + lx] = tile[lx][qq];
+  for (int c = 0; c < E; ++c) {
+    Words out;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      out[k] = sizeof(U) == 4 ? in[k][c % 4]
+                              : __builtin_amdgcn_perm(in[(2 * k + 1) % E][c / 2 % 4], in[2 * k % E][c / 2 % 4], c % 2 ? 0x07060302u : 0x05040100u);
+    __builtin_memcpy(dst + c * a.Rd, &out, 16);
   }
 }
 
-// The same for 2-byte elements with both extents even and 4-byte aligned tensors: every global access moves a
-// pair of elements (a wavefront reads and writes 256 contiguous bytes per tile row instead of 128).  The tile
-// sits in LDS as [r][q] with a pitch of 66 elements: the pair-wise writes along q are consecutive words, and
-// the reads of one column q for two consecutive rows land in 32 different banks across the 32 row pairs.
-__global__ __launch_bounds__(256) void transpose_pairs_kernel(TransposeArgs a) {
-  __shared__ unsigned short tile[64 * 66];
-  const long long blk = blockIdx.x;
-  const int tq = (int)(blk % a.tiles_q);
-  const long long rest = blk / a.tiles_q;
-  const int tr = (int)(rest % a.tiles_r);
-  const long long n = rest / a.tiles_r;
-  const long long r0 = (long long)tr * 64, q0 = (long long)tq * 64;
-  const unsigned short* src = static_cast<const unsigned short*>(a.src) + n * a.R * a.Q;
-  unsigned short* dst = static_cast<unsigned short*>(a.dst) + n * a.Rd * a.Q;
-  const int lx = threadIdx.x & 31, ly = threadIdx.x >> 5;      // 32 pairs per row, 8 rows per pass
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int r = ly + 8 * i;
-    if (r0 + r < a.Rd && q0 + 2 * lx < a.Q)
-      *reinterpret_cast<unsigned*>(&tile[r * 66 + 2 * lx]) = r0 + r < a.R ? *reinterpret_cast<const unsigned*>(src + (r0 + r) * a.Q + q0 + 2 * lx) : 0u;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int qq = ly + 8 * i;
-    if (q0 + qq < a.Q && r0 + 2 * lx < a.Rd) {
-      const unsigned v = (unsigned)tile[(2 * lx) * 66 + qq] | ((unsigned)tile[(2 * lx + 1) * 66 + qq] << 16);
-      *reinterpret_cast<unsigned*>(dst + (q0 + qq) * a.Rd + r0 + 2 * lx) = v;
-    }
-  }
+// Matrices narrower than a block on either side: a thread takes all of the narrow side
+template <typename U>
+__global__ __launch_bounds__(256) void transpose_narrow_kernel(TransposeArgs a) {
+  const bool rows = a.Rd < a.Q;                    // few rows: a thread takes a column
+  const long long wide = rows ? a.Q : a.Rd, i = (long long)blockIdx.x * 256 + threadIdx.x;
+  const long long n = i / wide, at = i - n * wide;
+  if (i >= a.n_blocks) return;
+  const U* const src = static_cast<const U*>(a.src) + n * a.R * a.Q;
+  U* const dst = static_cast<U*>(a.dst) + n * a.Rd * a.Q;
+  if (rows)
+    for (int r = 0; r < (int)a.Rd; ++r) dst[at * a.Rd + r] = r < a.R ? src[r * a.Q + at] : U(0);
+  else
+    for (int q = 0; q < (int)a.Q; ++q) dst[q * a.Rd + at] = at < a.R ? src[at * a.Q + q] : U(0);
 }
 
 static int transpose_padded(const void* src, void* dst, long long n, long long R, long long Q, long long Rd, int elem_size, void* stream) {
@@ -80,17 +81,19 @@ static int transpose_padded(const void* src, void* dst, long long n, long long R
   WC_CHECK_ARG(elem_size == 2 || elem_size == 4, "layout copy: element size %d", elem_size);
   TransposeArgs a;
   a.src = src; a.dst = dst; a.R = R; a.Q = Q; a.Rd = Rd;
-  a.tiles_r = (int)ceil_div_ll(Rd, 64); a.tiles_q = (int)ceil_div_ll(Q, 64);
-  a.n_blocks = n * a.tiles_r * a.tiles_q;
-  WC_CHECK_ARG(a.n_blocks < (1ll << 31), "layout copy: problem too large");
-  const bool pairs = elem_size == 2 && Rd % 2 == 0 && Q % 2 == 0 &&
-                     ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 3) == 0;
-  if (pairs)
-    hipLaunchKernelGGL(transpose_pairs_kernel, dim3((unsigned)a.n_blocks), dim3(256), 0, as_stream(stream), a);
-  else if (elem_size == 2)
-    hipLaunchKernelGGL(transpose_kernel<unsigned short>, dim3((unsigned)a.n_blocks), dim3(256), 0, as_stream(stream), a);
-  else
-    hipLaunchKernelGGL(transpose_kernel<unsigned>, dim3((unsigned)a.n_blocks), dim3(256), 0, as_stream(stream), a);
+  const int block = 16 / elem_size, side = 8 * block;
+  const bool narrow = Rd < block || Q < block;
+  a.tiles_r = (int)ceil_div_ll(Rd, side); a.tiles_q = (int)ceil_div_ll(Q, side);
+  a.n_blocks = narrow ? n * std::max(Rd, Q) : n * a.tiles_r * a.tiles_q;
+  const long long groups = ceil_div_ll(a.n_blocks, narrow ? 256 : 4);
+  WC_CHECK_ARG(groups < (1ll << 31), "layout copy: problem too large");
+  auto launch = [&](auto u) {
+    using U = decltype(u);
+    const auto fn = narrow ? transpose_narrow_kernel<U> : transpose_kernel<U>;
+    hipLaunchKernelGGL(fn, dim3((unsigned)groups), dim3(256), 0, as_stream(stream), a);
+  };
+  if (elem_size == 2) launch((unsigned short)0);
+  else launch(0u);
   WC_CHECK_LAUNCH("transpose_kernel");
   return WC_OK;
 }

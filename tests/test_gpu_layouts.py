@@ -135,3 +135,20 @@ def test_forward_with_channel_first_tensors(dev, dtype, tol, case, host_layer):
     om = (2, 4, 4) if (used == 4 and nd == 3) else used
     want = ow.dwm_conv(x, w, b, stride, pad, om, DISC[dtype], stacked=form)
     assert _rel(y, want) <= tol
+
+
+@pytest.mark.parametrize("es,block", [(2, 8), (4, 4)])
+def test_layout_copy_around_its_blocks(dev, es, block):
+    """Extents around the square blocks of 16 bytes and the squares of 64 of them, tensors that start at any element, and
+    nothing written beside the result."""
+    lib = _lib.load()
+    dt = torch.int16 if es == 2 else torch.int32
+    for c in (1, block - 1, block, block + 1, 8 * block - 1, 8 * block + 3):
+        for s in (1, block - 1, block, 2 * block - 1, 8 * block, 16 * block + 1):
+            for at in (0, 1):
+                x = torch.randint(-30000, 30000, (3, c, s), dtype=dt, device=dev)
+                src, out = torch.zeros(x.numel() + at, dtype=dt, device=dev)[at:], torch.full((x.numel() + at + 8,), 7, dtype=dt, device=dev)
+                src.copy_(x.reshape(-1))
+                _lib.check(lib.wc_layout_copy(engine._ptr(src), engine._ptr(out[at:]), 3, c, s, 1, es, engine._stream(x)))
+                assert torch.equal(out[at:at + x.numel()].view(3, s, c), x.transpose(1, 2)), (c, s, at)
+                assert bool((out[at + x.numel():] == 7).all()) and bool((out[:at] == 7).all())
