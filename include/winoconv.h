@@ -130,9 +130,9 @@ typedef struct {
                     *    (3 / 5 / 7 kernel rows of at most 8 taps, U (K, kH, 8, 4)) and 3-D 3x3x3 at stride 1 (rows of at
                     *    most 4 taps, U (K, 9, 4, 4)) - which have kernels of their own.  wc_conv_forward, wc_filter_transform,
                     *    wc_conv_workspace_bytes and wc_conv_u_elems honour it; the other stage functions do not apply. */
-  int row;         /* 1: the row form: the tile F(4,3) along the width axis only, the taps of the other axes in the reduction,
-                    *    everything in one kernel (no V or M in memory; sums in fp32 until the output transform, so the
-                    *    error is that of tile 2 or smaller).  16-bit types, stride 1, 3x3 and 3x3x3 kernels; m, stacked and
+  int row;         /* 1: the row form: the tile F(4,3), for 5x5 kernels F(2,5), along the width axis only, the taps of the other axes in
+                    *    the reduction, everything in one kernel (no V or M in memory; sums in fp32 until the output transform, so
+                    *    the error is that of tile 2 or smaller).  16-bit types, stride 1, 3x3, 3x3x3 and 5x5 kernels; m, stacked and
                     *    whole_kernel are ignored, U is in the kernel's own order.  No counterpart in the reference.
                     *    On entry to wc_conv_auto: -1 = may be chosen, 0 = never; wc_conv_forward,
                     *    wc_filter_transform, wc_conv_workspace_bytes and wc_conv_u_elems honour 1. */
@@ -185,7 +185,7 @@ int wc_plan_conv(const wc_conv_desc* desc, wc_plan* plan);
  * three-tap pieces on F(3,3) apply (fp16, 2-D, stride 1, at least 3 taps per axis and 5 on one), else by 2;
  * desc->direct == -1 on entry: the direct form is never chosen (and the field comes back 0); desc->row == -1 with
  * desc->stacked == -1: the row form is chosen (row = 1) - with m = 4 where it measured faster than that tile, else wherever the
- * one-kernel F(2x2,3x3) form does not run -, otherwise the field comes back 0.
+ * one-kernel F(2x2,3x3) form does not run; 5x5 layers of 33 to 40 output channels never -, otherwise the field comes back 0.
  * The caller reads the tile that will really be used back from desc->m.  No counterpart in the reference,
  * which has one form only (src/base_conv_launchers.cu:282-399).  Every other function wants stacked >= 0. */
 int wc_conv_auto(wc_conv_desc* desc);

@@ -1,5 +1,5 @@
-// One-kernel convolution on the tile F(4, 3) along the width axis only ("row form"): 16-bit types, stride 1, kernels
-// whose rows have three taps.
+// One-kernel convolution on the tile F(4, 3) along the width axis only ("row form"): 16-bit types, stride 1, 3x3 and 3x3x3
+// kernels.  5x5 kernels run on F(2, 5), which has the same six points and so the same V: below, 4 w is 2 w and A^T has two rows.
 //
 //   y[o_d, o_h, 4 w + i] = sum_t A^T[i][t]  sum_(r_d, r_h) sum_c  U[r][t][k][c]  V[o_d + r_d, o_h + r_h, w][t][c]
 //   V[., w][t] = sum_j B^T[t][j] x[., 4 w + j],      U[r][t] = sum_j G[t][j] w[r, j]
@@ -21,7 +21,7 @@ namespace {
 struct RowArgs {
   const void* x; const void* U; const void* bias; void* y;
   int N, D, H, W, C, K;           // x (N, D, H, W, C), y (N, oD, oH, oW, K)
-  int oD, oH, oW, nW;             // nW tiles of 4 outputs per row
+  int oD, oH, oW, nW;             // nW tiles of 4 (5x5: 2) outputs per row
   int pd, ph, pw;
   int bn, bd, bh, bw;             // output box of a workgroup: images, planes, rows, tiles of a row
   FastDiv f_bw, f_bh, f_bd, f_prow, f_irow;
@@ -76,10 +76,10 @@ __global__ __launch_bounds__(128 * KG * CS) __attribute__((amdgpu_waves_per_eu(2
 void row_conv_kernel(RowArgs a) {
   using Frag = typename MfmaRow<T>::Frag;
   constexpr int R = KD * KH, Q = 2 * R, NI = 3 * Q, THREADS = 128 * KG, UN = S * 4 / THREADS;
-  constexpr int TS = S * kRowPitch, BUF = 6 * TS;
-  constexpr int UD = 3, VD = 3;      // depth of the rings of filter and input fragments
+  constexpr int TS = S * kRowPitch, BUF = 6 * TS, OUT = row_outputs_of(KH);
+  constexpr int UD = Q % 3 == 0 ? 3 : 5, VD = 3;      // depth of the rings of filter and input fragments
   static_assert(RowItems<UN, NI>::ok(), "items of a step");
-  static_assert(S * 4 % THREADS == 0 && Q % UD == 0, "whole units per thread, ring of three");
+  static_assert(S * 4 % THREADS == 0 && Q % UD == 0, "whole units per thread, whole turns of the ring");
   extern __shared__ unsigned char lds_all[];
   static_assert(!STAY || CS == 1, "shares end after their box");
   // this XCD's boxes from the workgroup's own on; STAY: every (workgroups of the XCD)-th
@@ -129,7 +129,7 @@ void row_conv_kernel(RowArgs a) {
       const int in = fast_div(s, a.f_irow); s -= in * a.irow;
       const int zd = fast_div(s, a.f_prow); s -= zd * a.prow;
       const int zh = fast_div(s, a.f_bw), iw = s - zh * a.bw;
-      const int n = n0 + in, d = d0 + zd - a.pd, h = h0 + zh - a.ph, w = (w0 + iw) * 4 - a.pw;
+      const int n = n0 + in, d = d0 + zd - a.pd, h = h0 + zh - a.ph, w = (w0 + iw) * OUT - a.pw;
       const bool ok = in < a.bn && zd < sd && zh < sh && n < a.N && (unsigned)d < (unsigned)a.D && (unsigned)h < (unsigned)a.H;
       const int base = (((n * a.D + d) * a.H + h) * a.W + w) * a.C * 2 + g * 16;
 #pragma unroll
@@ -354,11 +354,11 @@ void row_conv_kernel(RowArgs a) {
         const int ti = tile_block(TG, c) * 32 + (lane & 31);
         int iw, ih, id, in;
         tile_of(ti, iw, ih, id, in);
-        const int n = at_n + in, od = at_d + id, oh = at_h + ih, ow = (at_w + iw) * 4;
+        const int n = at_n + in, od = at_d + id, oh = at_h + ih, ow = (at_w + iw) * OUT;
         const bool ok = ti < a.bn * a.bd * a.bh * a.bw && n < a.N && od < a.oD && oh < a.oH && k0 < a.K;
         T* const yp = static_cast<T*>(a.y) + ((((size_t)n * a.oD + od) * a.oH + oh) * a.oW + ow) * a.K + k0;
         const T* const bp = static_cast<const T*>(a.bias);
-        Pack<T, 8> bv, o[4];
+        Pack<T, 8> bv, o[OUT];
 #pragma unroll
         for (int e = 0; e < 8; ++e) bv.v[e] = T(0);
         if (bp) {
@@ -381,13 +381,13 @@ void row_conv_kernel(RowArgs a) {
             const float m0 = TG == 0 ? x : g[0][e], mi = TG == 0 ? g[0][e] : x;
             const float sa = TG == 0 ? p + m : g[1][e], sb = TG == 0 ? g[1][e] : p + m;
             const float da = TG == 0 ? p - m : g[2][e], db = TG == 0 ? g[2][e] : p - m;
-            const RowOutputs out = row_outputs(m0, sa, da, mi, sb, db, b);
+            const RowOutputs<OUT> out = row_outputs<OUT>(m0, sa, da, mi, sb, db, b);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) o[j].v[i] = static_cast<T>(out.o[j]);
+            for (int j = 0; j < OUT; ++j) o[j].v[i] = static_cast<T>(out.o[j]);
           }
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < OUT; ++i) {
           T* const dst = yp + (size_t)i * a.K;
           const bool in_row = ok && ow + i < a.oW;
           if constexpr (!KT) {
@@ -418,7 +418,7 @@ void row_conv_kernel(RowArgs a) {
 struct RowFilterArgs {
   const void* w; void* U;
   long long s[5];
-  int K, C, kd, kh, steps;
+  int K, C, kd, kh, kw, steps;
   long long total;
 };
 
@@ -441,22 +441,24 @@ __global__ __launch_bounds__(256) void row_filter_kernel(RowFilterArgs a) {
   Pack<T, 2> out[6];
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
-    float g[3] = {0.f, 0.f, 0.f};
+    float g[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
     if (k < a.K && c + e < a.C) {
       const T* p = static_cast<const T*>(a.w) + k * a.s[0] + (c + e) * a.s[1] + rd * a.s[2] + rh * a.s[3];
 #pragma unroll
-      for (int j = 0; j < 3; ++j) g[j] = static_cast<float>(p[j * a.s[4]]);
+      for (int j = 0; j < 5; ++j)
+        if (j < a.kw) g[j] = static_cast<float>(p[j * a.s[4]]);
     }
     // denominators: prod over the other points; 1 for 0 (a^2 b^2), 2 a^2 (a^2 - b^2) for +-a, 2 b^2 (b^2 - a^2) for +-b
     const float fa = 1.f / (2.f * kA2 * (kA2 - kB2)), fb = 1.f / (2.f * kB2 * (kB2 - kA2));
-    const float ea = __builtin_fmaf(kA2, g[2], g[0]), oa = kA * g[1];
-    const float eb = __builtin_fmaf(kB2, g[2], g[0]), ob = kB * g[1];
+    // polynomials in the square of the point: three taps leave g[3] and g[4] zero
+    const float ea = __builtin_fmaf(kA2, __builtin_fmaf(kA2, g[4], g[2]), g[0]), oa = kA * __builtin_fmaf(kA2, g[3], g[1]);
+    const float eb = __builtin_fmaf(kB2, __builtin_fmaf(kB2, g[4], g[2]), g[0]), ob = kB * __builtin_fmaf(kB2, g[3], g[1]);
     out[0].v[e] = static_cast<T>(g[0]);
     out[1].v[e] = static_cast<T>((ea + oa) * fa);
     out[2].v[e] = static_cast<T>((ea - oa) * fa);
     out[3].v[e] = static_cast<T>((eb + ob) * fb);
     out[4].v[e] = static_cast<T>((eb - ob) * fb);
-    out[5].v[e] = static_cast<T>(g[2]);
+    out[5].v[e] = static_cast<T>(a.kw == 5 ? g[4] : g[2]);
   }
   T* dst = static_cast<T*>(a.U) + ((idx >> 8) * 6) * 512 + lane * 8 + e2;
 #pragma unroll
@@ -512,7 +514,7 @@ RowPlan make_row_shape(int N, int oD, int oH, int nW, int kd, int kh, int K, int
   const long long n_wide = wide.boxes * ceil_div(K, 128), n_half = half.boxes * ceil_div(K, 64);
   p.wide_groups = n_wide;
   const RowBox small = choose_box(N, oD, oH, nW, kd, kh, 32, 64);
-  const double us_small = 1.2 * steps * kd + 4;
+  const double us_small = 0.4 * steps * kd * kh + 4;
   if (steps >= 4) {
     const RowBox split = choose_box(N, oD, oH, nW, kd, kh, 32, 32);
     if (split.boxes * ceil_div(K, 32) <= kCus) { p.shape = kRowSplit; p.box = split; p.us = us_small; return p; }
@@ -523,7 +525,7 @@ RowPlan make_row_shape(int N, int oD, int oH, int nW, int kd, int kh, int K, int
   const double t_wide = n_wide <= kCus ? 0.86 : 0.92 * (double)((n_wide + kCus - 1) / kCus), t_half = (kd == 1 ? 1.0 : 1.2) * (n_half / (2.0 * kCus) + 0.12);
   p.shape = t_wide <= t_half ? kRowWide : kRowHalf;
   p.box = p.shape == kRowWide ? wide : half;
-  p.us = std::min(t_wide, t_half) * ((kd == 1 ? 2.45 : 6.9) * steps + 7) / 0.92;
+  p.us = std::min(t_wide, t_half) * ((kd == 1 ? 0.82 * kh : 6.9) * steps + 7) / 0.92;
   return p;
 }
 
@@ -534,6 +536,7 @@ RowPlan make_row_shape(int N, int oD, int oH, int nW, int kd, int kh, int K, int
 // rounds | a box: 512 -> 512, 28x28 157 | 78 for 32 half blocks, 256 -> 256, 56x56 175 | 44 for 16).
 RowPlan make_row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int steps) {
   RowPlan best = make_row_shape(N, oD, oH, nW, kd, kh, K, steps);
+  if (kh != 3) return best;
   const double box_us = 2.1 * 2 * steps * kd + 10.5;
   const long long per_group = (long long)ceil_div(oH, 4) * ceil_div(K, 128), columns = (long long)oD * nW;
   const long long boxes = ceil_div_ll(N * columns, 32) * per_group;
@@ -596,14 +599,14 @@ int launch_row(const RowArgs& args, const RowBox& b, void* stream) {
 }  // namespace
 
 bool row_conv_fits(const wc_conv_desc* d) {
-  if (d->dtype == WC_F32 || d->stride != 1 || d->whole_kernel || d->kernel[2] != 3) return false;
-  const int kd = d->kernel[0], kh = d->kernel[1];
-  if (!((kd == 1 && kh == 3) || (kd == 3 && kh == 3))) return false;
+  if (d->dtype == WC_F32 || d->stride != 1 || d->whole_kernel) return false;
+  const int kd = d->kernel[0], kh = d->kernel[1], kw = d->kernel[2];
+  if (!((kd == 1 && kh == 3 && kw == 3) || (kd == 3 && kh == 3 && kw == 3) || (kd == 1 && kh == 5 && kw == 5 && d->ndim == 2))) return false;
   const int cp = wc_padded_channels8(d->C);
   for (int q = 0; q < 3; ++q)
     if (d->in[q] + 2 * d->pad[q] < d->kernel[q]) return false;
   const long long out = (long long)d->N * (d->in[0] + 2 * d->pad[0] - kd + 1) * (d->in[1] + 2 * d->pad[1] - kh + 1) *
-                        (d->in[2] + 2 * d->pad[2] - 2);
+                        (d->in[2] + 2 * d->pad[2] - kw + 1);
   return (long long)d->N * d->in[0] * d->in[1] * d->in[2] * cp * 2 < (1ll << 30) && out < (1ll << 31) &&
          row_u_elems(d) * 2 < (1ull << 30);
 }
@@ -617,7 +620,7 @@ int row_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5],
   RowFilterArgs a;
   a.w = w; a.U = U;
   for (int i = 0; i < 5; ++i) a.s[i] = w_strides[i];
-  a.K = d->K; a.C = d->C; a.kd = d->kernel[0]; a.kh = d->kernel[1]; a.steps = ceil_div(d->C, 32);
+  a.K = d->K; a.C = d->C; a.kd = d->kernel[0]; a.kh = d->kernel[1]; a.kw = d->kernel[2]; a.steps = ceil_div(d->C, 32);
   a.total = (long long)ceil_div(d->K, 32) * a.steps * a.kd * a.kh * 2 * 256;
   const unsigned blocks = (unsigned)ceil_div_ll(a.total, 256);
   if (d->dtype == WC_F16) hipLaunchKernelGGL(row_filter_kernel<half_t>, dim3(blocks), dim3(256), 0, as_stream(stream), a);
@@ -625,6 +628,15 @@ int row_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5],
   WC_CHECK_LAUNCH("row_filter_kernel");
   return WC_OK;
 }
+
+// 5x5 layers: F(2, 5) needs 15 products per output where the plan they replace, two- or three-tap pieces sharing one
+// transformed input, needs 20 on F(2x2, 2x2) and 11 on F(3x3, 3x3) (tile 4 in fp16), without V and M in memory, and is as
+// exact as the first (bf16 4.3e-3 | 4.5e-3 against fp64) and 2.5 times as the second (fp16 5.5e-4 | 1.4e-3).  us, row | other, bf16:
+// N=32 128 -> 128, 112x112 246 | 407, N=16 256 -> 256, 56x56 127 | 200, 64 -> 64 15 | 37, 512 -> 512, 14x14 60 | 71, N=6
+// 100 -> 150, 45x61 36 | 53, N=1 128 -> 128, 56x56 9 | 22, 64 -> 64, 28x28 7 | 16, 32 -> 32, 14x14 7 | 13; fp16 with tile 4: 248 | 365,
+// 131 | 134, 14 | 33, 57 | 62, 35 | 43, 9 | 17, 7 | 13, 7 | 12.  Layers of 33 to 40 output channels keep the other plan, though it
+// is slower (N=2 64 -> 40, 15x14 7 | 15): what has been promised to be outside of the row form stays outside.
+static bool row_preferred_5x5(const wc_conv_desc* d) { return d->K <= 32 || d->K > 40; }
 
 // Against the other forms, us (row | other), channels -> channels on P output pixels:
 //  * Where tile 2 is asked for (the modules in 3-D and in bfloat16): always.  The row form takes 9/8 (3-D: 27/16) times the products of
@@ -649,6 +661,7 @@ bool row_preferred(const wc_conv_desc* d) {
   wc_conv_desc e = *d;
   e.stacked = 0; e.direct = 0; e.row = 0;
   if (wc_plan_conv(&e, &plan) == WC_OK && thin_conv_fits(&e, &plan)) return false;
+  if (d->kernel[1] == 5) return row_preferred_5x5(d);
   if (d->m != 4) return true;
   const int kd = d->kernel[0], oD = d->in[0] + 2 * d->pad[0] - kd + 1, oH = d->in[1] + 2 * d->pad[1] - 2, oW = d->in[2] + 2 * d->pad[2] - 2;
   if (row_plan(d->N, oD, oH, ceil_div(oW, 4), kd, 3, d->K, ceil_div(d->C, 32)).wide_groups <= 3 * kCus / 2) return true;
@@ -659,14 +672,14 @@ bool row_preferred(const wc_conv_desc* d) {
 // x (N, D, H, W, Cx) channel-last with Cx = C rounded up to 8 (zeros beyond C), 16-byte aligned; images first_image ..
 // + n_images of the batch
 int row_conv(const wc_conv_desc* d, const void* x, int first_image, int n_images, const void* U, const void* bias, void* y, void* stream) {
-  WC_CHECK_ARG(row_conv_fits(d), "row form: 16-bit, stride 1, kernel rows of three taps");
+  WC_CHECK_ARG(row_conv_fits(d), "row form: 16-bit, stride 1, kernels 3x3, 3x3x3 and 5x5");
   WC_CHECK_ARG(((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(U)) & 15) == 0, "row form: x and U must be 16-byte aligned");
   RowArgs a{};
   a.x = x; a.U = U; a.bias = bias; a.y = y;
   a.N = n_images; a.D = d->in[0]; a.H = d->in[1]; a.W = d->in[2]; a.C = wc_padded_channels8(d->C); a.K = d->K;
   a.pd = d->pad[0]; a.ph = d->pad[1]; a.pw = d->pad[2];
-  a.oD = a.D + 2 * a.pd - d->kernel[0] + 1; a.oH = a.H + 2 * a.ph - d->kernel[1] + 1; a.oW = a.W + 2 * a.pw - 2;
-  a.nW = ceil_div(a.oW, 4);
+  a.oD = a.D + 2 * a.pd - d->kernel[0] + 1; a.oH = a.H + 2 * a.ph - d->kernel[1] + 1; a.oW = a.W + 2 * a.pw - d->kernel[2] + 1;
+  a.nW = ceil_div(a.oW, row_outputs_of(d->kernel[1]));
   a.steps = ceil_div(a.C, 32);
   a.x_bytes = (int)((long long)a.N * a.D * a.H * a.W * a.C * 2);
   a.u_bytes = (int)(row_u_elems(d) * 2);
@@ -674,7 +687,7 @@ int row_conv(const wc_conv_desc* d, const void* x, int first_image, int n_images
   // the shapes are the whole batch's, so that the passes of a batch add in the order of the batch in one pass
   RowPlan plan = row_plan(d->N, a.oD, a.oH, a.nW, d->kernel[0], d->kernel[1], a.K, a.steps);
   if (force >= 16 && force <= 19) { plan.shape = (RowShape)(force - 16); plan.tall_images = 0; }
-  if (force == 21) plan.tall_images = d->N;
+  if (force == 21 && d->kernel[1] == 3) plan.tall_images = d->N;
   const int tall = std::min(std::max(plan.tall_images - first_image, 0), n_images);
   if (tall > 0) {
     const int rc = tall_row_conv(d, x, tall, U, bias, y, stream);
@@ -700,13 +713,15 @@ int row_conv(const wc_conv_desc* d, const void* x, int first_image, int n_images
             // hides that input's way from memory behind the write-out and saves the start of a workgroup.  Measured, fp16, us,
             // a workgroup per box | this: N=64 256 -> 256, 56x56 196 | 185, 128 -> 128, 56x56 71 | 66, 256 -> 256, 28x28 53.3 | 52.0,
             // N=8 128 -> 128, 16x56x56 242 | 239.  Filters beyond an XCD's L2 (box_fast): 512 -> 512, N=16 28x28 48.1 | 49.3.
-            if (!filter_fits_l2(a) || ceil_div(a.K, 128) * p.box.boxes <= kCus) return launch_row<T, KD, KH, 4, 2, 128>(a, p.box, stream);
-            return launch_row<T, KD, KH, 4, 2, 128, 1, true>(a, p.box, stream);
+            if (KH == 5 || !filter_fits_l2(a) || ceil_div(a.K, 128) * p.box.boxes <= kCus) return launch_row<T, KD, KH, 4, 2, 128>(a, p.box, stream);
+            if constexpr (KH != 5) return launch_row<T, KD, KH, 4, 2, 128, 1, true>(a, p.box, stream);   // (spills with 5x5's ring)
+            [[fallthrough]];
           case kRowHalf: return launch_row<T, KD, KH, 2, 2, KD == 1 ? 64 : 128>(a, p.box, stream);
           case kRowSmall: return launch_row<T, KD, KH, 2, 1, 64>(a, p.box, stream);
           default: return launch_row<T, KD, KH, 1, 1, 32, 4>(a, p.box, stream);
         }
       };
+      if (d->kernel[1] == 5) return go(ic<1>{}, ic<5>{});
       if (d->kernel[0] == 1) return go(ic<1>{}, ic<3>{});
       return go(ic<3>{}, ic<3>{});
     }

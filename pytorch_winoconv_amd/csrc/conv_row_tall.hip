@@ -307,8 +307,8 @@ void tall_row_kernel(TallArgs a) {
             asm volatile("" : "+v"(two));          // converted here, not all of them ahead of time
             const float bv = static_cast<float>(__builtin_bit_cast(Pack<T, 2>, two).v[e % 2]);
             const float p = acc[P0][mine][first + i], m = acc[P0 + 1][mine][first + i], x = acc[X][mine][first + i];
-            const RowOutputs out = TG == 0 ? row_outputs(x, p + m, p - m, g[0][e], g[1][e], g[2][e], bv)
-                                           : row_outputs(g[0][e], g[1][e], g[2][e], x, p + m, p - m, bv);
+            const RowOutputs<4> out = TG == 0 ? row_outputs<4>(x, p + m, p - m, g[0][e], g[1][e], g[2][e], bv)
+                                           : row_outputs<4>(g[0][e], g[1][e], g[2][e], x, p + m, p - m, bv);
 #pragma unroll
             for (int j = 0; j < 4; ++j) o[j].v[i] = static_cast<T>(out.o[j]);
           }

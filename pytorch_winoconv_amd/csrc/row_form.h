@@ -1,4 +1,5 @@
-// The tile F(4, 3) of the row form (conv_row.hip, conv_row_tall.hip): its points, the arithmetic of one channel, MFMA.
+// The tile of the row form (conv_row.hip, conv_row_tall.hip), F(4, 3) or F(2, 5): its points, the arithmetic of one channel,
+// MFMA.
 //
 // Points of the tile: 0, +-a, +-1/a, infinity with a^2 = 0.425 instead of the customary 0, +-1, +-2.  They spread the
 // rounding of U and V evenly: with independent roundings of relative size e in both, the output's is 3.1 e in the root
@@ -55,12 +56,20 @@ __device__ __forceinline__ void row_input_channel(Pack<T, 2> (&x)[6], int e) {
   x[4].v[e] = static_cast<T>(__builtin_fmaf(-kB, ob, eb));
 }
 
+// Outputs of a tile: the six elements carry F(4, 3) and F(2, 5) alike, whose tiles start 4 and 2 pixels apart
+__host__ __device__ constexpr int row_outputs_of(int taps) { return 7 - taps; }
+
 // One output channel of a tile from the two halves of its elements, each reduced to (x, s, d): the element at 0 or infinity,
 // and sum and difference of the pair at +-a (first half) or +-1/a (second)
-struct RowOutputs { float o[4]; };
-__device__ __forceinline__ RowOutputs row_outputs(float m0, float sa, float da, float mi, float sb, float db, float b) {
-  return RowOutputs{{m0 + sa + sb + b, __builtin_fmaf(kA, da, __builtin_fmaf(kB, db, b)), __builtin_fmaf(kA2, sa, __builtin_fmaf(kB2, sb, b)),
-                     __builtin_fmaf(kA * kA2, da, __builtin_fmaf(kB * kB2, db, mi + b))}};
+template <int OUT> struct RowOutputs { float o[OUT]; };
+template <int OUT>
+__device__ __forceinline__ RowOutputs<OUT> row_outputs(float m0, float sa, float da, float mi, float sb, float db, float b) {
+  if constexpr (OUT == 2) {
+    return {{m0 + sa + sb + b, __builtin_fmaf(kA, da, __builtin_fmaf(kB, db, mi + b))}};
+  } else {
+    return {{m0 + sa + sb + b, __builtin_fmaf(kA, da, __builtin_fmaf(kB, db, b)), __builtin_fmaf(kA2, sa, __builtin_fmaf(kB2, sb, b)),
+             __builtin_fmaf(kA * kA2, da, __builtin_fmaf(kB * kB2, db, mi + b))}};
+  }
 }
 
 }  // namespace wc
