@@ -130,9 +130,9 @@ typedef struct {
                     *    (3 / 5 / 7 kernel rows of at most 8 taps, U (K, kH, 8, 4)) and 3-D 3x3x3 at stride 1 (rows of at
                     *    most 4 taps, U (K, 9, 4, 4)) - which have kernels of their own.  wc_conv_forward, wc_filter_transform,
                     *    wc_conv_workspace_bytes and wc_conv_u_elems honour it; the other stage functions do not apply. */
-  int row;         /* 1: the row form: the tile F(4,3), for 5x5 kernels F(2,5), along the width axis only, the taps of the other axes in
-                    *    the reduction, everything in one kernel (no V or M in memory; sums in fp32 until the output transform, so
-                    *    the error is that of tile 2 or smaller).  16-bit types, stride 1, 3x3, 3x3x3 and 5x5 kernels; m, stacked and
+  int row;         /* 1: the row form: the tile F(4,3), for 5x5 kernels F(2,5), for 7x7 kernels two of F(3,4), along the width axis only, the taps
+                    *    of the other axes in the reduction, everything in one kernel (no V or M in memory; sums in fp32 until the output transform, so
+                    *    the error is that of tile 2 or smaller).  16-bit types, stride 1, 3x3, 3x3x3, 5x5 and 7x7 kernels; m, stacked and
                     *    whole_kernel are ignored, U is in the kernel's own order.  No counterpart in the reference.
                     *    On entry to wc_conv_auto: -1 = may be chosen, 0 = never; wc_conv_forward,
                     *    wc_filter_transform, wc_conv_workspace_bytes and wc_conv_u_elems honour 1. */

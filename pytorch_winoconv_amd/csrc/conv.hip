@@ -88,7 +88,7 @@ int make_layout(const wc_conv_desc* d_in, Layout* L) {
   L->direct = d_in->direct == 1;
   L->row = d_in->row == 1;
   if (L->row) {
-    if (!row_conv_fits(d_in)) return fail(WC_ERR_UNSUPPORTED, "row form: 16-bit types, stride 1, 3x3, 3x3x3 or 5x5 kernels, x below 1 GiB");
+    if (!row_conv_fits(d_in)) return fail(WC_ERR_UNSUPPORTED, "row form: 16-bit types, stride 1, 3x3, 3x3x3, 5x5 or 7x7 kernels, x below 1 GiB");
     plain.direct = 0; plain.stacked = 0; plain.m = 2; plain.whole_kernel = 0; plain.unfused = 1; plain.row = 0;
     L->direct = false;
   }
@@ -278,7 +278,7 @@ int forward_impl(const wc_conv_desc* d, const void* x, const void* w, const int6
                  d->ndim, dt[d->dtype], d->N, d->C, d->K, d->in[0], d->in[1], d->in[2], d->kernel[0], d->kernel[1], d->kernel[2],
                  d->stride, d->pad[0], d->pad[1], d->pad[2], L.plan.m[0], L.plan.m[1], L.plan.m[2], L.plan.n_pieces, L.plan.t_total,
                  d->stacked, d->whole_kernel ? " whole-kernel tile" : "",
-                 L.row ? d->kernel[2] == 5 ? "row form: one fused kernel, F(2,5) along the width" : "row form: one fused kernel, F(4,3) along the width" : L.direct ? "direct form: the product reads x" : L.thin ? "one fused kernel" : L.fold ? "input transform (depth, height), shifted batched GEMM with the width taps along its reduction, output transform" : (L.shared ? "input transform, shifted batched GEMM, output transform"
+                 L.row ? d->kernel[2] == 7 ? "row form: one fused kernel, F(3,4) twice along the width" : d->kernel[2] == 5 ? "row form: one fused kernel, F(2,5) along the width" : "row form: one fused kernel, F(4,3) along the width" : L.direct ? "direct form: the product reads x" : L.thin ? "one fused kernel" : L.fold ? "input transform (depth, height), shifted batched GEMM with the width taps along its reduction, output transform" : (L.shared ? "input transform, shifted batched GEMM, output transform"
                                                          : "input transform, batched GEMM, output transform"),
                  L.images, L.tiles_per_image, need, L.u_bytes, L.whole() ? (size_t)0 : L.v_bytes,
                  L.whole() ? (size_t)0 : L.m_bytes, L.xcl_bytes, L.ycl_bytes,

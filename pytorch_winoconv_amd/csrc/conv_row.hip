@@ -1,5 +1,6 @@
 // One-kernel convolution on the tile F(4, 3) along the width axis only ("row form"): 16-bit types, stride 1, 3x3 and 3x3x3
-// kernels.  5x5 kernels run on F(2, 5), which has the same six points and so the same V: below, 4 w is 2 w and A^T has two rows.
+// kernels.  5x5 kernels run on F(2, 5), 7x7 kernels on two of F(3, 4) side by side, which have the same six points and so the
+// same V: below, 4 w is 2 w or 3 w and A^T has as many rows.
 //
 //   y[o_d, o_h, 4 w + i] = sum_t A^T[i][t]  sum_(r_d, r_h) sum_c  U[r][t][k][c]  V[o_d + r_d, o_h + r_h, w][t][c]
 //   V[., w][t] = sum_j B^T[t][j] x[., 4 w + j],      U[r][t] = sum_j G[t][j] w[r, j]
@@ -31,6 +32,8 @@ struct RowArgs {
   int box_fast;                   // 1: neighbouring workgroups share a channel block, 0: a box
   int steps, local_steps;         // ceil(C / 32), and the share of one of the CS groups of wavefronts that split the channels
   int x_bytes, u_bytes;
+  int lw;                         // tiles of a row of the box's input (7 taps: one more than bw)
+  FastDiv f_lw;
 };
 
 constexpr int kRowPitch = 64;     // LDS bytes per (element, row of a tile): 32 channels in four chunks of 16 bytes
@@ -75,9 +78,9 @@ template <typename T, int KD, int KH, int KG, int TB, int S, int CS, bool STAY, 
 __global__ __launch_bounds__(128 * KG * CS) __attribute__((amdgpu_waves_per_eu(2, TB == 2 ? 2 : 3)))
 void row_conv_kernel(RowArgs a) {
   using Frag = typename MfmaRow<T>::Frag;
-  constexpr int R = KD * KH, Q = 2 * R, NI = 3 * Q, THREADS = 128 * KG, UN = S * 4 / THREADS;
+  constexpr int KP = row_pieces(KH), R = KD * KH * KP, Q = 2 * R, NI = 3 * Q, THREADS = 128 * KG, UN = S * 4 / THREADS;
   constexpr int TS = S * kRowPitch, BUF = 6 * TS, OUT = row_outputs_of(KH);
-  constexpr int UD = Q % 3 == 0 ? 3 : 5, VD = 3;      // depth of the rings of filter and input fragments
+  constexpr int UD = Q % 3 == 0 ? 3 : Q % 5 == 0 ? 5 : 4, VD = 3;      // depth of the rings of filter and input fragments
   static_assert(RowItems<UN, NI>::ok(), "items of a step");
   static_assert(S * 4 % THREADS == 0 && Q % UD == 0, "whole units per thread, whole turns of the ring");
   extern __shared__ unsigned char lds_all[];
@@ -99,7 +102,7 @@ void row_conv_kernel(RowArgs a) {
     n0 = q_ / a.n_d * a.bn; d0 = b_d * a.bd; h0 = b_h * a.bh; w0 = b_w * a.bw;
   };
   go_to_box();
-  const int sd = a.bd + KD - 1, sh = a.bh + KH - 1;
+  const int sd = a.bd + KD - 1, sh = a.bh + KH - 1, lw = KP == 1 ? a.bw : a.lw;
 
   const int lane = threadIdx.x & 63, wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int cs = wave_all / (2 * KG), wave = wave_all - cs * 2 * KG, tid = wave * 64 + lane;
@@ -128,7 +131,7 @@ void row_conv_kernel(RowArgs a) {
       int s = u >> 2;
       const int in = fast_div(s, a.f_irow); s -= in * a.irow;
       const int zd = fast_div(s, a.f_prow); s -= zd * a.prow;
-      const int zh = fast_div(s, a.f_bw), iw = s - zh * a.bw;
+      const int zh = fast_div(s, KP == 1 ? a.f_bw : a.f_lw), iw = s - zh * lw;
       const int n = n0 + in, d = d0 + zd - a.pd, h = h0 + zh - a.ph, w = (w0 + iw) * OUT - a.pw;
       const bool ok = in < a.bn && zd < sd && zh < sh && n < a.N && (unsigned)d < (unsigned)a.D && (unsigned)h < (unsigned)a.H;
       const int base = (((n * a.D + d) * a.H + h) * a.W + w) * a.C * 2 + g * 16;
@@ -181,7 +184,7 @@ void row_conv_kernel(RowArgs a) {
     if (i >= a.bn * a.bd * a.bh * a.bw) i = 0;
     int iw, ih, id, in;
     tile_of(i, iw, ih, id, in);
-    vo[b] = in * a.irow + id * a.prow + ih * a.bw + iw;
+    vo[b] = in * a.irow + id * a.prow + ih * lw + iw;
   }
 
   f32x16 acc[3][TB];
@@ -229,7 +232,7 @@ void row_conv_kernel(RowArgs a) {
       cut_x(step + 2);
       u32x4 vf[VD][TB];
       auto load_v = [&](int item) {                  // element item % 3 of group item / 3
-        const int q = item / 3, r = q >> 1, off = (r / KH) * a.prow + r % KH * a.bw;
+        const int q = item / 3, r = (q >> 1) / KP, off = (r / KH) * a.prow + r % KH * lw + (q >> 1) % KP;
 #pragma unroll
         for (int b = 0; b < TB; ++b)
           vf[item % VD][b] = *reinterpret_cast<const u32x4*>(lds + cur + v_offset(vo[b] + off, (lane >> 5) + (q & 1) * 2) + item % 3 * TS);
@@ -418,7 +421,7 @@ void row_conv_kernel(RowArgs a) {
 struct RowFilterArgs {
   const void* w; void* U;
   long long s[5];
-  int K, C, kd, kh, kw, steps;
+  int K, C, kd, kh, kw, pieces, steps;
   long long total;
 };
 
@@ -426,7 +429,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void row_filter_kernel(RowFilterArgs a) {
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
   if (idx >= a.total) return;
-  const int R = a.kd * a.kh;
+  const int R = a.kd * a.kh * a.pieces;
   const int e2 = (int)(idx & 3) * 2;
   const int lane = (int)(idx >> 2) & 63;
   long long q = idx >> 8;
@@ -437,16 +440,17 @@ __global__ __launch_bounds__(256) void row_filter_kernel(RowFilterArgs a) {
   const int m = lane & 31;
   const int k = kb * 32 + ((m >> 2) & 1) * 16 + (m >> 3) * 4 + (m & 3);
   const int c = step * 32 + half * 16 + (lane >> 5) * 8 + e2;
-  const int rd = r / a.kh, rh = r - rd * a.kh;
+  const int piece = r % a.pieces, rr = r / a.pieces, rd = rr / a.kh, rh = rr - rd * a.kh;
+  const int taps = a.kw == 7 ? 3 + piece : a.kw, last = a.kw == 7 ? 3 : a.kw - 1;      // 7 taps: 0 to 2 and 3 to 6, as four each
   Pack<T, 2> out[6];
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
     float g[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
     if (k < a.K && c + e < a.C) {
-      const T* p = static_cast<const T*>(a.w) + k * a.s[0] + (c + e) * a.s[1] + rd * a.s[2] + rh * a.s[3];
+      const T* p = static_cast<const T*>(a.w) + k * a.s[0] + (c + e) * a.s[1] + rd * a.s[2] + rh * a.s[3] + piece * 3 * a.s[4];
 #pragma unroll
       for (int j = 0; j < 5; ++j)
-        if (j < a.kw) g[j] = static_cast<float>(p[j * a.s[4]]);
+        if (j < taps) g[j] = static_cast<float>(p[j * a.s[4]]);
     }
     // denominators: prod over the other points; 1 for 0 (a^2 b^2), 2 a^2 (a^2 - b^2) for +-a, 2 b^2 (b^2 - a^2) for +-b
     const float fa = 1.f / (2.f * kA2 * (kA2 - kB2)), fb = 1.f / (2.f * kB2 * (kB2 - kA2));
@@ -458,7 +462,7 @@ __global__ __launch_bounds__(256) void row_filter_kernel(RowFilterArgs a) {
     out[2].v[e] = static_cast<T>((ea - oa) * fa);
     out[3].v[e] = static_cast<T>((eb + ob) * fb);
     out[4].v[e] = static_cast<T>((eb - ob) * fb);
-    out[5].v[e] = static_cast<T>(a.kw == 5 ? g[4] : g[2]);
+    out[5].v[e] = static_cast<T>(last == 2 ? g[2] : last == 3 ? g[3] : g[4]);
   }
   T* dst = static_cast<T*>(a.U) + ((idx >> 8) * 6) * 512 + lane * 8 + e2;
 #pragma unroll
@@ -482,7 +486,7 @@ RowBox choose_box(int N, int oD, int oH, int nW, int kd, int kh, int tiles, int 
     for (int bd = 1; bd * bw <= tiles && bd <= oD; ++bd)
       for (int bh = 1; bh * bd * bw <= tiles && bh <= oH; ++bh) {
         RowBox b;
-        const int plane = bw * (bh + kh - 1);
+        const int plane = (bw + row_pieces(kh) - 1) * (bh + kh - 1);
         b.prow = bd > 1 ? padded(plane, bw * bh) : plane;
         const int image = (bd + kd - 2) * b.prow + plane, image_p = padded(image, bd * bh * bw);
         if (image > slots) break;
@@ -513,6 +517,19 @@ RowPlan make_row_shape(int N, int oD, int oH, int nW, int kd, int kh, int K, int
   const RowBox wide = choose_box(N, oD, oH, nW, kd, kh, 64, 128), half = kd == 1 ? choose_box(N, oD, oH, nW, kd, kh, 64, 64) : wide;
   const long long n_wide = wide.boxes * ceil_div(K, 128), n_half = half.boxes * ceil_div(K, 64);
   p.wide_groups = n_wide;
+  if (kh == 7) {
+    // Seven rows' halo leaves 64 tiles all of a wide workgroup's LDS, 32 a third of a CU's (kRowSmall) or, with the channels in
+    // two shares, two thirds (kRowSplit).  us a step of 32 channels: small 4 for every one that a CU gets, wide 7 alone and 10.5
+    // where all CUs have one.  Measured, wide | small | split, fp16: N=6 100 -> 150, 45x61 46 | 52 | 53, N=16 64 -> 64, 56x56
+    // 42 | 26 | 38, N=32 128 -> 128, 112x112 421 | 600 | 802, N=1 512 -> 512, 14x14 117 | 55 | 33, 64 -> 64, 28x28 18 | 9.8 | 8.7.
+    const RowBox small = choose_box(N, oD, oH, nW, kd, kh, 32, 64);
+    const long long n_small = small.boxes * ceil_div(K, 64), n_split = small.boxes * ceil_div(K, 32);
+    const double t_wide = (double)((n_wide + kCus - 1) / kCus) * (std::min(10.5, 7 + 3.5 * n_wide / kCus) * steps + 4);
+    if (steps >= 2 && n_split <= kCus) { p.shape = kRowSplit; p.box = small; }
+    else if (4.0 * steps * ((n_small + kCus - 1) / kCus) <= t_wide) { p.shape = kRowSmall; p.box = small; }
+    else { p.shape = kRowWide; p.box = wide; }
+    return p;
+  }
   const RowBox small = choose_box(N, oD, oH, nW, kd, kh, 32, 64);
   const double us_small = 0.4 * steps * kd * kh + 4;
   if (steps >= 4) {
@@ -577,9 +594,9 @@ bool filter_fits_l2(const RowArgs& a) { return a.u_bytes <= (3 << 20); }
 template <typename T, int KD, int KH, int KG, int TB, int S, int CS = 1, bool STAY = false>
 int launch_row(const RowArgs& args, const RowBox& b, void* stream) {
   RowArgs a = args;
-  a.bn = b.bn; a.bd = b.bd; a.bh = b.bh; a.bw = b.bw; a.prow = b.prow; a.irow = b.irow;
+  a.bn = b.bn; a.bd = b.bd; a.bh = b.bh; a.bw = b.bw; a.lw = b.bw + row_pieces(KH) - 1; a.prow = b.prow; a.irow = b.irow;
   a.f_bw = make_fast_div(b.bw); a.f_bh = make_fast_div(b.bh); a.f_bd = make_fast_div(b.bd);
-  a.f_prow = make_fast_div(b.prow); a.f_irow = make_fast_div(b.irow);
+  a.f_lw = make_fast_div(a.lw); a.f_prow = make_fast_div(b.prow); a.f_irow = make_fast_div(b.irow);
   a.n_d = b.n_d; a.n_h = b.n_h; a.n_w = b.n_w;
   a.n_box = (int)b.boxes;
   a.local_steps = ceil_div(a.steps, CS);
@@ -601,7 +618,7 @@ int launch_row(const RowArgs& args, const RowBox& b, void* stream) {
 bool row_conv_fits(const wc_conv_desc* d) {
   if (d->dtype == WC_F32 || d->stride != 1 || d->whole_kernel) return false;
   const int kd = d->kernel[0], kh = d->kernel[1], kw = d->kernel[2];
-  if (!((kd == 1 && kh == 3 && kw == 3) || (kd == 3 && kh == 3 && kw == 3) || (kd == 1 && kh == 5 && kw == 5 && d->ndim == 2))) return false;
+  if (!((kd == 1 && kh == 3 && kw == 3) || (kd == 3 && kh == 3 && kw == 3) || (kd == 1 && (kh == 5 || kh == 7) && kw == kh && d->ndim == 2))) return false;
   const int cp = wc_padded_channels8(d->C);
   for (int q = 0; q < 3; ++q)
     if (d->in[q] + 2 * d->pad[q] < d->kernel[q]) return false;
@@ -612,7 +629,7 @@ bool row_conv_fits(const wc_conv_desc* d) {
 }
 
 size_t row_u_elems(const wc_conv_desc* d) {
-  return (size_t)ceil_div(d->K, 32) * ceil_div(d->C, 32) * d->kernel[0] * d->kernel[1] * 2 * 6 * 512;
+  return (size_t)ceil_div(d->K, 32) * ceil_div(d->C, 32) * d->kernel[0] * d->kernel[1] * row_pieces(d->kernel[1]) * 2 * 6 * 512;
 }
 
 int row_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5], void* U, void* stream) {
@@ -620,8 +637,8 @@ int row_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5],
   RowFilterArgs a;
   a.w = w; a.U = U;
   for (int i = 0; i < 5; ++i) a.s[i] = w_strides[i];
-  a.K = d->K; a.C = d->C; a.kd = d->kernel[0]; a.kh = d->kernel[1]; a.kw = d->kernel[2]; a.steps = ceil_div(d->C, 32);
-  a.total = (long long)ceil_div(d->K, 32) * a.steps * a.kd * a.kh * 2 * 256;
+  a.K = d->K; a.C = d->C; a.kd = d->kernel[0]; a.kh = d->kernel[1]; a.kw = d->kernel[2]; a.pieces = row_pieces(a.kw); a.steps = ceil_div(d->C, 32);
+  a.total = (long long)ceil_div(d->K, 32) * a.steps * a.kd * a.kh * a.pieces * 2 * 256;
   const unsigned blocks = (unsigned)ceil_div_ll(a.total, 256);
   if (d->dtype == WC_F16) hipLaunchKernelGGL(row_filter_kernel<half_t>, dim3(blocks), dim3(256), 0, as_stream(stream), a);
   else hipLaunchKernelGGL(row_filter_kernel<bf16_t>, dim3(blocks), dim3(256), 0, as_stream(stream), a);
@@ -629,6 +646,12 @@ int row_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5],
   return WC_OK;
 }
 
+// 7x7 layers always: two of F(3, 4) a row are 28 products per output where pieces sharing a transformed input take 36 on F(2x2, 2x2)
+// and 25 on F(3x3, 3x3) (tile 4 in fp16), and the error is smaller than either's (bf16 3.9e-3 | 4.5e-3, fp16 4.8e-4 | 1.5e-3).  us,
+// row | other, bf16: N=32 128 -> 128, 112x112 408 | 565, N=16 256 -> 256, 56x56 228 | 319, 64 -> 64 26 | 45, 512 -> 512, 14x14
+// 108 | 144, N=6 100 -> 150, 45x61 47 | 72, N=1 128 -> 128, 56x56 12 | 30, 32 -> 32, 14x14 7.5 | 15; fp16 with tile 4: 415 | 520,
+// 235 | 248, 26 | 40, 108 | 135, 46 | 63, 12 | 24, 7.4 | 12.8.
+//
 // 5x5 layers: F(2, 5) needs 15 products per output where the plan they replace, two- or three-tap pieces sharing one
 // transformed input, needs 20 on F(2x2, 2x2) and 11 on F(3x3, 3x3) (tile 4 in fp16), without V and M in memory, and is as
 // exact as the first (bf16 4.3e-3 | 4.5e-3 against fp64) and 2.5 times as the second (fp16 5.5e-4 | 1.4e-3).  us, row | other, bf16:
@@ -661,6 +684,7 @@ bool row_preferred(const wc_conv_desc* d) {
   wc_conv_desc e = *d;
   e.stacked = 0; e.direct = 0; e.row = 0;
   if (wc_plan_conv(&e, &plan) == WC_OK && thin_conv_fits(&e, &plan)) return false;
+  if (d->kernel[1] == 7) return true;
   if (d->kernel[1] == 5) return row_preferred_5x5(d);
   if (d->m != 4) return true;
   const int kd = d->kernel[0], oD = d->in[0] + 2 * d->pad[0] - kd + 1, oH = d->in[1] + 2 * d->pad[1] - 2, oW = d->in[2] + 2 * d->pad[2] - 2;
@@ -672,7 +696,7 @@ bool row_preferred(const wc_conv_desc* d) {
 // x (N, D, H, W, Cx) channel-last with Cx = C rounded up to 8 (zeros beyond C), 16-byte aligned; images first_image ..
 // + n_images of the batch
 int row_conv(const wc_conv_desc* d, const void* x, int first_image, int n_images, const void* U, const void* bias, void* y, void* stream) {
-  WC_CHECK_ARG(row_conv_fits(d), "row form: 16-bit, stride 1, kernels 3x3, 3x3x3 and 5x5");
+  WC_CHECK_ARG(row_conv_fits(d), "row form: 16-bit, stride 1, kernels 3x3, 3x3x3, 5x5 and 7x7");
   WC_CHECK_ARG(((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(U)) & 15) == 0, "row form: x and U must be 16-byte aligned");
   RowArgs a{};
   a.x = x; a.U = U; a.bias = bias; a.y = y;
@@ -704,23 +728,32 @@ int row_conv(const wc_conv_desc* d, const void* x, int first_image, int n_images
         constexpr int KD = decltype(kd)::value, KH = decltype(kh)::value;
         RowPlan p = plan;
         if (a.N != d->N - p.tall_images || (force >= 16 && force <= 19)) {
-          const int tiles = p.shape <= kRowHalf ? 64 : 32, slots = p.shape == kRowWide ? 128 : p.shape == kRowSplit ? 32 : p.shape == kRowHalf && KD > 1 ? 128 : 64;
+          const int tiles = p.shape <= kRowHalf ? 64 : 32, slots = KH == 7 ? (tiles == 64 ? 128 : 64) : p.shape == kRowWide ? 128 : p.shape == kRowSplit ? 32 : p.shape == kRowHalf && KD > 1 ? 128 : 64;
           p.box = choose_box(a.N, a.oD, a.oH, a.nW, KD, KH, tiles, slots);
         }
-        switch (p.shape) {
-          case kRowWide:
-            // More boxes than CUs: a workgroup per CU that asks for its next box's input before it writes a box out, which
-            // hides that input's way from memory behind the write-out and saves the start of a workgroup.  Measured, fp16, us,
-            // a workgroup per box | this: N=64 256 -> 256, 56x56 196 | 185, 128 -> 128, 56x56 71 | 66, 256 -> 256, 28x28 53.3 | 52.0,
-            // N=8 128 -> 128, 16x56x56 242 | 239.  Filters beyond an XCD's L2 (box_fast): 512 -> 512, N=16 28x28 48.1 | 49.3.
-            if (KH == 5 || !filter_fits_l2(a) || ceil_div(a.K, 128) * p.box.boxes <= kCus) return launch_row<T, KD, KH, 4, 2, 128>(a, p.box, stream);
-            if constexpr (KH != 5) return launch_row<T, KD, KH, 4, 2, 128, 1, true>(a, p.box, stream);   // (spills with 5x5's ring)
-            [[fallthrough]];
-          case kRowHalf: return launch_row<T, KD, KH, 2, 2, KD == 1 ? 64 : 128>(a, p.box, stream);
-          case kRowSmall: return launch_row<T, KD, KH, 2, 1, 64>(a, p.box, stream);
-          default: return launch_row<T, KD, KH, 1, 1, 32, 4>(a, p.box, stream);
+        if constexpr (KH == 7) {
+          if (p.shape == kRowSplit) return launch_row<T, KD, KH, 1, 1, 64, 2>(a, p.box, stream);
+          if (p.shape == kRowSmall) return launch_row<T, KD, KH, 2, 1, 64>(a, p.box, stream);
+          return launch_row<T, KD, KH, 4, 2, 128>(a, p.box, stream);
+        } else {
+          switch (p.shape) {
+            case kRowWide:
+              // More boxes than CUs: a workgroup per CU that asks for its next box's input before it writes a box out, which
+              // hides that input's way from memory behind the write-out and saves the start of a workgroup.  Measured, fp16, us,
+              // a workgroup per box | this: N=64 256 -> 256, 56x56 196 | 185, 128 -> 128, 56x56 71 | 66, 256 -> 256, 28x28 53.3 |
+              // 52.0, N=8 128 -> 128, 16x56x56 242 | 239.  Filters beyond an XCD's L2 (box_fast): 512 -> 512, N=16 28x28 48.1 |
+              // 49.3.  (Not with the deeper ring of 5x5 kernels, whose registers do not hold the next box beside it.)
+              if constexpr (KH == 3) {
+                if (filter_fits_l2(a) && ceil_div(a.K, 128) * p.box.boxes > kCus) return launch_row<T, KD, KH, 4, 2, 128, 1, true>(a, p.box, stream);
+              }
+              return launch_row<T, KD, KH, 4, 2, 128>(a, p.box, stream);
+            case kRowHalf: return launch_row<T, KD, KH, 2, 2, KD == 1 ? 64 : 128>(a, p.box, stream);
+            case kRowSmall: return launch_row<T, KD, KH, 2, 1, 64>(a, p.box, stream);
+            default: return launch_row<T, KD, KH, 1, 1, 32, 4>(a, p.box, stream);
+          }
         }
       };
+      if (d->kernel[1] == 7) return go(ic<1>{}, ic<7>{});
       if (d->kernel[1] == 5) return go(ic<1>{}, ic<5>{});
       if (d->kernel[0] == 1) return go(ic<1>{}, ic<3>{});
       return go(ic<3>{}, ic<3>{});

@@ -56,15 +56,19 @@ __device__ __forceinline__ void row_input_channel(Pack<T, 2> (&x)[6], int e) {
   x[4].v[e] = static_cast<T>(__builtin_fmaf(-kB, ob, eb));
 }
 
-// Outputs of a tile: the six elements carry F(4, 3) and F(2, 5) alike, whose tiles start 4 and 2 pixels apart
-__host__ __device__ constexpr int row_outputs_of(int taps) { return 7 - taps; }
+// Outputs of a tile: the six elements carry F(4, 3), F(2, 5) and F(3, 4) alike, whose tiles start 4, 2 and 3 pixels apart.  A row
+// of 7 taps is two of F(3, 4): the first three taps, and the other four on the tile after, three pixels on.
+__host__ __device__ constexpr int row_outputs_of(int taps) { return taps == 7 ? 3 : 7 - taps; }
+__host__ __device__ constexpr int row_pieces(int taps) { return taps == 7 ? 2 : 1; }
 
 // One output channel of a tile from the two halves of its elements, each reduced to (x, s, d): the element at 0 or infinity,
 // and sum and difference of the pair at +-a (first half) or +-1/a (second)
 template <int OUT> struct RowOutputs { float o[OUT]; };
 template <int OUT>
 __device__ __forceinline__ RowOutputs<OUT> row_outputs(float m0, float sa, float da, float mi, float sb, float db, float b) {
-  if constexpr (OUT == 2) {
+  if constexpr (OUT == 3) {
+    return {{m0 + sa + sb + b, __builtin_fmaf(kA, da, __builtin_fmaf(kB, db, b)), __builtin_fmaf(kA2, sa, __builtin_fmaf(kB2, sb, mi + b))}};
+  } else if constexpr (OUT == 2) {
     return {{m0 + sa + sb + b, __builtin_fmaf(kA, da, __builtin_fmaf(kB, db, mi + b))}};
   } else {
     return {{m0 + sa + sb + b, __builtin_fmaf(kA, da, __builtin_fmaf(kB, db, b)), __builtin_fmaf(kA2, sa, __builtin_fmaf(kB2, sb, b)),
