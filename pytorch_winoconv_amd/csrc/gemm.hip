@@ -229,8 +229,7 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
         }
       }
       regs[set][i] = *reinterpret_cast<const Chunk16*>(gptr[i] + kt * BK + (SHIFT && i < BM / RPP ? vshift : 0));
-    }
-    if constexpr (DIRECT) {
+    }    if constexpr (DIRECT) {
       if (++tap_cb == g.cblocks) {
         tap_cb = 0;
         if (++tap_x == g.kw) { tap_x = 0; ++tap_y; }
@@ -298,10 +297,25 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
     if (nk > 1) { next_block(); gload(ic<1>{}, 1, vshift); }
   }
   __syncthreads();
-  auto stage = [&](int kt, auto set_c) {           // set_c: kt % AHEAD
-    constexpr int set = decltype(set_c)::value;
+  // set_c: kt % AHEAD; left_c: how many stages follow this one, 2 for two and more, -1 for what the loop does not know.  Loads
+  // and stores behind a branch are loads the compiler cannot count: it waits for the newest of them.  The 64 x 64 tile, whose
+  // stages are short, has its last stages apart instead (us, before | now: fp16 stride 2, N=1 512 -> 512, 7x7 28 | 23, 128 -> 128,
+  // 56x56 12.3 | 11.0; T=36, P 4, 512 -> 512 6.4 | 5.9; fp32, T=36, P 98, 512 -> 512 28 | 26); larger tiles need more registers
+  // that way (128 x 128: 206 for 152, a third fewer workgroups; 1x1 64 -> 256, N=64 56x56 26 | 31).
+  constexpr bool APART = WM * WN == 1;
+  auto stage = [&](int kt, auto set_c, auto left_c) {
+    constexpr int set = decltype(set_c)::value, left = decltype(left_c)::value;
     const int cur = kt & 1;
-    if (kt + AHEAD < nk) { next_block(); gload(set_c, kt + AHEAD, vshift); }
+    if constexpr (left >= AHEAD) { next_block(); gload(set_c, kt + AHEAD, vshift); }
+    if constexpr (left < 0) {
+      if (kt + AHEAD < nk) { next_block(); gload(set_c, kt + AHEAD, vshift); }
+    }
+    auto store_next = [&]() {
+      if constexpr (left > 0) lstore(ic<AHEAD == 2 ? 1 - set : 0>{}, cur ^ 1);
+      if constexpr (left < 0) {
+        if (kt + 1 < nk) lstore(ic<AHEAD == 2 ? 1 - set : 0>{}, cur ^ 1);
+      }
+    };
     const T* st = lds + cur * STAGE;
     if constexpr (SPLIT) {
       const unsigned char* const sb = lds_raw + cur * 3 * PLANE + (lhi ^ ((l32 >> 3) & 1)) * 16;
@@ -320,7 +334,7 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
 #pragma unroll
           for (int j = 0; j < WN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[qw][j], xf[qx][i], acc[i][j], 0, 0, 0);
       });
-      if (kt + 1 < nk) lstore(ic<AHEAD == 2 ? 1 - set : 0>{}, cur ^ 1);
+      store_next();
       __syncthreads();
       return;
     }
@@ -347,13 +361,32 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
         for (int j = 0; j < WN; ++j) acc[i][j] = MF::run(wf[kk & 1][j], xf[kk & 1][i], acc[i][j]);
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (kt + 1 < nk) lstore(ic<AHEAD == 2 ? 1 - set : 0>{}, cur ^ 1);
+    store_next();
     __syncthreads();
   };
-  for (int kt = 0; kt < nk; kt += AHEAD) {
-    stage(kt, ic<0>{});
-    if constexpr (AHEAD == 2) {
-      if (kt + 1 < nk) stage(kt + 1, ic<1>{});
+  if constexpr (APART) {
+    static_assert(!APART || AHEAD == 2, "two stages ahead");
+    int kt = 0;
+    for (; kt + 3 < nk; kt += 2) {
+      stage(kt, ic<0>{}, ic<2>{});
+      stage(kt + 1, ic<1>{}, ic<2>{});
+    }
+    if (nk - kt == 3) {
+      stage(kt, ic<0>{}, ic<2>{});
+      stage(kt + 1, ic<1>{}, ic<1>{});
+      stage(kt + 2, ic<0>{}, ic<0>{});
+    } else if (nk - kt == 2) {
+      stage(kt, ic<0>{}, ic<1>{});
+      stage(kt + 1, ic<1>{}, ic<0>{});
+    } else {
+      stage(kt, ic<0>{}, ic<0>{});
+    }
+  } else {
+    for (int kt = 0; kt < nk; kt += AHEAD) {
+      stage(kt, ic<0>{}, ic<-1>{});
+      if constexpr (AHEAD == 2) {
+        if (kt + 1 < nk) stage(kt + 1, ic<1>{}, ic<-1>{});
+      }
     }
   }
 
@@ -952,7 +985,9 @@ static GemmConfig choose_direct(int P, int K, int reduction) {
     // stride 2, N=64 112x112 60 | 62; 128 -> 128, N=32 64 | 58
     if (reduction > 768 && blocks(big) >= kCus) return big;
     GemmConfig mid = make_config<T, 2, 2, BK, 2, 2, true, true>();   // 128 x 128
-    if (blocks(mid) >= kCus) return mid;
+    // 128 x 128 | 64 x 64, N=16 and 20 128 -> 256, 56x56 (196 and 246 tiles of the first) 21.3 | 24.2 and 22.0 | 24.9, N=12
+    // (148 tiles) 20.3 | 16.8
+    if (blocks(mid) >= kCus || (blocks(mid) >= 3 * kCus / 4 && K % 128 == 0)) return mid;
   }
   return make_config<T, 1, 1, BK, 2, 2, true, true>();               // 64 x 64
 }
