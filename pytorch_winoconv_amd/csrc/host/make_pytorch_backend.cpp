@@ -313,8 +313,7 @@ std::vector<int> ints_of(py::object v, int nd, const char* what) {
 // used without a copy and a contiguous channel-first one is handed to the library as it is
 // (wc_conv_desc.x_layout); any other layout is made contiguous first.  The compiled form of the Python callers' common path (dwm.py:5-40, matrix_conv.py:70-135
 // of the reference end in the same call).
-// `flipped`: the filter is w reversed along every spatial axis, read through negative strides.  Only the row form's filter
-// kernel takes those: an undefined tensor, and nothing launched, where the library chooses another form.
+// `flipped`: the filter is w reversed along every spatial axis, read through negative strides.
 at::Tensor conv_impl(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bias, py::object stride, py::object padding,
                      int m, std::optional<at::Tensor> U, int chunk_images, bool whole_kernel, py::object stacked,
                      bool unfused, bool channels_first_out, py::object direct, bool row, bool flipped) {
@@ -371,7 +370,6 @@ at::Tensor conv_impl(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bias,
   d.unfused = unfused;
   d.row = row && !unfused ? -1 : 0;                                       // -1: the library may choose it
   check(wc_conv_auto(&d));
-  if (flipped && d.row != 1) return at::Tensor();
   int out[3], grid[3];
   check(wc_conv_out_dims(&d, out, grid));
   std::vector<int64_t> ys{x.size(0)};                      // channel-last shape of y
@@ -431,15 +429,13 @@ at::Tensor conv_forward(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bi
                    row, false);
 }
 
-// Input gradient of a stride-1 layer where the row form takes it (an undefined tensor elsewhere): dy convolved with w
-// flipped and its channel axes exchanged; `padding` is that convolution's.
-at::Tensor conv_backward_input_row(at::Tensor dy, at::Tensor w, py::object padding, int m) {
+// Input gradient of a stride-1 layer: dy convolved with w flipped and its channel axes exchanged; `padding` is that
+// convolution's.
+at::Tensor conv_backward_input_flipped(at::Tensor dy, at::Tensor w, py::object padding, int m) {
   return conv_impl(dy, w.transpose(0, 1), std::nullopt, py::int_(1), padding, m, std::nullopt, 0, false, py::none(), false, false,
                    py::none(), true, true);
 }
 
-// ---- gradients (the reference has no backward pass: src/back/utils.cu:15-24): engine.py's conv_backward_weight with the
-// form of the plan left to the library, and bias_gradient
 at::Tensor last_view(const at::Tensor& t) {       // (N, C, *) -> (N, *, C), contiguous
   std::vector<int64_t> order{0};
   for (int64_t a = 2; a < t.dim(); ++a) order.push_back(a);
@@ -447,6 +443,93 @@ at::Tensor last_view(const at::Tensor& t) {       // (N, C, *) -> (N, *, C), con
   return t.permute(order).contiguous();
 }
 
+wc_conv_desc desc_of(at::IntArrayRef x, at::IntArrayRef w, const std::vector<int>& pads, int stride, int m, int dtype) {
+  const int nd = (int)x.size() - 2;
+  wc_conv_desc d{};
+  d.ndim = nd;
+  d.N = (int)x[0]; d.C = (int)x[1]; d.K = (int)w[0];
+  d.in[0] = d.kernel[0] = 1;
+  for (int a = 0; a < nd; ++a) {
+    d.in[3 - nd + a] = (int)x[2 + a];
+    d.kernel[3 - nd + a] = (int)w[2 + a];
+    d.pad[3 - nd + a] = pads[a];
+  }
+  d.stride = stride; d.m = m; d.dtype = dtype;
+  return d;
+}
+
+void strides_of(const at::Tensor& w, int64_t s[5]) {
+  const int nd = (int)w.dim() - 2;
+  s[0] = w.stride(0); s[1] = w.stride(1);
+  for (int a = 0; a < 3; ++a) s[2 + a] = a < 3 - nd ? 0 : w.stride(2 + a - (3 - nd));
+}
+
+// Input gradient of a 2-D layer at stride 2 over the parity classes of its pixels (wc_conv_backward_input); an undefined
+// tensor, and nothing launched, where that does not apply.  engine.py's conv_backward_input has checked the padding.
+at::Tensor conv_backward_input_strided(at::Tensor dy, at::Tensor w, std::vector<int64_t> x_spatial, std::vector<int> pads) {
+  require_gpu(dy, "conv_backward_input");
+  require_gpu(w, "conv_backward_input");
+  wc_conv_desc d = desc_of({dy.size(0), w.size(1), x_spatial[0], x_spatial[1]}, w.sizes(), pads, 2, 2, dtype_of(dy));
+  int out[3], grid[3];
+  check(wc_conv_out_dims(&d, out, grid));
+  if (dy.size(2) != out[1] || dy.size(3) != out[2])
+    throw std::invalid_argument("dy of shape " + shape_str(dy.sizes()) + " does not belong to an input of extent " + shape_str(x_spatial));
+  size_t bytes = 0;
+  if (wc_conv_backward_input_workspace_bytes(&d, &bytes) != WC_OK) return at::Tensor();
+  if (w.scalar_type() != dy.scalar_type()) throw py::type_error("dy and the filter must share one dtype");
+  const at::Tensor dyl = last_view(dy);
+  at::Tensor dx = at::empty({dy.size(0), x_spatial[0], x_spatial[1], w.size(1)}, dy.options());
+  void* stream = stream_of(dy);
+  at::Tensor ws = workspace_for(dy, bytes, stream);
+  int64_t s[5];
+  strides_of(w, s);
+  {
+    py::gil_scoped_release nogil;
+    check(wc_conv_backward_input(&d, dyl.data_ptr(), w.data_ptr(), s, dx.data_ptr(), ws.data_ptr(), bytes, stream));
+  }
+  return dx.permute({0, 3, 1, 2});
+}
+
+// engine.py's transform_filter with the form left to the library, the row form allowed
+at::Tensor transform_filter(at::Tensor w, std::vector<int64_t> x_shape, py::object stride, py::object padding, int m) {
+  const int nd = (int)w.dim() - 2;
+  require_gpu(w, "transform_filter");
+  if ((nd != 2 && nd != 3) || (int)x_shape.size() != nd + 2)
+    throw std::invalid_argument("expected 4-D or 5-D input and matching filter, got " + shape_str(x_shape) + " and " + shape_str(w.sizes()));
+  if (x_shape[1] != w.size(1))
+    throw std::invalid_argument("input has " + std::to_string(x_shape[1]) + " channels, filter expects " + std::to_string(w.size(1)) +
+                                " (groups are not supported)");
+  const auto st = ints_of(stride, nd, "stride");
+  for (int a = 1; a < nd; ++a)
+    if (st[a] != st[0]) { PyErr_SetString(PyExc_NotImplementedError, "stride must be the same on every axis"); throw py::error_already_set(); }
+  wc_conv_desc d = desc_of(x_shape, w.sizes(), ints_of(padding, nd, "padding"), st[0], m, dtype_of(w));
+  d.stacked = d.row = -1;
+  check(wc_conv_auto(&d));
+  wc_plan plan{};
+  size_t n = 0;
+  check(wc_conv_u_elems(&d, &n));
+  std::vector<int64_t> shape{(int64_t)n};
+  if (d.direct) {          // taps outermost, channels innermost; first layers have their own rows
+    if (nd == 3) shape = {d.K, d.kernel[0] * d.kernel[1], 4, 4};
+    else if (n == (size_t)d.K * d.kernel[1] * d.kernel[2] * d.C) shape = {d.K, d.kernel[1], d.kernel[2], d.C};
+    else shape = {d.K, d.kernel[1], 8, 4};
+  } else if (!d.row) {
+    check(wc_plan_conv(&d, &plan));
+    shape = {plan.t_total, d.K, (int64_t)wc_padded_channels(d.C) * (d.stacked ? plan.n_pieces : 1)};
+  }
+  at::Tensor U = at::empty(shape, w.options().memory_format(at::MemoryFormat::Contiguous));
+  int64_t s[5];
+  strides_of(w, s);
+  void* stream = stream_of(w);
+  {
+    py::gil_scoped_release nogil;
+    check(wc_filter_transform(&d, &plan, w.data_ptr(), s, U.data_ptr(), stream));
+  }
+  return U;
+}
+
+// ---- gradients (the reference has no backward pass: src/back/utils.cu:15-24): engine.py's conv_backward_weight with the
+// form of the plan left to the library, and bias_gradient
 at::Tensor conv_backward_weight(at::Tensor x, at::Tensor dy, std::vector<int64_t> w_shape, py::object stride, py::object padding, int m) {
   const int nd = (int)x.dim() - 2;
   require_gpu(x, "conv_backward_weight");
@@ -508,6 +591,50 @@ at::Tensor bias_gradient(at::Tensor dy) {
   return db;
 }
 
+// All gradients of a layer in one call, each in the type of what it belongs to: (dx, dw, db), None for what is not asked for
+// and for what engine.py's functions have to do (an input gradient that neither function above has, the bias gradient of a dy
+// that is not channel-last memory).
+py::tuple conv_backward(at::Tensor x, at::Tensor w, at::Tensor dy, py::object stride, py::object padding, int m, bool need_dx,
+                        bool need_dw, bool need_db, py::object w_type, py::object b_type) {
+  const int nd = (int)x.dim() - 2;
+  if ((nd != 2 && nd != 3) || w.dim() != nd + 2 || dy.dim() != nd + 2)
+    throw std::invalid_argument("expected 4-D or 5-D input and matching filter, got " + shape_str(x.sizes()) + " and " + shape_str(w.sizes()));
+  const auto st = ints_of(stride, nd, "stride");
+  const auto pd = ints_of(padding, nd, "padding");
+  at::Tensor dx, dw, db;
+  if (need_dx) {
+    std::vector<int> flipped(nd);
+    bool fits = true;
+    for (int a = 0; a < nd; ++a) {
+      flipped[a] = (int)w.size(2 + a) - 1 - pd[a];
+      fits = fits && flipped[a] >= 0;
+    }
+    const std::vector<int64_t> size(x.sizes().begin() + 2, x.sizes().end());
+    if (fits && st[0] == 1) {
+      bool threes = true;
+      for (int a = 0; a < nd; ++a) threes = threes && w.size(2 + a) == 3;
+      const int tile = w.size(0) >= 8 && (m == 2 || nd == 2 || threes) ? m : 2;      // as in engine.py's conv_backward_input
+      at::Tensor t = conv_backward_input_flipped(dy, w, py::cast(flipped), tile);
+      if (t.sizes().slice(2) == at::IntArrayRef(size)) dx = t;
+    } else if (fits && nd == 2 && st[0] == 2) {
+      dx = conv_backward_input_strided(dy, w, size, pd);
+    }
+  }
+  if (need_dw) {
+    dw = conv_backward_weight(x, dy, w.sizes().vec(), stride, padding, m);
+    if (!w_type.is_none()) dw = dw.to(torch::python::detail::py_object_to_dtype(w_type));
+  }
+  std::vector<int64_t> last{0};
+  for (int a = 0; a < nd; ++a) last.push_back(2 + a);
+  last.push_back(1);
+  if (need_db && need_dw && dy.permute(last).is_contiguous()) {
+    db = bias_gradient(dy);
+    if (!b_type.is_none()) db = db.to(torch::python::detail::py_object_to_dtype(b_type));
+  }
+  auto out = [](const at::Tensor& t) -> py::object { return t.defined() ? py::cast(t) : py::none(); };
+  return py::make_tuple(out(dx), out(dw), out(db));
+}
+
 // The reference's native entry point (pybind/extern.hpp:7-9): VALID convolution.  The four scratch tensors
 // of the reference signature (dwm.py:122-125) are accepted and ignored: the engine sizes its own workspace.
 void DWM(at::Tensor Input, at::Tensor Weight, at::Tensor Output, int stride, py::object, py::object, py::object, py::object) {
@@ -547,7 +674,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("channels_first_out") = false, py::arg("direct") = py::none(), py::arg("row") = false);
   m.def("conv_backward_weight", &conv_backward_weight, py::arg("x"), py::arg("dy"), py::arg("w_shape"), py::arg("stride") = 1,
         py::arg("padding") = 0, py::arg("m") = 2);
-  m.def("conv_backward_input_row", &conv_backward_input_row, py::arg("dy"), py::arg("w"), py::arg("padding"), py::arg("m"));
+  m.def("conv_backward", &conv_backward, py::arg("x"), py::arg("w"), py::arg("dy"), py::arg("stride"), py::arg("padding"), py::arg("m"),
+        py::arg("need_dx"), py::arg("need_dw"), py::arg("need_db"), py::arg("w_type") = py::none(), py::arg("b_type") = py::none());
+  m.def("conv_backward_input_flipped", &conv_backward_input_flipped, py::arg("dy"), py::arg("w"), py::arg("padding"), py::arg("m"));
+  m.def("conv_backward_input_strided", &conv_backward_input_strided, py::arg("dy"), py::arg("w"), py::arg("x_spatial"), py::arg("pads"));
+  m.def("transform_filter", &transform_filter, py::arg("w"), py::arg("x_shape"), py::arg("stride") = 1, py::arg("padding") = 0, py::arg("m") = 2);
   m.def("bias_gradient", &bias_gradient, py::arg("dy"));
   m.def("version", []() { return std::string(wc_version()); });
 }

@@ -334,6 +334,8 @@ def check_u(desc, U):
 def transform_filter(w, x_shape, stride=1, padding=0, m=2, whole_kernel=False, stacked=None, direct=None, row=False):
     """Transformed filter U for later calls of conv_forward(..., U=U) with the same options."""
     _require_gpu(w)
+    if USE_EXT and row and x_shape[0] > 0 and not whole_kernel and stacked is None and direct is None:
+        return _ext.transform_filter(w, tuple(x_shape), stride, padding, m)
     if row and x_shape[0] > 0:                  # the module's call, once in a training step: its descriptor is kept
         desc = _forward_setup(tuple(x_shape), tuple(w.shape), w.dtype, stride, padding, m, 0, whole_kernel, stacked, direct=direct, row=row)[0]
     else:
@@ -522,6 +524,13 @@ def bias_gradient(dy):
     return db
 
 
+def conv_backward(x, w, dy, stride, padding, m, need_dx, need_dw, need_db, w_type=None, b_type=None):
+    """The gradients of conv_forward(x, w, bias, ...) that are asked for, in one call of the compiled host layer: (dx, dw, db), the
+    last two in `w_type` and `b_type` where those are given; None for what is left to the functions below and above."""
+    _require_gpu(x, w, dy)
+    return _ext.conv_backward(x, w, dy, stride, padding, m, need_dx, need_dw, need_db, w_type, b_type)
+
+
 def conv_backward_input(dy, w, x_spatial, stride=1, padding=0, m=2):
     """Gradient of sum(y * dy) with respect to the input: the convolution of dy (with zeros between
     its elements when stride is 2) with the filter flipped along every spatial axis and its two
@@ -538,6 +547,10 @@ def conv_backward_input(dy, w, x_spatial, stride=1, padding=0, m=2):
     if stride == 2 and nd == 2 and dy.shape[0] > 0:
         # the library's own input gradient of strided layers: the direct form over the parity classes of the pixels of dx
         # (wc_conv_backward_input); where it does not apply, the zero-filled dy below
+        if USE_EXT:
+            dx = _ext.conv_backward_input_strided(dy, w, want, pads)
+            if dx is not None:
+                return dx
         lib = _lib.load()
         x_shape = (dy.shape[0], w.shape[1]) + want
         desc = make_desc(x_shape, w.shape, dy.dtype, 2, padding, 2, 0, False, False, direct=False)
@@ -572,8 +585,9 @@ def conv_backward_input(dy, w, x_spatial, stride=1, padding=0, m=2):
     # 3e-2 with tile 4, 1e-3 with tile 2)
     mm = m if (stride == 1 and w.shape[0] >= 8 and (m == 2 or nd == 2 or ks == (3, 3, 3))) else 2
     pads = tuple(k - 1 - p for k, p in zip(ks, pads))
-    dx = _ext.conv_backward_input_row(dy, w, pads, mm) if USE_EXT and dy.shape[0] > 0 else None
-    if dx is None:
+    if USE_EXT and dy.shape[0] > 0:
+        dx = _ext.conv_backward_input_flipped(dy, w, pads, mm)      # the flipped filter read through negative strides
+    else:
         dx = conv_forward(dy, w.flip(tuple(range(2, 2 + nd))).transpose(0, 1), None, 1, pads, mm, row=True)
     if tuple(dx.shape[2:]) != want:
         raise ValueError("dy of shape %r does not belong to an input of extent %r" % (tuple(dy.shape), want))
