@@ -226,8 +226,8 @@ extern "C" int wc_conv_backward_input(const wc_conv_desc* d, const void* dy, con
     return 0;
   });
   WC_CHECK_LAUNCH("sub_filter_kernel");
-  // kernel rows of four taps and more have a kernel of their own (direct_rows.hip), one launch per class
-  if ((kw + 1) / 2 <= 3)
+  // one launch for all classes; fp32 classes of four and more taps a row, and direct_rows.hip's tiles in tests, one by one
+  if ((kw + 1) / 2 <= 3 || (d->dtype != WC_F32 && test_gemm_rows() != 2))
     return gemm_direct_classes(dy, cls, a.n, dx, d->N, out[1], out[2], d->K, d->C, d->dtype, stream, H, W);
   for (int i = 0; i < a.n; ++i) {
     const DirectClass& c = cls[i];

@@ -201,13 +201,10 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
     loff[i] = SPLIT ? row * 32 + ((lpart >> 1) ^ ((row >> 3) & 1)) * 16 + (lpart & 1) * 8 : row * LDS_STRIDE + (lpart ^ swizzle(row)) * EPC;
   }
 
-  // A reduction block is requested two stages before it is multiplied where the registers allow it, in the direct form, of
-  // fp32 in three parts and on the smallest tile of all (T=36, 64x64, fp16, us, one stage | two: P 98, 512 -> 512 9.0 | 8.5;
-  // P 784, T=16, 64 -> 64 3.9 | 3.5; fp32 stride 2, N=1 128 -> 128, 56x56 42 | 35): a stage of
-  // the smaller tiles is over before its pixels, behind their bounds checks, are there (fp16 stride 2, us, one stage | two:
-  // N=1 128 -> 128, 56x56 16.5 | 12.7; N=2 256 -> 512, 15x17 30 | 22; N=64 256 -> 512, 28x28 55 | 51; the 256 x 128 tile
-  // spills that way, N=32 128 -> 128, 112x112 63 | 77).
-  constexpr int AHEAD = (((DIRECT && sizeof(T) == 2) || SPLIT) && WM * WN <= 4) || WM * WN == 1 ? 2 : 1;
+  // A reduction block is requested two stages before it is multiplied where the registers allow it, of fp32 in three parts and
+  // on the smallest tile of all (T=36, 64x64, fp16, us, one stage | two: P 98, 512 -> 512 9.0 | 8.5; P 784, T=16, 64 -> 64
+  // 3.9 | 3.5; fp32 stride 2, N=1 128 -> 128, 56x56 42 | 35).
+  constexpr int AHEAD = (SPLIT && WM * WN <= 4) || WM * WN == 1 ? 2 : 1;
   Chunk16 regs[AHEAD][NLOAD];
   bool in_image[AHEAD][DIRECT ? BM / RPP : 1];
   // `vshift`: what the V operand has jumped by at reduction block kt (rows i < BM / RPP are V's)
@@ -221,7 +218,7 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
           const int j = i < BM / RPP ? i : 0;
           const bool inside = (unsigned)(iy0[j] + tap_y) < (unsigned)g.H && (unsigned)(ix0[j] + tap_x) < (unsigned)g.W;
           // always a load, of the first pixel where the tap is outside: behind a branch the compiler does not know how many
-          // loads are in flight and waits for all of them (N=32 128 -> 128, 112x112, fp16 at stride 2 69 us, now 63.5)
+          // loads are in flight and waits for all of them
           const T* const from = inside ? gptr[i] + kt * BK + vshift : Vt;
           regs[set][i] = *reinterpret_cast<const Chunk16*>(from);
           in_image[set][j] = inside;
@@ -299,9 +296,9 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
   __syncthreads();
   // set_c: kt % AHEAD; left_c: how many stages follow this one, 2 for two and more, -1 for what the loop does not know.  Loads
   // and stores behind a branch are loads the compiler cannot count: it waits for the newest of them.  The 64 x 64 tile, whose
-  // stages are short, has its last stages apart instead (us, before | now: fp16 stride 2, N=1 512 -> 512, 7x7 28 | 23, 128 -> 128,
-  // 56x56 12.3 | 11.0; T=36, P 4, 512 -> 512 6.4 | 5.9; fp32, T=36, P 98, 512 -> 512 28 | 26); larger tiles need more registers
-  // that way (128 x 128: 206 for 152, a third fewer workgroups; 1x1 64 -> 256, N=64 56x56 26 | 31).
+  // stages are short, has its last stages apart instead (us, before | now: T=36, P 4, 512 -> 512 6.4 | 5.9; fp32, T=36, P 98,
+  // 512 -> 512 28 | 26); larger tiles need more registers
+  // that way (128 x 128: 206 for 152, a third fewer workgroups).
   constexpr bool APART = WM * WN == 1;
   auto stage = [&](int kt, auto set_c, auto left_c) {
     constexpr int set = decltype(set_c)::value, left = decltype(left_c)::value;
@@ -955,41 +952,17 @@ int fold_filter_w(const void* U, void* Uw, int K, int Cp, int dtype, void* strea
   return WC_OK;
 }
 
-// Tiles of the direct form, chosen like those of the shifted operand.
+// Tiles of the direct form: fp32 products are bound by the MFMA rate and fill the chip best with small tiles (as in choose()).
+// 16-bit types come here only where direct_dma.hip does not reach (direct_dma_fits).
 template <typename T>
-static GemmConfig choose_direct(int P, int K, int reduction) {
+static GemmConfig choose_direct(int P, int K) {
   constexpr int BK = sizeof(T) == 4 ? 16 : 32;
-  auto blocks = [&](const GemmConfig& c) { return (long long)ceil_div(P, c.bm) * ceil_div(K, c.bn); };
-  switch (test_gemm_config()) {                       // wc_test_gemm_override: a tile shape forced by a test
-    case 0: return make_config<T, 2, 2, BK, 4, 2, true, true>();
-    case 1: return make_config<T, 2, 2, BK, 2, 2, true, true>();
-    case 2: return make_config<T, 4, 1, BK, 2, 2, true, true>();
-    case 3: return make_config<T, 1, 1, BK, 2, 2, true, true>();
-    case 4: return make_config<T, 4, 2, BK, 2, 2, true, true>();   // 256 x 128, four wavefronts
-    default: break;
-  }
-  // Measured on MI355X (fp16, stride 2): the largest tile that still gives every compute unit a workgroup
-  // wins: 256 x 128 over 128 x 128 by 15-25 % at 392 workgroups (N=32, C=K=128, 112x112: 54.9 against
-  // 63.7 us; C=K=256, 56x56: 93.5 against 115 us), and loses by 40 % at 196.  Four wavefronts of 128 x 64
-  // beat eight of 64 x 64 for the large tile (54.9 against 73.0 us): half the LDS reads per MFMA.
-  // fp32 products are bound by the MFMA rate and fill the chip best with small tiles (as in choose()).
+  const int force = test_gemm_config();               // wc_test_gemm_override: a tile shape forced by a test
+  const bool small = force == 3 || (force != 1 && sizeof(T) == 4 && (K <= 64 || (long long)ceil_div(P, 128) * ceil_div(K, 128) < 2048));
   if constexpr (sizeof(T) == 4) {
-    GemmConfig mid = make_config<T, 2, 2, BK, 2, 2, true, true>();     // 128 x 128
-    if (K > 64 && blocks(mid) >= 2048) return mid;
-    return make_config<T, 1, 1, BK, 2, 2, true, true>();               // 64 x 64
+    if (small) return make_config<T, 1, 1, BK, 2, 2, true, true>();  // 64 x 64
   }
-  if (K > 64) {
-    GemmConfig big = make_config<T, 4, 2, BK, 2, 2, true, true>();   // 256 x 128, four wavefronts
-    // a reduction of up to 24 blocks is mostly start and write-out, which 128 x 128 tiles, four to a CU and their loads two
-    // stages ahead, overlap better: 128 x 128 | 256 x 128, 64 -> 256 channels 1x1, N=64 56x56 28 | 34; 64 -> 128 3x3 at
-    // stride 2, N=64 112x112 60 | 62; 128 -> 128, N=32 64 | 58
-    if (reduction > 768 && blocks(big) >= kCus) return big;
-    GemmConfig mid = make_config<T, 2, 2, BK, 2, 2, true, true>();   // 128 x 128
-    // 128 x 128 | 64 x 64, N=16 and 20 128 -> 256, 56x56 (196 and 246 tiles of the first) 21.3 | 24.2 and 22.0 | 24.9, N=12
-    // (148 tiles) 20.3 | 16.8
-    if (blocks(mid) >= kCus || (blocks(mid) >= 3 * kCus / 4 && K % 128 == 0)) return mid;
-  }
-  return make_config<T, 1, 1, BK, 2, 2, true, true>();               // 64 x 64
+  return make_config<T, 2, 2, BK, 2, 2, true, true>();               // 128 x 128
 }
 
 // y (N, oH, oW, K) = direct convolution of x (N, H, W, C) with U (K, kh kw C): the batched product with the
@@ -1004,20 +977,25 @@ int gemm_direct_conv(const void* x, const void* U, const void* bias, void* y, in
   WC_CHECK_ARG(C > 0 && C % cq == 0 && K > 0 && K % 8 == 0, "gemm_direct_conv: C %d (multiple of %d), K %d (multiple of 8)", C, cq, K);
   const long long P = (long long)N * oH * oW;
   WC_CHECK_ARG(P > 0 && P < (1ll << 31) && (long long)kh * kw * C < (1ll << 24), "gemm_direct_conv: problem too large");
-  // Kernel rows of four and more taps over enough output to give a quarter of the CUs a 256 x 128 tile: one operand
-  // tile per kernel row (direct_rows.hip).  Measured against the tile per tap, fp16, stride 2, ms: N=32, 128 channels,
-  // 112x112: 4x4 0.091 | 0.102, 5x5 0.116 | 0.151, 7x7 0.181 | 0.264, 8x8 0.222 | 0.340; N=8: 7x7 0.081 | 0.122;
-  // 256 channels on 56x56: 7x7 0.166 | 0.249; 256 -> 512 on 28x28, N=64: 5x5 0.100 | 0.137; stride 1, 128 channels
-  // on 56x56: 5x5 0.103 | 0.135.  wc_test_gemm_override(., 2) takes it wherever it fits, (., 0) never.
+  // Kernel rows of six and more taps, and of five over 256 channels and more, whose 256 x 128 tiles are nearly one round of the
+  // chip: one operand tile per kernel row (direct_rows.hip), one workgroup per CU.  Everywhere else, and with shorter rows, the
+  // tile per tap (direct_dma.hip), two to a CU, is ahead.  us, rows | taps, fp16, stride 2, 128 channels, 112x112: 7x7 N=10 (123
+  // tiles) 83 | 68, N=13 (160) 85 | 95, N=16 91 | 97, N=20 103 | 110, N=26 177 | 160, N=32 182 | 178, N=64 365 | 356; 5x5 N=10 54 | 39,
+  // N=16 57 | 55, N=32 117 | 99, 256 -> 512 on 28x28 N=64 (196 tiles) 103 | 109; 6x6 256 channels on 56x56 N=32 136 | 147, 4x4 72 | 71.
+  // wc_test_gemm_override(., 2) takes it wherever it fits, (., 0) never.
   if (direct_rows_fits(N, C, K, kw, stride, oH, oW, dtype)) {
     const int mode = test_gemm_rows();
     const long long tiles = ceil_div_ll(P, 256) * ceil_div(K, 128);
     const bool k_fills = K % 128 == 0 || K % 128 >= 96;      // the last 128-channel tile is at least three quarters full
-    if (mode == 2 || (mode != 0 && tiles >= 64 && k_fills))
+    const bool long_rows = kw >= 6 || (kw == 5 && C >= 256);
+    if (mode == 2 || (mode != 0 && long_rows && tiles > kCus / 2 && tiles <= kCus && k_fills))
       return direct_rows_conv(x, U, bias, y, N, H, W, C, K, kh, kw, stride, pad_h, pad_w, oH, oW, dtype, stream, o_step, o_y0,
                               o_x0, o_H, o_W);
   }
-  GemmConfig c = dispatch_dtype(dtype, [&](auto t) { return choose_direct<decltype(t)>((int)P, K, kh * kw * C); });
+  const DirectClass whole{U, kh, kw, pad_h, pad_w, oH, oW, o_y0, o_x0};
+  if (dtype != WC_F32 && test_gemm_config() != 0 && direct_dma_fits(&whole, 1, H, W, C, K, stride))
+    return direct_dma(x, &whole, 1, bias, y, N, H, W, C, K, stride, dtype, stream, o_step, o_H, o_W);
+  GemmConfig c = dispatch_dtype(dtype, [&](auto t) { return choose_direct<decltype(t)>((int)P, K); });
   GemmArgs g;
   g.V = x; g.U = U; g.M = y; g.bias = bias;
   g.P = (int)P; g.K = K; g.ldm = K;
@@ -1041,62 +1019,60 @@ int gemm_direct_conv(const void* x, const void* U, const void* bias, void* y, in
   return WC_OK;
 }
 
-// The direct products of `n` parity classes in one launch, classes as in gemm_direct_conv's arguments (kernel rows of at
-// most 3 taps).  A class has a quarter of the pixels and at most four of nine taps, so one by one they leave most of the
-// chip idle.  Whole input gradient with its filter copy (also one launch now), us, before | now: bf16 N=32, 256 -> 128
-// channels, 28x28 -> 56x56 72 | 52; fp16 N=8 128 -> 64, 56x56 36 | 14; N=2 512 -> 256, 15x17 89 | 40; N=64 512 -> 256, 28x28
-// 120 | 95; N=64 128 -> 64, 112x112 119 | 116; fp32 N=8 128 -> 64, 56x56 64 | 33.  Tiles (256x128 | 128x128 | 64x64): the
-// first 52 | 57 | 59, the second 24 | 17 | 14, N=64 28x28 93 | 103 | 116.
+// The direct products of `n` parity classes in one launch, classes as in gemm_direct_conv's arguments.  A class has a quarter of
+// the pixels and at most four of nine taps, so one by one they leave most of the chip idle (us, one launch per class | one in all:
+// fp32 N=8 128 -> 64 channels, 28x28 -> 56x56 64 | 33).  16-bit types: direct_dma.hip.
 int gemm_direct_classes(const void* x, const DirectClass* classes, int n, void* y, int N, int H, int W, int C, int K,
                         int dtype, void* stream, int o_H, int o_W) {
   WC_CHECK_ARG(x && y && n > 0 && n <= 4, "gemm_direct_classes: %d classes", n);
   const int cq = dtype == WC_F32 ? 16 : 32;
   WC_CHECK_ARG(C > 0 && C % cq == 0 && K > 0 && K % 8 == 0, "gemm_direct_classes: C %d (multiple of %d), K %d (multiple of 8)", C, cq, K);
-  return dispatch_dtype(dtype, [&](auto t) -> int {
-    using T = decltype(t);
-    constexpr int BK = sizeof(T) == 4 ? 16 : 32;
-    auto launch = [&](auto wm, auto wn) -> int {
-      constexpr int WM = decltype(wm)::value, WN = decltype(wn)::value;
-      const GemmConfig c = make_config<T, WM, WN, BK, 2, 2, true, true>();        // the sizes of the tile
-      auto fn = &gemm_kernel<T, WM, WN, BK, 2, 2, true, true, true>;
-      GemmClassArgs g;
-      g.V = x; g.U = nullptr; g.M = y; g.bias = nullptr;
-      g.P = 0; g.K = K; g.ldm = K; g.Cp = 0; g.ldv = C; g.run_blocks = 0; g.jump = g.jump2 = 0; g.plane_runs = 0;
-      g.n_run = g.total_runs = g.run_rows = g.plane_extra = 0;
-      g.H = H; g.W = W; g.oH = g.oW = 1; g.conv_stride = 1; g.pad_h = g.pad_w = 0; g.kw = 1; g.cblocks = C / BK;
-      g.o_step = 2; g.o_y0 = g.o_x0 = 0; g.o_H = o_H; g.o_W = o_W;
-      g.sV = g.sU = g.sM = 0; g.tiles_p = 0; g.tiles_k = ceil_div(K, c.bn); g.T = 1;
-      g.n_classes = n;
-      int most = 0;
-      for (int i = 0; i < n; ++i) {
-        const DirectClass& d = classes[i];
-        const long long P = (long long)N * d.oH * d.oW;
-        WC_CHECK_ARG(d.U && P > 0 && P < (1ll << 31) && (long long)d.kh * d.kw * C < (1ll << 24), "gemm_direct_classes: problem too large");
-        g.cls[i] = {d.U, (long long)(W - d.kw) * C, (int)P, d.kh * d.kw * C, ceil_div((int)P, c.bm), d.kw * C / BK, d.kh + 1,
-                    d.oH, d.oW, d.pad_h, d.pad_w, d.kw, d.o_y0, d.o_x0};
-        most = std::max(most, g.cls[i].tiles_p);
-      }
-      const long long blocks = (long long)most * g.tiles_k * n;
-      WC_CHECK_ARG(blocks < (1ll << 30), "gemm_direct_classes: problem too large");
-      g.n_blocks = (int)blocks;
-      g.per_xcd = ceil_div((int)blocks, kXcds);
-      if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), c.lds)) return rc;
-      hipLaunchKernelGGL(fn, dim3((unsigned)(g.per_xcd * kXcds)), dim3(c.threads), c.lds, as_stream(stream), g);
-      WC_CHECK_LAUNCH("gemm_kernel (direct form, classes)");
-      return WC_OK;
-    };
-    // the rule of choose_direct over the tiles of all classes
-    long long P = 0;
-    for (int i = 0; i < n; ++i) P += (long long)N * classes[i].oH * classes[i].oW;
-    const long long mid = ceil_div_ll(P, 128) * ceil_div(K, 128);
-    if constexpr (sizeof(T) == 4) {
-      if (K > 64 && mid >= 2048) return launch(ic<2>{}, ic<2>{});
-    } else if (K > 64) {
-      if (ceil_div_ll(P, 256) * ceil_div(K, 128) >= kCus) return launch(ic<4>{}, ic<2>{});
-      if (mid >= kCus) return launch(ic<2>{}, ic<2>{});
+  if (dtype != WC_F32) {
+    if (test_gemm_config() != 0 && direct_dma_fits(classes, n, H, W, C, K, 1))
+      return direct_dma(x, classes, n, nullptr, y, N, H, W, C, K, 1, dtype, stream, 2, o_H, o_W);
+    for (int i = 0; i < n; ++i) {
+      const DirectClass& c = classes[i];
+      if (int rc = gemm_direct_conv(x, c.U, nullptr, y, N, H, W, C, K, c.kh, c.kw, 1, c.pad_h, c.pad_w, c.oH, c.oW, dtype, stream, 2, c.o_y0, c.o_x0,
+                                    o_H, o_W))
+        return rc;
     }
-    return launch(ic<1>{}, ic<1>{});
-  });
+    return WC_OK;
+  }
+  constexpr int BK = 16;
+  auto launch = [&](auto w) -> int {
+    constexpr int W_ = decltype(w)::value;
+    const GemmConfig c = make_config<float, W_, W_, BK, 2, 2, true, true>();        // the sizes of the tile
+    auto fn = &gemm_kernel<float, W_, W_, BK, 2, 2, true, true, true>;
+    GemmClassArgs g;
+    g.V = x; g.U = nullptr; g.M = y; g.bias = nullptr;
+    g.P = 0; g.K = K; g.ldm = K; g.Cp = 0; g.ldv = C; g.run_blocks = 0; g.jump = g.jump2 = 0; g.plane_runs = 0;
+    g.n_run = g.total_runs = g.run_rows = g.plane_extra = 0;
+    g.H = H; g.W = W; g.oH = g.oW = 1; g.conv_stride = 1; g.pad_h = g.pad_w = 0; g.kw = 1; g.cblocks = C / BK;
+    g.o_step = 2; g.o_y0 = g.o_x0 = 0; g.o_H = o_H; g.o_W = o_W;
+    g.sV = g.sU = g.sM = 0; g.tiles_p = 0; g.tiles_k = ceil_div(K, c.bn); g.T = 1;
+    g.n_classes = n;
+    int most = 0;
+    for (int i = 0; i < n; ++i) {
+      const DirectClass& d = classes[i];
+      const long long P = (long long)N * d.oH * d.oW;
+      WC_CHECK_ARG(d.U && P > 0 && P < (1ll << 31) && (long long)d.kh * d.kw * C < (1ll << 24), "gemm_direct_classes: problem too large");
+      g.cls[i] = {d.U, (long long)(W - d.kw) * C, (int)P, d.kh * d.kw * C, ceil_div((int)P, c.bm), d.kw * C / BK, d.kh + 1,
+                  d.oH, d.oW, d.pad_h, d.pad_w, d.kw, d.o_y0, d.o_x0};
+      most = std::max(most, g.cls[i].tiles_p);
+    }
+    const long long blocks = (long long)most * g.tiles_k * n;
+    WC_CHECK_ARG(blocks < (1ll << 30), "gemm_direct_classes: problem too large");
+    g.n_blocks = (int)blocks;
+    g.per_xcd = ceil_div((int)blocks, kXcds);
+    if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), c.lds)) return rc;
+    hipLaunchKernelGGL(fn, dim3((unsigned)(g.per_xcd * kXcds)), dim3(c.threads), c.lds, as_stream(stream), g);
+    WC_CHECK_LAUNCH("gemm_kernel (direct form, classes)");
+    return WC_OK;
+  };
+  // the rule of choose_direct over the tiles of all classes
+  long long P = 0;
+  for (int i = 0; i < n; ++i) P += (long long)N * classes[i].oH * classes[i].oW;
+  return K > 64 && ceil_div_ll(P, 128) * ceil_div(K, 128) >= 2048 ? launch(ic<2>{}) : launch(ic<1>{});
 }
 
 }  // namespace wc

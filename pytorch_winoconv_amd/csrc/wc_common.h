@@ -185,6 +185,12 @@ struct DirectClass { const void* U; int kh, kw, pad_h, pad_w, oH, oW, o_y0, o_x0
 int gemm_direct_classes(const void* x, const DirectClass* classes, int n, void* y, int N, int H, int W, int C, int K,
                         int dtype, void* stream, int o_H, int o_W);
 
+// Either with its operands brought to LDS by LDS-DMA (direct_dma.hip; 16-bit types): whether 32-bit offsets reach what a tile
+// reads and kernel rows and columns have at most 32 taps, and the launch
+bool direct_dma_fits(const DirectClass* classes, int n, int H, int W, int C, int K, int stride);
+int direct_dma(const void* x, const DirectClass* classes, int n, const void* bias, void* y, int N, int H, int W, int C, int K, int stride,
+               int dtype, void* stream, int o_step, int o_H, int o_W);
+
 // The direct form with one operand tile per kernel row (direct_rows.hip; 16-bit types, kernel rows of 4 to 8 taps, stride
 // 1 or 2): whether a problem is in its range (the input rows that 256 consecutive output pixels read, with their
 // padding, must fit a stage of kDirectRowsPixels pixels), and the launch, with the arguments of gemm_direct_conv.

@@ -1,0 +1,55 @@
+"""The direct form of 16-bit types on LDS-DMA: every tile shape, forward and input gradient, against fp64.
+
+Sizes at which it can go wrong: last tiles of pixels and channels that are partly or nearly empty, images that end inside a tile, taps
+outside the image on every side, tiles over many small images, output rows past the image's end (wide padding), reductions shorter
+than the loads in flight, kernels of one tap and of taps that a parity lacks."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from pytorch_winoconv_amd import engine
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # x shape, w shape, stride, pad
+    ((1, 32, 4, 4), (8, 32, 1, 1), 2, 0), ((3, 32, 9, 5), (32, 32, 1, 1), 2, 0), ((2, 64, 17, 23), (72, 64, 3, 3), 2, 1), ((2, 160, 17, 23), (96, 160, 3, 3), 2, 1), ((3, 32, 16, 15), (136, 32, 3, 3), 2, 1),
+    ((70, 32, 5, 3), (64, 32, 3, 3), 2, 1), ((2, 96, 9, 40), (264, 96, 2, 3), 2, (0, 1)), ((2, 32, 33, 31), (40, 32, 5, 5), 2, 2),
+    ((5, 32, 6, 7), (32, 32, 3, 5), 2, (3, 5)), ((2, 32, 20, 18), (128, 32, 7, 7), 2, 3), ((2, 64, 12, 11), (64, 64, 5, 4), 1, (4, 3)),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tile", [-1, 22, 23, 24, 25, 26])
+@pytest.mark.parametrize("case", CASES)
+def test_every_tile_is_exact_on_small_integers(dev, dtype, tile, case, gemm_override):
+    """Integers whose sums stay below 2^24 in fp32, so that only the last rounding remains, the same on both sides."""
+    xs, ws, stride, pad = case
+    g = torch.Generator().manual_seed(3)
+    x = torch.randint(-3, 4, xs, generator=g).double()
+    w = torch.randint(-2, 3, ws, generator=g).double()
+    b = torch.randint(-8, 9, (ws[0],), generator=g).double()
+    want = F.conv2d(x, w, b, stride, pad)
+    xd = x.to(dtype).to(dev).contiguous(memory_format=torch.channels_last)
+    gemm_override(config=tile, rows_mode=0)
+    y = engine.conv_forward(xd, w.to(dtype).to(dev), b.to(dtype).to(dev), stride, pad, 2, direct=True)
+    assert torch.equal(y.cpu(), want.float().to(dtype))
+    if stride == 2 and ws[0] % 32 == 0 and pad != (3, 5):       # other reductions are Winograd products, wider padding is refused
+        dy = torch.randint(-3, 4, tuple(want.shape), generator=g).double()
+        want = torch.nn.grad.conv2d_input(xs, w, dy, stride, pad)
+        dx = engine.conv_backward_input(dy.to(dtype).to(dev).contiguous(memory_format=torch.channels_last), w.to(dtype).to(dev), xs[2:], stride, pad, 2)
+        assert torch.equal(dx.cpu(), want.float().to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_where_the_register_staged_kernel_takes_over(dev, dtype, gemm_override):
+    """Forced here (kernel rows of more than 32 taps and images past 32-bit offsets take it by themselves)."""
+    g = torch.Generator().manual_seed(4)
+    x, w = torch.randint(-3, 4, (2, 32, 11, 13), generator=g).double(), torch.randint(-2, 3, (40, 32, 3, 3), generator=g).double()
+    gemm_override(config=0)
+    y = engine.conv_forward(x.to(dtype).to(dev), w.to(dtype).to(dev), None, 2, 1, 2, direct=True)
+    assert torch.equal(y.cpu(), F.conv2d(x, w, None, 2, 1).float().to(dtype))
+    dy = torch.randint(-3, 4, tuple(y.shape), generator=g).double()
+    dx = engine.conv_backward_input(dy.to(dtype).to(dev), w.to(dtype).to(dev), (11, 13), 2, 1, 2)
+    assert torch.equal(dx.cpu(), torch.nn.grad.conv2d_input((2, 32, 11, 13), w, dy, 2, 1).float().to(dtype))
