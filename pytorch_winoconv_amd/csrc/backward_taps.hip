@@ -12,9 +12,12 @@
 //
 // The transform domain multiplies less (8 products per pixel of a 3x3x3 filter against 27) but moves V and dM through
 // memory: N=8 128 -> 128, 16x56x56, fp16, 797 us of which 760 are that traffic; here 368 us, 0.95 PFLOP/s (a library
-// matrix product reaches 1.1 on this card).  The matrix unit is busy 52 % of the time at 1.95 GHz, the rest goes to feeding it:
-// 114 vector instructions beside the 24 products of a wavefront's step, and the LDS reads.  Variants that took more of either
-// were slower: dy turned channel by channel in LDS and read 16 bytes at a time 424 us, four wavefronts of all nine taps 439; operands
+// matrix product reaches 1.1 on this card) with x and dy through registers (taps_kernel) and 318 by LDS-DMA (taps_dma_kernel), sums
+// included.  Through registers 114 vector instructions stand beside the 24 products of a wavefront's step, most of them for
+// addresses; by LDS-DMA under forty, and a step takes 1.9 us for the 1.73 that its products take at the rate the matrix cores sustain with
+// changing operands.  Both | registers: N=64 64 -> 64, 56x56 33 | 42, 256 -> 256, 28x28 77 | 85, 128 -> 128, 28x28 37.5 | 40, N=8 64 -> 64, 8x28x28
+// 32.5 | 39.  Beside its steps a launch moves its partial sums, 59 MB each way where 200 workgroups share 0.6 MB of dw.  Variants that were
+// slower: dy turned channel by channel in LDS and read 16 bytes at a time 424 us, four wavefronts of all nine taps 439; operands
 // read a group ahead changed nothing (377).  Operands are exact, sums fp32.
 #include "wc_transform.h"
 
@@ -61,6 +64,43 @@ struct TapsArgs {
 
 template <int KG> constexpr int taps_tile_floats() { return KG * 6 * 24 * 64 * 4; }
 template <int KG> constexpr int taps_lds(int ring) { return 2 * kStep * kDyPitch<KG> + (ring + kMirror) * kXPitch; }
+
+// The products of 16 positions: x from `xb` on (rows XP bytes apart), two blocks of 32 output channels of dy
+template <typename T, int XP, int DP>
+__device__ __forceinline__ void taps_products(f32x16 (&acc)[3][2], const unsigned char* xb, const unsigned char* d0, const unsigned char* d1) {
+  typedef s16x4 __attribute__((address_space(3))) * LdsVec;
+  auto read_tr = [](const unsigned char* p) { return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsVec)(p))); };
+  const u32x2 e0 = read_tr(xb), e1 = read_tr(xb + 4 * XP), e2 = read_tr(xb + 8 * XP);
+  u32x4 df[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const unsigned char* const d = i ? d1 : d0;
+    const u32x2 lo = read_tr(d), hi = read_tr(d + 4 * DP);
+    df[i] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+  }
+  const u32x4 x0 = {e0[0], e0[1], e1[0], e1[1]}, x2 = {e0[1], e1[0], e1[1], e2[0]};
+  const u32x4 x1 = {__builtin_amdgcn_alignbit(e0[1], e0[0], 16), __builtin_amdgcn_alignbit(e1[0], e0[1], 16),
+                    __builtin_amdgcn_alignbit(e1[1], e1[0], 16), __builtin_amdgcn_alignbit(e2[0], e1[1], 16)};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    acc[0][i] = mfma(x0, df[i], acc[0][i], T{});
+    acc[1][i] = mfma(x1, df[i], acc[1][i], T{});
+    acc[2][i] = mfma(x2, df[i], acc[2][i], T{});
+  }
+}
+
+// Partial sums in the order of the accumulators: 1 KB per store
+__device__ __forceinline__ void taps_store(const f32x16 (&acc)[3][2], float* out) {
+#pragma unroll
+  for (int t = 0; t < 3; ++t)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4 o = {acc[t][i][4 * q], acc[t][i][4 * q + 1], acc[t][i][4 * q + 2], acc[t][i][4 * q + 3]};
+        *reinterpret_cast<f32x4*>(out + ((t * 2 + i) * 4 + q) * 256) = o;
+      }
+}
 
 template <typename T, int KG>
 __global__ __launch_bounds__(384 * KG) __attribute__((amdgpu_waves_per_eu(3, 3)))
@@ -167,8 +207,6 @@ void taps_kernel(TapsArgs a) {
   // 16 (b % 2) .. + 15
   const int frag_row = 8 * (lane >> 5) + ((lane & 15) >> 2), frag_col = ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
   const int x_lane = frag_row * XP + cb * 64 + frag_col, d_lane = frag_row * DP + kg * 128 + frag_col;
-  typedef s16x4 __attribute__((address_space(3))) * LdsVec;
-  auto read_tr = [](const unsigned char* p) { return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsVec)(p))); };
 
   int slot = 0;                                     // ring row of the step's first position
   for (int step = 0; step < steps; ++step) {
@@ -180,22 +218,7 @@ void taps_kernel(TapsArgs a) {
     for (int kk = 0; kk < kStep / 16; ++kk) {
       const int r = row + kk * 16 >= a.ring ? row + kk * 16 - a.ring : row + kk * 16;
       const unsigned char* const xb = lds_x + r * XP + x_lane;
-      const u32x2 e0 = read_tr(xb), e1 = read_tr(xb + 4 * XP), e2 = read_tr(xb + 8 * XP);
-      u32x4 df[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const u32x2 lo = read_tr(db + kk * 16 * DP + i * 64), hi = read_tr(db + (kk * 16 + 4) * DP + i * 64);
-        df[i] = u32x4{lo[0], lo[1], hi[0], hi[1]};
-      }
-      const u32x4 x0 = {e0[0], e0[1], e1[0], e1[1]}, x2 = {e0[1], e1[0], e1[1], e2[0]};
-      const u32x4 x1 = {__builtin_amdgcn_alignbit(e0[1], e0[0], 16), __builtin_amdgcn_alignbit(e1[0], e0[1], 16),
-                        __builtin_amdgcn_alignbit(e1[1], e1[0], 16), __builtin_amdgcn_alignbit(e2[0], e1[1], 16)};
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        acc[0][i] = mfma(x0, df[i], acc[0][i], T{});
-        acc[1][i] = mfma(x1, df[i], acc[1][i], T{});
-        acc[2][i] = mfma(x2, df[i], acc[2][i], T{});
-      }
+      taps_products<T, XP, DP>(acc, xb, db + kk * 16 * DP, db + kk * 16 * DP + 64);
     }
     if (more) {
       int to = slot + a.halo + kStep;               // ring = halo + 128: rows that no wavefront reads any more
@@ -207,17 +230,136 @@ void taps_kernel(TapsArgs a) {
     __syncthreads();
   }
 
-  // partial sums in the order of the accumulators: 1 KB per store
-  float* const out = a.part + (long long)wg * taps_tile_floats<KG>() + wave * 24 * 256 + lane * 4;
+  taps_store(acc, a.part + (long long)wg * taps_tile_floats<KG>() + wave * 24 * 256 + lane * 4);
+}
+
+// The same with x and dy brought to LDS by LDS-DMA, two steps ahead: channels in multiples of 8, 16-byte aligned tensors.  Where
+// the rows of a step lie is worked out once per position, by two wavefronts in turn, a step before it is needed, and read from a
+// table in LDS; positions outside the image are offsets outside the descriptor's range, which bring zeros.  Rows are not
+// padded: their 64-byte pieces are exchanged by the row instead (LDS-DMA writes rows one after the other), x in every other two rows,
+// dy of 128 channels by the row modulo 4.
+__device__ __forceinline__ void dma16(u32x4 desc, unsigned voff, unsigned lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" :: "v"(voff), "s"(desc), "s"(lds_addr) : "memory");
+}
+__device__ __forceinline__ u32x4 descriptor(const void* p, long long bytes) {
+  const unsigned long long u = reinterpret_cast<unsigned long long>(p);
+  const unsigned n = (unsigned)max(min(bytes, 0x7fffffffll), 0ll);
+  return u32x4{(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)u), (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(u >> 32)),
+               (unsigned)__builtin_amdgcn_readfirstlane((int)n), 0x00020000u};
+}
+
+template <int KG> constexpr int taps_dma_lds(int ring) { return 3 * kStep * KG * 128 + (ring + kMirror) * 128 + 4 * 2 * kStep * 4; }
+
+template <typename T, int KG>
+__global__ __launch_bounds__(384 * KG) __attribute__((amdgpu_waves_per_eu(3, 3)))
+void taps_dma_kernel(TapsArgs a) {
+  constexpr int NW = 6 * KG, ND = 8 * KG, NL = (ND + 8 + NW - 1) / NW;      // loads of 1 KB: ND of dy and 8 of x per step
+  constexpr int DP = KG * 128, XP = 128, DY_STAGE = kStep * DP, DROWS = 8 / KG;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+  unsigned char* const lds_x = lds + 3 * DY_STAGE;
+  unsigned* const table = reinterpret_cast<unsigned*>(lds_x + (a.ring + kMirror) * XP);      // of step s: (s & 3) * 128, dy, then x
+  const int wg = xcd_remap(blockIdx.x, a.per_xcd);
+  if (wg >= a.n_wg) return;
+  const int part = wg / a.tiles;
+  int tile = wg - part * a.tiles;
+  const int ct = tile % a.n_c; tile /= a.n_c;
+  const int kt = tile % a.n_k, kd = tile / a.n_k;
+  const int k0 = kt * 64 * KG, c0 = ct * 64;
+  const int q0 = part * a.part_steps * kStep, q_end = min(a.total, q0 + a.part_steps * kStep);
+  const int steps = (q_end - q0 + kStep - 1) / kStep;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int kg = wave / 6, kh = wave % 6 / 2, cb = wave & 1;
+
+  // offsets count from the plane of dy and the image of x that the part begins in
+  const int plane0 = fast_div(fast_div(q0, a.f_wp), a.f_hp), n0 = fast_div(plane0, a.f_od);
+  const long long dy_start = ((long long)plane0 * a.oH * a.oW * a.K + k0) * 2, x_start = ((long long)n0 * a.D * a.H * a.W * a.C + c0) * 2;
+  const u32x4 dyd = descriptor(static_cast<const unsigned char*>(a.dy) + dy_start, a.dy_elems * 2 - dy_start);
+  const u32x4 xd = descriptor(static_cast<const unsigned char*>(a.x) + x_start, a.x_elems * 2 - x_start);
+  auto place = [&](int pos, int& plane, int& h, int& w) {
+    const int row = fast_div(pos, a.f_wp);
+    w = pos - row * a.Wp;
+    plane = fast_div(row, a.f_hp);
+    h = row - plane * a.Hp;
+  };
+  auto dy_offset = [&](int pos) {
+    int plane, h, w;
+    place(pos, plane, h, w);
+    const bool ok = pos < q_end && h < a.oH && w < a.oW;
+    return ok ? (unsigned)(((plane - plane0) * a.oH + h) * a.oW + w) * (unsigned)a.K * 2u : kOutside;
+  };
+  auto x_offset = [&](int pos) {
+    int plane, h, w;
+    place(pos, plane, h, w);
+    const int n = fast_div(plane, a.f_od), d = plane - n * a.oD + kd - a.pd;
+    h -= a.ph; w -= a.pw;
+    const bool ok = pos < a.total && (unsigned)d < (unsigned)a.D && (unsigned)h < (unsigned)a.H && (unsigned)w < (unsigned)a.W;
+    return ok ? (unsigned)((((n - n0) * a.D + d) * a.H + h) * a.W + w) * (unsigned)a.C * 2u : kOutside;
+  };
+  auto fill = [&](int step, int which) {            // by one wavefront: the rows of dy (0) or x (1) of a step
+    table[(step & 3) * 2 * kStep + which * kStep + lane] = which ? x_offset(q0 + step * kStep + a.halo + lane) : dy_offset(q0 + step * kStep + lane);
+  };
+  // a lane's 16 bytes of a row, wherever the exchange puts them; channels that are not there lie outside
+  const int dy_chunk = KG == 2 ? (lane & 15) ^ ((lane >> 4) * 4) : (lane & 7) ^ ((lane >> 4) & 1) * 4, x_chunk = (lane & 7) ^ ((lane >> 4) & 1) * 4;
+  const unsigned dy_out = k0 + dy_chunk * 8 < a.K ? 0u : kOutside, x_out = c0 + x_chunk * 8 < a.C ? 0u : kOutside;
+  const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds, ldsx0 = lds0 + 3 * DY_STAGE;
+  auto load_x = [&](unsigned row_off, int slot, int v) {         // eight rows from ring row slot + 8 v on
+    const unsigned off = (row_off + x_chunk * 16) | x_out;
+    dma16(xd, off, ldsx0 + slot * XP + v * 1024);
+    if (slot == 0 && v * 8 < kMirror) dma16(xd, off, ldsx0 + a.ring * XP + v * 1024);
+  };
+  auto issue = [&](int step, int stage, int slot) {
+    const unsigned* const t = table + (step & 3) * 2 * kStep;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int u = wave + i * NW;
+      if (u < ND) dma16(dyd, (t[u * DROWS + lane / (8 * KG)] + dy_chunk * 16) | dy_out, lds0 + stage * DY_STAGE + u * 1024);
+      else if (u < ND + 8) load_x(t[kStep + (u - ND) * 8 + lane / 8], slot, u - ND);
+    }
+  };
+
+  f32x16 acc[3][2];
 #pragma unroll
   for (int t = 0; t < 3; ++t)
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const f32x4 o = {acc[t][i][4 * q], acc[t][i][4 * q + 1], acc[t][i][4 * q + 2], acc[t][i][4 * q + 3]};
-        *reinterpret_cast<f32x4*>(out + ((t * 2 + i) * 4 + q) * 256) = o;
-      }
+      for (int e = 0; e < 16; ++e) acc[t][i][e] = 0.f;
+
+  if (wave < 6) fill(wave >> 1, wave & 1);
+  for (int v = wave; v < a.halo / 8; v += NW) load_x(x_offset(q0 + v * 8 + lane / 8), v / 8 * 64, v % 8);
+  __syncthreads();
+  issue(0, 0, a.halo);
+  if (steps > 1) issue(1, 1, a.halo + kStep);
+
+  const int frag_row = 8 * (lane >> 5) + ((lane & 15) >> 2), frag_col = ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+  const int x_lane = frag_row * XP + ((cb * 64 + frag_col) ^ (((kh * a.Wp + frag_row) >> 1) & 1) * 64);
+  const int d_swap = KG == 2 ? (frag_row & 3) * 64 : ((frag_row >> 1) & 1) * 64;
+  const int d_lane0 = frag_row * DP + ((kg * 128 + frag_col) ^ d_swap), d_lane1 = frag_row * DP + ((kg * 128 + 64 + frag_col) ^ d_swap);
+
+  int slot = 0, to = a.halo + 2 * kStep, stage = 0, filler = 0;      // ring rows of the step's first position and of the loads two steps on
+  for (int step = 0; step < steps; ++step) {
+    // this step's loads are there (the next step's, at least two per wavefront, may be on their way), for all, and all are done
+    // with the last step's rows and the table's
+    if (step + 1 < steps) asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const int next = stage == 0 ? 2 : stage - 1;
+    if (step + 2 < steps) issue(step + 2, next, to);
+    if (step + 3 < steps && (wave >> 1) == filler) fill(step + 3, wave & 1);
+    filler = filler == NW / 2 - 1 ? 0 : filler + 1;
+    const int row = slot + kh * a.Wp;
+    const unsigned char* const db = lds + stage * DY_STAGE;
+#pragma unroll
+    for (int kk = 0; kk < kStep / 16; ++kk) {
+      const int r = row + kk * 16 >= a.ring ? row + kk * 16 - a.ring : row + kk * 16;
+      taps_products<T, XP, DP>(acc, lds_x + r * XP + x_lane, db + kk * 16 * DP + d_lane0, db + kk * 16 * DP + d_lane1);
+    }
+    slot += kStep;
+    if (slot >= a.ring) slot -= a.ring;
+    to += kStep;
+    if (to >= a.ring) to -= a.ring;
+    stage = stage == 2 ? 0 : stage + 1;
+  }
+  taps_store(acc, a.part + (long long)wg * taps_tile_floats<KG>() + wave * 24 * 256 + lane * 4);
 }
 
 // dw <- the sum of the parts, in a fixed order.  A workgroup owns one accumulator quarter (64 lanes x 4 input channels) of
@@ -257,19 +399,19 @@ __global__ __launch_bounds__(256) void taps_sum_kernel(TapsSumArgs a) {
 
 struct TapsPlan { int kg, halo, ring, total, steps, parts, part_steps, tiles; };
 
-// Parts of the line of positions.  A workgroup takes 1.7 us per step (2.2 with the whole chip at work; 1.3 for 64 output
+// Parts of the line of positions.  A workgroup takes 1.45 us per step (1.9 with the whole chip at work; 1.0 for 64 output
 // channels: two of those on a CU only share its LDS, one each is the most that pays), and its sums are written and read back, 0.29 MB per 128 x 64 channels: the
 // fewest microseconds for the slowest workgroup and that traffic.  Measured fp16, us over parts: N=64 128 -> 128, 28x28
-// 128: 42, 96: 41, 64: 44, 32: 63; 64 -> 64, 56x56 512: 53, 256: 41, 128: 55, 64: 91; N=8 64 -> 64, 28x28 128: 18, 64: 15;
-// N=8 128 -> 128, 16x56x56 42: 374, 31: 407, 21: 548.
+// 128: 39.6, 76: 37.2, 64: 38.5, 32: 53.5; 64 -> 64, 56x56 204: 34.4, 153: 37.7, 64: 66; 256 -> 256, 14x14 32: 43, 22: 41, 10: 55; N=8 64 -> 64, 28x28 128:
+// 17.5, 64: 14.2, 43: 13.6; N=8 128 -> 128, 16x56x56 42: 342, 28: 374, 19: 511.
 int taps_parts(int steps, int tiles, int kg) {
   int best = 1;
   double best_t = 1e30;
   for (int s = 1; s == 1 || s * tiles <= kCus; ++s) {
     const int per = ceil_div(steps, s), parts = ceil_div(steps, per);
     const double fill = (double)parts * tiles / kCus;
-    const double step_us = kg == 2 ? (fill > 0.5 ? 1.7 + 0.9 * (fill - 0.5) : 1.7) : 1.3;
-    const double t = per * step_us + parts * tiles * (kg * 0.147) / 5.0;
+    const double step_us = kg == 2 ? (fill > 0.5 ? 1.45 + 0.9 * (fill - 0.5) : 1.45) : 1.0;
+    const double t = per * step_us + parts * tiles * (kg * 0.147) / 4.0;
     if (t < best_t * (1.0 - 1e-9)) { best = s; best_t = t; }
   }
   return best;
@@ -307,9 +449,16 @@ int launch_taps(const wc_conv_desc* d, const int out[3], const TapsPlan& p, cons
   a.total = p.total; a.part_steps = p.part_steps; a.halo = p.halo; a.ring = p.ring;
   a.n_kd = d->kernel[0]; a.n_k = ceil_div(a.K, 64 * KG); a.n_c = ceil_div(a.C, 64); a.tiles = p.tiles;
   a.n_wg = p.tiles * p.parts; a.per_xcd = ceil_div(a.n_wg, kXcds);
-  const int lds = taps_lds<KG>(p.ring);
-  if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&taps_kernel<T, KG>), lds)) return rc;
-  hipLaunchKernelGGL((taps_kernel<T, KG>), dim3((unsigned)(a.per_xcd * kXcds)), dim3(384 * KG), lds, as_stream(stream), a);
+  // x and dy by LDS-DMA where rows are whole 16 bytes and 31-bit offsets reach what a part reads
+  const long long planes = ((p.part_steps + 4ll) * kStep + p.halo) / ((long long)a.Hp * a.Wp) + 2;
+  const int dma_ring = p.halo + 3 * kStep, dma_lds = taps_dma_lds<KG>(dma_ring);
+  const bool dma = a.C % 8 == 0 && a.K % 8 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy)) & 15) == 0 &&
+                   planes * a.oH * a.oW * a.K * 2 < (1ll << 31) && (planes / a.oD + 2) * a.D * a.H * a.W * a.C * 2 < (1ll << 31) && dma_lds <= 160 * 1024;
+  if (dma) a.ring = dma_ring;
+  const auto fn = dma ? &taps_dma_kernel<T, KG> : &taps_kernel<T, KG>;
+  const int lds = dma ? dma_lds : taps_lds<KG>(p.ring);
+  if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)) return rc;
+  hipLaunchKernelGGL(fn, dim3((unsigned)(a.per_xcd * kXcds)), dim3(384 * KG), lds, as_stream(stream), a);
   WC_CHECK_LAUNCH("taps_kernel");
   TapsSumArgs b;
   b.part = part; b.dw = dw;
@@ -322,17 +471,19 @@ int launch_taps(const wc_conv_desc* d, const int out[3], const TapsPlan& p, cons
 
 }  // namespace
 
-// Against the transform domain, fp16, us (taps | F(2,3), in 2-D also F(4,3) tiles): N=8 128 -> 128, 16x56x56 368 | 797;
-// N=8 32 -> 64, 16x40x40 81 | 174; N=2 128 -> 128, 4x14x14 24 | 50; N=64 128 -> 128, 28x28 41 | 67 | 53; 64 -> 64, 56x56 40 |
-// 119 | 72; N=64 256 -> 256, 14x14 45 | 50 | 49; N=1 128 -> 128, 28x28 15 | 20 | 21.  F(4,3) multiplies a quarter as much
-// and its traffic grows with C + K, the products here with C K (padded to tiles), so it is ahead on wide layers: 256 -> 256,
-// 56x56 257 | 420 | 275; 512 -> 512, 28x28 266 | 307 | 240, 14x14 52 | 60 | 54, N=64 7x7 55 | 62 | 53; 72 -> 136, N=30
-// 20x20 33 | 39 | 32; 100 -> 150, N=64 28x28 56 | 65 | 53, against F(2,3) alone still ahead: 50 -> 64, N=32 56x56 32 | 71; 3 -> 64,
-// N=64 112x112 106 | 334; 45 -> 77, N=2 8x28x28 33 | 61.  Small problems are launches and latency: two of them here, six there (512 -> 512, N=1 7x7 28 | 39 | 48).
+// Against the transform domain, fp16, us (taps | F(2,3), in 2-D also F(4,3) tiles): N=8 128 -> 128, 16x56x56 318 | 779; 64 -> 64,
+// 8x28x28 33 | 82; N=64 128 -> 128, 28x28 38 | 66 | 53; N=64 256 -> 256, 14x14 42 | 52 | 49; N=8 256 -> 256, 28x28 35 | 41 | 39; N=1 128 -> 128,
+// 28x28 15 | 20 | 21.  F(4,3) multiplies a quarter as much and its traffic grows with C + K, the products here with C K (padded to
+// tiles), so it is ahead on large wide layers, counted in steps of 64 positions and tiles of 128 x 64 channels: 512 -> 512, 56x56 N=32
+// (54000) 426 | 529 | 375, 28x28 N=64 (29000) 236 | 283 | 236, N=16 (7200) 86 | 96 | 110; 384 -> 384, 28x28 N=64 (16000) 146 | 212 | 143, 14x14 (4600) 62 | 85 |
+// 78; 1024 -> 1024, 14x14 N=64 (33000) 284 | 262 | 266, 7x7 (10400) 129 | 134 | 136; 256 -> 256, 56x56 N=64 (27000) 226 | 405 | 268; 72 -> 72, 56x56 (6700) 66 | 133 | 77.
+// Channels that are no multiples of 8 go through registers (us, F(4,3) | taps: 100 -> 150, N=64 28x28 53 | 56; against F(2,3) alone
+// still ahead: 50 -> 64, N=32 56x56 32 | 71; 3 -> 64, N=64 112x112 106 | 334).  Small problems are launches and latency: two of them
+// here, six there (512 -> 512, N=1 7x7 28 | 39 | 48).
 bool taps_gradient_fits(const wc_conv_desc* d, const int out[3], size_t* workspace_bytes) {
   TapsPlan p;
   if (test_gemm_config() == 20 || !taps_plan(d, out, &p)) return false;
-  if (d->ndim == 2 && d->m == 4 && (long long)p.steps * p.tiles > 2560) {
+  if (d->ndim == 2 && d->m == 4 && (long long)p.steps * p.tiles > (d->C % 8 == 0 && d->K % 8 == 0 ? 12000 : 2560)) {
     const long long padded = (long long)ceil_div(d->K, 64 * p.kg) * 64 * p.kg * ceil_div(d->C, 64) * 64;
     if (padded > 256 * 256 || padded * 5 > 8ll * d->C * d->K) return false;
   }

@@ -99,3 +99,31 @@ def test_positions_close_to_2g(dev, n):
     x[-2:], dy[-2:] = xl.to(dev), dyl.to(dev)
     # nine values of a sum over 73000 products: the transform domain as in test_gpu_backward.py
     assert _err(engine.conv_backward_weight(x, dy, shape, 1, pads, 2), ref) <= (BOUND[x.dtype] if n == 57343 else 2e-2)
+
+
+DMA_CASES = [
+    # x shape, K, pad: channels in multiples of 8, which LDS-DMA brings
+    ((1, 8, 3, 3), 8, 0), ((1, 8, 1, 1), 8, (2, 1)), ((1, 8, 1, 1, 1), 8, 1),           # fewer steps than loads in flight
+    ((2, 8, 9, 11), 72, 1), ((1, 64, 8, 16), 64, 1), ((3, 72, 20, 17), 136, (0, 2)),     # two steps and more; last channels on both sides
+    ((70, 16, 1, 2), 24, 1), ((9, 16, 2, 1, 3), 136, (1, 2, 1)),                         # many small images and planes in a step
+    ((1, 8, 4, 253), 24, 1), ((2, 136, 3, 6, 5), 200, (0, 1, 2)), ((4, 64, 33, 64), 64, 1),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", DMA_CASES)
+def test_by_lds_dma_exact_on_small_integers(dev, dtype, case):
+    """Integers whose sums stay below 2^24: exact in fp32, so only the last rounding remains, the same on both sides; NaN around x
+    and dy in memory, which positions outside the image must not read."""
+    xs, K, pad = case
+    x, dy, pads, shape, _ = _operands(xs, K, pad, dtype)
+    x, dy = (x * 2).round().clamp(-4, 4), (dy * 2).round().clamp(-4, 4)
+    grad = torch.nn.grad.conv2d_weight if len(xs) == 4 else torch.nn.grad.conv3d_weight
+    want = grad(x.double(), shape, dy.double(), padding=pads).float().to(dtype)
+
+    def guarded(t):
+        flat = torch.full((t.numel() + 4096,), float("nan"), dtype=dtype, device=dev)[2048:2048 + t.numel()]
+        last = t.to(dev).movedim(1, -1)
+        return flat.view(last.shape).copy_(last).movedim(-1, 1)
+
+    assert torch.equal(engine.conv_backward_weight(guarded(x), guarded(dy), shape, 1, pads, 2).cpu(), want)
