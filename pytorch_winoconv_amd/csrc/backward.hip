@@ -198,20 +198,37 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(float* __restrict__ dU, 
   *reinterpret_cast<float4*>(base) = sum;
 }
 
-// acc[t][i] = sum over s of dU[t][s][i]: the same sum, written densely (the layout grad_filter_store_kernel reads)
-__global__ __launch_bounds__(256) void sum_parts_out_kernel(const float* __restrict__ dU, float* __restrict__ acc, int S,
-                                                            long long n, long long total4) {
-  const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= total4) return;
+// dw[k][c][tap] through element strides <- the sum over s of dU[tap][s][k][c] (n = K C, C a multiple of 4), in a fixed order: the
+// wavefronts of a workgroup share out the parts of 256 values, with four loads of a thread on their way.  The whole gradient, us, with a
+// sum of one thread per value and a second kernel for the way to dw | so, fp16: 9 x 128 x 128 in 28 parts 60 | 48.5, in 24 parts 23 | 15.6,
+// 1x1 64 -> 256, 64 parts 40 | 24.5.
+template <typename T>
+__global__ __launch_bounds__(256) void sum_parts_store_kernel(const float* __restrict__ dU, T* __restrict__ dw, int S, long long n,
+                                                             long long total4, long long s0, long long s1, long long s3, long long s4, int C, int kW) {
+  __shared__ float4 sums[3][64];
+  const int lane = threadIdx.x & 63, group = threadIdx.x >> 6;
+  const long long idx = (long long)blockIdx.x * 64 + lane;
+  const bool in = idx < total4;
   const long long n4 = n / 4;
-  const long long t = idx / n4, i = (idx % n4) * 4;
-  const float* base = dU + t * S * n + i;
-  float4 sum = *reinterpret_cast<const float4*>(base);
-  for (int sp = 1; sp < S; ++sp) {
-    const float4 v = *reinterpret_cast<const float4*>(base + sp * n);
+  const long long t = in ? idx / n4 : 0, i = in ? (idx % n4) * 4 : 0;
+  const float* const base = dU + t * S * n + i;
+  float4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int p = group; p < S; p += 4) {
+    const float4 v = *reinterpret_cast<const float4*>(base + p * n);
     sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
   }
-  *reinterpret_cast<float4*>(acc + t * n + i) = sum;
+  if (group) sums[group - 1][lane] = sum;
+  __syncthreads();
+  if (group || !in) return;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const float4 v = sums[j][lane];
+    sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
+  }
+  const int k = (int)(i / C), c = (int)(i % C);
+  T* const dst = dw + k * s0 + c * s1 + (int)t / kW * s3 + (int)t % kW * s4;
+  dst[0] = static_cast<T>(sum.x); dst[s1] = static_cast<T>(sum.y); dst[2 * s1] = static_cast<T>(sum.z); dst[3 * s1] = static_cast<T>(sum.w);
 }
 
 // dw[k][c][tap] through element strides <- acc (taps, K, C)
@@ -293,7 +310,7 @@ bool gathered_layout(const wc_conv_desc* d, BwdLayout* L) {
   L->Pq = (int)(((P + S - 1) / S + 31) / 32 * 32);
   L->v_bytes = L->dm_bytes = 0;
   L->du_bytes = round256((size_t)taps * S * d->K * d->C * 4);
-  L->acc_bytes = round256((size_t)taps * d->K * d->C * 4);
+  L->acc_bytes = 0;
   return true;
 }
 
@@ -420,22 +437,24 @@ int wc_conv_backward_weight(const wc_conv_desc* d, const void* x, const void* dy
     const long long P = L.tiles_per_image * d->N;
     rc = batched_gemm_tn(dy, x, dU, 1, P, d->K, d->C, d->K, d->C, d->C, L.S, L.Pq, d->dtype, stream);
     if (rc) return rc;
-    if (L.S > 1) {
-      const long long n = (long long)d->K * d->C, total4 = n / 4;
-      hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)ceil_div_ll(total4, 256)), dim3(256), 0, s, dU, L.S, n, total4);
-      WC_CHECK_LAUNCH("sum_parts_kernel");
-    }
-    acc = dU;
   }
   if (L.gathered) {
     rc = gemm_tn_conv(dy, x, dU, d->N, d->in[1], d->in[2], d->C, d->K, d->kernel[1], d->kernel[2], d->stride, d->pad[1],
                       d->pad[2], L.out[1], L.out[2], L.S, L.Pq, d->dtype, stream);
     if (rc) return rc;
-    const long long n = (long long)d->K * d->C, total4 = (long long)taps * n / 4;
-    hipLaunchKernelGGL(sum_parts_out_kernel, dim3((unsigned)ceil_div_ll(total4, 256)), dim3(256), 0, s, dU, acc, L.S, n, total4);
-    WC_CHECK_LAUNCH("sum_parts_out_kernel");
   }
-  for (int b0 = 0; b0 < d->N && !L.one_tap && !L.gathered; b0 += L.chunk) {
+  if (L.one_tap || L.gathered) {
+    const long long n = (long long)d->K * d->C, total4 = (long long)taps * n / 4;
+    dispatch_dtype(d->dtype, [&](auto t) {
+      using TT = decltype(t);
+      hipLaunchKernelGGL(sum_parts_store_kernel<TT>, dim3((unsigned)ceil_div_ll(total4, 64)), dim3(256), 0, s, dU, static_cast<TT*>(dw), L.S, n, total4,
+                         (long long)dw_strides[0], (long long)dw_strides[1], (long long)dw_strides[3], (long long)dw_strides[4], d->C, d->kernel[2]);
+      return 0;
+    });
+    WC_CHECK_LAUNCH("sum_parts_store_kernel");
+    return WC_OK;
+  }
+  for (int b0 = 0; b0 < d->N; b0 += L.chunk) {
     const int n = std::min(L.chunk, d->N - b0);
     const long long P = L.tiles_per_image * n;
     rc = wc_input_transform(d, &L.plan, static_cast<const unsigned char*>(x) + b0 * x_image, n, V, stream);

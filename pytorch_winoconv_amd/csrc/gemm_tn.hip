@@ -21,6 +21,8 @@
 #include "wc_common.h"
 #include "wc_transform.h"
 
+#include <algorithm>
+
 namespace wc {
 
 namespace {
@@ -47,6 +49,11 @@ struct GemmTnArgs {
   // (stride oy + ky - pad_h, stride ox + kx - pad_w) of image b, zeros outside the image
   int H, W, oH, oW, conv_stride, pad_h, pad_w, kw;
   FastDiv div_per, div_oW;
+  long long b_elems;         // of x
+  // the taps of a part as neighbours, which read the same rows of dy and mostly the same of x, where these are more than L2
+  // holds; 0: the parts of a tap, which do not meet at the same lines (us, fp16, stride 2, taps | parts: N=32 128 -> 128, 112x112, 128 MB
+  // in all, 60 | 90, N=64 64 -> 64, 56x56, 32 MB 38 | 44; N=16 96 -> 96, 50x50, 10 MB 27.5 | 26.5, N=8 128 -> 128, 56x56, 8 MB 27 | 23)
+  int n_taps;
 };
 
 __device__ __forceinline__ floatx16 mfma16(short8v a, short8v b, floatx16 c, half_t) {
@@ -75,8 +82,8 @@ __global__ __launch_bounds__(256, 2) void gemm_tn_kernel(GemmTnArgs g) {
   const int tb = blk % g.tiles_b;
   const int ta = (blk / g.tiles_b) % g.tiles_a;
   const int ts = blk / (g.tiles_b * g.tiles_a);
-  const int s = ts % g.S;
-  const int t = ts / g.S;
+  const int s = GATHER && g.n_taps ? ts / g.n_taps : ts % g.S;
+  const int t = GATHER && g.n_taps ? ts % g.n_taps : ts / g.S;
   const int a0 = ta * BT, b0 = tb * BT;
   const long long p_begin = (long long)s * g.Pq;
   const long long p_end = min(g.P, p_begin + g.Pq);
@@ -216,6 +223,153 @@ __global__ __launch_bounds__(256, 2) void gemm_tn_kernel(GemmTnArgs g) {
   }
 }
 
+// 16-bit types with both operands brought to LDS by LDS-DMA, three stages of 32 rows ahead.  Rows are not padded: their 64-byte
+// pieces are exchanged by the row instead, so that the 4 rows of a transposing read fall into different banks.  Rows past the
+// part's end and pixels outside the image are offsets outside the descriptor's range, which bring zeros.  GATHER: where the
+// rows of x lie is worked out for 64 rows at a time by one wavefront and read from a table in LDS.
+// gemm_tn_kernel waits for each of its loads, which stand behind branches, a stage after it asked for them.  us, whole gradients in fp16, through
+// registers | by LDS-DMA: N=64 256 -> 512, 28x28 at stride 2 67 | 55, 1x1 64 -> 256, 56x56 54 | 40, F(4,3) of 512 -> 512, 56x56 N=32 372 | 339; N=32 128 ->
+// 128, 112x112 at stride 2 85 | 90, bound by the same rows of x and dy from beyond L2 for every tap, and 60 with the taps as neighbours (n_taps).
+__device__ __forceinline__ void dma16(Chunk16 desc, unsigned voff, unsigned lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" :: "v"(voff), "s"(desc), "s"(lds_addr) : "memory");
+}
+__device__ __forceinline__ Chunk16 descriptor(const void* p, long long bytes) {
+  const unsigned long long u = reinterpret_cast<unsigned long long>(p);
+  const unsigned n = (unsigned)max(min(bytes, 0x7fffffffll), 0ll);
+  return Chunk16{(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)u), (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(u >> 32)),
+                 (unsigned)__builtin_amdgcn_readfirstlane((int)n), 0x00020000u};
+}
+
+constexpr int kTnRows = 32, kTnStages = 4;
+template <int W> constexpr int tn_dma_lds() { return kTnStages * 2 * kTnRows * W * 128 + 4 * 64 * 4; }
+
+template <typename T, int W, bool GATHER>
+__global__ __launch_bounds__(256, 2) void gemm_tn_dma_kernel(GemmTnArgs g) {
+  constexpr int BT = 64 * W, PITCH = BT * 2, HALF = kTnRows * PITCH, STAGE = 2 * HALF;     // bytes: A's rows, then B's
+  constexpr int L = W, RPI = 8 / W;                // loads of 1 KB of each operand per wavefront and stage, rows per load
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds_raw[];
+  unsigned* const table = reinterpret_cast<unsigned*>(lds_raw + kTnStages * STAGE);        // rows 64 j .. 64 j + 63 of the part at (j & 3) * 64
+
+  const int blk = xcd_remap(blockIdx.x, g.per_xcd);
+  if (blk >= g.n_blocks) return;
+  const int tb = blk % g.tiles_b;
+  const int ta = (blk / g.tiles_b) % g.tiles_a;
+  const int ts = blk / (g.tiles_b * g.tiles_a);
+  const int s = GATHER && g.n_taps ? ts / g.n_taps : ts % g.S;
+  const int t = GATHER && g.n_taps ? ts % g.n_taps : ts / g.S;
+  const int a0 = ta * BT, b0 = tb * BT;
+  const long long p_begin = (long long)s * g.Pq;
+  const int rows = (int)max(min(g.P - p_begin, (long long)g.Pq), 0ll);
+  const int nk = (rows + kTnRows - 1) / kTnRows;
+
+  const T* const Ap = static_cast<const T*>(g.A) + ((GATHER ? 0 : (long long)t * g.P) + p_begin) * g.lda + a0;
+  const Chunk16 ad = descriptor(Ap, ((long long)rows * g.lda - a0) * 2);
+  const int image0 = GATHER ? fast_div((int)min(p_begin, g.P - 1), g.div_per) : 0;
+  const long long b_start = GATHER ? (long long)image0 * g.H * g.W * g.ldb + b0 : ((long long)t * g.P + p_begin) * g.ldb + b0;
+  const T* const Bp = static_cast<const T*>(g.B) + b_start;
+  const Chunk16 bd = descriptor(Bp, (GATHER ? g.b_elems - b_start : (long long)rows * g.ldb - b0) * 2);
+  const int tap_y = GATHER ? t / g.kw : 0, tap_x = GATHER ? t - tap_y * g.kw : 0;
+
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  auto fill = [&](int j) {                         // by one wavefront
+    const int row = j * 64 + lane, pi = (int)min(p_begin + row, g.P - 1);
+    const int b = fast_div(pi, g.div_per), rem = pi - b * (g.oH * g.oW);
+    const int oy = fast_div(rem, g.div_oW), ox = rem - oy * g.oW;
+    const int iy = oy * g.conv_stride + tap_y - g.pad_h, ix = ox * g.conv_stride + tap_x - g.pad_w;
+    const bool inside = row < rows && (unsigned)iy < (unsigned)g.H && (unsigned)ix < (unsigned)g.W;
+    table[(j & 3) * 64 + lane] = inside ? (unsigned)(((b - image0) * g.H + iy) * g.W + ix) * (unsigned)g.ldb * 2u : kOutside;
+  };
+  // a lane's 16 bytes of a row, wherever the exchange puts them; columns that are not there lie outside
+  const int lrow = lane / (8 * W), chunk = W == 2 ? (lane & 15) ^ (lrow & 3) * 4 : (lane & 7) ^ ((lrow >> 1) & 1) * 4;
+  const unsigned a_out = a0 + chunk * 8 < g.lda ? 0u : kOutside, b_out = b0 + chunk * 8 < g.ldb ? 0u : kOutside;
+  const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds_raw;
+  auto issue = [&](int kt) {
+    const unsigned to = lds0 + (kt % kTnStages) * STAGE + wave * L * 1024;
+#pragma unroll
+    for (int i = 0; i < L; ++i) {
+      const int row = kt * kTnRows + (wave * L + i) * RPI + lrow;
+      dma16(ad, ((unsigned)row * (unsigned)g.lda * 2u + chunk * 16) | a_out, to + i * 1024);
+      const unsigned off = GATHER ? table[row & 255] : (unsigned)row * (unsigned)g.ldb * 2u;
+      dma16(bd, (off + chunk * 16) | b_out, to + HALF + i * 1024);
+    }
+  };
+
+  const int wa = wave >> 1, wb = wave & 1, l32 = lane & 31, lhi = lane >> 5;
+  floatx16 acc[W][W];
+#pragma unroll
+  for (int i = 0; i < W; ++i)
+#pragma unroll
+    for (int j = 0; j < W; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+  // 16-lane group b reads rows 8 lhi + (0..3), columns 16 (b & 1) + (0..15), as in gemm_tn_kernel
+  int fa[W], fb[W];
+  {
+    const int sl = lane & 15, row = 8 * lhi + (sl >> 2), col = ((lane >> 4) & 1) * 32 + (sl & 3) * 8;
+    const int swap = W == 2 ? (row & 3) * 64 : ((row >> 1) & 1) * 64;
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      fa[i] = row * PITCH + ((((wa * W + i) * 64) + col) ^ swap);
+      fb[i] = HALF + row * PITCH + ((((wb * W + i) * 64) + col) ^ swap);
+    }
+  }
+
+  if constexpr (GATHER) {
+    if (wave < 2) fill(wave);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int k = 0; k < kTnStages - 1; ++k)
+    if (k < nk) issue(k);
+  for (int kt = 0; kt < nk; ++kt) {
+    if (kt + 2 < nk) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(4 * L) : "memory");
+    else if (kt + 1 < nk) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(2 * L) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (kt + kTnStages - 1 < nk) issue(kt + kTnStages - 1);
+    if constexpr (GATHER) {
+      // rows of the stages four and five on: the next step reads the first of them
+      if ((kt & 1) == 0 && kt + 4 < nk && wave == ((kt >> 1) & 3)) fill((kt >> 1) + 2);
+    }
+    const unsigned char* const st = lds_raw + (kt % kTnStages) * STAGE;
+    typedef short4v __attribute__((address_space(3))) * LdsVec;
+    auto read = [&](const unsigned char* src) {
+      const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsVec)(src));
+      const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsVec)(src + 4 * PITCH));
+      return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+#pragma unroll
+    for (int kk = 0; kk < kTnRows / 16; ++kk) {
+      short8v af[W], bf[W];
+#pragma unroll
+      for (int i = 0; i < W; ++i) af[i] = read(st + kk * 16 * PITCH + fa[i]);
+#pragma unroll
+      for (int j = 0; j < W; ++j) bf[j] = read(st + kk * 16 * PITCH + fb[j]);
+#pragma unroll
+      for (int i = 0; i < W; ++i)
+#pragma unroll
+        for (int j = 0; j < W; ++j) acc[i][j] = mfma16(bf[j], af[i], acc[i][j], T{});
+    }
+  }
+
+  float* const Dt = g.D + ((long long)t * g.S + s) * g.na * g.ldd;
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    const int row = a0 + (wa * W + i) * 32 + l32;
+    if (row >= g.na) continue;
+#pragma unroll
+    for (int j = 0; j < W; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int col = b0 + (wb * W + j) * 32 + 8 * q + 4 * lhi;
+        if (col < g.ldd) {
+          floatx4 o = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+          *reinterpret_cast<floatx4*>(Dt + (long long)row * g.ldd + col) = o;
+        }
+      }
+  }
+}
+
 template <typename T, int W, bool GATHER = false>
 int launch_tn(GemmTnArgs g, int T_, void* stream) {
   constexpr int BT = 64 * W;
@@ -227,6 +381,20 @@ int launch_tn(GemmTnArgs g, int T_, void* stream) {
   WC_CHECK_ARG(blocks < (1ll << 30), "batched_gemm_tn: problem too large");
   g.n_blocks = (int)blocks;
   g.per_xcd = ceil_div((int)blocks, kXcds);
+  if constexpr (sizeof(T) == 2) {
+    // by LDS-DMA where 31-bit offsets reach what a part reads, which its last stages overrun by up to 255 rows
+    const long long images = GATHER ? (long long)(g.Pq - 1) / ((long long)g.oH * g.oW) + 2 : 0;
+    const long long reach = (g.Pq + 256ll) * std::max(g.lda, GATHER ? 0 : g.ldb) * 2;
+    if (((reinterpret_cast<uintptr_t>(g.A) | reinterpret_cast<uintptr_t>(g.B)) & 15) == 0 && reach < (1ll << 31) &&
+        images * g.H * g.W * g.ldb * 2 < (1ll << 31) && g.P < (1ll << 31)) {
+      const auto fn = &gemm_tn_dma_kernel<T, W, GATHER>;
+      constexpr int dma_lds = tn_dma_lds<W>();
+      if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), dma_lds)) return rc;
+      hipLaunchKernelGGL(fn, dim3((unsigned)(g.per_xcd * kXcds)), dim3(256), dma_lds, as_stream(stream), g);
+      WC_CHECK_LAUNCH("gemm_tn_dma_kernel");
+      return WC_OK;
+    }
+  }
   if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_tn_kernel<T, W, BK, GATHER>), lds)) return rc;
   hipLaunchKernelGGL((gemm_tn_kernel<T, W, BK, GATHER>), dim3((unsigned)(g.per_xcd * kXcds)), dim3(256), lds, as_stream(stream), g);
   WC_CHECK_LAUNCH("gemm_tn_kernel");
@@ -247,7 +415,7 @@ int batched_gemm_tn(const void* A, const void* B, float* D, int T_, long long P,
   g.lda = lda; g.ldb = ldb; g.na = na; g.nb = nb; g.ldd = ldd;
   g.S = S; g.Pq = Pq;
   g.H = g.W = g.oH = g.oW = g.conv_stride = g.pad_h = g.pad_w = g.kw = 0;
-  g.div_per = g.div_oW = make_fast_div(1);
+  g.div_per = g.div_oW = make_fast_div(1); g.b_elems = 0; g.n_taps = 0;
   const bool big = na > 64 && nb > 64;
   return dispatch_dtype(dtype, [&](auto t) {
     using TT = decltype(t);
@@ -270,6 +438,9 @@ int gemm_tn_conv(const void* dy, const void* x, float* D, int N, int H, int W, i
   g.S = S; g.Pq = Pq;
   g.H = H; g.W = W; g.oH = oH; g.oW = oW; g.conv_stride = stride; g.pad_h = pad_h; g.pad_w = pad_w; g.kw = kw;
   g.div_per = make_fast_div(oH * oW); g.div_oW = make_fast_div(oW);
+  g.b_elems = (long long)N * H * W * C; 
+  const long long bytes = (g.b_elems + P * K) * (dtype == WC_F32 ? 4 : 2);
+  g.n_taps = bytes > (16 << 20) ? kh * kw : 0;
   const bool big = K > 64 && C > 64;
   return dispatch_dtype(dtype, [&](auto t) {
     using TT = decltype(t);
