@@ -510,7 +510,8 @@ RowBox choose_box(int N, int oD, int oH, int nW, int kd, int kh, int tiles, int 
 // 68 | 60 | 74; N=16, 256 -> 256, 14x14 21 | 15 | 12.4 | 10.6; N=1, 512 -> 512, 7x7 33 | 22 | 19 | 12.  (Layers of up to 128 input
 // channels come here in 3-D or with tile 4; with tile 2 the one-kernel F(2x2, 3x3) form takes most of them, see row_preferred.)
 enum RowShape { kRowWide, kRowHalf, kRowSmall, kRowSplit };
-struct RowPlan { RowShape shape; RowBox box; long long wide_groups; int tall_images; double us; };
+// tall_planes: output planes, images in 2-D, that go to tall boxes; the rest is rest_n images of rest_d planes
+struct RowPlan { RowShape shape; RowBox box; long long wide_groups; int tall_planes, rest_n, rest_d; double us; };
 
 RowPlan make_row_shape(int N, int oD, int oH, int nW, int kd, int kh, int K, int steps) {
   RowPlan p{};
@@ -546,27 +547,36 @@ RowPlan make_row_shape(int N, int oD, int oH, int nW, int kd, int kh, int K, int
   return p;
 }
 
-// The first `tall_images` of a batch in tall boxes (conv_row_tall.hip), the rest in the shape above.  A tall box takes the CU
+// The first `tall_planes` of a batch in tall boxes (conv_row_tall.hip), the rest in the shape above.  A tall box takes the CU
 // that has it 2.1 us per 16 channels and plane of taps and 10.5 beside them, so a batch is worth cutting where its last round
 // would be nearly empty: N=64 256 -> 256 channels, 56x56 has 784 boxes, three rounds and sixteen boxes; 61 images fill the
-// three and the other three images take 12 us.  The model's constants are measured ones (fp16, us, this shape alone in whole
-// rounds | a box: 512 -> 512, 28x28 157 | 78 for 32 half blocks, 256 -> 256, 56x56 175 | 44 for 16).
+// three and the other three images take 12 us.  A 3-D batch is cut within its last image (N=8 128 -> 128, 16x56x56, 756 of 784 boxes
+// hold 123 of 128 planes, 3 rounds, the other 5 planes 20 us; seven images and one were 3 rounds of 686 boxes and 37 us).  The
+// model's constants are measured ones (fp16, us, this shape alone in whole rounds | a box: 512 -> 512, 28x28 157 | 78 for 32 half
+// blocks, 256 -> 256, 56x56 175 | 44 for 16).
 RowPlan make_row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int steps) {
   RowPlan best = make_row_shape(N, oD, oH, nW, kd, kh, K, steps);
+  best.rest_n = N; best.rest_d = oD;
   if (kh != 3) return best;
   const double box_us = 2.1 * 2 * steps * kd + 10.5;
-  const long long per_group = (long long)ceil_div(oH, 4) * ceil_div(K, 128), columns = (long long)oD * nW;
-  const long long boxes = ceil_div_ll(N * columns, 32) * per_group;
+  const long long per_group = (long long)ceil_div(oH, 4) * ceil_div(K, 128), planes = (long long)N * oD;
+  const long long boxes = ceil_div_ll(planes * nW, 32) * per_group;
   const long long groups = boxes / kCus * kCus / per_group;       // groups of 32 columns in whole rounds
-  const long long cut = groups * 32 / columns;
+  long long cut = std::min(groups * 32 / nW, planes - 1);
+  if (planes - cut > oD) cut = cut / oD * oD;                     // the rest: whole images, or planes of the last one
   const double wide_groups = best.wide_groups;
-  for (const long long n : {(long long)N, std::min<long long>(cut, N - 1)}) {
+  for (const long long n : {planes, cut}) {
     if (n < 1) continue;
     RowPlan p{};
-    if (n < N) p = make_row_shape((int)(N - n), oD, oH, nW, kd, kh, K, steps);
-    const long long rounds = ceil_div_ll(ceil_div_ll(n * columns, 32) * per_group, kCus);
-    p.us += rounds * box_us + (n < N ? 2 : 0);
-    p.tall_images = (int)n;
+    const long long rest = planes - n;
+    if (rest > 0) {
+      const int rest_n = (int)ceil_div_ll(rest, oD), rest_d = rest_n > 1 ? oD : (int)rest;
+      p = make_row_shape(rest_n, rest_d, oH, nW, kd, kh, K, steps);
+      p.rest_n = rest_n; p.rest_d = rest_d;
+    }
+    const long long rounds = ceil_div_ll(ceil_div_ll(n * nW, 32) * per_group, kCus);
+    p.us += rounds * box_us + (rest > 0 ? 2 : 0);
+    p.tall_planes = (int)n;
     if (p.us < best.us) best = p;
   }
   best.wide_groups = (long long)wide_groups;
@@ -710,15 +720,18 @@ int row_conv(const wc_conv_desc* d, const void* x, int first_image, int n_images
   const int force = test_gemm_config();
   // the shapes are the whole batch's, so that the passes of a batch add in the order of the batch in one pass
   RowPlan plan = row_plan(d->N, a.oD, a.oH, a.nW, d->kernel[0], d->kernel[1], a.K, a.steps);
-  if (force >= 16 && force <= 19) { plan.shape = (RowShape)(force - 16); plan.tall_images = 0; }
-  if (force == 21 && d->kernel[1] == 3) plan.tall_images = d->N;
-  const int tall = std::min(std::max(plan.tall_images - first_image, 0), n_images);
+  if (force >= 16 && force <= 19) { plan.shape = (RowShape)(force - 16); plan.tall_planes = 0; plan.rest_n = -1; }
+  if (force == 21 && d->kernel[1] == 3) plan.tall_planes = d->N * a.oD;
+  const int tall = std::min(std::max(plan.tall_planes - first_image * a.oD, 0), n_images * a.oD);
   if (tall > 0) {
     const int rc = tall_row_conv(d, x, tall, U, bias, y, stream);
-    if (rc || tall == n_images) return rc;
-    a.x = static_cast<const unsigned char*>(x) + (long long)tall * a.D * a.H * a.W * a.C * 2;
-    a.y = static_cast<unsigned char*>(y) + (long long)tall * a.oD * a.oH * a.oW * a.K * 2;
-    a.N -= tall;
+    if (rc || tall == n_images * a.oD) return rc;
+    // the rest: the images from there on, of the first of them (the only one then) the planes from there on
+    const int images = tall / a.oD, first_d = tall - images * a.oD;
+    a.x = static_cast<const unsigned char*>(x) + (long long)images * a.D * a.H * a.W * a.C * 2;
+    a.y = static_cast<unsigned char*>(y) + (long long)tall * a.oH * a.oW * a.K * 2;
+    a.N -= images;
+    a.oD -= first_d; a.pd -= first_d;
     a.x_bytes = (int)((long long)a.N * a.D * a.H * a.W * a.C * 2);
   }
   return dispatch_dtype(d->dtype, [&](auto t) -> int {
@@ -727,7 +740,7 @@ int row_conv(const wc_conv_desc* d, const void* x, int first_image, int n_images
       auto go = [&](auto kd, auto kh) -> int {
         constexpr int KD = decltype(kd)::value, KH = decltype(kh)::value;
         RowPlan p = plan;
-        if (a.N != d->N - p.tall_images || (force >= 16 && force <= 19)) {
+        if (a.N != p.rest_n || a.oD != p.rest_d) {
           const int tiles = p.shape <= kRowHalf ? 64 : 32, slots = KH == 7 ? (tiles == 64 ? 128 : 64) : p.shape == kRowWide ? 128 : p.shape == kRowSplit ? 32 : p.shape == kRowHalf && KD > 1 ? 128 : 64;
           p.box = choose_box(a.N, a.oD, a.oH, a.nW, KD, KH, tiles, slots);
         }

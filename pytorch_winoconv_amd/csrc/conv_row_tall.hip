@@ -349,14 +349,16 @@ constexpr int kFilterInL2 = 3 << 20;
 
 }  // namespace
 
-int tall_row_conv(const wc_conv_desc* d, const void* x, int n_images, const void* U, const void* bias, void* y, void* stream) {
+// the first n_planes output planes (2-D: images) from x on
+int tall_row_conv(const wc_conv_desc* d, const void* x, int n_planes, const void* U, const void* bias, void* y, void* stream) {
   TallArgs a{};
   a.x = x; a.U = U; a.bias = bias; a.y = y;
-  a.N = n_images; a.D = d->in[0]; a.H = d->in[1]; a.W = d->in[2]; a.C = wc_padded_channels8(d->C); a.K = d->K;
+  a.D = d->in[0]; a.H = d->in[1]; a.W = d->in[2]; a.C = wc_padded_channels8(d->C); a.K = d->K;
   a.pd = d->pad[0]; a.ph = d->pad[1]; a.pw = d->pad[2]; a.kd = d->kernel[0];
   a.oD = a.D + 2 * a.pd - a.kd + 1; a.oH = a.H + 2 * a.ph - 2; a.oW = a.W + 2 * a.pw - 2;
+  a.N = ceil_div(n_planes, a.oD);
   a.nW = ceil_div(a.oW, 4);
-  a.n_col = a.N * a.oD * a.nW;
+  a.n_col = n_planes * a.nW;
   a.f_w = make_fast_div(a.nW); a.f_d = make_fast_div(a.oD);
   a.n_cg = ceil_div(a.n_col, 32); a.n_hb = ceil_div(a.oH, TB); a.n_kb = ceil_div(a.K, 128);
   a.n_box = a.n_cg * a.n_hb;

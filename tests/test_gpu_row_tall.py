@@ -47,3 +47,17 @@ def test_batch_cut_in_tall_boxes_and_others(dev, gemm_override):
     tall = _row(xd, wd, bd, 1)
     assert torch.equal(y[:61], tall[:61]) and not torch.equal(y[61:], tall[61:])
     assert torch.equal(passes, y)
+
+
+def test_batch_cut_within_the_last_image(dev, gemm_override):
+    """756 tall boxes hold 123 of 128 output planes; the other five, all of the last image, take another shape."""
+    x, w, b = _operands((8, 64, 16, 56, 56), 128, torch.float16)
+    xd, wd, bd = x.to(dev), w.to(dev), b.to(dev)
+    y = _row(xd, wd, bd, 1)
+    ref = torch.nn.functional.conv3d(x[7:, :, 9:].double(), w.double(), b.double(), padding=1)[:, :, 1:]
+    assert _err(y[7:, :, 10:], ref) <= BOUND[x.dtype]
+    passes = engine.conv_forward(xd, wd, bd, 1, 1, 2, chunk_images=3, row=True)
+    gemm_override(config=21)
+    tall = _row(xd, wd, bd, 1)
+    assert torch.equal(y[:7], tall[:7]) and torch.equal(y[7, :, :11], tall[7, :, :11]) and not torch.equal(y[7, :, 11:], tall[7, :, 11:])
+    assert torch.equal(passes, y)
