@@ -435,7 +435,7 @@ int wc_conv_backward_weight(const wc_conv_desc* d, const void* x, const void* dy
   if (L.taps) return taps_gradient(d, L.out, x, dy, dw, dw_strides, dU, stream);
   if (L.one_tap) {
     const long long P = L.tiles_per_image * d->N;
-    rc = batched_gemm_tn(dy, x, dU, 1, P, d->K, d->C, d->K, d->C, d->C, L.S, L.Pq, d->dtype, stream);
+    rc = batched_gemm_tn(dy, x, dU, 1, P, d->K, d->C, d->K, d->C, d->C, L.S, L.Pq, false, d->dtype, stream);
     if (rc) return rc;
   }
   if (L.gathered) {
@@ -506,7 +506,11 @@ int wc_conv_backward_weight(const wc_conv_desc* d, const void* x, const void* dy
     const int Pq = (int)(((P + L.S - 1) / L.S + 31) / 32 * 32);
     // dU[(t, s)] (K x C, fp32) = sum over the tiles of part s of dM[t][p][.] (x) V[t][p][.]: operands in
     // the storage type (their values already are), products summed in fp32
-    rc = batched_gemm_tn(dM, V, dU, T, P, L.ldm, L.Cp, d->K, L.ncol, L.ldc, L.S, Pq, d->dtype, stream);
+    // fp32 in three bf16 parts on 2-D plans of tile 4, whose transforms make most of the error, and which that leaves smaller
+    // (2-norm against fp64: N=16 128 -> 128, 56x56 3.5e-6 | 3.0e-6, N=4 512 -> 512, 14x14 1.5e-6 | 1.3e-6; tile 2 6.4e-7 | 7.1e-7;
+    // sums of fewer than eight tiles 7.3e-7 | 8.4e-7, of 8 to 12544 tiles 0.77 to 0.93 of it)
+    const bool split = d->ndim == 2 && L.plan.m[1] == 4 && L.plan.m[2] == 4 && P >= 8 && test_gemm_config() != 22;
+    rc = batched_gemm_tn(dM, V, dU, T, P, L.ldm, L.Cp, d->K, L.ncol, L.ldc, L.S, Pq, split, d->dtype, stream);
     if (rc) return rc;
     if (L.S > 1) {
       const long long n = (long long)d->K * L.ldc, total4 = (long long)T * n / 4;

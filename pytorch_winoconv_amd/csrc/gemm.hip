@@ -20,7 +20,7 @@
 // Plans whose pieces share one transformed input read V at a row offset per piece: gemm_kernel
 // with SHIFT walks the operand pointer piece by piece; gemm_rows_kernel serves the pieces of one
 // run (neighbours along the width) from a single operand tile that is n_run - 1 rows taller.
-#include "wc_common.h"
+#include "split_bf16.h"
 
 #include <algorithm>
 
@@ -111,27 +111,6 @@ typedef uint32_t Chunk16 __attribute__((ext_vector_type(4)));   // one 16-byte g
 // r mod 2 among 8 consecutive rows, and rows of equal r mod 4 among 16, distinct positions, which
 // is conflict-free for 128-byte and for 256-byte wide bank sets alike.
 __device__ __forceinline__ int swizzle(int r) { return (((r >> 1) ^ (r >> 3)) & 1) | (((r >> 2) & 1) << 1); }
-
-// fp32 products of the Winograd domain on the bf16 matrix cores: x = h + m + l with three bf16 numbers of 8 bits each, h the
-// upper half of x, m and l rounded to nearest, which together are x exactly, and x y = hh + hm + mh + mm + hl + lh, six of
-// the nine products.  What is left out, ml + lm + ll, is at most 2^-22 and in the root mean square 2^-26 of the product, less
-// than a rounding of fp32, and a sum of 16 products is rounded six times where eight v_mfma_f32_32x32x2_f32 round it eight.
-// 16-bit products have 16 times the rate of fp32 ones.
-struct Split { uint32_t h[2], m[2], l[2]; };
-__device__ __forceinline__ Split split_bf16(Chunk16 c) {
-  Split s;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const uint32_t a = c[2 * i], b = c[2 * i + 1];
-    s.h[i] = __builtin_amdgcn_perm(b, a, 0x07060302u);
-    const float ra = __uint_as_float(a) - __uint_as_float(a & 0xffff0000u), rb = __uint_as_float(b) - __uint_as_float(b & 0xffff0000u);
-    const Pack<bf16_t, 2> m = {{static_cast<bf16_t>(ra), static_cast<bf16_t>(rb)}};
-    s.m[i] = __builtin_bit_cast(uint32_t, m);
-    const Pack<bf16_t, 2> l = {{static_cast<bf16_t>(ra - __uint_as_float(s.m[i] << 16)), static_cast<bf16_t>(rb - __uint_as_float(s.m[i] & 0xffff0000u))}};
-    s.l[i] = __builtin_bit_cast(uint32_t, l);
-  }
-  return s;
-}
 
 template <typename T, int WM, int WN, int BK, int NWP = 2, int NWK = 2, bool SHIFT = false, bool DIRECT = false, bool CLASSES = false>
 __global__ __launch_bounds__(64 * NWP * NWK, (WM * WN <= 8 && NWP * NWK == 4 ? 2 : 1))

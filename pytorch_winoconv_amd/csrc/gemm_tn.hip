@@ -18,7 +18,7 @@
 // what fills the chip); the caller adds the parts.  Workgroup = 4 wavefronts (2 x 2), each owning
 // W x W blocks of 32 x 32.  V feeds the MFMA "A" side, so a lane ends up with 4 consecutive
 // columns of D and stores them as one 16-byte write.
-#include "wc_common.h"
+#include "split_bf16.h"
 #include "wc_transform.h"
 
 #include <algorithm>
@@ -370,8 +370,129 @@ __global__ __launch_bounds__(256, 2) void gemm_tn_dma_kernel(GemmTnArgs g) {
   }
 }
 
+// fp32 on the bf16 matrix cores, each operand in three parts (split_bf16.h): a stage of 16 rows is split on its way to LDS, three
+// planes of rows of bf16 that the transposing reads take like 16-bit rows, two stages ahead of the products in registers.
+// The caller chooses it where its error is the smaller one (see wc_conv_backward_weight).  Six products of 32x32x16 take 0.4 of the time of the eight
+// of 32x32x2 they replace, and the rest of a stage is splitting.  Whole gradients on F(4,3), us, fp32 instructions | so: N=16 128 -> 128, 56x56
+// 92 | 74, N=32 256 -> 256, 56x56 388 | 324, N=8 256 -> 256, 28x28 64 | 53, N=4 512 -> 512, 14x14 58 | 54, N=64 64 -> 64, 56x56 133 | 129.
+template <int W> constexpr int tn_split_lds() { return 2 * 2 * 3 * 16 * (W * 128 + 32); }
+
+template <int W>
+__global__ __launch_bounds__(256, 2) void gemm_tn_split_kernel(GemmTnArgs g) {
+  constexpr int BT = 64 * W, BK = 16, PITCH = BT * 2 + 32, PLANE = BK * PITCH, HALF = 3 * PLANE, STAGE = 2 * HALF;      // bytes
+  constexpr int CPR = BT / 4, RPP = 256 / CPR, NL = BK / RPP;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds_raw[];
+  const int blk = xcd_remap(blockIdx.x, g.per_xcd);
+  if (blk >= g.n_blocks) return;
+  const int tb = blk % g.tiles_b;
+  const int ta = (blk / g.tiles_b) % g.tiles_a;
+  const int ts = blk / (g.tiles_b * g.tiles_a);
+  const int s = ts % g.S, t = ts / g.S;
+  const int a0 = ta * BT, b0 = tb * BT;
+  const long long p_begin = (long long)s * g.Pq;
+  const int rows = (int)max(min(g.P - p_begin, (long long)g.Pq), 0ll);
+  const int nk = (rows + BK - 1) / BK;
+  // rows past the part's end and columns past the row's lie outside the descriptors: zeros
+  const float* const Ap = static_cast<const float*>(g.A) + ((long long)t * g.P + p_begin) * g.lda + a0;
+  const float* const Bp = static_cast<const float*>(g.B) + ((long long)t * g.P + p_begin) * g.ldb + b0;
+  const __amdgpu_buffer_rsrc_t ad = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Ap), 0, (int)max(((long long)rows * g.lda - a0) * 4, 0ll), 0x00020000);
+  const __amdgpu_buffer_rsrc_t bd = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Bp), 0, (int)max(((long long)rows * g.ldb - b0) * 4, 0ll), 0x00020000);
+
+  const int tid = threadIdx.x, lrow = tid / CPR, lcol = tid % CPR * 4;
+  const unsigned a_out = a0 + lcol < g.lda ? 0u : kOutside, b_out = b0 + lcol < g.ldb ? 0u : kOutside;
+  Chunk16 ra[2][NL], rb[2][NL];
+  auto gload = [&](auto set_c, int kt) {
+    constexpr int set = decltype(set_c)::value;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const unsigned row = kt * BK + lrow + i * RPP;
+      ra[set][i] = __builtin_amdgcn_raw_buffer_load_b128(ad, (int)(((row * (unsigned)g.lda + lcol) * 4) | a_out), 0, 0);
+      rb[set][i] = __builtin_amdgcn_raw_buffer_load_b128(bd, (int)(((row * (unsigned)g.ldb + lcol) * 4) | b_out), 0, 0);
+    }
+  };
+  auto lstore = [&](auto set_c, int buf) {
+    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int i = 0; i < NL; ++i) {
+        const Split p = split_bf16(half ? rb[decltype(set_c)::value][i] : ra[decltype(set_c)::value][i]);
+        unsigned char* const to = lds_raw + buf * STAGE + half * HALF + (lrow + i * RPP) * PITCH + lcol * 2;
+        *reinterpret_cast<u2*>(to) = u2{p.h[0], p.h[1]};
+        *reinterpret_cast<u2*>(to + PLANE) = u2{p.m[0], p.m[1]};
+        *reinterpret_cast<u2*>(to + 2 * PLANE) = u2{p.l[0], p.l[1]};
+      }
+  };
+
+  const int lane = tid & 63, wave = tid >> 6, wa = wave >> 1, wb = wave & 1, l32 = lane & 31, lhi = lane >> 5;
+  floatx16 acc[W][W];
+#pragma unroll
+  for (int i = 0; i < W; ++i)
+#pragma unroll
+    for (int j = 0; j < W; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  // as in gemm_tn_kernel
+  const int sl = lane & 15, frag = (8 * lhi + (sl >> 2)) * PITCH + ((lane >> 4) & 1) * 32 + (sl & 3) * 8;
+  const int fa = frag + wa * W * 64, fb = HALF + frag + wb * W * 64;
+
+  auto stage = [&](int kt, auto set_c) {
+    constexpr int set = decltype(set_c)::value;      // kt % 2
+    gload(set_c, kt + 2);                            // beyond the part: zeros
+    const unsigned char* const st = lds_raw + set * STAGE;
+    typedef short4v __attribute__((address_space(3))) * LdsVec;
+    auto read = [&](const unsigned char* src) {
+      const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsVec)(src));
+      const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsVec)(src + 4 * PITCH));
+      return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    short8v af[3][W], bf[3][W];
+#pragma unroll
+    for (int q : {2, 0, 1}) {
+#pragma unroll
+      for (int i = 0; i < W; ++i) af[q][i] = read(st + q * PLANE + fa + i * 64);
+#pragma unroll
+      for (int j = 0; j < W; ++j) bf[q][j] = read(st + q * PLANE + fb + j * 64);
+    }
+    static_for<0, 6>([&](auto q_c) {                 // the small products first, as in gemm_kernel
+      constexpr int q = decltype(q_c)::value, qa = q == 1 ? 2 : q == 2 || q == 4 ? 1 : 0, qb = q == 0 ? 2 : q == 2 || q == 3 ? 1 : 0;
+#pragma unroll
+      for (int i = 0; i < W; ++i)
+#pragma unroll
+        for (int j = 0; j < W; ++j) acc[i][j] = mfma16(bf[qb][j], af[qa][i], acc[i][j], bf16_t{});
+    });
+    lstore(ic<1 - set>{}, 1 - set);
+    __syncthreads();
+  };
+  gload(ic<0>{}, 0);
+  gload(ic<1>{}, 1);
+  lstore(ic<0>{}, 0);
+  __syncthreads();
+  for (int kt = 0; kt < nk; kt += 2) {               // a stage beyond the last adds zeros
+    stage(kt, ic<0>{});
+    stage(kt + 1, ic<1>{});
+  }
+
+  float* const Dt = g.D + ((long long)t * g.S + s) * g.na * g.ldd;
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    const int row = a0 + (wa * W + i) * 32 + l32;
+    if (row >= g.na) continue;
+#pragma unroll
+    for (int j = 0; j < W; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int col = b0 + (wb * W + j) * 32 + 8 * q + 4 * lhi;
+        if (col < g.ldd) {
+          floatx4 o = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+          *reinterpret_cast<floatx4*>(Dt + (long long)row * g.ldd + col) = o;
+        }
+      }
+  }
+}
+
 template <typename T, int W, bool GATHER = false>
-int launch_tn(GemmTnArgs g, int T_, void* stream) {
+int launch_tn(GemmTnArgs g, int T_, bool split, void* stream) {
   constexpr int BT = 64 * W;
   constexpr int BK = sizeof(T) == 2 ? 64 : 16;     // reduction rows per stage (64: measured 5 % faster than 32)
   constexpr size_t lds = (size_t)2 * 2 * BK * (BT + 32 / sizeof(T)) * sizeof(T);
@@ -395,6 +516,16 @@ int launch_tn(GemmTnArgs g, int T_, void* stream) {
       return WC_OK;
     }
   }
+  if constexpr (sizeof(T) == 4 && !GATHER) {
+    if (split && (g.Pq + 64ll) * std::max(g.lda, g.ldb) * 4 < (1ll << 31)) {
+      const auto fn = &gemm_tn_split_kernel<W>;
+      constexpr int split_lds = tn_split_lds<W>();
+      if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), split_lds)) return rc;
+      hipLaunchKernelGGL(fn, dim3((unsigned)(g.per_xcd * kXcds)), dim3(256), split_lds, as_stream(stream), g);
+      WC_CHECK_LAUNCH("gemm_tn_split_kernel");
+      return WC_OK;
+    }
+  }
   if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_tn_kernel<T, W, BK, GATHER>), lds)) return rc;
   hipLaunchKernelGGL((gemm_tn_kernel<T, W, BK, GATHER>), dim3((unsigned)(g.per_xcd * kXcds)), dim3(256), lds, as_stream(stream), g);
   WC_CHECK_LAUNCH("gemm_tn_kernel");
@@ -404,7 +535,7 @@ int launch_tn(GemmTnArgs g, int T_, void* stream) {
 }  // namespace
 
 int batched_gemm_tn(const void* A, const void* B, float* D, int T_, long long P, int lda, int ldb, int na, int nb,
-                    int ldd, int S, int Pq, int dtype, void* stream) {
+                    int ldd, int S, int Pq, bool split, int dtype, void* stream) {
   WC_CHECK_ARG(A && B && D, "batched_gemm_tn: null pointer");
   WC_CHECK_ARG(T_ > 0 && P > 0 && na > 0 && nb > 0 && S > 0 && Pq > 0, "batched_gemm_tn: empty problem");
   WC_CHECK_ARG(lda % 8 == 0 && ldb % 8 == 0 && ldd % 4 == 0 && lda >= na && ldb >= nb && ldd >= nb,
@@ -419,7 +550,7 @@ int batched_gemm_tn(const void* A, const void* B, float* D, int T_, long long P,
   const bool big = na > 64 && nb > 64;
   return dispatch_dtype(dtype, [&](auto t) {
     using TT = decltype(t);
-    return big ? launch_tn<TT, 2>(g, T_, stream) : launch_tn<TT, 1>(g, T_, stream);
+    return big ? launch_tn<TT, 2>(g, T_, split, stream) : launch_tn<TT, 1>(g, T_, split, stream);
   });
 }
 
@@ -444,7 +575,7 @@ int gemm_tn_conv(const void* dy, const void* x, float* D, int N, int H, int W, i
   const bool big = K > 64 && C > 64;
   return dispatch_dtype(dtype, [&](auto t) {
     using TT = decltype(t);
-    return big ? launch_tn<TT, 2, true>(g, kh * kw, stream) : launch_tn<TT, 1, true>(g, kh * kw, stream);
+    return big ? launch_tn<TT, 2, true>(g, kh * kw, false, stream) : launch_tn<TT, 1, true>(g, kh * kw, false, stream);
   });
 }
 

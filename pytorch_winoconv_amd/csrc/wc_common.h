@@ -221,9 +221,10 @@ int grad_filter_transform(const wc_conv_desc* d, const wc_plan* plan, const floa
                           bool first, void* stream);
 
 // D[t][s] (na x nb, fp32, row stride ldd) = sum over rows p in [s Pq, (s + 1) Pq) of
-// A[t][p][.] (x) B[t][p][.], operands (T, P, ld) of storage type `dtype` (gemm_tn.hip).
+// A[t][p][.] (x) B[t][p][.], operands (T, P, ld) of storage type `dtype`; split: fp32 in
+// three bf16 parts (gemm_tn.hip).
 int batched_gemm_tn(const void* A, const void* B, float* D, int T, long long P, int lda, int ldb, int na, int nb,
-                    int ldd, int S, int Pq, int dtype, void* stream);
+                    int ldd, int S, int Pq, bool split, int dtype, void* stream);
 // The weight gradient of a 2-D convolution taken directly: dW[(ky, kx)][s] (K x C) = sum over the output pixels of
 // part s of dy (x) the pixel of x that tap reads (gemm_tn.hip)
 int gemm_tn_conv(const void* dy, const void* x, float* D, int N, int H, int W, int C, int K, int kh, int kw, int stride,
