@@ -53,3 +53,16 @@ def test_where_the_register_staged_kernel_takes_over(dev, dtype, gemm_override):
     dy = torch.randint(-3, 4, tuple(y.shape), generator=g).double()
     dx = engine.conv_backward_input(dy.to(dtype).to(dev), w.to(dtype).to(dev), (11, 13), 2, 1, 2)
     assert torch.equal(dx.cpu(), torch.nn.grad.conv2d_input((2, 32, 11, 13), w, dy, 2, 1).float().to(dtype))
+
+
+@pytest.mark.parametrize("n,c,k,h,direct", [(1, 480, 64, 7, 1), (2, 384, 136, 9, 1), (1, 352, 32, 14, 1), (2, 384, 64, 9, 0)])
+def test_reductions_that_left_the_parity_phases(dev, n, c, k, h, direct):
+    """3x3 kernels at stride 2 over 356 to 500 channels, chosen by the library (but for fp32, the last): exact on small integers
+    where no transform is taken."""
+    dtype = torch.float16 if direct else torch.float32
+    assert engine.make_desc((n, c, h, h), (k, c, 3, 3), dtype, 2, 1, 2, stacked=None).direct == direct
+    g = torch.Generator().manual_seed(6)
+    x, w = torch.randint(-3, 4, (n, c, h, h), generator=g).double(), torch.randint(-2, 3, (k, c, 3, 3), generator=g).double()
+    y = engine.conv_forward(x.to(dtype).to(dev), w.to(dtype).to(dev), None, 2, 1, 2)
+    want = F.conv2d(x, w, None, 2, 1)
+    assert torch.equal(y.cpu(), want.float().to(dtype)) if direct else float((y.cpu() - want).abs().max()) <= 2e-4 * float(want.abs().max())
