@@ -1,8 +1,8 @@
-// Direct form with ONE operand tile per kernel row (16-bit types, kernel rows of 4 to 8 taps).
+// Direct form with ONE operand tile per kernel row (16-bit types, kernel rows of 4 to 8 taps; where it is taken: gemm_direct_conv,
+// gemm.hip).
 //
-// gemm_kernel<..., DIRECT> (gemm.hip) loads, for every tap, its own tile of 256 pixels x 32 channels of x: the taps of
-// one kernel row read nearly the same pixels, and the rate at which a CU can pull operands in is what bounds that
-// kernel (c4 7x7 at stride 2: x fetched 5.75 times from beyond L2).  Here a workgroup owns 256 consecutive output
+// A tile per tap (direct_dma.hip) loads, for every tap, its own tile of 256 pixels x 32 channels of x: the taps of
+// one kernel row read nearly the same pixels, and the rate at which a CU can pull operands in bounds that kernel.  Here a workgroup owns 256 consecutive output
 // pixels x 128 output channels (four wavefronts of 128 x 64, one workgroup per CU), and for every group (kernel row
 // ky, block of 32 channels) the input rows those pixels read are brought to LDS ONCE, with their zero padding, and
 // serve all KW taps of the row: tap kx of output pixel (oy, ox) is pixel stride ox + kx of the slot of row oy.  Only
