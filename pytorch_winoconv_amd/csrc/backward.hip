@@ -272,6 +272,24 @@ int pick_parts(long long tiles, long long rows, bool big_tiles) {
   return (int)best;
 }
 
+// The same for gradients of 16-bit types taken directly (gemm_tn_dma_kernel): a CU takes 0.31 us for each 32 rows of each of its
+// workgroups, 0.45 where it has one (64 x 64 tiles 0.25 | 0.15 | 0.125 | 0.11 with one, two, three, more), and every part's `sums`
+// values are written and read back.
+// us over parts, fp16: 3x3 at stride 2 N=32 128 -> 256, 56x56 28: 33.6, 14: 36.9, 64: 51.8; N=32 128 -> 128, 112x112 56: 49, 28: 60; N=16 96 -> 96, 50x50
+// 39: 17.7, 28: 15.3, 24: 15.2; 1x1 N=64 512 -> 512, 14x14 32: 25, 16: 21.9, 14: 21.3; N=8 64 -> 128, 56x56 24: 13.2, 14: 12.0.
+int pick_direct_parts(long long tiles, long long rows, long long sums, bool big_tiles) {
+  const long long most = std::max(1ll, std::min(64ll, rows / 256));
+  long long best = 1;
+  double best_us = 1e30;
+  for (long long S = 1; S <= most; ++S) {
+    const long long per_cu = (tiles * S + 255) / 256;
+    const double stage = big_tiles ? (per_cu > 1 ? 0.31 : 0.45) : per_cu > 3 ? 0.11 : per_cu == 3 ? 0.125 : per_cu == 2 ? 0.15 : 0.25;
+    const double us = per_cu * ((rows + 32 * S - 1) / (32 * S)) * stage + S * sums * 8 / 5e6;
+    if (us < best_us * (1.0 - 1e-9)) { best = S; best_us = us; }
+  }
+  return (int)best;
+}
+
 struct BwdLayout {
   wc_plan plan;
   int out[3], grid[3];
@@ -305,7 +323,8 @@ bool gathered_layout(const wc_conv_desc* d, BwdLayout* L) {
   L->tiles_per_image = (long long)L->out[1] * L->out[2];
   const int bt = (d->K > 64 && d->C > 64) ? 128 : 64;
   const long long tiles = (long long)taps * ((d->K + bt - 1) / bt) * ((d->C + bt - 1) / bt);
-  const long long S = pick_parts(tiles, P, bt == 128);
+  const long long S = d->dtype == WC_F32 ? pick_parts(tiles, P, bt == 128)
+                                           : pick_direct_parts(tiles, P, (long long)d->kernel[1] * d->kernel[2] * d->K * d->C, bt == 128);
   L->S = (int)S;
   L->Pq = (int)(((P + S - 1) / S + 31) / 32 * 32);
   L->v_bytes = L->dm_bytes = 0;
@@ -330,7 +349,8 @@ bool one_tap_layout(const wc_conv_desc* d, BwdLayout* L) {
   L->tiles_per_image = (long long)d->in[1] * d->in[2];
   const int bt = (d->K > 64 && d->C > 64) ? 128 : 64;
   const long long tiles = (long long)((d->K + bt - 1) / bt) * ((d->C + bt - 1) / bt);
-  const long long S = pick_parts(tiles, P, bt == 128);
+  const long long S = d->dtype == WC_F32 ? pick_parts(tiles, P, bt == 128)
+                                           : pick_direct_parts(tiles, P, (long long)d->kernel[1] * d->kernel[2] * d->K * d->C, bt == 128);
   L->S = (int)S;
   L->Pq = (int)(((P + S - 1) / S + 31) / 32 * 32);
   L->v_bytes = L->dm_bytes = L->acc_bytes = 0;
