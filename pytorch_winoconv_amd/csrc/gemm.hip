@@ -932,7 +932,7 @@ int fold_filter_w(const void* U, void* Uw, int K, int Cp, int dtype, void* strea
 }
 
 // Tiles of the direct form: fp32 products are bound by the MFMA rate and fill the chip best with small tiles (as in choose()).
-// 16-bit types come here only where direct_dma.hip does not reach (direct_dma_fits).
+// 16-bit types come here only where direct_dma.hip does not reach (direct_dma_fits, 16-byte alignment).
 template <typename T>
 static GemmConfig choose_direct(int P, int K) {
   constexpr int BK = sizeof(T) == 4 ? 16 : 32;
@@ -962,7 +962,9 @@ int gemm_direct_conv(const void* x, const void* U, const void* bias, void* y, in
   // tiles) 83 | 68, N=13 (160) 85 | 95, N=16 91 | 97, N=20 103 | 110, N=26 177 | 160, N=32 182 | 178, N=64 365 | 356; 5x5 N=10 54 | 39,
   // N=16 57 | 55, N=32 117 | 99, 256 -> 512 on 28x28 N=64 (196 tiles) 103 | 109; 6x6 256 channels on 56x56 N=32 136 | 147, 4x4 72 | 71.
   // wc_test_gemm_override(., 2) takes it wherever it fits, (., 0) never.
-  if (direct_rows_fits(N, C, K, kw, stride, oH, oW, dtype)) {
+  // LDS-DMA takes 16 bytes from multiples of 16: tensors that start elsewhere go through registers
+  const bool aligned = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(U)) & 15) == 0;
+  if (aligned && direct_rows_fits(N, C, K, kw, stride, oH, oW, dtype)) {
     const int mode = test_gemm_rows();
     const long long tiles = ceil_div_ll(P, 256) * ceil_div(K, 128);
     const bool k_fills = K % 128 == 0 || K % 128 >= 96;      // the last 128-channel tile is at least three quarters full
@@ -972,7 +974,7 @@ int gemm_direct_conv(const void* x, const void* U, const void* bias, void* y, in
                               o_x0, o_H, o_W);
   }
   const DirectClass whole{U, kh, kw, pad_h, pad_w, oH, oW, o_y0, o_x0};
-  if (dtype != WC_F32 && test_gemm_config() != 0 && direct_dma_fits(&whole, 1, H, W, C, K, stride))
+  if (dtype != WC_F32 && aligned && test_gemm_config() != 0 && direct_dma_fits(&whole, 1, H, W, C, K, stride))
     return direct_dma(x, &whole, 1, bias, y, N, H, W, C, K, stride, dtype, stream, o_step, o_H, o_W);
   GemmConfig c = dispatch_dtype(dtype, [&](auto t) { return choose_direct<decltype(t)>((int)P, K); });
   GemmArgs g;
@@ -1007,7 +1009,9 @@ int gemm_direct_classes(const void* x, const DirectClass* classes, int n, void* 
   const int cq = dtype == WC_F32 ? 16 : 32;
   WC_CHECK_ARG(C > 0 && C % cq == 0 && K > 0 && K % 8 == 0, "gemm_direct_classes: C %d (multiple of %d), K %d (multiple of 8)", C, cq, K);
   if (dtype != WC_F32) {
-    if (test_gemm_config() != 0 && direct_dma_fits(classes, n, H, W, C, K, 1))
+    bool aligned = (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+    for (int i = 0; i < n; ++i) aligned = aligned && (reinterpret_cast<uintptr_t>(classes[i].U) & 15) == 0;
+    if (aligned && test_gemm_config() != 0 && direct_dma_fits(classes, n, H, W, C, K, 1))
       return direct_dma(x, classes, n, nullptr, y, N, H, W, C, K, 1, dtype, stream, 2, o_H, o_W);
     for (int i = 0; i < n; ++i) {
       const DirectClass& c = classes[i];

@@ -66,3 +66,25 @@ def test_reductions_that_left_the_parity_phases(dev, n, c, k, h, direct):
     y = engine.conv_forward(x.to(dtype).to(dev), w.to(dtype).to(dev), None, 2, 1, 2)
     want = F.conv2d(x, w, None, 2, 1)
     assert torch.equal(y.cpu(), want.float().to(dtype)) if direct else float((y.cpu() - want).abs().max()) <= 2e-4 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("shift", [1, 2, 4])
+def test_tensors_that_start_anywhere(dev, shift):
+    """x, dy and U that start 2, 4 or 8 bytes past a multiple of 16: through registers."""
+    g = torch.Generator().manual_seed(8)
+    x, w = torch.randint(-3, 4, (2, 64, 9, 11), generator=g).double(), torch.randint(-2, 3, (64, 64, 3, 3), generator=g).double()
+    want = F.conv2d(x, w, None, 2, 1)
+    dy = torch.randint(-3, 4, tuple(want.shape), generator=g).double()
+
+    def moved(t):
+        return torch.empty(t.numel() + 8, dtype=torch.float16, device=dev)[shift:shift + t.numel()].view(t.shape).copy_(t)
+
+    def view(t):
+        return moved(t.movedim(1, -1)).movedim(-1, 1)
+
+    wd = w.half().to(dev)
+    U = engine.transform_filter(wd, (2, 64, 9, 11), 2, 1, 2, direct=True)
+    assert torch.equal(engine.conv_forward(view(x), wd, None, 2, 1, 2, U=U, direct=True).cpu(), want.half())
+    assert torch.equal(engine.conv_forward(x.half().to(dev), wd, None, 2, 1, 2, U=moved(U), direct=True).cpu(), want.half())
+    dx = engine.conv_backward_input(view(dy), wd, (9, 11), 2, 1, 2)
+    assert torch.equal(dx.cpu(), torch.nn.grad.conv2d_input((2, 64, 9, 11), w, dy, 2, 1).half())
