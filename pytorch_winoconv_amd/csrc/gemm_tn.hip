@@ -473,6 +473,30 @@ __global__ __launch_bounds__(256, 2) void gemm_tn_split_kernel(GemmTnArgs g) {
     stage(kt + 1, ic<1>{});
   }
 
+  // sums that an infinity has made no number, again on the fp32 instructions (as in gemm_kernel)
+#pragma unroll
+  for (int i = 0; i < W; ++i)
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
+      bool number = true;
+#pragma unroll
+      for (int e = 0; e < 16; e += 2) number = number && !__builtin_isunordered(acc[i][j][e], acc[i][j][e + 1]);
+      if (__all(number)) continue;
+      const int ca = (wa * W + i) * 32 + l32, cb = (wb * W + j) * 32 + l32;
+      const unsigned oa = a0 + ca < g.lda ? 0u : kOutside, ob = b0 + cb < g.ldb ? 0u : kOutside;
+      floatx16 again = {};
+#pragma unroll 4
+      for (int row = 0; row < rows; row += 2) {        // a row beyond the part: zeros
+        const unsigned r = row + lhi;
+        const uint32_t av = __builtin_amdgcn_raw_buffer_load_b32(ad, (int)(((r * (unsigned)g.lda + ca) * 4) | oa), 0, 0);
+        const uint32_t bv = __builtin_amdgcn_raw_buffer_load_b32(bd, (int)(((r * (unsigned)g.ldb + cb) * 4) | ob), 0, 0);
+        again = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(bv), __uint_as_float(av), again, 0, 0, 0);
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (acc[i][j][e] != acc[i][j][e]) acc[i][j][e] = again[e];
+    }
+
   float* const Dt = g.D + ((long long)t * g.S + s) * g.na * g.ldd;
 #pragma unroll
   for (int i = 0; i < W; ++i) {

@@ -4,7 +4,9 @@ Bound: what is left out is at most 2^-22 of a product; the sum is rounded (2^-24
 six times per 16 channels, twice that allowed for what an instruction rounds inside."""
 import pytest
 import torch
+import torch.nn.functional as F
 
+import pytorch_winoconv_amd as pkg
 from pytorch_winoconv_amd import engine
 
 pytestmark = pytest.mark.gpu
@@ -44,3 +46,58 @@ def test_infinities_and_nan_stay_in_their_rows(dev):
         assert not bool(torch.isfinite(got[1, 33]).any())
         got[1, 33] = M[1, 33]
         assert torch.equal(got, M)
+
+
+@pytest.mark.parametrize("config", [-1, 0, 1, 2, 3, 4])
+@pytest.mark.parametrize("value", [float("inf"), -float("inf")])
+def test_an_infinity_keeps_its_sign(dev, value, config, gemm_override):
+    """In either operand, against numbers with and without lower parts and against zero (no number then); every other sum
+    keeps its bits."""
+    g = torch.Generator().manual_seed(3)
+    V, U = torch.randn(2, 150, 64, generator=g).to(dev), torch.randn(2, 136, 64, generator=g).to(dev)
+    U[1, ::3, 17], U[1, 5, 17], V[0, ::3, 3], V[0, 149, 3] = -1.0, 0.0, 3.0, 0.0
+    gemm_override(config=config)
+    M = engine.batched_gemm(V, U)
+    W = V.clone()
+    W[1, 133, 17] = value
+    got = engine.batched_gemm(W, U)
+    assert torch.equal(torch.nan_to_num(got[1, 133], 7.0), torch.nan_to_num(value * U[1, :, 17], 7.0))
+    got[1, 133] = M[1, 133]
+    assert torch.equal(got, M)
+    W = U.clone()
+    W[0, 40, 3] = value
+    got = engine.batched_gemm(V, W)
+    assert torch.equal(torch.nan_to_num(got[0, :, 40], 7.0), torch.nan_to_num(value * V[0, :, 3], 7.0))
+    got[0, :, 40] = M[0, :, 40]
+    assert torch.equal(got, M)
+
+
+@pytest.mark.parametrize("nd,C,K,stride", [(2, 20, 100, 1), (2, 20, 100, 2), (2, 64, 100, 1), (3, 20, 36, 1), (3, 32, 40, 1)])
+def test_an_infinity_goes_through_layers_of_one_tap(dev, nd, C, K, stride):
+    """A tile of one tap has nothing to transform: y, dx and dw are infinite where a plain sum is, with its sign."""
+    g = torch.Generator().manual_seed(5)
+    size = (9, 8, 7)[:nd]
+    x, w = torch.randn(2, C, *size, generator=g), torch.randn(K, C, *[1] * nd, generator=g)
+    x[(1, 7) + (4,) * nd], x[(0, 3) + (2,) * nd] = float("inf"), -float("inf")
+    layer = (pkg.WinoConv2d if nd == 2 else pkg.WinoConv3d)(C, K, 1, stride=stride, bias=False, device=dev)
+    with torch.no_grad():
+        layer.weight.copy_(w)
+    conv = F.conv2d if nd == 2 else F.conv3d
+
+    def check(got, want):
+        assert not bool(torch.isfinite(want).all())
+        got, finite = got.detach().double().cpu(), torch.isfinite(want)
+        assert torch.equal(got[~finite], want[~finite])
+        if nd == 3 and got.shape[-1] > 1:       # outputs of a pair along the width meet in a product with zero
+            finite = finite & finite[..., (torch.arange(got.shape[-1]) ^ 1).clamp(max=got.shape[-1] - 1)]
+        assert bool(((got - want)[finite].abs() <= 1e-5 * want[finite].abs().max()).all())
+
+    xd = x.to(dev).requires_grad_(True)
+    y = layer(xd)
+    xr, wr = x.double().requires_grad_(True), w.double().requires_grad_(True)
+    yr = conv(xr, wr, stride=stride)
+    check(y, yr.detach())
+    dy = torch.randn(y.shape, generator=g)
+    check(torch.autograd.grad(y, layer.weight, dy.to(dev))[0], torch.autograd.grad(yr, wr, dy.double(), retain_graph=True)[0])
+    dy[(1, 11) + (1,) * nd] = float("inf")
+    check(torch.autograd.grad(layer(xd), xd, dy.to(dev))[0], torch.autograd.grad(yr, xr, dy.double())[0])
