@@ -66,7 +66,7 @@ __device__ __forceinline__ int lane_id() {
   return l;
 }
 
-// KT: rows of y that are no multiple of 16 bytes
+// KT: rows of y that are no multiple of 16 bytes, or a y or bias that starts elsewhere than at one (a view into another tensor)
 template <typename T, int UR, bool KT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void tall_row_kernel(TallArgs a) {
@@ -367,7 +367,7 @@ int tall_row_conv(const wc_conv_desc* d, const void* x, int n_planes, const void
   a.u_bytes = (int)(row_u_elems(d) * 2);
   a.box_fast = a.u_bytes > kFilterInL2;
   a.per_xcd = ceil_div(a.n_kb * a.n_box, kXcds);
-  const bool whole = a.K % 8 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
+  const bool whole = a.K % 8 == 0 && ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(bias)) & 15) == 0;
   // one workgroup per CU, and at most one per box
   const int grid = std::min(a.per_xcd * kXcds, kCus);
   return dispatch_dtype(d->dtype, [&](auto t) -> int {

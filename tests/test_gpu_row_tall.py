@@ -61,3 +61,20 @@ def test_batch_cut_within_the_last_image(dev, gemm_override):
     tall = _row(xd, wd, bd, 1)
     assert torch.equal(y[:7], tall[:7]) and torch.equal(y[7, :, :11], tall[7, :, :11]) and not torch.equal(y[7, :, 11:], tall[7, :, 11:])
     assert torch.equal(passes, y)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("xs,K", [((3, 40, 9, 30), 136), ((2, 32, 3, 5, 18), 64)])
+def test_bias_that_starts_anywhere(dev, dtype, xs, K, gemm_override, host_layer):
+    """A bias that is a view into a flat buffer gives the bits of an aligned one: the same values are added."""
+    x, w, b = _operands(xs, K, dtype)
+    xd, wd, bd = x.to(dev), w.to(dev), b.to(dev)
+    gemm_override(config=21)
+    want = _row(xd, wd, bd, 1)
+    assert _err(want, _conv64(x, w, b, 1)) <= BOUND[dtype]
+    layer = engine.conv_forward(xd, wd, bd, 1, 1, 2, row=True)
+    for first in (1, 2, 3, 4, 7):
+        view = torch.full((K + 16,), float("nan"), dtype=dtype, device=dev)[first:first + K].copy_(bd)
+        assert view.data_ptr() % 16 == 2 * first
+        assert torch.equal(_row(xd, wd, view, 1), want)
+        assert torch.equal(engine.conv_forward(xd, wd, view, 1, 1, 2, row=True), layer)
