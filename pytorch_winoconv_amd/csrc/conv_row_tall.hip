@@ -163,7 +163,6 @@ void tall_row_kernel(TallArgs a) {
 #pragma unroll
       for (int r = 0; r < 3; ++r) load_u(g, u_base, g / 3, g % 3, r);
   };
-  fill_u();
 
   // the first half block; the first one of every later box is transformed beside the last products of the box before
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -251,6 +250,12 @@ void tall_row_kernel(TallArgs a) {
       u_base = u_next; rd = x_rd; cb = x_cb;
       if (last) break;
     }
+    // A box's last fragments are loaded for nothing, but the waits for x have counted them (TallBeside::after_loads): they are
+    // used here, so that they stay.  (The bias, whose registers they have, waits for them anyway.)
+#pragma unroll
+    for (int g = 0; g < UR; ++g)
+#pragma unroll
+      for (int r = 0; r < 3; ++r) asm volatile("" :: "v"(uf[g][r]));
 
     // ---- output transform: elements 0 to 2 (points 0, a, -a) are with the first four wavefronts, 3 to 5 (1/a, -1/a, infinity)
     // with the others; each half finishes two of the four rows and hands three sums of the other two over through LDS
