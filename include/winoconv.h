@@ -163,7 +163,8 @@ const char* wc_last_error(void);
  * config 16 to 19: the row form with the wide, half, small or split workgroups whatever the problem (conv_row.hip).
  * config 21: the row form on tall boxes whatever the problem (conv_row_tall.hip).
  * config 22 to 26: the direct form of 16-bit types on tiles of 256 x 128, 128 x 128, 256 x 64, 128 x 64 or 64 x 64 whatever the
- * problem (direct_dma.hip); 22 also: fp32 weight gradients on the fp32 instructions.  config 0: the direct form of 16-bit
+ * problem (direct_dma.hip); 22 also: fp32 products and weight gradients on the fp32 instructions.
+ * config 0 to 4 in fp32: the tiles of the product in three bf16 parts.  config 0: the direct form of 16-bit
  * types through registers (gemm.hip).
  * Works only in a process started with WINOCONV_TEST_HOOKS=1 in its environment (WC_ERR_UNSUPPORTED
  * otherwise, and nothing changes); what it sets holds for the calling host thread only, so a caller
@@ -238,7 +239,9 @@ int wc_input_transform(const wc_conv_desc* desc, const wc_plan* plan,
                        const void* x, int n_images, void* V, void* stream);
 /* M[t] (P x K) = V[t] (P x Cp) . U[t]^T for t in [0, T).  Replaces forwardAssign +
  * cublas{S,H}gemmBatched (src/utils.cu:5-12, src/base_conv_launchers.cu:353-367,
- * src/base_conv_launchers_half.cu:231-236).  fp16 accumulates in fp32. */
+ * src/base_conv_launchers_half.cu:231-236).  fp16 accumulates in fp32; fp32 takes three bf16 parts of each
+ * operand for T >= 16 and 64 <= Cp <= 1024 (T < 36: 512), where whole layers come out more exact so, and the fp32 instructions elsewhere;
+ * wc_conv_forward takes these for kernels of one tap as well. */
 int wc_batched_gemm(const void* V, const void* U, void* M, int T, int P, int Cp, int K, int ldm,
                     int dtype, void* stream);
 /* y = sum over pieces of (AT x AT x AT) m, + bias, cropped.  Replaces outputWino2NormTransform +

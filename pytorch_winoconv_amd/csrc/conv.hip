@@ -358,7 +358,7 @@ int forward_impl(const wc_conv_desc* d, const void* x, const void* w, const int6
       rc = timer.run(WC_STAGE_PRODUCT, [&] {
         if (L.fold) return batched_gemm_shifted(V, Ufold, M, 16, (int)P, L.Cp, L.fold_shift, d->K, L.ldm, d->dtype, stream);
         return L.shared ? batched_gemm_shifted(V, U, M, L.plan.t_total, (int)P, L.vrow, L.shift, d->K, L.ldm, d->dtype, stream)
-                        : wc_batched_gemm(V, U, M, L.plan.t_total, (int)P, L.Cp, d->K, L.ldm, d->dtype, stream);
+                        : batched_gemm(V, U, M, L.plan.t_total, (int)P, L.Cp, d->K, L.ldm, d->kernel[0] * d->kernel[1] * d->kernel[2] > 1, d->dtype, stream);
       });
       if (rc) return rc;
       rc = timer.run(WC_STAGE_OUTPUT, [&] {

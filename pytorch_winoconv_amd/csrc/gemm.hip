@@ -14,8 +14,8 @@
 // conflicts.  The MFMA "A" operand is the
 // filter block and "B" the input block: a lane then holds 4 consecutive output channels of
 // one tile row per accumulator group and stores them as one 8-byte (fp16) / 16-byte (fp32)
-// write.  fp16 and bf16 accumulate in fp32; fp32 uses three bf16 parts per operand (Split), its direct form
-// v_mfma_f32_32x32x2_f32.
+// write.  fp16 and bf16 accumulate in fp32; fp32 uses v_mfma_f32_32x32x2_f32, or three bf16 parts per operand (Split) where
+// the caller finds their error the smaller one.
 //
 // Plans whose pieces share one transformed input read V at a row offset per piece: gemm_kernel
 // with SHIFT walks the operand pointer piece by piece; gemm_rows_kernel serves the pieces of one
@@ -112,10 +112,12 @@ typedef uint32_t Chunk16 __attribute__((ext_vector_type(4)));   // one 16-byte g
 // is conflict-free for 128-byte and for 256-byte wide bank sets alike.
 __device__ __forceinline__ int swizzle(int r) { return (((r >> 1) ^ (r >> 3)) & 1) | (((r >> 2) & 1) << 1); }
 
-template <typename T, int WM, int WN, int BK, int NWP = 2, int NWK = 2, bool SHIFT = false, bool DIRECT = false, bool CLASSES = false>
+// SPLIT: fp32 in three bf16 parts (split_bf16.h)
+template <typename T, int WM, int WN, int BK, int NWP = 2, int NWK = 2, bool SHIFT = false, bool DIRECT = false, bool CLASSES = false, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NWP * NWK, (WM * WN <= 8 && NWP * NWK == 4 ? 2 : 1))
 void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
   static_assert((!DIRECT || SHIFT) && (!CLASSES || DIRECT), "the direct form walks the taps like the shifted operand");
+  static_assert(!SPLIT || (sizeof(T) == 4 && !SHIFT), "fp32 of the plain product");
   GemmArgs g = args;
   using MF = Mfma<T>;
   constexpr int NT = 64 * NWP * NWK;               // threads: NWP x NWK wavefronts
@@ -126,7 +128,6 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
   constexpr int ROWS = BM + BN;
   constexpr int RPP = NT / CPR;                    // rows covered by one pass of the workgroup
   constexpr int NLOAD = ROWS / RPP;
-  constexpr bool SPLIT = sizeof(T) == 4 && !DIRECT;
   constexpr int PLANE = ROWS * 32;                 // SPLIT: bytes of one of the three parts of a stage, rows of 16 bf16
   constexpr int STAGE = SPLIT ? 3 * PLANE / 4 : ROWS * LDS_STRIDE;         // elements per LDS stage
   static_assert(ROWS % RPP == 0 && BM % RPP == 0, "tile rows must be a multiple of the load pass");
@@ -370,7 +371,6 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
   // instructions, operands from memory, which leave an infinity with its sign where there is one; all other sums keep their bits.  (Looking for them costs N=8
   // 256 -> 256, 56x56 0.6 of 86 us.)
   if constexpr (SPLIT) {
-    static_assert(!SHIFT, "row p of V is at p Cp");
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -460,14 +460,14 @@ struct GemmConfig {
   int threads;
 };
 
-template <typename T, int WM, int WN, int BK, int NWP = 2, int NWK = 2, bool SHIFT = false, bool DIRECT = false>
+template <typename T, int WM, int WN, int BK, int NWP = 2, int NWK = 2, bool SHIFT = false, bool DIRECT = false, bool SPLIT = false>
 static GemmConfig make_config() {
   constexpr int EPC = 16 / sizeof(T);
   constexpr int BM = 32 * NWP * WM, BN = 32 * NWK * WN;
   constexpr int EI = sizeof(T) == 4 ? 1 : (NWP * NWK == 4 ? WM : WM / 2);
-  constexpr size_t stages = (size_t)2 * (BM + BN) * (sizeof(T) == 4 && !DIRECT ? 96 : BK * sizeof(T));
+  constexpr size_t stages = (size_t)2 * (BM + BN) * (SPLIT ? 96 : BK * sizeof(T));
   constexpr size_t out_tile = (size_t)32 * NWP * EI * (BN + EPC) * sizeof(T);
-  return GemmConfig{&gemm_kernel<T, WM, WN, BK, NWP, NWK, SHIFT, DIRECT>, BM, BN, BK,
+  return GemmConfig{&gemm_kernel<T, WM, WN, BK, NWP, NWK, SHIFT, DIRECT, false, SPLIT>, BM, BN, BK,
                     stages > out_tile ? stages : out_tile, 64 * NWP * NWK};
 }
 
@@ -746,18 +746,43 @@ template <> struct Configs<bf16_t> {
     }
   }
 };
-template <> struct Configs<float> {
+template <> struct Configs<float> {              // in three bf16 parts
   static constexpr int n = 5;
+  template <int WM, int WN> static GemmConfig split() { return make_config<float, WM, WN, 16, 2, 2, false, false, true>(); }
   static GemmConfig get(int i) {
     switch (i) {
-      case 0: return make_config<float, 4, 2, 16>();
-      case 1: return make_config<float, 2, 2, 16>();
-      case 2: return make_config<float, 4, 1, 16>();
-      case 3: return make_config<float, 2, 1, 16>();
-      default: return make_config<float, 1, 1, 16>();
+      case 0: return split<4, 2>();
+      case 1: return split<2, 2>();
+      case 2: return split<4, 1>();
+      case 3: return split<2, 1>();
+      default: return split<1, 1>();
     }
   }
 };
+
+// Whether a product of fp32 is taken in three bf16 parts (split_bf16.h): where the error of a layer against fp64 is no larger than on the
+// fp32 instructions, as far as T and the reduction tell.  2-norm of that error, parts over fp32, for normal x and w | x cut off at zero, as
+// behind a ReLU | x and w without negative values, whose sums the bf16 instructions cut off on one side:
+//   T=36, 3x3 and tile 4: 66 channels 0.89 | 0.87 | 0.86, 256 0.83 | 0.86 | 0.85, 1024 0.85 | 0.86 | 0.81, 2048 0.86 | 0.86 | 1.07, 3072 0.85 | 0.87 | 2.7;
+//   four pieces in one sum, 5x5: 4 x 256 0.86 | 0.86 | 0.92, 4 x 512 0.88 | 0.90 | 2.1; 3x3 at stride 2: 4 x 132 0.86 | 0.93 | 0.80, 4 x 512 0.92 | 0.90 | 1.6
+//   T=64, 3x3x3: 64 channels 0.82 | 0.82 | 0.74, 256 0.84 | 0.85 | 0.80
+//   T=16, 3x3 and tile 2: 66 0.88 | 0.90 | 0.83, 1024 0.86 | 0.89 | 0.82; 5x5: 4 x 64 0.84 | 0.88 | 0.82, 4 x 256 0.87 | 0.90 | 0.99; 3x3 at stride 2, whose
+//   phases have axes of one tap: 4 x 256 0.86 | 1.08 | 1.17, 4 x 512 0.90 | 1.07 | 2.3
+//   T=4, phases of one tap: 4 x 64 0.83 | 1.14 | 0.84; kernels of one tap at any T: 100 channels 0.83 | 1.11 | 0.83
+//   1, 2, 3, 4 channels, which are padded to 32: 3x3 and tile 4 1.15, 1.09, 1.02, 1.03.  (In plans that add up pieces these are part of longer
+//   reductions, and lose: 5x5 1.35, 1.23, -, 1.07, 8 channels 0.87 again.)
+static bool fp32_in_parts(int T_, int Cp, bool transformed) {
+  const int force = test_gemm_config();
+  if (force >= 0 && force < Configs<float>::n) return true;
+  return transformed && force != 22 && T_ >= 16 && Cp >= 64 && Cp <= (T_ >= 36 ? 1024 : 512);
+}
+
+// fp32 on the fp32 instructions, which bound the product: the 64 x 64 tile fills the chip best, except for long reductions
+// with thousands of tiles, where 128 x 128 halves the LDS traffic (measured 5-9 % faster at Cp >= 256).
+static GemmConfig choose_fp32(int T_, int P, int K, int Cp) {
+  if (Cp >= 256 && K >= 128 && (long long)ceil_div(P, 128) * ceil_div(K, 128) * T_ >= 2048) return make_config<float, 2, 2, 16>();
+  return make_config<float, 1, 1, 16>();
+}
 
 // fp16: the largest tile that still gives the 256 CUs about two workgroups each and does not
 // waste more than half a tile on the channel axis (the big tile moves the fewest bytes, and the
@@ -1087,8 +1112,9 @@ int gemm_direct_classes(const void* x, const DirectClass* classes, int n, void* 
 
 using namespace wc;
 
-extern "C" int wc_batched_gemm(const void* V, const void* U, void* M, int T_, int P, int Cp, int K,
-                               int ldm, int dtype, void* stream) {
+namespace wc {
+
+int batched_gemm(const void* V, const void* U, void* M, int T_, int P, int Cp, int K, int ldm, bool transformed, int dtype, void* stream) {
   WC_CHECK_ARG(V && U && M, "wc_batched_gemm: null pointer");
   WC_CHECK_ARG(T_ > 0 && P > 0 && K > 0, "wc_batched_gemm: T %d, P %d, K %d", T_, P, K);
   WC_CHECK_ARG(Cp > 0 && Cp % 32 == 0, "wc_batched_gemm: reduction extent %d is not a multiple of 32", Cp);
@@ -1112,7 +1138,7 @@ extern "C" int wc_batched_gemm(const void* V, const void* U, void* M, int T_, in
     if (force == 10 || force == 13 || (force < 0 && by_size))
       return gemm_persistent(V, U, M, T_, P, Cp, K, ldm, dtype, force != 10 && rides, stream);
   }
-  GemmConfig c = dispatch_dtype(dtype, [&](auto t) { return choose<decltype(t)>(T_, P, K, Cp); });
+  GemmConfig c = dtype == WC_F32 && !fp32_in_parts(T_, Cp, transformed) ? choose_fp32(T_, P, K, Cp) : dispatch_dtype(dtype, [&](auto t) { return choose<decltype(t)>(T_, P, K, Cp); });
   GemmArgs g;
   g.V = V; g.U = U; g.M = M;
   g.P = P; g.K = K; g.Cp = Cp; g.ldm = ldm;
@@ -1131,4 +1157,10 @@ extern "C" int wc_batched_gemm(const void* V, const void* U, void* M, int T_, in
   hipLaunchKernelGGL(c.fn, dim3((unsigned)(g.per_xcd * kXcds)), dim3(c.threads), c.lds, as_stream(stream), g);
   WC_CHECK_LAUNCH("gemm_kernel");
   return WC_OK;
+}
+
+}  // namespace wc
+
+extern "C" int wc_batched_gemm(const void* V, const void* U, void* M, int T_, int P, int Cp, int K, int ldm, int dtype, void* stream) {
+  return batched_gemm(V, U, M, T_, P, Cp, K, ldm, true, dtype, stream);
 }

@@ -7,9 +7,12 @@ namespace wc {
 // upper half of x, m and l rounded to nearest, which together are x exactly, and x y = hh + hm + mh + mm + hl + lh, six of
 // the nine products.  What is left out, ml + lm + ll, is at most 2^-22 and in the root mean square 2^-26 of the product, less
 // than a rounding of fp32, and a sum of 16 products is rounded six times where eight v_mfma_f32_32x32x2_f32 round it eight.
-// 16-bit products have 16 times the rate of fp32 ones.  Against fp64 in the 2-norm, fp32 | this (T=4, 2048 x 512): 32 channels 1.1e-7 |
-// 7.2e-8, 8 channels 6.1e-8 | 3.8e-8, 4 channels 4.7e-8 | 3.9e-8, but a product that stands alone 2.5e-8 | 4.1e-8 (6e-8 | 2.9e-7 of it at
-// most), as the instruction cuts its sums off: with ml and lm as well still 3.4e-8.
+// 16-bit products have 16 times the rate of fp32 ones.
+// They cut their sums off, though, where the fp32 instructions round them.  Against fp64 in the 2-norm, fp32 | this (T=4, 1024 x 256 normal
+// numbers): one channel 2.5e-8 | 4.1e-8 (with ml and lm as well still 3.4e-8), 4 channels 4.0e-8 | 3.9e-8, 32 1.0e-7 | 7.2e-8, 512 4.1e-7 | 3.4e-7, 4096
+// 1.1e-6 | 1.0e-6; half of V zeros, whose products are not rounded: 32 7.5e-8 | 7.1e-8, 128 1.4e-7 | 1.6e-7; sums of one sign: 512 3.5e-7 | 2.9e-7,
+// 2048 7.0e-7 | 1.2e-6, 4096 9.9e-7 | 3.2e-6.  So the parts are for sums of some to a thousand products of transformed operands
+// (fp32_in_parts in gemm.hip; wc_conv_backward_weight, whose kernel adds up longer ones in fp32 outside of the instructions).
 //
 // h of an infinity is the infinity and m is no number, which it makes of every sum it enters.  The kernels take such sums again
 // with fp32 products: a plan whose tile has one tap, or a caller of the product alone, gets the infinity and its sign.

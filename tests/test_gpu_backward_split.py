@@ -4,6 +4,7 @@ spread of a sum of few values."""
 
 import pytest
 import torch
+import torch.nn.functional as F
 
 from pytorch_winoconv_amd import engine
 
@@ -24,6 +25,29 @@ def test_no_larger_error_than_the_fp32_instructions(dev, n, c, k, h, w, taps, ge
     def err():
         dw = engine.conv_backward_weight(x.to(dev), dy.to(dev), shape, 1, taps // 2, 4)
         return float((dw.cpu().double() - ref).norm() / ref.norm())
+
+    split = err()
+    gemm_override(config=22)
+    assert split <= 1.1 * err()
+
+
+def test_long_sums_of_one_sign(dev, gemm_override):
+    """Parts of some thousand tiles, x and dy without negative values, 32 of the input channels against fp64."""
+    n, c, h = 64, 256, 56
+    g = torch.Generator(device=dev).manual_seed(7)
+    x, dy = torch.randn(n, c, h, h, generator=g, device=dev).relu(), torch.randn(n, c, h, h, generator=g, device=dev).abs()
+    ref = torch.zeros(c, 32, 3, 3, dtype=torch.float64, device=dev)
+    for a in range(0, n, 8):
+        xp = F.pad(x[a:a + 8, :32].double(), [1] * 4)
+        d = dy[a:a + 8].double().movedim(1, -1).reshape(-1, c).t().contiguous()
+        for i in range(3):
+            for j in range(3):
+                ref[:, :, i, j] += d @ xp[:, :, i:i + h, j:j + h].movedim(1, -1).reshape(-1, 32).contiguous()
+    x, dy = (t.contiguous(memory_format=torch.channels_last) for t in (x, dy))
+
+    def err():
+        dw = engine.conv_backward_weight(x, dy, (c, c, 3, 3), 1, 1, 4)[:, :32]
+        return float((dw.double() - ref).norm() / ref.norm())
 
     split = err()
     gemm_override(config=22)

@@ -1,4 +1,5 @@
-"""fp32 wc_batched_gemm on the bf16 matrix cores (gemm.hip, Split): six of the nine products of three bf16 parts each.
+"""fp32 products on the bf16 matrix cores (gemm.hip, Split), as whole layers take them where their error is the smaller one and
+wc_batched_gemm on tiles forced here: six of the nine products of three bf16 parts each.
 
 Bound: what is left out is at most 2^-22 of a product; the sum is rounded (2^-24 of at most the sum of the absolute products)
 six times per 16 channels, twice that allowed for what an instruction rounds inside."""
@@ -101,3 +102,35 @@ def test_an_infinity_goes_through_layers_of_one_tap(dev, nd, C, K, stride):
     check(torch.autograd.grad(y, layer.weight, dy.to(dev))[0], torch.autograd.grad(yr, wr, dy.double(), retain_graph=True)[0])
     dy[(1, 11) + (1,) * nd] = float("inf")
     check(torch.autograd.grad(layer(xd), xd, dy.to(dev))[0], torch.autograd.grad(yr, xr, dy.double())[0])
+
+
+LAYERS = [
+    # kernel, stride, tile, channels: in parts from 64 to 1024 products a sum (512 for tiles of fewer than 36 elements), of transformed operands
+    ((1, 1), 1, 4, 100), ((1, 1), 2, 2, 100), ((3, 3), 1, 2, 1), ((3, 3), 1, 4, 2), ((3, 3), 1, 2, 33), ((3, 3), 1, 4, 33), ((3, 3), 1, 2, 512), ((3, 3), 1, 4, 1024),
+    ((3, 3), 1, 2, 2060), ((3, 3), 1, 4, 2060), ((1, 3), 1, 4, 256), ((4, 4), 1, 2, 520), ((5, 5), 1, 2, 128), ((5, 5), 1, 2, 512), ((5, 5), 1, 4, 256),
+    ((5, 5), 1, 4, 512), ((7, 7), 1, 4, 64), ((2, 2), 2, 2, 64), ((3, 3), 2, 2, 256), ((3, 3), 2, 4, 132), ((3, 3), 2, 4, 512),
+    ((3, 3, 3), 1, 2, 2), ((3, 3, 3), 1, 2, 64), ((1, 1, 1), 1, 2, 36), ((3, 3, 3), 2, 2, 8),
+]
+
+
+@pytest.mark.parametrize("kind", ["normal", "relu", "positive"])
+@pytest.mark.parametrize("ks,stride,m,C", LAYERS)
+def test_no_larger_error_than_the_fp32_instructions(dev, ks, stride, m, C, kind, gemm_override):
+    """Whole layers as the library takes them against the fp32 instructions, forced, both against fp64.  A twentieth for the spread of
+    two errors over some ten thousand values."""
+    nd = len(ks)
+    g = torch.Generator(device=dev).manual_seed(C)
+    x = torch.randn([2, C] + [14 if nd == 2 else 9] * nd, generator=g, device=dev)
+    w = torch.randn([72, C, *ks], generator=g, device=dev) * (2.0 / (C * ks[0] * ks[-1])) ** 0.5
+    x = x if kind == "normal" else x.relu() if kind == "relu" else x.abs()
+    w = w.abs() if kind == "positive" else w
+    ref = (F.conv2d if nd == 2 else F.conv3d)(x.double().cpu(), w.double().cpu(), stride=stride)
+
+    def err():
+        y = engine.conv_forward(x, w, None, stride, 0, m, unfused=True, direct=False)
+        assert tuple(y.shape) == tuple(ref.shape)
+        return float((y.double().cpu() - ref).norm() / ref.norm())
+
+    chosen = err()
+    gemm_override(config=22)
+    assert chosen <= 1.05 * err()
