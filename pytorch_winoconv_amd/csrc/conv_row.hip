@@ -662,14 +662,20 @@ int row_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5],
 // 108 | 144, N=6 100 -> 150, 45x61 47 | 72, N=1 128 -> 128, 56x56 12 | 30, 32 -> 32, 14x14 7.5 | 15; fp16 with tile 4: 415 | 520,
 // 235 | 248, 26 | 40, 108 | 135, 46 | 63, 12 | 24, 7.4 | 12.8.
 //
-// 5x5 layers: F(2, 5) needs 15 products per output where the plan they replace, two- or three-tap pieces sharing one
+// 5x5 layers: F(2, 5) needs 15 products per output where the plan it replaces, two- or three-tap pieces sharing one
 // transformed input, needs 20 on F(2x2, 2x2) and 11 on F(3x3, 3x3) (tile 4 in fp16), without V and M in memory, and is as
-// exact as the first (bf16 4.3e-3 | 4.5e-3 against fp64) and 2.5 times as the second (fp16 5.5e-4 | 1.4e-3).  us, row | other, bf16:
+// exact as the first (2-norm against fp64, bf16 5.2e-3 | 5.4e-3) and 2.5 times as the second (fp16 6.5e-4 | 1.7e-3).  us, row | other, bf16:
 // N=32 128 -> 128, 112x112 246 | 407, N=16 256 -> 256, 56x56 127 | 200, 64 -> 64 15 | 37, 512 -> 512, 14x14 60 | 71, N=6
 // 100 -> 150, 45x61 36 | 53, N=1 128 -> 128, 56x56 9 | 22, 64 -> 64, 28x28 7 | 16, 32 -> 32, 14x14 7 | 13; fp16 with tile 4: 248 | 365,
-// 131 | 134, 14 | 33, 57 | 62, 35 | 43, 9 | 17, 7 | 13, 7 | 12.  Layers of 33 to 40 output channels keep the other plan, though it
+// 131 | 134, 14 | 33, 57 | 62, 35 | 43, 9 | 17, 7 | 13, 7 | 12.  Over more than 256 channels it would replace stacked pieces.  Those of tile
+// 2 are slower (us, pieces | row, N=64 512 -> 512, 28x28 649 | 456) but more exact, bf16 4.8e-3 | 5.2e-3, fp16 6.0e-4 | 6.5e-4 over 288 channels (the points are the
+// best there are for F(2, 5)), and stay; those of tile 4 are four times less exact (fp16 2.8e-3).
+// Layers of 33 to 40 output channels keep the other plan, though it
 // is slower (N=2 64 -> 40, 15x14 7 | 15): what has been promised to be outside of the row form stays outside.
-static bool row_preferred_5x5(const wc_conv_desc* d) { return d->K <= 32 || d->K > 40; }
+static bool row_preferred_5x5(const wc_conv_desc* d) {
+  if (d->m == 2 && wc_padded_channels(d->C) > 256) return false;
+  return d->K <= 32 || d->K > 40;
+}
 
 // Against the other forms, us (row | other), channels -> channels on P output pixels:
 //  * Where tile 2 is asked for (the modules in 3-D and in bfloat16): always.  The row form takes 9/8 (3-D: 27/16) times the products of
