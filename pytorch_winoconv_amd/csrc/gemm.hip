@@ -184,7 +184,7 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
   // A reduction block is requested two stages before it is multiplied where the registers allow it, of fp32 in three parts and
   // on the smallest tile of all (T=36, 64x64, fp16, us, one stage | two: P 98, 512 -> 512 9.0 | 8.5; P 784, T=16, 64 -> 64
   // 3.9 | 3.5; fp32 stride 2, N=1 128 -> 128, 56x56 42 | 35).
-  constexpr int AHEAD = (SPLIT && WM * WN <= 4) || WM * WN == 1 ? 2 : 1;
+  constexpr int AHEAD = (SPLIT && WM * WN <= 4) || (DIRECT && sizeof(T) == 2 && WM * WN <= 4) || WM * WN == 1 ? 2 : 1;
   Chunk16 regs[AHEAD][NLOAD];
   bool in_image[AHEAD][DIRECT ? BM / RPP : 1];
   // `vshift`: what the V operand has jumped by at reduction block kt (rows i < BM / RPP are V's)
@@ -206,7 +206,8 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
         }
       }
       regs[set][i] = *reinterpret_cast<const Chunk16*>(gptr[i] + kt * BK + (SHIFT && i < BM / RPP ? vshift : 0));
-    }    if constexpr (DIRECT) {
+    }
+    if constexpr (DIRECT) {
       if (++tap_cb == g.cblocks) {
         tap_cb = 0;
         if (++tap_x == g.kw) { tap_x = 0; ++tap_y; }
@@ -981,17 +982,30 @@ int fold_filter_w(const void* U, void* Uw, int K, int Cp, int dtype, void* strea
   return WC_OK;
 }
 
-// Tiles of the direct form: fp32 products are bound by the MFMA rate and fill the chip best with small tiles (as in choose()).
-// 16-bit types come here only where direct_dma.hip does not reach (direct_dma_fits, 16-byte alignment).
-template <typename T>
-static GemmConfig choose_direct(int P, int K) {
-  constexpr int BK = sizeof(T) == 4 ? 16 : 32;
+// Tiles of the direct form over P pixels (of all classes): 256 x 128 (0), 128 x 128 (1), 64 x 64 (2).  fp32 products are bound by
+// the MFMA rate and fill the chip best with small tiles (as in choose_fp32()).  16-bit types come here only where direct_dma.hip does not reach (direct_dma_fits,
+// tensors that do not start at a multiple of 16 bytes): the largest tile that gives every CU a workgroup.  us, fp16, x one element further, 128 x 128 whatever
+// the problem | so: stride 2, 3x3 N=8 128 -> 8, 56x56 23 | 11.5, N=1 128 -> 128, 56x56 23 | 11, N=32 128 -> 128, 112x112 73 | 65, input
+// gradients, four launches | one, N=8 128 -> 128, 56x56 46 | 18.5, N=64 64 -> 64, 56x56 43 | 25.
+static int direct_tile(long long P, int K, int reduction, bool fp32) {
   const int force = test_gemm_config();               // wc_test_gemm_override: a tile shape forced by a test
-  const bool small = force == 3 || (force != 1 && sizeof(T) == 4 && (K <= 64 || (long long)ceil_div(P, 128) * ceil_div(K, 128) < 2048));
-  if constexpr (sizeof(T) == 4) {
-    if (small) return make_config<T, 1, 1, BK, 2, 2, true, true>();  // 64 x 64
+  if (force == 1 || force == 3) return force == 1 ? 1 : 2;
+  if (force == 4 && !fp32) return 0;
+  const long long mid = ceil_div_ll(P, 128) * ceil_div(K, 128);
+  if (K <= 64) return 2;
+  if (fp32) return mid >= 2048 ? 1 : 2;
+  if (reduction > 768 && ceil_div_ll(P, 256) * ceil_div(K, 128) >= kCus) return 0;      // shorter ones are mostly start and write-out
+  return mid >= kCus ? 1 : 2;
+}
+
+template <typename T>
+static GemmConfig choose_direct(int P, int K, int reduction) {
+  constexpr int BK = sizeof(T) == 4 ? 16 : 32;
+  const int tile = direct_tile(P, K, reduction, sizeof(T) == 4);
+  if constexpr (sizeof(T) == 2) {
+    if (tile == 0) return make_config<T, 4, 2, BK, 2, 2, true, true>();
   }
-  return make_config<T, 2, 2, BK, 2, 2, true, true>();               // 128 x 128
+  return tile == 1 ? make_config<T, 2, 2, BK, 2, 2, true, true>() : make_config<T, 1, 1, BK, 2, 2, true, true>();
 }
 
 // y (N, oH, oW, K) = direct convolution of x (N, H, W, C) with U (K, kh kw C): the batched product with the
@@ -1026,7 +1040,7 @@ int gemm_direct_conv(const void* x, const void* U, const void* bias, void* y, in
   const DirectClass whole{U, kh, kw, pad_h, pad_w, oH, oW, o_y0, o_x0};
   if (dtype != WC_F32 && aligned && test_gemm_config() != 0 && direct_dma_fits(&whole, 1, H, W, C, K, stride))
     return direct_dma(x, &whole, 1, bias, y, N, H, W, C, K, stride, dtype, stream, o_step, o_H, o_W);
-  GemmConfig c = dispatch_dtype(dtype, [&](auto t) { return choose_direct<decltype(t)>((int)P, K); });
+  GemmConfig c = dispatch_dtype(dtype, [&](auto t) { return choose_direct<decltype(t)>((int)P, K, kh * kw * C); });
   GemmArgs g;
   g.V = x; g.U = U; g.M = y; g.bias = bias;
   g.P = (int)P; g.K = K; g.ldm = K;
@@ -1052,7 +1066,7 @@ int gemm_direct_conv(const void* x, const void* U, const void* bias, void* y, in
 
 // The direct products of `n` parity classes in one launch, classes as in gemm_direct_conv's arguments.  A class has a quarter of
 // the pixels and at most four of nine taps, so one by one they leave most of the chip idle (us, one launch per class | one in all:
-// fp32 N=8 128 -> 64 channels, 28x28 -> 56x56 64 | 33).  16-bit types: direct_dma.hip.
+// fp32 N=8 128 -> 64 channels, 28x28 -> 56x56 64 | 33).  16-bit types: direct_dma.hip where it reaches.
 int gemm_direct_classes(const void* x, const DirectClass* classes, int n, void* y, int N, int H, int W, int C, int K,
                         int dtype, void* stream, int o_H, int o_W) {
   WC_CHECK_ARG(x && y && n > 0 && n <= 4, "gemm_direct_classes: %d classes", n);
@@ -1063,49 +1077,52 @@ int gemm_direct_classes(const void* x, const DirectClass* classes, int n, void* 
     for (int i = 0; i < n; ++i) aligned = aligned && (reinterpret_cast<uintptr_t>(classes[i].U) & 15) == 0;
     if (aligned && test_gemm_config() != 0 && direct_dma_fits(classes, n, H, W, C, K, 1))
       return direct_dma(x, classes, n, nullptr, y, N, H, W, C, K, 1, dtype, stream, 2, o_H, o_W);
-    for (int i = 0; i < n; ++i) {
-      const DirectClass& c = classes[i];
-      if (int rc = gemm_direct_conv(x, c.U, nullptr, y, N, H, W, C, K, c.kh, c.kw, 1, c.pad_h, c.pad_w, c.oH, c.oW, dtype, stream, 2, c.o_y0, c.o_x0,
-                                    o_H, o_W))
-        return rc;
-    }
-    return WC_OK;
   }
-  constexpr int BK = 16;
-  auto launch = [&](auto w) -> int {
-    constexpr int W_ = decltype(w)::value;
-    const GemmConfig c = make_config<float, W_, W_, BK, 2, 2, true, true>();        // the sizes of the tile
-    auto fn = &gemm_kernel<float, W_, W_, BK, 2, 2, true, true, true>;
-    GemmClassArgs g;
-    g.V = x; g.U = nullptr; g.M = y; g.bias = nullptr;
-    g.P = 0; g.K = K; g.ldm = K; g.Cp = 0; g.ldv = C; g.run_blocks = 0; g.jump = g.jump2 = 0; g.plane_runs = 0;
-    g.n_run = g.total_runs = g.run_rows = g.plane_extra = 0;
-    g.H = H; g.W = W; g.oH = g.oW = 1; g.conv_stride = 1; g.pad_h = g.pad_w = 0; g.kw = 1; g.cblocks = C / BK;
-    g.o_step = 2; g.o_y0 = g.o_x0 = 0; g.o_H = o_H; g.o_W = o_W;
-    g.sV = g.sU = g.sM = 0; g.tiles_p = 0; g.tiles_k = ceil_div(K, c.bn); g.T = 1;
-    g.n_classes = n;
-    int most = 0;
+  return dispatch_dtype(dtype, [&](auto t) -> int {
+    using T = decltype(t);
+    constexpr int BK = sizeof(T) == 4 ? 16 : 32;
+    auto launch = [&](auto wm, auto wn) -> int {
+      constexpr int WM = decltype(wm)::value, WN = decltype(wn)::value;
+      const GemmConfig c = make_config<T, WM, WN, BK, 2, 2, true, true>();        // the sizes of the tile
+      auto fn = &gemm_kernel<T, WM, WN, BK, 2, 2, true, true, true>;
+      GemmClassArgs g;
+      g.V = x; g.U = nullptr; g.M = y; g.bias = nullptr;
+      g.P = 0; g.K = K; g.ldm = K; g.Cp = 0; g.ldv = C; g.run_blocks = 0; g.jump = g.jump2 = 0; g.plane_runs = 0;
+      g.n_run = g.total_runs = g.run_rows = g.plane_extra = 0;
+      g.H = H; g.W = W; g.oH = g.oW = 1; g.conv_stride = 1; g.pad_h = g.pad_w = 0; g.kw = 1; g.cblocks = C / BK;
+      g.o_step = 2; g.o_y0 = g.o_x0 = 0; g.o_H = o_H; g.o_W = o_W;
+      g.sV = g.sU = g.sM = 0; g.tiles_p = 0; g.tiles_k = ceil_div(K, c.bn); g.T = 1;
+      g.n_classes = n;
+      int most = 0;
+      for (int i = 0; i < n; ++i) {
+        const DirectClass& d = classes[i];
+        const long long P = (long long)N * d.oH * d.oW;
+        WC_CHECK_ARG(d.U && P > 0 && P < (1ll << 31) && (long long)d.kh * d.kw * C < (1ll << 24), "gemm_direct_classes: problem too large");
+        g.cls[i] = {d.U, (long long)(W - d.kw) * C, (int)P, d.kh * d.kw * C, ceil_div((int)P, c.bm), d.kw * C / BK, d.kh + 1,
+                    d.oH, d.oW, d.pad_h, d.pad_w, d.kw, d.o_y0, d.o_x0};
+        most = std::max(most, g.cls[i].tiles_p);
+      }
+      const long long blocks = (long long)most * g.tiles_k * n;
+      WC_CHECK_ARG(blocks < (1ll << 30), "gemm_direct_classes: problem too large");
+      g.n_blocks = (int)blocks;
+      g.per_xcd = ceil_div((int)blocks, kXcds);
+      if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), c.lds)) return rc;
+      hipLaunchKernelGGL(fn, dim3((unsigned)(g.per_xcd * kXcds)), dim3(c.threads), c.lds, as_stream(stream), g);
+      WC_CHECK_LAUNCH("gemm_kernel (direct form, classes)");
+      return WC_OK;
+    };
+    long long P = 0;
+    int reduction = 0;
     for (int i = 0; i < n; ++i) {
-      const DirectClass& d = classes[i];
-      const long long P = (long long)N * d.oH * d.oW;
-      WC_CHECK_ARG(d.U && P > 0 && P < (1ll << 31) && (long long)d.kh * d.kw * C < (1ll << 24), "gemm_direct_classes: problem too large");
-      g.cls[i] = {d.U, (long long)(W - d.kw) * C, (int)P, d.kh * d.kw * C, ceil_div((int)P, c.bm), d.kw * C / BK, d.kh + 1,
-                  d.oH, d.oW, d.pad_h, d.pad_w, d.kw, d.o_y0, d.o_x0};
-      most = std::max(most, g.cls[i].tiles_p);
+      P += (long long)N * classes[i].oH * classes[i].oW;
+      reduction = std::max(reduction, classes[i].kh * classes[i].kw * C);
     }
-    const long long blocks = (long long)most * g.tiles_k * n;
-    WC_CHECK_ARG(blocks < (1ll << 30), "gemm_direct_classes: problem too large");
-    g.n_blocks = (int)blocks;
-    g.per_xcd = ceil_div((int)blocks, kXcds);
-    if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), c.lds)) return rc;
-    hipLaunchKernelGGL(fn, dim3((unsigned)(g.per_xcd * kXcds)), dim3(c.threads), c.lds, as_stream(stream), g);
-    WC_CHECK_LAUNCH("gemm_kernel (direct form, classes)");
-    return WC_OK;
-  };
-  // the rule of choose_direct over the tiles of all classes
-  long long P = 0;
-  for (int i = 0; i < n; ++i) P += (long long)N * classes[i].oH * classes[i].oW;
-  return K > 64 && ceil_div_ll(P, 128) * ceil_div(K, 128) >= 2048 ? launch(ic<2>{}) : launch(ic<1>{});
+    const int tile = direct_tile(P, K, sizeof(T) == 4 ? reduction : 1 << 24, sizeof(T) == 4);
+    if constexpr (sizeof(T) == 2) {
+      if (tile == 0) return launch(ic<4>{}, ic<2>{});
+    }
+    return tile == 1 ? launch(ic<2>{}, ic<2>{}) : launch(ic<1>{}, ic<1>{});
+  });
 }
 
 }  // namespace wc

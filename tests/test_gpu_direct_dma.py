@@ -88,3 +88,29 @@ def test_tensors_that_start_anywhere(dev, shift):
     assert torch.equal(engine.conv_forward(x.half().to(dev), wd, None, 2, 1, 2, U=moved(U), direct=True).cpu(), want.half())
     dx = engine.conv_backward_input(view(dy), wd, (9, 11), 2, 1, 2)
     assert torch.equal(dx.cpu(), torch.nn.grad.conv2d_input((2, 64, 9, 11), w, dy, 2, 1).half())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tile", [-1, 1, 3, 4])
+@pytest.mark.parametrize("case", [CASES[2], CASES[4], CASES[5], CASES[6], CASES[9], ((2, 64, 17, 40), (96, 64, 3, 3), 2, 1)])
+def test_every_tile_through_registers(dev, dtype, tile, case, gemm_override):
+    """Tensors that start two bytes past a multiple of 16, on the tile that their size asks for and on each of the three; the
+    parity classes of an input gradient in one launch.  Exact on small integers."""
+    xs, ws, stride, pad = case
+    g = torch.Generator().manual_seed(9)
+    x, w = torch.randint(-3, 4, xs, generator=g).double(), torch.randint(-2, 3, ws, generator=g).double()
+    b = torch.randint(-8, 9, (ws[0],), generator=g).double()
+    want = F.conv2d(x, w, b, stride, pad)
+
+    def view(t):
+        t = t.movedim(1, -1)
+        return torch.full((t.numel() + 1,), float("nan"), dtype=dtype, device=dev)[1:].view(t.shape).copy_(t).movedim(-1, 1)
+
+    wd = w.to(dtype).to(dev)
+    U = engine.transform_filter(wd, xs, stride, pad, 2, direct=True)
+    gemm_override(config=tile)
+    assert torch.equal(engine.conv_forward(view(x), wd, b.to(dtype).to(dev), stride, pad, 2, U=U, direct=True).cpu(), want.float().to(dtype))
+    if ws[0] % 32 == 0:
+        dy = torch.randint(-3, 4, tuple(want.shape), generator=g).double()
+        dx = engine.conv_backward_input(view(dy), wd, xs[2:], stride, pad, 2)
+        assert torch.equal(dx.cpu(), torch.nn.grad.conv2d_input(xs, w, dy, stride, pad).float().to(dtype))
