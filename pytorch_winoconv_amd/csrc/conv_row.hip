@@ -656,7 +656,7 @@ int row_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5],
   return WC_OK;
 }
 
-// 7x7 layers always: two of F(3, 4) a row are 28 products per output where pieces sharing a transformed input take 36 on F(2x2, 2x2)
+// 7x7 layers nearly always (row_no_slower_7x7): two of F(3, 4) a row are 28 products per output where pieces sharing a transformed input take 36 on F(2x2, 2x2)
 // and 25 on F(3x3, 3x3) (tile 4 in fp16), and the error is smaller than either's (bf16 3.9e-3 | 4.5e-3, fp16 4.8e-4 | 1.5e-3).  us,
 // row | other, bf16: N=32 128 -> 128, 112x112 408 | 565, N=16 256 -> 256, 56x56 228 | 319, 64 -> 64 26 | 45, 512 -> 512, 14x14
 // 108 | 144, N=6 100 -> 150, 45x61 47 | 72, N=1 128 -> 128, 56x56 12 | 30, 32 -> 32, 14x14 7.5 | 15; fp16 with tile 4: 415 | 520,
@@ -674,7 +674,33 @@ int row_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5],
 // is slower (N=2 64 -> 40, 15x14 7 | 15): what has been promised to be outside of the row form stays outside.
 static bool row_preferred_5x5(const wc_conv_desc* d) {
   if (d->m == 2 && wc_padded_channels(d->C) > 256) return false;
+  // fp16 with tile 4: the stacked pieces of F(4x4, .) multiply 9 times per output where F(2, 5) does 15 and are the faster ones where their
+  // product runs on whole rounds of persistent tiles and has the output channels to pay for four transformed inputs.  us, row | pieces:
+  // 512 -> 512 N=64 56x56 1718 | 1579, 28x28 463 | 416, N=8 56x56 251 | 228, N=64 20x20 260 | 228, 1024 -> 1024 N=32 28x28 922 | 659, 384 -> 768
+  // N=64 28x28 523 | 444, 288 -> 512 N=16 56x56 273 | 265, 320 -> 512 N=32 40x40 300 | 303; rounds or tiles short: 512 -> 512 N=24 28x28 199 | 207, N=64 14x14
+  // 126 | 175, N=8 60x60 268 | 313, 1024 -> 1024 N=64 14x14 490 | 515; 256 output channels: 512 -> 256 N=32 56x56 461 | 599.
+  if (d->m == 4 && d->dtype == WC_F16 && wc_padded_channels(d->C) > 256 && d->K >= 512) {
+    const int oH = d->in[1] + 2 * d->pad[1] - 4, oW = d->in[2] + 2 * d->pad[2] - 4;
+    if (persistent_pays(36, (long long)d->N * ceil_div(oH, 4) * ceil_div(oW, 4), 4 * wc_padded_channels(d->C), d->K, wc_padded_channels8(d->K), d->dtype)) return false;
+  }
   return d->K <= 32 || d->K > 40;
+}
+
+// 7x7 layers of fp16 with tile 4 over up to 256 channels: whether the row form takes no longer than the pieces that share one transformed
+// input on F(3x3, 3x3), which run on 512 x 128 tiles.  The row form's boxes of 64 tiles take 10.5 us a step of 32 channels and 4
+// beside them with all CUs at work, less in a last round that is nearly empty; the pieces, whose error is three times as large, are ahead where
+// that round is and theirs is not.  us, row | pieces (this model of both): 256 -> 256, 112x112 N=2 155 | 137 (151 | 139), N=3 164 | 202 (166 | 180), N=4 245 | 227
+// (241 | 222), N=8 422 | 404 (422 | 402), N=12 616 | 626 (604 | 624), N=16 801 | 826 (785 | 804); 256 -> 512, N=8 803 | 765 (785 | 764); 256 -> 256, 80x80
+// N=8 247 | 229 (241 | 232), 100x100 349 | 367 (345 | 364), 56x56 N=32 421 | 470 (433 | 465), 28x28 N=64 224 | 298 (250 | 304), 14x14 71 | 132; 224 -> 224,
+// 112x112 N=8 375 | 365 (372 | 368); 160 -> 256, 100x100 N=5 161 | 152 (158 | 156); 128 -> 128, 112x112 N=32 424 | 528 (410 | 563).
+static bool row_no_slower_7x7(const wc_conv_desc* d, const RowPlan& p) {
+  if (p.shape == kRowSplit || !(d->K % 128 == 0 || d->K % 128 >= 96)) return true;
+  const int oH = d->in[1] + 2 * d->pad[1] - 6, oW = d->in[2] + 2 * d->pad[2] - 6, steps = ceil_div(d->C, 32);
+  auto rounds = [](long long n, double start, double share) { return n / kCus + (n % kCus ? start + share * (n % kCus) / kCus : 0.0); };
+  const long long rows = (long long)d->N * (ceil_div(oH, 3) + 2) * (ceil_div(oW, 3) + 2), tiles = 25 * ceil_div_ll(rows, 512) * ceil_div(d->K, 128);
+  const double pieces = 1.02 * (tiles >= 2 * kCus ? rounds(tiles, 0.4, 0.6) : 1.25 * tiles / kCus) * (8 * steps + 8 + 8.0 * 256 / d->K);
+  const long long full = p.wide_groups / kCus, rest = p.wide_groups % kCus;
+  return full * (10.5 * steps + 4) + (rest ? (7 + 3.5 * rest / kCus) * steps + 4 : 0) <= pieces;
 }
 
 // Against the other forms, us (row | other), channels -> channels on P output pixels:
@@ -700,7 +726,11 @@ bool row_preferred(const wc_conv_desc* d) {
   wc_conv_desc e = *d;
   e.stacked = 0; e.direct = 0; e.row = 0;
   if (wc_plan_conv(&e, &plan) == WC_OK && thin_conv_fits(&e, &plan)) return false;
-  if (d->kernel[1] == 7) return true;
+  if (d->kernel[1] == 7) {
+    if (d->m != 4 || d->dtype != WC_F16 || wc_padded_channels(d->C) > 256) return true;
+    const int oH = d->in[1] + 2 * d->pad[1] - 6, oW = d->in[2] + 2 * d->pad[2] - 6;
+    return row_no_slower_7x7(d, row_plan(d->N, 1, oH, ceil_div(oW, 3), 1, 7, d->K, ceil_div(d->C, 32)));
+  }
   if (d->kernel[1] == 5) return row_preferred_5x5(d);
   if (d->m != 4) return true;
   const int kd = d->kernel[0], oD = d->in[0] + 2 * d->pad[0] - kd + 1, oH = d->in[1] + 2 * d->pad[1] - 2, oW = d->in[2] + 2 * d->pad[2] - 2;

@@ -128,6 +128,8 @@ int fold_filter_w(const void* U, void* Uw, int K, int Cp, int dtype, void* strea
 int output_transform_columns(const wc_conv_desc* d, const void* M, const void* bias, int n_images, void* y, void* stream);
 // wc_batched_gemm; transformed: the operands went through a transform (of kernels of one tap they did not)
 int batched_gemm(const void* V, const void* U, void* M, int T, int P, int Cp, int K, int ldm, bool transformed, int dtype, void* stream);
+// Whether that product runs on persistent 256 x 256 tiles, chosen by size (gemm.hip)
+bool persistent_pays(int T, long long P, int Cp, int K, int ldm, int dtype);
 // wc_batched_gemm on persistent 256 x 256 tiles fed by LDS-DMA (gemm_persistent.hip): 16-bit types, K a multiple of 256
 bool gemm_persistent_fits(int T, int P, int Cp, int K, int dtype);
 bool gemm_persistent_deferred_fits(int P, int Cp, int K, int ldm);      // ... with a tile written out during the next tile's first steps

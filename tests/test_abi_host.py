@@ -552,3 +552,19 @@ def test_the_test_hook_is_inert_in_a_process_that_did_not_opt_in():
     assert out.split()[0] == str(_lib.WC_ERR_UNSUPPORTED) and "WINOCONV_TEST_HOOKS" in out
     lib = _lib.load()
     assert lib.wc_test_gemm_override(-1, 1) == 0            # this process opted in
+
+
+@pytest.mark.parametrize("taps,N,C,K,H,row", [
+    # 5x5 over more than 256 channels into 512 and more, whole rounds of persistent tiles: the pieces of F(4,3) and F(4,2)
+    (5, 64, 512, 512, 56, 0), (5, 8, 512, 512, 56, 0), (5, 32, 1024, 1024, 28, 0), (5, 16, 288, 512, 56, 0),
+    # ... not with an emptier last round, fewer tiles, fewer channels on either side, output channels that are no multiple of 256
+    (5, 8, 512, 512, 60, 1), (5, 24, 512, 512, 28, 1), (5, 32, 512, 256, 56, 1), (5, 32, 256, 512, 56, 1), (5, 32, 512, 520, 56, 1), (5, 1, 512, 512, 14, 1),
+    # 7x7 over up to 256 channels: the row form's last round nearly empty, and not
+    (7, 2, 256, 256, 112, 0), (7, 4, 256, 256, 112, 0), (7, 8, 256, 512, 112, 0), (7, 8, 256, 256, 80, 0), (7, 3, 256, 256, 112, 1), (7, 16, 256, 256, 112, 1),
+    (7, 32, 128, 128, 112, 1), (7, 8, 192, 192, 112, 1), (7, 8, 257, 512, 112, 1), (7, 1, 64, 64, 14, 1)])
+def test_5x5_and_7x7_layers_of_tile_4_take_the_faster_form(taps, N, C, K, H, row):
+    """fp16 layers on the side of the crossover they measured on; bfloat16, whose tile is 2 in earnest, keeps the row form."""
+    def chosen(dtype, m):
+        return engine.make_desc((N, C, H, H), (K, C, taps, taps), dtype, 1, taps // 2, m, stacked=None, row=True).row
+    assert chosen(torch.float16, 4) == row and chosen(torch.bfloat16, 4) == 1
+    assert chosen(torch.float16, 2) == (0 if taps == 5 and C > 256 else 1)
