@@ -19,6 +19,7 @@
 // 32.5 | 39.  Beside its steps a launch moves its partial sums, 59 MB each way where 200 workgroups share 0.6 MB of dw.  Variants that were
 // slower: dy turned channel by channel in LDS and read 16 bytes at a time 424 us, four wavefronts of all nine taps 439; operands
 // read a group ahead changed nothing (377).  Operands are exact, sums fp32.
+#include "lds_dma.h"
 #include "wc_transform.h"
 
 #include <algorithm>
@@ -238,16 +239,6 @@ void taps_kernel(TapsArgs a) {
 // table in LDS; positions outside the image are offsets outside the descriptor's range, which bring zeros.  Rows are not
 // padded: their 64-byte pieces are exchanged by the row instead (LDS-DMA writes rows one after the other), x in every other two rows,
 // dy of 128 channels by the row modulo 4.
-__device__ __forceinline__ void dma16(u32x4 desc, unsigned voff, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" :: "v"(voff), "s"(desc), "s"(lds_addr) : "memory");
-}
-__device__ __forceinline__ u32x4 descriptor(const void* p, long long bytes) {
-  const unsigned long long u = reinterpret_cast<unsigned long long>(p);
-  const unsigned n = (unsigned)max(min(bytes, 0x7fffffffll), 0ll);
-  return u32x4{(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)u), (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(u >> 32)),
-               (unsigned)__builtin_amdgcn_readfirstlane((int)n), 0x00020000u};
-}
-
 template <int KG> constexpr int taps_dma_lds(int ring) { return 3 * kStep * KG * 128 + (ring + kMirror) * 128 + 4 * 2 * kStep * 4; }
 
 template <typename T, int KG>
@@ -273,8 +264,8 @@ void taps_dma_kernel(TapsArgs a) {
   // offsets count from the plane of dy and the image of x that the part begins in
   const int plane0 = fast_div(fast_div(q0, a.f_wp), a.f_hp), n0 = fast_div(plane0, a.f_od);
   const long long dy_start = ((long long)plane0 * a.oH * a.oW * a.K + k0) * 2, x_start = ((long long)n0 * a.D * a.H * a.W * a.C + c0) * 2;
-  const u32x4 dyd = descriptor(static_cast<const unsigned char*>(a.dy) + dy_start, a.dy_elems * 2 - dy_start);
-  const u32x4 xd = descriptor(static_cast<const unsigned char*>(a.x) + x_start, a.x_elems * 2 - x_start);
+  const u32x4 dyd = dma_descriptor(static_cast<const unsigned char*>(a.dy) + dy_start, a.dy_elems * 2 - dy_start);
+  const u32x4 xd = dma_descriptor(static_cast<const unsigned char*>(a.x) + x_start, a.x_elems * 2 - x_start);
   auto place = [&](int pos, int& plane, int& h, int& w) {
     const int row = fast_div(pos, a.f_wp);
     w = pos - row * a.Wp;

@@ -19,7 +19,7 @@
 // Measured, us, fp16, register-staged | this, x in rotation: stride 2, 3x3 128 -> 128, 112x112 N=8 27 | 18, N=16 32 | 28, N=32
 // 57 | 44, N=64 111 | 87; N=1 56x56 12.3 | 9.5; N=2 256 -> 512, 15x17 20 | 14.4; N=64 256 -> 512, 28x28 51 | 43; 1x1 64 -> 256 56x56 N=64 20.7 | 12.8; input
 // gradients N=32 128 <- 128, 112x112 86 | 61, 128 <- 256, 56x56 42 | 36, N=64 256 <- 512, 28x28 75 | 63.
-#include "wc_common.h"
+#include "lds_dma.h"
 #include "wc_transform.h"
 
 #include <algorithm>
@@ -58,16 +58,6 @@ struct DirectDmaArgs {
 
 __device__ __forceinline__ int row_swizzle(int r) { return (((r >> 1) ^ (r >> 3)) & 1) | (((r >> 2) & 1) << 1); }
 
-__device__ __forceinline__ void dma16(u32x4 desc, unsigned voff, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" :: "v"(voff), "s"(desc), "s"(lds_addr) : "memory");
-}
-
-__device__ __forceinline__ u32x4 descriptor(const void* p, unsigned bytes) {
-  const unsigned long long u = reinterpret_cast<unsigned long long>(p);
-  return u32x4{(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)u), (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(u >> 32)),
-               (unsigned)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
-}
-
 constexpr int direct_dma_lds(int BM, int BN, int S) {
   const int stages = S * (BM + BN) * 64, out = BM * (BN + 8) * 2;
   return stages > out ? stages : out;
@@ -96,8 +86,8 @@ __global__ __launch_bounds__(256, WM * WN >= 6 ? 2 : WM * WN >= 4 ? 3 : 4) void 
   const int b0 = fast_div(p0, c.f_image), oy0 = fast_div(p0 - b0 * per, c.f_row);
   const long long row0 = (long long)b0 * a.H + min(oy0 * a.stride, a.H) - c.pad_h;
   const long long start = (row0 * a.W - c.pad_w) * a.C * 2;
-  const u32x4 xd = descriptor(static_cast<const unsigned char*>(a.x) + start, (unsigned)max(min(a.x_bytes - start, 0x7fffffffll), 0ll));
-  const u32x4 ud = descriptor(c.U, (unsigned)c.u_bytes);
+  const u32x4 xd = dma_descriptor(static_cast<const unsigned char*>(a.x) + start, a.x_bytes - start);
+  const u32x4 ud = dma_descriptor(c.U, c.u_bytes);
   auto outside = [](int first, int size, int taps) {             // bit t: first + t is not in 0 .. size - 1
     const int lo = min(max(-first, 0), taps), hi = min(max(size - first, 0), taps);
     return ~(unsigned)(((1ull << hi) - 1) & ~((1ull << lo) - 1));

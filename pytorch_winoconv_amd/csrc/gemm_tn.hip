@@ -18,6 +18,7 @@
 // what fills the chip); the caller adds the parts.  Workgroup = 4 wavefronts (2 x 2), each owning
 // W x W blocks of 32 x 32.  V feeds the MFMA "A" side, so a lane ends up with 4 consecutive
 // columns of D and stores them as one 16-byte write.
+#include "lds_dma.h"
 #include "split_bf16.h"
 #include "wc_transform.h"
 
@@ -230,16 +231,6 @@ __global__ __launch_bounds__(256, 2) void gemm_tn_kernel(GemmTnArgs g) {
 // gemm_tn_kernel waits for each of its loads, which stand behind branches, a stage after it asked for them.  us, whole gradients in fp16, through
 // registers | by LDS-DMA: N=64 256 -> 512, 28x28 at stride 2 67 | 55, 1x1 64 -> 256, 56x56 54 | 40, F(4,3) of 512 -> 512, 56x56 N=32 372 | 339; N=32 128 ->
 // 128, 112x112 at stride 2 85 | 90, bound by the same rows of x and dy from beyond L2 for every tap, and 60 with the taps as neighbours (n_taps).
-__device__ __forceinline__ void dma16(Chunk16 desc, unsigned voff, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" :: "v"(voff), "s"(desc), "s"(lds_addr) : "memory");
-}
-__device__ __forceinline__ Chunk16 descriptor(const void* p, long long bytes) {
-  const unsigned long long u = reinterpret_cast<unsigned long long>(p);
-  const unsigned n = (unsigned)max(min(bytes, 0x7fffffffll), 0ll);
-  return Chunk16{(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)u), (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(u >> 32)),
-                 (unsigned)__builtin_amdgcn_readfirstlane((int)n), 0x00020000u};
-}
-
 constexpr int kTnRows = 32, kTnStages = 4;
 template <int W> constexpr int tn_dma_lds() { return kTnStages * 2 * kTnRows * W * 128 + 4 * 64 * 4; }
 
@@ -263,11 +254,11 @@ __global__ __launch_bounds__(256, 2) void gemm_tn_dma_kernel(GemmTnArgs g) {
   const int nk = (rows + kTnRows - 1) / kTnRows;
 
   const T* const Ap = static_cast<const T*>(g.A) + ((GATHER ? 0 : (long long)t * g.P) + p_begin) * g.lda + a0;
-  const Chunk16 ad = descriptor(Ap, ((long long)rows * g.lda - a0) * 2);
+  const Chunk16 ad = dma_descriptor(Ap, ((long long)rows * g.lda - a0) * 2);
   const int image0 = GATHER ? fast_div((int)min(p_begin, g.P - 1), g.div_per) : 0;
   const long long b_start = GATHER ? (long long)image0 * g.H * g.W * g.ldb + b0 : ((long long)t * g.P + p_begin) * g.ldb + b0;
   const T* const Bp = static_cast<const T*>(g.B) + b_start;
-  const Chunk16 bd = descriptor(Bp, (GATHER ? g.b_elems - b_start : (long long)rows * g.ldb - b0) * 2);
+  const Chunk16 bd = dma_descriptor(Bp, (GATHER ? g.b_elems - b_start : (long long)rows * g.ldb - b0) * 2);
   const int tap_y = GATHER ? t / g.kw : 0, tap_x = GATHER ? t - tap_y * g.kw : 0;
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
