@@ -226,8 +226,8 @@ extern "C" int wc_conv_backward_input(const wc_conv_desc* d, const void* dy, con
     return 0;
   });
   WC_CHECK_LAUNCH("sub_filter_kernel");
-  // one launch for all classes; fp32 classes of four and more taps a row, and direct_rows.hip's tiles in tests, one by one
-  if ((kw + 1) / 2 <= 3 || (d->dtype != WC_F32 && test_gemm_rows() != 2))
+  // one launch for all classes; fp32 classes of four and more taps a row one by one
+  if ((kw + 1) / 2 <= 3 || d->dtype != WC_F32)
     return gemm_direct_classes(dy, cls, a.n, dx, d->N, out[1], out[2], d->K, d->C, d->dtype, stream, H, W);
   for (int i = 0; i < a.n; ++i) {
     const DirectClass& c = cls[i];
@@ -238,5 +238,3 @@ extern "C" int wc_conv_backward_input(const wc_conv_desc* d, const void* dy, con
   return WC_OK;
 }
 
-namespace wc {
-}  // namespace wc

@@ -1,4 +1,4 @@
-// Direct form with ONE operand tile per kernel row (16-bit types, kernel rows of 4 to 8 taps; where it is taken: gemm_direct_conv,
+// Direct form with ONE operand tile per kernel row (16-bit types, kernel rows of 5 to 8 taps; where it is taken: gemm_direct_conv,
 // gemm.hip).
 //
 // A tile per tap (direct_dma.hip) loads, for every tap, its own tile of 256 pixels x 32 channels of x: the taps of
@@ -49,7 +49,6 @@ struct RowsArgs {
   int SR, VR;                 // pixels per slot (one input row with its padding), pixels of the whole tile
   int cblocks, Cp;            // C / 32, kh KW C (row length of U)
   int tiles_k, n_blocks, per_xcd;
-  int o_step, o_y0, o_x0, o_H, o_W;
 };
 
 __device__ __forceinline__ int row_swizzle(int r) { return (((r >> 1) ^ (r >> 3)) & 1) | (((r >> 2) & 1) << 1); }
@@ -84,7 +83,7 @@ constexpr int in_flight(int KW, int kx) {
 
 template <typename T, int KW>
 __global__ __launch_bounds__(256, 1) void direct_rows_kernel(RowsArgs g) {
-  static_assert(KW >= 4 && sizeof(T) == 2, "kernel rows of at least four taps, 16-bit types");
+  static_assert(KW >= 5 && sizeof(T) == 2, "kernel rows of at least five taps, 16-bit types");
   using MF = Mfma16<T>;
   constexpr int WM = 4, WN = 2, BM = 256, BN = 128;
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
@@ -285,16 +284,7 @@ __global__ __launch_bounds__(256, 1) void direct_rows_kernel(RowsArgs g) {
       const u32x4 val = *reinterpret_cast<const u32x4*>(stg + row * (CPR * 16) + ((c ^ (row & (CPR - 1))) * 16));
       const int p = p0 + wp * 128 + i * 32 + row;
       const int k = k0 + wk * 64 + c * 8;
-      if (p < g.P && k < g.K) {
-        long long orow = p;
-        if (g.o_step) {
-          const int per = g.oH * g.oW;
-          const int b = p / per, rem = p - b * per;
-          const int oy = rem / g.oW, ox = rem - oy * g.oW;
-          orow = ((long long)b * g.o_H + oy * g.o_step + g.o_y0) * g.o_W + ox * g.o_step + g.o_x0;
-        }
-        *reinterpret_cast<u32x4*>(yb + orow * g.K + k) = val;
-      }
+      if (p < g.P && k < g.K) *reinterpret_cast<u32x4*>(yb + (long long)p * g.K + k) = val;
     }
   }
 }
@@ -304,7 +294,6 @@ using RowsKernel = void (*)(RowsArgs);
 template <typename T>
 RowsKernel pick_rows(int kw) {
   switch (kw) {
-    case 4: return &direct_rows_kernel<T, 4>;
     case 5: return &direct_rows_kernel<T, 5>;
     case 6: return &direct_rows_kernel<T, 6>;
     case 7: return &direct_rows_kernel<T, 7>;
@@ -321,14 +310,13 @@ static int rows_tile_pixels(int stride, int oW, int kw) { return (255 / oW + 2) 
 
 bool direct_rows_fits(int N, int C, int K, int kw, int stride, int oH, int oW, int dtype) {
   if (dtype != WC_F16 && dtype != WC_BF16) return false;
-  if (kw < 4 || kw > 8 || (stride != 1 && stride != 2)) return false;
+  if (kw < 5 || kw > 8 || (stride != 1 && stride != 2)) return false;
   if (C % 32 != 0 || K % 8 != 0 || oW < 1 || oW > 256) return false;
   return rows_tile_pixels(stride, oW, kw) <= kDirectRowsPixels && (long long)N * oH * oW < (1ll << 31);
 }
 
 int direct_rows_conv(const void* x, const void* U, const void* bias, void* y, int N, int H, int W, int C, int K, int kh,
-                     int kw, int stride, int pad_h, int pad_w, int oH, int oW, int dtype, void* stream, int o_step,
-                     int o_y0, int o_x0, int o_H, int o_W) {
+                     int kw, int stride, int pad_h, int pad_w, int oH, int oW, int dtype, void* stream) {
   WC_CHECK_ARG(x && U && y, "direct_rows_conv: null pointer");
   WC_CHECK_ARG(direct_rows_fits(N, C, K, kw, stride, oH, oW, dtype), "direct_rows_conv: problem outside the kernel's range");
   WC_CHECK_ARG(kh >= 1 && (long long)kh * kw * C < (1ll << 24), "direct_rows_conv: kernel %d x %d", kh, kw);
@@ -343,7 +331,6 @@ int direct_rows_conv(const void* x, const void* U, const void* bias, void* y, in
   g.tiles_k = ceil_div(K, 128);
   g.n_blocks = ceil_div(g.P, 256) * g.tiles_k;
   g.per_xcd = ceil_div(g.n_blocks, kXcds);
-  g.o_step = o_step; g.o_y0 = o_y0; g.o_x0 = o_x0; g.o_H = o_H; g.o_W = o_W;
   RowsKernel fn = dtype == WC_F16 ? pick_rows<half_t>(kw) : pick_rows<bf16_t>(kw);
   WC_CHECK_ARG(fn != nullptr, "direct_rows_conv: kernel rows of %d taps", kw);
   constexpr size_t lds = 2 * (size_t)kVStage + (size_t)kUStages * kUStage;

@@ -1028,14 +1028,13 @@ int gemm_direct_conv(const void* x, const void* U, const void* bias, void* y, in
   // wc_test_gemm_override(., 2) takes it wherever it fits, (., 0) never.
   // LDS-DMA takes 16 bytes from multiples of 16: tensors that start elsewhere go through registers
   const bool aligned = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(U)) & 15) == 0;
-  if (aligned && direct_rows_fits(N, C, K, kw, stride, oH, oW, dtype)) {
+  if (aligned && o_step == 0 && direct_rows_fits(N, C, K, kw, stride, oH, oW, dtype)) {
     const int mode = test_gemm_rows();
     const long long tiles = ceil_div_ll(P, 256) * ceil_div(K, 128);
     const bool k_fills = K % 128 == 0 || K % 128 >= 96;      // the last 128-channel tile is at least three quarters full
     const bool long_rows = kw >= 6 || (kw == 5 && C >= 256);
     if (mode == 2 || (mode != 0 && long_rows && tiles > kCus / 2 && tiles <= kCus && k_fills))
-      return direct_rows_conv(x, U, bias, y, N, H, W, C, K, kh, kw, stride, pad_h, pad_w, oH, oW, dtype, stream, o_step, o_y0,
-                              o_x0, o_H, o_W);
+      return direct_rows_conv(x, U, bias, y, N, H, W, C, K, kh, kw, stride, pad_h, pad_w, oH, oW, dtype, stream);
   }
   const DirectClass whole{U, kh, kw, pad_h, pad_w, oH, oW, o_y0, o_x0};
   if (dtype != WC_F32 && aligned && test_gemm_config() != 0 && direct_dma_fits(&whole, 1, H, W, C, K, stride))

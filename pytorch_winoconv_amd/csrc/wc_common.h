@@ -195,14 +195,13 @@ bool direct_dma_fits(const DirectClass* classes, int n, int H, int W, int C, int
 int direct_dma(const void* x, const DirectClass* classes, int n, const void* bias, void* y, int N, int H, int W, int C, int K, int stride,
                int dtype, void* stream, int o_step, int o_H, int o_W);
 
-// The direct form with one operand tile per kernel row (direct_rows.hip; 16-bit types, kernel rows of 4 to 8 taps, stride
+// The direct form with one operand tile per kernel row (direct_rows.hip; 16-bit types, kernel rows of 5 to 8 taps, stride
 // 1 or 2): whether a problem is in its range (the input rows that 256 consecutive output pixels read, with their
 // padding, must fit a stage of kDirectRowsPixels pixels), and the launch, with the arguments of gemm_direct_conv.
 constexpr int kDirectRowsPixels = 768;
 bool direct_rows_fits(int N, int C, int K, int kw, int stride, int oH, int oW, int dtype);
 int direct_rows_conv(const void* x, const void* U, const void* bias, void* y, int N, int H, int W, int C, int K, int kh,
-                     int kw, int stride, int pad_h, int pad_w, int oH, int oW, int dtype, void* stream, int o_step,
-                     int o_y0, int o_x0, int o_H, int o_W);
+                     int kw, int stride, int pad_h, int pad_w, int oH, int oW, int dtype, void* stream);
 
 // Number of XCDs (L2 domains) a launch is spread over round-robin by workgroup id.
 constexpr int kXcds = 8;

@@ -120,7 +120,8 @@ def test_c4_stride_2_layers_at_full_size(dev):
 
 
 ROWS_CASES = [
-    # x shape, w shape, stride, pad: kernel rows of 4 to 8 taps, which the kernel with one operand tile per kernel row takes
+    # x shape, w shape, stride, pad: kernel rows of 5 to 8 taps, which the kernel with one operand tile per kernel row takes, and one
+    # of 4, which it leaves to the tile per tap
     ((2, 32, 15, 14), (8, 32, 7, 7), 2, 3), ((1, 96, 17, 19), (40, 96, 5, 5), 2, 2), ((2, 32, 10, 11), (8, 32, 4, 6), 2, (1, 2)),
     ((3, 64, 30, 30), (136, 64, 7, 7), 2, 3),          # two channel tiles, the second 8 wide; 675 pixels: three pixel tiles
     ((1, 32, 40, 61), (16, 32, 3, 8), 2, (1, 3)),      # rows of 8 taps, odd width
@@ -171,8 +172,8 @@ def test_one_operand_tile_per_kernel_row_against_fp64_and_the_oracle(dev, dtype,
 
 def test_strided_input_gradient_through_the_kernel_row_tiles(dev, gemm_override):
     """The input gradient of a 7x7 stride-2 layer is four stride-1 direct convolutions of dy, two of them with kernel
-    rows of four taps, each writing every second pixel of dx: with the kernel-row tiles forced, on small integers,
-    bit-equal to the gradient autograd gives in fp64."""
+    rows of four taps, each writing every second pixel of dx, which the kernel-row tiles do not: forced, they leave it to
+    the tile per tap.  On small integers, bit-equal to the gradient autograd gives in fp64."""
     g = torch.Generator().manual_seed(7)
     x = torch.zeros(2, 40, 18, 20, dtype=torch.double, requires_grad=True)
     w = torch.randint(-2, 3, (32, 40, 7, 7), generator=g).double()
