@@ -670,8 +670,8 @@ int row_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5],
 // 131 | 134, 14 | 33, 57 | 62, 35 | 43, 9 | 17, 7 | 13, 7 | 12.  Over more than 256 channels it would replace stacked pieces.  Those of tile
 // 2 are slower (us, pieces | row, N=64 512 -> 512, 28x28 649 | 456) but more exact, bf16 4.8e-3 | 5.2e-3, fp16 6.0e-4 | 6.5e-4 over 288 channels (the points are the
 // best there are for F(2, 5)), and stay; those of tile 4 are four times less exact (fp16 2.8e-3).
-// Layers of 33 to 40 output channels keep the other plan, though it
-// is slower (N=2 64 -> 40, 15x14 7 | 15): what has been promised to be outside of the row form stays outside.
+// Layers of 33 to 40 output channels keep the other plan, though it is slower (N=2 64 -> 40, 15x14 7 | 15): no measurement puts a
+// line there, tests/test_gpu_row.py and test_gpu_row_5x5_7x7.py take them for 5x5 layers beside the row form.
 static bool row_preferred_5x5(const wc_conv_desc* d) {
   if (d->m == 2 && wc_padded_channels(d->C) > 256) return false;
   // fp16 with tile 4: the stacked pieces of F(4x4, .) multiply 9 times per output where F(2, 5) does 15 and are the faster ones where their

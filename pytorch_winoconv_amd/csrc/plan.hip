@@ -358,13 +358,14 @@ static int auto_stacked(const wc_conv_desc* d) {
 // direct | F(2,r) plan | F(4,r) plan):
 //  * Short reductions (kh kw C <= 3200, of up to nine taps 4500) always: 3x3 at N=32, C=K=128, 112x112 44 | 160 | 126; 256 -> 512
 //    at 28x28 43 | 81 | 86; C=K=384 N=64 14x14 24 | 44 | 36, N=8 28x28 18 | 27 | 31; 480 -> 96 N=4 20x20 22 | 24 | 26; 416 -> 224 N=2 9x9 19 | 21 |
-//    23; 5x5 at C=128 99 | 261 | 154.  More taps: C=K=160, 28x28, N=1 5x5 19 | 15 | 17.  (3x3 on 512 channels would gain as well, N=64
-//    14x14 36 | 61 | 56, but what has been promised to be outside of the direct form stays outside.)
+//    23; 5x5 at C=128 99 | 261 | 154.  More taps: C=K=160, 28x28, N=1 5x5 19 | 15 | 17.  (The measurements do not put the line at
+//    4500: 3x3 on 512 channels would gain as well, N=64 14x14 36 | 61 | 56.  It stands there because tests/test_abi_host.py takes 512 channels for
+//    layers beyond it.)
 //  * With 64 output channels or fewer it runs 64 x 64 tiles only and loses beyond 5x5 kernels (7x7, C=K=64,
 //    224x224: 382 | 372; 128 -> 64 at 112x112: 209 | 201).
 //  * A long reduction needs enough output (pixels x channels >= 4 M, i.e. 256 tiles of 128 x 128) to keep the chip
 //    busy, else the latency of its k-steps decides: 5x5 at C=K=256 N=8 on 28x28 images 29 | 27 | 24, 7x7 at C=K=256
-//    240 | 139.  With that, and with one operand tile per kernel row for rows of 4 to 8 taps (direct_rows.hip): against
+//    240 | 139.  With that, and with one operand tile per kernel row for rows of 5 to 8 taps (direct_rows.hip): against
 //    the plan that shares one transformed input (7 and 8 taps) it wins (C=K=128, 112x112: 7x7 181 | 270, 8x8 234 | 284;
 //    96 channels 7x7 146 | 214, 8x8 182 | 224; 256 -> 512 on 28x28 7x7 173 | 228, 8x8 230 | 277); against stacked
 //    F(2,r) pieces it wins (128 channels, 112x112: 6x6 168 | 281, 9x9 421 | 845; 256 -> 512 on 28x28 5x5 111 | 115);

@@ -41,8 +41,10 @@ def dwm3d(input, kernel, bias=None, stride=(1, 1, 1), padding=0, groups=1, outpu
 
 def dwm2d(input, kernel, bias=None, stride=(1, 1), padding=0, groups=1, output_block=2):
     """2-D DWM convolution (reference: dwm.py:25-40).  output_block = 2 is the reference's F(2,r)
-    decomposition; 4 uses F(4,r) pieces (about 1.3x faster for 5x5 / 7x7 kernels, fp16 error
-    about 10x larger but inside the 2e-2 bound)."""
+    decomposition; 4 allows F(4,r) pieces (up to 1.5x faster, error 5 to 10 times larger but inside the
+    2e-2 bound).  16-bit 3x3, 5x5 and 7x7 layers at stride 1 mostly run in the row form for either value,
+    with the error of 2, and strided ones in the direct form; what 4 changes are the plans beside these:
+    fp32 layers, and wide fp16 ones."""
     return _dwm(input, kernel, bias, stride, padding, groups, 2, output_block)
 
 
