@@ -189,7 +189,8 @@ int wc_plan_conv(const wc_conv_desc* desc, wc_plan* plan);
  * three-tap pieces on F(3,3) apply (fp16, 2-D, stride 1, at least 3 taps per axis and 5 on one), else by 2;
  * desc->direct == -1 on entry: the direct form is never chosen (and the field comes back 0); desc->row == -1 with
  * desc->stacked == -1: the row form is chosen (row = 1) - with m = 4 where it measured faster than that tile, else wherever the
- * one-kernel F(2x2,3x3) form does not run and, for 5x5 kernels, over up to 256 input channels -, otherwise the field comes back 0.
+ * one-kernel F(2x2,3x3) form does not run and, for 5x5 kernels, over up to 256 input channels -, otherwise the field comes back 0
+ * (so it does for 5x5 layers of 33 to 40 output channels, which no caller should count on).
  * The caller reads the tile that will really be used back from desc->m.  No counterpart in the reference,
  * which has one form only (src/base_conv_launchers.cu:282-399).  Every other function wants stacked >= 0. */
 int wc_conv_auto(wc_conv_desc* desc);
