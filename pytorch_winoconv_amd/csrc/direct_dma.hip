@@ -18,7 +18,7 @@
 //
 // Measured, us, fp16, register-staged | this, x in rotation: stride 2, 3x3 128 -> 128, 112x112 N=8 27 | 18, N=16 32 | 28, N=32
 // 57 | 44, N=64 111 | 87; N=1 56x56 12.3 | 9.5; N=2 256 -> 512, 15x17 20 | 14.4; N=64 256 -> 512, 28x28 51 | 43; 1x1 64 -> 256 56x56 N=64 20.7 | 12.8; input
-// gradients N=32 128 <- 128, 112x112 86 | 61, 128 <- 256, 56x56 42 | 36, N=64 256 <- 512, 28x28 75 | 63.
+// gradients (classes turned, class_of_block) N=32 128 <- 128, 112x112 86 | 51, 128 <- 256, 56x56 42 | 29, N=64 256 <- 512, 28x28 75 | 54.
 #include "lds_dma.h"
 #include "wc_transform.h"
 
@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256, WM * WN >= 6 ? 2 : WM * WN >= 4 ? 3 : 4) void 
 
   int blk = xcd_remap(blockIdx.x, a.per_xcd);
   if (blk >= a.n_blocks) return;
-  const DirectDmaArgs::Class c = a.cls[blk % a.n_classes];
+  const DirectDmaArgs::Class c = a.cls[class_of_block(blk, a.n_classes, a.per_xcd)];
   blk /= a.n_classes;
   if (blk >= c.tiles_p * a.tiles_k) return;
   const int k0 = blk % a.tiles_k * BN, p0 = blk / a.tiles_k * BM;
@@ -282,11 +282,12 @@ static int launch_direct_dma(DirectDmaArgs a, const DirectClass* classes, int N,
 // P: pixels of all classes.  us, fp16, 256x128 | 128x128 | 64x64 tile (256x64 | 128x64 | 64x64 for 64 channels):
 //   forward, 256x128 tiles in all: 392 44 | 54 | 67, 294 41 | 40 | 52, 196 27.4 | 28 | 37 and 43 | 45 | 65, 98 24 | 18 | 22, 74 24 | 17.6 | 18; 128x128
 //   tiles in all: 79 14.4 | 10.4, 50 27 | 15;   64 channels, 256x64 tiles in all: 391 14.9 | 15.8 | 15.6, 98 11.3 | 8.7 | 9.1
-//   classes, 256x128 tiles in all: 1568 67 | 61 | 90, 784 41 | 37 | 50, 392 36 | 40 | 48 and 64 | 74 | 88, 245 26 | 25.4 | 34, 147 24.5 | 22 | 25; 128x128 tiles in
-//   all: 196 22 | 22 and 20 | 23, 28 34 | 25;   64 channels, 256x64 tiles in all: 3136 74 | 72 | 89, 1568 (32 channels) 31 | 29 | 34, 392 19 | 21 | 22
+//   classes, rounds of 256x128 tiles and input channels (those of dy), 256x128 | 128x128: 0.7 18.4 | 16.0 (128), 25.9 | 22.2 (256), 45 | 37 (512); 1.0
+//   20.2 | 19.1, 28.5 | 28.1, 49 | 51; 1.5 22.0 | 19.9, 30.9 | 28.9, 54 | 61; 2.2 33 | 28, 49 | 41, 86 | 73; 3.3 35.2 | 34.7, 53.7 | 54.4, 95 | 99; 5.5 50.2
+//   | 50.1, 81 | 84, 142 | 153; 128x128 | 64x64 in tiles of 128x128: 196 22 | 22 and 20 | 23, 28 34 | 25;   64 channels, 256x64 | 128x64: 0.7 rounds 13.2 | 14.5, 5.5 37 | 44
 // The large tile, two to a CU, wherever most CUs have one; classes, whose tiles are of four lengths, share out better in smaller
-// ones unless all of the large tiles are there at once.
-static int choose_tile(long long P, int K, bool classes) {
+// ones unless the reduction is long and the large tiles are there at once, or many.
+static int choose_tile(long long P, int C, int K, bool classes) {
   const int force = test_gemm_config();
   if (force >= 22 && force <= 26) return force - 22;
   auto tiles = [&](int bm, int bn) { return ceil_div_ll(P, bm) * ceil_div(K, bn); };
@@ -296,7 +297,7 @@ static int choose_tile(long long P, int K, bool classes) {
   }
   const long long big = tiles(256, 128), mid = tiles(128, 128);
   const bool full = K % 128 == 0 || K % 128 > 64;
-  if (full && (classes ? big >= kCus && big <= 2 * kCus : big >= 3 * kCus / 4)) return 0;
+  if (full && (classes ? (C >= 512 && big >= kCus && big <= 2 * kCus) || (C >= 256 && big >= 3 * kCus) : big >= 3 * kCus / 4)) return 0;
   return mid >= (classes ? 3 * kCus / 4 : kCus / 2) ? 1 : 4;
 }
 
@@ -304,7 +305,7 @@ int direct_dma(const void* x, const DirectClass* classes, int n, const void* bia
                int dtype, void* stream, int o_step, int o_H, int o_W) {
   long long P = 0;
   for (int i = 0; i < n; ++i) P += (long long)N * classes[i].oH * classes[i].oW;
-  const int tile = choose_tile(P, K, n > 1);
+  const int tile = choose_tile(P, C, K, n > 1);
   for (int i = 0; i < n; ++i)
     WC_CHECK_ARG(classes[i].U && classes[i].oH > 0 && classes[i].oW > 0 && (long long)N * classes[i].oH * classes[i].oW < (1ll << 31), "direct_dma: problem too large");
   DirectDmaArgs a{};

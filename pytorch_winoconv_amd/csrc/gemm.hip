@@ -139,7 +139,7 @@ void gemm_kernel(std::conditional_t<CLASSES, GemmClassArgs, GemmArgs> args) {
   int blk = xcd_remap(blockIdx.x, g.per_xcd);
   if (blk >= g.n_blocks) return;
   if constexpr (CLASSES) {
-    const typename GemmClassArgs::Class& c = args.cls[blk % args.n_classes];
+    const typename GemmClassArgs::Class& c = args.cls[class_of_block(blk, args.n_classes, args.per_xcd)];
     blk /= args.n_classes;
     if (blk >= c.tiles_p * g.tiles_k) return;
     g.U = c.U; g.jump = c.jump; g.P = c.P; g.Cp = c.Cp; g.tiles_p = c.tiles_p; g.run_blocks = c.run_blocks; g.plane_runs = c.plane_runs;

@@ -213,6 +213,14 @@ constexpr int kCus = 256;                  // compute units of an MI355X
 __device__ __forceinline__ int xcd_remap(int hw_id, int per_xcd) {
   return (hw_id % kXcds) * per_xcd + hw_id / kXcds;
 }
+// The class of logical workgroup `blk` of a launch whose workgroups alternate over classes of work of different lengths.  An XCD's
+// workgroups go round its compute units, so a unit's own are kCus / kXcds apart: turned by one class a round they are of different
+// classes.  (All of one, as blk % n_classes gives, the units with the longest class finish late: us, fp16 input gradients at
+// stride 2, same | turned: N=32 56x56 128 <- 256 37 | 29, 256 <- 512 28x28 N=63 68 | 54, N=230 190 | 142, 64 <- 128 N=115 45 | 38.)
+__device__ __forceinline__ int class_of_block(int blk, int n_classes, int per_xcd) {
+  const int round = blk / n_classes * n_classes % per_xcd / (kCus / kXcds);
+  return (blk + round) % n_classes;
+}
 
 // acc (taps, K, C) (+)= G^T dU G per piece of the plan; dU (T, S, K, ldc) with the parts already
 // summed into part 0; `first` overwrites acc instead of adding (backward_filter.hip).

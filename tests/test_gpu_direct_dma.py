@@ -114,3 +114,17 @@ def test_every_tile_through_registers(dev, dtype, tile, case, gemm_override):
         dy = torch.randint(-3, 4, tuple(want.shape), generator=g).double()
         dx = engine.conv_backward_input(view(dy), wd, xs[2:], stride, pad, 2)
         assert torch.equal(dx.cpu(), torch.nn.grad.conv2d_input(xs, w, dy, stride, pad).float().to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("n,c,k,h,w", [(8, 64, 32, 56, 56), (25, 128, 32, 31, 29), (7, 96, 64, 60, 1), (40, 32, 32, 33, 40)])
+def test_classes_of_more_than_one_round_of_an_xcd(dev, dtype, n, c, k, h, w, gemm_override):
+    """Input gradients whose launches have more workgroups than compute units, on the smallest tile: every tile of every class once, where
+    an XCD's share is no multiple of the classes (8 x 784 pixels in tiles of 64: 49) and with two classes only.  Exact on small integers."""
+    g = torch.Generator().manual_seed(11)
+    wt = torch.randint(-2, 3, (k, c, 3, 3), generator=g).double()
+    dy = torch.randint(-3, 4, (n, k, (h + 1) // 2, (w + 1) // 2), generator=g).double()
+    if dtype == torch.float16:
+        gemm_override(config=26)
+    dx = engine.conv_backward_input(dy.to(dtype).to(dev).contiguous(memory_format=torch.channels_last), wt.to(dtype).to(dev), (h, w), 2, 1, 2)
+    assert torch.equal(dx.cpu(), torch.nn.grad.conv2d_input((n, c, h, w), wt, dy, 2, 1).float().to(dtype))
