@@ -163,7 +163,8 @@ const char* wc_last_error(void);
  * config 16 to 19: the row form with the wide, half, small or split workgroups whatever the problem (conv_row.hip).
  * config 21: the row form on tall boxes whatever the problem (conv_row_tall.hip).
  * config 22 to 26: the direct form of 16-bit types on tiles of 256 x 128, 128 x 128, 256 x 64, 128 x 64 or 64 x 64 whatever the
- * problem (direct_dma.hip); 22 also: fp32 products and weight gradients on the fp32 instructions.
+ * problem (direct_dma.hip); 22 also: fp32 products and weight gradients on the fp32 instructions.  config 27 to 29: its forward
+ * products on tiles of 320, 384 or 448 x 128.
  * config 0 to 4 in fp32: the tiles of the product in three bf16 parts.  config 0: the direct form of 16-bit
  * types through registers (gemm.hip).
  * Works only in a process started with WINOCONV_TEST_HOOKS=1 in its environment (WC_ERR_UNSUPPORTED

@@ -128,3 +128,19 @@ def test_classes_of_more_than_one_round_of_an_xcd(dev, dtype, n, c, k, h, w, gem
         gemm_override(config=26)
     dx = engine.conv_backward_input(dy.to(dtype).to(dev).contiguous(memory_format=torch.channels_last), wt.to(dtype).to(dev), (h, w), 2, 1, 2)
     assert torch.equal(dx.cpu(), torch.nn.grad.conv2d_input((n, c, h, w), wt, dy, 2, 1).float().to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tile", [27, 28, 29])
+@pytest.mark.parametrize("case", CASES + [((3, 96, 37, 41), (200, 96, 3, 3), 2, 1), ((2, 32, 30, 31), (128, 32, 1, 1), 1, 0), ((1, 32, 43, 42), (136, 32, 2, 1), 2, 0)])
+def test_tall_tiles_are_exact_on_small_integers(dev, dtype, tile, case, gemm_override):
+    """Forward products on tiles of 320, 384 and 448 pixels: odd and even counts of stages, fewer stages than the ring has places,
+    last tiles of pixels and of channels that are nearly empty or of one row past a full one."""
+    xs, ws, stride, pad = case
+    g = torch.Generator().manual_seed(12)
+    x = torch.randint(-3, 4, xs, generator=g).double()
+    w = torch.randint(-2, 3, ws, generator=g).double()
+    b = torch.randint(-8, 9, (ws[0],), generator=g).double()
+    gemm_override(config=tile, rows_mode=0)
+    y = engine.conv_forward(x.to(dtype).to(dev).contiguous(memory_format=torch.channels_last), w.to(dtype).to(dev), b.to(dtype).to(dev), stride, pad, 2, direct=True)
+    assert torch.equal(y.cpu(), F.conv2d(x, w, b, stride, pad).float().to(dtype))
