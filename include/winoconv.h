@@ -326,6 +326,12 @@ int wc_conv_backward_input(const wc_conv_desc* desc, const void* dy, const void*
 int wc_conv_backward_weight(const wc_conv_desc* desc, const void* x, const void* dy, void* dw,
                             const int64_t dw_strides[5], void* workspace, size_t workspace_bytes,
                             void* stream);
+/* The weight gradient and, where db is not null, the bias gradient of one dy in one call, each in the operands' type or in fp32
+ * (unrounded: what a layer with fp32 parameters wants).  Kernels that have dy in LDS add its columns up on the way; the others are followed
+ * by the launches of wc_bias_gradient.  Workspace 256-byte aligned, enough for either. */
+int wc_conv_backward_parameters_workspace_bytes(const wc_conv_desc* desc, size_t* bytes);
+int wc_conv_backward_parameters(const wc_conv_desc* desc, const void* x, const void* dy, void* dw, const int64_t dw_strides[5],
+                                int dw_dtype, void* db, int db_dtype, void* workspace, size_t workspace_bytes, void* stream);
 /* Bias gradient (no counterpart in the reference): db[k] = sum over the rows of dy (rows, K), contiguous - the pixels of a
  * channel-last tensor of K channels -, in fp32, rounded once.  Workspace 16-byte aligned. */
 int wc_bias_gradient_workspace_bytes(long long rows, int K, int dtype, size_t* bytes);

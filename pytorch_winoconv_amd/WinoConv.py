@@ -72,15 +72,13 @@ class WinoConvFunction(torch.autograd.Function):
         if need_dx and dx is None:
             dx = engine.conv_backward_input(dy, w, x.shape[2:], stride, padding, m)
         if need_dw and dw is None:
-            dw = engine.conv_backward_weight(x, dy, w.shape, stride, padding, m)
-            dw = dw if w_type is None else dw.to(w_type)
-        if has_bias and need_db and db is None:
-            # the engine's kernel where this pass runs on it anyway; a gradient that is itself differentiated, or a dy
+            # the engine's bias gradient where this pass runs on it anyway; a gradient that is itself differentiated, or a dy
             # that the kernel would have to copy first, stays with torch
-            if need_dw and not torch.is_grad_enabled() and engine.channel_last_memory(dy):
-                db = engine.bias_gradient(dy)
-            else:
-                db = dy.sum(dim=[0] + list(range(2, dy.dim())))
+            both = has_bias and need_db and not torch.is_grad_enabled() and engine.channel_last_memory(dy)
+            dw, b = engine.conv_backward_parameters(x, dy, w.shape, stride, padding, m, both, w_type, b_type)
+            db = b if both else db
+        if has_bias and need_db and db is None:
+            db = dy.sum(dim=[0] + list(range(2, dy.dim())))
             db = db if b_type is None else db.to(b_type)
         return dx, dw, db, None, None, None, None, None
 

@@ -70,6 +70,8 @@ SIGNATURES = {
     "wc_conv_forward_timed": (_i, [_desc_p, _vp, _vp, _i64_5, _vp, _vp, _vp, _vp, _sz, _vp, ctypes.POINTER(ctypes.c_float)]),
     "wc_conv_backward_weight_workspace_bytes": (_i, [_desc_p, ctypes.POINTER(_sz)]),
     "wc_conv_backward_weight": (_i, [_desc_p, _vp, _vp, _vp, _i64_5, _vp, _sz, _vp]),
+    "wc_conv_backward_parameters_workspace_bytes": (_i, [_desc_p, ctypes.POINTER(_sz)]),
+    "wc_conv_backward_parameters": (_i, [_desc_p, _vp, _vp, _vp, _i64_5, _i, _vp, _i, _vp, _sz, _vp]),
     "wc_bias_gradient_workspace_bytes": (_i, [ctypes.c_longlong, _i, _i, ctypes.POINTER(_sz)]),
     "wc_bias_gradient": (_i, [_vp, _vp, ctypes.c_longlong, _i, _i, _vp, _sz, _vp]),
 }

@@ -13,6 +13,7 @@
 // whose products are exact in fp32; the sum over up to millions of tiles is kept in fp32 from the
 // first product to the last addition), split into parts that are added here, and a last kernel
 // applies G^T . G and accumulates over image chunks (backward_filter.hip).
+#include "column_sums.h"
 #include "wc_transform.h"
 #include <algorithm>
 
@@ -203,9 +204,11 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(float* __restrict__ dU, 
 // sum of one thread per value and a second kernel for the way to dw | so, fp16: 9 x 128 x 128 in 28 parts 60 | 48.5, in 24 parts 23 | 15.6,
 // 1x1 64 -> 256, 64 parts 40 | 24.5.
 template <typename T>
-__global__ __launch_bounds__(256) void sum_parts_store_kernel(const float* __restrict__ dU, T* __restrict__ dw, int S, long long n,
-                                                             long long total4, long long s0, long long s1, long long s3, long long s4, int C, int kW) {
+__global__ __launch_bounds__(256) void sum_parts_store_kernel(const float* __restrict__ dU, void* __restrict__ dw, int S, long long n,
+                                                             long long total4, long long s0, long long s1, long long s3, long long s4, int C, int kW,
+                                                             bool f32, int blocks, ColumnSums bias) {
   __shared__ float4 sums[3][64];
+  if (blockIdx.x >= (unsigned)blocks) return sum_columns<T>(bias, blockIdx.x - blocks, reinterpret_cast<float*>(sums));
   const int lane = threadIdx.x & 63, group = threadIdx.x >> 6;
   const long long idx = (long long)blockIdx.x * 64 + lane;
   const bool in = idx < total4;
@@ -227,13 +230,13 @@ __global__ __launch_bounds__(256) void sum_parts_store_kernel(const float* __res
     sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
   }
   const int k = (int)(i / C), c = (int)(i % C);
-  T* const dst = dw + k * s0 + c * s1 + (int)t / kW * s3 + (int)t % kW * s4;
-  dst[0] = static_cast<T>(sum.x); dst[s1] = static_cast<T>(sum.y); dst[2 * s1] = static_cast<T>(sum.z); dst[3 * s1] = static_cast<T>(sum.w);
+  const long long dst = k * s0 + c * s1 + (int)t / kW * s3 + (int)t % kW * s4;
+  store_as<T>(dw, dst, sum.x, f32); store_as<T>(dw, dst + s1, sum.y, f32); store_as<T>(dw, dst + 2 * s1, sum.z, f32); store_as<T>(dw, dst + 3 * s1, sum.w, f32);
 }
 
 // dw[k][c][tap] through element strides <- acc (taps, K, C)
 template <typename T>
-__global__ __launch_bounds__(256) void grad_filter_store_kernel(const float* __restrict__ acc, T* __restrict__ dw,
+__global__ __launch_bounds__(256) void grad_filter_store_kernel(const float* __restrict__ acc, void* __restrict__ dw, bool f32,
                                                                long long s0, long long s1, long long s2, long long s3,
                                                                long long s4, int K, int C, int kD, int kH, int kW,
                                                                long long total) {
@@ -244,7 +247,7 @@ __global__ __launch_bounds__(256) void grad_filter_store_kernel(const float* __r
   const int k = (int)(q % K);
   const int tap = (int)(q / K);
   const int x2 = tap % kW, x1 = (tap / kW) % kH, x0 = tap / (kW * kH);
-  dw[k * s0 + c * s1 + x0 * s2 + x1 * s3 + x2 * s4] = static_cast<T>(acc[idx]);
+  store_as<T>(dw, k * s0 + c * s1 + x0 * s2 + x1 * s3 + x2 * s4, acc[idx], f32);
 }
 
 }  // namespace wc
@@ -299,6 +302,7 @@ struct BwdLayout {
   long long tiles_per_image;
   size_t es;
   size_t v_bytes, dm_bytes, du_bytes, acc_bytes;
+  size_t sums_bytes;                // column sums of dy, where they are taken beside the product
   bool one_tap;                     // 1x1 kernel, stride 1, no padding: dw = dy^T x, no transforms
   bool gathered;                    // 2-D stride 2: dw[tap] = dy^T (the pixels of x that tap reads), no transforms
   bool taps;                        // 16-bit 3x3 and 3x3x3 at stride 1: the tap form (backward_taps.hip), du_bytes of partial sums
@@ -329,6 +333,7 @@ bool gathered_layout(const wc_conv_desc* d, BwdLayout* L) {
   L->Pq = (int)(((P + S - 1) / S + 31) / 32 * 32);
   L->v_bytes = L->dm_bytes = 0;
   L->du_bytes = round256((size_t)taps * S * d->K * d->C * 4);
+  L->sums_bytes = (size_t)tn_sum_rows(taps, d->K, d->C, L->S) * tn_sum_width(d->K, d->C) * 4;
   L->acc_bytes = 0;
   return true;
 }
@@ -355,6 +360,7 @@ bool one_tap_layout(const wc_conv_desc* d, BwdLayout* L) {
   L->Pq = (int)(((P + S - 1) / S + 31) / 32 * 32);
   L->v_bytes = L->dm_bytes = L->acc_bytes = 0;
   L->du_bytes = round256((size_t)S * d->K * d->C * 4);
+  L->sums_bytes = (size_t)tn_sum_rows(1, d->K, d->C, L->S) * tn_sum_width(d->K, d->C) * 4;
   return true;
 }
 
@@ -363,6 +369,7 @@ int make_bwd_layout(const wc_conv_desc* d, BwdLayout* L) {
   WC_CHECK_ARG(d->dtype == WC_F32 || d->dtype == WC_F16 || d->dtype == WC_BF16, "dtype %d", d->dtype);
   WC_CHECK_ARG((d->ndim == 2 || d->ndim == 3) && d->N > 0 && d->C > 0 && d->K > 0, "ndim %d, N %d, C %d, K %d", d->ndim, d->N, d->C, d->K);
   L->one_tap = L->gathered = L->taps = false;
+  L->sums_bytes = 0;
   if (one_tap_layout(d, L)) return WC_OK;
   if (gathered_layout(d, L)) return WC_OK;
   if (d && d->stacked == 2)
@@ -372,7 +379,7 @@ int make_bwd_layout(const wc_conv_desc* d, BwdLayout* L) {
   rc = wc_conv_out_dims(d, L->out, L->grid);
   if (rc) return rc;
   if (L->plan.t_total > 0xffff) return fail(WC_ERR_UNSUPPORTED, "plan with %d transform elements is too large", L->plan.t_total);
-  if (taps_gradient_fits(d, L->out, &L->du_bytes)) {
+  if (taps_gradient_fits(d, L->out, &L->du_bytes, &L->sums_bytes)) {
     L->taps = true;
     L->v_bytes = L->dm_bytes = L->acc_bytes = 0;
     return WC_OK;
@@ -416,31 +423,45 @@ int make_bwd_layout(const wc_conv_desc* d, BwdLayout* L) {
   return WC_OK;
 }
 
-}  // namespace
+size_t weight_bytes(const BwdLayout& L) { return L.v_bytes + L.dm_bytes + L.du_bytes + L.acc_bytes; }
+long long dy_rows(const wc_conv_desc* d, const int out[3]) { return (long long)d->N * out[0] * out[1] * out[2]; }
 
-extern "C" {
-
-int wc_conv_backward_weight_workspace_bytes(const wc_conv_desc* d, size_t* bytes) {
-  WC_CHECK_ARG(bytes != nullptr, "wc_conv_backward_weight_workspace_bytes: null output");
-  BwdLayout L{};
-  int rc = make_bwd_layout(d, &L);
-  if (rc) return rc;
-  *bytes = L.v_bytes + L.dm_bytes + L.du_bytes + L.acc_bytes;
+// Scratch of the bias gradient behind the weight gradient's: dy's column sums taken beside the product, or the workgroups' of a pass over dy
+int bias_scratch(const wc_conv_desc* d, const BwdLayout& L, size_t* bytes) {
+  int out[3], grid[3];
+  wc_conv_desc e = *d;
+  e.direct = e.stacked = e.row = e.whole_kernel = 0;
+  e.m = 2;
+  if (int rc = wc_conv_out_dims(&e, out, grid)) return rc;
+  *bytes = round256(std::max(L.sums_bytes, bias_part_bytes(dy_rows(d, out), d->K, d->dtype)));
   return WC_OK;
 }
 
-int wc_conv_backward_weight(const wc_conv_desc* d, const void* x, const void* dy, void* dw,
-                            const int64_t dw_strides[5], void* workspace, size_t workspace_bytes, void* stream) {
+// dw and, where to.db is not null, db
+int backward_weight(const wc_conv_desc* d, const void* x, const void* dy, GradOut to, void* workspace, size_t workspace_bytes, void* stream) {
   BwdLayout L{};
   int rc = make_bwd_layout(d, &L);
   if (rc) return rc;
-  WC_CHECK_ARG(x && dy && dw && dw_strides, "wc_conv_backward_weight: null pointer");
+  WC_CHECK_ARG(x && dy && to.dw, "wc_conv_backward_weight: null pointer");
   if (!workspace) return fail(WC_ERR_WORKSPACE, "wc_conv_backward_weight: null workspace");
-  const size_t need = L.v_bytes + L.dm_bytes + L.du_bytes + L.acc_bytes;
+  size_t bias_bytes = 0;
+  if (to.db && (rc = bias_scratch(d, L, &bias_bytes))) return rc;
+  const size_t need = to.db ? round256(weight_bytes(L)) + bias_bytes : weight_bytes(L);
   if (workspace_bytes < need)
     return fail(WC_ERR_WORKSPACE, "wc_conv_backward_weight: workspace of %zu bytes, %zu needed", workspace_bytes, need);
   if ((reinterpret_cast<uintptr_t>(workspace) & 255) != 0)
     return fail(WC_ERR_WORKSPACE, "wc_conv_backward_weight: workspace must be 256-byte aligned");
+  const int64_t* const dw_strides = to.s;
+  to.db_part = to.db ? reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + round256(weight_bytes(L))) : nullptr;
+  // the bias gradient of paths whose kernels do not have dy's rows in LDS
+  auto bias_alone = [&]() -> int {
+    int out[3], grid[3];
+    wc_conv_desc e = *d;
+    e.direct = e.stacked = e.row = e.whole_kernel = 0;
+    e.m = 2;
+    if (int r = wc_conv_out_dims(&e, out, grid)) return r;
+    return bias_sums(dy, to.db, dy_rows(d, out), d->K, d->dtype, to.db_f32, to.db_part, stream);
+  };
   hipStream_t s = as_stream(stream);
   unsigned char* ws = static_cast<unsigned char*>(workspace);
   void* V = ws;
@@ -452,23 +473,28 @@ int wc_conv_backward_weight(const wc_conv_desc* d, const void* x, const void* dy
   const size_t y_image = (size_t)L.out[0] * L.out[1] * L.out[2] * d->K * L.es;
   const int taps = d->kernel[0] * d->kernel[1] * d->kernel[2];
 
-  if (L.taps) return taps_gradient(d, L.out, x, dy, dw, dw_strides, dU, stream);
+  if (L.taps) return taps_gradient(d, L.out, x, dy, to, dU, stream);
+  bool summed = false;                              // dy's column sums taken beside the product
   if (L.one_tap) {
     const long long P = L.tiles_per_image * d->N;
-    rc = batched_gemm_tn(dy, x, dU, 1, P, d->K, d->C, d->K, d->C, d->C, L.S, L.Pq, false, d->dtype, stream);
+    rc = batched_gemm_tn(dy, x, dU, 1, P, d->K, d->C, d->K, d->C, d->C, L.S, L.Pq, false, d->dtype, stream, to.db_part, &summed);
     if (rc) return rc;
   }
   if (L.gathered) {
     rc = gemm_tn_conv(dy, x, dU, d->N, d->in[1], d->in[2], d->C, d->K, d->kernel[1], d->kernel[2], d->stride, d->pad[1],
-                      d->pad[2], L.out[1], L.out[2], L.S, L.Pq, d->dtype, stream);
+                      d->pad[2], L.out[1], L.out[2], L.S, L.Pq, d->dtype, stream, to.db_part, &summed);
     if (rc) return rc;
   }
+  if (to.db && !summed && (rc = bias_alone())) return rc;
   if (L.one_tap || L.gathered) {
     const long long n = (long long)d->K * d->C, total4 = (long long)taps * n / 4;
     dispatch_dtype(d->dtype, [&](auto t) {
       using TT = decltype(t);
-      hipLaunchKernelGGL(sum_parts_store_kernel<TT>, dim3((unsigned)ceil_div_ll(total4, 64)), dim3(256), 0, s, dU, static_cast<TT*>(dw), L.S, n, total4,
-                         (long long)dw_strides[0], (long long)dw_strides[1], (long long)dw_strides[3], (long long)dw_strides[4], d->C, d->kernel[2]);
+      const int blocks = (int)ceil_div_ll(total4, 64);
+      const ColumnSums sums = {to.db_part, to.db, tn_sum_rows(L.one_tap ? 1 : taps, d->K, d->C, L.S), tn_sum_width(d->K, d->C), d->K, to.db_f32};
+      hipLaunchKernelGGL(sum_parts_store_kernel<TT>, dim3((unsigned)(blocks + (summed ? ceil_div(d->K, 16) : 0))), dim3(256), 0, s, dU, to.dw, L.S, n, total4,
+                         (long long)dw_strides[0], (long long)dw_strides[1], (long long)dw_strides[3], (long long)dw_strides[4], d->C, d->kernel[2],
+                         to.dw_f32, blocks, sums);
       return 0;
     });
     WC_CHECK_LAUNCH("sum_parts_store_kernel");
@@ -544,13 +570,53 @@ int wc_conv_backward_weight(const wc_conv_desc* d, const void* x, const void* dy
   dispatch_dtype(d->dtype, [&](auto t) {
     using TT = decltype(t);
     hipLaunchKernelGGL(grad_filter_store_kernel<TT>, dim3((unsigned)ceil_div_ll(total, 256)), dim3(256), 0, s, acc,
-                       static_cast<TT*>(dw), (long long)dw_strides[0], (long long)dw_strides[1],
+                       to.dw, to.dw_f32, (long long)dw_strides[0], (long long)dw_strides[1],
                        (long long)dw_strides[2], (long long)dw_strides[3], (long long)dw_strides[4], d->K, d->C,
                        d->kernel[0], d->kernel[1], d->kernel[2], total);
     return 0;
   });
   WC_CHECK_LAUNCH("grad_filter_store_kernel");
   return WC_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int wc_conv_backward_weight_workspace_bytes(const wc_conv_desc* d, size_t* bytes) {
+  WC_CHECK_ARG(bytes != nullptr, "wc_conv_backward_weight_workspace_bytes: null output");
+  BwdLayout L{};
+  int rc = make_bwd_layout(d, &L);
+  if (rc) return rc;
+  *bytes = weight_bytes(L);
+  return WC_OK;
+}
+
+int wc_conv_backward_weight(const wc_conv_desc* d, const void* x, const void* dy, void* dw,
+                            const int64_t dw_strides[5], void* workspace, size_t workspace_bytes, void* stream) {
+  WC_CHECK_ARG(dw && dw_strides, "wc_conv_backward_weight: null pointer");
+  return backward_weight(d, x, dy, GradOut{dw, {dw_strides[0], dw_strides[1], dw_strides[2], dw_strides[3], dw_strides[4]}, false, nullptr, false, nullptr},
+                         workspace, workspace_bytes, stream);
+}
+
+int wc_conv_backward_parameters_workspace_bytes(const wc_conv_desc* d, size_t* bytes) {
+  WC_CHECK_ARG(bytes != nullptr, "wc_conv_backward_parameters_workspace_bytes: null output");
+  BwdLayout L{};
+  int rc = make_bwd_layout(d, &L);
+  if (rc) return rc;
+  size_t bias = 0;
+  if ((rc = bias_scratch(d, L, &bias))) return rc;
+  *bytes = round256(weight_bytes(L)) + bias;
+  return WC_OK;
+}
+
+int wc_conv_backward_parameters(const wc_conv_desc* d, const void* x, const void* dy, void* dw, const int64_t dw_strides[5], int dw_dtype,
+                                void* db, int db_dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  WC_CHECK_ARG(d && dw && dw_strides, "wc_conv_backward_parameters: null pointer");
+  WC_CHECK_ARG((dw_dtype == d->dtype || dw_dtype == WC_F32) && (!db || db_dtype == d->dtype || db_dtype == WC_F32),
+               "wc_conv_backward_parameters: gradients of dtypes %d and %d for operands of dtype %d: that type or fp32", dw_dtype, db_dtype, d->dtype);
+  return backward_weight(d, x, dy, GradOut{dw, {dw_strides[0], dw_strides[1], dw_strides[2], dw_strides[3], dw_strides[4]}, dw_dtype == WC_F32,
+                                           db, db_dtype == WC_F32, nullptr}, workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"

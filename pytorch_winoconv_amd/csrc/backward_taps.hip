@@ -19,6 +19,7 @@
 // 32.5 | 39.  Beside its steps a launch moves its partial sums, 59 MB each way where 200 workgroups share 0.6 MB of dw.  Variants that were
 // slower: dy turned channel by channel in LDS and read 16 bytes at a time 424 us, four wavefronts of all nine taps 439; operands
 // read a group ahead changed nothing (377).  Operands are exact, sums fp32.
+#include "column_sums.h"
 #include "lds_dma.h"
 #include "wc_transform.h"
 
@@ -52,6 +53,7 @@ template <int KG> constexpr int kDyPitch = KG * 128 + 64;
 
 struct TapsArgs {
   const void* x; const void* dy; float* part;
+  float* bias;                     // column sums of dy, a row of 64 KG per workgroup in order (part, depth tap, input and output channels); null: none
   int D, H, W, C, K;               // x (N, D, H, W, C), dy (N, oD, oH, oW, K)
   int oD, oH, oW, pd, ph, pw;
   long long x_elems, dy_elems;
@@ -117,6 +119,7 @@ void taps_kernel(TapsArgs a) {
   const int ct = tile % a.n_c; tile /= a.n_c;
   const int kt = tile % a.n_k, kd = tile / a.n_k;
   const int k0 = kt * 64 * KG, c0 = ct * 64;
+  const int holder = kd * a.n_c + ct;               // of those with this part's rows of dy
   const int q0 = part * a.part_steps * kStep, q_end = min(a.total, q0 + a.part_steps * kStep);
   const int steps = (q_end - q0 + kStep - 1) / kStep;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -210,11 +213,19 @@ void taps_kernel(TapsArgs a) {
   const int x_lane = frag_row * XP + cb * 64 + frag_col, d_lane = frag_row * DP + kg * 128 + frag_col;
 
   int slot = 0;                                     // ring row of the step's first position
+  const int turns = 6 * KG * a.n_kd * a.n_c;
+  int turn = wave + 6 * KG * holder;                    // steps until this wavefront adds one's rows of dy up
+  float colsum[2] = {0.f, 0.f};
   for (int step = 0; step < steps; ++step) {
     const bool more = step + 1 < steps;
     if (more) load(step + 1);
     const int row = slot + kh * a.Wp;
     const unsigned char* const db = lds + (step & 1) * kStep * DP + d_lane;
+    if (turn == 0) {
+      if (a.bias) add_rows<T, KG * 64, DP, false>(lds + (step & 1) * kStep * DP, kStep, lane, colsum);
+      turn = turns;
+    }
+    --turn;
 #pragma unroll
     for (int kk = 0; kk < kStep / 16; ++kk) {
       const int r = row + kk * 16 >= a.ring ? row + kk * 16 - a.ring : row + kk * 16;
@@ -231,6 +242,7 @@ void taps_kernel(TapsArgs a) {
     __syncthreads();
   }
 
+  if (a.bias) store_sums<6 * KG, KG * 64>(colsum, reinterpret_cast<float*>(lds), wave, lane, a.bias + (((long long)part * a.n_kd * a.n_c + holder) * a.n_k + kt) * 64 * KG);
   taps_store(acc, a.part + (long long)wg * taps_tile_floats<KG>() + wave * 24 * 256 + lane * 4);
 }
 
@@ -256,6 +268,7 @@ void taps_dma_kernel(TapsArgs a) {
   const int ct = tile % a.n_c; tile /= a.n_c;
   const int kt = tile % a.n_k, kd = tile / a.n_k;
   const int k0 = kt * 64 * KG, c0 = ct * 64;
+  const int holder = kd * a.n_c + ct;               // of those with this part's rows of dy
   const int q0 = part * a.part_steps * kStep, q_end = min(a.total, q0 + a.part_steps * kStep);
   const int steps = (q_end - q0 + kStep - 1) / kStep;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -328,6 +341,9 @@ void taps_dma_kernel(TapsArgs a) {
   const int d_lane0 = frag_row * DP + ((kg * 128 + frag_col) ^ d_swap), d_lane1 = frag_row * DP + ((kg * 128 + 64 + frag_col) ^ d_swap);
 
   int slot = 0, to = a.halo + 2 * kStep, stage = 0, filler = 0;      // ring rows of the step's first position and of the loads two steps on
+  const int turns = NW * a.n_kd * a.n_c;
+  int turn = wave + NW * holder;                    // steps until this wavefront adds one's rows of dy up
+  float colsum[2] = {0.f, 0.f};
   for (int step = 0; step < steps; ++step) {
     // this step's loads are there (the next step's, at least two per wavefront, may be on their way), for all, and all are done
     // with the last step's rows and the table's
@@ -339,6 +355,11 @@ void taps_dma_kernel(TapsArgs a) {
     filler = filler == NW / 2 - 1 ? 0 : filler + 1;
     const int row = slot + kh * a.Wp;
     const unsigned char* const db = lds + stage * DY_STAGE;
+    if (turn == 0) {
+      if (a.bias) add_rows<T, KG * 64, DP, true>(lds + stage * DY_STAGE, kStep, lane, colsum);
+      turn = turns;
+    }
+    --turn;
 #pragma unroll
     for (int kk = 0; kk < kStep / 16; ++kk) {
       const int r = row + kk * 16 >= a.ring ? row + kk * 16 - a.ring : row + kk * 16;
@@ -350,6 +371,7 @@ void taps_dma_kernel(TapsArgs a) {
     if (to >= a.ring) to -= a.ring;
     stage = stage == 2 ? 0 : stage + 1;
   }
+  if (a.bias) store_sums<6 * KG, KG * 64>(colsum, reinterpret_cast<float*>(lds), wave, lane, a.bias + (((long long)part * a.n_kd * a.n_c + holder) * a.n_k + kt) * 64 * KG);
   taps_store(acc, a.part + (long long)wg * taps_tile_floats<KG>() + wave * 24 * 256 + lane * 4);
 }
 
@@ -359,13 +381,17 @@ struct TapsSumArgs {
   const float* part;
   void* dw;
   long long s[5];
-  int S, tiles, n_k, n_c, K, C;
+  int S, tiles, n_k, n_c, K, C, f32;
+  int blocks;                      // beyond them: the bias gradient's
+  ColumnSums bias;
 };
 template <typename T, int KG>
 __global__ __launch_bounds__(256) void taps_sum_kernel(TapsSumArgs a) {
   __shared__ f32x4 sums[3][64];
+  static_assert(sizeof(sums) >= 256 * 4, "sum_columns takes as much");
   const int lane = threadIdx.x & 63, group = threadIdx.x >> 6;
   int b = blockIdx.x;
+  if (b >= a.blocks) return sum_columns<T>(a.bias, b - a.blocks, reinterpret_cast<float*>(sums));
   const int q = b & 3, i = (b >> 2) & 1, kw = (b >> 3) % 3, wave = b / 24 % (6 * KG);
   int tile = b / (24 * 6 * KG);
   const float* src = a.part + (long long)b * 256 + lane * 4;
@@ -382,10 +408,10 @@ __global__ __launch_bounds__(256) void taps_sum_kernel(TapsSumArgs a) {
   const int kt = tile % a.n_k, kd = tile / a.n_k;
   const int k = kt * 64 * KG + wave / 6 * 64 + i * 32 + (lane & 31), c = ct * 64 + (wave & 1) * 32 + 8 * q + 4 * (lane >> 5);
   if (k >= a.K) return;
-  T* const dst = static_cast<T*>(a.dw) + k * a.s[0] + c * a.s[1] + kd * a.s[2] + wave % 6 / 2 * a.s[3] + kw * a.s[4];
+  const long long dst = k * a.s[0] + c * a.s[1] + kd * a.s[2] + wave % 6 / 2 * a.s[3] + kw * a.s[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e)
-    if (c + e < a.C) dst[e * a.s[1]] = static_cast<T>(sum[e]);
+    if (c + e < a.C) store_as<T>(a.dw, dst + e * a.s[1], sum[e], a.f32);
 }
 
 struct TapsPlan { int kg, halo, ring, total, steps, parts, part_steps, tiles; };
@@ -428,10 +454,9 @@ bool taps_plan(const wc_conv_desc* d, const int out[3], TapsPlan* p) {
 }
 
 template <typename T, int KG>
-int launch_taps(const wc_conv_desc* d, const int out[3], const TapsPlan& p, const void* x, const void* dy, void* dw,
-                const int64_t s[5], float* part, void* stream) {
+int launch_taps(const wc_conv_desc* d, const int out[3], const TapsPlan& p, const void* x, const void* dy, const GradOut& to, float* part, void* stream) {
   TapsArgs a;
-  a.x = x; a.dy = dy; a.part = part;
+  a.x = x; a.dy = dy; a.part = part; a.bias = to.db ? to.db_part : nullptr;
   a.D = d->in[0]; a.H = d->in[1]; a.W = d->in[2]; a.C = d->C; a.K = d->K;
   a.oD = out[0]; a.oH = out[1]; a.oW = out[2]; a.pd = d->pad[0]; a.ph = d->pad[1]; a.pw = d->pad[2];
   a.x_elems = (long long)d->N * a.D * a.H * a.W * a.C; a.dy_elems = (long long)d->N * a.oD * a.oH * a.oW * a.K;
@@ -452,10 +477,12 @@ int launch_taps(const wc_conv_desc* d, const int out[3], const TapsPlan& p, cons
   hipLaunchKernelGGL(fn, dim3((unsigned)(a.per_xcd * kXcds)), dim3(384 * KG), lds, as_stream(stream), a);
   WC_CHECK_LAUNCH("taps_kernel");
   TapsSumArgs b;
-  b.part = part; b.dw = dw;
-  for (int i = 0; i < 5; ++i) b.s[i] = s[i];
+  b.part = part; b.dw = to.dw; b.f32 = to.dw_f32;
+  for (int i = 0; i < 5; ++i) b.s[i] = to.s[i];
   b.S = p.parts; b.tiles = p.tiles; b.n_k = a.n_k; b.n_c = a.n_c; b.K = a.K; b.C = a.C;
-  hipLaunchKernelGGL((taps_sum_kernel<T, KG>), dim3((unsigned)(p.tiles * 144 * KG)), dim3(256), 0, as_stream(stream), b);
+  b.blocks = p.tiles * 144 * KG;
+  b.bias = {a.bias, to.db, p.parts * a.n_kd * a.n_c, a.n_k * 64 * KG, a.K, to.db_f32};
+  hipLaunchKernelGGL((taps_sum_kernel<T, KG>), dim3((unsigned)(b.blocks + (to.db ? ceil_div(a.K, 16) : 0))), dim3(256), 0, as_stream(stream), b);
   WC_CHECK_LAUNCH("taps_sum_kernel");
   return WC_OK;
 }
@@ -471,26 +498,26 @@ int launch_taps(const wc_conv_desc* d, const int out[3], const TapsPlan& p, cons
 // Channels that are no multiples of 8 go through registers (us, F(4,3) | taps: 100 -> 150, N=64 28x28 53 | 56; against F(2,3) alone
 // still ahead: 50 -> 64, N=32 56x56 32 | 71; 3 -> 64, N=64 112x112 106 | 334).  Small problems are launches and latency: two of them
 // here, six there (512 -> 512, N=1 7x7 28 | 39 | 48).
-bool taps_gradient_fits(const wc_conv_desc* d, const int out[3], size_t* workspace_bytes) {
+bool taps_gradient_fits(const wc_conv_desc* d, const int out[3], size_t* workspace_bytes, size_t* bias_bytes) {
   TapsPlan p;
   if (test_gemm_config() == 20 || !taps_plan(d, out, &p)) return false;
   if (d->ndim == 2 && d->m == 4 && (long long)p.steps * p.tiles > (d->C % 8 == 0 && d->K % 8 == 0 ? 12000 : 2560)) {
     const long long padded = (long long)ceil_div(d->K, 64 * p.kg) * 64 * p.kg * ceil_div(d->C, 64) * 64;
     if (padded > 256 * 256 || padded * 5 > 8ll * d->C * d->K) return false;
   }
+  *bias_bytes = (size_t)p.parts * p.tiles * 64 * p.kg * 4;
   *workspace_bytes = (size_t)p.parts * p.tiles * (p.kg == 2 ? taps_tile_floats<2>() : taps_tile_floats<1>()) * 4;
   return true;
 }
 
-int taps_gradient(const wc_conv_desc* d, const int out[3], const void* x, const void* dy, void* dw,
-                  const int64_t dw_strides[5], float* part, void* stream) {
+int taps_gradient(const wc_conv_desc* d, const int out[3], const void* x, const void* dy, const GradOut& to, float* part, void* stream) {
   TapsPlan p;
   WC_CHECK_ARG(taps_plan(d, out, &p), "tap form of the weight gradient: 16-bit, 3x3 or 3x3x3, stride 1");
   return dispatch_dtype(d->dtype, [&](auto t) -> int {
     using T = decltype(t);
     if constexpr (sizeof(T) == 2) {
-      return p.kg == 2 ? launch_taps<T, 2>(d, out, p, x, dy, dw, dw_strides, part, stream)
-                       : launch_taps<T, 1>(d, out, p, x, dy, dw, dw_strides, part, stream);
+      return p.kg == 2 ? launch_taps<T, 2>(d, out, p, x, dy, to, part, stream)
+                       : launch_taps<T, 1>(d, out, p, x, dy, to, part, stream);
     }
     return fail(WC_ERR_UNSUPPORTED, "tap form of the weight gradient: 16-bit types");
   });

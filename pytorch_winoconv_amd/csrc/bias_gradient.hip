@@ -6,7 +6,7 @@
 // sums in a second kernel, all in a fixed order.  Measured, us, torch's sum | this: fp16 N=8 128 channels, 16x56x56 (103 MB)
 // 49 | 22 (4.7 TB/s), N=64 128 channels, 28x28 19 | 6.6, bf16 N=32 256 channels, 28x28 25 | 6.5, fp32 N=8 256 channels, 56x56
 // 24 | 7.8, N=1 512 channels, 7x7 (two launches) 5.8 | 5.6.
-#include "wc_common.h"
+#include "column_sums.h"
 
 #include <algorithm>
 
@@ -79,7 +79,7 @@ __global__ __launch_bounds__(kBiasThreads) void bias_rows_kernel(const T* __rest
 
 // db[k] = sum over the workgroups' rows; 16 channels a workgroup, 64 threads to a channel's sums
 template <typename T>
-__global__ __launch_bounds__(1024) void bias_parts_kernel(const float* __restrict__ part, T* __restrict__ db, int blocks, int K) {
+__global__ __launch_bounds__(1024) void bias_parts_kernel(const float* __restrict__ part, void* __restrict__ db, int blocks, int K, bool f32) {
   __shared__ float sums[64][16];
   const int c = threadIdx.x & 15, group = threadIdx.x >> 4, k = blockIdx.x * 16 + c;
   float s = 0.f;
@@ -93,10 +93,32 @@ __global__ __launch_bounds__(1024) void bias_parts_kernel(const float* __restric
     if (group < half) sums[group][c] += sums[group + half][c];
     __syncthreads();
   }
-  if (group == 0 && k < K) db[k] = static_cast<T>(sums[0][c]);
+  if (group == 0 && k < K) store_as<T>(db, k, sums[0][c], f32);
 }
 
 }  // namespace
+
+// (the number of workgroups is the larger where a thread reads 16 bytes)
+size_t bias_part_bytes(long long rows, int K, int dtype) {
+  return (size_t)std::max(bias_plan(rows, K, dtype, true).blocks, bias_plan(rows, K, dtype, false).blocks) * K * 4;
+}
+
+int bias_sums(const void* dy, void* db, long long rows, int K, int dtype, bool f32, float* part, void* stream) {
+  const BiasPlan p = bias_plan(rows, K, dtype, (reinterpret_cast<uintptr_t>(dy) & 15) == 0);
+  return dispatch_dtype(dtype, [&](auto t) -> int {
+    using T = decltype(t);
+    constexpr int FULL = 16 / sizeof(T);
+    auto fn = p.vec == FULL ? &bias_rows_kernel<T, FULL> : p.vec == 4 ? &bias_rows_kernel<T, 4> : p.vec == 2 ? &bias_rows_kernel<T, 2>
+                                                                                             : &bias_rows_kernel<T, 1>;
+    hipLaunchKernelGGL(fn, dim3((unsigned)p.blocks, (unsigned)p.col_tiles), dim3(kBiasThreads), 0, as_stream(stream),
+                       static_cast<const T*>(dy), part, rows, K, p.cols, p.groups, p.rows_per_block);
+    WC_CHECK_LAUNCH("bias_rows_kernel");
+    hipLaunchKernelGGL(bias_parts_kernel<T>, dim3((unsigned)ceil_div(K, 16)), dim3(1024), 0, as_stream(stream), part,
+                       db, p.blocks, K, f32);
+    WC_CHECK_LAUNCH("bias_parts_kernel");
+    return WC_OK;
+  });
+}
 
 }  // namespace wc
 
@@ -107,8 +129,7 @@ extern "C" {
 int wc_bias_gradient_workspace_bytes(long long rows, int K, int dtype, size_t* bytes) {
   WC_CHECK_ARG(bytes != nullptr, "wc_bias_gradient_workspace_bytes: null output");
   WC_CHECK_ARG(rows > 0 && K > 0 && (dtype == WC_F32 || dtype == WC_F16 || dtype == WC_BF16), "rows %lld, K %d, dtype %d", rows, K, dtype);
-  // (the number of workgroups is the larger where a thread reads 16 bytes)
-  *bytes = (size_t)std::max(bias_plan(rows, K, dtype, true).blocks, bias_plan(rows, K, dtype, false).blocks) * K * 4;
+  *bytes = bias_part_bytes(rows, K, dtype);
   return WC_OK;
 }
 
@@ -119,21 +140,7 @@ int wc_bias_gradient(const void* dy, void* db, long long rows, int K, int dtype,
   if (!workspace || workspace_bytes < need)
     return fail(WC_ERR_WORKSPACE, "wc_bias_gradient: workspace of %zu bytes, %zu needed", workspace ? workspace_bytes : (size_t)0, need);
   if ((reinterpret_cast<uintptr_t>(workspace) & 15) != 0) return fail(WC_ERR_WORKSPACE, "wc_bias_gradient: workspace must be 16-byte aligned");
-  const BiasPlan p = bias_plan(rows, K, dtype, (reinterpret_cast<uintptr_t>(dy) & 15) == 0);
-  float* const part = static_cast<float*>(workspace);
-  return dispatch_dtype(dtype, [&](auto t) -> int {
-    using T = decltype(t);
-    constexpr int FULL = 16 / sizeof(T);
-    auto fn = p.vec == FULL ? &bias_rows_kernel<T, FULL> : p.vec == 4 ? &bias_rows_kernel<T, 4> : p.vec == 2 ? &bias_rows_kernel<T, 2>
-                                                                                             : &bias_rows_kernel<T, 1>;
-    hipLaunchKernelGGL(fn, dim3((unsigned)p.blocks, (unsigned)p.col_tiles), dim3(kBiasThreads), 0, as_stream(stream),
-                       static_cast<const T*>(dy), part, rows, K, p.cols, p.groups, p.rows_per_block);
-    WC_CHECK_LAUNCH("bias_rows_kernel");
-    hipLaunchKernelGGL(bias_parts_kernel<T>, dim3((unsigned)ceil_div(K, 16)), dim3(1024), 0, as_stream(stream), part,
-                       static_cast<T*>(db), p.blocks, K);
-    WC_CHECK_LAUNCH("bias_parts_kernel");
-    return WC_OK;
-  });
+  return bias_sums(dy, db, rows, K, dtype, false, static_cast<float*>(workspace), stream);
 }
 
 }  // extern "C"

@@ -18,6 +18,7 @@
 // what fills the chip); the caller adds the parts.  Workgroup = 4 wavefronts (2 x 2), each owning
 // W x W blocks of 32 x 32.  V feeds the MFMA "A" side, so a lane ends up with 4 consecutive
 // columns of D and stores them as one 16-byte write.
+#include "column_sums.h"
 #include "lds_dma.h"
 #include "split_bf16.h"
 #include "wc_transform.h"
@@ -55,6 +56,8 @@ struct GemmTnArgs {
   // holds; 0: the parts of a tap, which do not meet at the same lines (us, fp16, stride 2, taps | parts: N=32 128 -> 128, 112x112, 128 MB
   // in all, 60 | 90, N=64 64 -> 64, 56x56, 32 MB 38 | 44; N=16 96 -> 96, 50x50, 10 MB 27.5 | 26.5, N=8 128 -> 128, 56x56, 8 MB 27 | 23)
   int n_taps;
+  float* sums;               // column sums of A, a row of tiles_a times the tile's columns per (s, t, tile of B); null: none
+  int T;
 };
 
 __device__ __forceinline__ floatx16 mfma16(short8v a, short8v b, floatx16 c, half_t) {
@@ -313,6 +316,9 @@ __global__ __launch_bounds__(256, 2) void gemm_tn_dma_kernel(GemmTnArgs g) {
 #pragma unroll
   for (int k = 0; k < kTnStages - 1; ++k)
     if (k < nk) issue(k);
+  const int holder = t * g.tiles_b + tb, turns = 4 * g.T * g.tiles_b;      // holders of these rows of A
+  int turn = wave + 4 * holder;                    // stages until this wavefront adds one's rows up
+  float colsum[2] = {0.f, 0.f};
   for (int kt = 0; kt < nk; ++kt) {
     if (kt + 2 < nk) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(4 * L) : "memory");
     else if (kt + 1 < nk) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(2 * L) : "memory");
@@ -323,6 +329,11 @@ __global__ __launch_bounds__(256, 2) void gemm_tn_dma_kernel(GemmTnArgs g) {
       if ((kt & 1) == 0 && kt + 4 < nk && wave == ((kt >> 1) & 3)) fill((kt >> 1) + 2);
     }
     const unsigned char* const st = lds_raw + (kt % kTnStages) * STAGE;
+    if (turn == 0) {
+      if (g.sums) add_rows<T, BT, PITCH, true>(st, kTnRows, lane, colsum);
+      turn = turns;
+    }
+    --turn;
     typedef short4v __attribute__((address_space(3))) * LdsVec;
     auto read = [&](const unsigned char* src) {
       const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsVec)(src));
@@ -343,6 +354,7 @@ __global__ __launch_bounds__(256, 2) void gemm_tn_dma_kernel(GemmTnArgs g) {
     }
   }
 
+  if (g.sums) store_sums<4, BT>(colsum, reinterpret_cast<float*>(lds_raw), wave, lane, g.sums + (((long long)s * g.T * g.tiles_b + holder) * g.tiles_a + ta) * BT);
   float* const Dt = g.D + ((long long)t * g.S + s) * g.na * g.ldd;
 #pragma unroll
   for (int i = 0; i < W; ++i) {
@@ -527,7 +539,7 @@ __global__ __launch_bounds__(256, 2) void gemm_tn_split_kernel(GemmTnArgs g) {
 }
 
 template <typename T, int W, bool GATHER = false>
-int launch_tn(GemmTnArgs g, int T_, bool split, void* stream) {
+int launch_tn(GemmTnArgs g, int T_, bool split, void* stream, bool* summed) {
   constexpr int BT = 64 * W;
   constexpr int BK = sizeof(T) == 2 ? 64 : 16;     // reduction rows per stage (64: measured 5 % faster than 32)
   constexpr size_t lds = (size_t)2 * 2 * BK * (BT + 32 / sizeof(T)) * sizeof(T);
@@ -543,6 +555,7 @@ int launch_tn(GemmTnArgs g, int T_, bool split, void* stream) {
     const long long reach = (g.Pq + 256ll) * std::max(g.lda, GATHER ? 0 : g.ldb) * 2;
     if (((reinterpret_cast<uintptr_t>(g.A) | reinterpret_cast<uintptr_t>(g.B)) & 15) == 0 && reach < (1ll << 31) &&
         images * g.H * g.W * g.ldb * 2 < (1ll << 31) && g.P < (1ll << 31)) {
+      if (summed) *summed = g.sums != nullptr;
       const auto fn = &gemm_tn_dma_kernel<T, W, GATHER>;
       constexpr int dma_lds = tn_dma_lds<W>();
       if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), dma_lds)) return rc;
@@ -569,8 +582,11 @@ int launch_tn(GemmTnArgs g, int T_, bool split, void* stream) {
 
 }  // namespace
 
+int tn_sum_width(int na, int nb) { return ceil_div(na, na > 64 && nb > 64 ? 128 : 64) * (na > 64 && nb > 64 ? 128 : 64); }
+int tn_sum_rows(int T_, int na, int nb, int S) { return S * T_ * ceil_div(nb, na > 64 && nb > 64 ? 128 : 64); }
+
 int batched_gemm_tn(const void* A, const void* B, float* D, int T_, long long P, int lda, int ldb, int na, int nb,
-                    int ldd, int S, int Pq, bool split, int dtype, void* stream) {
+                    int ldd, int S, int Pq, bool split, int dtype, void* stream, float* a_sums, bool* summed) {
   WC_CHECK_ARG(A && B && D, "batched_gemm_tn: null pointer");
   WC_CHECK_ARG(T_ > 0 && P > 0 && na > 0 && nb > 0 && S > 0 && Pq > 0, "batched_gemm_tn: empty problem");
   WC_CHECK_ARG(lda % 8 == 0 && ldb % 8 == 0 && ldd % 4 == 0 && lda >= na && ldb >= nb && ldd >= nb,
@@ -582,10 +598,11 @@ int batched_gemm_tn(const void* A, const void* B, float* D, int T_, long long P,
   g.S = S; g.Pq = Pq;
   g.H = g.W = g.oH = g.oW = g.conv_stride = g.pad_h = g.pad_w = g.kw = 0;
   g.div_per = g.div_oW = make_fast_div(1); g.b_elems = 0; g.n_taps = 0;
+  g.sums = a_sums; g.T = T_;
   const bool big = na > 64 && nb > 64;
   return dispatch_dtype(dtype, [&](auto t) {
     using TT = decltype(t);
-    return big ? launch_tn<TT, 2>(g, T_, split, stream) : launch_tn<TT, 1>(g, T_, split, stream);
+    return big ? launch_tn<TT, 2>(g, T_, split, stream, summed) : launch_tn<TT, 1>(g, T_, split, stream, summed);
   });
 }
 
@@ -593,7 +610,7 @@ int batched_gemm_tn(const void* A, const void* B, float* D, int T_, long long P,
 // x[b][stride oy + ky - pad_h][stride ox + kx - pad_w][0..C): the weight gradient taken directly, one batch per tap,
 // x gathered row by row (zeros outside the image).  dy (N oH oW, K) and x (N, H, W, C) as they lie in memory.
 int gemm_tn_conv(const void* dy, const void* x, float* D, int N, int H, int W, int C, int K, int kh, int kw, int stride,
-                 int pad_h, int pad_w, int oH, int oW, int S, int Pq, int dtype, void* stream) {
+                 int pad_h, int pad_w, int oH, int oW, int S, int Pq, int dtype, void* stream, float* dy_sums, bool* summed) {
   WC_CHECK_ARG(dy && x && D, "gemm_tn_conv: null pointer");
   WC_CHECK_ARG(C % 8 == 0 && K % 8 == 0 && S > 0 && Pq > 0, "gemm_tn_conv: C %d, K %d (multiples of 8)", C, K);
   const long long P = (long long)N * oH * oW;
@@ -607,10 +624,11 @@ int gemm_tn_conv(const void* dy, const void* x, float* D, int N, int H, int W, i
   g.b_elems = (long long)N * H * W * C; 
   const long long bytes = (g.b_elems + P * K) * (dtype == WC_F32 ? 4 : 2);
   g.n_taps = bytes > (16 << 20) ? kh * kw : 0;
+  g.sums = dy_sums; g.T = kh * kw;
   const bool big = K > 64 && C > 64;
   return dispatch_dtype(dtype, [&](auto t) {
     using TT = decltype(t);
-    return big ? launch_tn<TT, 2, true>(g, kh * kw, false, stream) : launch_tn<TT, 1, true>(g, kh * kw, false, stream);
+    return big ? launch_tn<TT, 2, true>(g, kh * kw, false, stream, summed) : launch_tn<TT, 1, true>(g, kh * kw, false, stream, summed);
   });
 }
 

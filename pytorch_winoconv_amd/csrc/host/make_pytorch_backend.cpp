@@ -18,6 +18,7 @@
 #include <stdexcept>
 #include <string>
 #include <thread>
+#include <tuple>
 #include <vector>
 
 #include "../../../include/winoconv.h"
@@ -530,7 +531,9 @@ at::Tensor transform_filter(at::Tensor w, std::vector<int64_t> x_shape, py::obje
 
 // ---- gradients (the reference has no backward pass: src/back/utils.cu:15-24): engine.py's conv_backward_weight with the
 // form of the plan left to the library, and bias_gradient
-at::Tensor conv_backward_weight(at::Tensor x, at::Tensor dy, std::vector<int64_t> w_shape, py::object stride, py::object padding, int m) {
+// (dw, db) with `bias`, each of type fp32 or x's
+std::pair<at::Tensor, at::Tensor> parameter_gradients(at::Tensor x, at::Tensor dy, std::vector<int64_t> w_shape, py::object stride,
+                                                      py::object padding, int m, bool bias, at::ScalarType w_type, at::ScalarType b_type) {
   const int nd = (int)x.dim() - 2;
   require_gpu(x, "conv_backward_weight");
   require_gpu(dy, "conv_backward_weight");
@@ -564,17 +567,36 @@ at::Tensor conv_backward_weight(at::Tensor x, at::Tensor dy, std::vector<int64_t
   std::vector<int64_t> ys{x.size(0), w_shape[0]};
   for (int a = 3 - nd; a < 3; ++a) ys.push_back(out[a]);
   if (dy.sizes().vec() != ys) throw std::invalid_argument("dy has shape " + shape_str(dy.sizes()) + ", the convolution gives " + shape_str(ys));
-  at::Tensor dw = at::empty(w_shape, x.options());
+  at::Tensor dw = at::empty(w_shape, x.options().dtype(w_type)), db;
+  if (bias) db = at::empty({w_shape[0]}, x.options().dtype(b_type));
+  const bool plain = !bias && w_type == x.scalar_type();
   const at::Tensor xl = last_view(x), dyl = last_view(dy);
   size_t bytes = 0;
-  check(wc_conv_backward_weight_workspace_bytes(&d, &bytes));
+  check(plain ? wc_conv_backward_weight_workspace_bytes(&d, &bytes) : wc_conv_backward_parameters_workspace_bytes(&d, &bytes));
   void* stream = stream_of(x);
   at::Tensor ws = workspace_for(x, bytes, stream);
   int64_t s[5] = {dw.stride(0), dw.stride(1), 0, 0, 0};
   for (int a = 0; a < nd; ++a) s[5 - nd + a] = dw.stride(2 + a);
-  py::gil_scoped_release nogil;
-  check(wc_conv_backward_weight(&d, xl.data_ptr(), dyl.data_ptr(), dw.data_ptr(), s, ws.data_ptr(), bytes, stream));
-  return dw;
+  {
+    py::gil_scoped_release nogil;
+    check(plain ? wc_conv_backward_weight(&d, xl.data_ptr(), dyl.data_ptr(), dw.data_ptr(), s, ws.data_ptr(), bytes, stream)
+                : wc_conv_backward_parameters(&d, xl.data_ptr(), dyl.data_ptr(), dw.data_ptr(), s, dtype_of(dw), bias ? db.data_ptr() : nullptr,
+                                              bias ? dtype_of(db) : WC_F32, ws.data_ptr(), bytes, stream));
+  }
+  return {dw, db};
+}
+
+at::Tensor conv_backward_weight(at::Tensor x, at::Tensor dy, std::vector<int64_t> w_shape, py::object stride, py::object padding, int m) {
+  return parameter_gradients(x, dy, w_shape, stride, padding, m, false, x.scalar_type(), x.scalar_type()).first;
+}
+
+py::object or_none(const at::Tensor& t) { return t.defined() ? py::cast(t) : py::none(); }
+
+py::tuple conv_backward_parameters(at::Tensor x, at::Tensor dy, std::vector<int64_t> w_shape, py::object stride, py::object padding, int m,
+                                   bool need_db, py::object w_type, py::object b_type) {
+  const auto g = parameter_gradients(x, dy, w_shape, stride, padding, m, need_db, torch::python::detail::py_object_to_dtype(w_type),
+                                     torch::python::detail::py_object_to_dtype(b_type));
+  return py::make_tuple(g.first, or_none(g.second));
 }
 
 at::Tensor bias_gradient(at::Tensor dy) {
@@ -621,18 +643,17 @@ py::tuple conv_backward(at::Tensor x, at::Tensor w, at::Tensor dy, py::object st
     }
   }
   if (need_dw) {
-    dw = conv_backward_weight(x, dy, w.sizes().vec(), stride, padding, m);
-    if (!w_type.is_none()) dw = dw.to(torch::python::detail::py_object_to_dtype(w_type));
+    std::vector<int64_t> last{0};
+    for (int a = 0; a < nd; ++a) last.push_back(2 + a);
+    last.push_back(1);
+    auto type = [&](const py::object& t) { return t.is_none() ? x.scalar_type() : torch::python::detail::py_object_to_dtype(t); };
+    auto own = [&](at::ScalarType t) { return t == at::kFloat ? t : x.scalar_type(); };      // any other type: a cast of its own
+    const at::ScalarType wt = type(w_type), bt = type(b_type);
+    std::tie(dw, db) = parameter_gradients(x, dy, w.sizes().vec(), stride, padding, m, need_db && dy.permute(last).is_contiguous(), own(wt), own(bt));
+    dw = dw.to(wt);
+    if (db.defined()) db = db.to(bt);
   }
-  std::vector<int64_t> last{0};
-  for (int a = 0; a < nd; ++a) last.push_back(2 + a);
-  last.push_back(1);
-  if (need_db && need_dw && dy.permute(last).is_contiguous()) {
-    db = bias_gradient(dy);
-    if (!b_type.is_none()) db = db.to(torch::python::detail::py_object_to_dtype(b_type));
-  }
-  auto out = [](const at::Tensor& t) -> py::object { return t.defined() ? py::cast(t) : py::none(); };
-  return py::make_tuple(out(dx), out(dw), out(db));
+  return py::make_tuple(or_none(dx), or_none(dw), or_none(db));
 }
 
 // The reference's native entry point (pybind/extern.hpp:7-9): VALID convolution.  The four scratch tensors
@@ -674,6 +695,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("channels_first_out") = false, py::arg("direct") = py::none(), py::arg("row") = false);
   m.def("conv_backward_weight", &conv_backward_weight, py::arg("x"), py::arg("dy"), py::arg("w_shape"), py::arg("stride") = 1,
         py::arg("padding") = 0, py::arg("m") = 2);
+  m.def("conv_backward_parameters", &conv_backward_parameters, py::arg("x"), py::arg("dy"), py::arg("w_shape"), py::arg("stride"), py::arg("padding"),
+        py::arg("m"), py::arg("need_db"), py::arg("w_type"), py::arg("b_type"));
   m.def("conv_backward", &conv_backward, py::arg("x"), py::arg("w"), py::arg("dy"), py::arg("stride"), py::arg("padding"), py::arg("m"),
         py::arg("need_dx"), py::arg("need_dw"), py::arg("need_db"), py::arg("w_type") = py::none(), py::arg("b_type") = py::none());
   m.def("conv_backward_input_flipped", &conv_backward_input_flipped, py::arg("dy"), py::arg("w"), py::arg("padding"), py::arg("m"));

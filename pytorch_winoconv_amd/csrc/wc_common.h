@@ -231,21 +231,34 @@ int input_filter_transform(const wc_conv_desc* d, const wc_plan* plan, const voi
 int grad_filter_transform(const wc_conv_desc* d, const wc_plan* plan, const float* dU, float* acc, int ldc, int S,
                           bool first, void* stream);
 
+// What a weight gradient writes: dw through element strides and, where db is not null, the bias gradient, each of the operands' type
+// or fp32.  db_part: scratch for the column sums of dy that kernels with dy in LDS take on the way (column_sums.h)
+struct GradOut {
+  void* dw; int64_t s[5]; bool dw_f32;
+  void* db; bool db_f32; float* db_part;
+};
+
 // D[t][s] (na x nb, fp32, row stride ldd) = sum over rows p in [s Pq, (s + 1) Pq) of
 // A[t][p][.] (x) B[t][p][.], operands (T, P, ld) of storage type `dtype`; split: fp32 in
 // three bf16 parts (gemm_tn.hip).
 int batched_gemm_tn(const void* A, const void* B, float* D, int T, long long P, int lda, int ldb, int na, int nb,
-                    int ldd, int S, int Pq, bool split, int dtype, void* stream);
+                    int ldd, int S, int Pq, bool split, int dtype, void* stream, float* a_sums = nullptr, bool* summed = nullptr);
+// The rows of column sums of A (of 64 or 128 columns, side by side tiles_a to a row of tn_sum_width) that a product of these sizes
+// writes to a_sums where it takes them (*summed): tiles of B times T times S
+int tn_sum_rows(int T, int na, int nb, int S);
+int tn_sum_width(int na, int nb);
 // The weight gradient of a 2-D convolution taken directly: dW[(ky, kx)][s] (K x C) = sum over the output pixels of
 // part s of dy (x) the pixel of x that tap reads (gemm_tn.hip)
 int gemm_tn_conv(const void* dy, const void* x, float* D, int N, int H, int W, int C, int K, int kh, int kw, int stride,
-                 int pad_h, int pad_w, int oH, int oW, int S, int Pq, int dtype, void* stream);
+                 int pad_h, int pad_w, int oH, int oW, int S, int Pq, int dtype, void* stream, float* dy_sums = nullptr, bool* summed = nullptr);
 
 // The tap form of the weight gradient (backward_taps.hip; 16-bit 3x3 and 3x3x3 layers at stride 1 with output extents `out`):
-// whether it is taken and the bytes of its partial sums, and the launch
-bool taps_gradient_fits(const wc_conv_desc* d, const int out[3], size_t* workspace_bytes);
-int taps_gradient(const wc_conv_desc* d, const int out[3], const void* x, const void* dy, void* dw,
-                  const int64_t dw_strides[5], float* part, void* stream);
+// whether it is taken and the bytes of its partial sums and of dy's column sums, and the launch
+bool taps_gradient_fits(const wc_conv_desc* d, const int out[3], size_t* workspace_bytes, size_t* bias_bytes);
+int taps_gradient(const wc_conv_desc* d, const int out[3], const void* x, const void* dy, const GradOut& to, float* part, void* stream);
+// Bytes and launches of a bias gradient of its own (bias_gradient.hip): db (of dy's type or fp32) = the column sums of dy (rows, K)
+size_t bias_part_bytes(long long rows, int K, int dtype);
+int bias_sums(const void* dy, void* db, long long rows, int K, int dtype, bool f32, float* part, void* stream);
 
 // One-kernel F(2x2, 3x3) forward pass for thin 16-bit layers (conv_thin.hip): whether the problem
 // with this single-piece plan is in its range, and the launch.  U (16, K, Cp) from wc_filter_transform.

@@ -480,6 +480,10 @@ def conv_backward_weight(x, dy, w_shape, stride=1, padding=0, m=2, whole_kernel=
     _require_gpu(x, dy)
     if USE_EXT and stacked is None and not whole_kernel and x.shape[0] > 0:
         return _ext.conv_backward_weight(x, dy, tuple(w_shape), stride, padding, m)
+    return _conv_backward_parameters(x, dy, w_shape, stride, padding, m, whole_kernel, stacked, False, x.dtype, x.dtype)[0]
+
+
+def _conv_backward_parameters(x, dy, w_shape, stride, padding, m, whole_kernel, stacked, need_db, w_type, b_type):
     stacked = _stack(stacked, x.dtype, x.dim() - 2, whole_kernel, w_shape, stride, m)
     if stacked == 2:
         stacked = True               # the weight gradient has no shared-input form: pieces stacked with their own V
@@ -492,16 +496,36 @@ def conv_backward_weight(x, dy, w_shape, stride=1, padding=0, m=2, whole_kernel=
     if tuple(dy.shape) != (x.shape[0], w_shape[0]) + tuple(osp):
         raise ValueError("dy has shape %r, the convolution gives %r"
                          % (tuple(dy.shape), (x.shape[0], w_shape[0]) + tuple(osp)))
-    dw = torch.empty(tuple(w_shape), dtype=x.dtype, device=x.device)
+    dw = torch.empty(tuple(w_shape), dtype=w_type, device=x.device)
+    db = torch.empty(w_shape[0], dtype=b_type, device=x.device) if need_db else None
     if x.shape[0] == 0:
-        return dw.zero_()
+        return dw.zero_(), None if db is None else db.zero_()
     x_cl, dy_cl = channel_last(x), channel_last(dy)
     nbytes = ctypes.c_size_t()
-    check(lib.wc_conv_backward_weight_workspace_bytes(ctypes.byref(desc), ctypes.byref(nbytes)))
+    if not need_db and w_type == x.dtype:
+        check(lib.wc_conv_backward_weight_workspace_bytes(ctypes.byref(desc), ctypes.byref(nbytes)))
+        ws = torch.empty(nbytes.value, dtype=torch.uint8, device=x.device)
+        check(lib.wc_conv_backward_weight(ctypes.byref(desc), _ptr(x_cl), _ptr(dy_cl), _ptr(dw), _w_strides(dw),
+                                          _ptr(ws), nbytes.value, _stream(x)))
+        return dw, None
+    check(lib.wc_conv_backward_parameters_workspace_bytes(ctypes.byref(desc), ctypes.byref(nbytes)))
     ws = torch.empty(nbytes.value, dtype=torch.uint8, device=x.device)
-    check(lib.wc_conv_backward_weight(ctypes.byref(desc), _ptr(x_cl), _ptr(dy_cl), _ptr(dw), _w_strides(dw),
-                                      _ptr(ws), nbytes.value, _stream(x)))
-    return dw
+    check(lib.wc_conv_backward_parameters(ctypes.byref(desc), _ptr(x_cl), _ptr(dy_cl), _ptr(dw), _w_strides(dw), _DTYPES[w_type],
+                                          _ptr(db), _DTYPES[b_type], _ptr(ws), nbytes.value, _stream(x)))
+    return dw, db
+
+
+def conv_backward_parameters(x, dy, w_shape, stride=1, padding=0, m=2, need_db=True, w_type=None, b_type=None):
+    """conv_backward_weight and, with `need_db`, bias_gradient of the same dy in one call: (dw, db or None), in `w_type` and `b_type`
+    (float32 sums unrounded where these are float32; any other type than x's is a cast of its own)."""
+    _require_gpu(x, dy)
+    w_type, b_type = w_type or x.dtype, b_type or x.dtype
+    w_own, b_own = (t if t == torch.float32 else x.dtype for t in (w_type, b_type))
+    if USE_EXT and x.shape[0] > 0:
+        dw, db = _ext.conv_backward_parameters(x, dy, tuple(w_shape), stride, padding, m, need_db, w_own, b_own)
+    else:
+        dw, db = _conv_backward_parameters(x, dy, w_shape, stride, padding, m, False, None, need_db, w_own, b_own)
+    return dw.to(w_type), None if db is None else db.to(b_type)
 
 
 def bias_gradient(dy):
