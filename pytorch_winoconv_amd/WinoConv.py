@@ -61,26 +61,30 @@ class WinoConvFunction(torch.autograd.Function):
     def backward(ctx, dy):
         x, w = ctx.saved_tensors
         stride, padding, m, has_bias = ctx.conf
-        dx = dw = db = None
         need_dx, need_dw, need_db = ctx.needs_input_grad[:3]
-        w_type, b_type = (None if t == x.dtype else t for t in ctx.types)
-        # One call on autograd's thread instead of three and the casts of two gradients (host time of a training step with float32
-        # parameters and float16 activations 211 us, now 124, at stride 2 212 and 98); what it leaves to the functions below comes
-        # back as None
+        need_db = has_bias and need_db
+        w_type, b_type = ctx.types
+        dx = dw = db = None
         if engine.USE_EXT and x.shape[0] > 0 and not torch.is_grad_enabled():
-            dx, dw, db = engine.conv_backward(x, w, dy, stride, padding, m, need_dx, need_dw, has_bias and need_db, w_type, b_type)
-        if need_dx and dx is None:
-            dx = engine.conv_backward_input(dy, w, x.shape[2:], stride, padding, m)
-        if need_dw and dw is None:
-            # the engine's bias gradient where this pass runs on it anyway; a gradient that is itself differentiated, or a dy
-            # that the kernel would have to copy first, stays with torch
-            both = has_bias and need_db and not torch.is_grad_enabled() and engine.channel_last_memory(dy)
-            dw, b = engine.conv_backward_parameters(x, dy, w.shape, stride, padding, m, both, w_type, b_type)
-            db = b if both else db
-        if has_bias and need_db and db is None:
-            db = dy.sum(dim=[0] + list(range(2, dy.dim())))
-            db = db if b_type is None else db.to(b_type)
+            dx, dw, db = engine.conv_backward(x, w, dy, stride, padding, m, need_dx, need_dw, need_db, w_type, b_type or x.dtype)
+        rest = gradients(x, w, dy, stride, padding, m, need_dx and dx is None, need_dw and dw is None, need_db and db is None, w_type, b_type)
+        dx, dw, db = (a if b is None else b for a, b in zip((dx, dw, db), rest))
         return dx, dw, db, None, None, None, None, None
+
+
+def gradients(x, w, dy, stride, padding, m, need_dx, need_dw, need_db, w_type, b_type):
+    """The gradients of a layer that are asked for, one function each, in the types of its parameters: what the compiled host layer's one
+    call for all leaves to them, and gradients that are themselves differentiated."""
+    dx = engine.conv_backward_input(dy, w, x.shape[2:], stride, padding, m) if need_dx else None
+    dw = db = None
+    if need_dw:
+        # the engine's bias gradient where this pass runs on it anyway; a gradient that is itself differentiated, or a dy
+        # that the kernel would have to copy first, stays with torch
+        both = need_db and not torch.is_grad_enabled() and engine.channel_last_memory(dy)
+        dw, db = engine.conv_backward_parameters(x, dy, w.shape, stride, padding, m, both, w_type, b_type)
+    if need_db and db is None:
+        db = dy.sum(dim=[0] + list(range(2, dy.dim()))).to(b_type)
+    return dx, dw, db
 
 
 class _WinoConvNd(nn.Module):
@@ -101,6 +105,13 @@ class _WinoConvNd(nn.Module):
         if self.bias is not None:
             nn.init.zeros_(self.bias)
         self._cache = None
+
+    # (hyperparameters, the compiled host layer's plan for the last input's shape or None, that shape): planned when a shape comes a
+    # second time running, so a program whose shapes alternate pays nothing.  Copies and files go without.
+    _plan = None
+
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k != "_plan"}
 
     def _winograd_ok(self, x):
         # The reference hands every strided or dilated layer (and every kernel up to 3 x 3) to the stock
@@ -148,6 +159,17 @@ class _WinoConvNd(nn.Module):
         return self._tile()
 
     def forward(self, x):
+        conf = (self.in_channels, self.out_channels, self.kernel_size, self.stride, self.padding, self.dilation, self.groups, self.output_block)
+        plan = self._plan
+        if x.is_cuda and plan is not None and plan[1] is not None and plan[0] == conf and engine.USE_EXT:
+            weight = self.weight
+            y = plan[1](x, weight, self.bias)
+            if type(y) is tuple:
+                y, renewed, U = y
+                self.__dict__["_plan"] = (conf, renewed, plan[2])
+                self.__dict__["_cache"] = ((weight._version, weight.data_ptr()) + self._cache[0][2:], U)
+            if y is not None:
+                return y
         conv = F.conv2d if self.nd == 2 else F.conv3d
         if not x.is_cuda:
             raise ValueError("WinoConv: the engine runs on the GPU only; got a CPU tensor")
@@ -166,6 +188,9 @@ class _WinoConvNd(nn.Module):
         if self._cache is None or self._cache[0] != key:
             U = engine.transform_filter(w.detach(), x.shape, self.stride[0], self.padding, m, row=True)
             self._cache = (key, U)
+        if engine.USE_EXT:
+            again = plan is not None and plan[2] == x.shape
+            self.__dict__["_plan"] = (conf, engine.layer_plan(x, weight, self.stride[0], self.padding, m, self._cache[1]) if again else None, x.shape)
         b = bias if bias is None or bias.dtype == x.dtype else bias.detach().to(x.dtype)
         if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad or (bias is not None and bias.requires_grad)):
             return WinoConvFunction.apply(x, weight, bias, self.stride[0], self.padding, m, self._cache[1],

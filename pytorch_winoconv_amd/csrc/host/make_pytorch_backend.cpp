@@ -10,6 +10,10 @@
 // Wider than the reference: float16 and bfloat16 are dispatched by tensor dtype (the reference binds
 // float only: bind.cpp:19-23), stride 2 and every kernel extent 1..10 work.
 #include <torch/extension.h>
+#include <torch/csrc/DynamicTypes.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
@@ -298,7 +302,7 @@ int winograd_conv(at::Tensor Input, at::Tensor Weight, at::Tensor Output, std::o
   return d.m;
 }
 
-std::vector<int> ints_of(py::object v, int nd, const char* what) {
+std::vector<int> ints_of(const py::object& v, int nd, const char* what) {
   std::vector<int> r;
   if (py::isinstance<py::int_>(v)) {
     r.assign(nd, v.cast<int>());
@@ -309,18 +313,34 @@ std::vector<int> ints_of(py::object v, int nd, const char* what) {
   return r;
 }
 
+int spatial_dims(at::IntArrayRef x, at::IntArrayRef w) {
+  if ((x.size() != 4 && x.size() != 5) || w.size() != x.size())
+    throw std::invalid_argument("expected 4-D or 5-D input and matching filter, got " + shape_str(x) + " and " + shape_str(w));
+  return (int)x.size() - 2;
+}
+
+int one_stride(const py::object& stride, int nd) {
+  const auto st = ints_of(stride, nd, "stride");
+  for (int a = 1; a < nd; ++a)
+    if (st[a] != st[0]) throw Unsupported("stride must be the same on every axis");
+  return st[0];
+}
+
 // Winograd / DWM convolution of an NC[D]HW tensor with a (K, C, [kD,] kH, kW) filter; returns an NC[D]HW
 // tensor whose memory is channel-last (or plain contiguous with channels_first_out).  A channel-last input is
 // used without a copy and a contiguous channel-first one is handed to the library as it is
 // (wc_conv_desc.x_layout); any other layout is made contiguous first.  The compiled form of the Python callers' common path (dwm.py:5-40, matrix_conv.py:70-135
 // of the reference end in the same call).
 // `flipped`: the filter is w reversed along every spatial axis, read through negative strides.
-at::Tensor conv_impl(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bias, py::object stride, py::object padding,
-                     int m, std::optional<at::Tensor> U, int chunk_images, bool whole_kernel, py::object stacked,
-                     bool unfused, bool channels_first_out, py::object direct, bool row, bool flipped) {
-  const int nd = (int)x.dim() - 2;
-  if ((nd != 2 && nd != 3) || w.dim() != nd + 2)
-    throw std::invalid_argument("expected 4-D or 5-D input and matching filter, got " + shape_str(x.sizes()) + " and " + shape_str(w.sizes()));
+// No function from here to the gradients touches Python: they run with and without the interpreter lock.
+struct ConvOptions {
+  int chunk_images = 0, stacked = -1, direct = 0;      // -1: the library chooses the form of the plan; 0: it may take the direct one
+  bool whole_kernel = false, unfused = false, channels_first_out = false, row = false, flipped = false;
+};
+
+at::Tensor conv_impl(at::Tensor x, const at::Tensor& w, const std::optional<at::Tensor>& bias, int stride, const std::vector<int>& pd, int m,
+                     std::optional<at::Tensor> U, const ConvOptions& o) {
+  const int nd = spatial_dims(x.sizes(), w.sizes());
   if (x.size(1) != w.size(1))
     throw std::invalid_argument("input has " + std::to_string(x.size(1)) + " channels, filter expects " + std::to_string(w.size(1)) +
                                 " (groups are not supported)");
@@ -348,11 +368,6 @@ at::Tensor conv_impl(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bias,
   require_gpu(x, "conv_forward");
   require_gpu(w, "conv_forward");
   if (w.scalar_type() != x.scalar_type()) throw py::type_error("input, filter and bias must share one dtype");
-  const auto st = ints_of(stride, nd, "stride");
-  for (int a = 1; a < nd; ++a)
-    if (st[a] != st[0]) { PyErr_SetString(PyExc_NotImplementedError, "stride must be the same on every axis"); throw py::error_already_set(); }
-  const auto pd = ints_of(padding, nd, "padding");
-
   wc_conv_desc d{};
   d.ndim = nd;
   d.N = (int)(x.size(0) > 0 ? x.size(0) : 1);      // an empty batch: the shape arithmetic runs on one image
@@ -363,13 +378,13 @@ at::Tensor conv_impl(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bias,
     d.kernel[3 - nd + a] = (int)w.size(2 + a);
     d.pad[3 - nd + a] = pd[a];
   }
-  d.stride = st[0]; d.m = m; d.dtype = dtype_of(x);
-  d.chunk_images = chunk_images;
-  d.whole_kernel = whole_kernel;
-  d.stacked = stacked.is_none() ? -1 : (py::isinstance<py::bool_>(stacked) ? (int)stacked.cast<bool>() : stacked.cast<int>());
-  d.direct = direct.is_none() ? 0 : (direct.cast<bool>() ? 1 : -1);      // None: the library may choose it
-  d.unfused = unfused;
-  d.row = row && !unfused ? -1 : 0;                                       // -1: the library may choose it
+  d.stride = stride; d.m = m; d.dtype = dtype_of(x);
+  d.chunk_images = o.chunk_images;
+  d.whole_kernel = o.whole_kernel;
+  d.stacked = o.stacked;
+  d.direct = o.direct;
+  d.unfused = o.unfused;
+  d.row = o.row && !o.unfused ? -1 : 0;                                   // -1: the library may choose it
   check(wc_conv_auto(&d));
   int out[3], grid[3];
   check(wc_conv_out_dims(&d, out, grid));
@@ -381,20 +396,20 @@ at::Tensor conv_impl(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bias,
   to_cl.push_back(1);
   std::vector<int64_t> ys_cf{ys[0], K};
   for (int a = 0; a < nd; ++a) ys_cf.push_back(ys[1 + a]);
-  at::Tensor y = at::empty(channels_first_out ? ys_cf : ys, x.options());
-  if (x.size(0) == 0) return channels_first_out ? y : y.permute(to_cf);
+  at::Tensor y = at::empty(o.channels_first_out ? ys_cf : ys, x.options());
+  if (x.size(0) == 0) return o.channels_first_out ? y : y.permute(to_cf);
   at::Tensor x_mem = x.permute(to_cl);
   if (!x_mem.is_contiguous()) {                            // not channel-last memory: channel-first, read as it is
     x_mem = x.is_contiguous() ? x : x.contiguous();
     d.x_layout = 1;
   }
-  d.y_layout = channels_first_out;
+  d.y_layout = o.channels_first_out;
   auto misaligned = [](const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) != 0; };
   if (d.row) {                                             // the row form reads aligned operands: copies of those that are not
     if (misaligned(x_mem)) x_mem = x_mem.clone();
     if (U && U->defined() && misaligned(*U)) U = U->clone();
   }
-  d.unfused = unfused || misaligned(x_mem) || (U && U->defined() && misaligned(*U));
+  d.unfused = o.unfused || misaligned(x_mem) || (U && U->defined() && misaligned(*U));
   if (U && U->defined()) {
     size_t ue = 0;
     check(wc_conv_u_elems(&d, &ue));
@@ -410,31 +425,42 @@ at::Tensor conv_impl(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bias,
   int64_t s[5] = {w.stride(0), w.stride(1), 0, 0, 0};
   for (int a = 0; a < nd; ++a) s[5 - nd + a] = w.stride(2 + a);
   const unsigned char* wp = static_cast<const unsigned char*>(w.data_ptr());
-  if (flipped)
+  if (o.flipped)
     for (int a = 0; a < nd; ++a) {
       wp += (w.size(2 + a) - 1) * w.stride(2 + a) * w.element_size();
       s[5 - nd + a] = -w.stride(2 + a);
     }
-  {
-    py::gil_scoped_release nogil;
-    check(wc_conv_forward(&d, x_mem.data_ptr(), wp, s, U && U->defined() ? U->data_ptr() : nullptr,
-                          bc.defined() ? bc.data_ptr() : nullptr, y.data_ptr(), ws.data_ptr(), bytes, stream));
-  }
-  return channels_first_out ? y : y.permute(to_cf);
+  check(wc_conv_forward(&d, x_mem.data_ptr(), wp, s, U && U->defined() ? U->data_ptr() : nullptr,
+                        bc.defined() ? bc.data_ptr() : nullptr, y.data_ptr(), ws.data_ptr(), bytes, stream));
+  return o.channels_first_out ? y : y.permute(to_cf);
 }
 
 at::Tensor conv_forward(at::Tensor x, at::Tensor w, std::optional<at::Tensor> bias, py::object stride, py::object padding,
                         int m, std::optional<at::Tensor> U, int chunk_images, bool whole_kernel, py::object stacked,
                         bool unfused, bool channels_first_out, py::object direct, bool row) {
-  return conv_impl(x, w, bias, stride, padding, m, U, chunk_images, whole_kernel, stacked, unfused, channels_first_out, direct,
-                   row, false);
+  const int nd = spatial_dims(x.sizes(), w.sizes());
+  ConvOptions o;
+  o.chunk_images = chunk_images; o.whole_kernel = whole_kernel; o.unfused = unfused; o.channels_first_out = channels_first_out; o.row = row;
+  o.stacked = stacked.is_none() ? -1 : (py::isinstance<py::bool_>(stacked) ? (int)stacked.cast<bool>() : stacked.cast<int>());
+  o.direct = direct.is_none() ? 0 : (direct.cast<bool>() ? 1 : -1);
+  const int st = one_stride(stride, nd);
+  const auto pd = ints_of(padding, nd, "padding");
+  py::gil_scoped_release nogil;
+  return conv_impl(std::move(x), w, bias, st, pd, m, std::move(U), o);
 }
 
 // Input gradient of a stride-1 layer: dy convolved with w flipped and its channel axes exchanged; `padding` is that
 // convolution's.
+at::Tensor backward_input_flipped(const at::Tensor& dy, const at::Tensor& w, const std::vector<int>& pads, int m) {
+  ConvOptions o;
+  o.row = o.flipped = true;
+  return conv_impl(dy, w.transpose(0, 1), std::nullopt, 1, pads, m, std::nullopt, o);
+}
+
 at::Tensor conv_backward_input_flipped(at::Tensor dy, at::Tensor w, py::object padding, int m) {
-  return conv_impl(dy, w.transpose(0, 1), std::nullopt, py::int_(1), padding, m, std::nullopt, 0, false, py::none(), false, false,
-                   py::none(), true, true);
+  const auto pads = ints_of(padding, (int)dy.dim() - 2, "padding");
+  py::gil_scoped_release nogil;
+  return backward_input_flipped(dy, w, pads, m);
 }
 
 at::Tensor last_view(const at::Tensor& t) {       // (N, C, *) -> (N, *, C), contiguous
@@ -467,7 +493,7 @@ void strides_of(const at::Tensor& w, int64_t s[5]) {
 
 // Input gradient of a 2-D layer at stride 2 over the parity classes of its pixels (wc_conv_backward_input); an undefined
 // tensor, and nothing launched, where that does not apply.  engine.py's conv_backward_input has checked the padding.
-at::Tensor conv_backward_input_strided(at::Tensor dy, at::Tensor w, std::vector<int64_t> x_spatial, std::vector<int> pads) {
+at::Tensor backward_input_strided(const at::Tensor& dy, const at::Tensor& w, at::IntArrayRef x_spatial, const std::vector<int>& pads) {
   require_gpu(dy, "conv_backward_input");
   require_gpu(w, "conv_backward_input");
   wc_conv_desc d = desc_of({dy.size(0), w.size(1), x_spatial[0], x_spatial[1]}, w.sizes(), pads, 2, 2, dtype_of(dy));
@@ -484,11 +510,13 @@ at::Tensor conv_backward_input_strided(at::Tensor dy, at::Tensor w, std::vector<
   at::Tensor ws = workspace_for(dy, bytes, stream);
   int64_t s[5];
   strides_of(w, s);
-  {
-    py::gil_scoped_release nogil;
-    check(wc_conv_backward_input(&d, dyl.data_ptr(), w.data_ptr(), s, dx.data_ptr(), ws.data_ptr(), bytes, stream));
-  }
+  check(wc_conv_backward_input(&d, dyl.data_ptr(), w.data_ptr(), s, dx.data_ptr(), ws.data_ptr(), bytes, stream));
   return dx.permute({0, 3, 1, 2});
+}
+
+at::Tensor conv_backward_input_strided(at::Tensor dy, at::Tensor w, std::vector<int64_t> x_spatial, std::vector<int> pads) {
+  py::gil_scoped_release nogil;
+  return backward_input_strided(dy, w, x_spatial, pads);
 }
 
 // engine.py's transform_filter with the form left to the library, the row form allowed
@@ -500,10 +528,8 @@ at::Tensor transform_filter(at::Tensor w, std::vector<int64_t> x_shape, py::obje
   if (x_shape[1] != w.size(1))
     throw std::invalid_argument("input has " + std::to_string(x_shape[1]) + " channels, filter expects " + std::to_string(w.size(1)) +
                                 " (groups are not supported)");
-  const auto st = ints_of(stride, nd, "stride");
-  for (int a = 1; a < nd; ++a)
-    if (st[a] != st[0]) { PyErr_SetString(PyExc_NotImplementedError, "stride must be the same on every axis"); throw py::error_already_set(); }
-  wc_conv_desc d = desc_of(x_shape, w.sizes(), ints_of(padding, nd, "padding"), st[0], m, dtype_of(w));
+  const int st = one_stride(stride, nd);
+  wc_conv_desc d = desc_of(x_shape, w.sizes(), ints_of(padding, nd, "padding"), st, m, dtype_of(w));
   d.stacked = d.row = -1;
   check(wc_conv_auto(&d));
   wc_plan plan{};
@@ -532,8 +558,8 @@ at::Tensor transform_filter(at::Tensor w, std::vector<int64_t> x_shape, py::obje
 // ---- gradients (the reference has no backward pass: src/back/utils.cu:15-24): engine.py's conv_backward_weight with the
 // form of the plan left to the library, and bias_gradient
 // (dw, db) with `bias`, each of type fp32 or x's
-std::pair<at::Tensor, at::Tensor> parameter_gradients(at::Tensor x, at::Tensor dy, std::vector<int64_t> w_shape, py::object stride,
-                                                      py::object padding, int m, bool bias, at::ScalarType w_type, at::ScalarType b_type) {
+std::pair<at::Tensor, at::Tensor> parameter_gradients(const at::Tensor& x, const at::Tensor& dy, at::IntArrayRef w_shape, int stride,
+                                                      const std::vector<int>& pd, int m, bool bias, at::ScalarType w_type, at::ScalarType b_type) {
   const int nd = (int)x.dim() - 2;
   require_gpu(x, "conv_backward_weight");
   require_gpu(dy, "conv_backward_weight");
@@ -543,16 +569,12 @@ std::pair<at::Tensor, at::Tensor> parameter_gradients(at::Tensor x, at::Tensor d
   if (x.size(1) != w_shape[1])
     throw std::invalid_argument("input has " + std::to_string(x.size(1)) + " channels, filter expects " + std::to_string(w_shape[1]) +
                                 " (groups are not supported)");
-  const auto st = ints_of(stride, nd, "stride");
-  for (int a = 1; a < nd; ++a)
-    if (st[a] != st[0]) { PyErr_SetString(PyExc_NotImplementedError, "stride must be the same on every axis"); throw py::error_already_set(); }
-  const auto pd = ints_of(padding, nd, "padding");
   wc_conv_desc d{};
   d.ndim = nd;
   d.C = (int)x.size(1); d.K = (int)w_shape[0];
   d.kernel[0] = d.in[0] = 1;
   for (int a = 0; a < nd; ++a) d.kernel[3 - nd + a] = (int)w_shape[2 + a];
-  d.stride = st[0]; d.m = m; d.dtype = dtype_of(x);
+  d.stride = stride; d.m = m; d.dtype = dtype_of(x);
   // the Winograd / DWM form of the forward plan, the direct one aside, whatever the batch; the gradient has no form whose
   // pieces share one transformed input: pieces stacked with their own V
   wc_conv_desc form = d;
@@ -566,7 +588,7 @@ std::pair<at::Tensor, at::Tensor> parameter_gradients(at::Tensor x, at::Tensor d
   check(wc_conv_out_dims(&d, out, grid));
   std::vector<int64_t> ys{x.size(0), w_shape[0]};
   for (int a = 3 - nd; a < 3; ++a) ys.push_back(out[a]);
-  if (dy.sizes().vec() != ys) throw std::invalid_argument("dy has shape " + shape_str(dy.sizes()) + ", the convolution gives " + shape_str(ys));
+  if (dy.sizes() != at::IntArrayRef(ys)) throw std::invalid_argument("dy has shape " + shape_str(dy.sizes()) + ", the convolution gives " + shape_str(ys));
   at::Tensor dw = at::empty(w_shape, x.options().dtype(w_type)), db;
   if (bias) db = at::empty({w_shape[0]}, x.options().dtype(b_type));
   const bool plain = !bias && w_type == x.scalar_type();
@@ -577,25 +599,31 @@ std::pair<at::Tensor, at::Tensor> parameter_gradients(at::Tensor x, at::Tensor d
   at::Tensor ws = workspace_for(x, bytes, stream);
   int64_t s[5] = {dw.stride(0), dw.stride(1), 0, 0, 0};
   for (int a = 0; a < nd; ++a) s[5 - nd + a] = dw.stride(2 + a);
-  {
-    py::gil_scoped_release nogil;
-    check(plain ? wc_conv_backward_weight(&d, xl.data_ptr(), dyl.data_ptr(), dw.data_ptr(), s, ws.data_ptr(), bytes, stream)
-                : wc_conv_backward_parameters(&d, xl.data_ptr(), dyl.data_ptr(), dw.data_ptr(), s, dtype_of(dw), bias ? db.data_ptr() : nullptr,
-                                              bias ? dtype_of(db) : WC_F32, ws.data_ptr(), bytes, stream));
-  }
+  check(plain ? wc_conv_backward_weight(&d, xl.data_ptr(), dyl.data_ptr(), dw.data_ptr(), s, ws.data_ptr(), bytes, stream)
+              : wc_conv_backward_parameters(&d, xl.data_ptr(), dyl.data_ptr(), dw.data_ptr(), s, dtype_of(dw), bias ? db.data_ptr() : nullptr,
+                                            bias ? dtype_of(db) : WC_F32, ws.data_ptr(), bytes, stream));
   return {dw, db};
 }
 
 at::Tensor conv_backward_weight(at::Tensor x, at::Tensor dy, std::vector<int64_t> w_shape, py::object stride, py::object padding, int m) {
-  return parameter_gradients(x, dy, w_shape, stride, padding, m, false, x.scalar_type(), x.scalar_type()).first;
+  const int nd = (int)x.dim() - 2, st = one_stride(stride, nd);
+  const auto pd = ints_of(padding, nd, "padding");
+  py::gil_scoped_release nogil;
+  return parameter_gradients(x, dy, w_shape, st, pd, m, false, x.scalar_type(), x.scalar_type()).first;
 }
 
 py::object or_none(const at::Tensor& t) { return t.defined() ? py::cast(t) : py::none(); }
 
 py::tuple conv_backward_parameters(at::Tensor x, at::Tensor dy, std::vector<int64_t> w_shape, py::object stride, py::object padding, int m,
                                    bool need_db, py::object w_type, py::object b_type) {
-  const auto g = parameter_gradients(x, dy, w_shape, stride, padding, m, need_db, torch::python::detail::py_object_to_dtype(w_type),
-                                     torch::python::detail::py_object_to_dtype(b_type));
+  const int nd = (int)x.dim() - 2, st = one_stride(stride, nd);
+  const auto pd = ints_of(padding, nd, "padding");
+  const auto wt = torch::python::detail::py_object_to_dtype(w_type), bt = torch::python::detail::py_object_to_dtype(b_type);
+  std::pair<at::Tensor, at::Tensor> g;
+  {
+    py::gil_scoped_release nogil;
+    g = parameter_gradients(x, dy, w_shape, st, pd, m, need_db, wt, bt);
+  }
   return py::make_tuple(g.first, or_none(g.second));
 }
 
@@ -613,17 +641,24 @@ at::Tensor bias_gradient(at::Tensor dy) {
   return db;
 }
 
-// All gradients of a layer in one call, each in the type of what it belongs to: (dx, dw, db), None for what is not asked for
-// and for what engine.py's functions have to do (an input gradient that neither function above has, the bias gradient of a dy
-// that is not channel-last memory).
-py::tuple conv_backward(at::Tensor x, at::Tensor w, at::Tensor dy, py::object stride, py::object padding, int m, bool need_dx,
-                        bool need_dw, bool need_db, py::object w_type, py::object b_type) {
-  const int nd = (int)x.dim() - 2;
-  if ((nd != 2 && nd != 3) || w.dim() != nd + 2 || dy.dim() != nd + 2)
+bool channel_last_memory(const at::Tensor& t) {
+  std::vector<int64_t> last{0};
+  for (int64_t a = 2; a < t.dim(); ++a) last.push_back(a);
+  last.push_back(1);
+  return t.permute(last).is_contiguous();
+}
+
+// All gradients of a layer in one call, each in the type of what it belongs to: undefined for what is not asked for and for what
+// engine.py's functions have to do (an input gradient that neither function above has, the bias gradient of a dy that is not
+// channel-last memory).
+struct Gradients { at::Tensor dx, dw, db; };
+
+Gradients backward_all(const at::Tensor& x, const at::Tensor& w, const at::Tensor& dy, int stride, const std::vector<int>& pd, int m,
+                       bool need_dx, bool need_dw, bool need_db, at::ScalarType w_type, at::ScalarType b_type) {
+  const int nd = spatial_dims(x.sizes(), w.sizes());
+  if (dy.dim() != x.dim())
     throw std::invalid_argument("expected 4-D or 5-D input and matching filter, got " + shape_str(x.sizes()) + " and " + shape_str(w.sizes()));
-  const auto st = ints_of(stride, nd, "stride");
-  const auto pd = ints_of(padding, nd, "padding");
-  at::Tensor dx, dw, db;
+  Gradients g;
   if (need_dx) {
     std::vector<int> flipped(nd);
     bool fits = true;
@@ -631,29 +666,223 @@ py::tuple conv_backward(at::Tensor x, at::Tensor w, at::Tensor dy, py::object st
       flipped[a] = (int)w.size(2 + a) - 1 - pd[a];
       fits = fits && flipped[a] >= 0;
     }
-    const std::vector<int64_t> size(x.sizes().begin() + 2, x.sizes().end());
-    if (fits && st[0] == 1) {
+    const at::IntArrayRef size = x.sizes().slice(2);
+    if (fits && stride == 1) {
       bool threes = true;
       for (int a = 0; a < nd; ++a) threes = threes && w.size(2 + a) == 3;
       const int tile = w.size(0) >= 8 && (m == 2 || nd == 2 || threes) ? m : 2;      // as in engine.py's conv_backward_input
-      at::Tensor t = conv_backward_input_flipped(dy, w, py::cast(flipped), tile);
-      if (t.sizes().slice(2) == at::IntArrayRef(size)) dx = t;
-    } else if (fits && nd == 2 && st[0] == 2) {
-      dx = conv_backward_input_strided(dy, w, size, pd);
+      at::Tensor t = backward_input_flipped(dy, w, flipped, tile);
+      if (t.sizes().slice(2) == size) g.dx = t;
+    } else if (fits && nd == 2 && stride == 2) {
+      g.dx = backward_input_strided(dy, w, size, pd);
     }
   }
   if (need_dw) {
-    std::vector<int64_t> last{0};
-    for (int a = 0; a < nd; ++a) last.push_back(2 + a);
-    last.push_back(1);
-    auto type = [&](const py::object& t) { return t.is_none() ? x.scalar_type() : torch::python::detail::py_object_to_dtype(t); };
     auto own = [&](at::ScalarType t) { return t == at::kFloat ? t : x.scalar_type(); };      // any other type: a cast of its own
-    const at::ScalarType wt = type(w_type), bt = type(b_type);
-    std::tie(dw, db) = parameter_gradients(x, dy, w.sizes().vec(), stride, padding, m, need_db && dy.permute(last).is_contiguous(), own(wt), own(bt));
-    dw = dw.to(wt);
-    if (db.defined()) db = db.to(bt);
+    std::tie(g.dw, g.db) = parameter_gradients(x, dy, w.sizes(), stride, pd, m, need_db && channel_last_memory(dy), own(w_type), own(b_type));
+    g.dw = g.dw.to(w_type);
+    if (g.db.defined()) g.db = g.db.to(b_type);
   }
-  return py::make_tuple(or_none(dx), or_none(dw), or_none(db));
+  return g;
+}
+
+py::tuple conv_backward(at::Tensor x, at::Tensor w, at::Tensor dy, py::object stride, py::object padding, int m, bool need_dx,
+                        bool need_dw, bool need_db, py::object w_type, py::object b_type) {
+  const int nd = spatial_dims(x.sizes(), w.sizes()), st = one_stride(stride, nd);
+  const auto pd = ints_of(padding, nd, "padding");
+  auto type = [&](const py::object& t) { return t.is_none() ? x.scalar_type() : torch::python::detail::py_object_to_dtype(t); };
+  const at::ScalarType wt = type(w_type), bt = type(b_type);
+  Gradients g;
+  {
+    py::gil_scoped_release nogil;
+    g = backward_all(x, w, dy, st, pd, m, need_dx, need_dw, need_db, wt, bt);
+  }
+  return py::make_tuple(or_none(g.dx), or_none(g.dw), or_none(g.db));
+}
+
+// ---- a module's forward pass ----------------------------------------------------------------------------------------
+// What WinoConv.py's modules work out anew for an input of another shape: the descriptor, the shape of the result and the
+// transformed filter.  Called with an input of the same shape, strides and type and a weight of the same kind, it runs the layer
+// without Python, with an autograd node of C++ where a gradient is wanted, and gives a plan for the filter where the weight has
+// changed; called with anything else it gives None, and the module goes its way.  It never changes after it is made, so
+// threads may share it; tensors are compared by what they are, and none but the transformed filter is kept.
+// Host time, us: a frozen layer 10.6 | 6.5 (a launch of torch's own 4.8), a training step in mixed precision 182 | 122, its backward
+// pass 102 | 69, of which 55 are the autograd engine and a thread's waking.
+class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
+ public:
+  at::ScalarType x_type, w_type;
+  at::Device device;
+  std::vector<int64_t> sizes, strides, w_sizes, y_sizes, y_strides;
+  wc_conv_desc d{};
+  size_t bytes = 0;
+  int nd, stride, m;
+  std::vector<int> pads;
+  at::Tensor U;
+  const void* w_data;
+  uint32_t w_version;
+
+  // None where the layer copies its input first or the filter is not the plan's
+  static std::shared_ptr<LayerPlan> make(const at::Tensor& x, const at::Tensor& weight, int stride, std::vector<int> pads, int m, const at::Tensor& U) {
+    const int nd = spatial_dims(x.sizes(), weight.sizes());
+    if ((int)pads.size() != nd || x.numel() == 0 || x.size(1) != weight.size(1) || !plain(x) || !plain(weight) || misaligned(x) || misaligned(U)) return nullptr;
+    const bool last = channel_last_memory(x);
+    if (!last && !x.is_contiguous()) return nullptr;
+    auto p = std::make_shared<LayerPlan>(x, weight, stride, std::move(pads), m, U);
+    p->d = desc_of(x.sizes(), weight.sizes(), p->pads, stride, m, dtype_of(x));
+    p->d.stacked = p->d.row = -1;
+    check(wc_conv_auto(&p->d));
+    p->d.x_layout = !last;
+    size_t ue = 0;
+    check(wc_conv_u_elems(&p->d, &ue));
+    if (!U.is_contiguous() || (size_t)U.numel() != ue || U.scalar_type() != x.scalar_type() || U.device() != x.device()) return nullptr;
+    int out[3], grid[3];
+    check(wc_conv_out_dims(&p->d, out, grid));
+    check(wc_conv_workspace_bytes(&p->d, &p->bytes));
+    const int64_t K = weight.size(0);
+    p->y_sizes = {x.size(0), K};
+    p->y_strides = {K * out[0] * out[1] * out[2], 1};
+    for (int a = 3 - nd; a < 3; ++a) p->y_sizes.push_back(out[a]);
+    if (nd == 3) p->y_strides.push_back(K * out[1] * out[2]);
+    p->y_strides.push_back(K * out[2]);
+    p->y_strides.push_back(K);
+    return p;
+  }
+  LayerPlan(const at::Tensor& x, const at::Tensor& weight, int s, std::vector<int> p, int m_, const at::Tensor& u)
+      : x_type(x.scalar_type()), w_type(weight.scalar_type()), device(x.device()), sizes(x.sizes().vec()), strides(x.strides().vec()),
+        w_sizes(weight.sizes().vec()), nd((int)x.dim() - 2), stride(s), m(m_), pads(std::move(p)), U(u), w_data(weight.data_ptr()),
+        w_version(weight.unsafeGetTensorImpl()->is_inference() ? 0 : weight._version()) {}
+
+  at::Tensor run(const at::Tensor& x, const at::Tensor& w, const at::Tensor& bias, const at::Tensor& u) const {
+    at::Tensor y = at::empty_strided(y_sizes, y_strides, x.options());
+    void* stream = stream_of(x);
+    at::Tensor ws = workspace_for(x, bytes, stream);
+    int64_t s[5];
+    strides_of(w, s);
+    check(wc_conv_forward(&d, x.data_ptr(), w.data_ptr(), s, u.defined() ? u.data_ptr() : nullptr, bias.defined() ? bias.data_ptr() : nullptr,
+                          y.data_ptr(), ws.data_ptr(), bytes, stream));
+    return y;
+  }
+
+  at::Tensor transform(const at::Tensor& w) const {
+    at::Tensor u = at::empty(U.sizes(), U.options());
+    wc_conv_desc f = d;
+    f.x_layout = 0;
+    wc_plan plan{};
+    if (!f.direct && !f.row) check(wc_plan_conv(&f, &plan));
+    int64_t s[5];
+    strides_of(w, s);
+    check(wc_filter_transform(&f, &plan, w.data_ptr(), s, u.data_ptr(), stream_of(w)));
+    return u;
+  }
+
+  // The result; with a weight that has changed since the plan was made (result, the plan for it, its transformed filter)
+  py::object call(const at::Tensor& x, const at::Tensor& weight, const std::optional<at::Tensor>& bias) const;
+
+ private:
+  static bool misaligned(const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) != 0; }
+  // a tensor with memory of its own on the GPU: no wrapper of a function transform, no subclass, nothing that carries a tangent
+  static bool plain(const at::Tensor& t) {
+    constexpr c10::DispatchKeySet wrapped({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                           c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor});
+    return t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(wrapped) && !t._fw_grad(0).defined();
+  }
+  bool fits(const at::Tensor& x, const at::Tensor& weight, const std::optional<at::Tensor>& bias) const {
+    return plain(x) && plain(weight) && (!bias || plain(*bias)) && x.scalar_type() == x_type && x.sizes() == at::IntArrayRef(sizes) &&
+           x.strides() == at::IntArrayRef(strides) && x.device() == device && !misaligned(x) && weight.scalar_type() == w_type &&
+           weight.sizes() == at::IntArrayRef(w_sizes) && weight.device() == device && !weight.is_inference() &&
+           (!bias || (bias->dim() == 1 && bias->size(0) == w_sizes[0] && bias->device() == device)) && !torch::jit::tracer::isTracing();
+  }
+};
+
+struct LayerOperands { std::shared_ptr<const LayerPlan> plan; at::Tensor w, bias, U; };       // w and bias in x's type
+
+struct LayerFunction : torch::autograd::Function<LayerFunction> {
+  static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& x, const at::Tensor& weight, const std::optional<at::Tensor>& bias,
+                            const LayerOperands& o) {
+    ctx->save_for_backward({x, o.w});
+    std::vector<int64_t> conf{o.plan->stride, o.plan->m, (int64_t)weight.scalar_type(), bias ? (int64_t)bias->scalar_type() : -1, weight.requires_grad()};
+    for (int p : o.plan->pads) conf.push_back(p);
+    ctx->saved_data["conf"] = std::move(conf);
+    return o.plan->run(x, o.w, o.bias, o.U);
+  }
+
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const at::Tensor &x = saved[0], &w = saved[1], &dy = grads[0];
+    const auto conf = ctx->saved_data["conf"].toIntVector();
+    const bool has_bias = conf[3] >= 0;
+    const int stride = (int)conf[0], m = (int)conf[1];
+    const std::vector<int> pads(conf.begin() + 5, conf.end());
+    const auto w_type = (at::ScalarType)conf[2], b_type = has_bias ? (at::ScalarType)conf[3] : w_type;
+    const bool dx = ctx->needs_input_grad(0), db = has_bias && ctx->needs_input_grad(2);
+    const bool dw = ctx->needs_input_grad(1) || (db && conf[4]);      // the sums of a bias gradient are taken beside the weight's
+    try {
+      Gradients g;
+      if (!at::GradMode::is_enabled()) g = backward_all(x, w, dy, stride, pads, m, dx, dw, db, w_type, b_type);
+      if ((dx && !g.dx.defined()) || (dw && !g.dw.defined()) || (db && !g.db.defined())) {
+        py::gil_scoped_acquire gil;                // what is left to the functions of WinoConv.py
+        const py::object rest = py::module_::import("pytorch_winoconv_amd.WinoConv").attr("gradients")(
+            x, w, dy, stride, py::tuple(py::cast(pads)), m, dx && !g.dx.defined(), dw && !g.dw.defined(), db && !g.db.defined(),
+            py::reinterpret_borrow<py::object>((PyObject*)torch::getTHPDtype(w_type)), py::reinterpret_borrow<py::object>((PyObject*)torch::getTHPDtype(b_type)));
+        const py::tuple t = rest.cast<py::tuple>();
+        if (!t[0].is_none()) g.dx = t[0].cast<at::Tensor>();
+        if (!t[1].is_none()) g.dw = t[1].cast<at::Tensor>();
+        if (!t[2].is_none()) g.db = t[2].cast<at::Tensor>();
+      }
+      return {g.dx, g.dw, g.db, at::Tensor()};
+    } catch (py::error_already_set& e) {           // exceptions reach the caller of backward() as the Python ones they are
+      py::gil_scoped_acquire gil;
+      e.restore();
+      raise();
+    } catch (const Unsupported& e) {
+      py::gil_scoped_acquire gil;
+      PyErr_SetString(PyExc_NotImplementedError, e.what());
+      raise();
+    } catch (const std::invalid_argument& e) {
+      py::gil_scoped_acquire gil;
+      PyErr_SetString(PyExc_ValueError, e.what());
+      raise();
+    } catch (const py::builtin_exception& e) {
+      py::gil_scoped_acquire gil;
+      e.set_error();
+      raise();
+    }
+  }
+
+ private:
+  [[noreturn]] static void raise() {
+    python_error error;
+    error.persist();
+    throw error;
+  }
+};
+
+py::object LayerPlan::call(const at::Tensor& x, const at::Tensor& weight, const std::optional<at::Tensor>& bias) const {
+  if (!fits(x, weight, bias)) return py::none();
+  at::Tensor y;
+  std::shared_ptr<LayerPlan> renewed;               // this plan with the filter of a weight that has changed
+  {
+    py::gil_scoped_release nogil;
+    const bool grad = at::GradMode::is_enabled() && (x.requires_grad() || weight.requires_grad() || (bias && bias->requires_grad()));
+    const bool same_weight = weight.data_ptr() == w_data && (uint32_t)weight._version() == w_version;
+    LayerOperands o{shared_from_this(), weight, bias ? *bias : at::Tensor(), U};
+    const bool cast_w = (grad || !same_weight) && w_type != x_type, cast_b = bias && bias->scalar_type() != x_type;
+    if (cast_w || cast_b) {
+      at::AutoGradMode no_grad(false);
+      if (cast_w) o.w = weight.to(x_type);
+      if (cast_b) o.bias = bias->to(x_type);
+    }
+    if (o.bias.defined()) o.bias = o.bias.contiguous();
+    if (!same_weight) {
+      renewed = std::make_shared<LayerPlan>(*this);
+      renewed->w_data = weight.data_ptr();
+      renewed->w_version = (uint32_t)weight._version();
+      renewed->U = o.U = transform(o.w);
+    }
+    y = grad ? LayerFunction::apply(x, weight, bias, o) : run(x, o.w, o.bias, o.U);
+  }
+  if (renewed) return py::make_tuple(y, renewed, renewed->U);
+  return py::cast(y);
 }
 
 // The reference's native entry point (pybind/extern.hpp:7-9): VALID convolution.  The four scratch tensors
@@ -695,6 +924,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("channels_first_out") = false, py::arg("direct") = py::none(), py::arg("row") = false);
   m.def("conv_backward_weight", &conv_backward_weight, py::arg("x"), py::arg("dy"), py::arg("w_shape"), py::arg("stride") = 1,
         py::arg("padding") = 0, py::arg("m") = 2);
+  py::class_<LayerPlan, std::shared_ptr<LayerPlan>>(m, "LayerPlan")
+      .def_static("make", &LayerPlan::make, py::arg("x"), py::arg("weight"), py::arg("stride"), py::arg("padding"), py::arg("m"), py::arg("U"))
+      .def("__call__", &LayerPlan::call, py::arg("x"), py::arg("weight"), py::arg("bias"));
   m.def("conv_backward_parameters", &conv_backward_parameters, py::arg("x"), py::arg("dy"), py::arg("w_shape"), py::arg("stride"), py::arg("padding"),
         py::arg("m"), py::arg("need_db"), py::arg("w_type"), py::arg("b_type"));
   m.def("conv_backward", &conv_backward, py::arg("x"), py::arg("w"), py::arg("dy"), py::arg("stride"), py::arg("padding"), py::arg("m"),

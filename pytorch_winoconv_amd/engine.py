@@ -548,6 +548,12 @@ def bias_gradient(dy):
     return db
 
 
+def layer_plan(x, weight, stride, padding, m, U):
+    """The compiled host layer's plan of conv_forward(x, weight, ..., U=U, row=True) for inputs of x's shape, strides and type, called as
+    plan(x, weight, bias); None where there is none."""
+    return _ext.LayerPlan.make(x, weight, stride, list(padding), m, U)
+
+
 def conv_backward(x, w, dy, stride, padding, m, need_dx, need_dw, need_db, w_type=None, b_type=None):
     """The gradients of conv_forward(x, w, bias, ...) that are asked for, in one call of the compiled host layer: (dx, dw, db), the
     last two in `w_type` and `b_type` where those are given; None for what is left to the functions below and above."""
