@@ -212,6 +212,10 @@ int wc_wino_split2d(const void* x, void* tiles, int B, int H, int W, int C,
 int wc_wino_split3d(const void* x, void* tiles, int B, int D, int H, int W, int C,
                     int block_D, int block_H, int block_W, int m, int nD, int nH, int nW,
                     int elem_size, void* stream);
+/* The same from x channel-first (B, C, D, H, W), 2-D with D = block_D = nD = 1; elements of 2 bytes: block_W and m even. */
+int wc_wino_split_channel_first(const void* x, void* tiles, int B, int C, int D, int H, int W,
+                                int block_D, int block_H, int block_W, int m, int nD, int nH, int nW,
+                                int elem_size, void* stream);
 /* Replaces WinoConcat<T> (pybind/extern.hpp:5-6, src/split_and_concat.cpp:44-76) and the
  * kernels winoConcatKernel2d / winoConcatKernel (src/split_and_concat_kernels.cu:107-129, :43-70).
  * tiles (B*[nD*]nH*nW, K, [m,] m, m) -> y channel-last (B, [oD,] oH, oW, K); partial edge

@@ -3,14 +3,14 @@
 Differences from the reference, none visible in the results for output_block_size = 2:
 the tile step follows output_block_size (the reference kernels hard-code 2:
 src/split_and_concat_kernels.cu:20-22,87-88), float16 is accepted besides float32, the
-tensors stay on the device of the input and a channel-last input is used without a copy.
+tensors stay on the device of the input and channel-last and channel-first inputs are used without a copy.
 """
 import ctypes
 
 import torch
 
 from . import _lib
-from .engine import _ptr, _stream, _require_gpu, channel_last, channel_first_view
+from .engine import _ptr, _stream, _require_gpu, channel_last, channel_last_memory, channel_first_view
 
 
 def wino_split(a, w_shape, output_block_size):
@@ -25,12 +25,16 @@ def wino_split(a, w_shape, output_block_size):
     sp = list(a.shape[2:])
     blocks = [int(w) + m - 1 for w in w_shape[2:]]
     n = [int((X + 1 - b) / m + 1) for X, b in zip(sp, blocks)]      # Split_and_Concat.py:21-23,40-41
-    a_cl = channel_last(a)                                          # Split_and_Concat.py:25,47
     n_tiles = B
     for v in n:
         n_tiles *= v
     out = torch.empty([n_tiles, C] + blocks, dtype=a.dtype, device=a.device)
     es = a.element_size()
+    if a.is_contiguous() and not channel_last_memory(a) and (es == 4 or (es == 2 and m % 2 == 0 and blocks[-1] % 2 == 0)):
+        one = [1] * (3 - nd)
+        _lib.check(lib.wc_wino_split_channel_first(_ptr(a), _ptr(out), B, C, *one, *sp, *one, *blocks, m, *one, *n, es, _stream(a)))
+        return out
+    a_cl = channel_last(a)                                          # Split_and_Concat.py:25,47
     if nd == 2:
         _lib.check(lib.wc_wino_split2d(_ptr(a_cl), _ptr(out), B, sp[0], sp[1], C, blocks[0], blocks[1],
                                        m, n[0], n[1], es, _stream(a)))

@@ -54,6 +54,7 @@ SIGNATURES = {
     "wc_padded_channels8": (_i, [_i]),
     "wc_wino_split2d": (_i, [_vp, _vp] + [_i] * 10 + [_vp]),
     "wc_wino_split3d": (_i, [_vp, _vp] + [_i] * 13 + [_vp]),
+    "wc_wino_split_channel_first": (_i, [_vp, _vp] + [_i] * 13 + [_vp]),
     "wc_wino_concat2d": (_i, [_vp, _vp] + [_i] * 6 + [_vp]),
     "wc_wino_concat3d": (_i, [_vp, _vp] + [_i] * 7 + [_vp]),
     "wc_layout_copy": (_i, [_vp, _vp, _i, _i, ctypes.c_longlong, _i, _i, _vp]),
