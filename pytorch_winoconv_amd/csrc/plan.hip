@@ -313,7 +313,7 @@ int wc_plan_conv(const wc_conv_desc* d, wc_plan* plan) {
 //    and 8x8 kernels, at most 256 channels: 1.2-1.75x) or, in 3-D, two or four (at most 128 channels:
 //    1.65-2.5x); kernels with three taps per phase are 1.8x slower that way and keep their stacked pieces.
 //  * fp32 (product bound by the MFMA rate, to which stacking adds zero taps): only 2-D plans of two to four
-//    pieces are stacked (5x5: 1.1-1.15x; 7x7 with nine pieces: 0.9-1.0x).
+//    pieces are stacked (5x5: 1.1-1.15x; 7x7 with nine pieces: 0.9-1.0x), and not all of those (pieces_apart).
 static int auto_stacked(const wc_conv_desc* d) {
   const int nd = d->ndim;
   if (d->whole_kernel || (nd == 3 && d->m != 2)) return 0;
@@ -351,6 +351,27 @@ static int auto_stacked(const wc_conv_desc* d) {
     n *= sum;
   }
   return n > 1 && n <= 4 ? 1 : 0;
+}
+
+// fp32 plans of four pieces whose products are taken apart, and added by the output transform, though auto_stacked adds them in one reduction.
+// That reduction is four times the channels, beyond what the bf16 parts of gemm.hip (fp32_in_parts) are taken for; apart each piece's
+// product is within, has a quarter of the steps on four times the workgroups and no zero taps (5x5: 121 for 144), and M, four times as long
+// to write and read, is small beside it.  The error against fp64 is half to a third (5x5, 480 channels 3.0e-6 | 6.1e-6, 3x3 stride 2, 512 1.35e-6 |
+// 4.1e-6).  us, apart | stacked, transformed filter kept: tile 4, 5x5 256 -> 64, N=1 14x14 33 | 41, 256 -> 256, N=16 28x28 133 | 152, 288 -> 128,
+// N=32 56x56 682 | 887, 288 -> 256, N=4 14x14 41.8 | 40.5 (the worst), 512 -> 512, N=16 14x14 121 | 202; tile 2, 256 -> 256, N=16 28x28 199 | 289; at stride
+// 2 as at stride 1; 4x4 256 channels 1.02 to 1.4 times as fast; 3x3 stride 2, 160 -> 256, N=4 28x28 29.9 | 29.4 (the worst), N=16 56x56
+// 72 | 95, 512 -> 64, N=1 28x28 35 | 56.  Below the lines the sides alternate with the size (5x5 of 160 channels 0.88 to 1.33), and 6x6, which has no zero
+// taps, is no faster up to 288 channels (0.85 to 1.1).  Filter transform included, 512 -> 512, N=2 14x14, all filter, 136 | 127, and where four times the
+// channels are just within the parts' range and the tiles fill the chip, 256 -> 256, N=32 28x28, 305 | 284.  The weight gradient (direct == -1) stays stacked: 5x5 256 -> 64, N=1 14x14 37 | 30, and less exact apart.
+static bool pieces_apart(const wc_conv_desc* d) {
+  if (d->dtype != WC_F32 || d->ndim != 2) return false;
+  const int kmin = d->kernel[1] < d->kernel[2] ? d->kernel[1] : d->kernel[2], kmax = d->kernel[1] + d->kernel[2] - kmin;
+  const int Cp = wc_padded_channels(d->C);
+  if (d->stride == 2 && kmin == 3 && kmax == 3) return Cp >= 160;
+  if (kmin < 4 || kmax > 5 || Cp < 256) return false;
+  long long tiles = d->N;
+  for (int a = 1; a < 3; ++a) tiles *= ceil_div((d->in[a] + 2 * d->pad[a] - d->kernel[a]) / d->stride + 1, d->m);
+  return (tiles >= 64 || (long long)Cp * d->K <= (1 << 17)) && (d->m != 4 || Cp > 256 || tiles <= 1024);
 }
 
 // Where the direct form measured faster than the Winograd plan the caller would otherwise get.  Stride 2 in 16-bit,
@@ -412,7 +433,7 @@ int wc_conv_auto(wc_conv_desc* d) {
   if (d->stacked == -1) {
     if (!d->direct && !never_direct && direct_conv_fits(d) && direct_preferred(d)) d->direct = 1;
     if (may_row && !d->direct && !d->unfused && row_conv_fits(d) && row_preferred(d)) d->row = 1;
-    d->stacked = d->direct || d->row ? 0 : auto_stacked(d);
+    d->stacked = d->direct || d->row || (!never_direct && pieces_apart(d)) ? 0 : auto_stacked(d);
   }
   if (d->stacked == 2 && d->m == 4) {
     // the shared-input plan exists for output tiles 2 and 3: tile 3 (F(3,3): fp16 error 3e-3 of the output
