@@ -165,10 +165,10 @@ int make_layout(const wc_conv_desc* d_in, Layout* L) {
   // through a channel-last copy of the images of a pass
   L->x_direct = d->x_layout == 1 && ((!L->whole() && input_transform_nchw_fits(d, &L->plan)) ||
                                      (L->direct && (direct_first_fits(d_in) || direct_first3d_fits(d_in))));      // ... and so do the first-layer kernels
-  // the row form reads channel-last x with its channels padded to a multiple of 8
+  // a copy of x for the row form has its channels padded to a multiple of 8
   const size_t x_image = (size_t)d->in[0] * d->in[1] * d->in[2] * (L->row ? wc_padded_channels8(d->C) : d->C) * L->es;
   const size_t y_image = (size_t)L->out[0] * L->out[1] * L->out[2] * d->K * L->es;
-  const bool copy_x = (d->x_layout == 1 && !L->x_direct) || (L->row && d->C % 8 != 0), copy_y = d->y_layout == 1;
+  const bool copy_x = (d->x_layout == 1 && !L->x_direct) || (L->row && row_reads_padded(d)), copy_y = d->y_layout == 1;
   // the row form's copies are the scratch that chunk_images bounds; without copies there is nothing to bound
   L->images = !L->whole() || (L->row && d->chunk_images > 0 && (copy_x || copy_y)) ? chunk : d->N;
   L->xcl_bytes = copy_x ? round256(L->images * x_image) : 0;
@@ -326,7 +326,7 @@ int forward_impl(const wc_conv_desc* d, const void* x, const void* w, const int6
     }
     void* ydst = L.ycl_bytes ? Ycl : yout;
     if (L.row) {
-      rc = timer.run(WC_STAGE_PRODUCT, [&] { return row_conv(&dcl, xin, b0, n, U, bias, ydst, stream); });
+      rc = timer.run(WC_STAGE_PRODUCT, [&] { return row_conv(&dcl, xin, L.xcl_bytes ? wc_padded_channels8(d->C) : d->C, b0, n, U, bias, ydst, stream); });
       if (rc) return rc;
     } else if (L.direct) {
       rc = timer.run(WC_STAGE_PRODUCT, [&] { return direct_conv(&dcl, xin, n, U, bias, ydst, stream); });

@@ -21,7 +21,8 @@ namespace {
 
 struct RowArgs {
   const void* x; const void* U; const void* bias; void* y;
-  int N, D, H, W, C, K;           // x (N, D, H, W, C), y (N, oD, oH, oW, K)
+  int N, D, H, W, C, K;           // x (N, D, H, W, C), C rounded up to 8; y (N, oD, oH, oW, K)
+  int x_row, tail;                // elements from a pixel of x to the next: C, or `tail` (below 8) fewer
   int oD, oH, oW, nW;             // nW tiles of 4 (5x5: 2) outputs per row
   int pd, ph, pw;
   int bn, bd, bh, bw;             // output box of a workgroup: images, planes, rows, tiles of a row
@@ -67,14 +68,32 @@ struct RowItems {
   }
 };
 
+// the first n < 8 of eight 16-bit elements, in at most three stores
+template <typename T>
+__device__ __forceinline__ void store_some(T* dst, u32x4 v, int n) {
+  unsigned next = v[0], after = v[1];
+  if (n & 4) {
+    __builtin_memcpy(dst, &v, 8);
+    dst += 4; next = v[2]; after = v[3];
+  }
+  if (n & 2) {
+    __builtin_memcpy(dst, &next, 4);
+    dst += 2; next = after;
+  }
+  if (n & 1) __builtin_memcpy(dst, &next, 2);
+}
+
 template <int KG, int TB, int S, int CS>
 constexpr int row_lds_bytes() {
   const int v = CS * 2 * 6 * S * kRowPitch, ex = 2 * KG * 3 * TB * 8 * 256, part = (CS - 1) * 2 * KG * 3 * TB * 16 * 256;
   return v > ex ? (v > part ? v : part) : (ex > part ? ex : part);
 }
 
-// KT: rows of y that are no multiple of 16 bytes.  STAY: a workgroup per CU that goes from box to box
-template <typename T, int KD, int KH, int KG, int TB, int S, int CS, bool STAY, bool KT>
+// ANY: rows of x or y that are no multiple of 16 bytes.  The last eight channels of x are loaded as they lie, ending with the last one, and
+// shifted into their places, zeros behind them, in the step that takes them: a copy of x with padded rows cost, us, C a multiple of 8 | two
+// channels fewer, copied | this: N=16 96 -> 64, 56x56 10.8 | 21.5 | 11.9, 320 -> 64 22.6 | 40.4 | 23.7, N=8 256 -> 128, 28x28 11.0 | 15.9 | 12.1, N=2 96 -> 96,
+// 28x28 7.8 | 10.2 | 8.4.  Of y's rows the last stores are cut: N=4 64 -> 464, 86x86 28, 466 channels 42 element by element, now 29.  STAY: a workgroup per CU that goes from box to box
+template <typename T, int KD, int KH, int KG, int TB, int S, int CS, bool STAY, bool ANY>
 __global__ __launch_bounds__(128 * KG * CS) __attribute__((amdgpu_waves_per_eu(2, TB == 2 ? 2 : 3)))
 void row_conv_kernel(RowArgs a) {
   using Frag = typename MfmaRow<T>::Frag;
@@ -134,15 +153,17 @@ void row_conv_kernel(RowArgs a) {
       const int zh = fast_div(s, KP == 1 ? a.f_bw : a.f_lw), iw = s - zh * lw;
       const int n = n0 + in, d = d0 + zd - a.pd, h = h0 + zh - a.ph, w = (w0 + iw) * OUT - a.pw;
       const bool ok = in < a.bn && zd < sd && zh < sh && n < a.N && (unsigned)d < (unsigned)a.D && (unsigned)h < (unsigned)a.H;
-      const int base = (((n * a.D + d) * a.H + h) * a.W + w) * a.C * 2 + g * 16;
+      const int row = ANY ? a.x_row : a.C, base = (((n * a.D + d) * a.H + h) * a.W + w) * row * 2 + g * 16;
 #pragma unroll
-      for (int j = 0; j < 6; ++j) xo[i][j] = ok && (unsigned)(w + j) < (unsigned)a.W ? base + j * a.C * 2 : (int)kOutside;
+      for (int j = 0; j < 6; ++j) xo[i][j] = ok && (unsigned)(w + j) < (unsigned)a.W ? base + j * row * 2 : (int)kOutside;
     }
   };
   find_x();
-  // the channel block is in the scalar offset; beyond the last channel of the last block lanes load zeros (cut_x)
+  // the channel block is in the scalar offset (ANY: the last one in the lane's, which shifts it); beyond the last channel of the last block
+  // lanes load zeros (cut_x)
   auto load_x = [&](int i, int j, int step) {
-    xr[i][j] = __builtin_amdgcn_raw_buffer_load_b128(xdesc, xo[i][j], min(step0 + step, a.steps - 1) * 64, 0);
+    const int block = ANY && step0 + step >= a.steps - 1 ? 0 : min(step0 + step, a.steps - 1);
+    xr[i][j] = __builtin_amdgcn_raw_buffer_load_b128(xdesc, xo[i][j], block * 64, 0);
   };
   auto cut_x = [&](int step) {
     if (step0 + step >= a.steps - 1 && (tid & 3) * 8 + (step0 + step) * 32 >= a.C) {
@@ -150,6 +171,31 @@ void row_conv_kernel(RowArgs a) {
       for (int i = 0; i < UN; ++i)
 #pragma unroll
         for (int j = 0; j < 6; ++j) xo[i][j] = (int)kOutside;
+    }
+    if constexpr (ANY) {                 // once a box; the lanes of the last eight channels start `tail` channels before (outside stays outside)
+      if (step0 + step == a.steps - 1) {
+        const unsigned by = (a.steps - 1) * 64 - ((tid & 3) * 8 + (a.steps - 1) * 32 == a.C - 8 ? a.tail * 2 : 0);
+#pragma unroll
+        for (int i = 0; i < UN; ++i)
+#pragma unroll
+          for (int j = 0; j < 6; ++j) xo[i][j] = (int)((unsigned)xo[i][j] + by);
+      }
+    }
+  };
+  auto shift_x = [&](int step) {
+    if constexpr (ANY) {
+      if (a.tail == 0 || step0 + step != a.steps - 1) return;
+      const int by = (tid & 3) * 8 + (a.steps - 1) * 32 == a.C - 8 ? a.tail : 0;
+#pragma unroll
+      for (int i = 0; i < UN; ++i)
+#pragma unroll
+        for (int j = 0; j < 6; ++j) {
+          u32x4 v = xr[i][j];
+          if (by & 4) v = u32x4{v[2], v[3], 0u, 0u};
+          if (by & 2) v = u32x4{v[1], v[2], v[3], 0u};
+          if (by & 1) v = u32x4{v[0] >> 16 | v[1] << 16, v[1] >> 16 | v[2] << 16, v[2] >> 16 | v[3] << 16, v[3] >> 16};
+          xr[i][j] = v;
+        }
     }
   };
   // one of a unit's eight channels at a time, in place: the six inputs of xr become the six elements of the tile
@@ -209,6 +255,7 @@ void row_conv_kernel(RowArgs a) {
       for (int i = from; i < to; ++i) load_u(i / 3, i / 3, i % 3);
     };
     load_u_groups(0, UD * 3 / 2);
+    shift_x(0);
     static_for<0, 8 * UN>([&](auto h_c) { transform_channel(ic<decltype(h_c)::value / 8>{}, ic<decltype(h_c)::value % 8>{}); });
 #pragma unroll
     for (int i = 0; i < UN; ++i) {
@@ -230,6 +277,7 @@ void row_conv_kernel(RowArgs a) {
         for (int b = 0; b < TB; ++b) asm volatile("" : "+v"(vo[b]));
       }
       cut_x(step + 2);
+      shift_x(step + 1);
       u32x4 vf[VD][TB];
       auto load_v = [&](int item) {                  // element item % 3 of group item / 3
         const int q = item / 3, r = (q >> 1) / KP, off = (r / KH) * a.prow + r % KH * lw + (q >> 1) % KP;
@@ -365,11 +413,14 @@ void row_conv_kernel(RowArgs a) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) bv.v[e] = T(0);
         if (bp) {
-          if constexpr (!KT) {
+          if constexpr (!ANY) {
             __builtin_memcpy(&bv, bp + min(k0, a.K - 8), 16);
+          } else if (k0 + 8 <= a.K) {
+            __builtin_memcpy(&bv, bp + k0, 16);
           } else {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) bv.v[e] = bp[min(k0 + e, a.K - 1)];
+            for (int e = 0; e < 7; ++e)
+              if (k0 + e < a.K) bv.v[e] = bp[k0 + e];
           }
         }
 #pragma unroll
@@ -393,15 +444,13 @@ void row_conv_kernel(RowArgs a) {
         for (int i = 0; i < OUT; ++i) {
           T* const dst = yp + (size_t)i * a.K;
           const bool in_row = ok && ow + i < a.oW;
-          if constexpr (!KT) {
+          if constexpr (!ANY) {
             if (in_row) *reinterpret_cast<u32x4*>(dst) = __builtin_bit_cast(u32x4, o[i]);
           } else {
             if (in_row && k0 + 8 <= a.K) {
               __builtin_memcpy(dst, &o[i], 16);          // rows of y start at any multiple of the element size
             } else if (in_row) {
-#pragma unroll
-              for (int e = 0; e < 8; ++e)
-                if (k0 + e < a.K) dst[e] = o[i].v[e];
+              store_some(dst, __builtin_bit_cast(u32x4, o[i]), a.K - k0);
             }
           }
         }
@@ -615,7 +664,7 @@ int launch_row(const RowArgs& args, const RowBox& b, void* stream) {
   a.box_fast = !filter_fits_l2(a);
   a.per_xcd = ceil_div(a.n_kb * a.n_box, kXcds);
   constexpr int bytes = row_lds_bytes<KG, TB, S, CS>();
-  const bool whole = a.K % 8 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
+  const bool whole = a.tail == 0 && a.K % 8 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
   auto fn = whole ? row_conv_kernel<T, KD, KH, KG, TB, S, CS, STAY, false> : row_conv_kernel<T, KD, KH, KG, TB, S, CS, STAY, true>;
   int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), bytes);
   if (rc) return rc;
@@ -745,19 +794,30 @@ bool row_preferred(const wc_conv_desc* d) {
   return kd == 1 ? 10.5 * products < 1500.0 * (C + K) + C * K : 3.6 * products < 512.0 * (C + K) + C * K;
 }
 
-// x (N, D, H, W, Cx) channel-last with Cx = C rounded up to 8 (zeros beyond C), 16-byte aligned; images first_image ..
-// + n_images of the batch
-int row_conv(const wc_conv_desc* d, const void* x, int first_image, int n_images, const void* U, const void* bias, void* y, void* stream) {
+// Whether x has to come with its channels padded to a multiple of 8: tall boxes, whose input goes straight to LDS, and rows of less than 16 bytes
+bool row_reads_padded(const wc_conv_desc* d) {
+  if (d->C % 8 == 0) return false;
+  const int force = test_gemm_config(), kd = d->kernel[0], kh = d->kernel[1];
+  if (d->C < 8 || (force == 21 && kh == 3)) return true;
+  if (kh != 3 || (force >= 16 && force <= 19)) return false;
+  return row_plan(d->N, d->in[0] + 2 * d->pad[0] - kd + 1, d->in[1] + 2 * d->pad[1] - 2, ceil_div(d->in[2] + 2 * d->pad[2] - 2, 4), kd, kh, d->K,
+                  ceil_div(d->C, 32)).tall_planes > 0;
+}
+
+// x (N, D, H, W, x_row) channel-last, 16-byte aligned: x_row is C, where row_reads_padded allows it, or C rounded up to 8 (zeros beyond C);
+// images first_image .. + n_images of the batch
+int row_conv(const wc_conv_desc* d, const void* x, int x_row, int first_image, int n_images, const void* U, const void* bias, void* y, void* stream) {
   WC_CHECK_ARG(row_conv_fits(d), "row form: 16-bit, stride 1, kernels 3x3, 3x3x3, 5x5 and 7x7");
   WC_CHECK_ARG(((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(U)) & 15) == 0, "row form: x and U must be 16-byte aligned");
   RowArgs a{};
   a.x = x; a.U = U; a.bias = bias; a.y = y;
   a.N = n_images; a.D = d->in[0]; a.H = d->in[1]; a.W = d->in[2]; a.C = wc_padded_channels8(d->C); a.K = d->K;
+  a.x_row = x_row; a.tail = a.C - x_row;
   a.pd = d->pad[0]; a.ph = d->pad[1]; a.pw = d->pad[2];
   a.oD = a.D + 2 * a.pd - d->kernel[0] + 1; a.oH = a.H + 2 * a.ph - d->kernel[1] + 1; a.oW = a.W + 2 * a.pw - d->kernel[2] + 1;
   a.nW = ceil_div(a.oW, row_outputs_of(d->kernel[1]));
   a.steps = ceil_div(a.C, 32);
-  a.x_bytes = (int)((long long)a.N * a.D * a.H * a.W * a.C * 2);
+  a.x_bytes = (int)((long long)a.N * a.D * a.H * a.W * a.x_row * 2);
   a.u_bytes = (int)(row_u_elems(d) * 2);
   const int force = test_gemm_config();
   // the shapes are the whole batch's, so that the passes of a batch add in the order of the batch in one pass
@@ -766,15 +826,16 @@ int row_conv(const wc_conv_desc* d, const void* x, int first_image, int n_images
   if (force == 21 && d->kernel[1] == 3) plan.tall_planes = d->N * a.oD;
   const int tall = std::min(std::max(plan.tall_planes - first_image * a.oD, 0), n_images * a.oD);
   if (tall > 0) {
+    WC_CHECK_ARG(a.tail == 0, "row form: tall boxes of %d channels", x_row);
     const int rc = tall_row_conv(d, x, tall, U, bias, y, stream);
     if (rc || tall == n_images * a.oD) return rc;
     // the rest: the images from there on, of the first of them (the only one then) the planes from there on
     const int images = tall / a.oD, first_d = tall - images * a.oD;
-    a.x = static_cast<const unsigned char*>(x) + (long long)images * a.D * a.H * a.W * a.C * 2;
+    a.x = static_cast<const unsigned char*>(x) + (long long)images * a.D * a.H * a.W * a.x_row * 2;
     a.y = static_cast<unsigned char*>(y) + (long long)tall * a.oH * a.oW * a.K * 2;
     a.N -= images;
     a.oD -= first_d; a.pd -= first_d;
-    a.x_bytes = (int)((long long)a.N * a.D * a.H * a.W * a.C * 2);
+    a.x_bytes = (int)((long long)a.N * a.D * a.H * a.W * a.x_row * 2);
   }
   return dispatch_dtype(d->dtype, [&](auto t) -> int {
     using T = decltype(t);

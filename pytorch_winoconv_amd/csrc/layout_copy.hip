@@ -10,7 +10,7 @@
 // tiles of 64 x 64 through LDS in accesses of 2 or 4 bytes | this, 16 bit: 6 x 100 x 2745 7.8 | 3.9, 64 x 256 x 3136 51 | 35 (5.8 TB/s),
 // back 50 | 35, 64 x 128 x 3136 20.4 | 18.2; 32 bit, 64 x 256 x 3136 102 | 74, 8 x 256 x 3136 12.0 | 9.9; 32 x 3 x 50176 (a thread to a
 // column) 42 | 9.
-#include "wc_common.h"
+#include "wc_transform.h"
 
 #include <algorithm>
 
@@ -103,31 +103,42 @@ int transpose_images(const void* src, void* dst, long long n, long long R, long 
   return transpose_padded(src, dst, n, R, Q, R, elem_size, stream);
 }
 
-// Rows of C 16-bit elements to rows of Cx, a multiple of 8: a thread writes 16 bytes from eight reads of two bytes that
-// neighbouring threads take from the same lines (rows of C elements start anywhere).
+// Rows of C 16-bit elements to rows of Cx, a multiple of 8: a thread moves 16 bytes, from wherever its row starts; the last of a row
+// comes from the row's last eight elements, shifted (rows of less than eight: element by element).
 struct PadArgs {
   const unsigned short* src; void* dst;
   int C, chunks;               // chunks of 8 elements in a row of dst
   long long total;             // rows x chunks
+  FastDiv f_chunks;
 };
 
 __global__ __launch_bounds__(256) void pad_rows_kernel(PadArgs a) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= a.total) return;
-  const long long row = i / a.chunks;
+  const long long row = a.total < (1ll << 31) ? fast_div((int)i, a.f_chunks) : i / a.chunks;
   const int c = (int)(i - row * a.chunks) * 8;
   const unsigned short* p = a.src + row * a.C + c;
-  Pack<unsigned short, 8> v;
+  unsigned long long v[2] = {0, 0};
+  if (c + 8 <= a.C) {
+    __builtin_memcpy(v, p, 16);
+  } else if (a.C >= 8) {
+    const int bits = (c + 8 - a.C) * 16;         // 16 to 112
+    __builtin_memcpy(v, p - bits / 16, 16);
+    if (bits >= 64) v[0] = v[1] >> (bits - 64), v[1] = 0;
+    else v[0] = v[0] >> bits | v[1] << (64 - bits), v[1] >>= bits;
+  } else {
 #pragma unroll
-  for (int e = 0; e < 8; ++e) v.v[e] = c + e < a.C ? p[e] : (unsigned short)0;
-  reinterpret_cast<Pack<unsigned short, 8>*>(a.dst)[i] = v;
+    for (int e = 0; e < 7; ++e)
+      if (e < a.C) v[e / 4] |= (unsigned long long)p[e] << e % 4 * 16;
+  }
+  __builtin_memcpy(static_cast<unsigned char*>(a.dst) + i * 16, v, 16);
 }
 
 int pad_channels(const void* src, void* dst, long long n, int C, int Cx, long long S, bool channel_first, void* stream) {
   WC_CHECK_ARG(src && dst && n > 0 && C > 0 && Cx >= C && Cx % 8 == 0 && S > 0, "pad_channels: null pointer or empty tensor");
   if (channel_first) return transpose_padded(src, dst, n, C, S, Cx, 2, stream);
   PadArgs a;
-  a.src = static_cast<const unsigned short*>(src); a.dst = dst; a.C = C; a.chunks = Cx / 8; a.total = n * S * a.chunks;
+  a.src = static_cast<const unsigned short*>(src); a.dst = dst; a.C = C; a.chunks = Cx / 8; a.total = n * S * a.chunks; a.f_chunks = make_fast_div(a.chunks);
   const long long blocks = ceil_div_ll(a.total, 256);
   WC_CHECK_ARG(blocks < (1ll << 31), "pad_channels: problem too large");
   hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), a);
