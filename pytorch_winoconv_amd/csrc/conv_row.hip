@@ -68,21 +68,6 @@ struct RowItems {
   }
 };
 
-// the first n < 8 of eight 16-bit elements, in at most three stores
-template <typename T>
-__device__ __forceinline__ void store_some(T* dst, u32x4 v, int n) {
-  unsigned next = v[0], after = v[1];
-  if (n & 4) {
-    __builtin_memcpy(dst, &v, 8);
-    dst += 4; next = v[2]; after = v[3];
-  }
-  if (n & 2) {
-    __builtin_memcpy(dst, &next, 4);
-    dst += 2; next = after;
-  }
-  if (n & 1) __builtin_memcpy(dst, &next, 2);
-}
-
 template <int KG, int TB, int S, int CS>
 constexpr int row_lds_bytes() {
   const int v = CS * 2 * 6 * S * kRowPitch, ex = 2 * KG * 3 * TB * 8 * 256, part = (CS - 1) * 2 * KG * 3 * TB * 16 * 256;
@@ -563,37 +548,54 @@ enum RowShape { kRowWide, kRowHalf, kRowSmall, kRowSplit };
 // tall_planes: output planes, images in 2-D, that go to tall boxes; the rest is rest_n images of rest_d planes
 struct RowPlan { RowShape shape; RowBox box; long long wide_groups; int tall_planes, rest_n, rest_d; double us; };
 
+//
+// How long a launch of each takes, in units of a full round of the wide shape, fitted to 330 layers drawn over 1 to 64 images, 32 to 512 channels and
+// 7 to 112 rows (3-D: 1 to 8, 32 to 128, 14 to 56; three boxes in four are no whole rounds), each timed in every shape.  Steps of a line are
+// where a CU's workgroups change their number: half boxes are two to a CU (one in 3-D, whose boxes take all of its LDS), small ones three.
+// Over 300 layers drawn anew the choice takes 1.6 % longer than the fastest shape of each in the mean, with a line through the origin for
+// half boxes, and small ones up to one a CU only, 3.2 %.  fp16, us, wide | half | small: 280 half boxes of 7 steps 25.2 | 25.9 |
+// 21.0, 252 of 7 steps 22.5 | 16.7 | 21.4; 3-D, 280 of 2 steps 18.0 | 26.2 | 20.6, 160 17.7 | 25.2 | 27.9 (two rounds of half boxes, one of wide
+// ones).  7x7, 532 small boxes of 8 steps of which half the channels are none 77 | - | 75, split 55.
+struct RowModel { double wide, wide_round, half, half_two, half_more, half_at, half_step, small_two, small_three, small_more; };
+constexpr RowModel kRow3x3{0.86, 0.92, 0.60, 0.97, 1.27, 1.0, 0.12, 1.6, 2.1, 0.82}, kRow5x5{0.82, 0.80, 0.58, 0.75, 1.15, 0.85, 0.10, 1.25, 1.7, 0.68},
+    kRow3d{0.78, 0.72, 0.53, 1.06, 0.0, 0.0, 0.0, 1.2, 1.7, 0.60};
+
 RowPlan make_row_shape(int N, int oD, int oH, int nW, int kd, int kh, int K, int steps) {
   RowPlan p{};
   const RowBox wide = choose_box(N, oD, oH, nW, kd, kh, 64, 128), half = kd == 1 ? choose_box(N, oD, oH, nW, kd, kh, 64, 64) : wide;
-  const long long n_wide = wide.boxes * ceil_div(K, 128), n_half = half.boxes * ceil_div(K, 64);
+  const RowBox small = choose_box(N, oD, oH, nW, kd, kh, 32, 64);
+  const long long n_wide = wide.boxes * ceil_div(K, 128), n_half = half.boxes * ceil_div(K, 64), n_small = small.boxes * ceil_div(K, 64);
+  auto rounds = [](long long n) { return (double)((n + kCus - 1) / kCus); };
+  auto take = [&](RowShape shape, const RowBox& box, double us) {
+    if (p.us == 0.0 || us < p.us) { p.shape = shape; p.box = box; p.us = us; }
+  };
   p.wide_groups = n_wide;
   if (kh == 7) {
     // Seven rows' halo leaves 64 tiles all of a wide workgroup's LDS, 32 a third of a CU's (kRowSmall) or, with the channels in
     // two shares, two thirds (kRowSplit).  us a step of 32 channels: small 4 for every one that a CU gets, wide 7 alone and 10.5
     // where all CUs have one.  Measured, wide | small | split, fp16: N=6 100 -> 150, 45x61 46 | 52 | 53, N=16 64 -> 64, 56x56
     // 42 | 26 | 38, N=32 128 -> 128, 112x112 421 | 600 | 802, N=1 512 -> 512, 14x14 117 | 55 | 33, 64 -> 64, 28x28 18 | 9.8 | 8.7.
-    const RowBox small = choose_box(N, oD, oH, nW, kd, kh, 32, 64);
-    const long long n_small = small.boxes * ceil_div(K, 64), n_split = small.boxes * ceil_div(K, 32);
-    const double t_wide = (double)((n_wide + kCus - 1) / kCus) * (std::min(10.5, 7 + 3.5 * n_wide / kCus) * steps + 4);
-    if (steps >= 2 && n_split <= kCus) { p.shape = kRowSplit; p.box = small; }
-    else if (4.0 * steps * ((n_small + kCus - 1) / kCus) <= t_wide) { p.shape = kRowSmall; p.box = small; }
-    else { p.shape = kRowWide; p.box = wide; }
+    const long long n_split = small.boxes * ceil_div(K, 32);
+    if (steps < 2 || n_split > kCus) {
+      take(kRowWide, wide, rounds(n_wide) * ((n_wide <= kCus ? 6.2 + 3.5 * n_wide / kCus : 10.5) * steps + 4));
+      take(kRowSmall, small, 4.0 * steps * std::max(1.0, 1.08 * n_small / kCus));
+    }
+    // in several rounds only where half of a small workgroup's channels would be none; beyond eight rounds its reads of x are no longer met in L2
+    if (steps >= 2 && (n_split <= kCus || (K <= 32 && n_split <= 8 * kCus))) take(kRowSplit, small, rounds(n_split) * (1.05 * steps + 1));
     return p;
   }
-  const RowBox small = choose_box(N, oD, oH, nW, kd, kh, 32, 64);
-  const double us_small = 0.4 * steps * kd * kh + 4;
+  const double us_small = 0.4 * steps * kd * kh + 4, unit = ((kd == 1 ? 0.82 * kh : 6.9) * steps + 7) / 0.92;
   if (steps >= 4) {
     const RowBox split = choose_box(N, oD, oH, nW, kd, kh, 32, 32);
-    if (split.boxes * ceil_div(K, 32) <= kCus) { p.shape = kRowSplit; p.box = split; p.us = us_small; return p; }
+    if (split.boxes * ceil_div(K, 32) <= kCus) { take(kRowSplit, split, us_small); return p; }
   }
-  if (small.boxes * ceil_div(K, 64) <= kCus) { p.shape = kRowSmall; p.box = small; p.us = us_small; return p; }
-  // rounds of the chip; of two workgroups per CU one starts as soon as another ends, so their last round is not a whole one.
-  // 3-D boxes of the half shape take two units of input per thread
-  const double t_wide = n_wide <= kCus ? 0.86 : 0.92 * (double)((n_wide + kCus - 1) / kCus), t_half = (kd == 1 ? 1.0 : 1.2) * (n_half / (2.0 * kCus) + 0.12);
-  p.shape = t_wide <= t_half ? kRowWide : kRowHalf;
-  p.box = p.shape == kRowWide ? wide : half;
-  p.us = std::min(t_wide, t_half) * ((kd == 1 ? 0.82 * kh : 6.9) * steps + 7) / 0.92;
+  if (n_small <= kCus) { take(kRowSmall, small, us_small); return p; }
+  const RowModel& m = kd == 3 ? kRow3d : kh == 5 ? kRow5x5 : kRow3x3;
+  // (seven whole rounds of 3-D boxes, N=8 128 -> 128, 16x56x56, took 0.84 of a unit each)
+  take(kRowWide, wide, unit * (n_wide <= kCus ? m.wide : (kd == 3 && n_wide > 4 * kCus ? 0.86 : m.wide_round) * rounds(n_wide)));
+  take(kRowHalf, half, unit * (n_half <= kCus ? m.half : kd == 3 ? m.half * rounds(n_half) : n_half <= 2 * kCus ? m.half_two
+                               : std::max(m.half_more, m.half_at * n_half / (2.0 * kCus) + m.half_step)));
+  take(kRowSmall, small, us_small * (n_small <= 2 * kCus ? m.small_two : n_small <= 3 * kCus ? m.small_three : m.small_more * n_small / kCus));
   return p;
 }
 
@@ -604,11 +606,14 @@ RowPlan make_row_shape(int N, int oD, int oH, int nW, int kd, int kh, int K, int
 // hold 123 of 128 planes, 3 rounds, the other 5 planes 20 us; seven images and one were 3 rounds of 686 boxes and 37 us).  The
 // model's constants are measured ones (fp16, us, this shape alone in whole rounds | a box: 512 -> 512, 28x28 157 | 78 for 32 half
 // blocks, 256 -> 256, 56x56 175 | 44 for 16).
-RowPlan make_row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int steps) {
+RowPlan make_row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int C) {
+  const int steps = ceil_div(C, 32);
   RowPlan best = make_row_shape(N, oD, oH, nW, kd, kh, K, steps);
   best.rest_n = N; best.rest_d = oD;
   if (kh != 3) return best;
   const double box_us = 2.1 * 2 * steps * kd + 10.5;
+  // tall boxes read padded rows: the copy at twice the rate that it reaches (tests/test_abi_host.py takes N=64 250 -> 256, 56x56 for a layer with one)
+  const double copy_us = C % 8 ? 3 + N * (double)oD * oH * nW * 4 * C * 4 / 9e6 : 0;
   const long long per_group = (long long)ceil_div(oH, 4) * ceil_div(K, 128), planes = (long long)N * oD;
   const long long boxes = ceil_div_ll(planes * nW, 32) * per_group;
   const long long groups = boxes / kCus * kCus / per_group;       // groups of 32 columns in whole rounds
@@ -625,7 +630,7 @@ RowPlan make_row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int 
       p.rest_n = rest_n; p.rest_d = rest_d;
     }
     const long long rounds = ceil_div_ll(ceil_div_ll(n * nW, 32) * per_group, kCus);
-    p.us += rounds * box_us + (rest > 0 ? 2 : 0);
+    p.us += rounds * box_us + (rest > 0 ? 2 : 0) + copy_us;
     p.tall_planes = (int)n;
     if (p.us < best.us) best = p;
   }
@@ -634,15 +639,15 @@ RowPlan make_row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int 
 }
 
 // The search over boxes takes some microseconds: the last plans of a host thread are kept.
-RowPlan row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int steps) {
+RowPlan row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int C) {
   struct Entry { int key[8]; RowPlan plan; };
   thread_local Entry cache[64] = {};
-  const int key[8] = {N, oD, oH, nW, kd, kh, K, steps};
+  const int key[8] = {N, oD, oH, nW, kd, kh, K, C};
   unsigned h = 2166136261u;
   for (int v : key) h = (h ^ (unsigned)v) * 16777619u;
   Entry& e = cache[(h ^ (h >> 15)) % 64];
   if (!std::equal(key, key + 8, e.key)) {
-    e.plan = make_row_plan(N, oD, oH, nW, kd, kh, K, steps);
+    e.plan = make_row_plan(N, oD, oH, nW, kd, kh, K, C);
     std::copy(key, key + 8, e.key);
   }
   return e.plan;
@@ -784,12 +789,12 @@ bool row_preferred(const wc_conv_desc* d) {
   if (d->kernel[1] == 7) {
     if (d->m != 4 || d->dtype != WC_F16 || wc_padded_channels(d->C) > 256) return true;
     const int oH = d->in[1] + 2 * d->pad[1] - 6, oW = d->in[2] + 2 * d->pad[2] - 6;
-    return row_no_slower_7x7(d, row_plan(d->N, 1, oH, ceil_div(oW, 3), 1, 7, d->K, ceil_div(d->C, 32)));
+    return row_no_slower_7x7(d, row_plan(d->N, 1, oH, ceil_div(oW, 3), 1, 7, d->K, d->C));
   }
   if (d->kernel[1] == 5) return row_preferred_5x5(d);
   if (d->m != 4) return true;
   const int kd = d->kernel[0], oD = d->in[0] + 2 * d->pad[0] - kd + 1, oH = d->in[1] + 2 * d->pad[1] - 2, oW = d->in[2] + 2 * d->pad[2] - 2;
-  if (row_plan(d->N, oD, oH, ceil_div(oW, 4), kd, 3, d->K, ceil_div(d->C, 32)).wide_groups <= 3 * kCus / 2) return true;
+  if (row_plan(d->N, oD, oH, ceil_div(oW, 4), kd, 3, d->K, d->C).wide_groups <= 3 * kCus / 2) return true;
   const double C = d->C, K = d->K, products = (double)wc_padded_channels(d->C) * (ceil_div(d->K, 64) * 64.0);
   return kd == 1 ? 10.5 * products < 1500.0 * (C + K) + C * K : 3.6 * products < 512.0 * (C + K) + C * K;
 }
@@ -801,7 +806,7 @@ bool row_reads_padded(const wc_conv_desc* d) {
   if (d->C < 8 || (force == 21 && kh == 3)) return true;
   if (kh != 3 || (force >= 16 && force <= 19)) return false;
   return row_plan(d->N, d->in[0] + 2 * d->pad[0] - kd + 1, d->in[1] + 2 * d->pad[1] - 2, ceil_div(d->in[2] + 2 * d->pad[2] - 2, 4), kd, kh, d->K,
-                  ceil_div(d->C, 32)).tall_planes > 0;
+                  d->C).tall_planes > 0;
 }
 
 // x (N, D, H, W, x_row) channel-last, 16-byte aligned: x_row is C, where row_reads_padded allows it, or C rounded up to 8 (zeros beyond C);
@@ -821,7 +826,7 @@ int row_conv(const wc_conv_desc* d, const void* x, int x_row, int first_image, i
   a.u_bytes = (int)(row_u_elems(d) * 2);
   const int force = test_gemm_config();
   // the shapes are the whole batch's, so that the passes of a batch add in the order of the batch in one pass
-  RowPlan plan = row_plan(d->N, a.oD, a.oH, a.nW, d->kernel[0], d->kernel[1], a.K, a.steps);
+  RowPlan plan = row_plan(d->N, a.oD, a.oH, a.nW, d->kernel[0], d->kernel[1], a.K, d->C);
   if (force >= 16 && force <= 19) { plan.shape = (RowShape)(force - 16); plan.tall_planes = 0; plan.rest_n = -1; }
   if (force == 21 && d->kernel[1] == 3) plan.tall_planes = d->N * a.oD;
   const int tall = std::min(std::max(plan.tall_planes - first_image * a.oD, 0), n_images * a.oD);

@@ -334,9 +334,7 @@ void tall_row_kernel(TallArgs a) {
             if (in_row && k0 + 8 <= a.K) {
               __builtin_memcpy(dst, &o[i], 16);          // rows of y start at any multiple of the element size
             } else if (in_row) {
-#pragma unroll
-              for (int e = 0; e < 8; ++e)
-                if (k0 + e < a.K) dst[e] = o[i].v[e];
+              store_some(dst, __builtin_bit_cast(u32x4, o[i]), a.K - k0);
             }
           }
         }

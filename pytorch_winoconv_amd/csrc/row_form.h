@@ -76,4 +76,19 @@ __device__ __forceinline__ RowOutputs<OUT> row_outputs(float m0, float sa, float
   }
 }
 
+// the first n < 8 of eight 16-bit elements, in at most three stores
+template <typename T>
+__device__ __forceinline__ void store_some(T* dst, u32x4 v, int n) {
+  unsigned next = v[0], after = v[1];
+  if (n & 4) {
+    __builtin_memcpy(dst, &v, 8);
+    dst += 4; next = v[2]; after = v[3];
+  }
+  if (n & 2) {
+    __builtin_memcpy(dst, &next, 4);
+    dst += 2; next = after;
+  }
+  if (n & 1) __builtin_memcpy(dst, &next, 2);
+}
+
 }  // namespace wc
