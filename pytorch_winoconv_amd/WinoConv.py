@@ -12,6 +12,7 @@ is cached and recomputed only when the weight changes.
 """
 import torch
 from torch import nn
+from torch.multiprocessing.reductions import StorageWeakRef
 import torch.nn.functional as F
 
 from . import engine, matrix_conv, matrix_conv3d
@@ -87,6 +88,12 @@ def gradients(x, w, dy, stride, padding, m, need_dx, need_dw, need_db, w_type, b
     return dx, dw, db
 
 
+def _held(weight):
+    """What a transformed filter was made from.  The weak reference keeps the storage's identity, though not its memory: weights that are
+    new tensors in every pass (functional_call, parametrizations) come to lie where the last one did."""
+    return weight._version, weight.data_ptr(), weight.stride(), StorageWeakRef(weight.untyped_storage())
+
+
 class _WinoConvNd(nn.Module):
     nd = 2
 
@@ -104,14 +111,15 @@ class _WinoConvNd(nn.Module):
         nn.init.kaiming_normal_(self.weight)
         if self.bias is not None:
             nn.init.zeros_(self.bias)
-        self._cache = None
 
+    # (what the filter was transformed from and for, the transformed filter)
+    _cache = None
     # (hyperparameters, the compiled host layer's plan for the last input's shape or None, that shape): planned when a shape comes a
     # second time running, so a program whose shapes alternate pays nothing.  Copies and files go without.
     _plan = None
 
     def __getstate__(self):
-        return {k: v for k, v in self.__dict__.items() if k != "_plan"}
+        return {k: v for k, v in self.__dict__.items() if k not in ("_plan", "_cache")}
 
     def _winograd_ok(self, x):
         # The reference hands every strided or dilated layer (and every kernel up to 3 x 3) to the stock
@@ -167,7 +175,7 @@ class _WinoConvNd(nn.Module):
             if type(y) is tuple:
                 y, renewed, U = y
                 self.__dict__["_plan"] = (conf, renewed, plan[2])
-                self.__dict__["_cache"] = ((weight._version, weight.data_ptr()) + self._cache[0][2:], U)
+                self.__dict__["_cache"] = (_held(weight) + self._cache[0][4:], U)
             if y is not None:
                 return y
         conv = F.conv2d if self.nd == 2 else F.conv3d
@@ -184,7 +192,7 @@ class _WinoConvNd(nn.Module):
         # the form of the plan (Winograd pieces, or the direct form the library takes for large strided problems)
         # depends on the batch size too, and the transformed filter of one form does not fit the other
         form = engine.plan_form(x.shape, w.shape, x.dtype, self.stride[0], self.padding, m, row=True)
-        key = (weight._version, weight.data_ptr(), tuple(x.shape[2:]), x.dtype, m, form)
+        key = _held(weight) + (tuple(x.shape[2:]), x.dtype, m, form)
         if self._cache is None or self._cache[0] != key:
             U = engine.transform_filter(w.detach(), x.shape, self.stride[0], self.padding, m, row=True)
             self._cache = (key, U)

@@ -724,6 +724,9 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
   int nd, stride, m;
   std::vector<int> pads;
   at::Tensor U;
+  // the weight that U was made from; the weak pointer keeps the storage's identity and not its memory
+  c10::weak_intrusive_ptr<c10::StorageImpl> w_storage;
+  std::vector<int64_t> w_strides;
   const void* w_data;
   uint32_t w_version;
 
@@ -755,8 +758,8 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
   }
   LayerPlan(const at::Tensor& x, const at::Tensor& weight, int s, std::vector<int> p, int m_, const at::Tensor& u)
       : x_type(x.scalar_type()), w_type(weight.scalar_type()), device(x.device()), sizes(x.sizes().vec()), strides(x.strides().vec()),
-        w_sizes(weight.sizes().vec()), nd((int)x.dim() - 2), stride(s), m(m_), pads(std::move(p)), U(u), w_data(weight.data_ptr()),
-        w_version(weight.unsafeGetTensorImpl()->is_inference() ? 0 : weight._version()) {}
+        w_sizes(weight.sizes().vec()), nd((int)x.dim() - 2), stride(s), m(m_), pads(std::move(p)), U(u), w_storage(weight.storage().getWeakStorageImpl()),
+        w_strides(weight.strides().vec()), w_data(weight.data_ptr()), w_version(weight.unsafeGetTensorImpl()->is_inference() ? 0 : weight._version()) {}
 
   at::Tensor run(const at::Tensor& x, const at::Tensor& w, const at::Tensor& bias, const at::Tensor& u) const {
     at::Tensor y = at::empty_strided(y_sizes, y_strides, x.options());
@@ -870,7 +873,8 @@ py::object LayerPlan::call(const at::Tensor& x, const at::Tensor& weight, const 
   {
     py::gil_scoped_release nogil;
     const bool grad = at::GradMode::is_enabled() && (x.requires_grad() || weight.requires_grad() || (bias && bias->requires_grad()));
-    const bool same_weight = weight.data_ptr() == w_data && (uint32_t)weight._version() == w_version;
+    const bool same_weight = weight.data_ptr() == w_data && (uint32_t)weight._version() == w_version && weight.strides() == at::IntArrayRef(w_strides) &&
+                             weight.storage().unsafeGetStorageImpl() == w_storage._unsafe_get_target();
     LayerOperands o{shared_from_this(), weight, bias ? *bias : at::Tensor(), U};
     const bool cast_w = (grad || !same_weight) && w_type != x_type, cast_b = bias && bias->scalar_type() != x_type;
     if (cast_w || cast_b) {
@@ -881,6 +885,8 @@ py::object LayerPlan::call(const at::Tensor& x, const at::Tensor& weight, const 
     if (o.bias.defined()) o.bias = o.bias.contiguous();
     if (!same_weight) {
       renewed = std::make_shared<LayerPlan>(*this);
+      renewed->w_storage = weight.storage().getWeakStorageImpl();
+      renewed->w_strides = weight.strides().vec();
       renewed->w_data = weight.data_ptr();
       renewed->w_version = (uint32_t)weight._version();
       renewed->U = o.U = transform(o.w);

@@ -110,3 +110,23 @@ def test_threads_and_streams(dev):
     for t in threads:
         t.join()
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_weights_that_lie_where_the_last_one_did(dev):
+    """New tensors in every call, freed after it; the same memory in another order; a module that was copied."""
+    layer = pkg.WinoConv2d(24, 24, 3, padding=1, bias=False, device=dev, dtype=torch.float16).requires_grad_(False)
+    x = torch.randn(2, 24, 10, 11, device=dev).half().contiguous(memory_format=torch.channels_last)
+    places = set()
+    for i in range(6):
+        w = torch.full((24, 24, 3, 3), float(i), device=dev, dtype=torch.float16)
+        places.add(w.data_ptr())
+        y = torch.func.functional_call(layer, {"weight": w}, (x,))
+        del w
+        assert torch.equal(y, pkg.engine.conv_forward(x, torch.full((24, 24, 3, 3), float(i), device=dev, dtype=torch.float16), None, 1, 1, layer._tile_for(x.dtype), row=True))
+    assert len(places) < 6
+    w = torch.randn(24, 24, 3, 3, device=dev).half()
+    for _ in range(2):
+        for v in (w, w.transpose(0, 1), w.transpose(2, 3), w):
+            y = torch.func.functional_call(layer, {"weight": v}, (x,))
+            assert torch.equal(y, pkg.engine.conv_forward(x, v.contiguous(), None, 1, 1, layer._tile_for(x.dtype), row=True))
+    assert copy.deepcopy(layer)._cache is None and torch.equal(copy.deepcopy(layer)(x), layer(x))
