@@ -22,7 +22,6 @@ namespace {
 struct RowArgs {
   const void* x; const void* U; const void* bias; void* y;
   int N, D, H, W, C, K;           // x (N, D, H, W, C), C rounded up to 8; y (N, oD, oH, oW, K)
-  int x_row, tail;                // elements from a pixel of x to the next: C, or `tail` (below 8) fewer
   int oD, oH, oW, nW;             // nW tiles of 4 (5x5: 2) outputs per row
   int pd, ph, pw;
   int bn, bd, bh, bw;             // output box of a workgroup: images, planes, rows, tiles of a row
@@ -35,6 +34,7 @@ struct RowArgs {
   int x_bytes, u_bytes;
   int lw;                         // tiles of a row of the box's input (7 taps: one more than bw)
   FastDiv f_lw;
+  int x_row, tail;                // elements from a pixel of x to the next: C, or `tail` (below 8) fewer
 };
 
 constexpr int kRowPitch = 64;     // LDS bytes per (element, row of a tile): 32 channels in four chunks of 16 bytes
@@ -138,9 +138,9 @@ void row_conv_kernel(RowArgs a) {
       const int zh = fast_div(s, KP == 1 ? a.f_bw : a.f_lw), iw = s - zh * lw;
       const int n = n0 + in, d = d0 + zd - a.pd, h = h0 + zh - a.ph, w = (w0 + iw) * OUT - a.pw;
       const bool ok = in < a.bn && zd < sd && zh < sh && n < a.N && (unsigned)d < (unsigned)a.D && (unsigned)h < (unsigned)a.H;
-      const int row = ANY ? a.x_row : a.C, base = (((n * a.D + d) * a.H + h) * a.W + w) * row * 2 + g * 16;
+      const int base = (((n * a.D + d) * a.H + h) * a.W + w) * (ANY ? a.x_row : a.C) * 2 + g * 16;
 #pragma unroll
-      for (int j = 0; j < 6; ++j) xo[i][j] = ok && (unsigned)(w + j) < (unsigned)a.W ? base + j * row * 2 : (int)kOutside;
+      for (int j = 0; j < 6; ++j) xo[i][j] = ok && (unsigned)(w + j) < (unsigned)a.W ? base + j * (ANY ? a.x_row : a.C) * 2 : (int)kOutside;
     }
   };
   find_x();
