@@ -12,15 +12,29 @@
 // compile-time body of their piece; anything else (whole-kernel tiles) the generic kernel.
 #include "filter_transform_impl.h"
 
+#include <cstdlib>
+
 namespace wc {
 
-// Single piece with compile-time kinds: one thread per (k, VEC channels).
+// Single piece with compile-time kinds: one thread per (k, VEC channels).  `k_fast`: w's output channels are closer in memory than its input
+// channels (an input gradient's filter, which is the layer's with the two exchanged): a wavefront takes 8 of them x 8 vectors of channels, so
+// that a load meets a quarter of the lines that one along the channels does, and U is written in runs of 64 bytes.  Bound by the
+// way of its loads from L2, on few workgroups: those of one wavefront spread it over the chip.  us, along the channels | this, tile 2,
+// fp16 128 -> 128 6.5 | 3.3, 128 <- 256 6.6 | 3.4, fp32 128 -> 128 4.6 | 3.2; tile 4, fp16 256 -> 256 7.6 | 4.4, 512 -> 512 11.2 | 9.7, fp32 256 -> 256
+// 6.2 | 5.8, 512 -> 512 16.9 | 14.9, but 181 <- 384 5.9 | 7.0: fp32 only in whole groups of 8.
 template <typename T, int K0, int K1, int K2, bool DENSE>
-__global__ __launch_bounds__(256) void filter_transform_fast_kernel(const FilterFastArgs a) {
-  filter_fast_body<T, K0, K1, K2, DENSE>(a, blockIdx.x * 256 + threadIdx.x);
+__global__ __launch_bounds__(256) void filter_transform_fast_kernel(const FilterFastArgs a, int k_fast) {
+  int idx = blockIdx.x * blockDim.x + threadIdx.x;
+  if (!DENSE && k_fast) {
+    const int cvecs = a.Cp / fast_vec<T, K0, K1, K2>(), blocks = (cvecs + 7) / 8, block = idx >> 6;
+    const int k = block / blocks * 8 + (idx & 7), cv = block % blocks * 8 + (idx >> 3 & 7);
+    if (cv >= cvecs) return;
+    idx = k * cvecs + cv;                // a k beyond the last is beyond the last index
+  }
+  filter_fast_body<T, K0, K1, K2, DENSE>(a, idx);
 }
 
-using FilterFastKernel = void (*)(FilterFastArgs);
+using FilterFastKernel = void (*)(FilterFastArgs, int);
 
 template <typename T, bool DENSE>
 static FilterFastKernel pick_fast(int k0, int k1, int k2) {
@@ -178,9 +192,11 @@ extern "C" int wc_filter_transform(const wc_conv_desc* d, const wc_plan* plan, c
       FilterFastKernel fn = dispatch_dtype(d->dtype, [&](auto t) {
         return dense ? pick_fast<decltype(t), true>(k0, k1, k2) : pick_fast<decltype(t), false>(k0, k1, k2);
       });
-      const long long n = (long long)d->K * (f.Cp / vec);
+      const bool k_fast = !dense && std::llabs(f.s[0]) < std::llabs(f.s[1]) && (d->dtype != WC_F32 || d->K % 8 == 0);
+      const long long n = k_fast ? (long long)ceil_div(d->K, 8) * ceil_div(f.Cp / vec, 8) * 64 : (long long)d->K * (f.Cp / vec);
       WC_CHECK_ARG(n < (1ll << 31), "wc_filter_transform: problem too large");
-      hipLaunchKernelGGL(fn, dim3((unsigned)ceil_div_ll(n, 256)), dim3(256), 0, as_stream(stream), f);
+      const int threads = k_fast && n <= 64 * 4 * kCus ? 64 : 256;
+      hipLaunchKernelGGL(fn, dim3((unsigned)ceil_div_ll(n, threads)), dim3(threads), 0, as_stream(stream), f, (int)k_fast);
       WC_CHECK_LAUNCH("filter_transform_fast_kernel");
       return WC_OK;
     }
