@@ -251,7 +251,8 @@ def _stack(stacked, dtype, nd, whole_kernel, w_shape=None, stride=1, m=2):
     """`stacked=None` picks what measured faster on MI355X (the rule itself lives in the library, wc_conv_auto): pieces summed by the batched GEMM for
     16-bit plans (2-D: 1.15-1.3x for 5x5 and 7x7 kernels; 3-D: 1.05-1.4x; fewer bytes moved); for
     fp32, whose product is bound by the MFMA rate and to which stacking adds zero taps, only 2-D
-    plans of up to four pieces (5x5: 1.1-1.15x; 7x7, nine pieces: 0.9-1.0x).  16-bit stride-1
+    plans of up to four pieces (5x5: 1.1-1.15x; 7x7, nine pieces: 0.9-1.0x; the forward pass of
+    four pieces over many channels takes them apart again, pieces_apart in csrc/plan.hip).  16-bit stride-1
     kernels of 4 to 10 taps over at most 256 input channels (3-D: 4 to 8 taps over at most 128, or
     4 taps over at most 256) get the plan whose two-tap pieces share one transformed input (2;
     make_desc then uses output tile 2).  Against stacked F(2,r) pieces it measured, in 2-D, 1.7x
