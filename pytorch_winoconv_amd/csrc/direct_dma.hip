@@ -142,10 +142,29 @@ struct DirectOperands {
 #pragma unroll
     for (int i = 0; i < LA + LB; ++i) issue_part(i);
   }
+  // BRANCHES: most taps need the first two lines only, which is faster between short stages (us, 1 x 192 -> 32, 29x29 stride 2 12.7 | 11.1, N=25 128 ->
+  // 224, 34x34 15.0 | 13.4); without, a step is one block of code for the scheduler
+  template <bool BRANCHES>
   __device__ __forceinline__ void advance(const DirectDmaArgs& a, const DirectDmaArgs::Class& c) {
     --left;
     sload = sload == RING - 1 ? 0 : sload + 1;
-    // without branches, so that a step is one block of code for the scheduler
+    if constexpr (BRANCHES) {
+      tap_x += a.stride;
+      if (tap_x >= c.kw) {
+        tap_x = phase_x;
+        tap_y += a.stride;
+        if (tap_y >= c.kh) {
+          tap_y = phase_y;
+          if (++cb == a.cblocks) {
+            cb = 0;
+            if (++phase_x == min(a.stride, c.kw)) { phase_x = 0; tap_y = ++phase_y; }
+            tap_x = phase_x;
+          }
+        }
+      }
+      offsets(a, c);
+      return;
+    }
     const int nx = tap_x + a.stride;
     const bool row_done = nx >= c.kw;
     const int ny = tap_y + (row_done ? a.stride : 0);
@@ -212,7 +231,7 @@ __global__ __launch_bounds__(256, WM * WN >= 6 ? 2 : WM * WN >= 4 ? 3 : 4) void 
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
 #pragma unroll
-  for (int s = 0; s < (S - 1) * SUB; ++s) { in.issue(); in.advance(a, c); }
+  for (int s = 0; s < (S - 1) * SUB; ++s) { in.issue(); in.template advance<true>(a, c); }
   int cur = 0;
   for (int kt = 0; kt < nk; kt += SUB) {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"((LA + LB) * (S - 2) * SUB) : "memory");
@@ -231,7 +250,7 @@ __global__ __launch_bounds__(256, WM * WN >= 6 ? 2 : WM * WN >= 4 ? 3 : 4) void 
       if ((kk & 1) == 0) in.issue();
       if (kk + 1 < 2 * SUB) fload(kk + 1);
       __builtin_amdgcn_sched_barrier(0);
-      if ((kk & 1) == 0) in.advance(a, c);
+      if ((kk & 1) == 0) in.template advance<true>(a, c);
 #pragma unroll
       for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -311,7 +330,7 @@ __global__ __launch_bounds__(256, 1) void direct_wide_kernel(DirectDmaArgs a) {
   };
 
 #pragma unroll
-  for (int s = 0; s < S; ++s) { in.issue(); in.advance(a, c); }
+  for (int s = 0; s < S; ++s) { in.issue(); in.template advance<false>(a, c); }
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(L * (S - 1)) : "memory");
   fload(ic<0>{});
   // Stage kt is in registers; kt + 1 must have landed (two more may be on their way), and everyone has read kt, whose place takes kt + S
@@ -332,7 +351,7 @@ __global__ __launch_bounds__(256, 1) void direct_wide_kernel(DirectDmaArgs a) {
       __builtin_amdgcn_sched_barrier(0);
       in.issue_part(i);
       if (i < 2) in.issue_part(WM + i);
-      if (i == WM - 1) in.advance(a, c);
+      if (i == WM - 1) in.template advance<false>(a, c);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
