@@ -357,21 +357,24 @@ static int auto_stacked(const wc_conv_desc* d) {
 // That reduction is four times the channels, beyond what the bf16 parts of gemm.hip (fp32_in_parts) are taken for; apart each piece's
 // product is within, has a quarter of the steps on four times the workgroups and no zero taps (5x5: 121 for 144), and M, four times as long
 // to write and read, is small beside it.  The error against fp64 is half to a third (5x5, 480 channels 3.0e-6 | 6.1e-6, 3x3 stride 2, 512 1.35e-6 |
-// 4.1e-6).  us, apart | stacked, transformed filter kept: tile 4, 5x5 256 -> 64, N=1 14x14 33 | 41, 256 -> 256, N=16 28x28 133 | 152, 288 -> 128,
-// N=32 56x56 682 | 887, 288 -> 256, N=4 14x14 41.8 | 40.5 (the worst), 512 -> 512, N=16 14x14 121 | 202; tile 2, 256 -> 256, N=16 28x28 199 | 289; at stride
-// 2 as at stride 1; 4x4 256 channels 1.02 to 1.4 times as fast; 3x3 stride 2, 160 -> 256, N=4 28x28 29.9 | 29.4 (the worst), N=16 56x56
-// 72 | 95, 512 -> 64, N=1 28x28 35 | 56.  Below the lines the sides alternate with the size (5x5 of 160 channels 0.88 to 1.33), and 6x6, which has no zero
-// taps, is no faster up to 288 channels (0.85 to 1.1).  Filter transform included, 512 -> 512, N=2 14x14, all filter, 136 | 127, and where four times the
-// channels are just within the parts' range and the tiles fill the chip, 256 -> 256, N=32 28x28, 305 | 284.  The weight gradient (direct == -1) stays stacked: 5x5 256 -> 64, N=1 14x14 37 | 30, and less exact apart.
+// 4.1e-6).
+//
+// The line goes by the layer alone, not by the batch or the image: a filter that a caller transformed once is that of every call.  4x4 stays
+// stacked: its two plans have filters of one size (four pieces of two taps), so one in the place of the other could not be told by it.  us, apart |
+// stacked, transformed filter kept: tile 2, 5x5 256 -> 256, N=1 7x7 23 | 32, N=8 28x28 107 | 171, 256 -> 1024 N=1 14x14 37 | 38 (the worst), 512 -> 512
+// 39 | 56, N=2 28x28 121 | 176, 4x5 256 -> 64 N=16 28x28 88 | 100; tile 4, 5x5 256 -> 64, N=1 14x14 34 | 42, N=16 28x28 74 | 76, 256 -> 128 N=32 56x56 637 | 643, 1024 ->
+// 128 N=2 14x14 61 | 102, 384 -> 256 N=1 7x7 43 | 47, 512 -> 256 N=16 28x28 1.2 times as fast; at stride 2 as at stride 1; 3x3 stride 2, 160 -> 256, N=4 28x28
+// 29.9 | 29.4 (the worst), N=16 56x56 72 | 95, 512 -> 64, N=1 28x28 35 | 56.  With tile 4 and more output channels the sides alternate with the
+// tiles: 512 -> 512 N=1 14x14 100 | 88, N=16 121 | 202, 288 -> 384 44.5 | 40.6 and N=16 28x28 233 | 287, 256 -> 192 N=32 56x56 911 | 905, 4x5 256 -> 256 N=2 28x28 47.6 | 44.1.  Below
+// 225 channels they do so too (5x5 of 160 channels 0.88 to 1.33), and 6x6, which has no zero taps, is no faster up to 288 channels (0.85 to 1.1).
+// The weight gradient (direct == -1) stays stacked: 5x5 256 -> 64, N=1 14x14 37 | 30, and less exact apart.
 static bool pieces_apart(const wc_conv_desc* d) {
   if (d->dtype != WC_F32 || d->ndim != 2) return false;
   const int kmin = d->kernel[1] < d->kernel[2] ? d->kernel[1] : d->kernel[2], kmax = d->kernel[1] + d->kernel[2] - kmin;
   const int Cp = wc_padded_channels(d->C);
   if (d->stride == 2 && kmin == 3 && kmax == 3) return Cp >= 160;
-  if (kmin < 4 || kmax > 5 || Cp < 256) return false;
-  long long tiles = d->N;
-  for (int a = 1; a < 3; ++a) tiles *= ceil_div((d->in[a] + 2 * d->pad[a] - d->kernel[a]) / d->stride + 1, d->m);
-  return (tiles >= 64 || (long long)Cp * d->K <= (1 << 17)) && (d->m != 4 || Cp > 256 || tiles <= 1024);
+  if (kmin < 4 || kmax != 5 || Cp < 256) return false;
+  return d->m == 2 || d->K <= 128 || (kmin == 5 && Cp >= 384 && d->K <= 256);
 }
 
 // Where the direct form measured faster than the Winograd plan the caller would otherwise get.  Stride 2 in 16-bit,

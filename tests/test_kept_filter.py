@@ -1,0 +1,48 @@
+"""A transformed filter that a caller keeps (transform_filter "once per weight update"; the reference transforms it in every call:
+src/split_kernel.cu:14-53) belongs to the layer, not to the batch or the image it was made for, wherever the plan's form is a
+matter of the layer alone: every fp32 layer."""
+import itertools
+
+import pytest
+import torch
+
+from pytorch_winoconv_amd import engine
+
+IMAGES = [(1, 7, 7), (1, 14, 14), (2, 28, 28), (4, 14, 14), (16, 28, 28), (32, 28, 28), (3, 45, 61), (32, 56, 56)]
+
+
+@pytest.mark.parametrize("m", [2, 4])
+@pytest.mark.parametrize("kernel,stride", [((4, 4), 1), ((4, 5), 1), ((5, 5), 1), ((5, 4), 2), ((4, 4), 2), ((5, 5), 2), ((6, 6), 1), ((3, 3), 2), ((3, 3), 1), ((7, 7), 1)])
+def test_form_of_fp32_layers_is_the_layers(m, kernel, stride):
+    for C, K in itertools.product((3, 64, 160, 225, 256, 288, 512, 1024), (8, 64, 128, 256, 512)):
+        forms = set()
+        for n, h, w in IMAGES:
+            d = engine.make_desc((n, C, h, w), (K, C) + kernel, torch.float32, stride, kernel[0] // 2, m, stacked=None, row=True)
+            forms.add((d.stacked, d.direct, d.row, d.m))
+        assert len(forms) == 1, (C, K, forms)
+
+
+def test_filters_of_different_plans_differ_in_size():
+    """The size is all that tells a filter of other options: the plan that is chosen has no other of its size in another order."""
+    for kernel, stride, m, C, K in itertools.product(((4, 4), (4, 5), (5, 5), (3, 3)), (1, 2), (2, 4), (64, 256, 288, 512), (16, 512)):
+        if kernel == (3, 3) and stride == 1:
+            continue
+        desc = lambda stacked: engine.make_desc((2, C, 30, 30), (K, C) + kernel, torch.float32, stride, 2, m, stacked=stacked, direct=False)
+        size = lambda d: engine.plan_conv(d).t_total * engine._row(d, engine.plan_conv(d))
+        if kernel == (4, 4):
+            assert desc(None).stacked == 1        # both plans have four pieces of two taps an axis
+        else:
+            assert size(desc(False)) != size(desc(True))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("C,K,kernel,m,made,used", [
+    (256, 256, (4, 4), 4, (16, 28, 28), (32, 28, 28)), (512, 512, (4, 4), 2, (1, 14, 14), (4, 14, 14)), (512, 512, (5, 5), 2, (4, 14, 14), (1, 14, 14)),
+    (288, 512, (5, 5), 4, (1, 14, 14), (4, 28, 28)),
+])
+def test_filter_of_one_batch_in_another(dev, host_layer, C, K, kernel, m, made, used):
+    g = torch.Generator().manual_seed(3)
+    w = (torch.randn(K, C, *kernel, generator=g) * (2.0 / (C * kernel[0] * kernel[1])) ** 0.5).to(dev)
+    x = torch.randn(used[0], C, *used[1:], generator=g).to(dev)
+    U = engine.transform_filter(w, (made[0], C) + made[1:], 1, 2, m)
+    assert torch.equal(engine.conv_forward(x, w, None, 1, 2, m, U=U), engine.conv_forward(x, w, None, 1, 2, m))
