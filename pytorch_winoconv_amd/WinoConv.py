@@ -114,8 +114,8 @@ class _WinoConvNd(nn.Module):
 
     # (what the filter was transformed from and for, the transformed filter)
     _cache = None
-    # (hyperparameters, the compiled host layer's plan for the last input's shape or None, that shape): planned when a shape comes a
-    # second time running, so a program whose shapes alternate pays nothing.  Copies and files go without.
+    # (hyperparameters, the compiled host layer's plan for the last input's shape or None, that shape, what its filter is transformed
+    # for): planned when a shape comes a second time running, so a program whose shapes alternate pays nothing.  Copies and files go without.
     _plan = None
 
     def __getstate__(self):
@@ -174,8 +174,8 @@ class _WinoConvNd(nn.Module):
             y = plan[1](x, weight, self.bias)
             if type(y) is tuple:
                 y, renewed, U = y
-                self.__dict__["_plan"] = (conf, renewed, plan[2])
-                self.__dict__["_cache"] = (_held(weight) + self._cache[0][4:], U)
+                self.__dict__["_plan"] = (conf, renewed) + plan[2:]
+                self.__dict__["_cache"] = (_held(weight) + plan[3], U)
             if y is not None:
                 return y
         conv = F.conv2d if self.nd == 2 else F.conv3d
@@ -192,13 +192,14 @@ class _WinoConvNd(nn.Module):
         # the form of the plan (Winograd pieces, or the direct form the library takes for large strided problems)
         # depends on the batch size too, and the transformed filter of one form does not fit the other
         form = engine.plan_form(x.shape, w.shape, x.dtype, self.stride[0], self.padding, m, row=True)
-        key = _held(weight) + (tuple(x.shape[2:]), x.dtype, m, form)
+        made_for = (tuple(x.shape[2:]), x.dtype, m, form)
+        key = _held(weight) + made_for
         if self._cache is None or self._cache[0] != key:
             U = engine.transform_filter(w.detach(), x.shape, self.stride[0], self.padding, m, row=True)
             self._cache = (key, U)
         if engine.USE_EXT:
             again = plan is not None and plan[2] == x.shape
-            self.__dict__["_plan"] = (conf, engine.layer_plan(x, weight, self.stride[0], self.padding, m, self._cache[1]) if again else None, x.shape)
+            self.__dict__["_plan"] = (conf, engine.layer_plan(x, weight, self.stride[0], self.padding, m, self._cache[1]) if again else None, x.shape, made_for)
         b = bias if bias is None or bias.dtype == x.dtype else bias.detach().to(x.dtype)
         if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad or (bias is not None and bias.requires_grad)):
             return WinoConvFunction.apply(x, weight, bias, self.stride[0], self.padding, m, self._cache[1],
