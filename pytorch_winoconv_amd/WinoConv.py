@@ -169,9 +169,11 @@ class _WinoConvNd(nn.Module):
     def forward(self, x):
         conf = (self.in_channels, self.out_channels, self.kernel_size, self.stride, self.padding, self.dilation, self.groups, self.output_block)
         plan = self._plan
-        if x.is_cuda and plan is not None and plan[1] is not None and plan[0] == conf and engine.USE_EXT:
-            weight = self.weight
-            y = plan[1](x, weight, self.bias)
+        weight = bias = None             # read once in a pass: a parametrization runs, and may move on, each time
+        planned = x.is_cuda and plan is not None and plan[1] is not None and plan[0] == conf and engine.USE_EXT
+        if planned:
+            weight, bias = self.weight, self.bias
+            y = plan[1](x, weight, bias)
             if type(y) is tuple:
                 y, renewed, U = y
                 self.__dict__["_plan"] = (conf, renewed) + plan[2:]
@@ -183,10 +185,11 @@ class _WinoConvNd(nn.Module):
             raise ValueError("WinoConv: the engine runs on the GPU only; got a CPU tensor")
         if x.dtype not in (torch.float16, torch.bfloat16, torch.float32):
             raise NotImplementedError(f"WinoConv: dtype {x.dtype} (float32, float16 and bfloat16 only)")
+        if not planned:
+            weight, bias = self.weight, self.bias
         if not self._winograd_ok(x):
-            return conv(x, self.weight, self.bias, self.stride, self.padding, self.dilation, self.groups)
+            return conv(x, weight, bias, self.stride, self.padding, self.dilation, self.groups)
         # (to() and detach() that change nothing still cost a microsecond each of a 12 us call)
-        weight, bias = self.weight, self.bias
         w = weight if weight.dtype == x.dtype else weight.detach().to(x.dtype)
         m = self._tile_for(x.dtype)
         # the form of the plan (Winograd pieces, or the direct form the library takes for large strided problems)

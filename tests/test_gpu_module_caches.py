@@ -36,3 +36,28 @@ def test_a_renewed_filter_is_kept_for_what_it_was_made_for(dev, monkeypatch):
     monkeypatch.setattr(engine, "USE_EXT", False)
     _close(layer(single), layer, single)
     _close(layer(half), layer, half)
+
+
+class _Counted(torch.nn.Module):
+    """A parametrization with state, like a spectral norm's power iteration."""
+
+    def __init__(self):
+        super().__init__()
+        self.calls = 0
+
+    def forward(self, w):
+        self.calls += 1
+        return w * 1.0
+
+
+def test_parameters_are_read_once_in_a_pass(dev):
+    layer = pkg.WinoConv2d(16, 24, 3, padding=1, device=dev, dtype=torch.float16)
+    counted = {}
+    for name in ("weight", "bias"):
+        torch.nn.utils.parametrize.register_parametrization(layer, name, _Counted())
+        counted[name] = layer.parametrizations[name][0]
+    shapes = [(2, 16, 9, 11)] * 4 + [(1, 16, 9, 11), (2, 16, 9, 11), (2, 16, 8, 11), (2, 16, 9, 11), (2, 16, 9, 11), (2, 16, 9, 11)]
+    for i, shape in enumerate(shapes):
+        before = counted["weight"].calls, counted["bias"].calls
+        layer(_input(dev, *shape) if i % 3 else _input(dev, *shape).contiguous())
+        assert (counted["weight"].calls, counted["bias"].calls) == (before[0] + 1, before[1] + 1), i
