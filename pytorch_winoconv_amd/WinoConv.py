@@ -201,7 +201,8 @@ class _WinoConvNd(nn.Module):
             U = engine.transform_filter(w.detach(), x.shape, self.stride[0], self.padding, m, row=True)
             self._cache = (key, U)
         if engine.USE_EXT:
-            again = plan is not None and plan[2] == x.shape
+            # (a list may change in place, and its plan would not see it)
+            again = plan is not None and plan[2] == x.shape and all(v is None or type(v) in (int, tuple) for v in conf)
             self.__dict__["_plan"] = (conf, engine.layer_plan(x, weight, self.stride[0], self.padding, m, self._cache[1]) if again else None, x.shape, made_for)
         b = bias if bias is None or bias.dtype == x.dtype else bias.detach().to(x.dtype)
         if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad or (bias is not None and bias.requires_grad)):

@@ -61,3 +61,14 @@ def test_parameters_are_read_once_in_a_pass(dev):
         before = counted["weight"].calls, counted["bias"].calls
         layer(_input(dev, *shape) if i % 3 else _input(dev, *shape).contiguous())
         assert (counted["weight"].calls, counted["bias"].calls) == (before[0] + 1, before[1] + 1), i
+
+
+def test_hyperparameters_that_change_in_place(dev):
+    layer = pkg.WinoConv2d(16, 24, 3, padding=1, device=dev, dtype=torch.float16).requires_grad_(False)
+    layer.padding = [1, 1]
+    x = _input(dev, 2, 16, 9, 11)
+    for _ in range(4):
+        _close(layer(x), layer, x)
+    layer.padding[0] = 0
+    assert layer(x).shape == (2, 24, 7, 11)
+    _close(layer(x), layer, x)
