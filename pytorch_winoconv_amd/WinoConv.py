@@ -12,7 +12,6 @@ is cached and recomputed only when the weight changes.
 """
 import torch
 from torch import nn
-from torch.multiprocessing.reductions import StorageWeakRef
 import torch.nn.functional as F
 
 from . import engine, matrix_conv, matrix_conv3d
@@ -88,12 +87,6 @@ def gradients(x, w, dy, stride, padding, m, need_dx, need_dw, need_db, w_type, b
     return dx, dw, db
 
 
-def _held(weight):
-    """What a transformed filter was made from.  The weak reference keeps the storage's identity, though not its memory: weights that are
-    new tensors in every pass (functional_call, parametrizations) come to lie where the last one did."""
-    return weight._version, weight.data_ptr(), weight.stride(), StorageWeakRef(weight.untyped_storage())
-
-
 class _WinoConvNd(nn.Module):
     nd = 2
 
@@ -112,7 +105,7 @@ class _WinoConvNd(nn.Module):
         if self.bias is not None:
             nn.init.zeros_(self.bias)
 
-    # (what the filter was transformed from and for, the transformed filter)
+    # (what the filter is transformed for, the engine's KeptFilter)
     _cache = None
     # (hyperparameters, the compiled host layer's plan for the last input's shape or None, that shape, what its filter is transformed
     # for): planned when a shape comes a second time running, so a program whose shapes alternate pays nothing.  Copies and files go without.
@@ -175,9 +168,9 @@ class _WinoConvNd(nn.Module):
             weight, bias = self.weight, self.bias
             y = plan[1](x, weight, bias)
             if type(y) is tuple:
-                y, renewed, U = y
+                y, renewed, kept = y
                 self.__dict__["_plan"] = (conf, renewed) + plan[2:]
-                self.__dict__["_cache"] = (_held(weight) + plan[3], U)
+                self.__dict__["_cache"] = (plan[3], kept)
             if y is not None:
                 return y
         conv = F.conv2d if self.nd == 2 else F.conv3d
@@ -189,26 +182,30 @@ class _WinoConvNd(nn.Module):
             weight, bias = self.weight, self.bias
         if not self._winograd_ok(x):
             return conv(x, weight, bias, self.stride, self.padding, self.dilation, self.groups)
-        # (to() and detach() that change nothing still cost a microsecond each of a 12 us call)
-        w = weight if weight.dtype == x.dtype else weight.detach().to(x.dtype)
         m = self._tile_for(x.dtype)
         # the form of the plan (Winograd pieces, or the direct form the library takes for large strided problems)
         # depends on the batch size too, and the transformed filter of one form does not fit the other
-        form = engine.plan_form(x.shape, w.shape, x.dtype, self.stride[0], self.padding, m, row=True)
+        form = engine.plan_form(x.shape, weight.shape, x.dtype, self.stride[0], self.padding, m, row=True)
         made_for = (tuple(x.shape[2:]), x.dtype, m, form)
-        key = _held(weight) + made_for
-        if self._cache is None or self._cache[0] != key:
+        cache = self._cache
+        U = cache[1].on_stream() if cache is not None and cache[0] == made_for and cache[1].holds(weight) else None
+        if U is None:
+            cache = (made_for, engine.KeptFilter(weight))
+        # (to() and detach() that change nothing still cost a microsecond each of a 12 us call)
+        w = weight if weight.dtype == x.dtype else weight.detach().to(x.dtype)
+        if U is None:
             U = engine.transform_filter(w.detach(), x.shape, self.stride[0], self.padding, m, row=True)
-            self._cache = (key, U)
+            cache[1].made(U)
+            self.__dict__["_cache"] = cache
         if engine.USE_EXT:
             # (a list may change in place, and its plan would not see it)
             again = plan is not None and plan[2] == x.shape and all(v is None or type(v) in (int, tuple) for v in conf)
-            self.__dict__["_plan"] = (conf, engine.layer_plan(x, weight, self.stride[0], self.padding, m, self._cache[1]) if again else None, x.shape, made_for)
+            self.__dict__["_plan"] = (conf, engine.layer_plan(x, weight, self.stride[0], self.padding, m, cache[1]) if again else None, x.shape, made_for)
         b = bias if bias is None or bias.dtype == x.dtype else bias.detach().to(x.dtype)
         if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad or (bias is not None and bias.requires_grad)):
-            return WinoConvFunction.apply(x, weight, bias, self.stride[0], self.padding, m, self._cache[1],
+            return WinoConvFunction.apply(x, weight, bias, self.stride[0], self.padding, m, U,
                                           None if w is weight and b is bias else (w, b))
-        return engine.conv_forward(x, w, b, self.stride[0], self.padding, m, U=self._cache[1], row=True)
+        return engine.conv_forward(x, w, b, self.stride[0], self.padding, m, U=U, row=True)
 
 
 class WinoConv2d(_WinoConvNd):

@@ -14,9 +14,13 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/jit/frontend/tracer.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/VirtualGuardImpl.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
+#include <mutex>
 #include <optional>
 #include <sstream>
 #include <stdexcept>
@@ -88,17 +92,17 @@ struct KeptWorkspaces {
   }
 };
 
+bool capturing(void* stream) {
+  if (stream == nullptr) return false;          // the default stream cannot be captured
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status) != hipSuccess || status != hipStreamCaptureStatusNone;
+}
+
 at::Tensor workspace_for(const at::Tensor& like, size_t bytes, void* stream) {
   constexpr size_t kKept = 1u << 20;
   constexpr size_t kKeptSlots = 4;
   auto fresh = [&](size_t n) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); };
-  if (bytes > kKept) return fresh(bytes);
-  if (stream != nullptr) {                      // the default stream cannot be captured
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &capturing) != hipSuccess ||
-        capturing != hipStreamCaptureStatusNone)
-      return fresh(bytes);
-  }
+  if (bytes > kKept || capturing(stream)) return fresh(bytes);
   thread_local KeptWorkspaces kept;
   const int device = like.device().index();
   for (auto& k : kept.slots)
@@ -706,12 +710,71 @@ py::tuple conv_backward(at::Tensor x, at::Tensor w, at::Tensor dy, py::object st
   return py::make_tuple(or_none(g.dx), or_none(g.dw), or_none(g.db));
 }
 
+// ---- a module's transformed filter between its passes --------------------------------------------------------------------
+// It is the filter of one weight: the weak pointer keeps the storage's identity and not its memory (weights that are new tensors in every pass,
+// as functional_call and parametrizations make them, come to lie where the last one did).  It was made on one stream; a pass on another waits for
+// that, once, and its memory is given back when the passes of all of them are through with it.  (engine.py's _KeptFilter does the same without
+// this module.)
+class KeptFilter {
+ public:
+  // `weight` before anything is read of it: what changes it from here on makes it another one
+  explicit KeptFilter(const at::Tensor& weight)
+      : version_((uint32_t)weight._version()), storage_(weight.storage().getWeakStorageImpl()), data_(weight.data_ptr()), strides_(weight.strides().vec()) {}
+
+  // u: what was launched for it on the current stream
+  void made(const at::Tensor& u) {
+    U_ = u;
+    stream_ = stream_of(u);
+  }
+
+  bool holds(const at::Tensor& weight) const {
+    return !weight.is_inference() && (uint32_t)weight._version() == version_ && weight.data_ptr() == data_ && weight.strides() == at::IntArrayRef(strides_) &&
+           weight.storage().unsafeGetStorageImpl() == storage_._unsafe_get_target();
+  }
+
+  const at::Tensor& U() const { return U_; }
+
+  // U for a launch on the current stream; undefined where that cannot be ordered behind U's making.  (A capture cannot wait for what is outside
+  // of it: its caller has, before the first replay, as for every other tensor that a graph reads.)
+  at::Tensor on_stream() const {
+    void* const now = stream_of(U_);
+    if (now == stream_) return U_;
+    const std::lock_guard<std::mutex> lock(mutex_);
+    if (std::find(ordered_.begin(), ordered_.end(), now) != ordered_.end() || capturing(now)) return U_;
+    if (capturing(stream_)) return at::Tensor();
+    const c10::DeviceGuard device(U_.device());
+    hipEvent_t event;
+    bool ok = hipEventCreateWithFlags(&event, hipEventDisableTiming) == hipSuccess;
+    if (ok) {
+      ok = hipEventRecord(event, static_cast<hipStream_t>(stream_)) == hipSuccess && hipStreamWaitEvent(static_cast<hipStream_t>(now), event, 0) == hipSuccess;
+      (void)hipEventDestroy(event);
+    }
+    if (!ok) {                                      // a stream that is no more
+      (void)hipGetLastError();
+      return at::Tensor();
+    }
+    U_.record_stream(c10::impl::VirtualGuardImpl(U_.device().type()).getStream(U_.device()));
+    ordered_.push_back(now);
+    return U_;
+  }
+
+ private:
+  uint32_t version_;
+  c10::weak_intrusive_ptr<c10::StorageImpl> storage_;
+  const void* data_;
+  std::vector<int64_t> strides_;
+  at::Tensor U_;
+  void* stream_ = nullptr;
+  mutable std::mutex mutex_;
+  mutable std::vector<void*> ordered_;              // streams that have waited
+};
+
 // ---- a module's forward pass ----------------------------------------------------------------------------------------
 // What WinoConv.py's modules work out anew for an input of another shape: the descriptor, the shape of the result and the
 // transformed filter.  Called with an input of the same shape, strides and type and a weight of the same kind, it runs the layer
 // without Python, with an autograd node of C++ where a gradient is wanted, and gives a plan for the filter where the weight has
 // changed; called with anything else it gives None, and the module goes its way.  It never changes after it is made, so
-// threads may share it; tensors are compared by what they are, and none but the transformed filter is kept.
+// threads and streams may share it; tensors are compared by what they are, and none but the transformed filter is kept.
 // Host time, us: a frozen layer 10.6 | 6.5 (a launch of torch's own 4.8), a training step in mixed precision 182 | 122, its backward
 // pass 102 | 69, of which 55 are the autograd engine and a thread's waking.
 class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
@@ -723,20 +786,17 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
   size_t bytes = 0;
   int nd, stride, m;
   std::vector<int> pads;
-  at::Tensor U;
-  // the weight that U was made from; the weak pointer keeps the storage's identity and not its memory
-  c10::weak_intrusive_ptr<c10::StorageImpl> w_storage;
-  std::vector<int64_t> w_strides;
-  const void* w_data;
-  uint32_t w_version;
+  std::shared_ptr<KeptFilter> filter;
 
   // None where the layer copies its input first or the filter is not the plan's
-  static std::shared_ptr<LayerPlan> make(const at::Tensor& x, const at::Tensor& weight, int stride, std::vector<int> pads, int m, const at::Tensor& U) {
+  static std::shared_ptr<LayerPlan> make(const at::Tensor& x, const at::Tensor& weight, int stride, std::vector<int> pads, int m,
+                                         const std::shared_ptr<KeptFilter>& filter) {
     const int nd = spatial_dims(x.sizes(), weight.sizes());
+    const at::Tensor& U = filter->U();
     if ((int)pads.size() != nd || x.numel() == 0 || x.size(1) != weight.size(1) || !plain(x) || !plain(weight) || misaligned(x) || misaligned(U)) return nullptr;
     const bool last = channel_last_memory(x);
     if (!last && !x.is_contiguous()) return nullptr;
-    auto p = std::make_shared<LayerPlan>(x, weight, stride, std::move(pads), m, U);
+    auto p = std::make_shared<LayerPlan>(x, weight, stride, std::move(pads), m, filter);
     p->d = desc_of(x.sizes(), weight.sizes(), p->pads, stride, m, dtype_of(x));
     p->d.stacked = p->d.row = -1;
     check(wc_conv_auto(&p->d));
@@ -756,10 +816,9 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
     p->y_strides.push_back(K);
     return p;
   }
-  LayerPlan(const at::Tensor& x, const at::Tensor& weight, int s, std::vector<int> p, int m_, const at::Tensor& u)
+  LayerPlan(const at::Tensor& x, const at::Tensor& weight, int s, std::vector<int> p, int m_, const std::shared_ptr<KeptFilter>& f)
       : x_type(x.scalar_type()), w_type(weight.scalar_type()), device(x.device()), sizes(x.sizes().vec()), strides(x.strides().vec()),
-        w_sizes(weight.sizes().vec()), nd((int)x.dim() - 2), stride(s), m(m_), pads(std::move(p)), U(u), w_storage(weight.storage().getWeakStorageImpl()),
-        w_strides(weight.strides().vec()), w_data(weight.data_ptr()), w_version(weight.unsafeGetTensorImpl()->is_inference() ? 0 : weight._version()) {}
+        w_sizes(weight.sizes().vec()), nd((int)x.dim() - 2), stride(s), m(m_), pads(std::move(p)), filter(f) {}
 
   at::Tensor run(const at::Tensor& x, const at::Tensor& w, const at::Tensor& bias, const at::Tensor& u) const {
     at::Tensor y = at::empty_strided(y_sizes, y_strides, x.options());
@@ -773,7 +832,7 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
   }
 
   at::Tensor transform(const at::Tensor& w) const {
-    at::Tensor u = at::empty(U.sizes(), U.options());
+    at::Tensor u = at::empty_like(filter->U());
     wc_conv_desc f = d;
     f.x_layout = 0;
     wc_plan plan{};
@@ -784,7 +843,7 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
     return u;
   }
 
-  // The result; with a weight that has changed since the plan was made (result, the plan for it, its transformed filter)
+  // The result; with a weight that has changed since the plan was made (result, the plan for it, its filter)
   py::object call(const at::Tensor& x, const at::Tensor& weight, const std::optional<at::Tensor>& bias) const;
 
  private:
@@ -873,27 +932,26 @@ py::object LayerPlan::call(const at::Tensor& x, const at::Tensor& weight, const 
   {
     py::gil_scoped_release nogil;
     const bool grad = at::GradMode::is_enabled() && (x.requires_grad() || weight.requires_grad() || (bias && bias->requires_grad()));
-    const bool same_weight = weight.data_ptr() == w_data && (uint32_t)weight._version() == w_version && weight.strides() == at::IntArrayRef(w_strides) &&
-                             weight.storage().unsafeGetStorageImpl() == w_storage._unsafe_get_target();
-    LayerOperands o{shared_from_this(), weight, bias ? *bias : at::Tensor(), U};
-    const bool cast_w = (grad || !same_weight) && w_type != x_type, cast_b = bias && bias->scalar_type() != x_type;
+    LayerOperands o{shared_from_this(), weight, bias ? *bias : at::Tensor(), filter->holds(weight) ? filter->on_stream() : at::Tensor()};
+    const bool anew = !o.U.defined();
+    if (anew) {
+      renewed = std::make_shared<LayerPlan>(*this);
+      renewed->filter = std::make_shared<KeptFilter>(weight);
+    }
+    const bool cast_w = (grad || anew) && w_type != x_type, cast_b = bias && bias->scalar_type() != x_type;
     if (cast_w || cast_b) {
       at::AutoGradMode no_grad(false);
       if (cast_w) o.w = weight.to(x_type);
       if (cast_b) o.bias = bias->to(x_type);
     }
     if (o.bias.defined()) o.bias = o.bias.contiguous();
-    if (!same_weight) {
-      renewed = std::make_shared<LayerPlan>(*this);
-      renewed->w_storage = weight.storage().getWeakStorageImpl();
-      renewed->w_strides = weight.strides().vec();
-      renewed->w_data = weight.data_ptr();
-      renewed->w_version = (uint32_t)weight._version();
-      renewed->U = o.U = transform(o.w);
+    if (anew) {
+      o.U = transform(o.w);
+      renewed->filter->made(o.U);
     }
     y = grad ? LayerFunction::apply(x, weight, bias, o) : run(x, o.w, o.bias, o.U);
   }
-  if (renewed) return py::make_tuple(y, renewed, renewed->U);
+  if (renewed) return py::make_tuple(y, renewed, renewed->filter);
   return py::cast(y);
 }
 
@@ -936,8 +994,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("channels_first_out") = false, py::arg("direct") = py::none(), py::arg("row") = false);
   m.def("conv_backward_weight", &conv_backward_weight, py::arg("x"), py::arg("dy"), py::arg("w_shape"), py::arg("stride") = 1,
         py::arg("padding") = 0, py::arg("m") = 2);
+  py::class_<KeptFilter, std::shared_ptr<KeptFilter>>(m, "KeptFilter")
+      .def(py::init<const at::Tensor&>(), py::arg("weight"))
+      .def("made", &KeptFilter::made, py::arg("U"))
+      .def("holds", &KeptFilter::holds, py::arg("weight"))
+      .def("on_stream", [](const KeptFilter& f) { return or_none(f.on_stream()); });
   py::class_<LayerPlan, std::shared_ptr<LayerPlan>>(m, "LayerPlan")
-      .def_static("make", &LayerPlan::make, py::arg("x"), py::arg("weight"), py::arg("stride"), py::arg("padding"), py::arg("m"), py::arg("U"))
+      .def_static("make", &LayerPlan::make, py::arg("x"), py::arg("weight"), py::arg("stride"), py::arg("padding"), py::arg("m"), py::arg("filter"))
       .def("__call__", &LayerPlan::call, py::arg("x"), py::arg("weight"), py::arg("bias"));
   m.def("conv_backward_parameters", &conv_backward_parameters, py::arg("x"), py::arg("dy"), py::arg("w_shape"), py::arg("stride"), py::arg("padding"),
         py::arg("m"), py::arg("need_db"), py::arg("w_type"), py::arg("b_type"));

@@ -6,6 +6,7 @@ stream only; all arithmetic is done by the HIP kernels behind libwinoconv_hip.so
 import ctypes
 
 import torch
+from torch.multiprocessing.reductions import StorageWeakRef
 
 from . import _lib
 from ._lib import ConvDesc, Plan, check
@@ -549,10 +550,42 @@ def bias_gradient(dy):
     return db
 
 
-def layer_plan(x, weight, stride, padding, m, U):
-    """The compiled host layer's plan of conv_forward(x, weight, ..., U=U, row=True) for inputs of x's shape, strides and type, called as
-    plan(x, weight, bias); None where there is none."""
-    return _ext.LayerPlan.make(x, weight, stride, list(padding), m, U)
+class _KeptFilter:
+    """A module's transformed filter between its passes, as the compiled host layer's KeptFilter is where there is one: of one weight, made on one
+    stream, ordered behind that for passes on another, its memory given back when all of them are through with it."""
+
+    def __init__(self, weight):
+        # before anything is read of the weight.  The weak reference keeps the storage's identity, though not its memory: weights that are
+        # new tensors in every pass (functional_call, parametrizations) come to lie where the last one did
+        self._held = self._identity(weight)
+        self._ordered = set()
+
+    @staticmethod
+    def _identity(weight):
+        return weight._version, weight.data_ptr(), weight.stride(), StorageWeakRef(weight.untyped_storage())
+
+    def made(self, U):
+        self._U, self._stream = U, torch.cuda.current_stream(U.device)
+
+    def holds(self, weight):
+        return self._held == self._identity(weight)
+
+    def on_stream(self):
+        now = torch.cuda.current_stream(self._U.device)
+        if now != self._stream and now not in self._ordered and not torch.cuda.is_current_stream_capturing():
+            now.wait_stream(self._stream)
+            self._U.record_stream(now)
+            self._ordered.add(now)
+        return self._U
+
+
+KeptFilter = getattr(_ext, "KeptFilter", _KeptFilter)      # (_KeptFilter without a compiled host layer, and while an older one is being replaced)
+
+
+def layer_plan(x, weight, stride, padding, m, kept):
+    """The compiled host layer's plan of conv_forward(x, weight, ..., U=kept.on_stream(), row=True) for inputs of x's shape, strides and type,
+    called as plan(x, weight, bias); None where there is none."""
+    return _ext.LayerPlan.make(x, weight, stride, list(padding), m, kept)
 
 
 def conv_backward(x, w, dy, stride, padding, m, need_dx, need_dw, need_db, w_type=None, b_type=None):

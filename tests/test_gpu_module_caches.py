@@ -72,3 +72,58 @@ def test_hyperparameters_that_change_in_place(dev):
     layer.padding[0] = 0
     assert layer(x).shape == (2, 24, 7, 11)
     _close(layer(x), layer, x)
+
+
+@pytest.fixture(params=["compiled", "ctypes", "python"])
+def passes(request, monkeypatch):
+    """Through the plan, past it, and without the compiled host layer's part of what is kept."""
+    monkeypatch.setattr(engine, "USE_EXT", request.param == "compiled")
+    if request.param == "python":
+        monkeypatch.setattr(engine, "KeptFilter", engine._KeptFilter)
+    return 4 if request.param == "compiled" else 1
+
+
+_A_WHILE = 20_000_000                     # cycles: some ten milliseconds
+
+
+@pytest.mark.parametrize("own", [torch.float16, torch.float32])
+def test_a_filter_made_on_another_stream(dev, passes, own):
+    """Two streams that are ordered behind the weight's update and not with each other: the one that comes second waits for the filter
+    that the first one makes."""
+    layer = pkg.WinoConv2d(64, 96, 5, padding=2, device=dev, dtype=own).requires_grad_(False)
+    xa, xb = _input(dev, 2, 64, 15, 14), _input(dev, 2, 64, 15, 14, seed=2)
+    for _ in range(passes):
+        layer(xa)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    for turn in range(3):
+        layer.weight.mul_(-1.5)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(a):
+            torch.cuda._sleep(_A_WHILE)
+            ya = layer(xa)
+        with torch.cuda.stream(b):
+            yb = [layer(xb) for _ in range(2)]
+        torch.cuda.synchronize()
+        _close(ya, layer, xa)
+        for y in yb:
+            _close(y, layer, xb)
+
+
+def test_a_filter_is_given_back_when_every_stream_is_through(dev, passes):
+    """The filter is replaced, and its memory taken by others on the stream that it was made on, while another stream has yet to read it."""
+    layer = pkg.WinoConv2d(64, 96, 5, padding=2, device=dev, dtype=torch.float16).requires_grad_(False)
+    x = _input(dev, 2, 64, 15, 14)
+    for _ in range(passes):
+        layer(x)
+    other = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    want = layer(x)
+    with torch.cuda.stream(other):
+        torch.cuda._sleep(_A_WHILE)
+        got = layer(x)
+    layer.weight.zero_()
+    layer(x)                               # another filter; the first one's memory goes back
+    U = engine.transform_filter(layer.weight, x.shape, 1, 2, 4, row=True)
+    taken = [torch.full_like(U, 7.0) for _ in range(8)]
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and len(taken) == 8

@@ -46,3 +46,18 @@ def test_filter_of_one_batch_in_another(dev, host_layer, C, K, kernel, m, made, 
     x = torch.randn(used[0], C, *used[1:], generator=g).to(dev)
     U = engine.transform_filter(w, (made[0], C) + made[1:], 1, 2, m)
     assert torch.equal(engine.conv_forward(x, w, None, 1, 2, m, U=U), engine.conv_forward(x, w, None, 1, 2, m))
+
+
+@pytest.mark.parametrize("kind", [engine.KeptFilter, engine._KeptFilter])
+def test_the_weight_a_module_keeps_a_filter_of(kind):
+    w = torch.nn.Parameter(torch.randn(8, 8, 3, 3), requires_grad=False)
+    kept = kind(w)
+    assert kept.holds(w) and kept.holds(w.detach()) and kept.holds(w.view(8, 8, 3, 3))
+    assert not kept.holds(w.transpose(0, 1)) and not kept.holds(w.clone())
+    w.add_(1)
+    assert not kept.holds(w) and kind(w).holds(w)
+    place, kept = w.data_ptr(), kind(w)
+    del w
+    for _ in range(8):                           # another weight, perhaps where the first one was
+        assert not kept.holds(torch.randn(8, 8, 3, 3))
+    assert place
