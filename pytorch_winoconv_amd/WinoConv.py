@@ -196,8 +196,9 @@ class _WinoConvNd(nn.Module):
         if U is None:
             U = engine.transform_filter(w.detach(), x.shape, self.stride[0], self.padding, m, row=True)
             cache[1].made(U)
-            self.__dict__["_cache"] = cache
-        if engine.USE_EXT:
+            if not cache[1].captured:
+                self.__dict__["_cache"] = cache
+        if engine.USE_EXT and not cache[1].captured:
             # (a list may change in place, and its plan would not see it)
             again = plan is not None and plan[2] == x.shape and all(v is None or type(v) in (int, tuple) for v in conf)
             self.__dict__["_plan"] = (conf, engine.layer_plan(x, weight, self.stride[0], self.padding, m, cache[1]) if again else None, x.shape, made_for)

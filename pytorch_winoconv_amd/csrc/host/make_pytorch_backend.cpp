@@ -725,7 +725,11 @@ class KeptFilter {
   void made(const at::Tensor& u) {
     U_ = u;
     stream_ = stream_of(u);
+    captured_ = capturing(stream_);
   }
+
+  // made inside a capture: there when the graph is replayed, and only then.  Not for other passes
+  bool captured() const { return captured_; }
 
   bool holds(const at::Tensor& weight) const {
     return !weight.is_inference() && (uint32_t)weight._version() == version_ && weight.data_ptr() == data_ && weight.strides() == at::IntArrayRef(strides_) &&
@@ -765,6 +769,7 @@ class KeptFilter {
   std::vector<int64_t> strides_;
   at::Tensor U_;
   void* stream_ = nullptr;
+  bool captured_ = false;
   mutable std::mutex mutex_;
   mutable std::vector<void*> ordered_;              // streams that have waited
 };
@@ -843,7 +848,7 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
     return u;
   }
 
-  // The result; with a weight that has changed since the plan was made (result, the plan for it, its filter)
+  // The result; with a weight that has changed since the plan was made (result, the plan for it, its filter), outside of captures
   py::object call(const at::Tensor& x, const at::Tensor& weight, const std::optional<at::Tensor>& bias) const;
 
  private:
@@ -951,7 +956,7 @@ py::object LayerPlan::call(const at::Tensor& x, const at::Tensor& weight, const 
     }
     y = grad ? LayerFunction::apply(x, weight, bias, o) : run(x, o.w, o.bias, o.U);
   }
-  if (renewed) return py::make_tuple(y, renewed, renewed->filter);
+  if (renewed && !renewed->filter->captured()) return py::make_tuple(y, renewed, renewed->filter);
   return py::cast(y);
 }
 
@@ -997,6 +1002,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   py::class_<KeptFilter, std::shared_ptr<KeptFilter>>(m, "KeptFilter")
       .def(py::init<const at::Tensor&>(), py::arg("weight"))
       .def("made", &KeptFilter::made, py::arg("U"))
+      .def_property_readonly("captured", &KeptFilter::captured)
       .def("holds", &KeptFilter::holds, py::arg("weight"))
       .def("on_stream", [](const KeptFilter& f) { return or_none(f.on_stream()); });
   py::class_<LayerPlan, std::shared_ptr<LayerPlan>>(m, "LayerPlan")

@@ -565,7 +565,7 @@ class _KeptFilter:
         return weight._version, weight.data_ptr(), weight.stride(), StorageWeakRef(weight.untyped_storage())
 
     def made(self, U):
-        self._U, self._stream = U, torch.cuda.current_stream(U.device)
+        self._U, self._stream, self.captured = U, torch.cuda.current_stream(U.device), torch.cuda.is_current_stream_capturing()
 
     def holds(self, weight):
         return self._held == self._identity(weight)

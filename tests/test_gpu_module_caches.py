@@ -127,3 +127,28 @@ def test_a_filter_is_given_back_when_every_stream_is_through(dev, passes):
     taken = [torch.full_like(U, 7.0) for _ in range(8)]
     torch.cuda.synchronize()
     assert torch.equal(got, want) and len(taken) == 8
+
+
+@pytest.mark.parametrize("warm", [False, True])
+def test_a_filter_made_inside_a_capture(dev, passes, warm):
+    """It is there once the graph has been replayed and stays the graph's: passes outside make their own."""
+    layer = pkg.WinoConv2d(64, 96, 5, padding=2, device=dev, dtype=torch.float16).requires_grad_(False)
+    x = _input(dev, 2, 64, 15, 14)
+    if warm:
+        for _ in range(passes):
+            layer(x)
+        layer.weight.mul_(-1)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = layer(x)
+    taken = [torch.full((256, 1024), 7.0, device=dev) for _ in range(4)]
+    eager = layer(x)
+    _close(eager, layer, x)
+    for i in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, eager) and torch.equal(layer(x), eager)
+        x.copy_(_input(dev, 2, 64, 15, 14, seed=5 + i))
+        eager = layer(x)
+    assert len(taken) == 4
