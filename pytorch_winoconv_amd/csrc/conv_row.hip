@@ -809,11 +809,12 @@ bool row_reads_padded(const wc_conv_desc* d) {
                   d->C).tall_planes > 0;
 }
 
-// x (N, D, H, W, x_row) channel-last, 16-byte aligned: x_row is C, where row_reads_padded allows it, or C rounded up to 8 (zeros beyond C);
+// x (N, D, H, W, x_row) channel-last: x_row is C, where row_reads_padded allows it, or C rounded up to 8 (zeros beyond C).  Rows of whole 16
+// bytes start at a multiple of 16; others, of which a pass's first image starts anywhere, at any element;
 // images first_image .. + n_images of the batch
 int row_conv(const wc_conv_desc* d, const void* x, int x_row, int first_image, int n_images, const void* U, const void* bias, void* y, void* stream) {
   WC_CHECK_ARG(row_conv_fits(d), "row form: 16-bit, stride 1, kernels 3x3, 3x3x3, 5x5 and 7x7");
-  WC_CHECK_ARG(((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(U)) & 15) == 0, "row form: x and U must be 16-byte aligned");
+  WC_CHECK_ARG(((x_row % 8 == 0 ? reinterpret_cast<uintptr_t>(x) : 0) | reinterpret_cast<uintptr_t>(U)) % 16 == 0, "row form: x and U must be 16-byte aligned");
   RowArgs a{};
   a.x = x; a.U = U; a.bias = bias; a.y = y;
   a.N = n_images; a.D = d->in[0]; a.H = d->in[1]; a.W = d->in[2]; a.C = wc_padded_channels8(d->C); a.K = d->K;

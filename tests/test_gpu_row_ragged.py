@@ -1,10 +1,12 @@
 """The row form on rows of x and y that are no multiple of 16 bytes, read and written as they lie: bit for bit what the same layer gives with
 its channels padded with zeros (the reference pads to 32: src/base_conv_launchers.cu:325-352), infinities and NaN included, in every
 shape of workgroup."""
+import ctypes
+
 import pytest
 import torch
 
-from pytorch_winoconv_amd import engine
+from pytorch_winoconv_amd import _lib, engine
 
 pytestmark = pytest.mark.gpu
 
@@ -58,6 +60,29 @@ def test_passes_of_a_batch(dev, C):
     for chunk in (1, 2):
         assert torch.equal(engine.conv_forward(x, w, None, 1, 1, 2, chunk_images=chunk, row=True), whole)
         assert torch.equal(engine.conv_forward(x.contiguous(), w, None, 1, 1, 2, chunk_images=chunk, row=True), whole)
+
+
+@pytest.mark.parametrize("C,H", [(9, 9), (33, 9), (11, 7), (102, 45), (65, 9)])
+def test_passes_that_start_anywhere(dev, host_layer, C, H):
+    """Passes of a batch whose images of x are no multiple of 16 bytes: a channel-first y is written through a copy, x is read as it lies."""
+    W = {45: 61, 7: 7}.get(H, 10)
+    x = torch.randn(5, C, H, W, device=dev).half().contiguous(memory_format=torch.channels_last)
+    w, b = torch.randn(40, C, 3, 3, device=dev).half(), torch.randn(40, device=dev).half()
+    whole = engine.conv_forward(x, w, b, 1, 1, 2, row=True)
+    for chunk in (1, 2, 3):
+        assert torch.equal(engine.conv_forward(x, w, b, 1, 1, 2, chunk_images=chunk, row=True, channels_first_out=True), whole)
+    # the entry points of the library: passes that it chooses itself, and an x that starts anywhere
+    lib, y = _lib.load(), torch.empty(5, 40, H, W, device=dev, dtype=torch.float16)
+    desc = engine.make_desc(x.shape, w.shape, x.dtype, 1, 1, 2, 1, stacked=None, row=True, y_layout=1)
+    assert desc.row == 1
+    _lib.check(lib.wc_conv_forward_static(ctypes.byref(desc), engine._ptr(x), engine._ptr(w), engine._w_strides(w), None, engine._ptr(b), engine._ptr(y), engine._stream(x)))
+    assert torch.equal(y, whole)
+    if C % 8:
+        flat = torch.empty(x.numel() + 8, device=dev, dtype=torch.float16)
+        view = flat[3:3 + x.numel()].copy_(x.permute(0, 2, 3, 1).reshape(-1))
+        y.zero_()
+        _lib.check(lib.wc_conv_forward_static(ctypes.byref(desc), engine._ptr(view), engine._ptr(w), engine._w_strides(w), None, engine._ptr(b), engine._ptr(y), engine._stream(x)))
+        assert torch.equal(y, whole)
 
 
 @pytest.mark.parametrize("C", list(range(1, 18)) + [31, 63, 100])
