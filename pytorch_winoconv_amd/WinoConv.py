@@ -105,10 +105,11 @@ class _WinoConvNd(nn.Module):
         if self.bias is not None:
             nn.init.zeros_(self.bias)
 
-    # (what the filter is transformed for, the engine's KeptFilter)
+    # ((type, the engine's filter_form), its KeptFilter): the filter of the last pass
     _cache = None
-    # (hyperparameters, the compiled host layer's plan for the last input's shape or None, that shape, what its filter is transformed
-    # for): planned when a shape comes a second time running, so a program whose shapes alternate pays nothing.  Copies and files go without.
+    # (hyperparameters, the compiled host layer's plan for the last input's shape, what _cache has for it, the tile asked for).  Every
+    # pass is one of a plan's where there is one, also the first: a plan costs what the call without it works out too.  Copies and files
+    # go without.
     _plan = None
 
     def __getstate__(self):
@@ -159,38 +160,57 @@ class _WinoConvNd(nn.Module):
             return 2
         return self._tile()
 
+    def _conf(self):
+        return (self.in_channels, self.out_channels, self.kernel_size, self.stride, self.padding, self.dilation, self.groups, self.output_block)
+
+    def _run(self, plan, x, weight, bias):
+        """The plan's result, None where it is not this pass's; with a filter that it made, that one is kept."""
+        y = plan[1](x, weight, bias)
+        if type(y) is tuple:
+            y, renewed, kept = y
+            plan = (plan[0], renewed) + plan[2:]
+            self.__dict__["_cache"] = (plan[2], kept)
+        # (hyperparameters in a list may change in place, and no plan would see it)
+        if plan is not self._plan and y is not None and all(v is None or type(v) in (int, tuple) for v in plan[0]):
+            self.__dict__["_plan"] = plan
+        return y
+
     def forward(self, x):
-        conf = (self.in_channels, self.out_channels, self.kernel_size, self.stride, self.padding, self.dilation, self.groups, self.output_block)
-        plan = self._plan
-        weight = bias = None             # read once in a pass: a parametrization runs, and may move on, each time
-        planned = x.is_cuda and plan is not None and plan[1] is not None and plan[0] == conf and engine.USE_EXT
-        if planned:
+        plan = self._plan if x.is_cuda and engine.USE_EXT else None
+        if plan is not None and plan[0] != self._conf():
+            plan = None
+        # weight and bias are read once in a pass: a parametrization runs, and may move on, each time
+        if plan is not None:
             weight, bias = self.weight, self.bias
-            y = plan[1](x, weight, bias)
-            if type(y) is tuple:
-                y, renewed, kept = y
-                self.__dict__["_plan"] = (conf, renewed) + plan[2:]
-                self.__dict__["_cache"] = (plan[3], kept)
+            y = self._run(plan, x, weight, bias)
             if y is not None:
                 return y
-        conv = F.conv2d if self.nd == 2 else F.conv3d
         if not x.is_cuda:
             raise ValueError("WinoConv: the engine runs on the GPU only; got a CPU tensor")
         if x.dtype not in (torch.float16, torch.bfloat16, torch.float32):
             raise NotImplementedError(f"WinoConv: dtype {x.dtype} (float32, float16 and bfloat16 only)")
-        if not planned:
+        if plan is None:
             weight, bias = self.weight, self.bias
-        if not self._winograd_ok(x):
+        if plan is not None and plan[2][0] == x.dtype:
+            m = plan[3]
+        elif not self._winograd_ok(x):
+            conv = F.conv2d if self.nd == 2 else F.conv3d
             return conv(x, weight, bias, self.stride, self.padding, self.dilation, self.groups)
-        m = self._tile_for(x.dtype)
+        else:
+            m = self._tile_for(x.dtype)
+        cache = self._cache
+        if engine.USE_EXT:
+            made = engine.layer_plan(x, weight, self.stride[0], self.padding, m, cache and cache[1])
+            if made is not None:
+                y = self._run((self._conf(), made, (x.dtype, made.form), m), x, weight, bias)
+                if y is not None:
+                    return y
         # the form of the plan (Winograd pieces, or the direct form the library takes for large strided problems)
         # depends on the batch size too, and the transformed filter of one form does not fit the other
-        form = engine.plan_form(x.shape, weight.shape, x.dtype, self.stride[0], self.padding, m, row=True)
-        made_for = (tuple(x.shape[2:]), x.dtype, m, form)
-        cache = self._cache
-        U = cache[1].on_stream() if cache is not None and cache[0] == made_for and cache[1].holds(weight) else None
+        form = engine.filter_form(x.shape, weight.shape, x.dtype, self.stride[0], self.padding, m)
+        U = cache[1].on_stream() if cache is not None and cache[0] == (x.dtype, form) and cache[1].holds(weight) else None
         if U is None:
-            cache = (made_for, engine.KeptFilter(weight))
+            cache = ((x.dtype, form), engine.KeptFilter(weight, form))
         # (to() and detach() that change nothing still cost a microsecond each of a 12 us call)
         w = weight if weight.dtype == x.dtype else weight.detach().to(x.dtype)
         if U is None:
@@ -198,10 +218,6 @@ class _WinoConvNd(nn.Module):
             cache[1].made(U)
             if not cache[1].captured:
                 self.__dict__["_cache"] = cache
-        if engine.USE_EXT and not cache[1].captured:
-            # (a list may change in place, and its plan would not see it)
-            again = plan is not None and plan[2] == x.shape and all(v is None or type(v) in (int, tuple) for v in conf)
-            self.__dict__["_plan"] = (conf, engine.layer_plan(x, weight, self.stride[0], self.padding, m, cache[1]) if again else None, x.shape, made_for)
         b = bias if bias is None or bias.dtype == x.dtype else bias.detach().to(x.dtype)
         if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad or (bias is not None and bias.requires_grad)):
             return WinoConvFunction.apply(x, weight, bias, self.stride[0], self.padding, m, U,

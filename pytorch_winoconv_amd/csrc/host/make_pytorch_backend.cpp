@@ -711,15 +711,19 @@ py::tuple conv_backward(at::Tensor x, at::Tensor w, at::Tensor dy, py::object st
 }
 
 // ---- a module's transformed filter between its passes --------------------------------------------------------------------
-// It is the filter of one weight: the weak pointer keeps the storage's identity and not its memory (weights that are new tensors in every pass,
+// It is the filter of one weight in one form of the plan: the weak pointer keeps the storage's identity and not its memory (weights that are new tensors in every pass,
 // as functional_call and parametrizations make them, come to lie where the last one did).  It was made on one stream; a pass on another waits for
 // that, once, and its memory is given back when the passes of all of them are through with it.  (engine.py's _KeptFilter does the same without
 // this module.)
+// direct, stacked, tile, row and the elements of the filter (fewer for an image of depth 1, whose plan has no tile along it): what a transformed
+// filter depends on beside the weight and the type
+using PlanForm = std::tuple<int, int, int, int, int64_t>;
+
 class KeptFilter {
  public:
   // `weight` before anything is read of it: what changes it from here on makes it another one
-  explicit KeptFilter(const at::Tensor& weight)
-      : version_((uint32_t)weight._version()), storage_(weight.storage().getWeakStorageImpl()), data_(weight.data_ptr()), strides_(weight.strides().vec()) {}
+  KeptFilter(const at::Tensor& weight, const PlanForm& form)
+      : form_(form), version_((uint32_t)weight._version()), storage_(weight.storage().getWeakStorageImpl()), data_(weight.data_ptr()), strides_(weight.strides().vec()) {}
 
   // u: what was launched for it on the current stream
   void made(const at::Tensor& u) {
@@ -736,7 +740,11 @@ class KeptFilter {
            weight.storage().unsafeGetStorageImpl() == storage_._unsafe_get_target();
   }
 
-  const at::Tensor& U() const { return U_; }
+  // a 16-byte aligned U of this form and type
+  bool suits(const PlanForm& form, at::ScalarType type, at::Device device) const {
+    return form == form_ && U_.numel() == std::get<4>(form) && U_.scalar_type() == type && U_.device() == device && U_.is_contiguous() &&
+           (reinterpret_cast<uintptr_t>(U_.data_ptr()) & 15) == 0;
+  }
 
   // U for a launch on the current stream; undefined where that cannot be ordered behind U's making.  (A capture cannot wait for what is outside
   // of it: its caller has, before the first replay, as for every other tensor that a graph reads.)
@@ -763,6 +771,7 @@ class KeptFilter {
   }
 
  private:
+  PlanForm form_;
   uint32_t version_;
   c10::weak_intrusive_ptr<c10::StorageImpl> storage_;
   const void* data_;
@@ -777,38 +786,37 @@ class KeptFilter {
 // ---- a module's forward pass ----------------------------------------------------------------------------------------
 // What WinoConv.py's modules work out anew for an input of another shape: the descriptor, the shape of the result and the
 // transformed filter.  Called with an input of the same shape, strides and type and a weight of the same kind, it runs the layer
-// without Python, with an autograd node of C++ where a gradient is wanted, and gives a plan for the filter where the weight has
-// changed; called with anything else it gives None, and the module goes its way.  It never changes after it is made, so
+// without Python, with an autograd node of C++ where a gradient is wanted, and gives a plan with the filter where that has to be
+// made; called with anything else it gives None, and the module goes its way.  It never changes after it is made, so
 // threads and streams may share it; tensors are compared by what they are, and none but the transformed filter is kept.
-// Host time, us: a frozen layer 10.6 | 6.5 (a launch of torch's own 4.8), a training step in mixed precision 182 | 122, its backward
-// pass 102 | 69, of which 55 are the autograd engine and a thread's waking.
+// Host time, us, every call by itself | planned: a frozen layer 10.8 | 6.6 (a launch of torch's own 4.8), on two batch sizes in turn 11.1 | 9.9 (a plan
+// is made for each, and its filter kept), on a first input 30 | 29; a training step in mixed precision 182 | 122, its backward pass 102 | 69, of
+// which 55 are the autograd engine and a thread's waking.
 class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
  public:
   at::ScalarType x_type, w_type;
   at::Device device;
   std::vector<int64_t> sizes, strides, w_sizes, y_sizes, y_strides;
   wc_conv_desc d{};
-  size_t bytes = 0;
+  size_t bytes = 0, u_elems = 0;
   int nd, stride, m;
   std::vector<int> pads;
-  std::shared_ptr<KeptFilter> filter;
+  std::shared_ptr<KeptFilter> filter;               // null: not made yet
 
-  // None where the layer copies its input first or the filter is not the plan's
+  // None where the layer copies its input first.  `kept`: the filter of the module's last pass, taken where it is this one's
   static std::shared_ptr<LayerPlan> make(const at::Tensor& x, const at::Tensor& weight, int stride, std::vector<int> pads, int m,
-                                         const std::shared_ptr<KeptFilter>& filter) {
+                                         const std::shared_ptr<KeptFilter>& kept) {
     const int nd = spatial_dims(x.sizes(), weight.sizes());
-    const at::Tensor& U = filter->U();
-    if ((int)pads.size() != nd || x.numel() == 0 || x.size(1) != weight.size(1) || !plain(x) || !plain(weight) || misaligned(x) || misaligned(U)) return nullptr;
+    if ((int)pads.size() != nd || x.numel() == 0 || x.size(1) != weight.size(1) || !plain(x) || !plain(weight) || misaligned(x)) return nullptr;
     const bool last = channel_last_memory(x);
     if (!last && !x.is_contiguous()) return nullptr;
-    auto p = std::make_shared<LayerPlan>(x, weight, stride, std::move(pads), m, filter);
+    auto p = std::make_shared<LayerPlan>(x, weight, stride, std::move(pads), m);
     p->d = desc_of(x.sizes(), weight.sizes(), p->pads, stride, m, dtype_of(x));
     p->d.stacked = p->d.row = -1;
     check(wc_conv_auto(&p->d));
     p->d.x_layout = !last;
-    size_t ue = 0;
-    check(wc_conv_u_elems(&p->d, &ue));
-    if (!U.is_contiguous() || (size_t)U.numel() != ue || U.scalar_type() != x.scalar_type() || U.device() != x.device()) return nullptr;
+    check(wc_conv_u_elems(&p->d, &p->u_elems));
+    if (kept && kept->suits(p->form(), x.scalar_type(), x.device())) p->filter = kept;
     int out[3], grid[3];
     check(wc_conv_out_dims(&p->d, out, grid));
     check(wc_conv_workspace_bytes(&p->d, &p->bytes));
@@ -821,9 +829,11 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
     p->y_strides.push_back(K);
     return p;
   }
-  LayerPlan(const at::Tensor& x, const at::Tensor& weight, int s, std::vector<int> p, int m_, const std::shared_ptr<KeptFilter>& f)
+  LayerPlan(const at::Tensor& x, const at::Tensor& weight, int s, std::vector<int> p, int m_)
       : x_type(x.scalar_type()), w_type(weight.scalar_type()), device(x.device()), sizes(x.sizes().vec()), strides(x.strides().vec()),
-        w_sizes(weight.sizes().vec()), nd((int)x.dim() - 2), stride(s), m(m_), pads(std::move(p)), filter(f) {}
+        w_sizes(weight.sizes().vec()), nd((int)x.dim() - 2), stride(s), m(m_), pads(std::move(p)) {}
+
+  PlanForm form() const { return {d.direct, d.stacked, d.m, d.row, (int64_t)u_elems}; }
 
   at::Tensor run(const at::Tensor& x, const at::Tensor& w, const at::Tensor& bias, const at::Tensor& u) const {
     at::Tensor y = at::empty_strided(y_sizes, y_strides, x.options());
@@ -837,9 +847,9 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
   }
 
   at::Tensor transform(const at::Tensor& w) const {
-    at::Tensor u = at::empty_like(filter->U());
     wc_conv_desc f = d;
     f.x_layout = 0;
+    at::Tensor u = at::empty({(int64_t)u_elems}, w.options());
     wc_plan plan{};
     if (!f.direct && !f.row) check(wc_plan_conv(&f, &plan));
     int64_t s[5];
@@ -848,7 +858,7 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
     return u;
   }
 
-  // The result; with a weight that has changed since the plan was made (result, the plan for it, its filter), outside of captures
+  // The result; where the filter had to be made, outside of captures (result, the plan with it, the filter)
   py::object call(const at::Tensor& x, const at::Tensor& weight, const std::optional<at::Tensor>& bias) const;
 
  private:
@@ -937,11 +947,11 @@ py::object LayerPlan::call(const at::Tensor& x, const at::Tensor& weight, const 
   {
     py::gil_scoped_release nogil;
     const bool grad = at::GradMode::is_enabled() && (x.requires_grad() || weight.requires_grad() || (bias && bias->requires_grad()));
-    LayerOperands o{shared_from_this(), weight, bias ? *bias : at::Tensor(), filter->holds(weight) ? filter->on_stream() : at::Tensor()};
+    LayerOperands o{shared_from_this(), weight, bias ? *bias : at::Tensor(), filter && filter->holds(weight) ? filter->on_stream() : at::Tensor()};
     const bool anew = !o.U.defined();
     if (anew) {
       renewed = std::make_shared<LayerPlan>(*this);
-      renewed->filter = std::make_shared<KeptFilter>(weight);
+      renewed->filter = std::make_shared<KeptFilter>(weight, form());
     }
     const bool cast_w = (grad || anew) && w_type != x_type, cast_b = bias && bias->scalar_type() != x_type;
     if (cast_w || cast_b) {
@@ -1000,13 +1010,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("conv_backward_weight", &conv_backward_weight, py::arg("x"), py::arg("dy"), py::arg("w_shape"), py::arg("stride") = 1,
         py::arg("padding") = 0, py::arg("m") = 2);
   py::class_<KeptFilter, std::shared_ptr<KeptFilter>>(m, "KeptFilter")
-      .def(py::init<const at::Tensor&>(), py::arg("weight"))
+      .def(py::init<const at::Tensor&, const PlanForm&>(), py::arg("weight"), py::arg("form"))
       .def("made", &KeptFilter::made, py::arg("U"))
       .def_property_readonly("captured", &KeptFilter::captured)
       .def("holds", &KeptFilter::holds, py::arg("weight"))
       .def("on_stream", [](const KeptFilter& f) { return or_none(f.on_stream()); });
   py::class_<LayerPlan, std::shared_ptr<LayerPlan>>(m, "LayerPlan")
-      .def_static("make", &LayerPlan::make, py::arg("x"), py::arg("weight"), py::arg("stride"), py::arg("padding"), py::arg("m"), py::arg("filter"))
+      .def_static("make", &LayerPlan::make, py::arg("x"), py::arg("weight"), py::arg("stride"), py::arg("padding"), py::arg("m"), py::arg("kept"))
+      .def_property_readonly("form", &LayerPlan::form)
       .def("__call__", &LayerPlan::call, py::arg("x"), py::arg("weight"), py::arg("bias"));
   m.def("conv_backward_parameters", &conv_backward_parameters, py::arg("x"), py::arg("dy"), py::arg("w_shape"), py::arg("stride"), py::arg("padding"),
         py::arg("m"), py::arg("need_db"), py::arg("w_type"), py::arg("b_type"));

@@ -136,6 +136,13 @@ def plan_form(x_shape, w_shape, dtype, stride=1, padding=0, m=2, row=False):
     return (int(d.direct), int(d.stacked), int(d.m)) + ((int(d.row),) if row else ())
 
 
+def filter_form(x_shape, w_shape, dtype, stride, padding, m):
+    """plan_form with `row` and the elements of the transformed filter (fewer for an image of depth 1, whose plan has no tile along it): what a
+    filter that the modules keep depends on beside the weight and the type."""
+    d, _, _, elements = _forward_setup(tuple(x_shape), tuple(w_shape), dtype, stride, tuple(padding), m, 0, False, None, row=True)
+    return int(d.direct), int(d.stacked), int(d.m), int(d.row), elements
+
+
 def plan_conv(desc):
     plan = Plan()
     check(_lib.load().wc_plan_conv(ctypes.byref(desc), ctypes.byref(plan)))
@@ -551,10 +558,10 @@ def bias_gradient(dy):
 
 
 class _KeptFilter:
-    """A module's transformed filter between its passes, as the compiled host layer's KeptFilter is where there is one: of one weight, made on one
-    stream, ordered behind that for passes on another, its memory given back when all of them are through with it."""
+    """A module's transformed filter between its passes, as the compiled host layer's KeptFilter is where there is one: of one weight in one
+    form of the plan (filter_form), made on one stream, ordered behind that for passes on another, its memory given back when all of them are through with it."""
 
-    def __init__(self, weight):
+    def __init__(self, weight, form):
         # before anything is read of the weight.  The weak reference keeps the storage's identity, though not its memory: weights that are
         # new tensors in every pass (functional_call, parametrizations) come to lie where the last one did
         self._held = self._identity(weight)
@@ -583,8 +590,8 @@ KeptFilter = getattr(_ext, "KeptFilter", _KeptFilter)      # (_KeptFilter withou
 
 
 def layer_plan(x, weight, stride, padding, m, kept):
-    """The compiled host layer's plan of conv_forward(x, weight, ..., U=kept.on_stream(), row=True) for inputs of x's shape, strides and type,
-    called as plan(x, weight, bias); None where there is none."""
+    """The compiled host layer's plan of conv_forward(x, weight, ..., row=True) for inputs of x's shape, strides and type, called as plan(x, weight,
+    bias); None where there is none.  `kept`: a KeptFilter that it takes where it is of its form, or None."""
     return _ext.LayerPlan.make(x, weight, stride, list(padding), m, kept)
 
 

@@ -1,5 +1,4 @@
-"""The modules' planned forward pass (LayerPlan of the compiled host layer) against the unplanned one, bit for bit: a shape's first two
-passes go through Python, the third through the plan.  The reference has no such modules that work (conv.py:324-339)."""
+"""The modules' planned forward pass (LayerPlan of the compiled host layer) against the unplanned one, bit for bit.  The reference has no such modules that work (conv.py:324-339)."""
 import copy
 import threading
 

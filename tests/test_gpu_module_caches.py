@@ -152,3 +152,27 @@ def test_a_filter_made_inside_a_capture(dev, passes, warm):
         x.copy_(_input(dev, 2, 64, 15, 14, seed=5 + i))
         eager = layer(x)
     assert len(taken) == 4
+
+
+@pytest.mark.parametrize("own", [torch.float16, torch.float32])
+def test_shapes_types_and_memory_orders_in_turn(dev, passes, own):
+    """Each pass with the filter of its own form: batches on either side of the direct form's line, images, types and orders in memory."""
+    layer = pkg.WinoConv2d(128, 128, 7, 2, 3, device=dev, dtype=own).requires_grad_(False)
+    xs = [_input(dev, n, 128, h, w, dtype=t) for t in {torch.float16, own} for n, h, w in ((1, 30, 29), (40, 60, 60), (2, 31, 30))]
+    forms = {engine.filter_form(x.shape, layer.weight.shape, x.dtype, 2, (3, 3), layer._tile_for(x.dtype))[0] for x in xs}
+    assert forms == {0, 1}
+    for turn in range(2):
+        for x in xs + xs[::-1]:
+            _close(layer(x), layer, x)
+            _close(layer(x.contiguous()), layer, x)
+        layer.weight.mul_(-1)
+
+
+def test_images_of_one_plane_and_of_more_in_turn(dev, passes):
+    """A kernel of one tap along the depth: the plan of a single plane has no tile along it, and a smaller filter."""
+    layer = pkg.WinoConv3d(24, 16, (1, 3, 3), padding=(0, 1, 1), device=dev).requires_grad_(False)
+    for turn in range(3):
+        for depth in (1, 4, 1, 5):
+            x = _input(dev, 2, 24, depth, 9, 10, dtype=torch.float32)
+            want = F.conv3d(x.double(), layer.weight.double(), layer.bias.double(), 1, (0, 1, 1))
+            assert (layer(x).double() - want).norm() <= 1e-5 * want.norm()

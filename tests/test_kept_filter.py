@@ -51,12 +51,12 @@ def test_filter_of_one_batch_in_another(dev, host_layer, C, K, kernel, m, made, 
 @pytest.mark.parametrize("kind", [engine.KeptFilter, engine._KeptFilter])
 def test_the_weight_a_module_keeps_a_filter_of(kind):
     w = torch.nn.Parameter(torch.randn(8, 8, 3, 3), requires_grad=False)
-    kept = kind(w)
+    kept = kind(w, (0, 0, 4, 0, 2304))
     assert kept.holds(w) and kept.holds(w.detach()) and kept.holds(w.view(8, 8, 3, 3))
     assert not kept.holds(w.transpose(0, 1)) and not kept.holds(w.clone())
     w.add_(1)
-    assert not kept.holds(w) and kind(w).holds(w)
-    place, kept = w.data_ptr(), kind(w)
+    assert not kept.holds(w) and kind(w, (0, 0, 4, 0, 2304)).holds(w)
+    place, kept = w.data_ptr(), kind(w, (0, 0, 4, 0, 2304))
     del w
     for _ in range(8):                           # another weight, perhaps where the first one was
         assert not kept.holds(torch.randn(8, 8, 3, 3))
