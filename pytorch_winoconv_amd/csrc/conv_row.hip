@@ -555,7 +555,7 @@ struct RowPlan { RowShape shape; RowBox box; long long wide_groups; int tall_pla
 // Over 300 layers drawn anew the choice takes 1.6 % longer than the fastest shape of each in the mean, with a line through the origin for
 // half boxes, and small ones up to one a CU only, 3.2 %.  fp16, us, wide | half | small: 280 half boxes of 7 steps 25.2 | 25.9 |
 // 21.0, 252 of 7 steps 22.5 | 16.7 | 21.4; 3-D, 280 of 2 steps 18.0 | 26.2 | 20.6, 160 17.7 | 25.2 | 27.9 (two rounds of half boxes, one of wide
-// ones).  7x7, 532 small boxes of 8 steps of which half the channels are none 77 | - | 75, split 55.
+// ones).
 struct RowModel { double wide, wide_round, half, half_two, half_more, half_at, half_step, small_two, small_three, small_more; };
 constexpr RowModel kRow3x3{0.86, 0.92, 0.60, 0.97, 1.27, 1.0, 0.12, 1.6, 2.1, 0.82}, kRow5x5{0.82, 0.80, 0.58, 0.75, 1.15, 0.85, 0.10, 1.25, 1.7, 0.68},
     kRow3d{0.78, 0.72, 0.53, 1.06, 0.0, 0.0, 0.0, 1.2, 1.7, 0.60};
@@ -572,16 +572,17 @@ RowPlan make_row_shape(int N, int oD, int oH, int nW, int kd, int kh, int K, int
   p.wide_groups = n_wide;
   if (kh == 7) {
     // Seven rows' halo leaves 64 tiles all of a wide workgroup's LDS, 32 a third of a CU's (kRowSmall) or, with the channels in
-    // two shares, two thirds (kRowSplit).  us a step of 32 channels: small 4 for every one that a CU gets, wide 7 alone and 10.5
-    // where all CUs have one.  Measured, wide | small | split, fp16: N=6 100 -> 150, 45x61 46 | 52 | 53, N=16 64 -> 64, 56x56
-    // 42 | 26 | 38, N=32 128 -> 128, 112x112 421 | 600 | 802, N=1 512 -> 512, 14x14 117 | 55 | 33, 64 -> 64, 28x28 18 | 9.8 | 8.7.
+    // two shares, two thirds (kRowSplit), which alone in a round is the fastest.  Else whole rounds of each, of 470 layers drawn over 1 to 64 images, 24
+    // to 512 channels and 7 to 112 rows, each timed in every shape: 0.15 % over the fastest in the mean (0.16 and 0.14 % on the halves that the
+    // lines were and were not fitted to; 0.2 % measured on 200 others), a line without rounds for small boxes and split ones for K <= 32 alone 1.4 %.  fp16, us, wide | small | split:
+    // N=51 96 -> 192, 23x25 67 | 71 | 121, N=26 296 -> 54, 32x38 78 | 105 | 110, N=32 43 -> 29, 28x73 41 | 31 | 37, N=5 501 -> 150, 58x25 126 | 117 | 75, N=6
+    // 100 -> 150, 45x61 46 | 52 | 53, N=32 128 -> 128, 112x112 421 | 600 | 802, N=1 512 -> 512, 14x14 117 | 55 | 33.
     const long long n_split = small.boxes * ceil_div(K, 32);
     if (steps < 2 || n_split > kCus) {
-      take(kRowWide, wide, rounds(n_wide) * ((n_wide <= kCus ? 6.2 + 3.5 * n_wide / kCus : 10.5) * steps + 4));
-      take(kRowSmall, small, 4.0 * steps * std::max(1.0, 1.08 * n_small / kCus));
+      take(kRowWide, wide, rounds(n_wide) * (std::min(10.5, 7 + 3.5 * n_wide / kCus) * steps + 6));
+      take(kRowSmall, small, rounds(n_small) * (3.6 * steps + 2));
     }
-    // in several rounds only where half of a small workgroup's channels would be none; beyond eight rounds its reads of x are no longer met in L2
-    if (steps >= 2 && (n_split <= kCus || (K <= 32 && n_split <= 8 * kCus))) take(kRowSplit, small, rounds(n_split) * (1.05 * steps + 1));
+    if (steps >= 2) take(kRowSplit, small, rounds(n_split) * (2.3 * steps + 6));
     return p;
   }
   const double us_small = 0.4 * steps * kd * kh + 4, unit = ((kd == 1 ? 0.82 * kh : 6.9) * steps + 7) / 0.92;
@@ -754,7 +755,7 @@ static bool row_preferred_5x5(const wc_conv_desc* d) {
 // N=8 247 | 229 (241 | 232), 100x100 349 | 367 (345 | 364), 56x56 N=32 421 | 470 (433 | 465), 28x28 N=64 224 | 298 (250 | 304), 14x14 71 | 132; 224 -> 224,
 // 112x112 N=8 375 | 365 (372 | 368); 160 -> 256, 100x100 N=5 161 | 152 (158 | 156); 128 -> 128, 112x112 N=32 424 | 528 (410 | 563).
 static bool row_no_slower_7x7(const wc_conv_desc* d, const RowPlan& p) {
-  if (p.shape == kRowSplit || !(d->K % 128 == 0 || d->K % 128 >= 96)) return true;
+  if ((p.shape == kRowSplit && p.box.boxes * ceil_div(d->K, 32) <= kCus) || !(d->K % 128 == 0 || d->K % 128 >= 96)) return true;
   const int oH = d->in[1] + 2 * d->pad[1] - 6, oW = d->in[2] + 2 * d->pad[2] - 6, steps = ceil_div(d->C, 32);
   auto rounds = [](long long n, double start, double share) { return n / kCus + (n % kCus ? start + share * (n % kCus) / kCus : 0.0); };
   const long long rows = (long long)d->N * (ceil_div(oH, 3) + 2) * (ceil_div(oW, 3) + 2), tiles = 25 * ceil_div_ll(rows, 512) * ceil_div(d->K, 128);
