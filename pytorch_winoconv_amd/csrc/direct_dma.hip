@@ -45,13 +45,19 @@ template <> struct MfmaD<bf16_t> {
 };
 
 // acc += a b in place.  The builtin's result may be another register than its addend, and with two stages of a loop's body the compiler
-// chose so, and copied every accumulator back.  It does not know these as matrix instructions: their results are read after a wait.
+// chose so, and copied every accumulator back.  It does not know these as matrix instructions, and waits for none of their results: nothing
+// but them may touch the accumulators up to mfma16_done (tests/test_wide_tile_code.py looks the built code through for that).
 template <typename T>
 __device__ __forceinline__ void mfma16(f32x4& acc, typename MfmaD<T>::Frag a, typename MfmaD<T>::Frag b) {
   if constexpr (std::is_same_v<T, half_t>)
     asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
   else
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+
+// The wait, of eight passes at most, that a row of accumulators goes through before it is read
+__device__ __forceinline__ void mfma16_done(f32x4 (&a)[8]) {
+  asm volatile("s_nop 15" : "+a"(a[0]), "+a"(a[1]), "+a"(a[2]), "+a"(a[3]), "+a"(a[4]), "+a"(a[5]), "+a"(a[6]), "+a"(a[7]));
 }
 
 struct DirectDmaArgs {
@@ -361,7 +367,9 @@ __global__ __launch_bounds__(256, 1) void direct_wide_kernel(DirectDmaArgs a) {
     step(ic<1>{});
     kt += 2;
   } while (kt < nk);
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier\n\ts_nop 15\n\ts_nop 15" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < WM; ++i) mfma16_done(acc[i]);
 
   constexpr int CS = BN + 8;
   T* const cs = reinterpret_cast<T*>(lds_raw);
