@@ -607,14 +607,18 @@ RowPlan make_row_shape(int N, int oD, int oH, int nW, int kd, int kh, int K, int
 // hold 123 of 128 planes, 3 rounds, the other 5 planes 20 us; seven images and one were 3 rounds of 686 boxes and 37 us).  The
 // model's constants are measured ones (fp16, us, this shape alone in whole rounds | a box: 512 -> 512, 28x28 157 | 78 for 32 half
 // blocks, 256 -> 256, 56x56 175 | 44 for 16).
-RowPlan make_row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int C) {
+//
+// copied: x comes with channels padded to a multiple of 8
+RowPlan make_row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int C, bool copied) {
   const int steps = ceil_div(C, 32);
   RowPlan best = make_row_shape(N, oD, oH, nW, kd, kh, K, steps);
   best.rest_n = N; best.rest_d = oD;
   if (kh != 3) return best;
   const double box_us = 2.1 * 2 * steps * kd + 10.5;
-  // tall boxes read padded rows: the copy at twice the rate that it reaches (tests/test_abi_host.py takes N=64 250 -> 256, 56x56 for a layer with one)
-  const double copy_us = C % 8 ? 3 + N * (double)oD * oH * nW * 4 * C * 4 / 9e6 : 0;
+  // Tall boxes read padded rows.  What their copy takes between two layers that differ by it alone, over 109 layers: tall boxes and the others are
+  // chosen with 0.1 % lost in the mean (at 3 us and 9 TB/s 0.4 %: N=31 175 -> 232, 66x25 52 us, 47 in wide boxes).  Where x is copied in any case
+  // (channel-first) the other boxes find the copy in L2 and are ahead by less of it: without a price the same mean, but N=27 105 -> 144, 83x37 48 | 56 us.
+  const double bytes = N * (double)oD * oH * nW * 4 * C * 4, copy_us = C % 8 == 0 ? 0 : copied ? 3 + bytes / 9e6 : 5 + bytes / 7e6;
   const long long per_group = (long long)ceil_div(oH, 4) * ceil_div(K, 128), planes = (long long)N * oD;
   const long long boxes = ceil_div_ll(planes * nW, 32) * per_group;
   const long long groups = boxes / kCus * kCus / per_group;       // groups of 32 columns in whole rounds
@@ -640,16 +644,16 @@ RowPlan make_row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int 
 }
 
 // The search over boxes takes some microseconds: the last plans of a host thread are kept.
-RowPlan row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int C) {
-  struct Entry { int key[8]; RowPlan plan; };
+RowPlan row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int C, bool copied = false) {
+  struct Entry { int key[9]; RowPlan plan; };
   thread_local Entry cache[64] = {};
-  const int key[8] = {N, oD, oH, nW, kd, kh, K, C};
+  const int key[9] = {N, oD, oH, nW, kd, kh, K, C, copied};
   unsigned h = 2166136261u;
   for (int v : key) h = (h ^ (unsigned)v) * 16777619u;
   Entry& e = cache[(h ^ (h >> 15)) % 64];
-  if (!std::equal(key, key + 8, e.key)) {
-    e.plan = make_row_plan(N, oD, oH, nW, kd, kh, K, C);
-    std::copy(key, key + 8, e.key);
+  if (!std::equal(key, key + 9, e.key)) {
+    e.plan = make_row_plan(N, oD, oH, nW, kd, kh, K, C, copied);
+    std::copy(key, key + 9, e.key);
   }
   return e.plan;
 }
@@ -828,7 +832,7 @@ int row_conv(const wc_conv_desc* d, const void* x, int x_row, int first_image, i
   a.u_bytes = (int)(row_u_elems(d) * 2);
   const int force = test_gemm_config();
   // the shapes are the whole batch's, so that the passes of a batch add in the order of the batch in one pass
-  RowPlan plan = row_plan(d->N, a.oD, a.oH, a.nW, d->kernel[0], d->kernel[1], a.K, d->C);
+  RowPlan plan = row_plan(d->N, a.oD, a.oH, a.nW, d->kernel[0], d->kernel[1], a.K, d->C, x_row != d->C);
   if (force >= 16 && force <= 19) { plan.shape = (RowShape)(force - 16); plan.tall_planes = 0; plan.rest_n = -1; }
   if (force == 21 && d->kernel[1] == 3) plan.tall_planes = d->N * a.oD;
   const int tall = std::min(std::max(plan.tall_planes - first_image * a.oD, 0), n_images * a.oD);
