@@ -115,6 +115,10 @@ class _WinoConvNd(nn.Module):
     def __getstate__(self):
         return {k: v for k, v in self.__dict__.items() if k not in ("_plan", "_cache")}
 
+    # ... and files that were written with a filter, of whatever form it was then, are read without
+    def __setstate__(self, state):
+        super().__setstate__({k: v for k, v in state.items() if k not in ("_plan", "_cache")})
+
     def _winograd_ok(self, x):
         # The reference hands every strided or dilated layer (and every kernel up to 3 x 3) to the stock
         # convolution (conv.py:326-332, 467-473).  This engine keeps strided layers, with one exception: strided

@@ -1,12 +1,13 @@
 """A transformed filter that a caller keeps (transform_filter "once per weight update"; the reference transforms it in every call:
 src/split_kernel.cu:14-53) belongs to the layer, not to the batch or the image it was made for, wherever the plan's form is a
 matter of the layer alone: every fp32 layer."""
+import io
 import itertools
 
 import pytest
 import torch
 
-from pytorch_winoconv_amd import engine
+from pytorch_winoconv_amd import WinoConv2d, engine
 
 IMAGES = [(1, 7, 7), (1, 14, 14), (2, 28, 28), (4, 14, 14), (16, 28, 28), (32, 28, 28), (3, 45, 61), (32, 56, 56)]
 
@@ -61,3 +62,17 @@ def test_the_weight_a_module_keeps_a_filter_of(kind):
     for _ in range(8):                           # another weight, perhaps where the first one was
         assert not kept.holds(torch.randn(8, 8, 3, 3))
     assert place
+
+
+def test_modules_of_files_that_hold_a_filter():
+    """Modules were once written with what they keep, a key and a tensor: what a pass would take for a filter of now."""
+    layer = WinoConv2d(8, 16, 3, padding=1)
+    state = dict(layer.__getstate__(), _cache=((0, 1, (9, 9), torch.float16, 4, (0, 0, 4, 0)), torch.zeros(36 * 16 * 32)), _plan=None)
+    old = WinoConv2d.__new__(WinoConv2d)
+    old.__setstate__(state)
+    assert old._cache is None and old._plan is None and torch.equal(old.weight, layer.weight)
+    file = io.BytesIO()
+    torch.save(layer, file)
+    file.seek(0)
+    again = torch.load(file, weights_only=False)
+    assert again._cache is None and torch.equal(again.weight, layer.weight) and again.padding == layer.padding
