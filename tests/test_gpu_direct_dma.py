@@ -144,3 +144,19 @@ def test_tall_tiles_are_exact_on_small_integers(dev, dtype, tile, case, gemm_ove
     gemm_override(config=tile, rows_mode=0)
     y = engine.conv_forward(x.to(dtype).to(dev).contiguous(memory_format=torch.channels_last), w.to(dtype).to(dev), b.to(dtype).to(dev), stride, pad, 2, direct=True)
     assert torch.equal(y.cpu(), F.conv2d(x, w, b, stride, pad).float().to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("taps", [1, 2, 3])
+def test_tall_tiles_pass_infinities_and_nan_on(dev, dtype, taps, gemm_override):
+    """Odd and even counts of stages, the odd one with a stage of zeros behind it: what is no number reaches the pixels that read it, and no others."""
+    g = torch.Generator().manual_seed(13)
+    x = torch.randint(-3, 4, (2, 32, 41, 39), generator=g).double()
+    x[0, 31, 40, 38], x[1, 0, 0, 0], x[1, 7, 20, 20] = float("inf"), float("nan"), float("-inf")
+    w = torch.randint(1, 3, (136, 32, taps, taps), generator=g).double()
+    w[5, 7] = float("inf")
+    want = F.conv2d(x, w, None, 2).float().to(dtype)
+    for tile in (27, 28, 29):
+        gemm_override(config=tile, rows_mode=0)
+        y = engine.conv_forward(x.to(dtype).to(dev).contiguous(memory_format=torch.channels_last), w.to(dtype).to(dev), None, 2, 0, 2, direct=True).cpu()
+        assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y.nan_to_num(7.0), want.nan_to_num(7.0))

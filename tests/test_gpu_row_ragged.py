@@ -40,7 +40,6 @@ def test_as_padded(dev, case, dtype, gemm_override):
     w8[:K], b8[:K] = w, b
     for config in [-1, 16, 18, 19] + ([17] if taps < 7 else []) + ([21] if taps == 3 else []):
         for t in (x, odd):
-            print(case, dtype, config, flush=True)
             ragged = t[:, :C].to(dev).contiguous(memory_format=last)
             gemm_override(config=config)
             got = engine.conv_forward(ragged, w[:, :C].to(dev), b, 1, pad, 2, row=True)
@@ -58,7 +57,7 @@ def test_passes_of_a_batch(dev, C):
     w = torch.randn(40, C, 3, 3, device=dev).half()
     whole = engine.conv_forward(x, w, None, 1, 1, 2, row=True)
     for chunk in (1, 2):
-        assert torch.equal(engine.conv_forward(x, w, None, 1, 1, 2, chunk_images=chunk, row=True), whole)
+        assert torch.equal(engine.conv_forward(x, w, None, 1, 1, 2, chunk_images=chunk, row=True, channels_first_out=True), whole)
         assert torch.equal(engine.conv_forward(x.contiguous(), w, None, 1, 1, 2, chunk_images=chunk, row=True), whole)
 
 
