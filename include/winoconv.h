@@ -312,7 +312,9 @@ int wc_conv_forward_static(const wc_conv_desc* desc, const void* x,
  * helper exists for one, src/back/utils.cu:15-24; include/split_functions_grad.h:3-6 is empty).
  * dw[k][c][taps] = gradient of sum(y * dy) with respect to the filter, for the same descriptor as
  * the forward call: x (N, D, H, W, C) and dy (N, oD, oH, oW, K) channel-last contiguous, dw written
- * through element strides for the axes (K, C, kD, kH, kW).  Computed directly for 1x1, strided 2-D and most 16-bit 3x3 and
+ * through element strides for the axes (K, C, kD, kH, kW).  Any plan but stacked = 2 is taken; fp32 layers
+ * want the one that wc_conv_auto gives with direct = -1 (where the forward pass takes its pieces apart, a gradient taken so is
+ * up to 1.9 times as far from fp64).  Computed directly for 1x1, strided 2-D and most 16-bit 3x3 and
  * 3x3x3 layers, else in the transform domain
  * (dU = sum over tiles of dM x V, dw = G^T dU G) with every sum in fp32.  The input gradient needs
  * no entry point of its own: it is wc_conv_forward of dy with the flipped, transposed filter. */

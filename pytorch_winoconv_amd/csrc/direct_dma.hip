@@ -299,8 +299,8 @@ __global__ __launch_bounds__(256, WM * WN >= 6 ? 2 : WM * WN >= 4 ? 3 : 4) void 
 // A wavefront is alone on its SIMD, so nothing may wait: the fragments of a stage are read while the one before is multiplied (the only way that
 // 4 WM + 32 registers of operands are free again in time is two sets of them, hence two stages a turn of the loop), and a stage's loads are
 // spread over its rows of products (all at once, at its start, they hold the wavefront up until the last is taken: 40.2 | 36.6 us at N=8).
-// Of a stage of 448 x 128, 0.74 us, products and their fragment reads alone take 0.48 and the loads alone 0.47 (a CU takes in 85 GB/s
-// from L2): they overlap by half.  fp16, x in rotation, 256 x 128 | here: N=32 128 -> 128, 112x112 stride 2 52 | 49 us (50.5 | 50.3 with more between the calls), N=22 47.5 | 37.3, N=44 256 -> 256, 56x56 75 | 59.
+// Of a stage of 448 x 128, 0.74 us, products and their fragment reads alone take 0.48 and the loads alone 0.47 (78 KB/us into each
+// CU from L2): they overlap by half, and 36 stages are 27 us of the 47 below: x from memory, first loads and write-out are the rest.  fp16, x in rotation, 256 x 128 | here: N=32 128 -> 128, 112x112 stride 2 52 | 49 us (50.5 | 50.3 with more between the calls), N=22 47.5 | 37.3, N=44 256 -> 256, 56x56 75 | 59.
 template <typename T, int WM>
 __global__ __launch_bounds__(256, 1) void direct_wide_kernel(DirectDmaArgs a) {
   using MF = MfmaD<T>;
