@@ -435,7 +435,11 @@ int wc_conv_auto(wc_conv_desc* d) {
   if (never_direct) d->direct = 0;
   if (d->stacked == -1) {
     if (!d->direct && !never_direct && direct_conv_fits(d) && direct_preferred(d)) d->direct = 1;
-    if (may_row && !d->direct && !d->unfused && row_conv_fits(d) && row_preferred(d)) d->row = 1;
+    if (may_row && !d->direct && !d->unfused && d->K > 0) {
+      wc_conv_desc e = *d;
+      if (e.N < 1) e.N = 1;            // an empty batch has the form of one image (boxes of no images are no numbers)
+      if (row_conv_fits(&e) && row_preferred(&e)) d->row = 1;
+    }
     d->stacked = d->direct || d->row || (!never_direct && pieces_apart(d)) ? 0 : auto_stacked(d);
   }
   if (d->stacked == 2 && d->m == 4) {

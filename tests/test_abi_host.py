@@ -568,3 +568,22 @@ def test_5x5_and_7x7_layers_of_tile_4_take_the_faster_form(taps, N, C, K, H, row
         return engine.make_desc((N, C, H, H), (K, C, taps, taps), dtype, 1, taps // 2, m, stacked=None, row=True).row
     assert chosen(torch.float16, 4) == row and chosen(torch.bfloat16, 4) == 1
     assert chosen(torch.float16, 2) == (0 if taps == 5 and C > 256 else 1)
+
+
+def test_the_plan_of_an_empty_batch():
+    """It is asked for like any other (the reference fails in its launches: src/base_conv_launchers.cu:282-399), and so is that of no output channels,
+    which later functions refuse."""
+    import subprocess
+    import sys
+    code = ("import ctypes, sys, torch; sys.path.insert(0, %r)\n"
+            "from pytorch_winoconv_amd import _lib, engine\n"
+            "for kernel, pad in (((3, 3), (1, 3)), ((3, 3), (0, 0)), ((3, 3, 3), (1, 1, 1)), ((5, 5), (2, 2)), ((7, 7), (3, 3))):\n"
+            "    for dtype in (torch.float16, torch.bfloat16, torch.float32):\n"
+            "        for m in (2, 4):\n"
+            "            forms = [engine.make_desc((n, 35) + (9,) * len(kernel), (k, 35) + kernel, dtype, 1, pad, m, stacked=None, row=True)\n"
+            "                     for n, k in ((0, 24), (1, 24), (2, 0))]\n"
+            "            assert (forms[0].row, forms[0].m, forms[0].stacked) == (forms[1].row, forms[1].m, forms[1].stacked), (kernel, dtype, m)\n"
+            "            assert _lib.load().wc_conv_workspace_bytes(ctypes.byref(forms[2]), ctypes.byref(ctypes.c_size_t())) != 0\n"
+            % os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    run = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=110)
+    assert run.returncode == 0, run.stderr[-2000:]
