@@ -361,12 +361,13 @@ static int auto_stacked(const wc_conv_desc* d) {
 //
 // The line goes by the layer alone, not by the batch or the image: a filter that a caller transformed once is that of every call.  4x4 stays
 // stacked: its two plans have filters of one size (four pieces of two taps), so one in the place of the other could not be told by it.  us, apart |
-// stacked, transformed filter kept: tile 2, 5x5 256 -> 256, N=1 7x7 23 | 32, N=8 28x28 107 | 171, 256 -> 1024 N=1 14x14 37 | 38 (the worst), 512 -> 512
-// 39 | 56, N=2 28x28 121 | 176, 4x5 256 -> 64 N=16 28x28 88 | 100; tile 4, 5x5 256 -> 64, N=1 14x14 34 | 42, N=16 28x28 74 | 76, 256 -> 128 N=32 56x56 637 | 643, 1024 ->
-// 128 N=2 14x14 61 | 102, 384 -> 256 N=1 7x7 43 | 47, 512 -> 256 N=16 28x28 1.2 times as fast; at stride 2 as at stride 1; 3x3 stride 2, 160 -> 256, N=4 28x28
-// 29.9 | 29.4 (the worst), N=16 56x56 72 | 95, 512 -> 64, N=1 28x28 35 | 56.  With tile 4 and more output channels the sides alternate with the
-// tiles: 512 -> 512 N=1 14x14 100 | 88, N=16 121 | 202, 288 -> 384 44.5 | 40.6 and N=16 28x28 233 | 287, 256 -> 192 N=32 56x56 911 | 905, 4x5 256 -> 256 N=2 28x28 47.6 | 44.1.  Below
-// 225 channels they do so too (5x5 of 160 channels 0.88 to 1.33), and 6x6, which has no zero taps, is no faster up to 288 channels (0.85 to 1.1).
+// stacked, transformed filter kept, tile 2: 5x5 256 -> 256, N=1 7x7 23 | 32, N=8 28x28 107 | 171, 256 -> 1024 N=1 14x14 37 | 38 (the worst), 512 -> 512
+// 39 | 56, N=2 28x28 121 | 176, 4x5 256 -> 64 N=16 28x28 88 | 100; at stride 2 as at stride 1; 3x3 stride 2, 160 -> 256, N=4 28x28 29.9 | 29.4 (the worst), N=16
+// 56x56 72 | 95, 512 -> 64, N=1 28x28 35 | 56.  With tile 4, apart over stacked in the mean of twelve images from N=1 7x7 to N=8 56x56 (least, most):
+// 5x5 256 -> 160 0.91 (0.87, 0.97), 320 0.96 (0.91, 1.03), 384 0.99, 512 1.11 (0.83, 1.36); 288 -> 256 0.86 (0.74, 1.03), 512 0.90 (0.67, 1.25); 384 -> 384 0.83, 512 0.85
+// (0.61, 1.19), 768 0.78, 1024 0.97 (0.62, 1.43); 512 -> 512 0.80 (0.56, 1.13), 768 0.71, 1024 0.93 (0.61, 1.38); 4x5 256 -> 192 0.91, 384 0.96 (0.83, 1.07), 512 1.08 (0.70, 1.67), 512 ->
+// 384 0.83, 512 0.96 (0.63, 1.57): what loses is one image of few tiles into many channels.  Below 225 channels the sides alternate with the tiles (5x5 of
+// 160 channels 0.88 to 1.33), and 6x6, which has no zero taps, is no faster up to 288 channels (0.85 to 1.1).
 // The weight gradient (direct == -1) stays stacked: 5x5 256 -> 64, N=1 14x14 37 | 30, and less exact apart.
 static bool pieces_apart(const wc_conv_desc* d) {
   if (d->dtype != WC_F32 || d->ndim != 2) return false;
@@ -374,7 +375,7 @@ static bool pieces_apart(const wc_conv_desc* d) {
   const int Cp = wc_padded_channels(d->C);
   if (d->stride == 2 && kmin == 3 && kmax == 3) return Cp >= 160;
   if (kmin < 4 || kmax != 5 || Cp < 256) return false;
-  return d->m == 2 || d->K <= 128 || (kmin == 5 && Cp >= 384 && d->K <= 256);
+  return d->m == 2 || d->K <= (kmin == 4 ? 384 : Cp >= 288 ? 768 : 320);
 }
 
 // Where the direct form measured faster than the Winograd plan the caller would otherwise get.  Stride 2 in 16-bit,

@@ -23,6 +23,14 @@ def test_form_of_fp32_layers_is_the_layers(m, kernel, stride):
         assert len(forms) == 1, (C, K, forms)
 
 
+@pytest.mark.parametrize("kernel,C,K,apart", [
+    ((5, 5), 224, 64, (0, 0)), ((5, 5), 225, 320, (1, 1)), ((5, 5), 256, 321, (1, 0)), ((5, 5), 257, 768, (1, 1)), ((5, 5), 512, 769, (1, 0)),
+    ((4, 5), 224, 64, (0, 0)), ((4, 5), 225, 384, (1, 1)), ((5, 4), 512, 385, (1, 0)), ((4, 4), 512, 64, (0, 0)), ((6, 6), 512, 64, (0, 0)),
+])
+def test_where_the_pieces_of_fp32_layers_are_apart(kernel, C, K, apart):
+    assert apart == tuple(int(engine.make_desc((2, C, 30, 30), (K, C) + kernel, torch.float32, 1, 2, m, stacked=None).stacked == 0) for m in (2, 4))
+
+
 def test_filters_of_different_plans_differ_in_size():
     """The size is all that tells a filter of other options: the plan that is chosen has no other of its size in another order."""
     for kernel, stride, m, C, K in itertools.product(((4, 4), (4, 5), (5, 5), (3, 3)), (1, 2), (2, 4), (64, 256, 288, 512), (16, 512)):
