@@ -571,8 +571,7 @@ def test_5x5_and_7x7_layers_of_tile_4_take_the_faster_form(taps, N, C, K, H, row
 
 
 def test_the_plan_of_an_empty_batch():
-    """It is asked for like any other (the reference fails in its launches: src/base_conv_launchers.cu:282-399), and so is that of no output channels,
-    which later functions refuse."""
+    """It is asked for like any other, and so is that of no output channels, which later functions refuse."""
     import subprocess
     import sys
     code = ("import ctypes, sys, torch; sys.path.insert(0, %r)\n"
