@@ -161,7 +161,7 @@ const char* wc_last_error(void);
  * the number of tiles (9 only where the channel count allows it).
  * config 20: the weight gradient never takes the tap form (backward_taps.hip).
  * config 16 to 19: the row form with the wide, half, small or split workgroups whatever the problem (conv_row.hip).
- * config 21: the row form on tall boxes whatever the problem (conv_row_tall.hip).
+ * config 21: the row form on tall boxes whatever the problem (conv_row_tall.hip); config 30: on boxes of few tiles (conv_row_few.hip).
  * config 22 to 26: the direct form of 16-bit types on tiles of 256 x 128, 128 x 128, 256 x 64, 128 x 64 or 64 x 64 whatever the
  * problem (direct_dma.hip); 22 also: fp32 products and weight gradients on the fp32 instructions.  config 27 to 29: its forward
  * products on tiles of 320, 384 or 448 x 128.

@@ -37,14 +37,6 @@ struct RowArgs {
   int x_row, tail;                // elements from a pixel of x to the next: C, or `tail` (below 8) fewer
 };
 
-constexpr int kRowPitch = 64;     // LDS bytes per (element, row of a tile): 32 channels in four chunks of 16 bytes
-// Chunk g of row s lies at position g ^ (s / 4 % 4).  A 16-byte read is served in four phases of sixteen lanes over 64
-// banks, lanes 0-3, 12-15, 20-27 in the first, 4-11, 16-19, 28-31 in the second and the same 32 further up: of the lanes of
-// a phase with the same row modulo 4 each has another row / 4 modulo 4, so one chunk of 32 consecutive rows, from any
-// row on, is read without conflicts, and so is what a store writes, all chunks of 16 rows.  Two lanes of a phase whose
-// different rows agree modulo 16 take a cycle each: what the boxes make of that, see choose_box.
-__device__ __forceinline__ int v_offset(int s, int g) { return s * kRowPitch + ((g ^ (s >> 2)) & 3) * 16; }
-
 // What the NI items of a step carry beside their products: the transform of 8 UN channels, over the first two thirds of the
 // items, and for each unit six moves (an element to LDS, the next load of its register) behind its last channel
 template <int UN, int NI>
@@ -174,13 +166,7 @@ void row_conv_kernel(RowArgs a) {
 #pragma unroll
       for (int i = 0; i < UN; ++i)
 #pragma unroll
-        for (int j = 0; j < 6; ++j) {
-          u32x4 v = xr[i][j];
-          if (by & 4) v = u32x4{v[2], v[3], 0u, 0u};
-          if (by & 2) v = u32x4{v[1], v[2], v[3], 0u};
-          if (by & 1) v = u32x4{v[0] >> 16 | v[1] << 16, v[1] >> 16 | v[2] << 16, v[2] >> 16 | v[3] << 16, v[3] >> 16};
-          xr[i][j] = v;
-        }
+        for (int j = 0; j < 6; ++j) xr[i][j] = shift_channels(xr[i][j], by);
     }
   };
   // one of a unit's eight channels at a time, in place: the six inputs of xr become the six elements of the tile
@@ -512,7 +498,8 @@ __global__ __launch_bounds__(256) void row_filter_kernel(RowFilterArgs a) {
 // tile 0.  Cycles for the conflict-free number of them, per pass over the taps: N=64, 56x56 (4 images of 8 rows x 2 tiles) 24
 // for 12, 14x14 (14 rows x 4 tiles) 18 for 12, 28x28 15 for 12, 16x56x56 (4 planes of 14 rows x 1 tile) 72 for 36, N=1 7x7 6 for
 // 6; counted by SQ_LDS_BANK_CONFLICT at N=64 256 -> 256, 56x56: 14.45 M of 36.1 M cycles of the LDS.
-struct RowBox { int bn, bd, bh, bw, n_n, n_d, n_h, n_w, prow, irow; long long boxes; };
+}  // namespace
+
 RowBox choose_box(int N, int oD, int oH, int nW, int kd, int kh, int tiles, int slots) {
   RowBox best{};
   long long best_rows = 0;
@@ -536,6 +523,8 @@ RowBox choose_box(int N, int oD, int oH, int nW, int kd, int kh, int tiles, int 
   return best;
 }
 
+namespace {
+
 // The shapes of workgroup, by what fills the chip.  Measured, fp16, us (wide, a workgroup per box | half | small | split):
 //   wide   eight wavefronts, 64 tiles x 128 channels, one workgroup per CU: every byte of V is used for 128 channels
 //   half   four, 64 tiles x 64 channels, two per CU: the transform of one runs beside the products of the other, finer rounds
@@ -545,8 +534,9 @@ RowBox choose_box(int N, int oD, int oH, int nW, int kd, int kh, int tiles, int 
 // 68 | 60 | 74; N=16, 256 -> 256, 14x14 21 | 15 | 12.4 | 10.6; N=1, 512 -> 512, 7x7 33 | 22 | 19 | 12.  (Layers of up to 128 input
 // channels come here in 3-D or with tile 4; with tile 2 the one-kernel F(2x2, 3x3) form takes most of them, see row_preferred.)
 enum RowShape { kRowWide, kRowHalf, kRowSmall, kRowSplit };
-// tall_planes: output planes, images in 2-D, that go to tall boxes; the rest is rest_n images of rest_d planes
-struct RowPlan { RowShape shape; RowBox box; long long wide_groups; int tall_planes, rest_n, rest_d; double us; };
+// tall_planes: output planes, images in 2-D, that go to tall boxes; the rest is rest_n images of rest_d planes.  few: all in boxes of few tiles instead
+// (conv_row_few.hip)
+struct RowPlan { RowShape shape; RowBox box; long long wide_groups; int tall_planes, rest_n, rest_d; bool few; double us; };
 
 //
 // How long a launch of each takes, in units of a full round of the wide shape, fitted to 330 layers drawn over 1 to 64 images, 32 to 512 channels and
@@ -613,7 +603,8 @@ RowPlan make_row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int 
   const int steps = ceil_div(C, 32);
   RowPlan best = make_row_shape(N, oD, oH, nW, kd, kh, K, steps);
   best.rest_n = N; best.rest_d = oD;
-  if (kh != 3) return best;
+  best.few = row_few_pays((long long)N * oD, oH, nW, kd, kh, K, C, copied);
+  if (kh != 3 || best.few) return best;
   const double box_us = 2.1 * 2 * steps * kd + 10.5;
   // Tall boxes read padded rows.  What their copy takes between two layers that differ by it alone, over 109 layers: tall boxes and the others are
   // chosen with 0.1 % lost in the mean (at 3 us and 9 TB/s 0.4 %: N=31 175 -> 232, 66x25 52 us, 47 in wide boxes).  Where x is copied in any case
@@ -809,7 +800,7 @@ bool row_reads_padded(const wc_conv_desc* d) {
   if (d->C % 8 == 0) return false;
   const int force = test_gemm_config(), kd = d->kernel[0], kh = d->kernel[1];
   if (d->C < 8 || (force == 21 && kh == 3)) return true;
-  if (kh != 3 || (force >= 16 && force <= 19)) return false;
+  if (kh != 3 || (force >= 16 && force <= 19) || force == 30) return false;
   return row_plan(d->N, d->in[0] + 2 * d->pad[0] - kd + 1, d->in[1] + 2 * d->pad[1] - 2, ceil_div(d->in[2] + 2 * d->pad[2] - 2, 4), kd, kh, d->K,
                   d->C).tall_planes > 0;
 }
@@ -836,6 +827,7 @@ int row_conv(const wc_conv_desc* d, const void* x, int x_row, int first_image, i
   if (force >= 16 && force <= 19) { plan.shape = (RowShape)(force - 16); plan.tall_planes = 0; plan.rest_n = -1; }
   if (force == 21 && d->kernel[1] == 3) plan.tall_planes = d->N * a.oD;
   const int tall = std::min(std::max(plan.tall_planes - first_image * a.oD, 0), n_images * a.oD);
+  if (force == 30 || (plan.few && force != 21 && (force < 16 || force > 19))) return row_few_conv(d, x, x_row, n_images, U, bias, y, stream);
   if (tall > 0) {
     WC_CHECK_ARG(a.tail == 0, "row form: tall boxes of %d channels", x_row);
     const int rc = tall_row_conv(d, x, tall, U, bias, y, stream);

@@ -91,4 +91,29 @@ __device__ __forceinline__ void store_some(T* dst, u32x4 v, int n) {
   if (n & 1) __builtin_memcpy(dst, &next, 2);
 }
 
+constexpr int kRowPitch = 64;     // LDS bytes per (element, row of a tile): 32 channels in four chunks of 16 bytes
+// Chunk g of row s lies at position g ^ (s / 4 % 4).  A 16-byte read is served in four phases of sixteen lanes over 64
+// banks, lanes 0-3, 12-15, 20-27 in the first, 4-11, 16-19, 28-31 in the second and the same 32 further up: of the lanes of
+// a phase with the same row modulo 4 each has another row / 4 modulo 4, so one chunk of 32 consecutive rows, from any
+// row on, is read without conflicts, and so is what a store writes, all chunks of 16 rows.  Two lanes of a phase whose
+// different rows agree modulo 16 take a cycle each: what the boxes make of that, see choose_box.
+__device__ __forceinline__ int v_offset(int s, int g) { return s * kRowPitch + ((g ^ (s >> 2)) & 3) * 16; }
+
+// eight 16-bit elements without the first `by` < 8, zeros behind them
+__device__ __forceinline__ u32x4 shift_channels(u32x4 v, int by) {
+  if (by & 4) v = u32x4{v[2], v[3], 0u, 0u};
+  if (by & 2) v = u32x4{v[1], v[2], v[3], 0u};
+  if (by & 1) v = u32x4{v[0] >> 16 | v[1] << 16, v[1] >> 16 | v[2] << 16, v[2] >> 16 | v[3] << 16, v[3] >> 16};
+  return v;
+}
+
+// The box of output tiles of a workgroup (conv_row.hip): images, planes, rows, tiles of a row, how many along each axis, the LDS rows of a plane and an image
+struct RowBox { int bn, bd, bh, bw, n_n, n_d, n_h, n_w, prow, irow; long long boxes; };
+RowBox choose_box(int N, int oD, int oH, int nW, int kd, int kh, int tiles, int slots);
+
+// Few tiles (conv_row_few.hip): whether the kernel is taken for `planes` output planes (padded: x with channels padded to a multiple of 8), and the
+// launch with the arguments of row_conv
+bool row_few_pays(long long planes, int oH, int nW, int kd, int kh, int K, int C, bool padded);
+int row_few_conv(const wc_conv_desc* d, const void* x, int x_row, int n_images, const void* U, const void* bias, void* y, void* stream);
+
 }  // namespace wc
