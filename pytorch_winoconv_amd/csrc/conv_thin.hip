@@ -18,8 +18,7 @@
 // a product is added into the accumulators it belongs to), the height half in fp32 registers.  The
 // window of the next block is requested before the products of this one, and LDS is
 // double-buffered, so there is one barrier per block.  With 128 channels U would take the whole
-// register file: eight wavefronts then share a block, four per pair of element rows, and the
-// upper four hand their share of each output tile to the lower four through LDS (a second barrier).
+// register file: thin_rows_kernel gives a wavefront one row of the elements.
 // Launches with few blocks of tiles use workgroups of half the size (32 output channels), and U reaches the
 // registers through LDS: see thin_conv3x3_kernel.
 #include "wc_transform.h"
@@ -67,6 +66,13 @@ static_assert(Mats<KIND_23>::at(0, 0) == 1 && Mats<KIND_23>::at(0, 1) == 1 && Ma
 constexpr int kThinTiles = 16;      // tiles per block
 constexpr int kThinK = 64;          // output channels per workgroup
 
+// Rows of U and V that fill a line of LDS (thin_rows_kernel), and the threads and the LDS of a workgroup: of those, a wavefront per row of
+// elements and 32 output channels, and V of two blocks of tiles with what the rows hand over behind it
+template <typename T, int CP> constexpr bool kThinRows = CP * sizeof(T) == 256;
+template <typename T, int CP, int KSUB> constexpr int kThinThreads = (kThinRows<T, CP> ? 128 : 64) * KSUB;
+template <typename T, int CP, int KSUB>
+constexpr int kThinLds = 2 * 16 * kThinTiles * CP * (int)sizeof(T) + (kThinRows<T, CP> ? KSUB * 8 * 1024 : 0);
+
 struct ThinArgs {
   const void* x;
   const void* U;
@@ -85,27 +91,27 @@ struct ThinArgs {
   FastDiv div_nW, div_nH;
 };
 
-// Store of one lane's share of an output tile: tile p, output channels ko .. ko + 4, the 2 x 2 output positions
-// in out[oa][ob], bias bv added.  Stores go through a buffer descriptor and are issued unconditionally: a
+// Store of one lane's share of an output tile: tile p, output channels ko .. ko + 4, both output rows and the OBN output columns
+// from ob0 on in out[oa][ob], bias bv added.  Stores go through a buffer descriptor and are issued unconditionally: a
 // position outside (oH, oW), a tile beyond the last or a lane without work (`live` false) gets an offset beyond
 // the buffer and is dropped by the hardware.  No branch around the stores matters for speed: loads and stores
 // share one in-order counter, and only with straight-line code can the wait for the next block's window leave
 // this block's stores in flight.
-template <typename T, bool KW>
+template <typename T, bool KW, int OBN>
 __device__ __forceinline__ void store_tile(const ThinArgs& a, __amdgpu_buffer_rsrc_t ydesc, int p, int ko, bool live,
-                                           const float (&bv)[4], const floatx4 (&out)[2][2]) {
+                                           const float (&bv)[4], const floatx4 (&out)[2][OBN], int ob0 = 0) {
   const int q = fast_div(p, a.div_nW);
   const int tw = p - q * a.nW;
   const int b = fast_div(q, a.div_nH);
   const int th = q - b * a.nH;
-  const unsigned o00 = (((unsigned)b * a.oH + 2 * th) * a.oW + 2 * tw) * a.K + ko;   // in elements
-  const bool h1 = 2 * th + 1 < a.oH, w1 = 2 * tw + 1 < a.oW;
+  const unsigned o00 = (((unsigned)b * a.oH + 2 * th) * a.oW + 2 * tw + ob0) * a.K + ko;   // in elements
+  const bool h1 = 2 * th + 1 < a.oH;
 #pragma unroll
   for (int oa = 0; oa < 2; ++oa) {
 #pragma unroll
-    for (int ob = 0; ob < 2; ++ob) {
+    for (int ob = 0; ob < OBN; ++ob) {
       const floatx4 s4 = out[oa][ob];
-      const bool inside = live && (oa == 0 || h1) && (ob == 0 || w1);
+      const bool inside = live && (oa == 0 || h1) && 2 * tw + ob0 + ob < a.oW;
       const unsigned off = o00 + (oa * a.oW + ob) * a.K;
       Pack<T, 4> o;
 #pragma unroll
@@ -141,19 +147,28 @@ __device__ __forceinline__ void load_bias(const ThinArgs& a, int ko, float (&bv)
 }
 
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+struct TwoFloats {                  // (a vector of two costs moves of register pairs)
+  float lo, hi;
+  __device__ __forceinline__ TwoFloats operator+(TwoFloats o) const { return {lo + o.lo, hi + o.hi}; }
+  __device__ __forceinline__ TwoFloats operator-(TwoFloats o) const { return {lo - o.lo, hi - o.hi}; }
+};
 
-// B^T of F(2,3) along one axis of a 4 x 4 block (STRIDE: distance between the four elements,
-// OTHER: distance between the four lines).
-template <int STRIDE, int OTHER, typename V>
-__device__ __forceinline__ void bt23(const V (&in)[16], V (&out)[16]) {
+// B^T of F(2,3) on four elements, STRIDE apart
+template <int STRIDE, typename V>
+__device__ __forceinline__ void bt23(V* d) {
+  const V d0 = d[0], d1 = d[STRIDE], d2 = d[2 * STRIDE], d3 = d[3 * STRIDE];
+  d[0] = d0 - d2;
+  d[STRIDE] = d1 + d2;
+  d[2 * STRIDE] = d2 - d1;
+  d[3 * STRIDE] = d1 - d3;
+}
+// the whole block: along its lines, then its columns
+template <typename V>
+__device__ __forceinline__ void transform(V (&d)[16]) {
 #pragma unroll
-  for (int l = 0; l < 4; ++l) {
-    const V d0 = in[l * OTHER], d1 = in[l * OTHER + STRIDE], d2 = in[l * OTHER + 2 * STRIDE], d3 = in[l * OTHER + 3 * STRIDE];
-    out[l * OTHER] = d0 - d2;
-    out[l * OTHER + STRIDE] = d1 + d2;
-    out[l * OTHER + 2 * STRIDE] = d2 - d1;
-    out[l * OTHER + 3 * STRIDE] = d1 - d3;
-  }
+  for (int l = 0; l < 4; ++l) bt23<1>(d + 4 * l);
+#pragma unroll
+  for (int l = 0; l < 4; ++l) bt23<4>(d + l);
 }
 static_assert(Mats<KIND_23>::bt(0, 0) == 1 && Mats<KIND_23>::bt(0, 2) == -1 && Mats<KIND_23>::bt(1, 1) == 1 &&
               Mats<KIND_23>::bt(1, 2) == 1 && Mats<KIND_23>::bt(2, 1) == -1 && Mats<KIND_23>::bt(2, 2) == 1 &&
@@ -166,15 +181,12 @@ static_assert(Mats<KIND_23>::bt(0, 0) == 1 && Mats<KIND_23>::bt(0, 2) == -1 && M
 // would leave more than half of the CUs idle (a workgroup with one block spends most of its time fetching U and,
 // in fp32, multiplying).
 template <typename T, int CP, bool KW, int KSUB>
-__global__ __launch_bounds__((CP * sizeof(T) > 128 ? 128 : 64) * KSUB) __attribute__((amdgpu_waves_per_eu(KSUB / 2, KSUB / 2))) void thin_conv3x3_kernel(ThinArgs a) {
-  // Up to 64 channels a wavefront holds U of all 16 elements (4 wavefronts).  With 128 that is twice
-  // the register file, so SPLIT: 8 wavefronts, the upper four take the element rows 2 and 3 and hand
-  // their share of the output tile to the lower four through LDS.
-  constexpr bool SPLIT = CP * sizeof(T) > 128;       // 128 channels of a 16-bit type, 64 of fp32
+__global__ __launch_bounds__(64 * KSUB) __attribute__((amdgpu_waves_per_eu(KSUB / 2, KSUB / 2))) void thin_conv3x3_kernel(ThinArgs a) {
+  static_assert(CP * sizeof(T) <= 128, "a wavefront holds U of all 16 elements");
   constexpr bool PLAIN = sizeof(T) == 4;             // one accumulator per element, width transform in VALU (measured: no gain for 16-bit types)
   constexpr int EPF = 16 / sizeof(T);                // channels per 16-byte fragment
-  constexpr int NT = (SPLIT ? 128 : 64) * KSUB;
-  constexpr int NROW = SPLIT ? 2 : 4;     // element rows per wavefront
+  constexpr int NT = 64 * KSUB;
+  constexpr int NROW = 4;                 // element rows
   constexpr int VEC = kThinTiles * CP / NT;   // channels per thread in the transform
   constexpr int CVECS = CP / VEC;
   constexpr int KS = CP / (4 * EPF);      // fragment steps along the channels (four lane groups x EPF channels each)
@@ -184,9 +196,9 @@ __global__ __launch_bounds__((CP * sizeof(T) > 128 ? 128 : 64) * KSUB) __attribu
   // (rows padded by 16 bytes, which are conflict-free for 128-byte wide LDS, measured half that rate).  With R rows
   // per 256 bytes, chunk c of row r sits at position c ^ ((r / R) mod chunks per row).
   constexpr int PITCH = CP * sizeof(T);
-  constexpr int CPRW = PITCH / 16;             // chunks per row: 4, 8 or 16
+  constexpr int CPRW = PITCH / 16;             // chunks per row: 4 or 8
   constexpr int RPL = 16 / CPRW;               // rows per 256-byte line
-  static_assert(CPRW == 4 || CPRW == 8 || CPRW == 16, "rows of 64, 128 or 256 bytes");
+  static_assert(CPRW == 4 || CPRW == 8, "rows of 64 or 128 bytes");
   static_assert(VEC * sizeof(T) <= 16, "a thread's channels stay inside one chunk");
   constexpr int BUF = 16 * kThinTiles * PITCH;
   using MF = Mfma16<T>;
@@ -194,8 +206,7 @@ __global__ __launch_bounds__((CP * sizeof(T) > 128 ? 128 : 64) * KSUB) __attribu
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int kbase = (blockIdx.y * KSUB + wave % KSUB) * 16;
-  const int row0i = SPLIT ? 2 * (wave / KSUB) : 0;       // first element row of this wavefront
+  const int kbase = (blockIdx.y * KSUB + wave) * 16;
 
   // transform role: tile pl of the block, channels c .. c + VEC.  x is read through a buffer descriptor:
   // one 32-bit offset per load, and a window element outside the image is an offset beyond the
@@ -265,7 +276,7 @@ __global__ __launch_bounds__((CP * sizeof(T) > 128 ? 128 : 64) * KSUB) __attribu
       constexpr int t = decltype(t_)::value;
 #pragma unroll
       for (int i = 0; i < KS; ++i) {
-        const long long row = (long long)(row0i * 4 + t) * a.K + min(kbase + srow[i], a.K - 1);
+        const long long row = (long long)t * a.K + min(kbase + srow[i], a.K - 1);
         tmp[t][i] = *reinterpret_cast<const uint4v*>(Ub + row * PITCH + scol[i]);
       }
     });
@@ -319,22 +330,20 @@ __global__ __launch_bounds__((CP * sizeof(T) > 128 ? 128 : 64) * KSUB) __attribu
     static_for<0, VEC / 2>([&](auto h_) {
       constexpr int h = decltype(h_)::value;
       if constexpr (std::is_same<T, half_t>::value) {
-        half2v d[16], t2[16];
+        half2v d[16];
 #pragma unroll
         for (int e = 0; e < 16; ++e) d[e] = half2v{raw[e].v[2 * h], raw[e].v[2 * h + 1]};
-        bt23<1, 4>(d, t2);
-        bt23<4, 1>(t2, d);
+        transform(d);
 #pragma unroll
         for (int e = 0; e < 16; ++e)
           *reinterpret_cast<half2v*>(vdst + e * (kThinTiles * PITCH / (int)sizeof(T)) + 2 * h) = d[e];
       } else {
         typedef float float2v __attribute__((ext_vector_type(2)));
-        float2v d[16], t2[16];
+        float2v d[16];
 #pragma unroll
         for (int e = 0; e < 16; ++e)
           d[e] = float2v{static_cast<float>(raw[e].v[2 * h]), static_cast<float>(raw[e].v[2 * h + 1])};
-        bt23<1, 4>(d, t2);
-        bt23<4, 1>(t2, d);
+        transform(d);
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
           const float o[2] = {d[e][0], d[e][1]};
@@ -352,7 +361,7 @@ __global__ __launch_bounds__((CP * sizeof(T) > 128 ? 128 : 64) * KSUB) __attribu
     // MFMAs are cheap and registers are what is short.  fp32, whose MFMAs are sixteen times slower and bound the
     // kernel, keeps one accumulator per element and adds in VALU.  Consecutive MFMAs write different accumulators.
     floatx4 zw[NROW][2];
-    const unsigned char* vrow = buf + (lane & 15) * PITCH + row0i * 4 * kThinTiles * PITCH;
+    const unsigned char* vrow = buf + (lane & 15) * PITCH;
     const int vswz = ((lane & 15) / RPL) & (CPRW - 1);
     if constexpr (PLAIN) {
       floatx4 mm[NROW][4];
@@ -414,38 +423,317 @@ __global__ __launch_bounds__((CP * sizeof(T) > 128 ? 128 : 64) * KSUB) __attribu
     // Height half of the output transform: out[0][b] = zw[0][b] + zw[1][b] + zw[2][b], out[1][b] = zw[1][b] -
     // zw[2][b] - zw[3][b].
     floatx4 out[2][2];
-    if constexpr (!SPLIT) {
 #pragma unroll
-      for (int ob = 0; ob < 2; ++ob) {
-        out[0][ob] = zw[0][ob] + zw[1][ob] + zw[2][ob];
-        out[1][ob] = zw[1][ob] - zw[2][ob] - zw[3][ob];
-      }
-    } else {
-      // the upper wavefronts (rows 2, 3) pass their share through LDS to the lower ones (rows 0, 1)
-      floatx4* xch = reinterpret_cast<floatx4*>(lds + 2 * BUF) + ((wave % KSUB) * 4) * 64 + lane;
-      const bool upper = wave >= KSUB;
-#pragma unroll
-      for (int ob = 0; ob < 2; ++ob) {
-        const floatx4 za = zw[0][ob], zb = zw[1][ob];
-        out[0][ob] = upper ? za : za + zb;
-        out[1][ob] = upper ? -za - zb : zb;
-      }
-      if (upper) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) xch[q * 64] = out[q >> 1][q & 1];
-      }
-      __syncthreads();
-      if (!upper) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) out[q >> 1][q & 1] += xch[q * 64];
-      }
+    for (int ob = 0; ob < 2; ++ob) {
+      out[0][ob] = zw[0][ob] + zw[1][ob] + zw[2][ob];
+      out[1][ob] = zw[1][ob] - zw[2][ob] - zw[3][ob];
     }
 
     // lane = tile lane % 16, output channels ko .. ko + 4
     const int p = blk * kThinTiles + (lane & 15);
     const int ko = kbase + 4 * (lane >> 4);
-    store_tile<T, KW>(a, ydesc, p, ko, p < a.P && ko < a.K && (!SPLIT || wave < KSUB), bv, out);
+    store_tile<T, KW, 2>(a, ydesc, p, ko, p < a.P && ko < a.K, bv, out);
   }
+}
+
+// The same for rows of U and V of 256 bytes: 128 channels of a 16-bit type, 64 of fp32.  U of 16 output channels and all
+// elements would be twice the register file, so a wavefront has one row of elements and 32 output channels (KB groups of 16), and the
+// rows meet in LDS.  One workgroup is all a CU's LDS holds, so nothing else runs while its wavefronts wait for each other: the
+// transform of the next block, the loads of the one after and the output of the one before are dealt out over a block's
+// products, and a block has one barrier that waits for LDS and one that waits for nothing.
+//
+// Two rows of elements and 16 output channels a wavefront, each phase of a block behind the last one, took 73 us (2.6 a block) where this
+// takes 58 (fp16 N=64 128 -> 128, 56x56; 28x28 25.3 | 21.4; bf16 77 | 65; fp32 N=64 64 -> 64, 56x56 79 | 70).  The dealing out
+// alone is 70: fragments of V fed one product and a half, LDS 256 KB of reads a block.  What is left of 1.8 us a block: taken out one at a
+// time, the loads are 0.35 of it (64 KB through L1, the same from a footprint of 4 KB), products 0.4, the output 0.3, transform and its stores 0.2.
+// Of a thin_conv3x3_kernel with 128-byte rows two run on a CU, side by side, and the same order of its work was slower (64 channels 23.0 | 23.8).
+template <typename T, int CP, bool KW, int KSUB>
+__global__ __launch_bounds__((kThinThreads<T, CP, KSUB>)) __attribute__((amdgpu_waves_per_eu(KSUB / 2, KSUB / 2))) void thin_rows_kernel(ThinArgs a) {
+  constexpr bool PLAIN = sizeof(T) == 4;             // one accumulator per element, width transform in VALU (measured: no gain for 16-bit types)
+  constexpr int EPF = 16 / sizeof(T);                // channels per 16-byte fragment
+  constexpr int NT = kThinThreads<T, CP, KSUB>, NW = NT / 64;
+  constexpr int KB = KSUB * 4 / NW;                  // groups of 16 output channels per wavefront, of one row of elements
+  constexpr int VEC = kThinTiles * CP / NT;   // channels per thread in the transform
+  constexpr int CVECS = CP / VEC;
+  constexpr int KS = CP / (4 * EPF);      // fragment steps along the channels (four lane groups x EPF channels each)
+  // rows of an (element, tile) in LDS as in thin_conv3x3_kernel: chunk c of row r at position c ^ r
+  static_assert(CP * sizeof(T) == 256, "a row is a line of LDS");
+  constexpr int PITCH = CP * sizeof(T);
+  static_assert(VEC * sizeof(T) >= 4 && VEC * sizeof(T) <= 16, "a thread's channels stay inside one chunk");
+  constexpr int ELEM = kThinTiles * PITCH, BUF = 16 * ELEM;
+  using MF = Mfma16<T>;
+  using Frag = typename MF::Frag;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row = wave & 3;                              // this wavefront's row of elements
+  const int kbase = (blockIdx.y * KSUB + (wave >> 2) * KB) * 16;
+
+  // transform role: tile pl of the block, channels c .. c + VEC.  x is read through a buffer descriptor:
+  // one 32-bit offset per load, and a window element outside the image is an offset beyond the
+  // buffer, which reads as zero.
+  const int pl = tid / CVECS;
+  const int c = (tid % CVECS) * VEC;
+  const bool c_ok = c < a.C;
+  const __amdgpu_buffer_rsrc_t rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.x), 0, a.x_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t ydesc = __builtin_amdgcn_make_buffer_rsrc(a.y, 0, a.y_bytes, 0x00020000);
+  using Words = Pack<uint32_t, VEC * (int)sizeof(T) / 4>;
+  Words raw[16];
+
+  // Offset of a window element = row part + column part.  A row outside the image contributes
+  // 2^31 and a column outside 2^30: with x below 1 GiB every sum that contains one of them lies
+  // beyond the buffer, so no per-element select is needed.
+  unsigned rowoff[4], coloff[4];
+  auto find_window = [&](int blk) {
+    const int p = blk * kThinTiles + pl;
+    const bool valid = (p < a.P) & c_ok;
+    const int q = fast_div(p, a.div_nW);
+    const int tw = p - q * a.nW;
+    const int b = fast_div(q, a.div_nH);
+    const int th = q - b * a.nH;
+    const int y0 = 2 * th - a.pad1, x0 = 2 * tw - a.pad2;
+    const unsigned row0 = (unsigned)(b * a.H + y0) * (unsigned)a.row_bytes;
+    const unsigned col0 = (unsigned)(x0 * a.C + c) * (unsigned)sizeof(T);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      rowoff[i] = valid & ((unsigned)(y0 + i) < (unsigned)a.H) ? row0 + i * a.row_bytes : 0x80000000u;
+      coloff[i] = (unsigned)(x0 + i) < (unsigned)a.W ? col0 + i * a.C * (unsigned)sizeof(T) : 0x40000000u;
+    }
+  };
+  auto load_element = [&](int e) { raw[e] = __builtin_bit_cast(Words, buffer_load_pack<T, VEC>(rsrc, rowoff[e >> 2] + coloff[e & 3])); };
+  auto load_window = [&](int blk) {
+    find_window(blk);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) load_element(e);
+  };
+
+  const int nwg = gridDim.x;
+  int blk = xcd_remap(blockIdx.x, a.per_xcd);
+  if (blk < a.n_blocks) load_window(blk);   // in flight while U arrives
+
+  // this wavefront's part of U: row operand, lane = output channel kbase + lane % 16, 8 channels
+  // from 8 * (lane / 16).  Rows beyond K repeat row K - 1: a row of U only reaches the same row of the
+  // product, and those rows are never stored.
+  // Memory is read in whole rows (consecutive lanes take consecutive 16 bytes) and the fragments go to the lanes
+  // that need them through this wavefront's own slice of LDS, which nothing else uses yet: a load whose
+  // neighbouring lanes address different rows, as the operand layout would have it, measured 3.8 times slower per
+  // byte with every line in L2, and for a workgroup with one block of tiles that load is most of the kernel.
+  constexpr int NEL = 4 * KB;                          // blocks of 16 rows of U: element t / KB of the row, channels 16 (t % KB)
+  Frag u[NEL][KS];
+  {
+    constexpr int SLICE = 2 * BUF / NW;                // bytes of LDS per wavefront
+    constexpr int EPR = SLICE / (16 * PITCH) < NEL ? SLICE / (16 * PITCH) : NEL;          // blocks per round: 16 rows of U each
+    static_assert(EPR >= 1 && NEL % EPR == 0 && KS == PITCH / 64, "staging of U");
+    unsigned char* slice = lds + wave * SLICE;
+    const unsigned char* Ub = static_cast<const unsigned char*>(a.U);
+    uint4v tmp[NEL][KS];
+    int srow[KS], scol[KS];
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+      const int off = (i * 64 + lane) * 16;            // byte of the 16-row block
+      srow[i] = off / PITCH;
+      scol[i] = off % PITCH;
+    }
+    static_for<0, NEL>([&](auto t_) {
+      constexpr int t = decltype(t_)::value;
+#pragma unroll
+      for (int i = 0; i < KS; ++i) {
+        const long long r = (long long)(row * 4 + t / KB) * a.K + min(kbase + t % KB * 16 + srow[i], a.K - 1);
+        tmp[t][i] = *reinterpret_cast<const uint4v*>(Ub + r * PITCH + scol[i]);
+      }
+    });
+    const int fswz = lane & 15;
+    static_for<0, NEL / EPR>([&](auto r_) {
+      constexpr int rd = decltype(r_)::value;
+      static_for<0, EPR>([&](auto e_) {
+        constexpr int e = decltype(e_)::value;
+#pragma unroll
+        for (int i = 0; i < KS; ++i)
+          *reinterpret_cast<uint4v*>(slice + (e * 16 + srow[i]) * PITCH +
+                                     (((scol[i] >> 4) ^ (srow[i] & 15)) << 4)) = tmp[rd * EPR + e][i];
+      });
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      static_for<0, EPR>([&](auto e_) {
+        constexpr int e = decltype(e_)::value;
+        static_for<0, KS>([&](auto s_) {
+          constexpr int s2 = decltype(s_)::value;
+          u[rd * EPR + e][s2] = *reinterpret_cast<const Frag*>(slice + (e * 16 + (lane & 15)) * PITCH +
+                                                              ((((lane >> 4) + 4 * s2) ^ fswz) << 4));
+        });
+      });
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    });
+  }
+
+  // What this lane finishes: four output channels (`quad` of the workgroup's) of a tile, in one output column.  Neighbouring
+  // lanes have neighbouring channels, so that stores are 128 bytes (64 of 32 output channels) at a time.
+  constexpr int QUADS = 4 * KSUB;
+  static_assert(2 * kThinTiles * QUADS == NT, "a column of a quad for every thread");
+  const int quad = lane % QUADS, ob = wave & 1, my_tile = (wave >> 1) * (64 / QUADS) + lane / QUADS;
+  const int ko = blockIdx.y * KSUB * 16 + quad * 4;
+
+  // U and the bias have arrived before the loop starts: a wait for them inside the loop would also wait, on
+  // every pass, for the window loads of the next block, which are younger (loads return in order).
+  float bv[4];
+  load_bias<T>(a, ko, bv);
+#pragma unroll
+  for (int t = 0; t < NEL; ++t)
+#pragma unroll
+    for (int s2 = 0; s2 < KS; ++s2) asm volatile("" : "+v"(u[t][s2]));
+#pragma unroll
+  for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(bv[r]));
+  __syncthreads();   // the first block's V goes where other wavefronts staged their U
+
+  // Input transform in units: B^T on a line of two channels' windows, or on a column, whose results go back to where the window was.
+  // fp16 adds pairs of channels in fp16 like the reference's kernels (calculation_kernels.cu:786-806 computes in T); bf16,
+  // which has no packed add, goes through fp32.
+  using Two = std::conditional_t<std::is_same<T, half_t>::value, half2v, TwoFloats>;
+  constexpr int UNITS = 4 * VEC;               // per pair of channels four lines, then four columns
+  Two d[16];
+  auto transform_unit = [&](auto u_) {
+    constexpr int u = decltype(u_)::value, h = u / 8, l = u % 4;
+    if constexpr (u % 8 < 4) {
+#pragma unroll
+      for (int e = 4 * l; e < 4 * l + 4; ++e) {
+        if constexpr (std::is_same<T, half_t>::value) d[e] = __builtin_bit_cast(half2v, raw[e].v[h]);
+        else if constexpr (sizeof(T) == 2) d[e] = TwoFloats{__builtin_bit_cast(float, raw[e].v[h] << 16), __builtin_bit_cast(float, raw[e].v[h] & 0xffff0000u)};
+        else d[e] = TwoFloats{__builtin_bit_cast(float, raw[e].v[2 * h]), __builtin_bit_cast(float, raw[e].v[2 * h + 1])};
+      }
+      bt23<1>(d + 4 * l);
+    } else {
+      bt23<4>(d + l);
+#pragma unroll
+      for (int e = l; e < 16; e += 4) {
+        if constexpr (std::is_same<T, half_t>::value) {
+          raw[e].v[h] = __builtin_bit_cast(uint32_t, d[e]);
+        } else if constexpr (sizeof(T) == 2) {
+          const Pack<T, 2> two = {{static_cast<T>(d[e].lo), static_cast<T>(d[e].hi)}};
+          raw[e].v[h] = __builtin_bit_cast(uint32_t, two);
+        } else {
+          raw[e].v[2 * h] = __builtin_bit_cast(uint32_t, d[e].lo);
+          raw[e].v[2 * h + 1] = __builtin_bit_cast(uint32_t, d[e].hi);
+        }
+      }
+    }
+  };
+  // all channels of this thread lie in one chunk
+  const int cb = c * (int)sizeof(T);
+  unsigned char* const vdst = lds + pl * PITCH + ((((cb >> 4) ^ pl) << 4) | (cb & 15));
+  auto store_element = [&](int e, int buf) {
+    typedef uint32_t vec __attribute__((ext_vector_type(VEC * sizeof(T) / 4)));
+    *reinterpret_cast<vec*>(vdst + buf + e * ELEM) = __builtin_bit_cast(vec, raw[e]);
+  };
+  auto meet = [&]() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+  };
+
+  // The height half of the output transform takes the four rows of elements, which are four wavefronts': each leaves its
+  // zw[0 .. 1] of KB groups of 16 channels in LDS behind V, 1 KB each, and a block later all finish what these add up to.
+  // A lane leaves the channels 4 (lane / 16) .. + 4 of tile lane % 16; the tiles of a quad are exchanged by the quad's number, which
+  // lets the lanes of a tile read from different banks.
+  constexpr int LEFT = 2 * KB * 1024;           // bytes of a wavefront
+  unsigned char* const leave = lds + 2 * BUF + wave * LEFT + (lane >> 4) * 256;
+  const unsigned char* const take =
+      lds + 2 * BUF + quad / 4 / KB * 4 * LEFT + quad / 4 % KB * 2048 + ob * 1024 + quad % 4 * 256 + ((my_tile ^ quad) & 15) * 16;
+  auto finish = [&](bool live, int blk) {
+    floatx4 z[4], out[2][1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) z[i] = *reinterpret_cast<const floatx4*>(take + i * LEFT);
+    out[0][0] = z[0] + z[1] + z[2];
+    out[1][0] = z[1] - (z[2] + z[3]);
+    asm volatile("" : "+v"(out[0][0]), "+v"(out[1][0]));       // read before the barrier that comes
+    const int p = max(blk, 0) * kThinTiles + my_tile;
+    store_tile<T, KW, 1>(a, ydesc, p, ko, live & (p < a.P) & (ko < a.K), bv, out, ob);
+  };
+
+  // of a fragment of the first channel step; that of step s lies 4 s chunks on, which the permutation makes an exclusive or
+  int vrow = (lane & 15) * PITCH + row * 4 * ELEM + (((lane >> 4) ^ (lane & 15)) << 4);
+
+  // A block: the products M[i][j] = U[i][j] V[i][j] over the channels, and the width half of the output transform,
+  // zw[i][0] = M[i][0] + M[i][1] + M[i][2], zw[i][1] = M[i][1] - M[i][2] - M[i][3].  16-bit types do the sums in
+  // the accumulators (z0 takes j = 0, 1, 2; zp takes j = 1 and zn j = 2, 3, so that no operand needs its sign
+  // changed): 24 MFMAs per channel step instead of 16, 12 accumulators instead of 16, no VALU work - their
+  // MFMAs are cheap and registers are what is short.  fp32, whose MFMAs are sixteen times slower and bound the
+  // kernel, keeps one accumulator per element and adds in VALU.  Consecutive MFMAs write different accumulators.
+  //
+  // The products are a stream of items, one step of channels of one element each.  The transform of the
+  // next block, its way to LDS and the loads of the block after are dealt out over the items (MORE: there is a next block).
+  auto block = [&](auto more_, int it) {
+    constexpr bool MORE = decltype(more_)::value != 0;
+    constexpr int NI = KS * 4, VD = 3, FROM = std::is_same<T, bf16_t>::value ? NI * 5 / 8 : NI / 4, MEET = 2;
+    const int cur = (it & 1) * BUF, next = BUF - cur;
+    asm volatile("" : "+v"(vrow));                // addresses are worked out again: registers are short
+    floatx4 acc[PLAIN ? 4 : 3][KB];          // PLAIN: M; else z0, zp, zn
+#pragma unroll
+    for (int j = 0; j < (PLAIN ? 4 : 3); ++j)
+#pragma unroll
+      for (int k = 0; k < KB; ++k) acc[j][k] = floatx4{0.f, 0.f, 0.f, 0.f};
+    Frag vf[VD];
+    auto load_v = [&](int item) { vf[item % VD] = *reinterpret_cast<const Frag*>(lds + ((vrow ^ (item / 4 * 64)) + cur) + item % 4 * ELEM); };
+#pragma unroll
+    for (int i = 0; i < VD - 1; ++i) load_v(i);
+    static_for<0, NI>([&](auto item_) {
+      constexpr int item = decltype(item_)::value, s = item / 4, j = item % 4;
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (item + VD - 1 < NI) load_v(item + VD - 1);
+#pragma unroll
+      for (int k = 0; k < KB; ++k) {
+        if constexpr (PLAIN) acc[j][k] = MF::run(u[j * KB + k][s], vf[item % VD], acc[j][k]);
+        else if constexpr (j <= 2) acc[0][k] = MF::run(u[j * KB + k][s], vf[item % VD], acc[0][k]);
+      }
+#pragma unroll
+      for (int k = 0; k < KB; ++k)
+        if constexpr (!PLAIN && j >= 1) acc[j == 1 ? 1 : 2][k] = MF::run(u[j * KB + k][s], vf[item % VD], acc[j == 1 ? 1 : 2][k]);
+      if constexpr (item == MEET - 1) finish(it > 0, blk - nwg);
+      if constexpr (item == MEET) __builtin_amdgcn_s_barrier();             // all have read what the last block left: its place may be written
+      if constexpr (MORE) {
+        constexpr auto first = [](int i) { return i <= FROM ? 0 : (i - FROM) * UNITS / (NI - FROM); };
+        static_assert(first(MEET) <= UNITS - 4, "written behind the barrier");
+        static_for<first(item), first(item + 1)>([&](auto u_) {
+          constexpr int unit = decltype(u_)::value;
+          if constexpr (unit == UNITS - 4) find_window(blk + 2 * nwg);
+          transform_unit(u_);
+          if constexpr (unit >= UNITS - 4) {
+#pragma unroll
+            for (int e = unit % 4; e < 16; e += 4) {
+              store_element(e, next);
+              load_element(e);
+            }
+          }
+        });
+      }
+    });
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < KB; ++k) {
+      floatx4 zw[2] = {acc[0][k], acc[1][k] - acc[2][k]};
+      if constexpr (PLAIN) {
+        zw[0] = acc[0][k] + acc[1][k] + acc[2][k];
+        zw[1] -= acc[3][k];
+      }
+      const int quad_left = (wave >> 2) * 4 * KB + 4 * k + (lane >> 4);
+#pragma unroll
+      for (int b = 0; b < 2; ++b) *reinterpret_cast<floatx4*>(leave + (2 * k + b) * 1024 + ((lane ^ quad_left) & 15) * 16) = zw[b];
+    }
+    meet();
+  };
+
+  if (blk >= a.n_blocks) return;
+  static_for<0, UNITS>([&](auto u_) { transform_unit(u_); });
+#pragma unroll
+  for (int e = 0; e < 16; ++e) store_element(e, 0);
+  if (blk + nwg < a.n_blocks) load_window(blk + nwg);
+  meet();
+  int it = 0;
+  for (; blk + nwg < a.n_blocks; blk += nwg, ++it) block(ic<1>{}, it);
+  block(ic<0>{}, it);
+  finish(true, blk);
 }
 
 // The same for at most 4 input channels (first layers: grey or RGB images), any storage type.  Padding 3
@@ -515,11 +803,10 @@ __global__ __launch_bounds__(256) void tiny_conv3x3_kernel(ThinArgs a) {
   for (int it = 0; blk < a.n_blocks; blk += nwg, ++it) {
     float* buf = ldsf + (it & 1) * BUF;
     {
-      float d[16], t2[16];
+      float d[16];
 #pragma unroll
       for (int e = 0; e < 16; ++e) d[e] = static_cast<float>(raw[e].v[0]);
-      bt23<1, 4>(d, t2);
-      bt23<4, 1>(t2, d);
+      transform(d);
 #pragma unroll
       for (int e = 0; e < 16; ++e) buf[(e * TILES + pl) * 4 + c] = d[e];
     }
@@ -557,7 +844,7 @@ __global__ __launch_bounds__(256) void tiny_conv3x3_kernel(ThinArgs a) {
       }
       const int p = blk * TILES + cb * 16 + (lane & 15);
       const int ko = kbase + 4 * (lane >> 4);
-      store_tile<T, KW>(a, ydesc, p, ko, p < a.P && ko < a.K, bv, out);
+      store_tile<T, KW, 2>(a, ydesc, p, ko, p < a.P && ko < a.K, bv, out);
     }
   }
 }
@@ -580,26 +867,25 @@ int launch_tiny(ThinArgs a, int k_groups, void* stream) {
 
 template <typename T, int CP, int KSUB>
 int launch_thin_groups(ThinArgs a, void* stream) {
-  constexpr bool split = CP * sizeof(T) > 128;
-  constexpr int lds = 2 * 16 * kThinTiles * CP * (int)sizeof(T) + (split ? KSUB * 4 * 64 * 16 : 0);
+  constexpr int lds = kThinLds<T, CP, KSUB>, threads = kThinThreads<T, CP, KSUB>;
   const int k_groups = ceil_div(a.K, 16 * KSUB);
-  // workgroups that stay resident (registers and LDS): two per CU, one of the eight-wavefront form;
+  // workgroups that stay resident (registers and LDS): two per CU, one of thin_rows_kernel;
   // shared among the groups of output channels, in whole multiples of the 8 XCDs
-  int wgs = std::min(a.n_blocks, std::max(kXcds, (split ? 256 : 512) / k_groups / kXcds * kXcds));
+  int wgs = std::min(a.n_blocks, std::max(kXcds, (kThinRows<T, CP> ? 256 : 512) / k_groups / kXcds * kXcds));
   a.per_xcd = ceil_div(wgs, kXcds);
-  auto fn = a.k_whole ? &thin_conv3x3_kernel<T, CP, true, KSUB> : &thin_conv3x3_kernel<T, CP, false, KSUB>;
+  void (*fn)(ThinArgs);
+  if constexpr (kThinRows<T, CP>) fn = a.k_whole ? &thin_rows_kernel<T, CP, true, KSUB> : &thin_rows_kernel<T, CP, false, KSUB>;
+  else fn = a.k_whole ? &thin_conv3x3_kernel<T, CP, true, KSUB> : &thin_conv3x3_kernel<T, CP, false, KSUB>;
   if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)) return rc;
-  hipLaunchKernelGGL(fn, dim3((unsigned)(a.per_xcd * kXcds), (unsigned)k_groups),
-                     dim3((split ? 128 : 64) * KSUB), lds, as_stream(stream), a);
+  hipLaunchKernelGGL(fn, dim3((unsigned)(a.per_xcd * kXcds), (unsigned)k_groups), dim3(threads), lds, as_stream(stream), a);
   WC_CHECK_LAUNCH("thin_conv3x3_kernel");
   return WC_OK;
 }
 
 template <typename T, int CP>
 int launch_thin(ThinArgs a, void* stream) {
-  // half-size workgroups while the full-size ones would fill at most half of the CUs (their threads transform
-  // twice the channels each, and a thread's channels must be all inside C or all outside)
-  constexpr int vec2 = kThinTiles * CP / ((CP * sizeof(T) > 128 ? 128 : 64) * 2);
+  // half-size workgroups while the full-size ones would fill at most half of the CUs (a thread's channels must be all inside C or all outside)
+  constexpr int vec2 = kThinTiles * CP / kThinThreads<T, CP, 2>;
   const int forced = test_gemm_config();            // wc_test_gemm_override: 8 = full size, 9 = half size
   const bool half = forced == 9 || (forced != 8 && (long long)a.n_blocks * ceil_div(a.K, kThinK) * 2 <= kCus);
   if (half && a.C % vec2 == 0) return launch_thin_groups<T, CP, 2>(a, stream);
