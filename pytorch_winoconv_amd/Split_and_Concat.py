@@ -9,12 +9,16 @@ import ctypes
 
 import torch
 
-from . import _lib
+from . import _lib, engine
 from .engine import _ptr, _stream, _require_gpu, channel_last, channel_last_memory, channel_first_view
 
 
 def wino_split(a, w_shape, output_block_size):
     """a (B, C, [D,] H, W) -> tiles (B*[nD*]nH*nW, C, [bD,] bH, bW), b = w + m - 1."""
+    if engine.USE_EXT:
+        out = engine._ext.wino_split(a, w_shape, output_block_size)
+        if out is not None:
+            return out
     _require_gpu(a)
     lib = _lib.load()
     m = int(output_block_size)
@@ -46,6 +50,10 @@ def wino_split(a, w_shape, output_block_size):
 
 def wino_concat(a, output_size, output_block_size):
     """a (B*[nD*]nH*nW, K, [m,] m, m) -> (B, K, [oD,] oH, oW) with partial edge tiles cropped."""
+    if engine.USE_EXT:
+        out = engine._ext.wino_concat(a, output_size, output_block_size)
+        if out is not None:
+            return out
     _require_gpu(a)
     lib = _lib.load()
     m = int(output_block_size)

@@ -783,6 +783,119 @@ class KeptFilter {
   mutable std::vector<void*> ordered_;              // streams that have waited
 };
 
+// a tensor with memory of its own on the GPU: no wrapper of a function transform, no subclass, nothing that carries a tangent
+bool plain(const at::Tensor& t) {
+  constexpr c10::DispatchKeySet wrapped({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                         c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor});
+  return t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(wrapped) && !t._fw_grad(0).defined();
+}
+
+// Split_and_Concat.py's two functions for the arguments that they are called with in earnest (tensors of the GPU, sequences of ints); None for
+// anything else, for what they refuse and for what the library does, which they then find and say themselves.  Through ctypes a call of
+// each took 22 to 23 us of host time together, which is what all but the largest images waited for; here 9.5 to 10.3, two launches.
+std::optional<std::vector<int64_t>> whole_numbers(py::handle h, size_t count) {
+  const bool tuple = PyTuple_Check(h.ptr());
+  if ((!tuple && !PyList_Check(h.ptr())) || (size_t)(tuple ? PyTuple_GET_SIZE(h.ptr()) : PyList_GET_SIZE(h.ptr())) != count) return std::nullopt;
+  std::vector<int64_t> v(count);
+  for (size_t i = 0; i < count; ++i) {
+    PyObject* const o = tuple ? PyTuple_GET_ITEM(h.ptr(), i) : PyList_GET_ITEM(h.ptr(), i);
+    if (!PyLong_CheckExact(o)) return std::nullopt;
+    int over = 0;
+    v[i] = PyLong_AsLongLongAndOverflow(o, &over);
+    if (over || v[i] < 1 || v[i] >= (1 << 30)) return std::nullopt;
+  }
+  return v;
+}
+
+// a tensor of the kernels' types with memory of its own on the GPU, its extents ints
+const at::Tensor* tile_tensor(py::handle h) {
+  if (!THPVariable_Check(h.ptr())) return nullptr;
+  const at::Tensor& t = THPVariable_Unpack(h.ptr());
+  const auto type = t.scalar_type();
+  if (!plain(t) || (type != at::kFloat && type != at::kHalf && type != at::kBFloat16) || torch::jit::tracer::isTracing()) return nullptr;
+  for (const int64_t v : t.sizes())
+    if (v < 1 || v >= (1 << 30)) return nullptr;
+  return &t;
+}
+
+std::optional<int> tile_extent(py::handle h) {
+  if (!PyLong_CheckExact(h.ptr())) return std::nullopt;
+  int over = 0;
+  const int64_t m = PyLong_AsLongLongAndOverflow(h.ptr(), &over);
+  return over || m < 1 || m > 1024 ? std::nullopt : std::optional<int>((int)m);
+}
+
+py::object wino_split(py::handle a_, py::handle w_shape, py::handle m_) {
+  const at::Tensor* const a = tile_tensor(a_);
+  const auto m = tile_extent(m_);
+  if (!a || !m) return py::none();
+  const int nd = (int)a->dim() - 2;
+  if (nd != 2 && nd != 3) return py::none();
+  const auto w = whole_numbers(w_shape, nd + 2);
+  if (!w) return py::none();
+  int sp[3] = {1, 1, 1}, block[3] = {1, 1, 1}, n[3] = {1, 1, 1};
+  int64_t tiles = a->size(0);
+  std::vector<int64_t> shape{0, a->size(1)};
+  for (int q = 0; q < nd; ++q) {
+    const int at = 3 - nd + q;
+    sp[at] = (int)a->size(2 + q);
+    const int64_t extent = (*w)[2 + q] + *m - 1;
+    if (extent > sp[at]) return py::none();
+    block[at] = (int)extent;
+    n[at] = (sp[at] - block[at] + 1) / *m + 1;         // of a float's whole part: 1 + (X + 1 - b) / m
+    tiles *= n[at];
+    shape.push_back(extent);
+  }
+  shape[0] = tiles;
+  at::Tensor out, src;
+  int rc;
+  {
+    py::gil_scoped_release nogil;
+    const int es = (int)a->element_size(), B = (int)a->size(0), C = (int)a->size(1);
+    const bool first = a->is_contiguous() && !channel_last_memory(*a) && (es == 4 || (*m % 2 == 0 && block[2] % 2 == 0));
+    src = first ? *a : last_view(*a).contiguous();
+    out = at::empty(shape, a->options());
+    void* const stream = stream_of(*a);
+    if (first)
+      rc = wc_wino_split_channel_first(src.data_ptr(), out.data_ptr(), B, C, sp[0], sp[1], sp[2], block[0], block[1], block[2], *m, n[0], n[1], n[2], es, stream);
+    else if (nd == 2)
+      rc = wc_wino_split2d(src.data_ptr(), out.data_ptr(), B, sp[1], sp[2], C, block[1], block[2], *m, n[1], n[2], es, stream);
+    else
+      rc = wc_wino_split3d(src.data_ptr(), out.data_ptr(), B, sp[0], sp[1], sp[2], C, block[0], block[1], block[2], *m, n[0], n[1], n[2], es, stream);
+  }
+  return rc == WC_OK ? py::cast(out) : py::none();
+}
+
+py::object wino_concat(py::handle a_, py::handle size_, py::handle m_) {
+  const at::Tensor* const a = tile_tensor(a_);
+  const auto m = tile_extent(m_);
+  if (!a || !m) return py::none();
+  const int nd = (int)a->dim() - 2;
+  if (nd != 2 && nd != 3) return py::none();
+  const auto size = whole_numbers(size_, nd);
+  if (!size) return py::none();
+  int64_t per = 1;
+  for (const int64_t o : *size) per *= (o + *m - 1) / *m;
+  if (a->size(0) % per) return py::none();
+  const int64_t B = a->size(0) / per, K = a->size(1);
+  at::Tensor out;
+  int rc;
+  {
+    py::gil_scoped_release nogil;
+    const at::Tensor tiles = a->contiguous();
+    std::vector<int64_t> shape{B}, order{0, nd + 1};
+    for (int q = 0; q < nd; ++q) { shape.push_back((*size)[q]); order.push_back(1 + q); }
+    shape.push_back(K);
+    const at::Tensor last = at::empty(shape, a->options());
+    const int es = (int)a->element_size();
+    void* const stream = stream_of(*a);
+    rc = nd == 2 ? wc_wino_concat2d(tiles.data_ptr(), last.data_ptr(), (int)B, (int)shape[1], (int)shape[2], (int)K, *m, es, stream)
+                 : wc_wino_concat3d(tiles.data_ptr(), last.data_ptr(), (int)B, (int)shape[1], (int)shape[2], (int)shape[3], (int)K, *m, es, stream);
+    out = last.permute(order);
+  }
+  return rc == WC_OK ? py::cast(out) : py::none();
+}
+
 // ---- a module's forward pass ----------------------------------------------------------------------------------------
 // What WinoConv.py's modules work out anew for an input of another shape: the descriptor, the shape of the result and the
 // transformed filter.  Called with an input of the same shape, strides and type and a weight of the same kind, it runs the layer
@@ -863,12 +976,6 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
 
  private:
   static bool misaligned(const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) != 0; }
-  // a tensor with memory of its own on the GPU: no wrapper of a function transform, no subclass, nothing that carries a tangent
-  static bool plain(const at::Tensor& t) {
-    constexpr c10::DispatchKeySet wrapped({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
-                                           c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor});
-    return t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(wrapped) && !t._fw_grad(0).defined();
-  }
   bool fits(const at::Tensor& x, const at::Tensor& weight, const std::optional<at::Tensor>& bias) const {
     return plain(x) && plain(weight) && (!bias || plain(*bias)) && x.scalar_type() == x_type && x.sizes() == at::IntArrayRef(sizes) &&
            x.strides() == at::IntArrayRef(strides) && x.device() == device && !misaligned(x) && weight.scalar_type() == w_type &&
@@ -996,6 +1103,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("AddGPU", &AddGPU);
   m.def("WinoSplit", &WinoSplit);
   m.def("WinoConcat", &WinoConcat);
+  m.def("wino_split", &wino_split, py::arg("a"), py::arg("w_shape"), py::arg("output_block_size"));
+  m.def("wino_concat", &wino_concat, py::arg("a"), py::arg("output_size"), py::arg("output_block_size"));
   m.def("DWM", &DWM, py::arg("Input"), py::arg("Weight"), py::arg("Output"), py::arg("stride"),
         py::arg("tmp_input_buffer") = py::none(), py::arg("tmp_weight_buffer") = py::none(),
         py::arg("tmp_product_buffer") = py::none(), py::arg("tmp_ptr_buffer") = py::none());
