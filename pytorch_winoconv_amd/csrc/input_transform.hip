@@ -41,6 +41,9 @@ int input_transform_impl(const wc_conv_desc* d, const wc_plan* plan, const void*
   int vec = 1;
   for (int v = want; v > 1; v /= 2)
     if (d->C % v == 0) { vec = v; break; }
+  // Small 2-D plans of several pieces, which get threads of their own below: fewer channels a thread until every CU has a workgroup.
+  // (One piece alone was slower with them: fp32 N=2 88 -> 96, 19x24 15.5 | 15.9, N=1 512 -> 512, 7x7 29.6 | 31.6.)
+  while (plan->n_pieces > 1 && flat && !shared && vec > 1 && P * (Cp / vec) * plan->n_pieces < 256 * kCus) vec /= 2;
   InArgs a;
   a.x = x; a.V = V;
   a.D = d->in[0]; a.H = d->in[1]; a.W = d->in[2]; a.C = d->C; a.Cp = row;
@@ -83,11 +86,14 @@ int input_transform_impl(const wc_conv_desc* d, const wc_plan* plan, const void*
     small_taps = pc.r[1] >= 1 && pc.r[1] <= 3 && pc.r[2] >= 1 && pc.r[2] <= 3 && pc.tap0[1] < 16 && pc.tap0[2] < 16;
   }
   if (small_taps && plan->m[1] == plan->m[2]) {
-    // Stacked plans of small problems give every piece its own threads (one thread per tile and
+    // Small problems give every piece its own threads (one thread per tile and
     // channel group, looping over the pieces, then leaves most of the chip idle: 2.2x faster at
     // N=8, C=24, 56x56, 7x7); large ones keep the loop, which reads each window from cache once per
-    // piece and measured 7-30 % faster there.
-    const bool per_piece_threads = stacked && a.total < 512 * 1024;
+    // piece and measured 7-30 % faster there.  Stacked plans have the pieces beside the channels, others in the grid's second
+    // dimension.  fp32 without stacking, us of a layer with its filter, in a loop | apart, and both transforms with fewer channels a thread:
+    // 7x7 on tile 2 and 4, N=5 88 -> 96, 14x14 44.1 | 32.4 and 60.5 | 38.5, N=2 32 -> 64, 28x28 38.0 | 25.4 and 50.8 | 29.3, N=8 64 -> 64,
+    // 56x56 148 | 140 and 91 | 81, N=32 128 -> 128, 56x56 (too large for it) 1119 and 778; 5x5 on tile 4, N=4 480 -> 128, 21x28 64.1 | 56.4.
+    const bool apart = a.total < 512 * 1024, per_piece_threads = stacked && apart;
     InPiecesKernel fn = per_piece_threads ? pick_in_2d_stacked(d->dtype, plan->m[1], vec)
                                           : pick_in_2d_pieces(d->dtype, plan->m[1], vec);
     if (fn) {
@@ -99,6 +105,8 @@ int input_transform_impl(const wc_conv_desc* d, const wc_plan* plan, const void*
         a.per_xcd = (int)ceil_div_ll(ceil_div_ll(a.total, 256), kXcds);
         WC_CHECK_ARG((long long)a.per_xcd * kXcds < (1ll << 31), "wc_input_transform: problem too large");
         launch = dim3((unsigned)(a.per_xcd * kXcds));
+      } else if (apart) {
+        launch.y = (unsigned)plan->n_pieces;
       }
       g.o = a;
       g.n_pieces = plan->n_pieces;

@@ -9,7 +9,7 @@ __global__ __launch_bounds__(256) void input_transform_pieces_kernel(InPiecesArg
   InWhere w;
   if (!in_decode(a, xcd_remap(blockIdx.x, a.per_xcd), VEC, w)) return;
   constexpr int KA = MO == 4 ? KIND_41 : KIND_21, KB = MO == 4 ? KIND_42 : KIND_22, KC = MO == 4 ? KIND_43 : KIND_23;
-  for (int s = 0; s < g.n_pieces; ++s) {
+  for (int s = blockIdx.y; s < g.n_pieces; s += gridDim.y) {
     const int info = g.info[s];
     const int t_offset = info & 0xffff;
     const int base1 = ((info >> 16) & 15) - g.pad1, base2 = ((info >> 20) & 15) - g.pad2;

@@ -367,7 +367,10 @@ extern "C" int wc_output_transform(const wc_conv_desc* d, const wc_plan* plan_in
   WC_CHECK_ARG(plan->n_pieces > 0 && plan->n_pieces <= WC_MAX_PIECES, "wc_output_transform: bad plan");
   const int ldm = wc_padded_channels8(d->K);
   const long long P = (long long)n_images * grid[0] * grid[1] * grid[2];
-  const int vec = (d->K % 4 == 0) ? 4 : 1;
+  // Small 2-D layers: a channel a thread, so that more CUs have a workgroup.  fp32, F(4,3), us of a layer: N=28 128 -> 64, 12x12 18.9 | 18.3,
+  // N=2 88 -> 96, 19x24 15.5 | 14.8, N=4 256 -> 256, 14x14 20.9 | 20.2
+  const bool small = plan->m[0] == 1 && plan->m[1] == 4 && P * (d->K / 2) < 256 * kCus;
+  const int vec = d->K % 4 == 0 && !small ? 4 : 1;
   OutArgs a;
   a.M = M; a.bias = bias; a.y = y;
   a.oD = out[0]; a.oH = out[1]; a.oW = out[2]; a.K = d->K; a.ldm = ldm;
@@ -415,7 +418,8 @@ extern "C" int wc_output_transform(const wc_conv_desc* d, const wc_plan* plan_in
   }
   if (flat) {
     // 2-D plans: compile-time body per piece; F(4,r) tiles use 2 channels per thread
-    const int v = (tile4 && vec == 4) ? 2 : vec;
+    int v = (tile4 && vec == 4) ? 2 : vec;
+    if (P * (d->K / v) < 256 * kCus) v = 1;           // as above
     g.o.n_kvec = d->K / v;
     g.o.total = P * g.o.n_kvec;
     g.o.per_xcd = (int)ceil_div_ll(ceil_div_ll(g.o.total, 256), kXcds);
