@@ -33,6 +33,8 @@ struct GradOutArgs {
   int m[3];
   int n_pieces;
   long long total;           // T * P * ldm
+  int blocks;                // grad_output_pieces_kernel: workgroups of dM, behind them those of the bias gradient's sums over rows of dy
+  RowSums bias;
   wc_piece piece[WC_MAX_PIECES];
 };
 
@@ -99,6 +101,12 @@ struct MatA {
 // M0 x MO x MO is the output tile: 1 x 2 x 2, 1 x 4 x 4, 2 x 2 x 2 or 2 x 4 x 4.
 template <typename T, int M0, int MO, int VEC>
 __global__ __launch_bounds__(256) void grad_output_pieces_kernel(const GradOutArgs a) {
+  __shared__ float sums[256 * (16 / sizeof(T) + 1)];
+  if ((int)blockIdx.x >= a.blocks) {
+    const int b = blockIdx.x - a.blocks, tile = b / a.bias.blocks;
+    sum_rows_any<T>(a.bias, b - tile * a.bias.blocks, tile, sums);
+    return;
+  }
   const int n_kvec = a.ldm / VEC;
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
   if (idx >= a.P * n_kvec) return;
@@ -485,7 +493,19 @@ int backward_weight(const wc_conv_desc* d, const void* x, const void* dy, GradOu
                       d->pad[2], L.out[1], L.out[2], L.S, L.Pq, d->dtype, stream, to.db_part, &summed);
     if (rc) return rc;
   }
-  if (to.db && !summed && (rc = bias_alone())) return rc;
+  auto small_taps = [](const wc_plan& plan) {
+    bool small = true;
+    for (int i = 0; i < plan.n_pieces; ++i)
+      for (int q = 0; q < 3; ++q) small = small && plan.piece[i].r[q] <= 3;
+    return small;
+  };
+  // In the transform domain the bias gradient's two steps ride on the launches that read dy and that write dw, which writes it from the last
+  // chunk's sums: three launches fewer, whose host time most training steps in fp32 wait for.  us of a step, apart | so, fp32: N=28 128 -> 64, 12x12 97 | 89,
+  // N=2 96 -> 416, 44x44 127 | 120, N=1 32 -> 32, 14x14 80 | 74, stride 2, N=4 76 -> 64, 70x58 127 | 117, N=2 64 -> 49, 12x37x37 279 | 252.
+  const bool stores = !L.one_tap && !L.gathered && grad_filter_stores(d, &L.plan);
+  const bool beside = stores && to.db && small_taps(L.dm_plan);
+  const RowSums rows = beside ? row_sums_of(dy, to.db_part, dy_rows(d, L.out), d->K, d->dtype) : RowSums{};
+  if (to.db && !summed && !beside && (rc = bias_alone())) return rc;
   if (L.one_tap || L.gathered) {
     const long long n = (long long)d->K * d->C, total4 = (long long)taps * n / 4;
     dispatch_dtype(d->dtype, [&](auto t) {
@@ -519,13 +539,10 @@ int backward_weight(const wc_conv_desc* d, const void* x, const void* dy, GradOu
       a.total = (long long)T * P * L.ldm;
       const long long blocks = ceil_div_ll(a.total, 256);
       WC_CHECK_ARG(blocks < (1ll << 31), "wc_conv_backward_weight: problem too large");
-      bool small_taps = true;
-      for (int i = 0; i < gp.n_pieces; ++i)
-        for (int q = 0; q < 3; ++q) small_taps = small_taps && gp.piece[i].r[q] <= 3;
       const int m0 = L.plan.m[0], mo = L.plan.m[1];
       void (*fn)(GradOutArgs) = nullptr;
       long long threads = a.total;
-      if (small_taps && L.plan.m[2] == mo && (mo == 2 || mo == 4) && (m0 == 1 || m0 == 2)) {
+      if (small_taps(gp) && L.plan.m[2] == mo && (mo == 2 || mo == 4) && (m0 == 1 || m0 == 2)) {
         // 2 channels per thread when K is even, except for the 144-element tile of the 3-D tile 4
         const int vec = ((m0 == 2 && mo == 4) || d->K % 2) ? 1 : 2;
         threads = P * (L.ldm / vec);
@@ -544,8 +561,10 @@ int backward_weight(const wc_conv_desc* d, const void* x, const void* dy, GradOu
           return &grad_output_transform_kernel<decltype(t)>;
         });
       }
-      const long long nblocks = ceil_div_ll(threads, 256);
-      hipLaunchKernelGGL(fn, dim3((unsigned)nblocks), dim3(256), 0, s, a);
+      a.blocks = (int)ceil_div_ll(threads, 256);
+      a.bias = rows;
+      const int more = beside && b0 == 0 ? rows.blocks * rows.col_tiles : 0;
+      hipLaunchKernelGGL(fn, dim3((unsigned)(a.blocks + more)), dim3(256), 0, s, a);
       WC_CHECK_LAUNCH("grad_output_transform_kernel");
     }
     // the part length of this pass (the last pass may hold fewer images)
@@ -563,9 +582,11 @@ int backward_weight(const wc_conv_desc* d, const void* x, const void* dy, GradOu
       hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)ceil_div_ll(total4, 256)), dim3(256), 0, s, dU, L.S, n, total4);
       WC_CHECK_LAUNCH("sum_parts_kernel");
     }
-    rc = grad_filter_transform(d, &L.plan, dU, acc, L.ldc, L.S, b0 == 0, stream);
+    const bool last = b0 + L.chunk >= d->N;
+    rc = grad_filter_transform(d, &L.plan, dU, acc, L.ldc, L.S, b0 == 0, last && stores ? &to : nullptr, beside ? rows.blocks : 0, stream);
     if (rc) return rc;
   }
+  if (stores) return WC_OK;
   const long long total = (long long)taps * d->K * d->C;
   dispatch_dtype(d->dtype, [&](auto t) {
     using TT = decltype(t);

@@ -2,6 +2,7 @@
 // chunks into acc (taps, K, C) in fp32.  dU (T, S, K, ldc) holds, in part 0 of every transform
 // element, the sum over the tiles.  No counterpart in the reference (its backward pass was never
 // written: src/back/utils.cu:15-24); the adjoint of the filter transform of filter_transform.hip.
+#include "column_sums.h"
 #include "wc_transform.h"
 
 namespace wc {
@@ -26,6 +27,11 @@ struct GradFilterArgs {
   int rp[3];
   int first;                 // 1: overwrite acc, 0: add to it
   long long total;           // taps * K * C
+  // the last chunk of images (grad_filter_pieces_kernel): dw, through element strides, takes the place of acc
+  void* dw;
+  long long s[5];
+  int f32, blocks;           // dw is fp32 whatever T; workgroups of the filter, behind them the bias gradient's
+  ColumnSums bias;
   wc_piece piece[WC_MAX_PIECES];
 };
 
@@ -85,11 +91,17 @@ struct MatGT {
 
 // One (k, c) of one piece with compile-time kinds: loads the piece's alpha^d sums once (lanes
 // along c: coalesced), applies G^T along each axis in registers and adds the result to the
-// piece's taps.
-template <int K0, int K1, int K2>
-__device__ __forceinline__ void grad_taps(const float* __restrict__ src, long long t_stride, float* __restrict__ acc,
-                                          long long plane, const int (&tap0)[3], int step, int kH, int kW, bool first,
-                                          const int (&taps)[3]) {
+// piece's taps; in the last chunk of images what they add up to goes to dw.
+struct TapsOut {
+  float* acc;                // of (k, c) and the piece's first tap
+  void* dw;                  // null: not the last chunk
+  long long dst;             // its element of that tap
+  long long acc_step[3], dw_step[3];     // from tap to tap
+  int n[3];                  // the piece's taps
+  bool first, f32;
+};
+template <typename T, int K0, int K1, int K2>
+__device__ __forceinline__ void grad_taps(const float* __restrict__ src, long long t_stride, const TapsOut to) {
   constexpr int R0 = Mats<K0>::r, R1 = Mats<K1>::r, R2 = Mats<K2>::r;
   constexpr int A0 = Mats<K0>::alpha, A1 = Mats<K1>::alpha, A2 = Mats<K2>::alpha;
   float u[A0 * A1 * A2][1];
@@ -103,39 +115,48 @@ __device__ __forceinline__ void grad_taps(const float* __restrict__ src, long lo
   apply_axis<MatGT<K1>, 1, A0, A1, R2, 1>(g2, g1);
   float g0[R0 * R1 * R2][1];
   apply_axis<MatGT<K0>, 0, A0, R1, R2, 1>(g1, g0);
-  static_for<0, R0>([&](auto j0_) {
-    static_for<0, R1>([&](auto j1_) {
-      static_for<0, R2>([&](auto j2_) {
-        constexpr int j0 = decltype(j0_)::value, j1 = decltype(j1_)::value, j2 = decltype(j2_)::value;
+#pragma unroll
+  for (int j0 = 0; j0 < R0; ++j0)
+#pragma unroll
+    for (int j1 = 0; j1 < R1; ++j1)
+#pragma unroll
+      for (int j2 = 0; j2 < R2; ++j2) {
         // (a stacked plan transforms with the tile of the longest piece: taps this piece lacks are dropped)
-        if (j0 < taps[0] && j1 < taps[1] && j2 < taps[2]) {
-          const int tap = ((tap0[0] + j0 * step) * kH + tap0[1] + j1 * step) * kW + tap0[2] + j2 * step;
-          float* dst = acc + tap * plane;
-          const float v = g0[(j0 * R1 + j1) * R2 + j2][0];
-          *dst = first ? v : *dst + v;
+        if (j0 < to.n[0] && j1 < to.n[1] && j2 < to.n[2]) {
+          float* const sum = to.acc + j0 * to.acc_step[0] + j1 * to.acc_step[1] + j2 * to.acc_step[2];
+          float v = g0[(j0 * R1 + j1) * R2 + j2][0];
+          if (!to.first) v = *sum + v;
+          if (to.dw) store_as<T>(to.dw, to.dst + j0 * to.dw_step[0] + j1 * to.dw_step[1] + j2 * to.dw_step[2], v, to.f32);
+          else *sum = v;
         }
-      });
-    });
-  });
+      }
 }
 
 // The same transform for plans whose pieces have 1..3 taps per axis (every DWM plan): blockIdx.y is
 // the piece, one thread per (k, c); the piece's taps select a compile-time body (uniform over the
 // workgroup).  M0 x MO x MO is the output tile: 1 x 2 x 2, 1 x 4 x 4, 2 x 2 x 2 or 2 x 4 x 4.
-template <int M0, int MO>
+// It writes dw itself and takes the last step of the bias gradient along, which were a launch each; what it needs of
+// its piece is read by value (by reference the kernel's arguments went to scratch memory: 3-D fp32, 64 -> 49 channels, 24.8 us | 7.7).
+template <typename T, int M0, int MO>
 __global__ __launch_bounds__(256) void grad_filter_pieces_kernel(const GradFilterArgs a) {
+  __shared__ float sums[256];
+  if ((int)blockIdx.x >= a.blocks) {
+    if (blockIdx.y == 0) sum_columns_halves<T>(a.bias, blockIdx.x - a.blocks, sums);
+    return;
+  }
   const int idx = blockIdx.x * 256 + threadIdx.x;
   if (idx >= a.K * a.C) return;
-  const wc_piece& pc = a.piece[blockIdx.y];
-  const int c = idx % a.C, k = idx / a.C;
-  const long long t_stride = (long long)a.S * a.K * a.ldc;
-  const float* src = a.dU + pc.t_offset * t_stride + (long long)k * a.ldc + (a.stacked ? (int)blockIdx.y * a.Cp : 0) + c;
-  const int r0 = a.stacked ? a.rp[0] : pc.r[0], r1 = a.stacked ? a.rp[1] : pc.r[1], r2 = a.stacked ? a.rp[2] : pc.r[2];
-  float* acc = a.acc + idx;
-  const long long plane = (long long)a.K * a.C;
-  const bool first = a.first != 0;
+  const int c = idx % a.C, k = idx / a.C, s = blockIdx.y;
+  const int n0 = a.piece[s].r[0], n1 = a.piece[s].r[1], n2 = a.piece[s].r[2];
+  const int x0 = a.piece[s].tap0[0], x1 = a.piece[s].tap0[1], x2 = a.piece[s].tap0[2];
+  const int step = a.step, kH = a.kernel[1], kW = a.kernel[2];
+  const long long plane = (long long)a.K * a.C, t_stride = (long long)a.S * a.K * a.ldc;
+  const float* src = a.dU + a.piece[s].t_offset * t_stride + (long long)k * a.ldc + (a.stacked ? s * a.Cp : 0) + c;
+  const TapsOut to = {a.acc + ((x0 * kH + x1) * kW + x2) * plane + idx, a.dw, k * a.s[0] + c * a.s[1] + x0 * a.s[2] + x1 * a.s[3] + x2 * a.s[4],
+                      {step * kH * kW * plane, step * kW * plane, step * plane}, {step * a.s[2], step * a.s[3], step * a.s[4]}, {n0, n1, n2}, a.first != 0, a.f32 != 0};
+  const int r0 = a.stacked ? a.rp[0] : n0, r1 = a.stacked ? a.rp[1] : n1, r2 = a.stacked ? a.rp[2] : n2;
   constexpr int KA = MO == 4 ? KIND_41 : KIND_21, KB = MO == 4 ? KIND_42 : KIND_22, KC = MO == 4 ? KIND_43 : KIND_23;
-#define WC_BODY(K0, K1, K2) grad_taps<K0, K1, K2>(src, t_stride, acc, plane, pc.tap0, a.step, a.kernel[1], a.kernel[2], first, pc.r)
+#define WC_BODY(K0, K1, K2) grad_taps<T, K0, K1, K2>(src, t_stride, to)
 #define WC_ROW(K0, K1) \
   switch (r2) { case 1: WC_BODY(K0, K1, KA); break; case 2: WC_BODY(K0, K1, KB); break; default: WC_BODY(K0, K1, KC); }
 #define WC_PLANE(K0) \
@@ -152,8 +173,16 @@ __global__ __launch_bounds__(256) void grad_filter_pieces_kernel(const GradFilte
 
 }  // namespace
 
+bool grad_filter_stores(const wc_conv_desc* d, const wc_plan* plan) {
+  const int m0 = plan->m[0], mo = plan->m[1];
+  bool small_taps = true;
+  for (int i = 0; i < plan->n_pieces; ++i)
+    for (int q = 0; q < 3; ++q) small_taps = small_taps && plan->piece[i].r[q] <= 3;
+  return small_taps && plan->m[2] == mo && (mo == 2 || mo == 4) && (m0 == 1 || m0 == 2) && (long long)d->K * d->C < (1ll << 31);
+}
+
 int grad_filter_transform(const wc_conv_desc* d, const wc_plan* plan, const float* dU, float* acc, int ldc, int S,
-                          bool first, void* stream) {
+                          bool first, const GradOut* to, int bias_rows, void* stream) {
   hipStream_t s = as_stream(stream);
   GradFilterArgs g;
   g.dU = dU; g.acc = acc;
@@ -168,14 +197,19 @@ int grad_filter_transform(const wc_conv_desc* d, const wc_plan* plan, const floa
   stacked_taps(plan, g.rp);
   g.total = (long long)d->kernel[0] * d->kernel[1] * d->kernel[2] * d->K * d->C;
   const int m0 = plan->m[0], mo = plan->m[1];
-  bool small_taps = true;
-  for (int i = 0; i < plan->n_pieces; ++i)
-    for (int q = 0; q < 3; ++q) small_taps = small_taps && plan->piece[i].r[q] <= 3;
-  if (small_taps && plan->m[2] == mo && (mo == 2 || mo == 4) && (m0 == 1 || m0 == 2) &&
-      (long long)d->K * d->C < (1ll << 31)) {
-    void (*fn)(GradFilterArgs) = m0 == 1 ? (mo == 4 ? &grad_filter_pieces_kernel<1, 4> : &grad_filter_pieces_kernel<1, 2>)
-                                         : (mo == 4 ? &grad_filter_pieces_kernel<2, 4> : &grad_filter_pieces_kernel<2, 2>);
-    const dim3 grid((unsigned)ceil_div_ll((long long)d->K * d->C, 256), (unsigned)plan->n_pieces);
+  if (grad_filter_stores(d, plan)) {
+    g.dw = to ? to->dw : nullptr;
+    for (int i = 0; i < 5; ++i) g.s[i] = to ? to->s[i] : 0;
+    g.f32 = to && to->dw_f32;
+    g.blocks = (int)ceil_div_ll((long long)d->K * d->C, 256);
+    g.bias = {};
+    if (to && bias_rows) g.bias = {to->db_part, to->db, bias_rows, d->K, d->K, to->db_f32};
+    const dim3 grid((unsigned)(g.blocks + (g.bias.part ? ceil_div(d->K, 16) : 0)), (unsigned)plan->n_pieces);
+    void (*fn)(GradFilterArgs) = dispatch_dtype(d->dtype, [&](auto t) -> void (*)(GradFilterArgs) {
+      using T = decltype(t);
+      return m0 == 1 ? (mo == 4 ? &grad_filter_pieces_kernel<T, 1, 4> : &grad_filter_pieces_kernel<T, 1, 2>)
+                     : (mo == 4 ? &grad_filter_pieces_kernel<T, 2, 4> : &grad_filter_pieces_kernel<T, 2, 2>);
+    });
     hipLaunchKernelGGL(fn, grid, dim3(256), 0, s, g);
   } else {
     if (g.stacked) return fail(WC_ERR_UNSUPPORTED, "stacked weight gradient needs a 2-D plan with output tile 2 or 4");

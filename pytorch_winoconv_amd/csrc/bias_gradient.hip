@@ -36,45 +36,9 @@ BiasPlan bias_plan(long long P, int K, int dtype, bool aligned) {
 }
 
 template <typename T, int VEC>
-__global__ __launch_bounds__(kBiasThreads) void bias_rows_kernel(const T* __restrict__ dy, float* __restrict__ part, long long P, int K,
-                                                                 int cols, int groups, long long rows_per_block) {
-  __shared__ float sums[kBiasThreads][VEC + (VEC > 1)];
-  const int group = threadIdx.x / cols, col = threadIdx.x - group * cols;
-  const int k = (blockIdx.y * cols + col) * VEC;
-  const long long begin = blockIdx.x * rows_per_block, end = min(P, begin + rows_per_block);
-  float s[VEC];
-#pragma unroll
-  for (int e = 0; e < VEC; ++e) s[e] = 0.f;
-  if (group < groups && k < K) {
-    const T* p = dy + (begin + group) * K + k;
-    const long long step = (long long)groups * K;
-    long long r = begin + group;
-    for (; r + 3 * groups < end; r += 4 * groups, p += 4 * step) {
-      Pack<T, VEC> v[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const Pack<T, VEC>*>(p + i * step);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) s[e] += static_cast<float>(v[i].v[e]);
-    }
-    for (; r < end; r += groups, p += step) {
-      const Pack<T, VEC> v = *reinterpret_cast<const Pack<T, VEC>*>(p);
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) s[e] += static_cast<float>(v.v[e]);
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < VEC; ++e) sums[threadIdx.x][e] = s[e];
-  __syncthreads();
-  for (int i = threadIdx.x; i < cols * VEC; i += kBiasThreads) {
-    const int c = i / VEC, e = i - c * VEC;
-    const int kk = (blockIdx.y * cols + c) * VEC + e;
-    if (kk >= K) continue;
-    float t = 0.f;
-    for (int g = 0; g < groups; ++g) t += sums[g * cols + c][e];
-    part[(long long)blockIdx.x * K + kk] = t;
-  }
+__global__ __launch_bounds__(kBiasThreads) void bias_rows_kernel(RowSums a) {
+  __shared__ float sums[kBiasThreads * (VEC + (VEC > 1))];
+  sum_rows<T, VEC>(a, blockIdx.x, blockIdx.y, sums);
 }
 
 // db[k] = sum over the workgroups' rows; 16 channels a workgroup, 64 threads to a channel's sums
@@ -103,18 +67,22 @@ size_t bias_part_bytes(long long rows, int K, int dtype) {
   return (size_t)std::max(bias_plan(rows, K, dtype, true).blocks, bias_plan(rows, K, dtype, false).blocks) * K * 4;
 }
 
-int bias_sums(const void* dy, void* db, long long rows, int K, int dtype, bool f32, float* part, void* stream) {
+RowSums row_sums_of(const void* dy, float* part, long long rows, int K, int dtype) {
   const BiasPlan p = bias_plan(rows, K, dtype, (reinterpret_cast<uintptr_t>(dy) & 15) == 0);
+  return {dy, part, rows, p.rows_per_block, K, p.vec, p.cols, p.groups, p.blocks, p.col_tiles};
+}
+
+int bias_sums(const void* dy, void* db, long long rows, int K, int dtype, bool f32, float* part, void* stream) {
+  const RowSums a = row_sums_of(dy, part, rows, K, dtype);
   return dispatch_dtype(dtype, [&](auto t) -> int {
     using T = decltype(t);
     constexpr int FULL = 16 / sizeof(T);
-    auto fn = p.vec == FULL ? &bias_rows_kernel<T, FULL> : p.vec == 4 ? &bias_rows_kernel<T, 4> : p.vec == 2 ? &bias_rows_kernel<T, 2>
+    auto fn = a.vec == FULL ? &bias_rows_kernel<T, FULL> : a.vec == 4 ? &bias_rows_kernel<T, 4> : a.vec == 2 ? &bias_rows_kernel<T, 2>
                                                                                              : &bias_rows_kernel<T, 1>;
-    hipLaunchKernelGGL(fn, dim3((unsigned)p.blocks, (unsigned)p.col_tiles), dim3(kBiasThreads), 0, as_stream(stream),
-                       static_cast<const T*>(dy), part, rows, K, p.cols, p.groups, p.rows_per_block);
+    hipLaunchKernelGGL(fn, dim3((unsigned)a.blocks, (unsigned)a.col_tiles), dim3(kBiasThreads), 0, as_stream(stream), a);
     WC_CHECK_LAUNCH("bias_rows_kernel");
     hipLaunchKernelGGL(bias_parts_kernel<T>, dim3((unsigned)ceil_div(K, 16)), dim3(1024), 0, as_stream(stream), part,
-                       db, p.blocks, K, f32);
+                       db, a.blocks, K, f32);
     WC_CHECK_LAUNCH("bias_parts_kernel");
     return WC_OK;
   });

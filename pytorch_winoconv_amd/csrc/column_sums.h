@@ -78,4 +78,85 @@ __device__ __forceinline__ void sum_columns(const ColumnSums& a, int b, float* l
   store_as<T>(a.db, k, t, a.f32);
 }
 
+// The same from rows of a pass over dy of its own, in the order of bias_parts_kernel (bias_gradient.hip): 64 runs of rows, then halves
+template <typename T>
+__device__ __forceinline__ void sum_columns_halves(const ColumnSums& a, int b, float* lds) {
+  const int c = threadIdx.x & 15, group = threadIdx.x >> 4, k = b * 16 + c;
+  float t[4] = {0.f, 0.f, 0.f, 0.f};
+  if (k < a.K) {
+    for (int r = group; r < a.rows; r += 64) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (r + 16 * j < a.rows) t[j] += a.part[(long long)(r + 16 * j) * a.ld + k];
+    }
+  }
+  float s = (t[0] + t[2]) + (t[1] + t[3]);
+  for (int half = 8; half > 0; half >>= 1) {
+    lds[threadIdx.x] = s;
+    __syncthreads();
+    if (group < half) s += lds[threadIdx.x + half * 16];
+    __syncthreads();
+  }
+  if (group == 0 && k < a.K) store_as<T>(a.db, k, s, a.f32);
+}
+
+// Sums over runs of dy's rows by workgroups of 256, `blocks` runs times `col_tiles`: a thread adds `vec` columns up, `cols` of them side by side
+struct RowSums {
+  const void* dy;
+  float* part;             // (blocks, K)
+  long long rows, rows_per_block;
+  int K, vec, cols, groups, blocks, col_tiles;
+};
+RowSums row_sums_of(const void* dy, float* part, long long rows, int K, int dtype);
+
+template <typename T, int VEC>
+__device__ __forceinline__ void sum_rows(const RowSums& a, int block, int tile, float* lds) {
+  constexpr int PITCH = VEC + (VEC > 1);
+  const int group = threadIdx.x / a.cols, col = threadIdx.x - group * a.cols;
+  const int k = (tile * a.cols + col) * VEC;
+  const long long begin = block * a.rows_per_block, end = min(a.rows, begin + a.rows_per_block);
+  float s[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) s[e] = 0.f;
+  if (group < a.groups && k < a.K) {
+    const T* p = static_cast<const T*>(a.dy) + (begin + group) * a.K + k;
+    const long long step = (long long)a.groups * a.K;
+    long long r = begin + group;
+    for (; r + 3 * a.groups < end; r += 4 * a.groups, p += 4 * step) {
+      Pack<T, VEC> v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const Pack<T, VEC>*>(p + i * step);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) s[e] += static_cast<float>(v[i].v[e]);
+    }
+    for (; r < end; r += a.groups, p += step) {
+      const Pack<T, VEC> v = *reinterpret_cast<const Pack<T, VEC>*>(p);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) s[e] += static_cast<float>(v.v[e]);
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) lds[threadIdx.x * PITCH + e] = s[e];
+  __syncthreads();
+  for (int i = threadIdx.x; i < a.cols * VEC; i += 256) {
+    const int c = i / VEC, e = i - c * VEC;
+    const int kk = (tile * a.cols + c) * VEC + e;
+    if (kk >= a.K) continue;
+    float t = 0.f;
+    for (int g = 0; g < a.groups; ++g) t += lds[(g * a.cols + c) * PITCH + e];
+    a.part[(long long)block * a.K + kk] = t;
+  }
+}
+
+// whatever the width of a thread's loads; lds: 256 (16 / sizeof(T) + 1) floats
+template <typename T>
+__device__ __forceinline__ void sum_rows_any(const RowSums& a, int block, int tile, float* lds) {
+  if (sizeof(T) == 2 && a.vec == 8) sum_rows<T, 16 / sizeof(T)>(a, block, tile, lds);
+  else if (a.vec == 4) sum_rows<T, 4>(a, block, tile, lds);
+  else if (a.vec == 2) sum_rows<T, 2>(a, block, tile, lds);
+  else sum_rows<T, 1>(a, block, tile, lds);
+}
+
 }  // namespace wc

@@ -223,14 +223,10 @@ __device__ __forceinline__ int class_of_block(int blk, int n_classes, int per_xc
   return (blk + round) % n_classes;
 }
 
-// acc (taps, K, C) (+)= G^T dU G per piece of the plan; dU (T, S, K, ldc) with the parts already
-// summed into part 0; `first` overwrites acc instead of adding (backward_filter.hip).
 // wc_input_transform and wc_filter_transform of one call: one launch where a kernel holds both (single-piece 2-D
 // plans of 3x3 kernels with a dense filter), two launches otherwise
 int input_filter_transform(const wc_conv_desc* d, const wc_plan* plan, const void* x, int n_images, void* V,
                            const void* w, const int64_t w_strides[5], void* U, void* stream);
-int grad_filter_transform(const wc_conv_desc* d, const wc_plan* plan, const float* dU, float* acc, int ldc, int S,
-                          bool first, void* stream);
 
 // What a weight gradient writes: dw through element strides and, where db is not null, the bias gradient, each of the operands' type
 // or fp32.  db_part: scratch for the column sums of dy that kernels with dy in LDS take on the way (column_sums.h)
@@ -238,6 +234,14 @@ struct GradOut {
   void* dw; int64_t s[5]; bool dw_f32;
   void* db; bool db_f32; float* db_part;
 };
+
+// acc (taps, K, C) (+)= G^T dU G per piece of the plan; dU (T, S, K, ldc) with the parts already
+// summed into part 0; `first` overwrites acc instead of adding (backward_filter.hip).
+// `to` (the last chunk of images) where grad_filter_stores: dw itself is written, and the bias gradient from `bias_rows` rows of K sums in
+// to->db_part (0: none)
+bool grad_filter_stores(const wc_conv_desc* d, const wc_plan* plan);
+int grad_filter_transform(const wc_conv_desc* d, const wc_plan* plan, const float* dU, float* acc, int ldc, int S,
+                          bool first, const GradOut* to, int bias_rows, void* stream);
 
 // D[t][s] (na x nb, fp32, row stride ldd) = sum over rows p in [s Pq, (s + 1) Pq) of
 // A[t][p][.] (x) B[t][p][.], operands (T, P, ld) of storage type `dtype`; split: fp32 in
