@@ -267,6 +267,9 @@ int wc_output_transform(const wc_conv_desc* desc, const wc_plan* plan,
  * instead (see wc_conv_desc.unfused); the workspace then only holds U. */
 int wc_conv_workspace_bytes(const wc_conv_desc* desc, size_t* bytes);
 int wc_conv_u_elems(const wc_conv_desc* desc, size_t* elems);
+/* takes = 1: wc_conv_forward's one kernel for this problem takes this filter as it is, so a filter that is new to every call is better not
+ * transformed beforehand (row form, 3x3 layers of few tiles, taps in a row). */
+int wc_conv_takes_filter(const wc_conv_desc* desc, const void* w, const int64_t w_strides[5], int* takes);
 int wc_conv_forward(const wc_conv_desc* desc, const void* x,
                     const void* w, const int64_t w_strides[5], const void* U_cached,
                     const void* bias, void* y, void* workspace, size_t workspace_bytes,

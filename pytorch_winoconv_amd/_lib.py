@@ -64,6 +64,7 @@ SIGNATURES = {
     "wc_output_transform": (_i, [_desc_p, _plan_p, _vp, _vp, _i, _vp, _vp]),
     "wc_conv_workspace_bytes": (_i, [_desc_p, ctypes.POINTER(_sz)]),
     "wc_conv_u_elems": (_i, [_desc_p, ctypes.POINTER(_sz)]),
+    "wc_conv_takes_filter": (_i, [_desc_p, _vp, ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int)]),
     "wc_conv_forward": (_i, [_desc_p, _vp, _vp, _i64_5, _vp, _vp, _vp, _vp, _sz, _vp]),
     "wc_conv_forward_static": (_i, [_desc_p, _vp, _vp, _i64_5, _vp, _vp, _vp, _vp]),
     "wc_conv_backward_input_workspace_bytes": (_i, [_desc_p, ctypes.POINTER(_sz)]),

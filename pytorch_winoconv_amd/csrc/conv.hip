@@ -238,6 +238,14 @@ int wc_conv_u_elems(const wc_conv_desc* d, size_t* elems) {
   return WC_OK;
 }
 
+int wc_conv_takes_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5], int* takes) {
+  WC_CHECK_ARG(w && w_strides && takes, "wc_conv_takes_filter: null pointer");
+  Layout L;
+  if (int rc = make_layout(d, &L)) return rc;
+  *takes = L.row && row_takes_filter(d, w, w_strides);
+  return WC_OK;
+}
+
 int wc_conv_forward(const wc_conv_desc* d, const void* x, const void* w, const int64_t w_strides[5],
                     const void* U_cached, const void* bias, void* y, void* workspace,
                     size_t workspace_bytes, void* stream) {
@@ -299,11 +307,13 @@ int forward_impl(const wc_conv_desc* d, const void* x, const void* w, const int6
   // the three-kernel path transforms the filter in the launch of the first chunk's input transform (unless the
   // stages are being timed one by one)
   bool filter_with_input = !U && !stage_ms && !L.whole();
-  if (!U && !filter_with_input) {
+  // ... and layers of few tiles in the row form in the one kernel that they are
+  const bool filter_taken = !U && !stage_ms && L.row && row_takes_filter(d, w, w_strides);
+  if (!U && !filter_with_input && !filter_taken) {
     rc = timer.run(WC_STAGE_FILTER, [&] { return wc_filter_transform(d, &L.plan, w, w_strides, Uws, stream); });
     if (rc) return rc;
   }
-  if (!U) U = Uws;
+  if (!U && !filter_taken) U = Uws;
   wc_conv_desc dcl = *d;                  // the stages behind a scratch copy see channel-last tensors
   dcl.x_layout = L.x_direct ? 1 : 0;
   dcl.y_layout = 0;
@@ -326,7 +336,7 @@ int forward_impl(const wc_conv_desc* d, const void* x, const void* w, const int6
     }
     void* ydst = L.ycl_bytes ? Ycl : yout;
     if (L.row) {
-      rc = timer.run(WC_STAGE_PRODUCT, [&] { return row_conv(&dcl, xin, L.xcl_bytes ? wc_padded_channels8(d->C) : d->C, b0, n, U, bias, ydst, stream); });
+      rc = timer.run(WC_STAGE_PRODUCT, [&] { return row_conv(&dcl, xin, L.xcl_bytes ? wc_padded_channels8(d->C) : d->C, b0, n, U, bias, ydst, stream, w, w_strides); });
       if (rc) return rc;
     } else if (L.direct) {
       rc = timer.run(WC_STAGE_PRODUCT, [&] { return direct_conv(&dcl, xin, n, U, bias, ydst, stream); });

@@ -473,16 +473,12 @@ __global__ __launch_bounds__(256) void row_filter_kernel(RowFilterArgs a) {
       for (int j = 0; j < G; ++j)
         if (KW != 7 || j < 3 + piece) g[j] = static_cast<float>(p[j * a.s[4]]);
     }
-    // denominators: prod over the other points; 1 for 0 (a^2 b^2), 2 a^2 (a^2 - b^2) for +-a, 2 b^2 (b^2 - a^2) for +-b
-    const float fa = 1.f / (2.f * kA2 * (kA2 - kB2)), fb = 1.f / (2.f * kB2 * (kB2 - kA2));
-    // polynomials in the square of the point: three taps leave g[3] and g[4] zero
-    const float ea = __builtin_fmaf(kA2, __builtin_fmaf(kA2, g[4], g[2]), g[0]), oa = kA * __builtin_fmaf(kA2, g[3], g[1]);
-    const float eb = __builtin_fmaf(kB2, __builtin_fmaf(kB2, g[4], g[2]), g[0]), ob = kB * __builtin_fmaf(kB2, g[3], g[1]);
+    const RowPair a2 = row_filter_pair(g[0], g[1], g[2], g[3], g[4], kA, kA2, kRowFa), b2 = row_filter_pair(g[0], g[1], g[2], g[3], g[4], kB, kB2, kRowFb);
     out[0].v[e] = static_cast<T>(g[0]);
-    out[1].v[e] = static_cast<T>((ea + oa) * fa);
-    out[2].v[e] = static_cast<T>((ea - oa) * fa);
-    out[3].v[e] = static_cast<T>((eb + ob) * fb);
-    out[4].v[e] = static_cast<T>((eb - ob) * fb);
+    out[1].v[e] = static_cast<T>(a2.plus);
+    out[2].v[e] = static_cast<T>(a2.minus);
+    out[3].v[e] = static_cast<T>(b2.plus);
+    out[4].v[e] = static_cast<T>(b2.minus);
     out[5].v[e] = static_cast<T>(g[G - 1]);
   }
   T* dst = static_cast<T*>(a.U) + ((idx >> 8) * 6) * 512 + lane * 8 + e2;
@@ -805,10 +801,23 @@ bool row_reads_padded(const wc_conv_desc* d) {
                   d->C).tall_planes > 0;
 }
 
+static bool takes_few(const RowPlan& plan) {
+  const int force = test_gemm_config();
+  return force == 30 || (plan.few && force != 21 && (force < 16 || force > 19));
+}
+
+// Whether the layer's one kernel takes this filter as it is, so that nothing has to be transformed before it
+bool row_takes_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5]) {
+  if (!row_conv_fits(d) || d->kernel[1] != 3 || !row_few_takes_filter(d, w, w_strides)) return false;
+  return takes_few(row_plan(d->N, d->in[0] + 2 * d->pad[0] - d->kernel[0] + 1, d->in[1] + 2 * d->pad[1] - 2, ceil_div(d->in[2] + 2 * d->pad[2] - 2, 4), d->kernel[0], 3,
+                            d->K, d->C));
+}
+
 // x (N, D, H, W, x_row) channel-last: x_row is C, where row_reads_padded allows it, or C rounded up to 8 (zeros beyond C).  Rows of whole 16
 // bytes start at a multiple of 16; others, of which a pass's first image starts anywhere, at any element;
-// images first_image .. + n_images of the batch
-int row_conv(const wc_conv_desc* d, const void* x, int x_row, int first_image, int n_images, const void* U, const void* bias, void* y, void* stream) {
+// images first_image .. + n_images of the batch.  U null: the filter is w, which row_takes_filter
+int row_conv(const wc_conv_desc* d, const void* x, int x_row, int first_image, int n_images, const void* U, const void* bias, void* y, void* stream,
+             const void* w, const int64_t* w_strides) {
   WC_CHECK_ARG(row_conv_fits(d), "row form: 16-bit, stride 1, kernels 3x3, 3x3x3, 5x5 and 7x7");
   WC_CHECK_ARG(((x_row % 8 == 0 ? reinterpret_cast<uintptr_t>(x) : 0) | reinterpret_cast<uintptr_t>(U)) % 16 == 0, "row form: x and U must be 16-byte aligned");
   RowArgs a{};
@@ -827,7 +836,8 @@ int row_conv(const wc_conv_desc* d, const void* x, int x_row, int first_image, i
   if (force >= 16 && force <= 19) { plan.shape = (RowShape)(force - 16); plan.tall_planes = 0; plan.rest_n = -1; }
   if (force == 21 && d->kernel[1] == 3) plan.tall_planes = d->N * a.oD;
   const int tall = std::min(std::max(plan.tall_planes - first_image * a.oD, 0), n_images * a.oD);
-  if (force == 30 || (plan.few && force != 21 && (force < 16 || force > 19))) return row_few_conv(d, x, x_row, n_images, U, bias, y, stream);
+  if (takes_few(plan)) return row_few_conv(d, x, x_row, n_images, U, w, w_strides, bias, y, stream);
+  WC_CHECK_ARG(U, "row form: no transformed filter");
   if (tall > 0) {
     WC_CHECK_ARG(a.tail == 0, "row form: tall boxes of %d channels", x_row);
     const int rc = tall_row_conv(d, x, tall, U, bias, y, stream);

@@ -31,7 +31,12 @@ struct FewArgs {
   int steps, items, shares;       // channel blocks, channel blocks times planes of taps, the wavefront pairs that share them
   int x_bytes, u_bytes;
   int x_row, tail;                // elements from a pixel of x to the next: C, or `tail` (below 8) fewer
+  const void* w; long long w_k, w_c;      // the filter itself where U is null: elements from an output channel and an input channel to the next
 };
+
+// How a workgroup comes by its filter: as row_filter_kernel left it, or itself from 3x3 taps in a row, in the order of memory or against it.  kByBlock: the
+// taps of 8 channels in a row as well, at a multiple of 16 bytes
+enum FewFilter { kTransformed, kByBlock, kTaps, kTapsBack };
 
 template <typename T> struct MfmaFew;
 template <> struct MfmaFew<half_t> {
@@ -49,9 +54,14 @@ template <> struct MfmaFew<bf16_t> {
 // four rows apart, sixteen tiles each; reads: sixteen channels of four tiles)
 constexpr int kPartRow = 20, kPart = 16 * kPartRow;
 
+// FW, for 3x3 layers whose filter is new to every call (training, the functions): a launch of its own for the transform costs the host 3 us and the
+// chain as much, where all such a layer takes is 4 to 9.  A lane's fragments are 8 channels of an output channel: 144 bytes of w
+// where U is 288, and some 250 vector instructions an item.  The numbers are row_filter_kernel's.  us of a call, two launches | one, fp16:
+// N=24 96 -> 96, 9x7 10.2 | 6.9, N=1 96 -> 64, 28x28 10.3 | 7.1, 256 -> 256, 14x14 15.0 | 9.0, 512 -> 512, 7x7 22.5 | 17.1.
+//
 // SLOTS: rows of LDS for a box's input.  RC: row taps whose filter fragments are in registers at a time.  ANY: as in conv_row.hip
 // ONE: no pair has more than one item
-template <typename T, int KH, int SLOTS, int RC, int THREADS, bool ONE, bool ANY>
+template <typename T, int KH, int SLOTS, int RC, int THREADS, bool ONE, bool ANY, int FW>
 __global__ __launch_bounds__(THREADS) void row_few_kernel(FewArgs a) {
   constexpr int KP = row_pieces(KH), R = KH * KP, OUT = row_outputs_of(KH), UN = SLOTS / 32, TS = SLOTS * kRowPitch, BUF = 6 * TS;
   static_assert(BUF >= 6 * kPart * 4 && R % RC == 0 && SLOTS % 32 == 0, "partial sums in the place of the input, whole turns");
@@ -132,7 +142,7 @@ __global__ __launch_bounds__(THREADS) void row_few_kernel(FewArgs a) {
   const int kb = kg >> 1, kp = kg & 1, u_base = kb * (a.steps * a.kd * R * 2) * 6144;
   const int u_lane = (lane >> 5) * 6144 + (((lane >> 4) & 1) * 32 + kp * 16 + (lane & 15)) * 16 + tg * 3072;
   // R == RC: two sets, the next item's comes while this one's is multiplied
-  constexpr int SETS = R == RC && !ONE ? 2 : 1;
+  constexpr int SETS = R == RC && !ONE && FW == kTransformed ? 2 : 1;
   u32x4 uf[SETS][RC][3];
   auto load_u = [&](auto to_c, int item, int part, int from, int to_row) {
     constexpr int to = decltype(to_c)::value % SETS;
@@ -142,6 +152,61 @@ __global__ __launch_bounds__(THREADS) void row_few_kernel(FewArgs a) {
     for (int r = from; r < to_row; ++r)
 #pragma unroll
       for (int t = 0; t < 3; ++t) uf[to][r][t] = __builtin_amdgcn_raw_buffer_load_b128(udesc, u_lane + t * 1024, at + r * 2 * 6144, 0);
+  };
+
+  // ---- the same from the filter itself: its taps on their way, and what becomes of them
+  static_assert(FW == kTransformed || (KH == 3 && RC == R && !ANY), "three rows of three taps, whole chunks of channels");
+  constexpr int WL = FW == kByBlock ? 9 : FW == kTransformed ? 1 : 8;
+  u32x4 wr[WL];
+  unsigned short last[FW == kTaps || FW == kTapsBack ? 8 : 1];
+  const int w_m = kp * 16 + (lane & 15), w_row = min(kb * 32 + ((w_m >> 2) & 1) * 16 + (w_m >> 3) * 4 + (w_m & 3), a.K - 1);     // (rows beyond K are not stored)
+  auto load_w = [&](int item) {
+    const int c = item * 32 + (lane >> 4) * 8;
+    const bool there = c < a.C;
+    const T* const p = static_cast<const T*>(a.w) + w_row * a.w_k + (there ? c : 0) * a.w_c;
+    if constexpr (FW == kByBlock) {
+#pragma unroll
+      for (int i = 0; i < 9; ++i) wr[i] = *reinterpret_cast<const u32x4*>(p + i * 8);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const T* const q = p + e * a.w_c - (FW == kTapsBack ? 8 : 0);
+        __builtin_memcpy(&wr[e], q, 16);
+        __builtin_memcpy(&last[e], q + 8, 2);
+      }
+    }
+    if (!there) {                       // a last block of fewer channels: zeros, as x has them
+#pragma unroll
+      for (int i = 0; i < WL; ++i) wr[i] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+      for (unsigned short& l : last) l = 0;
+    }
+  };
+  auto make_u = [&]() {
+    auto tap = [&](int e, int t) -> float {
+      if (FW == kTapsBack) t = 8 - t;
+      const int at = FW == kByBlock ? e * 9 + t : t;
+      if (FW != kByBlock && t == 8) return static_cast<float>(__builtin_bit_cast(T, last[FW == kByBlock ? 0 : e]));
+      const unsigned two = wr[FW == kByBlock ? at / 8 : e][at % 8 / 2];
+      return static_cast<float>(__builtin_bit_cast(Pack<T, 2>, two).v[at % 2]);
+    };
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+      for (int word = 0; word < 4; ++word) {
+        Pack<T, 2> o[3];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float g0 = tap(word * 2 + e, r * 3), g1 = tap(word * 2 + e, r * 3 + 1), g2 = tap(word * 2 + e, r * 3 + 2);
+          const RowPair pair = row_filter_pair(g0, g1, g2, 0.f, 0.f, tg == 0 ? kA : kB, tg == 0 ? kA2 : kB2, tg == 0 ? kRowFa : kRowFb);
+          const T plus = static_cast<T>(pair.plus), minus = static_cast<T>(pair.minus);
+          o[0].v[e] = tg == 0 ? static_cast<T>(g0) : plus;
+          o[1].v[e] = tg == 0 ? plus : minus;
+          o[2].v[e] = tg == 0 ? minus : static_cast<T>(g2);
+        }
+#pragma unroll
+        for (int t = 0; t < 3; ++t) uf[0][r][t][word] = __builtin_bit_cast(unsigned, o[t]);
+      }
   };
 
   // this lane's tile
@@ -157,7 +222,8 @@ __global__ __launch_bounds__(THREADS) void row_few_kernel(FewArgs a) {
 #pragma unroll
   for (int t = 0; t < 3; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   load_x(ic<0>{}, share);
-  load_u(ic<0>{}, share, 0, 0, RC);
+  if constexpr (FW == kTransformed) load_u(ic<0>{}, share, 0, 0, RC);
+  else load_w(share);
   if constexpr (!ONE) {
     if (share + a.shares < a.items) load_x(ic<1>{}, share + a.shares);
   }
@@ -169,6 +235,10 @@ __global__ __launch_bounds__(THREADS) void row_few_kernel(FewArgs a) {
       store_v(cur_c, item);
       if constexpr (SETS == 2) {
         if (more) load_u(ic<1 - cur>{}, item + a.shares, 0, 0, RC);
+      }
+      if constexpr (FW != kTransformed) {
+        make_u();
+        if (more) load_w(item + a.shares);
       }
     }
     __syncthreads();
@@ -184,7 +254,7 @@ __global__ __launch_bounds__(THREADS) void row_few_kernel(FewArgs a) {
         }
       }
       if constexpr (!ONE) {
-        if constexpr (SETS == 1) {
+        if constexpr (SETS == 1 && FW == kTransformed) {
           if (more) load_u(ic<0>{}, item + a.shares, 0, 0, RC);
         }
         if (item + 2 * a.shares < a.items) load_x(cur_c, item + 2 * a.shares);
@@ -264,10 +334,27 @@ bool row_few_pays(long long planes, int oH, int nW, int kd, int kh, int K, int C
   return few_box((int)planes, oH, nW, kh).boxes * groups <= (long long)resident * kCus;
 }
 
-// Images n_images from x on; x as row_conv takes it
-int row_few_conv(const wc_conv_desc* d, const void* x, int x_row, int n_images, const void* U, const void* bias, void* y, void* stream) {
+// How the kernel can take the filter as it is (kTransformed: not)
+static FewFilter few_filter(const wc_conv_desc* d, const void* w, const int64_t s[5]) {
+  if (d->kernel[0] != 1 || d->kernel[1] != 3 || d->kernel[2] != 3 || d->C % 8 || (s[4] != 1 && s[4] != -1) || s[3] != 3 * s[4] || (reinterpret_cast<uintptr_t>(w) & 1)) return kTransformed;
+  if (s[4] == 1 && s[1] == 9 && s[0] % 8 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0) return kByBlock;
+  // Sixteen loads of scattered channels an item instead of nine: ahead where the reduction has an item to a pair (input gradients, us, two launches | one, 256 -> 256,
+  // 14x14 14.0 | 10.0, N=24 96 -> 96, 9x7 10.3 | 7.9), behind with more (512 -> 512, 7x7 20.2 | 20.4, N=2 416 -> 224, 19x17 16.8 | 17.5) and with planes of
+  // taps (128 -> 128, 3x9x9 14.6 | 17.2, forward 15.8 | 26.6)
+  if (ceil_div(d->C, 32) > few_shares(3, true)) return kTransformed;
+  return s[4] == 1 ? kTaps : kTapsBack;
+}
+bool row_few_takes_filter(const wc_conv_desc* d, const void* w, const int64_t s[5]) { return few_filter(d, w, s) != kTransformed; }
+
+// Images n_images from x on; x as row_conv takes it.  U null: the filter is w
+int row_few_conv(const wc_conv_desc* d, const void* x, int x_row, int n_images, const void* U, const void* w, const int64_t* w_strides, const void* bias, void* y,
+                 void* stream) {
   FewArgs a{};
   const int kh = d->kernel[1];
+  const FewFilter how = U ? kTransformed : few_filter(d, w, w_strides);
+  WC_CHECK_ARG(U || how != kTransformed, "row form, few tiles: neither a transformed filter nor one that the kernel takes");
+  a.w = w;
+  if (!U) { a.w_k = w_strides[0]; a.w_c = w_strides[1]; }
   a.x = x; a.U = U; a.bias = bias; a.y = y;
   a.N = n_images; a.D = d->in[0]; a.H = d->in[1]; a.W = d->in[2]; a.C = wc_padded_channels8(d->C); a.K = d->K;
   a.x_row = x_row; a.tail = a.C - x_row;
@@ -293,7 +380,12 @@ int row_few_conv(const wc_conv_desc* d, const void* x, int x_row, int n_images, 
         constexpr int KH = decltype(kh_c)::value, SLOTS = few_slots(KH), RC = KH;
         constexpr bool ONE = decltype(one_c)::value != 0;
         constexpr int SHARES = few_shares(KH, ONE), THREADS = 128 * SHARES;
-        const auto fn = a.tail ? &row_few_kernel<T, KH, SLOTS, RC, THREADS, ONE, true> : &row_few_kernel<T, KH, SLOTS, RC, THREADS, ONE, false>;
+        auto fn = a.tail ? &row_few_kernel<T, KH, SLOTS, RC, THREADS, ONE, true, kTransformed> : &row_few_kernel<T, KH, SLOTS, RC, THREADS, ONE, false, kTransformed>;
+        if constexpr (KH == 3) {
+          if (how == kByBlock) fn = &row_few_kernel<T, KH, SLOTS, RC, THREADS, ONE, false, kByBlock>;
+          else if (how == kTaps) fn = &row_few_kernel<T, KH, SLOTS, RC, THREADS, ONE, false, kTaps>;
+          else if (how == kTapsBack) fn = &row_few_kernel<T, KH, SLOTS, RC, THREADS, ONE, false, kTapsBack>;
+        }
         constexpr int bytes = 6 * SLOTS * kRowPitch;          // of a pair
         if (const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), SHARES * bytes)) return rc;
         hipLaunchKernelGGL(fn, dim3(a.per_xcd * kXcds), dim3(128 * a.shares), a.shares * bytes, as_stream(stream), a);

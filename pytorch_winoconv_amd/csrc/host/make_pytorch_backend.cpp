@@ -914,6 +914,7 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
   size_t bytes = 0, u_elems = 0;
   int nd, stride, m;
   std::vector<int> pads;
+  std::vector<int64_t> taken_strides;               // of weights that the layer's kernel takes as they are; empty: none
   std::shared_ptr<KeptFilter> filter;               // null: not made yet
 
   // None where the layer copies its input first.  `kept`: the filter of the module's last pass, taken where it is this one's
@@ -930,6 +931,11 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
     p->d.x_layout = !last;
     check(wc_conv_u_elems(&p->d, &p->u_elems));
     if (kept && kept->suits(p->form(), x.scalar_type(), x.device())) p->filter = kept;
+    int64_t s[5];
+    int takes = 0;
+    strides_of(weight, s);
+    check(wc_conv_takes_filter(&p->d, weight.data_ptr(), s, &takes));
+    if (takes) p->taken_strides = weight.strides().vec();
     int out[3], grid[3];
     check(wc_conv_out_dims(&p->d, out, grid));
     check(wc_conv_workspace_bytes(&p->d, &p->bytes));
@@ -1055,12 +1061,14 @@ py::object LayerPlan::call(const at::Tensor& x, const at::Tensor& weight, const 
     py::gil_scoped_release nogil;
     const bool grad = at::GradMode::is_enabled() && (x.requires_grad() || weight.requires_grad() || (bias && bias->requires_grad()));
     LayerOperands o{shared_from_this(), weight, bias ? *bias : at::Tensor(), filter && filter->holds(weight) ? filter->on_stream() : at::Tensor()};
-    const bool anew = !o.U.defined();
+    // a pass with gradients, after which the weight is likely another one: nothing to keep where the kernel takes the filter itself
+    const bool taken = grad && !o.U.defined() && !taken_strides.empty() && weight.strides() == at::IntArrayRef(taken_strides);
+    const bool anew = !o.U.defined() && !taken;
     if (anew) {
       renewed = std::make_shared<LayerPlan>(*this);
       renewed->filter = std::make_shared<KeptFilter>(weight, form());
     }
-    const bool cast_w = (grad || anew) && w_type != x_type, cast_b = bias && bias->scalar_type() != x_type;
+    const bool cast_w = (grad || anew || taken) && w_type != x_type, cast_b = bias && bias->scalar_type() != x_type;
     if (cast_w || cast_b) {
       at::AutoGradMode no_grad(false);
       if (cast_w) o.w = weight.to(x_type);

@@ -56,6 +56,18 @@ __device__ __forceinline__ void row_input_channel(Pack<T, 2> (&x)[6], int e) {
   x[4].v[e] = static_cast<T>(__builtin_fmaf(-kB, ob, eb));
 }
 
+// The pair of elements at +p and -p (p^2 = p2) of a row of five taps: three leave g3 and g4 zero.  Explicit, so that kernels
+// that transform a filter for themselves find the numbers of those that do it for them
+struct RowPair { float plus, minus; };
+__device__ __forceinline__ RowPair row_filter_pair(float g0, float g1, float g2, float g3, float g4, float p, float p2, float f) {
+  const float even = __builtin_fmaf(p2, __builtin_fmaf(p2, g4, g2), g0), odd = __builtin_fmaf(p2, g3, g1);
+  RowPair o = {__builtin_fmaf(p, odd, even) * f, __builtin_fmaf(-p, odd, even) * f};
+  asm("" : "+v"(o.plus), "+v"(o.minus));          // a product in fp32: not rounded to T within one instruction here and in two there
+  return o;
+}
+// denominators: prod over the other points; 1 for 0 (a^2 b^2), 2 a^2 (a^2 - b^2) for +-a, 2 b^2 (b^2 - a^2) for +-b
+constexpr float kRowFa = 1.f / (2.f * kA2 * (kA2 - kB2)), kRowFb = 1.f / (2.f * kB2 * (kB2 - kA2));
+
 // Outputs of a tile: the six elements carry F(4, 3), F(2, 5) and F(3, 4) alike, whose tiles start 4, 2 and 3 pixels apart.  A row
 // of 7 taps is two of F(3, 4): the first three taps, and the other four on the tile after, three pixels on.
 __host__ __device__ constexpr int row_outputs_of(int taps) { return taps == 7 ? 3 : 7 - taps; }
@@ -114,6 +126,8 @@ RowBox choose_box(int N, int oD, int oH, int nW, int kd, int kh, int tiles, int 
 // Few tiles (conv_row_few.hip): whether the kernel is taken for `planes` output planes (padded: x with channels padded to a multiple of 8), and the
 // launch with the arguments of row_conv
 bool row_few_pays(long long planes, int oH, int nW, int kd, int kh, int K, int C, bool padded);
-int row_few_conv(const wc_conv_desc* d, const void* x, int x_row, int n_images, const void* U, const void* bias, void* y, void* stream);
+bool row_few_takes_filter(const wc_conv_desc* d, const void* w, const int64_t s[5]);      // as it is, instead of U
+int row_few_conv(const wc_conv_desc* d, const void* x, int x_row, int n_images, const void* U, const void* w, const int64_t* w_strides, const void* bias, void* y,
+                 void* stream);
 
 }  // namespace wc

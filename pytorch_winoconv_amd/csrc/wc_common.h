@@ -163,7 +163,9 @@ bool row_preferred(const wc_conv_desc* d);        // where it measured faster th
 size_t row_u_elems(const wc_conv_desc* d);
 int row_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5], void* U, void* stream);
 bool row_reads_padded(const wc_conv_desc* d);
-int row_conv(const wc_conv_desc* d, const void* x, int x_row, int first_image, int n_images, const void* U, const void* bias, void* y, void* stream);
+bool row_takes_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5]);
+int row_conv(const wc_conv_desc* d, const void* x, int x_row, int first_image, int n_images, const void* U, const void* bias, void* y, void* stream,
+             const void* w = nullptr, const int64_t* w_strides = nullptr);
 int tall_row_conv(const wc_conv_desc* d, const void* x, int n_planes, const void* U, const void* bias, void* y, void* stream);   // conv_row_tall.hip
 // Strided first layers (direct_first.hip): at most 4 input channels, stride 2, kernels of 3, 5 or 7 rows and at most 8
 // columns, 16-bit types.  U is (K, kh, 8 taps, 4 channels), zero where the filter has no tap or channel.
