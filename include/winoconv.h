@@ -225,6 +225,9 @@ int wc_wino_concat2d(const void* tiles, void* y, int B, int oH, int oW, int K, i
 int wc_wino_concat3d(const void* tiles, void* y, int B, int oD, int oH, int oW, int K, int m,
                      int elem_size, void* stream);
 
+/* n_w and n_bias (0: none) fp32 values rounded to the 16-bit type `dtype`, in one launch. */
+int wc_cast_parameters(const float* w, void* w_out, long long n_w, const float* bias, void* bias_out, long long n_bias, int dtype, void* stream);
+
 /* Bit-exact copy between channel-first (n, C, S) and channel-last (n, S, C) memory, S = [D] H W positions;
  * to_channel_last = 1 for the first direction.  Replaces the permute passes of the reference's Python callers
  * (dwm.py:129-133,143-144; Split_and_Concat.py:25,47,64,81).  elem_size is 2 or 4 bytes. */

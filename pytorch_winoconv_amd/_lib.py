@@ -57,6 +57,7 @@ SIGNATURES = {
     "wc_wino_split_channel_first": (_i, [_vp, _vp] + [_i] * 13 + [_vp]),
     "wc_wino_concat2d": (_i, [_vp, _vp] + [_i] * 6 + [_vp]),
     "wc_wino_concat3d": (_i, [_vp, _vp] + [_i] * 7 + [_vp]),
+    "wc_cast_parameters": (_i, [_vp, _vp, ctypes.c_longlong, _vp, _vp, ctypes.c_longlong, _i, _vp]),
     "wc_layout_copy": (_i, [_vp, _vp, _i, _i, ctypes.c_longlong, _i, _i, _vp]),
     "wc_filter_transform": (_i, [_desc_p, _plan_p, _vp, _i64_5, _vp, _vp]),
     "wc_input_transform": (_i, [_desc_p, _plan_p, _vp, _i, _vp, _vp]),

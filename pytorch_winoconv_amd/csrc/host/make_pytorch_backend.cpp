@@ -1071,8 +1071,16 @@ py::object LayerPlan::call(const at::Tensor& x, const at::Tensor& weight, const 
     const bool cast_w = (grad || anew || taken) && w_type != x_type, cast_b = bias && bias->scalar_type() != x_type;
     if (cast_w || cast_b) {
       at::AutoGradMode no_grad(false);
-      if (cast_w) o.w = weight.to(x_type);
-      if (cast_b) o.bias = bias->to(x_type);
+      if (cast_w && w_type == at::kFloat && weight.is_non_overlapping_and_dense() && weight.numel() > 0) {
+        const bool both = cast_b && bias->scalar_type() == at::kFloat && bias->is_contiguous();
+        o.w = at::empty_strided(weight.sizes(), weight.strides(), x.options());
+        if (both) o.bias = at::empty_strided(bias->sizes(), bias->strides(), x.options());
+        check(wc_cast_parameters(weight.data_ptr<float>(), o.w.data_ptr(), weight.numel(), both ? bias->data_ptr<float>() : nullptr,
+                                 both ? o.bias.data_ptr() : nullptr, both ? bias->numel() : 0, dtype_of(x), stream_of(x)));
+      } else if (cast_w) {
+        o.w = weight.to(x_type);
+      }
+      if (cast_b && o.bias.scalar_type() != x_type) o.bias = bias->to(x_type);
     }
     if (o.bias.defined()) o.bias = o.bias.contiguous();
     if (anew) {

@@ -146,9 +146,46 @@ int pad_channels(const void* src, void* dst, long long n, int C, int Cx, long lo
   return WC_OK;
 }
 
+// The fp32 parameters of a layer in its activations' type, weight and bias in one launch: as two casts they were two launches of some
+// 5 us of host time each, in a training step that waits for the host (us, fp16 N=64 128 -> 128, 28x28: 99.9 | 89.8).
+struct CastArgs {
+  const float* src[2]; void* dst[2];
+  long long n[2];
+  int blocks;                      // of the first, 1024 elements each; the second's behind them
+};
+template <typename T>
+__global__ __launch_bounds__(256) void cast_kernel(CastArgs a) {
+  const int which = (int)blockIdx.x >= a.blocks;
+  const float* const src = a.src[which];
+  T* const dst = static_cast<T*>(a.dst[which]);
+  const long long i = ((long long)(blockIdx.x - (which ? a.blocks : 0)) * 256 + threadIdx.x) * 4, n = a.n[which];
+  if (i >= n) return;
+  if (i + 4 <= n) {                // either tensor may start at any element
+    float v[4];
+    Pack<T, 4> o;
+    __builtin_memcpy(v, src + i, 16);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o.v[e] = static_cast<T>(v[e]);
+    __builtin_memcpy(dst + i, &o, 8);
+  } else {
+    for (long long e = i; e < n; ++e) dst[e] = static_cast<T>(src[e]);
+  }
+}
+
 }  // namespace wc
 
 using namespace wc;
+
+extern "C" int wc_cast_parameters(const float* w, void* w_out, long long n_w, const float* bias, void* bias_out, long long n_bias, int dtype, void* stream) {
+  WC_CHECK_ARG(w && w_out && n_w > 0 && (n_bias == 0 || (n_bias > 0 && bias && bias_out)), "wc_cast_parameters: null pointer or empty tensor");
+  WC_CHECK_ARG(dtype == WC_F16 || dtype == WC_BF16, "wc_cast_parameters: dtype %d, a 16-bit type is needed", dtype);
+  const long long blocks = ceil_div_ll(n_w, 1024), more = ceil_div_ll(n_bias, 1024);
+  WC_CHECK_ARG(blocks + more < (1ll << 31), "wc_cast_parameters: problem too large");
+  const CastArgs a = {{w, bias}, {w_out, bias_out}, {n_w, n_bias}, (int)blocks};
+  hipLaunchKernelGGL(dtype == WC_F16 ? &cast_kernel<half_t> : &cast_kernel<bf16_t>, dim3((unsigned)(blocks + more)), dim3(256), 0, as_stream(stream), a);
+  WC_CHECK_LAUNCH("cast_kernel");
+  return WC_OK;
+}
 
 extern "C" int wc_layout_copy(const void* src, void* dst, int n_images, int channels, long long spatial,
                               int to_channel_last, int elem_size, void* stream) {
