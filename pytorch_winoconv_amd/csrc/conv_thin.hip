@@ -443,9 +443,9 @@ __global__ __launch_bounds__(64 * KSUB) __attribute__((amdgpu_waves_per_eu(KSUB 
 // products, and a block has one barrier that waits for LDS and one that waits for nothing.
 //
 // Two rows of elements and 16 output channels a wavefront, each phase of a block behind the last one, took 73 us (2.6 a block) where this
-// takes 58 (fp16 N=64 128 -> 128, 56x56; 28x28 25.3 | 21.4; bf16 77 | 65; fp32 N=64 64 -> 64, 56x56 79 | 70).  The dealing out
+// takes 57 (fp16 N=64 128 -> 128, 56x56; 28x28 25.5 | 21.4; bf16 77 | 63; fp32 N=64 64 -> 64, 56x56 79 | 69.5).  The dealing out
 // alone is 70: fragments of V fed one product and a half, LDS 256 KB of reads a block.  What is left of 1.8 us a block: taken out one at a
-// time, the loads are 0.35 of it (64 KB through L1, the same from a footprint of 4 KB), products 0.4, the output 0.3, transform and its stores 0.2.
+// time, the loads are 0.4 of it (64 KB through L1, the same from a footprint of 4 KB), products 0.4, the hand-over and the output 0.3.
 // Of a thin_conv3x3_kernel with 128-byte rows two run on a CU, side by side, and the same order of its work was slower (64 channels 23.0 | 23.8).
 template <typename T, int CP, bool KW, int KSUB>
 __global__ __launch_bounds__((kThinThreads<T, CP, KSUB>)) __attribute__((amdgpu_waves_per_eu(KSUB / 2, KSUB / 2))) void thin_rows_kernel(ThinArgs a) {
@@ -666,6 +666,8 @@ __global__ __launch_bounds__((kThinThreads<T, CP, KSUB>)) __attribute__((amdgpu_
   // next block, its way to LDS and the loads of the block after are dealt out over the items (MORE: there is a next block).
   auto block = [&](auto more_, int it) {
     constexpr bool MORE = decltype(more_)::value != 0;
+    // Fragments two items ahead; the transform from the first quarter on, of bf16, whose numbers take twice the registers, in the last three
+    // eighths, before which its loads are not waited for either (us, from 1/4 | 5/8: fp16 57.1 | 60.8, fp32 69.5 | 69.6, bf16 spilling 72 | 62.7)
     constexpr int NI = KS * 4, VD = 3, FROM = std::is_same<T, bf16_t>::value ? NI * 5 / 8 : NI / 4, MEET = 2;
     const int cur = (it & 1) * BUF, next = BUF - cur;
     asm volatile("" : "+v"(vrow));                // addresses are worked out again: registers are short
