@@ -541,9 +541,11 @@ struct RowPlan { RowShape shape; RowBox box; long long wide_groups; int tall_pla
 // Over 300 layers drawn anew the choice takes 1.6 % longer than the fastest shape of each in the mean, with a line through the origin for
 // half boxes, and small ones up to one a CU only, 3.2 %.  fp16, us, wide | half | small: 280 half boxes of 7 steps 25.2 | 25.9 |
 // 21.0, 252 of 7 steps 22.5 | 16.7 | 21.4; 3-D, 280 of 2 steps 18.0 | 26.2 | 20.6, 160 17.7 | 25.2 | 27.9 (two rounds of half boxes, one of wide
-// ones).
+// ones).  Half boxes of 5x5 filters, one a CU, against two small ones, of 4 and more steps: 0.43 to 0.50 of a unit in 29 layers of 130 to 256 half
+// boxes, the faster in each (0.58, fitted to boxes of any number, took small ones from 7 steps on): 4 steps 12.6 | 14.7, 6 16.5 | 19.5, 7 17.7 | 21.8
+// (195 boxes) and 18.6 | 23.8 (231), 8 19.3 | 24.3.
 struct RowModel { double wide, wide_round, half, half_two, half_more, half_at, half_step, small_two, small_three, small_more; };
-constexpr RowModel kRow3x3{0.86, 0.92, 0.60, 0.97, 1.27, 1.0, 0.12, 1.6, 2.1, 0.82}, kRow5x5{0.82, 0.80, 0.58, 0.75, 1.15, 0.85, 0.10, 1.25, 1.7, 0.68},
+constexpr RowModel kRow3x3{0.86, 0.92, 0.60, 0.97, 1.27, 1.0, 0.12, 1.6, 2.1, 0.82}, kRow5x5{0.82, 0.80, 0.46, 0.75, 1.15, 0.85, 0.10, 1.25, 1.7, 0.68},
     kRow3d{0.78, 0.72, 0.53, 1.06, 0.0, 0.0, 0.0, 1.2, 1.7, 0.60};
 
 RowPlan make_row_shape(int N, int oD, int oH, int nW, int kd, int kh, int K, int steps) {
