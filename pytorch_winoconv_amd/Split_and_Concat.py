@@ -62,6 +62,8 @@ def wino_concat(a, output_size, output_block_size):
         raise ValueError("wino_concat: tiles and output_size disagree")
     osz = [int(o) for o in output_size]
     n = [(o + m - 1) // m for o in osz]                              # Split_and_Concat.py:58-60,72-73
+    if any(v != m for v in a.shape[2:]):
+        raise ValueError("wino_concat: tiles of %s for an output block of %d" % (tuple(a.shape[2:]), m))
     per_image = 1
     for v in n:
         per_image *= v

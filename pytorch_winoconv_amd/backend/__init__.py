@@ -79,6 +79,8 @@ def WinoConcat(in_a, out, output_block_size, two_dimension):
     if not in_a.is_contiguous() or not out.is_contiguous():
         raise ValueError("WinoConcat: tensors must be contiguous")
     lib, m, es = _lib.load(), int(output_block_size), in_a.element_size()
+    if any(v != m for v in in_a.shape[2:]):
+        raise ValueError("WinoConcat: tiles of shape %r for an output tile of %d" % (tuple(in_a.shape), m))
     N, K = in_a.shape[:2]
     osz = list(out.shape[1:-1])
     per = 1

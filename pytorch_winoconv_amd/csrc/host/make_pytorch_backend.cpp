@@ -189,6 +189,9 @@ void WinoConcat(at::Tensor in_a, at::Tensor out, int output_block_size, bool two
   const int nd = two_dimension ? 2 : 3, m = output_block_size;
   if (in_a.dim() != nd + 2 || out.dim() != nd + 2 || m < 1)
     throw std::invalid_argument("WinoConcat: expected tiles (N, K, [m,] m, m) and a channel-last output");
+  for (int a = 0; a < nd; ++a)
+    if (in_a.size(2 + a) != m)
+      throw std::invalid_argument("WinoConcat: tiles of shape " + shape_str(in_a.sizes()) + " for an output tile of " + std::to_string(m));
   const int64_t N = in_a.size(0), K = in_a.size(1);
   int64_t per = 1;
   for (int a = 0; a < nd; ++a) per *= (out.size(1 + a) + m - 1) / m;
@@ -875,7 +878,11 @@ py::object wino_concat(py::handle a_, py::handle size_, py::handle m_) {
   const auto size = whole_numbers(size_, nd);
   if (!size) return py::none();
   int64_t per = 1;
-  for (const int64_t o : *size) per *= (o + *m - 1) / *m;
+  for (int q = 0; q < nd; ++q) {
+    if (a->size(2 + q) != *m) return py::none();
+    per *= ((*size)[q] + *m - 1) / *m;
+    if (per > a->size(0)) return py::none();           // no whole image; and the product of three extents may wrap around to 0
+  }
   if (a->size(0) % per) return py::none();
   const int64_t B = a->size(0) / per, K = a->size(1);
   at::Tensor out;

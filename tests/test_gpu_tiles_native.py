@@ -3,7 +3,7 @@ refusals, under capture and on another stream."""
 import pytest
 import torch
 
-from pytorch_winoconv_amd import engine, wino_concat, wino_split
+from pytorch_winoconv_amd import backend, engine, wino_concat, wino_split
 
 pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not engine.USE_EXT, reason="no compiled host layer")]
 
@@ -48,7 +48,25 @@ def test_refused_as_before(dev):
     for args, error in [((x.cpu(), (8, 8), 2), ValueError), ((x, (8, 8, 8), 2), ValueError), ((torch.randn(3, 4, 2, 2, device=dev), (4, 4), 2), ValueError)]:
         with pytest.raises(error):
             wino_concat(*args)
+    # extents whose product is a multiple of 2^64
+    with pytest.raises(ValueError):
+        wino_concat(torch.randn(1, 1, 1, 1, 1, device=dev), (1 << 22, 1 << 21, 1 << 21), 1)
     assert torch.equal(wino_split(x, (4, 4, 3.0, 3), 2), wino_split(x, (4, 4, 3, 3), 2))      # whatever int() takes
+
+
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("shape,size,m", [((16, 4, 2, 2), (16, 16), 4), ((16, 4, 4, 2), (16, 16), 4), ((16, 4, 4, 4), (8, 8), 2), ((16, 4, 1, 4), (8, 8), 2),
+                                          ((8, 4, 2, 2, 2), (8, 8, 8), 4), ((8, 4, 3, 2, 2), (4, 4, 4), 2)])
+def test_tiles_of_another_extent_are_refused(dev, monkeypatch, native, shape, size, m):
+    """They would be read as tiles of m, beyond their memory where they are smaller."""
+    monkeypatch.setattr(engine, "USE_EXT", native)
+    tiles = torch.randn(shape, device=dev)
+    with pytest.raises(ValueError):
+        wino_concat(tiles, size, m)
+    out = torch.empty((1,) + size + (4,), device=dev)
+    concat = engine._ext.WinoConcat if native else backend.WinoConcat
+    with pytest.raises(ValueError):
+        concat(tiles, out, m, len(size) == 2)
 
 
 def test_captured_and_on_another_stream(dev):
