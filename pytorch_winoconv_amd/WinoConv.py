@@ -213,6 +213,9 @@ class _WinoConvNd(nn.Module):
         # depends on the batch size too, and the transformed filter of one form does not fit the other
         form = engine.filter_form(x.shape, weight.shape, x.dtype, self.stride[0], self.padding, m)
         U = cache[1].on_stream() if cache is not None and cache[0] == (x.dtype, form) and cache[1].holds(weight) else None
+        # a graph of a pass that is trained is replayed with other weights: it makes its filter itself
+        if U is not None and weight.requires_grad and torch.is_grad_enabled() and torch.cuda.is_current_stream_capturing():
+            U = None
         if U is None:
             cache = ((x.dtype, form), engine.KeptFilter(weight, form))
         # (to() and detach() that change nothing still cost a microsecond each of a 12 us call)

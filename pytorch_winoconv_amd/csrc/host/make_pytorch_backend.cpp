@@ -1067,7 +1067,9 @@ py::object LayerPlan::call(const at::Tensor& x, const at::Tensor& weight, const 
   {
     py::gil_scoped_release nogil;
     const bool grad = at::GradMode::is_enabled() && (x.requires_grad() || weight.requires_grad() || (bias && bias->requires_grad()));
-    LayerOperands o{shared_from_this(), weight, bias ? *bias : at::Tensor(), filter && filter->holds(weight) ? filter->on_stream() : at::Tensor()};
+    // A graph of a pass that is trained is replayed with other weights: it makes its filter itself
+    const bool known = filter && filter->holds(weight) && !(grad && weight.requires_grad() && capturing(stream_of(x)));
+    LayerOperands o{shared_from_this(), weight, bias ? *bias : at::Tensor(), known ? filter->on_stream() : at::Tensor()};
     // a pass with gradients, after which the weight is likely another one: nothing to keep where the kernel takes the filter itself
     const bool taken = grad && !o.U.defined() && !taken_strides.empty() && weight.strides() == at::IntArrayRef(taken_strides);
     const bool anew = !o.U.defined() && !taken;

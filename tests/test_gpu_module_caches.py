@@ -155,6 +155,32 @@ def test_a_filter_made_inside_a_capture(dev, passes, warm):
 
 
 @pytest.mark.parametrize("own", [torch.float16, torch.float32])
+@pytest.mark.parametrize("c,k,taps", [(64, 96, 5), (160, 64, 3)])
+def test_a_captured_pass_of_a_trained_weight(dev, passes, own, c, k, taps):
+    """Its graph is replayed after updates of the weight, whose filter the passes before the capture have kept, and gives what an eager pass does."""
+    layer = pkg.WinoConv2d(c, k, taps, padding=taps // 2, device=dev, dtype=own)
+    x = _input(dev, 2, c, 15, 14)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(max(passes, 3)):
+            layer(x)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = layer(x)
+    assert y.requires_grad
+    for i in range(3):
+        with torch.no_grad():
+            layer.weight.mul_(-1.5)
+        x.copy_(_input(dev, 2, c, 15, 14, seed=5 + i))
+        graph.replay()
+        torch.cuda.synchronize()
+        _close(y.detach(), layer, x)
+        assert torch.equal(y, layer(x))
+
+
+@pytest.mark.parametrize("own", [torch.float16, torch.float32])
 def test_shapes_types_and_memory_orders_in_turn(dev, passes, own):
     """Each pass with the filter of its own form: batches on either side of the direct form's line, images, types and orders in memory."""
     layer = pkg.WinoConv2d(128, 128, 7, 2, 3, device=dev, dtype=own).requires_grad_(False)
