@@ -94,3 +94,57 @@ def test_module_passes_with_and_without_gradients(dev, own):
         with torch.no_grad():
             layer.weight -= 1e-3 * layer.weight.grad
             assert torch.equal(layer(x), layer(x))
+
+
+def _kept(layer):
+    """The filter that the module's next pass finds, None if it finds none."""
+    return layer._cache[1].on_stream() if layer._cache is not None and layer._cache[1].holds(layer.weight) else None
+
+
+def _module(dev, own, seed):
+    torch.manual_seed(seed)
+    layer = WinoConv2d(160, 64, 3, padding=1, device=dev, dtype=own)
+    x = torch.randn(1, 160, 14, 14, device=dev, dtype=torch.float16).contiguous(memory_format=torch.channels_last)
+    assert _takes(x, layer.weight.detach().half()) == 1
+
+    def reference(v):
+        U = engine.transform_filter(layer.weight.detach().half(), v.shape, 1, 1, layer._tile_for(v.dtype), row=True)
+        return engine.conv_forward(v.detach(), layer.weight.detach().half(), layer.bias.detach().half(), 1, 1, layer._tile_for(v.dtype), U=U, row=True)
+    return layer, x, reference
+
+
+@pytest.mark.skipif(not engine.USE_EXT, reason="no compiled host layer")
+@pytest.mark.parametrize("own", [torch.float16, torch.float32])
+@pytest.mark.parametrize("bias_too", [False, True])
+def test_a_frozen_filter_is_kept_in_passes_with_gradients(dev, own, bias_too):
+    """Where the input or the bias alone needs a gradient, the first pass makes the filter and the others find it."""
+    layer, x, reference = _module(dev, own, 1)
+    layer.weight.requires_grad_(False)
+    layer.bias.requires_grad_(bias_too)
+    x.requires_grad_(not bias_too)
+    y = layer(x)
+    U = _kept(layer)
+    assert U is not None and y.requires_grad
+    for _ in range(2):
+        assert torch.equal(layer(x), y) and _kept(layer).data_ptr() == U.data_ptr()
+    assert torch.equal(y.detach(), reference(x))
+    with torch.no_grad():
+        assert torch.equal(layer(x), y) and _kept(layer).data_ptr() == U.data_ptr()
+
+
+@pytest.mark.skipif(not engine.USE_EXT, reason="no compiled host layer")
+@pytest.mark.parametrize("own", [torch.float16, torch.float32])
+def test_a_filter_is_kept_from_the_second_pass_on(dev, own):
+    """A trained weight's first pass takes it as it is; the next with the same weight makes its filter, also on another batch size."""
+    layer, x, reference = _module(dev, own, 2)
+    more = torch.cat([x, -x]).contiguous(memory_format=torch.channels_last)
+    for second in (x, more, x):
+        y = layer(x)
+        assert _kept(layer) is None and torch.equal(y.detach(), reference(x))
+        y = layer(second)
+        U = _kept(layer)
+        assert U is not None and torch.equal(y.detach(), reference(second))
+        assert torch.equal(layer(x).detach(), reference(x)) and _kept(layer).data_ptr() == U.data_ptr()
+        y.sum().backward()
+        with torch.no_grad():
+            layer.weight -= 1e-3 * layer.weight.grad
