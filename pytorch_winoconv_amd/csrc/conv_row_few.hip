@@ -60,7 +60,9 @@ constexpr int kPartRow = 20, kPart = 16 * kPartRow;
 // N=24 96 -> 96, 9x7 10.2 | 6.9, N=1 96 -> 64, 28x28 10.3 | 7.1, 256 -> 256, 14x14 15.0 | 9.0, 512 -> 512, 7x7 22.5 | 17.1.
 //
 // SLOTS: rows of LDS for a box's input.  RC: row taps whose filter fragments are in registers at a time.  ANY: as in conv_row.hip
-// ONE: no pair has more than one item
+// ONE: no pair has more than one item.  7x7 with more: two sets of 12 fragments of input leave 2 of 14 row taps room (all seven of a half spilled 7 to 11
+// registers; us so | two at a time: N=1 512 -> 160, 7x7 25.5 | 21.4, 160 -> 160, 28x28 11.9 | 9.9, N=4 250 -> 512, 7x7 15.4 | 13.5, N=2 384 -> 96, 14x14
+// 19.7 | 17.0; the other shapes' fastest of the four 29.9, 14.9, 18.2, 24.0)
 template <typename T, int KH, int SLOTS, int RC, int THREADS, bool ONE, bool ANY, int FW>
 __global__ __launch_bounds__(THREADS) void row_few_kernel(FewArgs a) {
   constexpr int KP = row_pieces(KH), R = KH * KP, OUT = row_outputs_of(KH), UN = SLOTS / 32, TS = SLOTS * kRowPitch, BUF = 6 * TS;
@@ -99,7 +101,7 @@ __global__ __launch_bounds__(THREADS) void row_few_kernel(FewArgs a) {
     constexpr int to = decltype(to_c)::value;
     const int rd = item / a.steps, step = item - rd * a.steps;
     const bool there = step * 32 + chunk * 8 < a.C;
-    // the lanes of the last eight channels start `tail` channels before and shift (shift_x)
+    // the lanes of the last eight channels start `tail` channels before and shift (store_v)
     const int back = ANY && step * 32 + chunk * 8 == a.C - 8 ? a.tail * 2 : 0;
 #pragma unroll
     for (int i = 0; i < UN; ++i) {
@@ -377,8 +379,8 @@ int row_few_conv(const wc_conv_desc* d, const void* x, int x_row, int n_images, 
     using T = decltype(t);
     if constexpr (sizeof(T) == 2) {
       auto launch = [&](auto kh_c, auto one_c) -> int {
-        constexpr int KH = decltype(kh_c)::value, SLOTS = few_slots(KH), RC = KH;
         constexpr bool ONE = decltype(one_c)::value != 0;
+        constexpr int KH = decltype(kh_c)::value, SLOTS = few_slots(KH), RC = KH == 7 && !ONE ? 2 : KH;
         constexpr int SHARES = few_shares(KH, ONE), THREADS = 128 * SHARES;
         auto fn = a.tail ? &row_few_kernel<T, KH, SLOTS, RC, THREADS, ONE, true, kTransformed> : &row_few_kernel<T, KH, SLOTS, RC, THREADS, ONE, false, kTransformed>;
         if constexpr (KH == 3) {
