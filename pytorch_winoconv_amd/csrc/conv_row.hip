@@ -530,9 +530,9 @@ namespace {
 // 68 | 60 | 74; N=16, 256 -> 256, 14x14 21 | 15 | 12.4 | 10.6; N=1, 512 -> 512, 7x7 33 | 22 | 19 | 12.  (Layers of up to 128 input
 // channels come here in 3-D or with tile 4; with tile 2 the one-kernel F(2x2, 3x3) form takes most of them, see row_preferred.)
 enum RowShape { kRowWide, kRowHalf, kRowSmall, kRowSplit };
-// tall_planes: output planes, images in 2-D, that go to tall boxes; the rest is rest_n images of rest_d planes.  few: all in boxes of few tiles instead
-// (conv_row_few.hip)
-struct RowPlan { RowShape shape; RowBox box; long long wide_groups; int tall_planes, rest_n, rest_d; bool few; double us; };
+// tall_planes: output planes, images in 2-D, that go to tall boxes; the rest is rest_n images of rest_d planes.  few: the workgroups
+// where all goes in boxes of few tiles instead (conv_row_few.hip), else 0
+struct RowPlan { RowShape shape; RowBox box; long long wide_groups; int tall_planes, rest_n, rest_d, few; double us; };
 
 //
 // How long a launch of each takes, in units of a full round of the wide shape, fitted to 330 layers drawn over 1 to 64 images, 32 to 512 channels and
@@ -601,7 +601,7 @@ RowPlan make_row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int 
   const int steps = ceil_div(C, 32);
   RowPlan best = make_row_shape(N, oD, oH, nW, kd, kh, K, steps);
   best.rest_n = N; best.rest_d = oD;
-  best.few = row_few_pays((long long)N * oD, oH, nW, kd, kh, K, C, copied);
+  best.few = row_few_workgroups((long long)N * oD, oH, nW, kd, kh, K, C, copied);
   if (kh != 3 || best.few) return best;
   const double box_us = 2.1 * 2 * steps * kd + 10.5;
   // Tall boxes read padded rows.  What their copy takes between two layers that differ by it alone, over 109 layers: tall boxes and the others are
@@ -805,14 +805,15 @@ bool row_reads_padded(const wc_conv_desc* d) {
 
 static bool takes_few(const RowPlan& plan) {
   const int force = test_gemm_config();
-  return force == 30 || (plan.few && force != 21 && (force < 16 || force > 19));
+  return force == 30 || (plan.few > 0 && force != 21 && (force < 16 || force > 19));
 }
 
 // Whether the layer's one kernel takes this filter as it is, so that nothing has to be transformed before it
 bool row_takes_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5]) {
   if (!row_conv_fits(d) || d->kernel[1] != 3 || !row_few_takes_filter(d, w, w_strides)) return false;
-  return takes_few(row_plan(d->N, d->in[0] + 2 * d->pad[0] - d->kernel[0] + 1, d->in[1] + 2 * d->pad[1] - 2, ceil_div(d->in[2] + 2 * d->pad[2] - 2, 4), d->kernel[0], 3,
-                            d->K, d->C));
+  const RowPlan plan = row_plan(d->N, d->in[0] + 2 * d->pad[0] - d->kernel[0] + 1, d->in[1] + 2 * d->pad[1] - 2, ceil_div(d->in[2] + 2 * d->pad[2] - 2, 4), d->kernel[0], 3,
+                                d->K, d->C);
+  return takes_few(plan) && (test_gemm_config() == 30 || row_few_filter_pays(d, plan.few));
 }
 
 // x (N, D, H, W, x_row) channel-last: x_row is C, where row_reads_padded allows it, or C rounded up to 8 (zeros beyond C).  Rows of whole 16

@@ -57,7 +57,7 @@ constexpr int kPartRow = 20, kPart = 16 * kPartRow;
 // FW, for 3x3 layers whose filter is new to every call (training, the functions): a launch of its own for the transform costs the host 3 us and the
 // chain as much, where all such a layer takes is 4 to 9.  A lane's fragments are 8 channels of an output channel: 144 bytes of w
 // where U is 288, and some 250 vector instructions an item.  The numbers are row_filter_kernel's.  us of a call, two launches | one, fp16:
-// N=24 96 -> 96, 9x7 10.2 | 6.9, N=1 96 -> 64, 28x28 10.3 | 7.1, 256 -> 256, 14x14 15.0 | 9.0, 512 -> 512, 7x7 22.5 | 17.1.
+// N=24 96 -> 96, 9x7 9.5 | 6.5, N=1 96 -> 64, 28x28 9.8 | 6.4, 256 -> 256, 14x14 11.2 | 10.8, 512 -> 512, 7x7 20.1 | 18.1 (where not: row_few_filter_pays).
 //
 // SLOTS: rows of LDS for a box's input.  RC: row taps whose filter fragments are in registers at a time.  ANY: as in conv_row.hip
 // ONE: no pair has more than one item.  7x7 with more: two sets of 12 fragments of input leave 2 of 14 row taps room (all seven of a half spilled 7 to 11
@@ -320,33 +320,47 @@ RowBox few_box(int planes, int oH, int nW, int kh) { return choose_box(planes, 1
 
 }  // namespace
 
-// Where all workgroups are on the chip at once, at most three to a CU.  Of 600 layers drawn over 1 to 32 images (3-D: 8), 32 to 512 channels (128) and 7 to 56
+// The workgroups of the launch where all are on the chip at once, at most three to a CU; else 0.  Of 600 layers drawn over 1 to 32 images (3-D: 8), 32 to 512 channels (128) and 7 to 56
 // rows, at most 2000 of these workgroups, the launch takes 0.80 of the time of the other shapes' choice in the mean so, 1.02 of it where a few are
 // left for a second round; the faster of the two for each would be 0.80 as well.  us, other shapes | this, fp16 and bf16, launches in a row: N=1 512 -> 512, 7x7 12.2 | 9.5, 256 -> 256,
 // 14x14 9.5 | 6.3, N=4 9.8 | 6.5, N=8 (two rounds) 9.8 | 11.2, N=1 160 -> 160, 28x28 9.4 | 5.5, N=4 64 -> 96, 24x24 6.6 | 4.3, N=4 384 -> 288, 12x12 11.7 | 8.6,
 // 5x5 N=9 160 -> 96, 10x10 10.0 | 5.8, 7x7 N=2 119 -> 391, 15x13 13.0 | 8.9, 3-D N=1 64 -> 64, 4x14x14 8.1 | 5.6; more to a CU: N=25 32 -> 64, 31x31 6.0 | 7.4.
-bool row_few_pays(long long planes, int oH, int nW, int kd, int kh, int K, int C, bool padded) {
+int row_few_workgroups(long long planes, int oH, int nW, int kd, int kh, int K, int C, bool padded) {
   const int groups = few_groups(K), items = ceil_div(C, 32) * kd;
-  if (planes * oH * nW > 16ll * 3 * kCus * 4) return false;
+  if (planes * oH * nW > 16ll * 3 * kCus * 4) return 0;
   const bool one = items <= few_shares(kh, true), any = C % 8 != 0 && !padded;
   const int pairs = few_pairs(items, kh);
   // the wavefronts that the registers let a CU have, and the workgroups of LDS
   const int waves = !one ? 8 : kh == 7 ? (any ? 12 : 16) : any ? 16 : kh == 5 ? 20 : 24;
   const int resident = std::max(1, std::min({3, 160 * 1024 / (pairs * 6 * few_slots(kh) * kRowPitch), waves / (2 * pairs)}));
-  return few_box((int)planes, oH, nW, kh).boxes * groups <= (long long)resident * kCus;
+  const long long workgroups = few_box((int)planes, oH, nW, kh).boxes * groups;
+  return workgroups <= (long long)resident * kCus ? (int)workgroups : 0;
 }
 
 // How the kernel can take the filter as it is (kTransformed: not)
 static FewFilter few_filter(const wc_conv_desc* d, const void* w, const int64_t s[5]) {
   if (d->kernel[0] != 1 || d->kernel[1] != 3 || d->kernel[2] != 3 || d->C % 8 || (s[4] != 1 && s[4] != -1) || s[3] != 3 * s[4] || (reinterpret_cast<uintptr_t>(w) & 1)) return kTransformed;
   if (s[4] == 1 && s[1] == 9 && s[0] % 8 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0) return kByBlock;
-  // Sixteen loads of scattered channels an item instead of nine: ahead where the reduction has an item to a pair (input gradients, us, two launches | one, 256 -> 256,
-  // 14x14 14.0 | 10.0, N=24 96 -> 96, 9x7 10.3 | 7.9), behind with more (512 -> 512, 7x7 20.2 | 20.4, N=2 416 -> 224, 19x17 16.8 | 17.5) and with planes of
+  // Sixteen loads of scattered channels an item instead of nine: ahead where the reduction has an item to a pair (input gradients, us of a call, two launches | one, 256 -> 256,
+  // 14x14 13.2 | 11.9, N=24 96 -> 96, 9x7 11.9 | 8.7), behind with more (512 -> 512, 7x7 20.2 | 20.4, N=2 416 -> 224, 19x17 16.8 | 17.5) and with planes of
   // taps (128 -> 128, 3x9x9 14.6 | 17.2, forward 15.8 | 26.6)
   if (ceil_div(d->C, 32) > few_shares(3, true)) return kTransformed;
   return s[4] == 1 ? kTaps : kTapsBack;
 }
 bool row_few_takes_filter(const wc_conv_desc* d, const void* w, const int64_t s[5]) { return few_filter(d, w, s) != kTransformed; }
+
+// Every workgroup transforms the filter that it takes, every box of a channel group anew, and a CU does so one item after the other: one launch is the
+// faster call where a CU has at most eight items of it.  Of 93 layers, us of a call, two launches | one (the GPU's part of it): three items, up to two workgroups a CU 9.7 | 8.8 (8.1 | 8.4),
+// three 10.0 | 11.8 (9.0 | 11.4); four 9.8 | 9.6 and 10.8 | 13.6; five, one 9.8 | 7.8, two 11.1 | 12.8; eight, one 10.7 | 9.8; one and two items are ahead with three
+// workgroups a CU as well, 9.8 | 6.9 and 9.8 | 8.2.
+// With more than an item to a pair the time goes by C and that of the two launches by the filter, C K.  Of 106 layers: 288 -> 256 12.0 | 12.7, 320 12.7 | 12.4, 384 -> 256
+// 14.3 | 14.8, 320 15.0 | 14.8, 448 -> 224 15.2 | 16.1, 384 16.8 | 16.4, 512 -> 128 14.5 | 18.2, 320 18.0 | 18.7, 512 19.9 | 18.6, 640 -> 384 21.1 | 22.0, 512 22.3 | 21.8, 768 -> 448
+// 24.9 | 25.7, 640 26.9 | 25.8, 1024 -> 64 21.6 | 33.1, 640 32.8 | 32.6.
+bool row_few_filter_pays(const wc_conv_desc* d, int workgroups) {
+  const int items = ceil_div(d->C, 32);
+  if (items > few_shares(3, true)) return d->K >= 320 && 4 * d->K >= 3 * d->C;
+  return ceil_div(workgroups, kCus) * items <= 8;
+}
 
 // Images n_images from x on; x as row_conv takes it.  U null: the filter is w
 int row_few_conv(const wc_conv_desc* d, const void* x, int x_row, int n_images, const void* U, const void* w, const int64_t* w_strides, const void* bias, void* y,
