@@ -146,12 +146,12 @@ __global__ __launch_bounds__(THREADS) void row_few_kernel(FewArgs a) {
   // R == RC: two sets, the next item's comes while this one's is multiplied
   constexpr int SETS = R == RC && !ONE && FW == kTransformed ? 2 : 1;
   u32x4 uf[SETS][RC][3];
-  auto load_u = [&](auto to_c, int item, int part, int from, int to_row) {
+  auto load_u = [&](auto to_c, int item, int part) {
     constexpr int to = decltype(to_c)::value % SETS;
     const int rd = item / a.steps, step = item - rd * a.steps;
     const int at = u_base + ((step * a.kd + rd) * R + part * RC) * 2 * 6144;
 #pragma unroll
-    for (int r = from; r < to_row; ++r)
+    for (int r = 0; r < RC; ++r)
 #pragma unroll
       for (int t = 0; t < 3; ++t) uf[to][r][t] = __builtin_amdgcn_raw_buffer_load_b128(udesc, u_lane + t * 1024, at + r * 2 * 6144, 0);
   };
@@ -224,7 +224,7 @@ __global__ __launch_bounds__(THREADS) void row_few_kernel(FewArgs a) {
 #pragma unroll
   for (int t = 0; t < 3; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   load_x(ic<0>{}, share);
-  if constexpr (FW == kTransformed) load_u(ic<0>{}, share, 0, 0, RC);
+  if constexpr (FW == kTransformed) load_u(ic<0>{}, share, 0);
   else load_w(share);
   if constexpr (!ONE) {
     if (share + a.shares < a.items) load_x(ic<1>{}, share + a.shares);
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(THREADS) void row_few_kernel(FewArgs a) {
     if (mine) {
       store_v(cur_c, item);
       if constexpr (SETS == 2) {
-        if (more) load_u(ic<1 - cur>{}, item + a.shares, 0, 0, RC);
+        if (more) load_u(ic<1 - cur>{}, item + a.shares, 0);
       }
       if constexpr (FW != kTransformed) {
         make_u();
@@ -247,7 +247,7 @@ __global__ __launch_bounds__(THREADS) void row_few_kernel(FewArgs a) {
     if (mine) {
 #pragma unroll
       for (int part = 0; part < R / RC; ++part) {
-        if (part > 0) load_u(ic<0>{}, item, part, 0, RC);
+        if (part > 0) load_u(ic<0>{}, item, part);
 #pragma unroll
         for (int r = part * RC; r < part * RC + RC; ++r) {
           const unsigned char* const v = lds + v_offset(vo + r / KP * a.lw + r % KP, lane >> 4) + tg * 3 * TS;
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(THREADS) void row_few_kernel(FewArgs a) {
       }
       if constexpr (!ONE) {
         if constexpr (SETS == 1 && FW == kTransformed) {
-          if (more) load_u(ic<0>{}, item + a.shares, 0, 0, RC);
+          if (more) load_u(ic<0>{}, item + a.shares, 0);
         }
         if (item + 2 * a.shares < a.items) load_x(cur_c, item + 2 * a.shares);
       }
@@ -399,8 +399,10 @@ int row_few_conv(const wc_conv_desc* d, const void* x, int x_row, int n_images, 
         auto fn = a.tail ? &row_few_kernel<T, KH, SLOTS, RC, THREADS, ONE, true, kTransformed> : &row_few_kernel<T, KH, SLOTS, RC, THREADS, ONE, false, kTransformed>;
         if constexpr (KH == 3) {
           if (how == kByBlock) fn = &row_few_kernel<T, KH, SLOTS, RC, THREADS, ONE, false, kByBlock>;
-          else if (how == kTaps) fn = &row_few_kernel<T, KH, SLOTS, RC, THREADS, ONE, false, kTaps>;
-          else if (how == kTapsBack) fn = &row_few_kernel<T, KH, SLOTS, RC, THREADS, ONE, false, kTapsBack>;
+          if constexpr (ONE) {                // scattered taps have an item to a pair (few_filter)
+            if (how == kTaps) fn = &row_few_kernel<T, KH, SLOTS, RC, THREADS, ONE, false, kTaps>;
+            else if (how == kTapsBack) fn = &row_few_kernel<T, KH, SLOTS, RC, THREADS, ONE, false, kTapsBack>;
+          }
         }
         constexpr int bytes = 6 * SLOTS * kRowPitch;          // of a pair
         if (const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), SHARES * bytes)) return rc;

@@ -32,7 +32,7 @@ def kernels(tmp_path_factory):
         if name and "private_segment_fixed_size" in entry:
             key = (name[1],) + tuple(int(v) for v in name.groups()[1:])
             found[key] = {k: int(v) for k, v in re.findall(r"\.(vgpr_count|private_segment_fixed_size|vgpr_spill_count): +(\d+)", entry)}
-    assert len(found) >= 32
+    assert len(found) == 32          # 3x3: eight of each type, 5x5 and 7x7 four
     return found
 
 
