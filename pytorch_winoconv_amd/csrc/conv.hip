@@ -240,9 +240,10 @@ int wc_conv_u_elems(const wc_conv_desc* d, size_t* elems) {
 
 int wc_conv_takes_filter(const wc_conv_desc* d, const void* w, const int64_t w_strides[5], int* takes) {
   WC_CHECK_ARG(w && w_strides && takes, "wc_conv_takes_filter: null pointer");
-  Layout L;
-  if (int rc = make_layout(d, &L)) return rc;
-  *takes = L.row && row_takes_filter(d, w, w_strides);
+  int out[3], grid[3];
+  if (int rc = wc_conv_out_dims(d, out, grid)) return rc;          // (a program may ask in every pass: no layout for the answer)
+  if (d->row == 1 && !row_conv_fits(d)) return fail(WC_ERR_UNSUPPORTED, "row form: 16-bit types, stride 1, 3x3, 3x3x3, 5x5 or 7x7 kernels, x below 1 GiB");
+  *takes = d->row == 1 && row_takes_filter(d, w, w_strides);
   return WC_OK;
 }
 

@@ -327,14 +327,16 @@ RowBox few_box(int planes, int oH, int nW, int kh) { return choose_box(planes, 1
 // 5x5 N=9 160 -> 96, 10x10 10.0 | 5.8, 7x7 N=2 119 -> 391, 15x13 13.0 | 8.9, 3-D N=1 64 -> 64, 4x14x14 8.1 | 5.6; more to a CU: N=25 32 -> 64, 31x31 6.0 | 7.4.
 int row_few_workgroups(long long planes, int oH, int nW, int kd, int kh, int K, int C, bool padded) {
   const int groups = few_groups(K), items = ceil_div(C, 32) * kd;
-  if (planes * oH * nW > 16ll * 3 * kCus * 4) return 0;
   const bool one = items <= few_shares(kh, true), any = C % 8 != 0 && !padded;
   const int pairs = few_pairs(items, kh);
   // the wavefronts that the registers let a CU have, and the workgroups of LDS
   const int waves = !one ? 8 : kh == 7 ? (any ? 12 : 16) : any ? 16 : kh == 5 ? 20 : 24;
   const int resident = std::max(1, std::min({3, 160 * 1024 / (pairs * 6 * few_slots(kh) * kRowPitch), waves / (2 * pairs)}));
+  const long long most = (long long)resident * kCus;
+  // a box holds sixteen tiles at most, which spares most layers the search for it (a plan of N=64 256 -> 256, 14x14 4.2 us with it, 3.8 without)
+  if (ceil_div_ll(planes * oH * nW, 16) * groups > most) return 0;
   const long long workgroups = few_box((int)planes, oH, nW, kh).boxes * groups;
-  return workgroups <= (long long)resident * kCus ? (int)workgroups : 0;
+  return workgroups <= most ? (int)workgroups : 0;
 }
 
 // How the kernel can take the filter as it is (kTransformed: not)

@@ -923,7 +923,6 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
   size_t bytes = 0, u_elems = 0;
   int nd, stride, m;
   std::vector<int> pads;
-  std::vector<int64_t> taken_strides;               // of weights that the layer's kernel takes as they are; empty: none
   std::shared_ptr<KeptFilter> filter;               // null: no pass yet
 
   // None where the layer copies its input first.  `kept`: the filter of the module's last pass, taken where it is this one's
@@ -941,11 +940,6 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
     check(wc_conv_u_elems(&p->d, &p->u_elems));
     if (kept && kept->suits(p->form(), x.scalar_type(), x.device())) p->filter = kept;
     else if (kept && kept->holds(weight)) p->filter = std::make_shared<KeptFilter>(weight, p->form());      // known, its filter not made for this plan
-    int64_t s[5];
-    int takes = 0;
-    strides_of(weight, s);
-    check(wc_conv_takes_filter(&p->d, weight.data_ptr(), s, &takes));
-    if (takes) p->taken_strides = weight.strides().vec();
     int out[3], grid[3];
     check(wc_conv_out_dims(&p->d, out, grid));
     check(wc_conv_workspace_bytes(&p->d, &p->bytes));
@@ -991,6 +985,16 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
   py::object call(const at::Tensor& x, const at::Tensor& weight, const std::optional<at::Tensor>& bias) const;
 
  private:
+  // whether the layer's kernel takes this weight, or a copy of it in x's type, as it is
+  bool takes(const at::Tensor& weight) const {
+    int yes = 0;
+    if (d.row == 1) {
+      int64_t s[5];
+      strides_of(weight, s);
+      check(wc_conv_takes_filter(&d, weight.data_ptr(), s, &yes));
+    }
+    return yes != 0;
+  }
   static bool misaligned(const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) != 0; }
   bool fits(const at::Tensor& x, const at::Tensor& weight, const std::optional<at::Tensor>& bias) const {
     return plain(x) && plain(weight) && (!bias || plain(*bias)) && x.scalar_type() == x_type && x.sizes() == at::IntArrayRef(sizes) &&
@@ -1076,7 +1080,7 @@ py::object LayerPlan::call(const at::Tensor& x, const at::Tensor& weight, const 
     // After a pass with a gradient of its own a weight is likely another one: nothing to make where the kernel takes the filter as it is.  A frozen
     // weight stays, and one that a second pass finds as it was (gradients of several passes added up, passes whose gradients nobody asks for) may
     // stay: their filters are made and kept.  us of a pass, fp16, x needs a gradient: 512 -> 512, 7x7, the filter taken 18.1, kept 9.5, 256 -> 256, 14x14 10.9 | 8.7.
-    const bool taken = trained && !known && !taken_strides.empty() && weight.strides() == at::IntArrayRef(taken_strides);
+    const bool taken = trained && !known && takes(weight);
     const bool anew = !o.U.defined() && !taken;
     if (anew || (taken && !captured)) {
       renewed = std::make_shared<LayerPlan>(*this);
