@@ -8,7 +8,8 @@ decomposition (output tile 4 in 2-D, 2 in 3-D); grouped, dilated, stride > 2 or 
 convolutions, which the Winograd algorithm here does not cover, go to
 torch.nn.functional.conv2d/conv3d on the same device like the reference does (conv.py:326-332).
 There is no CPU path: a CPU tensor, or a missing HIP library, raises.  The transformed filter
-is cached and recomputed only when the weight changes.
+is cached and recomputed only when the weight changes; a graph that is captured without gradients, or of a frozen
+weight, reads the filter as it was then.
 """
 import torch
 from torch import nn
@@ -217,7 +218,8 @@ class _WinoConvNd(nn.Module):
         if U is not None and weight.requires_grad and torch.is_grad_enabled() and torch.cuda.is_current_stream_capturing():
             U = None
         if U is None:
-            cache = ((x.dtype, form), engine.KeptFilter(weight, form))
+            last, cache = cache, ((x.dtype, form), engine.KeptFilter(weight, form))
+            cache[1].follows(last and last[1])
         # (to() and detach() that change nothing still cost a microsecond each of a 12 us call)
         w = weight if weight.dtype == x.dtype else weight.detach().to(x.dtype)
         if U is None:

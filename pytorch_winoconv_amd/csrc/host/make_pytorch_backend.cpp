@@ -20,6 +20,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <optional>
 #include <sstream>
@@ -735,6 +736,9 @@ class KeptFilter {
     captured_ = capturing(stream_);
   }
 
+  // In the place of `last`: filters that graphs were captured with are kept for as long as those may be replayed, which is the module's life
+  void follows(const std::shared_ptr<KeptFilter>& last) { before_ = !last || last->in_graph_ ? last : last->before_; }
+
   // made inside a capture: there when the graph is replayed, and only then.  Not for other passes
   bool captured() const { return captured_; }
 
@@ -755,9 +759,11 @@ class KeptFilter {
   at::Tensor on_stream() const {
     if (!U_.defined()) return U_;
     void* const now = stream_of(U_);
-    if (now == stream_) return U_;
+    const bool graph = capturing(now);
+    if (graph) in_graph_ = true;
+    if (now == stream_ || graph) return U_;
     const std::lock_guard<std::mutex> lock(mutex_);
-    if (std::find(ordered_.begin(), ordered_.end(), now) != ordered_.end() || capturing(now)) return U_;
+    if (std::find(ordered_.begin(), ordered_.end(), now) != ordered_.end()) return U_;
     if (capturing(stream_)) return at::Tensor();
     const c10::DeviceGuard device(U_.device());
     hipEvent_t event;
@@ -784,6 +790,8 @@ class KeptFilter {
   at::Tensor U_;
   void* stream_ = nullptr;
   bool captured_ = false;
+  mutable std::atomic<bool> in_graph_{false};
+  std::shared_ptr<KeptFilter> before_;              // read by a graph
   mutable std::mutex mutex_;
   mutable std::vector<void*> ordered_;              // streams that have waited
 };
@@ -923,7 +931,7 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
   size_t bytes = 0, u_elems = 0;
   int nd, stride, m;
   std::vector<int> pads;
-  std::shared_ptr<KeptFilter> filter;               // null: no pass yet
+  std::shared_ptr<KeptFilter> filter, last;         // null: no pass yet; then the one that the first pass's takes the place of
 
   // None where the layer copies its input first.  `kept`: the filter of the module's last pass, taken where it is this one's
   static std::shared_ptr<LayerPlan> make(const at::Tensor& x, const at::Tensor& weight, int stride, std::vector<int> pads, int m,
@@ -939,7 +947,8 @@ class LayerPlan : public std::enable_shared_from_this<LayerPlan> {
     p->d.x_layout = !last;
     check(wc_conv_u_elems(&p->d, &p->u_elems));
     if (kept && kept->suits(p->form(), x.scalar_type(), x.device())) p->filter = kept;
-    else if (kept && kept->holds(weight)) p->filter = std::make_shared<KeptFilter>(weight, p->form());      // known, its filter not made for this plan
+    else if (kept && kept->holds(weight)) (p->filter = std::make_shared<KeptFilter>(weight, p->form()))->follows(kept);      // known, its filter not made for this plan
+    else p->last = kept;
     int out[3], grid[3];
     check(wc_conv_out_dims(&p->d, out, grid));
     check(wc_conv_workspace_bytes(&p->d, &p->bytes));
@@ -1085,6 +1094,8 @@ py::object LayerPlan::call(const at::Tensor& x, const at::Tensor& weight, const 
     if (anew || (taken && !captured)) {
       renewed = std::make_shared<LayerPlan>(*this);
       renewed->filter = std::make_shared<KeptFilter>(weight, form());
+      renewed->filter->follows(filter ? filter : last);
+      renewed->last = nullptr;
     }
     const bool cast_w = (grad || anew || taken) && w_type != x_type, cast_b = bias && bias->scalar_type() != x_type;
     if (cast_w || cast_b) {
@@ -1155,6 +1166,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   py::class_<KeptFilter, std::shared_ptr<KeptFilter>>(m, "KeptFilter")
       .def(py::init<const at::Tensor&, const PlanForm&>(), py::arg("weight"), py::arg("form"))
       .def("made", &KeptFilter::made, py::arg("U"))
+      .def("follows", &KeptFilter::follows, py::arg("last"))
       .def_property_readonly("captured", &KeptFilter::captured)
       .def("holds", &KeptFilter::holds, py::arg("weight"))
       .def("on_stream", [](const KeptFilter& f) { return or_none(f.on_stream()); });

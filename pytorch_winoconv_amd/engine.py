@@ -566,6 +566,11 @@ class _KeptFilter:
         # new tensors in every pass (functional_call, parametrizations) come to lie where the last one did
         self._held = self._identity(weight)
         self._ordered = set()
+        self._in_graph, self._before = False, None
+
+    def follows(self, last):
+        """In the place of `last`: filters that graphs were captured with are kept for as long as those may be replayed, which is the module's life."""
+        self._before = last if last is None or last._in_graph else last._before
 
     @staticmethod
     def _identity(weight):
@@ -579,7 +584,9 @@ class _KeptFilter:
 
     def on_stream(self):
         now = torch.cuda.current_stream(self._U.device)
-        if now != self._stream and now not in self._ordered and not torch.cuda.is_current_stream_capturing():
+        if torch.cuda.is_current_stream_capturing():
+            self._in_graph = True
+        elif now != self._stream and now not in self._ordered:
             now.wait_stream(self._stream)
             self._U.record_stream(now)
             self._ordered.add(now)

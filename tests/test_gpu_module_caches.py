@@ -180,6 +180,30 @@ def test_a_captured_pass_of_a_trained_weight(dev, passes, own, c, k, taps):
         assert torch.equal(y, layer(x))
 
 
+def test_a_filter_that_a_graph_reads_stays(dev, passes):
+    """The module goes on with another type's and another weight's filter; the captured one's memory is not given to others."""
+    layer = pkg.WinoConv2d(64, 96, 5, padding=2, device=dev).requires_grad_(False)
+    x, other = _input(dev, 2, 64, 15, 14), _input(dev, 2, 64, 15, 14, dtype=torch.float32)
+    for _ in range(passes):
+        want = layer(x)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = layer(x)
+    elems = engine.transform_filter(layer.weight.half(), x.shape, 1, 2, 4, row=True).numel()
+    for change in (False, True):
+        if change:
+            layer.weight.mul_(-1)
+        _close(layer(other), layer, other)
+        _close(layer(x), layer, x)
+        _close(layer(other), layer, other)
+        taken = [torch.full((elems,), 7.0, dtype=torch.float16, device=dev) for _ in range(16)]
+        for _ in range(2):
+            y.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, want) and len(taken) == 16
+
+
 @pytest.mark.parametrize("own", [torch.float16, torch.float32])
 def test_shapes_types_and_memory_orders_in_turn(dev, passes, own):
     """Each pass with the filter of its own form: batches on either side of the direct form's line, images, types and orders in memory."""
