@@ -1,6 +1,7 @@
 // Host entry of the input transform: picks the kernel of each piece and launches it.
 #include "filter_transform_impl.h"
 #include "input_transform_impl.h"
+#include "transform_threads.h"
 #include <algorithm>
 
 using namespace wc;
@@ -41,9 +42,9 @@ int input_transform_impl(const wc_conv_desc* d, const wc_plan* plan, const void*
   int vec = 1;
   for (int v = want; v > 1; v /= 2)
     if (d->C % v == 0) { vec = v; break; }
-  // Small 2-D plans of several pieces, which get threads of their own below: fewer channels a thread until every CU has a workgroup.
+  // Small 2-D plans of several pieces get threads of their own below, and fewer channels each.
   // (One piece alone was slower with them: fp32 N=2 88 -> 96, 19x24 15.5 | 15.9, N=1 512 -> 512, 7x7 29.6 | 31.6.)
-  while (plan->n_pieces > 1 && flat && !shared && vec > 1 && P * (Cp / vec) * plan->n_pieces < 256 * kCus) vec /= 2;
+  if (plan->n_pieces > 1 && flat && !shared) vec = input_channels(vec, P, Cp, plan->n_pieces, stacked, d->dtype == WC_F32, plan->m[1]);
   InArgs a;
   a.x = x; a.V = V;
   a.D = d->in[0]; a.H = d->in[1]; a.W = d->in[2]; a.C = d->C; a.Cp = row;

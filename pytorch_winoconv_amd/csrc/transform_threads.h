@@ -1,0 +1,18 @@
+// How the transforms of 2-D plans of several pieces share their work out over threads (input_transform.hip).  Host code without HIP.
+#pragma once
+
+namespace wc {
+
+// Channels a thread of the input transform, of `vec` at most: fewer until every CU has a workgroup of its own (65536 threads over tiles, rows of Cp
+// channels and pieces).  fp32 on tile 2, stacked, where a thread's channels are 16 bytes and the pieces write columns of one row, gains up to half as many threads only:
+// us, all four channels | line at 65536 | 32768, 5x5 stride 2, 243 tiles of 16 channels 4.02 | 3.60 | 3.60, 464 of 120 6.31 | 6.66 | 6.31, 425 of 88 5.38 | 5.99 | 5.38,
+// 500 of 152 7.21 with any.  Over 364 launches of 16 to 380 channels the time against all channels a thread, mean and worst: stacked, fp32 on tile 2 0.980 and 1.11 | 0.978 and
+// 1.00; at 65536 fp16 on tile 2 0.903 and 1.00, fp32 on tile 4 0.928 and 1.00, fp16 and bf16 on tile 4 0.964 and 0.960 and 1.03 (0.966, 0.956 and 1.00 at 32768).
+// Against one channel for all as well, not stacked: 16-bit types 1.004 to 1.009 and 1.08 of the faster, fp32 1.009 and 1.045, 1.10 and 1.16.
+inline int input_channels(int vec, long long tiles, int Cp, int n_pieces, bool stacked, bool f32, int m) {
+  const long long enough = stacked && f32 && m == 2 ? 32768 : 65536;
+  while (vec > 1 && tiles * (Cp / vec) * n_pieces < enough) vec /= 2;
+  return vec;
+}
+
+}  // namespace wc
