@@ -87,14 +87,11 @@ int input_transform_impl(const wc_conv_desc* d, const wc_plan* plan, const void*
     small_taps = pc.r[1] >= 1 && pc.r[1] <= 3 && pc.r[2] >= 1 && pc.r[2] <= 3 && pc.tap0[1] < 16 && pc.tap0[2] < 16;
   }
   if (small_taps && plan->m[1] == plan->m[2]) {
-    // Small problems give every piece its own threads (one thread per tile and
-    // channel group, looping over the pieces, then leaves most of the chip idle: 2.2x faster at
-    // N=8, C=24, 56x56, 7x7); large ones keep the loop, which reads each window from cache once per
-    // piece and measured 7-30 % faster there.  Stacked plans have the pieces beside the channels, others in the grid's second
+    // Small problems give every piece its own threads.  Stacked plans have the pieces beside the channels, others in the grid's second
     // dimension.  fp32 without stacking, us of a layer with its filter, in a loop | apart, and both transforms with fewer channels a thread:
     // 7x7 on tile 2 and 4, N=5 88 -> 96, 14x14 44.1 | 32.4 and 60.5 | 38.5, N=2 32 -> 64, 28x28 38.0 | 25.4 and 50.8 | 29.3, N=8 64 -> 64,
-    // 56x56 148 | 140 and 91 | 81, N=32 128 -> 128, 56x56 (too large for it) 1119 and 778; 5x5 on tile 4, N=4 480 -> 128, 21x28 64.1 | 56.4.
-    const bool apart = a.total < 512 * 1024, per_piece_threads = stacked && apart;
+    // 56x56 148 | 140 and 91 | 81; 5x5 on tile 4, N=4 480 -> 128, 21x28 64.1 | 56.4.
+    const bool apart = pieces_apart(a.total, plan->n_pieces, stacked, d->dtype == WC_F32, plan->m[1]), per_piece_threads = stacked && apart;
     InPiecesKernel fn = per_piece_threads ? pick_in_2d_stacked(d->dtype, plan->m[1], vec)
                                           : pick_in_2d_pieces(d->dtype, plan->m[1], vec);
     if (fn) {

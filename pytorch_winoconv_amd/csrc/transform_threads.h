@@ -15,4 +15,15 @@ inline int input_channels(int vec, long long tiles, int Cp, int n_pieces, bool s
   return vec;
 }
 
+// Whether every piece gets threads of its own, of `threads` over tiles and channels: large launches keep one thread for all pieces of a tile, which reads each
+// window from cache once per piece.  Stacked plans: 2.2 times as fast apart at N=8, 24 channels, 56x56, 7x7, in the loop 7 to 30 % the faster further up.  Others, over
+// 240 launches of 30 to 530 thousand threads, apart against the loop: nine pieces 0.62 to 1.07, 0.83 in the mean of 16-bit types on tile 4 and 0.93 of fp32 on
+// tile 2; four of fp32 0.90 in the mean on tile 4, 0.98 on tile 2; four of 16-bit types 0.69 at 70 thousand and 1.00 to 1.12 from 290 thousand on on tile 4,
+// 0.71 at 30 and 1.05 to 1.13 from 185 thousand on on tile 2.  us, fp16 5x5, loop | apart: tile 2, N=13 48 channels, 78x78 26.4 | 25.3, N=9 160, 73x73 35.4 | 39.6; tile 4, N=51 136, 25x25
+// 28.0 | 24.0, N=9 336, 68x68 46.9 | 52.5.
+inline bool pieces_apart(long long threads, int n_pieces, bool stacked, bool f32, int m) {
+  const int thousands = stacked || f32 || n_pieces > 4 ? 512 : m == 2 ? 160 : 288;
+  return threads < thousands * 1024ll;
+}
+
 }  // namespace wc

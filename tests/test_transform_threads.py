@@ -30,3 +30,13 @@ def test_channels_of_an_input_transform(tmp_path):
         ((1, 4, 32, 4, True, True, 2), 1), ((8, 100000, 512, 9, True, False, 2), 8),
     ]
     assert _rows(tmp_path, "input_channels", [c[0] for c in cases]) == [c[1] for c in cases]
+
+
+def test_pieces_of_an_input_transform_apart(tmp_path):
+    """(threads, pieces, stacked, fp32, tile) -> threads of its own for every piece"""
+    cases = [
+        ((158184, 4, False, False, 2), 1), ((186984, 4, False, False, 2), 0), ((258048, 4, False, False, 2), 0), ((199920, 4, False, False, 4), 1),
+        ((368640, 4, False, False, 4), 0), ((457776, 4, False, False, 4), 0), ((258720, 9, False, False, 2), 1), ((460800, 9, False, False, 4), 1),
+        ((492840, 4, False, True, 2), 1), ((460800, 9, False, True, 4), 1), ((802816, 9, False, True, 2), 0), ((500000, 4, True, False, 2), 1), ((600000, 9, True, True, 4), 0),
+    ]
+    assert _rows(tmp_path, "pieces_apart", [c[0] for c in cases]) == [c[1] for c in cases]
