@@ -13,6 +13,7 @@
 // every piece and sums the pieces in registers; and a streaming one for 3-D DWM plans, where
 // each loaded tile row is transformed along the width and then scattered into the m^d
 // accumulators with coefficients from a constant table.
+#include "transform_threads.h"
 #include "wc_transform.h"
 #include <type_traits>
 
@@ -367,9 +368,8 @@ extern "C" int wc_output_transform(const wc_conv_desc* d, const wc_plan* plan_in
   WC_CHECK_ARG(plan->n_pieces > 0 && plan->n_pieces <= WC_MAX_PIECES, "wc_output_transform: bad plan");
   const int ldm = wc_padded_channels8(d->K);
   const long long P = (long long)n_images * grid[0] * grid[1] * grid[2];
-  // Small 2-D layers: a channel a thread, so that more CUs have a workgroup.  fp32, F(4,3), us of a layer: N=28 128 -> 64, 12x12 18.9 | 18.3,
-  // N=2 88 -> 96, 19x24 15.5 | 14.8, N=4 256 -> 256, 14x14 20.9 | 20.2
-  const bool small = plan->m[0] == 1 && plan->m[1] == 4 && P * (d->K / 2) < 256 * kCus;
+  // small 2-D layers, on tile 4 of two channels a thread, here, on tile 2 where the pieces are known
+  const bool f32 = d->dtype == WC_F32, small = plan->m[0] == 1 && plan->m[1] == 4 && output_one_channel(P, d->K, 2, plan->n_pieces, f32, 4);
   const int vec = d->K % 4 == 0 && !small ? 4 : 1;
   OutArgs a;
   a.M = M; a.bias = bias; a.y = y;
@@ -419,7 +419,7 @@ extern "C" int wc_output_transform(const wc_conv_desc* d, const wc_plan* plan_in
   if (flat) {
     // 2-D plans: compile-time body per piece; F(4,r) tiles use 2 channels per thread
     int v = (tile4 && vec == 4) ? 2 : vec;
-    if (P * (d->K / v) < 256 * kCus) v = 1;           // as above
+    if (output_one_channel(P, d->K, v, plan->n_pieces, f32, plan->m[1])) v = 1;
     g.o.n_kvec = d->K / v;
     g.o.total = P * g.o.n_kvec;
     g.o.per_xcd = (int)ceil_div_ll(ceil_div_ll(g.o.total, 256), kXcds);

@@ -1,4 +1,4 @@
-// How the transforms of 2-D plans of several pieces share their work out over threads (input_transform.hip).  Host code without HIP.
+// How the transforms of 2-D plans share their work out over threads (input_transform.hip, output_transform.hip).  Host code without HIP.
 #pragma once
 
 namespace wc {
@@ -24,6 +24,15 @@ inline int input_channels(int vec, long long tiles, int Cp, int n_pieces, bool s
 inline bool pieces_apart(long long threads, int n_pieces, bool stacked, bool f32, int m) {
   const int thousands = stacked || f32 || n_pieces > 4 ? 512 : m == 2 ? 160 : 288;
   return threads < thousands * 1024ll;
+}
+
+// Whether a thread of the output transform takes one channel instead of `vec`, so that more CUs have a workgroup: up to 65536 threads over tiles and groups
+// of vec channels, where a thread gathers several pieces or in fp32 on tile 4, else up to half as many.  Of 400 launches of 16 to 380 output channels, time against vec
+// channels a thread, mean and worst, line at 65536 | 32768: one piece, fp16 on tile 4 0.968 and 1.043 | 0.966 and 1.00, on tile 2 0.983 and 1.035 |
+// 0.982 and 1.013, fp32 on tile 2 1.003 and 1.057 | 1.001 and 1.024, on tile 4 0.89 and 1.00 | 0.90 and 1.00; several 0.82 to 0.91 and 1.00 (fp32 on tile 2 once 1.05) | 0.84 to
+// 0.92 and 1.00.  us, vec channels | one: fp16 6x6 N=4 136, 54x54 5.01 | 5.27, fp32 4x4 N=3 216, 34x34 3.86 | 4.32; F(4,3) fp32 N=8 352, 9x9 5.02 | 4.24, N=8 64, 60x60 5.83 | 5.44.
+inline bool output_one_channel(long long tiles, int K, int vec, int n_pieces, bool f32, int m) {
+  return tiles * (K / vec) < (n_pieces > 1 || (f32 && m == 4) ? 65536 : 32768);
 }
 
 }  // namespace wc

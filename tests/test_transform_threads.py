@@ -40,3 +40,13 @@ def test_pieces_of_an_input_transform_apart(tmp_path):
         ((492840, 4, False, True, 2), 1), ((460800, 9, False, True, 4), 1), ((802816, 9, False, True, 2), 0), ((500000, 4, True, False, 2), 1), ((600000, 9, True, True, 4), 0),
     ]
     assert _rows(tmp_path, "pieces_apart", [c[0] for c in cases]) == [c[1] for c in cases]
+
+
+def test_channels_of_an_output_transform(tmp_path):
+    """(tiles, output channels, channels at most, pieces, fp32, tile) -> one channel a thread"""
+    cases = [
+        ((784, 136, 2, 1, False, 4), 0), ((1600, 64, 2, 1, False, 4), 0), ((480, 112, 2, 1, False, 4), 1), ((784, 136, 2, 1, True, 4), 1), ((1800, 64, 2, 1, True, 4), 1),
+        ((972, 216, 4, 1, True, 2), 0), ((972, 216, 4, 1, False, 2), 0), ((841, 64, 4, 1, False, 2), 1), ((3072, 56, 4, 4, True, 2), 1), ((2000, 40, 2, 4, False, 4), 1),
+        ((4000, 40, 2, 4, False, 4), 0), ((4000, 40, 2, 1, True, 4), 0),
+    ]
+    assert _rows(tmp_path, "output_one_channel", [c[0] for c in cases]) == [c[1] for c in cases]
