@@ -531,8 +531,8 @@ namespace {
 // channels come here in 3-D or with tile 4; with tile 2 the one-kernel F(2x2, 3x3) form takes most of them, see row_preferred.)
 enum RowShape { kRowWide, kRowHalf, kRowSmall, kRowSplit };
 // tall_planes: output planes, images in 2-D, that go to tall boxes; the rest is rest_n images of rest_d planes.  few: the workgroups
-// where all goes in boxes of few tiles instead (conv_row_few.hip), else 0
-struct RowPlan { RowShape shape; RowBox box; long long wide_groups; int tall_planes, rest_n, rest_d, few; double us; };
+// where all goes in boxes of few tiles instead (conv_row_few.hip), of few_box, else 0
+struct RowPlan { RowShape shape; RowBox box, few_box; long long wide_groups; int tall_planes, rest_n, rest_d, few; double us; };
 
 //
 // How long a launch of each takes, in units of a full round of the wide shape, fitted to 330 layers drawn over 1 to 64 images, 32 to 512 channels and
@@ -601,7 +601,7 @@ RowPlan make_row_plan(int N, int oD, int oH, int nW, int kd, int kh, int K, int 
   const int steps = ceil_div(C, 32);
   RowPlan best = make_row_shape(N, oD, oH, nW, kd, kh, K, steps);
   best.rest_n = N; best.rest_d = oD;
-  best.few = row_few_workgroups((long long)N * oD, oH, nW, kd, kh, K, C, copied);
+  best.few = row_few_workgroups((long long)N * oD, oH, nW, kd, kh, K, C, copied, &best.few_box);
   if (kh != 3 || best.few) return best;
   const double box_us = 2.1 * 2 * steps * kd + 10.5;
   // Tall boxes read padded rows.  What their copy takes between two layers that differ by it alone, over 109 layers: tall boxes and the others are
@@ -839,7 +839,7 @@ int row_conv(const wc_conv_desc* d, const void* x, int x_row, int first_image, i
   if (force >= 16 && force <= 19) { plan.shape = (RowShape)(force - 16); plan.tall_planes = 0; plan.rest_n = -1; }
   if (force == 21 && d->kernel[1] == 3) plan.tall_planes = d->N * a.oD;
   const int tall = std::min(std::max(plan.tall_planes - first_image * a.oD, 0), n_images * a.oD);
-  if (takes_few(plan)) return row_few_conv(d, x, x_row, n_images, U, w, w_strides, bias, y, stream);
+  if (takes_few(plan)) return row_few_conv(d, x, x_row, n_images, plan.few > 0 && n_images == d->N ? &plan.few_box : nullptr, U, w, w_strides, bias, y, stream);
   WC_CHECK_ARG(U, "row form: no transformed filter");
   if (tall > 0) {
     WC_CHECK_ARG(a.tail == 0, "row form: tall boxes of %d channels", x_row);

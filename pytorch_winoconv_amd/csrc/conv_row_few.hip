@@ -325,7 +325,7 @@ RowBox few_box(int planes, int oH, int nW, int kh) { return choose_box(planes, 1
 // left for a second round; the faster of the two for each would be 0.80 as well.  us, other shapes | this, fp16 and bf16, launches in a row: N=1 512 -> 512, 7x7 12.2 | 9.5, 256 -> 256,
 // 14x14 9.5 | 6.3, N=4 9.8 | 6.5, N=8 (two rounds) 9.8 | 11.2, N=1 160 -> 160, 28x28 9.4 | 5.5, N=4 64 -> 96, 24x24 6.6 | 4.3, N=4 384 -> 288, 12x12 11.7 | 8.6,
 // 5x5 N=9 160 -> 96, 10x10 10.0 | 5.8, 7x7 N=2 119 -> 391, 15x13 13.0 | 8.9, 3-D N=1 64 -> 64, 4x14x14 8.1 | 5.6; more to a CU: N=25 32 -> 64, 31x31 6.0 | 7.4.
-int row_few_workgroups(long long planes, int oH, int nW, int kd, int kh, int K, int C, bool padded) {
+int row_few_workgroups(long long planes, int oH, int nW, int kd, int kh, int K, int C, bool padded, RowBox* box) {
   const int groups = few_groups(K), items = ceil_div(C, 32) * kd;
   const bool one = items <= few_shares(kh, true), any = C % 8 != 0 && !padded;
   const int pairs = few_pairs(items, kh);
@@ -335,7 +335,8 @@ int row_few_workgroups(long long planes, int oH, int nW, int kd, int kh, int K, 
   const long long most = (long long)resident * kCus;
   // a box holds sixteen tiles at most, which spares most layers the search for it (a plan of N=64 256 -> 256, 14x14 4.2 us with it, 3.8 without)
   if (ceil_div_ll(planes * oH * nW, 16) * groups > most) return 0;
-  const long long workgroups = few_box((int)planes, oH, nW, kh).boxes * groups;
+  *box = few_box((int)planes, oH, nW, kh);
+  const long long workgroups = box->boxes * groups;
   return workgroups <= most ? (int)workgroups : 0;
 }
 
@@ -364,8 +365,9 @@ bool row_few_filter_pays(const wc_conv_desc* d, int workgroups) {
   return ceil_div(workgroups, kCus) * items <= 8;
 }
 
-// Images n_images from x on; x as row_conv takes it.  U null: the filter is w
-int row_few_conv(const wc_conv_desc* d, const void* x, int x_row, int n_images, const void* U, const void* w, const int64_t* w_strides, const void* bias, void* y,
+// Images n_images from x on; x as row_conv takes it.  box: the plan's, whose search took a call 0.2 to 0.4 us of the host; null: the images are not
+// the plan's.  U null: the filter is w
+int row_few_conv(const wc_conv_desc* d, const void* x, int x_row, int n_images, const RowBox* box, const void* U, const void* w, const int64_t* w_strides, const void* bias, void* y,
                  void* stream) {
   FewArgs a{};
   const int kh = d->kernel[1];
@@ -379,7 +381,7 @@ int row_few_conv(const wc_conv_desc* d, const void* x, int x_row, int n_images, 
   a.pd = d->pad[0]; a.ph = d->pad[1]; a.pw = d->pad[2]; a.kd = d->kernel[0];
   a.oD = a.D + 2 * a.pd - a.kd + 1; a.oH = a.H + 2 * a.ph - kh + 1; a.oW = a.W + 2 * a.pw - kh + 1;
   a.n_img = a.N * a.oD;
-  const RowBox b = few_box(a.n_img, a.oH, ceil_div(a.oW, row_outputs_of(kh)), kh);
+  const RowBox b = box ? *box : few_box(a.n_img, a.oH, ceil_div(a.oW, row_outputs_of(kh)), kh);
   a.bn = b.bn; a.bh = b.bh; a.bw = b.bw; a.n_h = b.n_h; a.n_w = b.n_w;
   a.lw = b.bw + row_pieces(kh) - 1; a.irow = b.irow;
   a.f_lw = make_fast_div(a.lw); a.f_irow = make_fast_div(a.irow); a.f_bw = make_fast_div(a.bw); a.f_bh = make_fast_div(a.bh); a.f_d = make_fast_div(a.oD);

@@ -123,12 +123,12 @@ __device__ __forceinline__ u32x4 shift_channels(u32x4 v, int by) {
 struct RowBox { int bn, bd, bh, bw, n_n, n_d, n_h, n_w, prow, irow; long long boxes; };
 RowBox choose_box(int N, int oD, int oH, int nW, int kd, int kh, int tiles, int slots);
 
-// Few tiles (conv_row_few.hip): the workgroups of the kernel where it is taken for `planes` output planes, else 0 (padded: x with channels padded to a
-// multiple of 8), and the launch with the arguments of row_conv
-int row_few_workgroups(long long planes, int oH, int nW, int kd, int kh, int K, int C, bool padded);
+// Few tiles (conv_row_few.hip): the workgroups of the kernel where it is taken for `planes` output planes, and their box, else 0 (padded: x with channels
+// padded to a multiple of 8), and the launch with the arguments of row_conv (box null: to be searched)
+int row_few_workgroups(long long planes, int oH, int nW, int kd, int kh, int K, int C, bool padded, RowBox* box);
 bool row_few_takes_filter(const wc_conv_desc* d, const void* w, const int64_t s[5]);      // whether the kernel can take it as it is, instead of U
 bool row_few_filter_pays(const wc_conv_desc* d, int workgroups);                          // and is the faster then
-int row_few_conv(const wc_conv_desc* d, const void* x, int x_row, int n_images, const void* U, const void* w, const int64_t* w_strides, const void* bias, void* y,
+int row_few_conv(const wc_conv_desc* d, const void* x, int x_row, int n_images, const RowBox* box, const void* U, const void* w, const int64_t* w_strides, const void* bias, void* y,
                  void* stream);
 
 }  // namespace wc
