@@ -500,7 +500,7 @@ int backward_weight(const wc_conv_desc* d, const void* x, const void* dy, GradOu
     return small;
   };
   // In the transform domain the bias gradient's two steps ride on the launches that read dy and that write dw, which writes it from the last
-  // chunk's sums: three launches fewer, whose host time most training steps in fp32 wait for.  us of a step, apart | so, fp32: N=28 128 -> 64, 12x12 97 | 89,
+  // chunk's sums: three launches fewer, whose host time most training steps in fp32 wait for.  us of a step, apart | so, on one machine, fp32: N=28 128 -> 64, 12x12 97 | 89,
   // N=2 96 -> 416, 44x44 127 | 120, N=1 32 -> 32, 14x14 80 | 74, stride 2, N=4 76 -> 64, 70x58 127 | 117, N=2 64 -> 49, 12x37x37 279 | 252.
   const bool stores = !L.one_tap && !L.gathered && grad_filter_stores(d, &L.plan);
   const bool beside = stores && to.db && small_taps(L.dm_plan);

@@ -486,6 +486,8 @@ __global__ __launch_bounds__(256) void row_filter_kernel(RowFilterArgs a) {
   for (int t = 0; t < 6; ++t) *reinterpret_cast<Pack<T, 2>*>(dst + t * 512) = out[t];
 }
 
+}  // namespace
+
 // Box of a workgroup: at most `tiles` tiles whose input rows, with the halo of the taps, fill at most `slots` rows of LDS;
 // the fewest boxes over the output, and among those the fewest rows.  Fragment reads take the tiles of a box in order, which
 // is free of bank conflicts where their rows are consecutive modulo 16 (the period of v_offset).  Planes and images are padded
@@ -494,8 +496,6 @@ __global__ __launch_bounds__(256) void row_filter_kernel(RowFilterArgs a) {
 // tile 0.  Cycles for the conflict-free number of them, per pass over the taps: N=64, 56x56 (4 images of 8 rows x 2 tiles) 24
 // for 12, 14x14 (14 rows x 4 tiles) 18 for 12, 28x28 15 for 12, 16x56x56 (4 planes of 14 rows x 1 tile) 72 for 36, N=1 7x7 6 for
 // 6; counted by SQ_LDS_BANK_CONFLICT at N=64 256 -> 256, 56x56: 14.45 M of 36.1 M cycles of the LDS.
-}  // namespace
-
 RowBox choose_box(int N, int oD, int oH, int nW, int kd, int kh, int tiles, int slots) {
   RowBox best{};
   long long best_rows = 0;

@@ -147,7 +147,8 @@ int pad_channels(const void* src, void* dst, long long n, int C, int Cx, long lo
 }
 
 // The fp32 parameters of a layer in its activations' type, weight and bias in one launch: as two casts they were two launches of some
-// 5 us of host time each, in a training step that waits for the host (us, fp16 N=64 128 -> 128, 28x28: 99.9 | 89.8).
+// 5 us of host time each, in a training step that waits for the host (us, fp16 N=64 128 -> 128, 28x28, twelve processes each: 93-96 | 91-93 where autograd's thread
+// wakes quickly, a matter of the process, and 114-122 | 110-115 where it does not).
 struct CastArgs {
   const float* src[2]; void* dst[2];
   long long n[2];
